@@ -55,6 +55,11 @@ SIGNATURES = {
         C.c_int,
         [_P, _P, _P, _P, _P, _P] + [_I64] * 4 + [_I64] * 12 + [C.c_float, C.c_int, _I64, _P, _I64, _P],
     ),
+    "based_linear_attn_prefill_f32_plan": (C.c_int, [_I64] * 4 + [C.POINTER(_I64), C.POINTER(_I64)]),
+    "based_linear_attn_prefill_f32": (
+        C.c_int,
+        [_P, _P, _P, _P, _P, _P] + [_I64] * 4 + [_I64] * 12 + [C.c_float, C.c_int, _I64, _P, _I64, _P],
+    ),
     "based_linear_attn_prefill_split_static": (
         C.c_int,
         [_P, _P, _P, _P, _P, _P] + [_I64] * 4 + [_I64] * 12 + [C.c_float, C.c_int, _I64, _P],

@@ -29,10 +29,9 @@
 //    transposing LDS read.  At the end the 160-slot state is expanded to the (dv, 273) decode
 //    layout.
 //
-//  * lin_prefill_f32_kernel (fp32 or bf16 in/out, fp32 arithmetic throughout): a plain
-//    recurrent evaluation, four tokens per round.  It serves fp32 callers (tolerance 1e-4
-//    is out of reach of bf16 operands) and is an independent second implementation that
-//    the tests compare the MFMA kernel against at sizes the CPU cannot reach.
+//  * lin_prefill_f32_kernel (linear_attn_f32.hip; fp32 or bf16 in/out, fp32 arithmetic throughout):
+//    fp32 callers (tolerance 1e-4 is out of reach of bf16 operands) and other head dims; the tests
+//    compare the MFMA kernel against it at sizes the CPU cannot reach.
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -41,6 +40,11 @@
 #include "common.hpp"
 
 namespace based {
+
+int launch_prefill_f32(const char* who, const void* q, const void* k, const void* v, void* y, float* kv_state, float* k_state, int64_t B,
+                       int64_t H, int64_t L, int64_t dv, int64_t q_sb, int64_t q_sh, int64_t q_sl, int64_t k_sb, int64_t k_sh, int64_t k_sl,
+                       int64_t v_sb, int64_t v_sh, int64_t v_sl, int64_t y_sb, int64_t y_sh, int64_t y_sl, float eps, int io_dtype,
+                       int64_t n_seg, float* ws, hipStream_t s);
 
 // ------------------------------------------------------------------------------------------
 // compile-time loop: body(std::integral_constant<int, I>{}) for I in [0, N)
@@ -928,118 +932,6 @@ __global__ __launch_bounds__(256) void lin_prefill_prefix_kernel(float* __restri
   }
 }
 
-// ------------------------------------------------------------------------------------------
-// fp32-arithmetic recurrent kernel.  Workgroup = (b, h, 64-channel block), 256 threads:
-// thread (e = tid % 64, fg = tid / 64) owns state entries S[f][e] for f = 4 i + fg.
-// ------------------------------------------------------------------------------------------
-constexpr int kRound = 4;                       // tokens per synchronisation round
-constexpr int kOwn = (kExp + 3) / 4;            // 69 state entries per thread
-
-__device__ __forceinline__ float phi_full(const float* x, int f) {
-  if (f == 0) return 1.0f;
-  if (f <= kFeat) return x[f - 1] * 0.5f;
-  const int g = f - 1 - kFeat;
-  return x[g >> 4] * x[g & 15] * 0.17677669529663687f;
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void lin_prefill_f32_kernel(
-    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, T* __restrict__ y,
-    float* __restrict__ kv_state, float* __restrict__ k_state, int H, int L, int dv, long q_sb,
-    long q_sh, long q_sl, long k_sb, long k_sh, long k_sl, long v_sb, long v_sh, long v_sl,
-    long y_sb, long y_sh, long y_sl, float eps) {
-  __shared__ float s_x[kRound][2][kFeat];          // [token][0 = k, 1 = q]
-  __shared__ float s_v[kRound][64];
-  __shared__ float s_phi[kRound][2][kExp + 3];
-  __shared__ float s_part[kRound][4][64];
-  __shared__ float s_den[kRound][4];
-
-  const int tid = threadIdx.x;
-  const int e = tid & 63, fg = tid >> 6;
-  const long bh = blockIdx.x;
-  const int eb = blockIdx.y;
-  const int b = (int)(bh / H), h = (int)(bh % H);
-  const int ew = dv - 64 * eb < 64 ? dv - 64 * eb : 64;  // live channels in this block
-  q += b * q_sb + h * q_sh;
-  k += b * k_sb + h * k_sh;
-  v += b * v_sb + h * v_sh + 64 * eb;
-  y += b * y_sb + h * y_sh + 64 * eb;
-
-  float S[kOwn];
-#pragma unroll
-  for (int i = 0; i < kOwn; ++i) S[i] = 0.f;
-  float ks0 = 0.f, ks1 = 0.f;  // normaliser state for features tid and tid + 256
-
-  for (int t0 = 0; t0 < L; t0 += kRound) {
-    const int nt = L - t0 < kRound ? L - t0 : kRound;
-    if (tid < kRound * 2 * kFeat) {
-      const int tt = tid / (2 * kFeat), which = (tid / kFeat) & 1, i = tid % kFeat;
-      float x = 0.f;
-      if (tt < nt) x = to_f32((which ? q : k)[(long)(t0 + tt) * (which ? q_sl : k_sl) + i]);
-      s_x[tt][which][i] = x;
-    }
-    {
-      const int tt = tid >> 6;
-      float x = 0.f;
-      if (tt < nt && e < ew) x = to_f32(v[(long)(t0 + tt) * v_sl + e]);
-      s_v[tt][e] = x;
-    }
-    __syncthreads();
-    for (int idx = tid; idx < kRound * 2 * kExp; idx += 256) {
-      const int tt = idx / (2 * kExp), rem = idx % (2 * kExp);
-      const int which = rem / kExp, f = rem % kExp;
-      s_phi[tt][which][f] = phi_full(s_x[tt][which], f);
-    }
-    __syncthreads();
-    for (int tt = 0; tt < nt; ++tt) {
-      const float ve = s_v[tt][e];
-      float acc = 0.f;
-#pragma unroll
-      for (int i = 0; i < kOwn; ++i) {
-        const int f = 4 * i + fg;
-        if (f < kExp) {
-          S[i] = __builtin_fmaf(s_phi[tt][0][f], ve, S[i]);
-          acc = __builtin_fmaf(s_phi[tt][1][f], S[i], acc);
-        }
-      }
-      s_part[tt][fg][e] = acc;
-      ks0 += s_phi[tt][0][tid];
-      float dpart = s_phi[tt][1][tid] * ks0;
-      if (tid + 256 < kExp) {
-        ks1 += s_phi[tt][0][tid + 256];
-        dpart = __builtin_fmaf(s_phi[tt][1][tid + 256], ks1, dpart);
-      }
-      dpart = wave_sum(dpart);
-      if (e == 0) s_den[tt][fg] = dpart;
-    }
-    __syncthreads();
-    {
-      const int tt = tid >> 6;
-      if (tt < nt && e < ew) {
-        const float num = s_part[tt][0][e] + s_part[tt][1][e] + s_part[tt][2][e] + s_part[tt][3][e];
-        const float den = s_den[tt][0] + s_den[tt][1] + s_den[tt][2] + s_den[tt][3];
-        y[(long)(t0 + tt) * y_sl + e] = from_f32<T>(num / (den + eps));
-      }
-    }
-    __syncthreads();
-  }
-
-  if (kv_state != nullptr) {
-    if (e < ew) {
-      float* row = kv_state + (bh * dv + 64 * eb + e) * kExp;
-#pragma unroll
-      for (int i = 0; i < kOwn; ++i) {
-        const int f = 4 * i + fg;
-        if (f < kExp) row[f] = S[i];
-      }
-    }
-    if (eb == 0) {
-      k_state[bh * kExp + tid] = ks0;
-      if (tid + 256 < kExp) k_state[bh * kExp + tid + 256] = ks1;
-    }
-  }
-}
-
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // Head dims the MFMA kernel serves: whole 16-channel tiles.  A block of 64 channels per workgroup;
@@ -1089,17 +981,8 @@ extern "C" BASED_API int based_linear_attn_prefill(
   }
   BASED_REQUIRE(dv >= 1 && dv <= 1024, BASED_ERR_SHAPE, "linear_attn_prefill: head dim %ld unsupported",
                 (long)dv);
-  dim3 grid((unsigned)(B * H), (unsigned)((dv + 63) / 64)), block(256);
-  if (io_dtype == BASED_BF16) {
-    hipLaunchKernelGGL(lin_prefill_f32_kernel<__bf16>, grid, block, 0, s, (const __bf16*)q,
-                       (const __bf16*)k, (const __bf16*)v, (__bf16*)y, kv_state, k_state, (int)H, (int)L,
-                       (int)dv, q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl, y_sb, y_sh, y_sl, eps);
-  } else {
-    hipLaunchKernelGGL(lin_prefill_f32_kernel<float>, grid, block, 0, s, (const float*)q,
-                       (const float*)k, (const float*)v, (float*)y, kv_state, k_state, (int)H, (int)L,
-                       (int)dv, q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl, y_sb, y_sh, y_sl, eps);
-  }
-  return check_launch("linear_attn_prefill");
+  return launch_prefill_f32("linear_attn_prefill", q, k, v, y, kv_state, k_state, B, H, L, dv, q_sb, q_sh, q_sl, k_sb, k_sh, k_sl,
+                            v_sb, v_sh, v_sl, y_sb, y_sh, y_sl, eps, io_dtype, 1, nullptr, s);
 }
 
 // Workgroup slots of one full wave of the MFMA prefill kernel on MI355X (256 CUs x 2 resident

@@ -381,7 +381,11 @@ def linear_attn_prefill(q, k, v, eps: float = 1e-12, return_state: bool = False,
         k_state = torch.empty(B, H, 1, 1, EXPANDED_DIM, dtype=torch.float32, device=q.device)
     lib = _lib.lib()
     n_seg, ws_bytes = ctypes.c_int64(1), ctypes.c_int64(0)
-    if split is not False:
+    run_split = lib.based_linear_attn_prefill_split
+    if split is None and (q.dtype == torch.float32 or dv % 16 != 0):  # fp32 arithmetic
+        _lib.check(lib.based_linear_attn_prefill_f32_plan(B, H, L, dv, ctypes.byref(n_seg), ctypes.byref(ws_bytes)))
+        run_split = lib.based_linear_attn_prefill_f32
+    elif split is not False:
         _lib.check(lib.based_linear_attn_prefill_plan(B, H, L, dv, _dtype_code(q), ctypes.byref(n_seg),
                                                       ctypes.byref(ws_bytes)))
     if isinstance(split, int) and not isinstance(split, bool) and split > 1:
@@ -397,8 +401,7 @@ def linear_attn_prefill(q, k, v, eps: float = 1e-12, return_state: bool = False,
         if n_seg.value > 1:
             # scratch for the per-segment states; torch's caching allocator makes this cheap
             ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=q.device)
-            _lib.check(lib.based_linear_attn_prefill_split(*args, n_seg.value, ws.data_ptr(), ws_bytes.value,
-                                                           _stream_ptr(q)))
+            _lib.check(run_split(*args, n_seg.value, ws.data_ptr(), ws_bytes.value, _stream_ptr(q)))
         else:
             _lib.check(lib.based_linear_attn_prefill(*args, _stream_ptr(q)))
     return y, kv_state, k_state

@@ -151,6 +151,23 @@ BASED_API int based_linear_attn_prefill_split(const void* q, const void* k, cons
                               int64_t n_seg, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * based_linear_attn_prefill in fp32 arithmetic (what it runs for fp32 tensors and for bf16 head dims that are no
+ * multiple of 16) with the sequences cut into up to 16 segments of whole 64-token chunks where few (batch, head) pairs
+ * would leave the GPU idle.  The plan reports the segment count for a shape (1 = do not split) and the bytes of 16-byte
+ * aligned workspace it needs; contents need no initialisation.  Any head dim up to 1024, any strides and alignment.
+ */
+BASED_API int based_linear_attn_prefill_f32_plan(int64_t B, int64_t H, int64_t L, int64_t dv, int64_t* n_seg, int64_t* workspace_bytes);
+BASED_API int based_linear_attn_prefill_f32(const void* q, const void* k, const void* v, void* y,
+                              float* kv_state, float* k_state,
+                              int64_t B, int64_t H, int64_t L, int64_t dv,
+                              int64_t q_sb, int64_t q_sh, int64_t q_sl,
+                              int64_t k_sb, int64_t k_sh, int64_t k_sl,
+                              int64_t v_sb, int64_t v_sh, int64_t v_sl,
+                              int64_t y_sb, int64_t y_sh, int64_t y_sl,
+                              float eps, int io_dtype,
+                              int64_t n_seg, void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * based_linear_attn_prefill_split without a workspace argument and without any allocation.
  * No counterpart in the reference: it exists for callers that cannot allocate device memory
  * (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc).  The
