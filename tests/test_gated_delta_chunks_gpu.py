@@ -1,0 +1,120 @@
+"""The gated delta rule in chunks of 64 tokens against the recurrence in 64 bits and against blocks of 16 tokens: lengths around whole
+chunks and tiles, head sizes with and without whole 16-byte pieces, shared heads, states that go on, decays that vanish, prompts
+longer than the workspace holds, and the shapes that stay with the blocks."""
+import pytest
+import torch
+
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+# fp32 sums over 64 tokens and 128 channels, errors of random signs that the recurrence contracts: below 32 roundings of 2^-24
+TOL = 2e-6
+
+
+def make(seed, B, L, H, G, d, dv, dtype, strong=False, pad=0):
+    g = torch.Generator().manual_seed(seed)
+    n = 2 * G * d + H * dv + pad
+    x = torch.nn.functional.silu(torch.randn(B, L, n, generator=g)).to(dtype)
+    ab = (torch.randn(B, L, 2 * H, generator=g) * (4 if strong else 1)).to(dtype)
+    return x, ab, (torch.randn(H, generator=g) + (3 if strong else -2)).to(dtype), torch.randn(H, generator=g).to(dtype)
+
+
+def reference(x, ab, a_log, dt_bias, H, G, d, dv, S=None):
+    B, L = x.shape[:2]
+    x, ab = x.double(), ab.double()
+    unit = lambda t: t / (t.square().sum(-1, keepdim=True) + 1e-6).sqrt()
+    share = lambda t: t.repeat_interleave(H // G, 2)
+    q = share(unit(x[..., :G * d].view(B, L, G, d)) * d ** -0.5)
+    k = share(unit(x[..., G * d:2 * G * d].view(B, L, G, d)))
+    v = x[..., 2 * G * d:2 * G * d + H * dv].view(B, L, H, dv)
+    decay = torch.exp(-torch.exp(a_log.double()) * torch.nn.functional.softplus(ab[..., :H] + dt_bias.double()))
+    beta = torch.sigmoid(ab[..., H:])
+    S = torch.zeros(B, H, d, dv, dtype=torch.float64, device=x.device) if S is None else S.double()
+    out = torch.empty(B, L, H, dv, dtype=torch.float64, device=x.device)
+    for t in range(L):
+        S = S * decay[:, t, :, None, None]
+        u = beta[:, t, :, None] * (v[:, t] - (k[:, t, :, None] @ S)[:, :, 0])
+        S = S + k[:, t, :, :, None] * u[:, :, None]
+        out[:, t] = (q[:, t, :, None] @ S)[:, :, 0]
+    return out, S
+
+
+def run(case, H, G, d, dv, state, fresh=True):
+    from based_amd import ops
+
+    x, ab, a_log, dt_bias = case
+    o = ops.gated_delta_scan(x[..., :G * d], x[..., G * d:2 * G * d], x[..., 2 * G * d:2 * G * d + H * dv], ab[..., :H], ab[..., H:], a_log,
+                             dt_bias, state, H, G, fresh)
+    return o, state[..., :dv]
+
+
+def in_chunks(B, L, H, d, dv):
+    from based_amd import _lib
+
+    return _lib.lib().based_gated_delta_scan_work(B, L, H, d, dv) > 0
+
+
+def empty_state(B, H, d, dv, dev):
+    return torch.full((B, H, d, (dv + 3) // 4 * 4), float("nan"), device=dev)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("L", [256, 257, 271, 272, 319, 320, 321, 500])
+def test_lengths(dev, dtype, L):
+    case = [t.to(dev) for t in make(L, 2, L, 3, 3, 64, 48, dtype)]
+    assert in_chunks(2, L, 3, 64, 48)
+    o, S = run(case, 3, 3, 64, 48, empty_state(2, 3, 64, 48, dev))
+    ref, S_ref = reference(*case, 3, 3, 64, 48)
+    assert rel_l2(o, ref) < TOL and rel_l2(S, S_ref) < TOL
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("strong", [False, True])
+@pytest.mark.parametrize("H,G,d,dv,pad", [(4, 2, 16, 16, 0), (2, 1, 18, 10, 3), (3, 3, 20, 70, 1), (1, 1, 64, 256, 0), (6, 2, 72, 36, 0), (4, 4, 128, 128, 8)])
+def test_heads(dev, dtype, strong, H, G, d, dv, pad):
+    L = 300
+    case = [t.to(dev) for t in make(d, 1, L, H, G, d, dv, dtype, strong, pad)]
+    assert in_chunks(1, L, H, d, dv)
+    state = empty_state(1, H, d, dv, dev)
+    o, S = run(case, H, G, d, dv, state)
+    ref, S_ref = reference(*case, H, G, d, dv)
+    assert rel_l2(o, ref) < TOL and rel_l2(S, S_ref) < TOL
+    # the same tokens again behind that state
+    o, S = run(case, H, G, d, dv, state, fresh=False)
+    ref, S_ref = reference(*case, H, G, d, dv, S_ref)
+    assert rel_l2(o, ref) < TOL and rel_l2(S, S_ref) < TOL
+
+
+def test_spans_of_a_long_prompt(dev):
+    """More chunks than the workspace holds at once."""
+    from based_amd import _lib
+
+    B, L, H, d, dv = 4, 1990, 16, 128, 128
+    chunks = (L + 63) // 64
+    floats = _lib.lib().based_gated_delta_scan_work(B, L, H, d, dv)
+    assert 0 < floats <= 64 << 20 and floats < _lib.lib().based_gated_delta_scan_work(B, 64 * 8, H, d, dv) // 8 * chunks
+    case = [t.to(dev) for t in make(3, B, L, H, H, d, dv, torch.bfloat16)]
+    o, S = run(case, H, H, d, dv, empty_state(B, H, d, dv, dev))
+    ref, S_ref = reference(*case, H, H, d, dv)
+    assert rel_l2(o, ref) < TOL and rel_l2(S, S_ref) < TOL
+
+
+@pytest.mark.parametrize("B,L,H,d,dv", [(1, 255, 4, 64, 64), (1, 300, 2, 129, 64), (5, 256, 13, 64, 64), (1, 256, 64, 64, 132)])
+def test_shapes_that_stay_with_blocks(dev, B, L, H, d, dv):
+    assert not in_chunks(B, L, H, d, dv)
+    case = [t.to(dev) for t in make(4, B, L, H, H, d, dv, torch.float32)]
+    o, S = run(case, H, H, d, dv, empty_state(B, H, d, dv, dev))
+    ref, S_ref = reference(*case, H, H, d, dv)
+    assert rel_l2(o, ref) < 3e-6 and rel_l2(S, S_ref) < 3e-6
+
+
+def test_rows_of_no_whole_pieces(dev):
+    """Heads of more than 64 channels whose rows start anywhere: blocks."""
+    H, d, dv, L = 2, 96, 32, 300
+    x, ab, a_log, dt_bias = (t.to(dev) for t in make(6, 1, L, H, H, d, dv, torch.float32, pad=1))
+    state = empty_state(1, H, d, dv, dev)
+    wide = torch.zeros(1, L, x.shape[-1] + 2, device=dev)
+    wide[..., 1:-1] = x
+    o, S = run((wide[..., 1:], ab, a_log, dt_bias), H, H, d, dv, state)
+    ref, S_ref = reference(x, ab, a_log, dt_bias, H, H, d, dv)
+    assert rel_l2(o, ref) < 3e-6 and rel_l2(S, S_ref) < 3e-6
