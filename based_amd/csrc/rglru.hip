@@ -3,12 +3,10 @@
 //   r = sigmoid(ra u + rb),  i = sigmoid(ri u + ib)      ra, ri block-diagonal: n x n per block
 //   log a = -c r softplus(lam),   S_t = a S_{t-1} + sqrt(1 - a^2) i u,   out = S * gelu_tanh(y)
 //
-//   rglru_gates  both gate products of 64 tokens x 64 channels on MFMA (bf16, or fp32 MFMA for fp32
-//                tensors), with the decay a and the input x = sqrt(1 - a^2) i u formed behind them, in
-//                fp32; and, for its 64 tokens, what the recurrence does to any state that enters
-//                them: S -> P S + X.
-//   rglru_scan   64 tokens per thread and channel: the state that enters them from the (P, X) of the
-//                segments before, then the recurrence and the output gate.
+//   rglru_segment  both gate products of 64 tokens x 64 channels on MFMA (bf16, or fp32 MFMA for fp32
+//                tensors), the decay a and the input x = sqrt(1 - a^2) i u formed behind them in fp32, the
+//                recurrence over the 64 tokens as S -> P S + X, and, from the (P, X) of the segments in
+//                front, the outputs.
 //   rglru_step   one token per sequence: the short convolution on its ring of past inputs, the gates,
 //                the state update and the output gate.
 #include "stream_common.hpp"
@@ -25,15 +23,16 @@ struct RglruArgs {
   const void* ri;
   const void* ib;
   const void* lam;
-  float* ga;   // (B, L, W) decay
-  float* gx;   // (B, L, W) input
-  float* agg;  // (B, segments + 1, 2, W): P and X; entry 0 is the state that enters the call
+  unsigned long long* agg;  // (B, segments, W): P below X, kUnset until a segment has them
+  int* tickets;  // (B, tiles) ticket_step apart: segments begun
+  int ticket_step;
   float* state;  // (B, W)
   void* out;
   int B, L, W, n, segs;
   long u_sb, u_sl, y_sb, y_sl, o_sb, o_sl;
   float c;
   int fresh;
+  bool vec_u, vec_y;  // rows of u, ra and ri, and of y and out, in 16-byte pieces
 };
 
 template <typename T> struct GateMma;
@@ -61,67 +60,92 @@ __device__ __forceinline__ void lru_gates(float zr, float zi, float sp, float u,
   x = __builtin_amdgcn_sqrtf(one_minus_square(a, log_a)) * i * u;
 }
 
-// grid: x = segment of the sequence, y = 64-channel tile within its block (ceil(n / 64) per block), z = sequence
+// lru_gates with the products before their biases: nrb, nib = -log2(e) times the bias, k2 = -2 c softplus(lam), kl = log2(e) / 2 times that.
+__device__ __forceinline__ void lru_gates_of(float zr, float zi, float nrb, float nib, float k2, float kl, float u, float& a, float& x) {
+  constexpr float kL = 1.4426950408889634f;
+  const float r = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(__builtin_fmaf(zr, -kL, nrb)));
+  const float i = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(__builtin_fmaf(zi, -kL, nib)));
+  a = __builtin_amdgcn_exp2f(kl * r);
+  x = __builtin_amdgcn_sqrtf(one_minus_square_of(a, k2 * r)) * (i * u);
+}
+
+constexpr unsigned long long kUnset = ~0ull;  // P as a NaN that no segment leaves
+
+__global__ __launch_bounds__(256) void rglru_begin_kernel(unsigned long long* agg, long n, int* tickets, int count, int step) {
+  const long at = (long)blockIdx.x * 256 + threadIdx.x, all = (long)gridDim.x * 256;
+  for (long i = at; i < n; i += all) agg[i] = kUnset;
+  for (long i = at; i < count; i += all) tickets[i * step] = 0;
+}
+
+// grid: x = segments of the sequence, y = 64-channel tile within its block (ceil(n / 64) per block), z = sequence.
+// A workgroup takes the next segment of its tile and sequence, forms the gates of 64 tokens, leaves what they do to any state that enters
+// them for the segments behind, and takes the state that enters its own from those in front.  It waits for them only after its own is
+// left; they were taken before it by workgroups that run or have run, so each wait ends.  P and X travel in one 64-bit word, which is
+// its own flag.  (Gates as fp32 pairs through memory for a second kernel, 134 of 184 MB at B = 4, L = 2048, W = 1024: 51 us; gates
+// formed by two kernels, 43 us: the vector unit is the bound, three exponentials, two reciprocals and a square root an element.)
+// The products lie with 16 consecutive tokens of a channel in one lane, where the recurrence is two instructions an element, and 64 in
+// a wavefront.  B = 4, L = 2048, W = 1024, 8 blocks: 29 us with the kernel in front; B = 8, L = 4096: 111 (237).
 template <typename T>
-__global__ __launch_bounds__(256) void rglru_gates_kernel(const RglruArgs a) {
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_kernel(const RglruArgs a) {
   typedef GateMma<T> M;
-  constexpr int KT = 128 / (int)sizeof(T);             // contraction staged at a time
-  constexpr int PAD = 16 / (int)sizeof(T);
-  constexpr int KS = KT + PAD;
-  constexpr int SPAD = 4;
-  // the operands, and after them the decays and inputs of the tile
-  constexpr int kOperands = 3 * 64 * KS * (int)sizeof(T), kTile = 2 * 64 * (64 + SPAD) * 4;
-  __shared__ __attribute__((aligned(16))) char s_mem[kOperands > kTile ? kOperands : kTile];
-  T* s_u = reinterpret_cast<T*>(s_mem);
-  T* s_r = s_u + 64 * KS;
-  T* s_i = s_r + 64 * KS;
-  float(*s_a)[64 + SPAD] = reinterpret_cast<float(*)[64 + SPAD]>(s_mem);  // [token][channel]
-  float(*s_x)[64 + SPAD] = s_a + 64;
-  __shared__ float s_const[3][64];
+  typedef typename Pack<T>::type vec_t;
+  constexpr int V = Pack<T>::kN;
+  constexpr int KT = 64, KS = KT + 16 / (int)sizeof(T);  // contraction staged at a time
+  __shared__ __attribute__((aligned(16))) T s_u[64 * KS], s_r[64 * KS], s_i[64 * KS];
+  T* s_y = s_r;  // (the output gate, then the output, once the products are done)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4;
   const int tiles = (a.n + 63) / 64;
   const int blk = blockIdx.y / tiles, c0 = (blockIdx.y % tiles) * 64;  // first output channel within the block
-  const int b = blockIdx.z, seg = blockIdx.x, l0 = seg * kSeg;
+  const int b = blockIdx.z;
+  __shared__ int s_seg;
+  if (a.segs > 1) {
+    if (tid == 0) s_seg = atomicAdd(a.tickets + ((long)b * gridDim.y + blockIdx.y) * a.ticket_step, 1);
+    __syncthreads();
+  }
+  const int seg = a.segs > 1 ? __builtin_amdgcn_readfirstlane(s_seg) : 0, l0 = seg * kSeg;
   const T* u = static_cast<const T*>(a.u) + b * a.u_sb + (long)blk * a.n;
   const T* ra = static_cast<const T*>(a.ra) + (long)blk * a.n * a.n;
   const T* ri = static_cast<const T*>(a.ri) + (long)blk * a.n * a.n;
-  if (tid < 64) {
-    const int ch = c0 + tid < a.n ? c0 + tid : a.n - 1, w = blk * a.n + ch;
-    s_const[0][tid] = to_f32(static_cast<const T*>(a.rb)[w]);
-    s_const[1][tid] = to_f32(static_cast<const T*>(a.ib)[w]);
-    s_const[2][tid] = softplus_f(to_f32(static_cast<const T*>(a.lam)[w]));
+  const int ch = c0 + wave * 16 + l16;  // a channel per column of a wavefront's products
+  const int w = blk * a.n + (ch < a.n ? ch : a.n - 1);
+  constexpr float kL = 1.4426950408889634f;
+  const float nrb = -kL * to_f32(static_cast<const T*>(a.rb)[w]), nib = -kL * to_f32(static_cast<const T*>(a.ib)[w]);
+  const float k2 = -2.0f * a.c * softplus_f(to_f32(static_cast<const T*>(a.lam)[w]));
+  const float kl = (0.5f * kL) * k2;
+  // Token q * 16 + i * 4 + j of the segment stands in row i * 16 + q * 4 + j: element j of product i in the lanes of quad q.
+  const auto token_of = [](int row) { return (row >> 2 & 3) * 16 + (row >> 4) * 4 + (row & 3); };
+  constexpr int YP = 64 * 64 / V / 256;
+  vec_t yv[YP];
+  const T* y = static_cast<const T*>(a.y) + b * a.y_sb + (long)blk * a.n + c0;
+  if (a.vec_y) {
+#pragma unroll
+    for (int i = 0; i < YP; ++i) {
+      const int p = i * 256 + tid, e = p % (64 / V) * V, t = l0 + token_of(p / (64 / V));
+      yv[i] = *reinterpret_cast<const vec_t*>(y + (t < a.L ? t : a.L - 1) * a.y_sl + (c0 + e < a.n ? e : 0));
+    }
   }
-  f32x4 zr[4], zi[4];  // wavefront: 16 tokens (columns) x 64 channels (rows)
+  f32x4 zr[4], zi[4];  // wavefront: 64 tokens (rows) x 16 channels (columns)
 #pragma unroll
   for (int i = 0; i < 4; ++i) zr[i] = zi[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  constexpr int V = Pack<T>::kN;
-  const bool vec = a.n % V == 0 && a.u_sb % V == 0 && a.u_sl % V == 0 && ((uintptr_t)a.u & 15) == 0 && ((uintptr_t)a.ra & 15) == 0 &&
-                   ((uintptr_t)a.ri & 15) == 0;
-  for (int k0 = 0; k0 < a.n; k0 += KT) {
-    __syncthreads();
-    typedef typename Pack<T>::type vec_t;
+  for (int it = 1, k0 = c0; it <= tiles; ++it) {  // the tile's own channels last: their u stays staged
+    k0 = k0 + KT < tiles * KT ? k0 + KT : 0;
+    if (it > 1) __syncthreads();
     constexpr int PIECES = 64 * (KT / V) / 256;
-    if (vec) {
+    if (a.vec_u) {
       vec_t xu[PIECES], xr[PIECES], xi[PIECES];
 #pragma unroll
       for (int i = 0; i < PIECES; ++i) {
         const int p = i * 256 + tid, row = p / (KT / V), e = (p % (KT / V)) * V;
-        const int tok = l0 + row < a.L ? l0 + row : a.L - 1, ch = c0 + row < a.n ? c0 + row : a.n - 1;
+        const int t = l0 + token_of(row), c = c0 + row < a.n ? c0 + row : a.n - 1;
         const int k = k0 + e < a.n ? k0 + e : 0;
-        xu[i] = *reinterpret_cast<const vec_t*>(u + tok * a.u_sl + k);
-        xr[i] = *reinterpret_cast<const vec_t*>(ra + (long)ch * a.n + k);
-        xi[i] = *reinterpret_cast<const vec_t*>(ri + (long)ch * a.n + k);
+        xu[i] = *reinterpret_cast<const vec_t*>(u + (t < a.L ? t : a.L - 1) * a.u_sl + k);
+        xr[i] = *reinterpret_cast<const vec_t*>(ra + (long)c * a.n + k);
+        xi[i] = *reinterpret_cast<const vec_t*>(ri + (long)c * a.n + k);
       }
 #pragma unroll
       for (int i = 0; i < PIECES; ++i) {
         const int p = i * 256 + tid, row = p / (KT / V), e = (p % (KT / V)) * V;
-        const bool in = k0 + e < a.n;
-#pragma unroll
-        for (int j = 0; j < V; ++j) {
-          xu[i][j] = in ? xu[i][j] : (T)0.0f;
-          xr[i][j] = in ? xr[i][j] : (T)0.0f;
-          xi[i][j] = in ? xi[i][j] : (T)0.0f;
-        }
+        if (k0 + e >= a.n) xu[i] = xr[i] = xi[i] = vec_t{};
         *reinterpret_cast<vec_t*>(&s_u[row * KS + e]) = xu[i];
         *reinterpret_cast<vec_t*>(&s_r[row * KS + e]) = xr[i];
         *reinterpret_cast<vec_t*>(&s_i[row * KS + e]) = xi[i];
@@ -129,10 +153,10 @@ __global__ __launch_bounds__(256) void rglru_gates_kernel(const RglruArgs a) {
     } else {
       for (int p = tid; p < 64 * KT; p += 256) {
         const int row = p / KT, e = p % KT;
-        const int tok = l0 + row < a.L ? l0 + row : a.L - 1, ch = c0 + row < a.n ? c0 + row : a.n - 1;
+        const int t = l0 + token_of(row), c = c0 + row < a.n ? c0 + row : a.n - 1;
         const bool in = k0 + e < a.n;
         const int k = in ? k0 + e : 0;
-        const T xu = u[tok * a.u_sl + k], xr = ra[(long)ch * a.n + k], xi = ri[(long)ch * a.n + k];
+        const T xu = u[(t < a.L ? t : a.L - 1) * a.u_sl + k], xr = ra[(long)c * a.n + k], xi = ri[(long)c * a.n + k];
         s_u[row * KS + e] = in ? xu : (T)0.0f;
         s_r[row * KS + e] = in ? xr : (T)0.0f;
         s_i[row * KS + e] = in ? xi : (T)0.0f;
@@ -142,128 +166,131 @@ __global__ __launch_bounds__(256) void rglru_gates_kernel(const RglruArgs a) {
 #pragma unroll
     for (int kk = 0; kk < KT; kk += M::kK) {
       const int e = kk + quad * M::kPer;
-      const typename M::frag_t fu = *reinterpret_cast<const typename M::frag_t*>(&s_u[(wave * 16 + l16) * KS + e]);
+      const typename M::frag_t fr = *reinterpret_cast<const typename M::frag_t*>(&s_r[(wave * 16 + l16) * KS + e]);
+      const typename M::frag_t fi = *reinterpret_cast<const typename M::frag_t*>(&s_i[(wave * 16 + l16) * KS + e]);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        zr[i] = M::run(*reinterpret_cast<const typename M::frag_t*>(&s_r[(i * 16 + l16) * KS + e]), fu, zr[i]);
-        zi[i] = M::run(*reinterpret_cast<const typename M::frag_t*>(&s_i[(i * 16 + l16) * KS + e]), fu, zi[i]);
+        const typename M::frag_t fu = *reinterpret_cast<const typename M::frag_t*>(&s_u[(i * 16 + l16) * KS + e]);
+        zr[i] = M::run(fu, fr, zr[i]);
+        zi[i] = M::run(fu, fi, zi[i]);
       }
     }
-  }
-  __syncthreads();  // the operands are done with
-  // lane: token wave*16 + l16, channels i*16 + quad*4 ..
-  const int tl = wave * 16 + l16, tok = l0 + tl;
-  const bool tok_in = tok < a.L;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int ch = i * 16 + quad * 4;
-    f32x4 ov, xv;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int cc = c0 + ch + j < a.n ? c0 + ch + j : a.n - 1;
-      const float uv = to_f32(u[(tok_in ? tok : a.L - 1) * a.u_sl + cc]);
-      float av, x;
-      lru_gates(zr[i][j] + s_const[0][ch + j], zi[i][j] + s_const[1][ch + j], s_const[2][ch + j], uv, a.c, av, x);
-      ov[j] = av, xv[j] = x;
-    }
-    *reinterpret_cast<f32x4*>(&s_a[tl][ch]) = ov;
-    *reinterpret_cast<f32x4*>(&s_x[tl][ch]) = xv;
   }
   __syncthreads();
-  // the tile in rows of 64 channels, and the segment's effect on a state that enters it
-  const int ntok = a.L - l0 < kSeg ? a.L - l0 : kSeg;
-  const int nch = a.n - c0 < 64 ? a.n - c0 : 64;
-  const long base = ((long)b * a.L + l0) * a.W + (long)blk * a.n + c0;
-  for (int p = tid; p < ntok * 64; p += 256) {
-    const int t = p >> 6, ch = p & 63;
-    if (ch < nch) {
-      a.ga[base + (long)t * a.W + ch] = s_a[t][ch];
-      a.gx[base + (long)t * a.W + ch] = s_x[t][ch];
+  if (a.vec_y) {
+#pragma unroll
+    for (int i = 0; i < YP; ++i) {
+      const int p = i * 256 + tid;
+      *reinterpret_cast<vec_t*>(&s_y[p / (64 / V) * KS + p % (64 / V) * V]) = yv[i];
+    }
+  } else {
+    for (int p = tid; p < 64 * 64; p += 256) {
+      const int row = p / 64, e = p % 64, t = l0 + token_of(row);
+      s_y[row * KS + e] = y[(t < a.L ? t : a.L - 1) * a.y_sl + (c0 + e < a.n ? e : 0)];
     }
   }
-  if (tid < nch) {
-    float P = 1.f, X = 0.f;
-    for (int t = 0; t < ntok; ++t) {
-      const float av = s_a[t][tid];
-      P *= av;
-      X = __builtin_fmaf(av, X, s_x[t][tid]);
-    }
-    const int w = blk * a.n + c0 + tid;
-    float* g = a.agg + ((long)b * (a.segs + 1) + seg + 1) * 2 * a.W + w;
-    g[0] = P;
-    g[a.W] = X;
-    if (seg == 0) {
-      float* g0 = a.agg + (long)b * (a.segs + 1) * 2 * a.W + w;
-      g0[0] = 0.f;
-      g0[a.W] = a.fresh ? 0.f : a.state[(long)b * a.W + w];
+  __syncthreads();
+  float A[4][4], I[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      lru_gates_of(zr[i][j], zi[i][j], nrb, nib, k2, kl, to_f32(s_u[(i * 16 + quad * 4 + j) * KS + wave * 16 + l16]), A[i][j], I[i][j]);
+  if (l0 + kSeg > a.L) {  // tokens behind the last one change nothing
+    const int live = a.L - l0 - quad * 16;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      A[t / 4][t % 4] = t < live ? A[t / 4][t % 4] : 1.f;
+      I[t / 4][t % 4] = t < live ? I[t / 4][t % 4] : 0.f;
     }
   }
-}
-
-// C consecutive channels as floats / from floats
-template <typename T, int C> __device__ __forceinline__ void load_ch(const T* p, float (&out)[C]) {
-  typedef __attribute__((ext_vector_type(C))) T vec_t;
-  const vec_t x = *reinterpret_cast<const vec_t*>(p);
+  float P = A[0][0], X = I[0][0];
 #pragma unroll
-  for (int c = 0; c < C; ++c) out[c] = to_f32(x[c]);
-}
-
-// grid: x = tile of 256 C channels, y = segment, z = sequence; C channels per thread
-template <typename T, int C>
-__global__ __launch_bounds__(256) void rglru_scan_kernel(const RglruArgs a) {
-  const int w = (blockIdx.x * 256 + threadIdx.x) * C;
-  if (w >= a.W) return;
-  const int seg = blockIdx.y, b = blockIdx.z, l0 = seg * kSeg;
-  const float* g = a.agg + (long)b * (a.segs + 1) * 2 * a.W + w;
-  float S[C];
-#pragma unroll
-  for (int c = 0; c < C; ++c) S[c] = 0.f;
-  constexpr int U = 8;
-  for (int i0 = 0; i0 <= seg; i0 += U) {
-    float P[U][C], X[U][C];
-#pragma unroll
-    for (int i = 0; i < U; ++i) {
-      const long at = (long)(i0 + i <= seg ? i0 + i : seg) * 2 * a.W;
-      load_ch<float, C>(g + at, P[i]);
-      load_ch<float, C>(g + at + a.W, X[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < U; ++i)
-#pragma unroll
-      for (int c = 0; c < C; ++c) S[c] = i0 + i <= seg ? __builtin_fmaf(P[i][c], S[c], X[i][c]) : S[c];
+  for (int t = 1; t < 16; ++t) {
+    X = __builtin_fmaf(A[t / 4][t % 4], X, I[t / 4][t % 4]);
+    P *= A[t / 4][t % 4];
   }
-  const int ntok = a.L - l0 < kSeg ? a.L - l0 : kSeg;
-  const float* pa = a.ga + ((long)b * a.L + l0) * a.W + w;
-  const float* px = a.gx + ((long)b * a.L + l0) * a.W + w;
-  const T* py = static_cast<const T*>(a.y) + b * a.y_sb + l0 * a.y_sl + w;
-  T* po = static_cast<T*>(a.out) + b * a.o_sb + l0 * a.o_sl + w;
-  for (int t0 = 0; t0 < ntok; t0 += U) {
-    float av[U][C], xv[U][C], yv[U][C];
+  // the quads in front of this one
+  float before_p = 1.f, before_x = 0.f;
 #pragma unroll
-    for (int i = 0; i < U; ++i) {
-      const int t = t0 + i < ntok ? t0 + i : ntok - 1;
-      load_ch<float, C>(pa + (long)t * a.W, av[i]);
-      load_ch<float, C>(px + (long)t * a.W, xv[i]);
-      load_ch<T, C>(py + t * a.y_sl, yv[i]);
+  for (int q = 0; q < 3; ++q) {
+    const float p = __shfl(P, q * 16 + l16), x = __shfl(X, q * 16 + l16);
+    before_x = q < quad ? __builtin_fmaf(p, before_x, x) : before_x;
+    before_p = q < quad ? p * before_p : before_p;
+  }
+  float S = seg == 0 && !a.fresh ? a.state[(long)b * a.W + w] : 0.f;
+  unsigned long long* g = a.agg + (long)b * a.segs * a.W + w;
+  if (seg < a.segs - 1 && quad == 3 && ch < a.n) {
+    float xw = __builtin_fmaf(P, before_x, X), pw = P * before_p;
+    if (seg == 0) {  // (what enters the call is part of it: the last segment replaces the state)
+      xw = __builtin_fmaf(pw, S, xw);
+      pw = 0.f;
     }
+    unsigned int bits = __builtin_bit_cast(unsigned int, pw);
+    bits = bits == ~0u ? 0x7fc00000u : bits;
+    __hip_atomic_store(g + (long)seg * a.W, (unsigned long long)__builtin_bit_cast(unsigned int, xw) << 32 | bits, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (seg > 0) {
+    // a quarter of the segments in front for each quad
+    const int each = (seg + 3) / 4, first = quad * each;
+    float p = 1.f, x = 0.f;
+    constexpr int U = 4;
+    for (int i0 = 0; i0 < each; i0 += U) {
+      unsigned long long v[U];
+      bool wait;
+      do {
+        wait = false;
 #pragma unroll
-    for (int i = 0; i < U; ++i) {
-      if (t0 + i < ntok) {
-        typedef __attribute__((ext_vector_type(C))) T vec_t;
-        vec_t o;
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-          S[c] = __builtin_fmaf(av[i][c], S[c], xv[i][c]);
-          o[c] = from_f32<T>(S[c] * gelu_tanh_f(yv[i][c]));
+        for (int i = 0; i < U; ++i) {
+          const int at = first + i0 + i;
+          v[i] = __hip_atomic_load(g + (long)(at < seg ? at : seg - 1) * a.W, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        *reinterpret_cast<vec_t*>(po + (t0 + i) * a.o_sl) = o;
+#pragma unroll
+        for (int i = 0; i < U; ++i) wait |= (unsigned int)v[i] == ~0u;
+      } while (__any(wait));
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        const bool in = i0 + i < each && first + i0 + i < seg;
+        const float pi = __builtin_bit_cast(float, (unsigned int)v[i]), xi = __builtin_bit_cast(float, (unsigned int)(v[i] >> 32));
+        x = in ? __builtin_fmaf(pi, x, xi) : x;
+        p = in ? p * pi : p;
       }
     }
-  }
-  if (seg == a.segs - 1) {
+    S = __shfl(x, l16);
 #pragma unroll
-    for (int c = 0; c < C; ++c) a.state[(long)b * a.W + w + c] = S[c];
+    for (int q = 1; q < 4; ++q) S = __builtin_fmaf(__shfl(p, q * 16 + l16), S, __shfl(x, q * 16 + l16));
   }
+  S = __builtin_fmaf(before_p, S, before_x);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      S = __builtin_fmaf(A[i][j], S, I[i][j]);
+      T* at = &s_y[(i * 16 + quad * 4 + j) * KS + wave * 16 + l16];
+      *at = from_f32<T>(S * gelu_tanh_f(to_f32(*at)));
+    }
+  if (seg == a.segs - 1 && quad == 3 && ch < a.n) a.state[(long)b * a.W + w] = S;
+  __syncthreads();
+  T* out = static_cast<T*>(a.out) + b * a.o_sb + (long)blk * a.n + c0;
+  if (a.vec_y) {
+#pragma unroll
+    for (int i = 0; i < YP; ++i) {
+      const int p = i * 256 + tid, row = p / (64 / V), e = p % (64 / V) * V, t = l0 + token_of(row);
+      if (t < a.L && c0 + e < a.n) *reinterpret_cast<vec_t*>(out + t * a.o_sl + e) = *reinterpret_cast<const vec_t*>(&s_y[row * KS + e]);
+    }
+  } else {
+    for (int p = tid; p < 64 * 64; p += 256) {
+      const int row = p / 64, e = p % 64, t = l0 + token_of(row);
+      if (t < a.L && c0 + e < a.n) out[t * a.o_sl + e] = s_y[row * KS + e];
+    }
+  }
+}
+
+// Rows from the scratch to an output that shares memory with the input.
+template <typename T> __global__ __launch_bounds__(256) void rglru_copy_kernel(const T* src, T* dst, int L, int W, long o_sb, long o_sl) {
+  for (int l = blockIdx.x * kSeg; l < L && l < ((int)blockIdx.x + 1) * kSeg; ++l)
+    for (int w = threadIdx.x; w < W; w += 256) dst[blockIdx.y * o_sb + l * o_sl + w] = src[((long)blockIdx.y * L + l) * W + w];
 }
 
 // ---- one token per sequence ----
@@ -430,15 +457,36 @@ __global__ __launch_bounds__(256) void rglru_step_kernel(const RglruStepArgs a) 
   }
 }
 
-template <typename T> void launch_rglru_prefill(const RglruArgs& a, int tiles, bool pairs, hipStream_t s) {
-  const int per = pairs ? 512 : 256;
-  const dim3 g1((unsigned)a.segs, (unsigned)tiles, (unsigned)a.B);
-  const dim3 g2((unsigned)((a.W + per - 1) / per), (unsigned)a.segs, (unsigned)a.B), block(256);
-  hipLaunchKernelGGL(rglru_gates_kernel<T>, g1, block, 0, s, a);
-  if (pairs)
-    hipLaunchKernelGGL((rglru_scan_kernel<T, 2>), g2, block, 0, s, a);
-  else
-    hipLaunchKernelGGL((rglru_scan_kernel<T, 1>), g2, block, 0, s, a);
+template <typename T> void launch_rglru_prefill(const RglruArgs& a, int tiles, T* apart, hipStream_t s) {
+  const dim3 grid((unsigned)a.segs, (unsigned)tiles, (unsigned)a.B), block(256);
+  RglruArgs t = a;
+  if (apart) {
+    t.out = apart;
+    t.o_sl = a.W;
+    t.o_sb = (long)a.L * a.W;
+    t.vec_y = a.vec_y && aligned_to(apart, 16);
+  }
+  if (a.segs > 1) {
+    const long words = (long)a.B * a.segs * a.W;
+    const long groups = (words + 1023) / 1024;
+    hipLaunchKernelGGL(rglru_begin_kernel, dim3((unsigned)(groups < 2048 ? groups : 2048)), block, 0, s, a.agg, words, a.tickets, a.B * tiles,
+                       a.ticket_step);
+  }
+  hipLaunchKernelGGL(rglru_segment_kernel<T>, grid, block, 0, s, t);
+  if (apart)
+    hipLaunchKernelGGL(rglru_copy_kernel<T>, dim3((unsigned)a.segs, (unsigned)a.B), block, 0, s, apart, static_cast<T*>(a.out), a.L, a.W,
+                       a.o_sb, a.o_sl);
+}
+
+// whether two (B, L, W) tensors lie in overlapping stretches of memory
+bool rglru_meet(const void* p, int64_t p_sb, int64_t p_sl, const void* q, int64_t q_sb, int64_t q_sl, int64_t B, int64_t L, int64_t W,
+                int64_t size) {
+  const auto edge = [&](const void* base, int64_t sb, int64_t sl, bool high) {
+    int64_t e = high ? W : 0;
+    for (const int64_t d : {(B - 1) * sb, (L - 1) * sl}) e += (d > 0) == high ? d : 0;
+    return (int64_t)(uintptr_t)base + e * size;
+  };
+  return edge(p, p_sb, p_sl, false) < edge(q, q_sb, q_sl, true) && edge(q, q_sb, q_sl, false) < edge(p, p_sb, p_sl, true);
 }
 
 }  // namespace based
@@ -456,15 +504,23 @@ extern "C" BASED_API int based_rglru_prefill(const void* u, const void* y, const
   const int64_t n = W / blocks, segs = (L + kSeg - 1) / kSeg, tiles = blocks * ((n + 63) / 64);
   BASED_REQUIRE(B < 65536 && segs < 65536 && tiles < 65536 && L < (1ll << 31), BASED_ERR_SHAPE, "rglru_prefill: grid too large");
   if (B == 0 || L == 0) return BASED_OK;
-  const RglruArgs a{u,      y,      ra,     rb,     ri,        ib,   lam,  work_a, work_x, work_agg, state, out, (int)B,
-                    (int)L, (int)W, (int)n, (int)segs, u_sb, u_sl, y_sb,   y_sl,   o_sb,     o_sl,  c,   fresh};
+  const int64_t size = io_dtype == BASED_BF16 ? 2 : 4;
+  const int64_t v = 16 / size;
+  const auto whole = [&](const void* p, int64_t sb, int64_t sl) { return sl % v == 0 && (B == 1 || sb % v == 0) && aligned_to(p, 16); };
+  const bool vec_u = n % v == 0 && whole(u, u_sb, u_sl) && aligned_to(ra, 16) && aligned_to(ri, 16);
+  const bool vec_y = n % v == 0 && whole(y, y_sb, y_sl) && whole(out, o_sb, o_sl);
+  // 64-bit words of every segment from the first aligned address on; the tickets, at most W of a sequence, in the last entry's 2 W values
+  unsigned long long* agg = reinterpret_cast<unsigned long long*>(((uintptr_t)work_agg + 7) & ~(uintptr_t)7);
+  const int step = (int)(2 * W / tiles);
+  const RglruArgs a{u, y, ra, rb, ri, ib, lam, agg, reinterpret_cast<int*>(agg + B * segs * W), step, state, out, (int)B, (int)L, (int)W, (int)n, (int)segs, u_sb, u_sl, y_sb, y_sl,
+                    o_sb, o_sl, c, fresh, vec_u, vec_y};
+  // A workgroup reads channels of u that others' outputs would replace.
+  const bool apart = rglru_meet(u, u_sb, u_sl, out, o_sb, o_sl, B, L, W, size);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool pairs = W % 2 == 0 && y_sb % 2 == 0 && y_sl % 2 == 0 && o_sb % 2 == 0 && o_sl % 2 == 0 && aligned_to(y, 8) &&
-                     aligned_to(out, 8) && aligned_to(work_a, 8) && aligned_to(work_x, 8) && aligned_to(work_agg, 8);
   if (io_dtype == BASED_BF16)
-    launch_rglru_prefill<__bf16>(a, (int)tiles, pairs, s);
+    launch_rglru_prefill<__bf16>(a, (int)tiles, apart ? reinterpret_cast<__bf16*>(work_x) : nullptr, s);
   else
-    launch_rglru_prefill<float>(a, (int)tiles, pairs, s);
+    launch_rglru_prefill<float>(a, (int)tiles, apart ? work_x : nullptr, s);
   return check_launch("rglru_prefill");
 }
 

@@ -37,13 +37,14 @@ __device__ __forceinline__ float tanh_f(float z) {
   const float near = z * (1.0f - q * (1.0f / 3.0f - q * (2.0f / 15.0f)));
   return fabsf(z) < 0.05f ? near : far;
 }
-// 1 - a^2 for a = exp(log_a) <= 1 without cancellation: the series of 1 - exp(x), x = 2 log_a, above -1/4 (the
+// 1 - a^2 for a = exp(x / 2) <= 1 without cancellation: the series of 1 - exp(x) above -1/4 (the
 // next term is 5e-8 of the sum)
-__device__ __forceinline__ float one_minus_square(float a, float log_a) {
-  const float x = 2.0f * log_a, p = x * (1.f / 720.f) + 1.f / 120.f;
+__device__ __forceinline__ float one_minus_square_of(float a, float x) {
+  const float p = x * (1.f / 720.f) + 1.f / 120.f;
   const float series = -x * (1.f + x * (0.5f + x * (1.f / 6.f + x * (1.f / 24.f + x * p))));
   return x > -0.25f ? series : __builtin_fmaf(-a, a, 1.0f);
 }
+__device__ __forceinline__ float one_minus_square(float a, float log_a) { return one_minus_square_of(a, 2.0f * log_a); }
 // x as the element type would keep it
 template <typename T> __device__ __forceinline__ float round_to(float x) { return to_f32(from_f32<T>(x)); }
 

@@ -1,0 +1,55 @@
+"""The gated recurrence over portions whose length, block width and rows put its 16-token, 64-token and 64-channel edges everywhere."""
+import pytest
+import torch
+
+from oracle import sozilix_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("L,W,blocks,rows,carry", [
+    (1, 64, 1, "own", True), (15, 8, 2, "own", True), (16, 68, 1, "own", False), (17, 60, 1, "shifted", True), (63, 192, 3, "sliced", True),
+    (64, 33, 1, "own", True), (65, 260, 2, "sliced", False), (577, 72, 1, "own", True), (2049, 16, 2, "shifted", True),
+    (130, 136, 1, "over u", True), (200, 66, 2, "over y", True), (1000, 8, 1, "beside u", False), (6000, 1024, 16, "own", True)])
+def test_rglru_segments(dev, dtype, L, W, blocks, rows, carry):
+    """`rows`: tensors of their own; rows that start off an aligned address; slices of wider rows; an output in the place of an input
+    or in the same rows."""
+    from based_amd import ops
+
+    B, n = 3, W // blocks
+    g = torch.Generator().manual_seed(L * 131 + W)
+    u, y = (torch.randn(B, L, W, generator=g).to(dtype) for _ in range(2))
+    ra, ri = ((torch.randn(blocks, n, n, generator=g) * n ** -0.5).to(dtype) for _ in range(2))
+    rb, ib = (torch.randn(W, generator=g).to(dtype) for _ in range(2))
+    lam = (2 * torch.randn(W, generator=g) - 3).to(dtype)
+    start = torch.randn(B, W, generator=g)
+
+    def placed(t):
+        if rows == "shifted":
+            return torch.empty(B, L, W + 5, dtype=dtype, device=dev)[..., 3:3 + W].copy_(t)
+        if rows == "sliced":
+            return torch.empty(B, L, 2 * W + 8, dtype=dtype, device=dev)[..., W:2 * W].copy_(t)
+        return t.to(dev)
+
+    ud, yd, out = placed(u), placed(y), placed(torch.full((B, L, W), float("nan"), dtype=dtype))
+    if rows == "beside u":
+        both = torch.full((B, L, 2 * W), float("nan"), dtype=dtype, device=dev)
+        ud, out = both[..., :W].copy_(u), both[..., W:]
+    out = {"over u": ud, "over y": yd}.get(rows, out)
+    state = start.to(dev) if carry else torch.full((B, W), float("nan"), device=dev)
+    ops.rglru_prefill(ud, yd, *(t.to(dev) for t in (ra, rb, ri, ib, lam)), state, 8.0, fresh=not carry, out=out)
+    # in 64 bits; a start state decays as a zero-input sequence does: the recurrence is linear in (u i sqrt, S)
+    zr = torch.einsum("blkn,kmn->blkm", u.double().view(B, L, blocks, n), ra.double()).reshape(B, L, W) + rb.double()
+    zi = torch.einsum("blkn,kmn->blkm", u.double().view(B, L, blocks, n), ri.double()).reshape(B, L, W) + ib.double()
+    log_a = -8.0 * torch.sigmoid(zr) * torch.nn.functional.softplus(lam.double())
+    x = torch.sqrt(-torch.expm1(2 * log_a)) * torch.sigmoid(zi) * u.double()
+    S, ref = start.double() if carry else torch.zeros(B, W, dtype=torch.float64), []
+    for t in range(L):
+        S = log_a[:, t].exp() * S + x[:, t]
+        ref.append(S * O.gelu_tanh(y[:, t].double()))
+    ref = torch.stack(ref, 1)
+    # fp32: a dozen roundings of 2^-24 each through gates, decays and the scan; bf16 outputs add half of 2^-8 each
+    rel = lambda a, b: ((a.double().cpu() - b).norm() / b.norm()).item()  # noqa: E731
+    assert rel(state, S) < 2e-6, rel(state, S)
+    assert rel(out, ref) < (2e-6 if dtype == torch.float32 else 2.5e-3), rel(out, ref)
