@@ -13,6 +13,7 @@
 //                        all of them and a tile of tokens is short against the window.  Scores are
 //                        formed transposed (keys x queries), which leaves the weights in the lanes
 //                        that the product with the values wants them in.
+//   window_prefill_f32   fp32: 64 rows per workgroup, 16 per wavefront, otherwise alike, on fp32 MFMA
 //   window_prefill_any   any element type and size: one wavefront per query
 //   window_step          one token per sequence: rotation, value norm, cache write and attention,
 //                        one workgroup per (sequence, key/value head)
@@ -394,6 +395,215 @@ __global__ __launch_bounds__(256, KC <= 3 && VC <= 2 ? 3 : 1) void window_prefil
         }
       }
     }
+  }
+}
+
+// ---- prefill, fp32, fp32 MFMA ----
+// KB, VB: 64-channel blocks of the key and value sizes (rounded up; channels past the real sizes are zeros).  64 (token, head) rows
+// per workgroup, 16 per wavefront, keys and values 32 at a time in LDS for the four.  As in bf16, scores come transposed: the four
+// weights of a lane are what the products with the values take, one each, where product j contracts keys j, 4 + j, 8 + j and 12 + j;
+// keys and queries give up their channels in the same order, so that a lane reads 16 bytes for four products.
+// Bound by the fp32 matrix rate from some thousand rows on and by the chain of one wavefront below.  16 heads on 4, size 64, 129 keys:
+// B = 1, L = 777, with the cache write: 19 us (a wavefront per query on the vector unit: 70); B = 4, L = 2048: 89 us (661).
+constexpr int kF32Keys = 32, kF32Rows = 64;
+
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// channels c .. c + 3 of a row, turned; c and the rotary size (its half in half-split pairs) multiples of 4
+__device__ __forceinline__ f32x4 turned4(const float* row, int c, int pos, const WindowArgs& a) {
+  f32x4 x = *reinterpret_cast<const f32x4*>(row + c);
+  if (c < a.rot) {
+    const int half = a.rot / 2;
+    if (a.half_split) {
+      const int pair = c < half ? c : c - half;
+      const float sgn = c < half ? -1.f : 1.f;
+      const f32x4 y = *reinterpret_cast<const f32x4*>(row + (c < half ? c + half : c - half));
+      const float *cs = a.cos_t + (long)pos * half + pair, *sn = a.sin_t + (long)pos * half + pair;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = x[j] * cs[j] + sgn * y[j] * sn[j];
+    } else {
+      const float *cs = a.cos_t + (long)pos * half + c / 2, *sn = a.sin_t + (long)pos * half + c / 2;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const float u = x[2 * j], v = x[2 * j + 1];
+        x[2 * j] = u * cs[j] - v * sn[j];
+        x[2 * j + 1] = v * cs[j] + u * sn[j];
+      }
+    }
+  }
+  return x;
+}
+
+template <int KB, int VB>
+__global__ __launch_bounds__(256) void window_prefill_f32_kernel(const WindowArgs a) {
+  constexpr int D = KB * 64, DV = VB * 64, KS = D + 4, VS = DV + 4;
+  __shared__ __attribute__((aligned(16))) float lds_k[kF32Keys * KS], lds_v[kF32Keys * VS];
+  __shared__ int s_odd[4];  // values of this tile that are not finite, by the wavefront that staged them
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4;
+  const int b = blockIdx.y / a.G, g = blockIdx.y % a.G, qpk = a.H / a.G, n_rows = a.L * qpk;
+  const int r0 = blockIdx.x * kF32Rows, row_w = r0 + wave * 16;
+  const auto token_of = [&](int row) { return (row < n_rows ? row : n_rows - 1) / qpk; };
+  const float* kv = static_cast<const float*>(a.kv) + b * a.kv_sb + (long)g * (a.d + a.dv);
+  const int tok = token_of(row_w + l16), pos = a.pos_host + tok;
+  const int head = g * qpk + (row_w + l16 < n_rows ? row_w + l16 : n_rows - 1) % qpk;
+  const int first = a.pos_host + token_of(r0), last = a.pos_host + token_of(r0 + kF32Rows - 1);
+  const int wave_lo = a.pos_host + token_of(row_w), wave_hi = a.pos_host + token_of(row_w + 15);
+  const int lo = first - a.window + 1 > 0 ? first - a.window + 1 : 0;
+
+  f32x4 kbuf[2 * KB], vbuf[2 * VB];
+  const auto fetch = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < 2 * KB; ++i) {
+      const int p = i * 256 + tid, key = p / (D / 4), e = p % (D / 4) * 4;
+      kbuf[i] = *reinterpret_cast<const f32x4*>(kv + (long)(k0 + key <= last ? k0 + key : last) * a.kv_st + (e < a.d ? e : 0));
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * VB; ++i) {
+      const int p = i * 256 + tid, key = p / (DV / 4), e = p % (DV / 4) * 4;
+      vbuf[i] = *reinterpret_cast<const f32x4*>(kv + (long)(k0 + key <= last ? k0 + key : last) * a.kv_st + a.d + (e < a.dv ? e : 0));
+    }
+  };
+  fetch(lo);
+  f32x4 qf[4 * KB];
+  {
+    const float* q = static_cast<const float*>(a.q) + b * a.q_sb + tok * a.q_sl + (long)head * a.d;
+#pragma unroll
+    for (int c = 0; c < 4 * KB; ++c) {
+      const int e = c * 16 + quad * 4;
+      qf[c] = turned4(q, e < a.d ? e : 0, pos, a);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) qf[c][j] = e < a.d ? (a.scale < 0.f ? -qf[c][j] : qf[c][j]) : 0.f;
+    }
+  }
+  f32x4 acc[VB][4];  // channels vb * 64 + (quad * 4 + i) * 4 + c of row l16 in [vb][c][i]
+#pragma unroll
+  for (int vb = 0; vb < VB; ++vb)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[vb][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+  // Powers of two of the differences, which are exact where they count; the sign is the queries'.  At scale 0 every difference is
+  // all but lost, while a key out of sight stays at minus infinity.
+  const float scale2 = a.scale == 0.f ? 1e-38f : fabsf(a.scale) * 1.4426950408889634f;
+
+  for (int k0 = lo; k0 <= last; k0 += kF32Keys) {
+    __syncthreads();  // every wavefront is done with the tile before
+    bool odd = false;
+#pragma unroll
+    for (int i = 0; i < 2 * KB; ++i) {
+      const int p = i * 256 + tid, key = p / (D / 4), e = p % (D / 4) * 4;
+      *reinterpret_cast<f32x4*>(&lds_k[key * KS + e]) = e < a.d ? kbuf[i] : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * VB; ++i) {
+      const int p = i * 256 + tid, key = p / (DV / 4), e = p % (DV / 4) * 4;
+      const f32x4 x = vbuf[i];
+      const float zero = (x[0] * 0.f + x[1] * 0.f) + (x[2] * 0.f + x[3] * 0.f);
+      odd |= !(zero == 0.f);
+      *reinterpret_cast<f32x4*>(&lds_v[key * VS + e]) = e < a.dv ? x : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    odd = __any(odd);
+    if (lane == 0) s_odd[wave] = odd;
+    __syncthreads();
+    if (k0 + kF32Keys <= last) fetch(k0 + kF32Keys);
+    if (k0 > wave_hi || k0 + kF32Keys - 1 <= wave_lo - a.window) continue;
+    const bool all = k0 + kF32Keys - 1 <= wave_lo && k0 > wave_hi - a.window;  // does every row see every key?
+    const bool kt_in[2] = {k0 + 15 > wave_lo - a.window, k0 + 16 <= wave_hi};  // does any see one of these 16?
+    f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+      if (kt_in[kt]) {
+        f32x4 half = {0.f, 0.f, 0.f, 0.f};  // (two sums of half the channels each round less than one)
+#pragma unroll
+        for (int c = 0; c < 4 * KB; c += 2) {
+          const f32x4 k0f = *reinterpret_cast<const f32x4*>(&lds_k[(kt * 16 + l16) * KS + c * 16 + quad * 4]);
+          const f32x4 k1f = *reinterpret_cast<const f32x4*>(&lds_k[(kt * 16 + l16) * KS + (c + 1) * 16 + quad * 4]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            s[kt] = mfma_f32(k0f[j], qf[c][j], s[kt]);
+            half = mfma_f32(k1f[j], qf[c + 1][j], half);
+          }
+        }
+        s[kt] += half;
+      }
+    const int d0 = pos - k0 - quad * 4;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float sc = s[kt][i];
+        if (!all) sc = (unsigned)(d0 - kt * 16 - i) < (unsigned)a.window ? sc : -INFINITY;
+        s[kt][i] = sc;
+        mx = fmaxf(mx, sc);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (__any(mx > m_run)) {
+      const float m_new = fmaxf(m_run, mx);
+      // no key seen yet: every weight is 2^-inf = 0
+      const float alpha = __builtin_amdgcn_exp2f((m_run - (m_new == -INFINITY ? 0.f : m_new)) * scale2);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int vb = 0; vb < VB; ++vb)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[vb][c] *= alpha;
+    }
+    const float m2 = m_run == -INFINITY ? 0.f : m_run;
+    float sum = 0.f;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[kt][i] = __builtin_amdgcn_exp2f((s[kt][i] - m2) * scale2);
+        sum += s[kt][i];
+      }
+    l_run += sum;  // this lane's keys; the four quads are added at the end
+    if (all || !(s_odd[0] | s_odd[1] | s_odd[2] | s_odd[3])) {
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+        if (kt_in[kt]) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int vb = 0; vb < VB; ++vb) {
+              const f32x4 vf = *reinterpret_cast<const f32x4*>(&lds_v[(kt * 16 + quad * 4 + j) * VS + vb * 64 + l16 * 4]);
+#pragma unroll
+              for (int c = 0; c < 4; ++c) acc[vb][c] = mfma_f32(vf[c], s[kt][j], acc[vb][c]);
+            }
+        }
+    } else {
+      // a weight of zero would not keep an infinity or NaN out of the rows that do not see its key
+      for (int key = 0; key < kF32Keys; ++key) {
+        float mine = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) mine = (key >> 4) * 4 + (key & 3) == e ? s[e / 4][e % 4] : mine;
+        const float p = __shfl(mine, (key >> 2 & 3) * 16 + l16);
+        if ((unsigned)(pos - k0 - key) < (unsigned)a.window) {
+#pragma unroll
+          for (int vb = 0; vb < VB; ++vb)
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                acc[vb][c][i] = __builtin_fmaf(p, lds_v[key * VS + vb * 64 + (quad * 4 + i) * 4 + c], acc[vb][c][i]);
+        }
+      }
+    }
+  }
+  float l = l_run;
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  const float inv = a.out_scale / l;
+  if (row_w + l16 < n_rows) {
+    float* o = static_cast<float*>(a.o) + b * a.o_sb + tok * a.o_sl + (long)head * a.dv;
+#pragma unroll
+    for (int vb = 0; vb < VB; ++vb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int e = vb * 64 + (quad * 4 + i) * 4;
+        if (e < a.dv) *reinterpret_cast<f32x4*>(o + e) = f32x4{acc[vb][0][i], acc[vb][1][i], acc[vb][2][i], acc[vb][3][i]} * inv;
+      }
   }
 }
 
@@ -1031,6 +1241,13 @@ static bool window_vec(const WindowArgs& a, int n) {
          aligned_to(a.q, 16) && aligned_to(a.k, 16) && aligned_to(a.v, 16) && aligned_to(a.kv, 16) && aligned_to(a.o, 16);
 }
 
+// fp32 rows in 16-byte pieces that are turned whole.
+static bool window_f32(const WindowArgs& a, int io_dtype) {
+  return io_dtype == BASED_F32 && a.d <= 128 && a.dv <= 128 && a.rot % (a.half_split ? 8 : 4) == 0 && a.d % 4 == 0 && a.dv % 4 == 0 &&
+         a.q_sb % 4 == 0 && a.q_sl % 4 == 0 && a.o_sb % 4 == 0 && a.o_sl % 4 == 0 && a.kv_sb % 4 == 0 && a.kv_st % 4 == 0 &&
+         aligned_to(a.q, 16) && aligned_to(a.kv, 16) && aligned_to(a.o, 16);
+}
+
 // The attention of a portion whose keys and values are in place.
 static void launch_window_attend(const WindowArgs& a, bool vec, int io_dtype, hipStream_t s) {
   if (vec) {
@@ -1046,6 +1263,16 @@ static void launch_window_attend(const WindowArgs& a, bool vec, int io_dtype, hi
       launch_window_mfma<4>(a, grid, s);
     else
       launch_window_mfma<8>(a, grid, s);
+  } else if (window_f32(a, io_dtype)) {
+    const dim3 grid((unsigned)(((long)a.L * (a.H / a.G) + kF32Rows - 1) / kF32Rows), (unsigned)(a.B * a.G));
+    if (a.d <= 64 && a.dv <= 64)
+      hipLaunchKernelGGL((window_prefill_f32_kernel<1, 1>), grid, dim3(256), 0, s, a);
+    else if (a.d <= 64)
+      hipLaunchKernelGGL((window_prefill_f32_kernel<1, 2>), grid, dim3(256), 0, s, a);
+    else if (a.dv <= 64)
+      hipLaunchKernelGGL((window_prefill_f32_kernel<2, 1>), grid, dim3(256), 0, s, a);
+    else
+      hipLaunchKernelGGL((window_prefill_f32_kernel<2, 2>), grid, dim3(256), 0, s, a);
   } else {
     const dim3 grid((unsigned)a.L, (unsigned)a.H, (unsigned)a.B);
     if (io_dtype == BASED_BF16)

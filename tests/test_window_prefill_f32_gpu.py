@@ -1,0 +1,67 @@
+"""Window attention over fp32 prompts: the matrix form and, for rows off a 16-byte address, the general one, both against 64 bits."""
+import pytest
+import torch
+
+from oracle import sozilix_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(dev, q, k, v, window, scale, start, rope, shift):
+    """The portion from `start` on, the rows before it already in the cache; rows of q and the output `shift` elements off."""
+    from based_amd import ops
+
+    B, L, H, d = q.shape
+    G, dv = v.shape[2:]
+    cache = torch.full((B, L, G, d + dv), float("nan"), device=dev)
+
+    def placed(t, rows):
+        return torch.empty(B, rows, t + shift, device=dev)[..., shift:]
+
+    kw = dict(rope=rope, out_scale=0.5)
+    qd, kd, vd = (t.to(dev).flatten(2) for t in (q, k, v))
+    if start:
+        ops.window_attn_prefill(qd[:, :start], kd[:, :start], vd[:, :start], cache, H, G, window, scale, 0,
+                                out=torch.empty(B, start, H * dv, device=dev), **kw)
+    qs, out = placed(H * d, L - start).copy_(qd[:, start:]), placed(H * dv, L - start)
+    ops.window_attn_prefill(qs, kd[:, start:], vd[:, start:], cache, H, G, window, scale, start, out=out, **kw)
+    return 2 * out.double().cpu().view(B, L - start, H, dv)
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("H,G,d,dv,L,start,window,rot,half,scale", [
+    (4, 1, 64, 64, 1, 0, 1, 0, False, 0.2), (16, 4, 64, 64, 131, 0, 33, 32, False, 0.125), (3, 1, 60, 36, 97, 31, 16, 4, False, 0.2),
+    (6, 2, 68, 64, 65, 0, 100, 8, True, -0.1), (2, 2, 4, 128, 200, 7, 31, 0, False, 0.5), (5, 1, 128, 100, 160, 96, 64, 128, True, 0.1),
+    (1, 1, 32, 4, 300, 290, 500, 24, True, 0.0)])
+def test_window_prefill_f32(dev, H, G, d, dv, L, start, window, rot, half, scale, shift):
+    from based_amd.mixers.window_attention import _ExactRotary
+
+    B = 2
+    g = torch.Generator().manual_seed(H * L + window)
+    q, k, v = (torch.randn(B, L, n, m, generator=g) for n, m in ((H, d), (G, d), (G, dv)))
+    rope = _ExactRotary(rot, base=100.0, interleaved=not half).tables(L, dev) if rot else None
+    out = _run(dev, q, k, v, window, scale, start, rope, shift)
+    qq, kk = q.double(), k.double()
+    if rot:
+        perm = torch.arange(d)
+        if half:
+            perm[:rot] = torch.tensor([c // 2 + (c % 2) * (rot // 2) for c in range(rot)])
+        qq, kk = (torch.stack([O.rotate(x[b][..., perm], 100.0, rot) for b in range(B)]) for x in (qq, kk))
+    ref = torch.stack([O.window_softmax(qq[b], kk[b], v[b].double(), scale, window) for b in range(B)])[:, start:]
+    err = (out - ref).norm(dim=-1) / ref.norm(dim=-1)
+    # scores of up to 20 and sums of 128 products: 20 * 2^-24 on every weight, and as much again from the rotation
+    assert float(err.max()) < 3e-6, float(err.max())
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_rows_that_do_not_see_a_key_do_not_take_its_value(dev, bad):
+    B, L, H, G, d, window, at = 1, 150, 4, 2, 64, 40, 70
+    g = torch.Generator().manual_seed(9)
+    q, k, v = (torch.randn(B, L, n, d, generator=g) for n in (H, G, G))
+    clean = _run(dev, q, k, v, window, 0.1, 0, None, 0)
+    k[:, at, 0], v[:, at, 0, 5] = bad, bad
+    out = _run(dev, q, k, v, window, 0.1, 0, None, 0)
+    sees = torch.zeros(L, dtype=torch.bool)
+    sees[at:at + window] = True
+    assert not out[:, sees][:, :, :2].isfinite().all(-1).any()
+    assert torch.allclose(out[:, ~sees], clean[:, ~sees], rtol=1e-5, atol=1e-6) and torch.equal(out[:, :, 2:], clean[:, :, 2:])
