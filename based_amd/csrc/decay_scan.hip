@@ -12,7 +12,7 @@
 //                     per wavefront.  Long sequences are cut into segments: a first pass leaves what every
 //                     segment adds to the state, `decay_join` turns that into the state at every segment's
 //                     start, and the second pass starts there.
-//   decay_scan_any    any element type and size: a thread holds some key channels of one value channel.
+//   decay_scan_any    any element type and size, in segments too: a thread holds some key channels of one value channel.
 //   decay_step        one token per sequence; for channel decays with the low-rank decay in front and the
 //                     head norm and gate behind.
 //   group_norm_gate   o / rms(o) * w * act(g) over groups of a row.
@@ -568,37 +568,54 @@ __global__ __launch_bounds__(256) void decay_join_kernel(const DecayScanArgs a) 
 }
 
 // ---- any element type and size ----
-// 16 lanes per value channel, channels l16 + 16 i of the key; 16 value channels per workgroup.
-template <typename T, int CPT, bool CHANNEL>
+// 16 lanes per value channel, groups of four channels of the key each; 16 value channels per workgroup.  Token by token, so what counts is
+// the length of the chain and the workgroups beside each other: long portions go in segments, as on MFMA.  fp32, B = 1, H = 16,
+// d = dv = 64, channel decays, L = 777: 47 us (one chain, four channels 16 apart to a lane: 230); L = 2048: 86 (715).
+template <typename T, int CPT, bool CHANNEL, bool STATE_ONLY>
 __global__ __launch_bounds__(256) void decay_scan_any_kernel(const DecayScanArgs a) {
-  constexpr int kTile = 8;  // tokens staged at once
+  constexpr int kTile = 16;  // tokens staged at once
   constexpr int CH = 16 * CPT;
-  __shared__ float sq[kTile][CH], sk[kTile][CH], sw[CHANNEL ? kTile : 1][CH], sv[kTile][16];
+  __shared__ __attribute__((aligned(16))) float sq[STATE_ONLY ? 1 : kTile][CH], sk[kTile][CH], sw[CHANNEL ? kTile : 1][CH];
+  __shared__ float sv[kTile][16];
   const int tid = threadIdx.x, l16 = tid & 15, col = tid >> 4;
-  const int b = blockIdx.x / a.H, h = blockIdx.x % a.H, dv0 = blockIdx.y * 16;
+  const int b = blockIdx.x / a.H, h = blockIdx.x % a.H, dv0 = blockIdx.y * 16, sg = blockIdx.z;
   const bool col_in = dv0 + col < a.dv;
   const T* qp = static_cast<const T*>(a.q) + b * a.q_sb + (long)h * a.d;
   const T* kp = static_cast<const T*>(a.k) + b * a.k_sb + (long)h * a.d;
   const T* vp = static_cast<const T*>(a.v) + b * a.v_sb + (long)h * a.dv;
-  float* st = a.state + (((long)b * a.H + h) * a.dv + (col_in ? dv0 + col : 0)) * a.dp;
-  float S[CPT], u[CPT];
+  const long bh = (long)b * a.H + h, row = col_in ? dv0 + col : 0;
+  float* st = a.state + (bh * a.dv + row) * a.dp;
+  float* sgp = a.segs > 1 ? a.seg + ((bh * a.segs + sg) * a.dv + row) * a.dp : nullptr;
+  const float* from = a.segs > 1 ? sgp : st;
+  const bool zero = STATE_ONLY || (a.segs == 1 && a.fresh);
+  f32x4 S[CPT / 4], u[CPT / 4];
+  float log2_all = 0.f;  // (state pass) what this thread stages of the decay over the segment: always of channel tid % CH
+  static_assert(256 % CH == 0, "a thread stages one channel");
   const float head_w = CHANNEL ? 0.f : a.head_lw[a.H + h];
 #pragma unroll
-  for (int i = 0; i < CPT; ++i) {
-    const int c = l16 + 16 * i;
-    S[i] = !a.fresh && col_in && c < a.d ? st[c] : 0.f;
-    u[i] = CHANNEL && c < a.d ? to_f32(static_cast<const T*>(a.u)[(long)h * a.d + c]) : 0.f;
-  }
+  for (int g = 0; g < CPT / 4; ++g)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = g * 64 + l16 * 4 + j;
+      S[g][j] = !zero && col_in && c < a.d ? from[c] : 0.f;
+      u[g][j] = CHANNEL && !STATE_ONLY && c < a.d ? to_f32(static_cast<const T*>(a.u)[(long)h * a.d + c]) : 0.f;
+    }
   auto active = [&](T x) { return a.silu ? round_to<T>(silu_exact(to_f32(x))) : to_f32(x); };
-  for (int t0 = 0; t0 < a.L; t0 += kTile) {
-    const int n = a.L - t0 < kTile ? a.L - t0 : kTile;
+  const int begin = sg * a.seg_chunks * kScanTokens;
+  const int end = sg < a.segs - 1 ? begin + a.seg_chunks * kScanTokens : a.L;
+  for (int t0 = begin; t0 < end; t0 += kTile) {
+    const int n = end - t0 < kTile ? end - t0 : kTile;
     __syncthreads();
     for (int i = tid; i < kTile * CH; i += 256) {
       const int t = i / CH, c = i % CH;
       const bool in = t < n && c < a.d;
-      sq[t][c] = in ? active(qp[(t0 + t) * a.q_sl + c]) : 0.f;
+      if constexpr (!STATE_ONLY) sq[t][c] = in ? active(qp[(t0 + t) * a.q_sl + c]) : 0.f;
       sk[t][c] = in ? active(kp[(t0 + t) * a.k_sl + c]) : 0.f;
-      if constexpr (CHANNEL) sw[t][c] = in ? exp2f(a.lw[(((long)b * a.L + t0 + t) * a.H + h) * a.d + c]) : 1.f;
+      if constexpr (CHANNEL) {
+        const float lw = in ? a.lw[(((long)b * a.L + t0 + t) * a.H + h) * a.d + c] : 0.f;
+        sw[t][c] = exp2f(lw);
+        if constexpr (STATE_ONLY) log2_all += lw;
+      }
     }
     for (int i = tid; i < kTile * 16; i += 256) {
       const int t = i / 16, c = i % 16;
@@ -609,25 +626,52 @@ __global__ __launch_bounds__(256) void decay_scan_any_kernel(const DecayScanArgs
       const float v = sv[t][col];
       float o = 0.f;
 #pragma unroll
-      for (int i = 0; i < CPT; ++i) {
-        const int c = l16 + 16 * i;
-        const float kv = sk[t][c] * v;
-        if constexpr (CHANNEL) {
-          o = __builtin_fmaf(__builtin_fmaf(u[i], kv, S[i]), sq[t][c], o);
-          S[i] = __builtin_fmaf(sw[t][c], S[i], kv);
-        } else {
-          S[i] = __builtin_fmaf(head_w, S[i], kv);
-          o = __builtin_fmaf(S[i], sq[t][c], o);
+      for (int g = 0; g < CPT / 4; ++g) {
+        const int c = g * 64 + l16 * 4;
+        const f32x4 k = *reinterpret_cast<const f32x4*>(&sk[t][c]);
+        f32x4 q, w;
+        if constexpr (!STATE_ONLY) q = *reinterpret_cast<const f32x4*>(&sq[t][c]);
+        if constexpr (CHANNEL) w = *reinterpret_cast<const f32x4*>(&sw[t][c]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float kv = k[j] * v;
+          if constexpr (CHANNEL) {
+            if constexpr (!STATE_ONLY) o = __builtin_fmaf(__builtin_fmaf(u[g][j], kv, S[g][j]), q[j], o);
+            S[g][j] = __builtin_fmaf(w[j], S[g][j], kv);
+          } else {
+            S[g][j] = __builtin_fmaf(head_w, S[g][j], kv);
+            if constexpr (!STATE_ONLY) o = __builtin_fmaf(S[g][j], q[j], o);
+          }
         }
       }
-      o = sum16(o);
-      if (l16 == 0 && col_in) static_cast<T*>(a.o)[b * a.o_sb + (t0 + t) * a.o_sl + (long)h * a.dv + dv0 + col] = from_f32<T>(o);
+      if constexpr (!STATE_ONLY) {
+        o = sum16(o);
+        if (l16 == 0 && col_in) static_cast<T*>(a.o)[b * a.o_sb + (t0 + t) * a.o_sl + (long)h * a.dv + dv0 + col] = from_f32<T>(o);
+      }
     }
   }
 #pragma unroll
-  for (int i = 0; i < CPT; ++i) {
-    const int c = l16 + 16 * i;
-    if (col_in && c < a.d) st[c] = S[i];
+  for (int g = 0; g < CPT / 4; ++g)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = g * 64 + l16 * 4 + j;
+      if (c >= a.d) continue;
+      if constexpr (STATE_ONLY) {
+        if (col_in) sgp[c] = S[g][j];
+      } else if (col_in && sg == a.segs - 1) {
+        st[c] = S[g][j];
+      }
+    }
+  if constexpr (CHANNEL && STATE_ONLY) {
+    // the power of a sum of logarithms loses less than a product of decays that were each rounded
+    if (blockIdx.y != 0) return;
+    __syncthreads();
+    float* sum = &sk[0][0];
+    sum[tid] = log2_all;
+    __syncthreads();
+    if (tid >= CH || tid >= a.d) return;
+    for (int i = tid + CH; i < 256; i += CH) log2_all += sum[i];
+    a.seg_lw[(bh * a.segs + sg) * a.dp + tid] = exp2f(log2_all);
   }
 }
 
@@ -850,6 +894,11 @@ template <typename T, bool VEC> void launch_group_norm(const GroupNormArgs& a, h
     hipLaunchKernelGGL((group_norm_gate_kernel<T, VEC, 64>), grid, block, 0, s, a);
 }
 
+void launch_decay_join(const DecayScanArgs& a, hipStream_t s) {
+  const long items = (long)a.B * a.H * a.dv * (a.dp / 4);
+  hipLaunchKernelGGL(decay_join_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, a);
+}
+
 template <int DT, int HALVES, bool CHANNEL> int launch_decay_mfma(const DecayScanArgs& a, hipStream_t s) {
   const size_t bytes = sizeof(ScanLds<DT, HALVES, CHANNEL>);
   if (bytes > 64 * 1024) {
@@ -868,8 +917,7 @@ template <int DT, int HALVES, bool CHANNEL> int launch_decay_mfma(const DecaySca
     dim3 all_but_last = grid;
     all_but_last.z -= 1;
     hipLaunchKernelGGL((decay_scan_mfma_kernel<DT, HALVES, CHANNEL, true>), all_but_last, dim3(256 * HALVES), bytes, s, a);
-    const long items = (long)a.B * a.H * a.dv * (a.dp / 4);
-    hipLaunchKernelGGL(decay_join_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, a);
+    launch_decay_join(a, s);
   }
   hipLaunchKernelGGL((decay_scan_mfma_kernel<DT, HALVES, CHANNEL, false>), grid, dim3(256 * HALVES), bytes, s, a);
   return BASED_OK;
@@ -881,15 +929,22 @@ template <bool CHANNEL> int launch_decay_scan_mfma(const DecayScanArgs& a, hipSt
   return launch_decay_mfma<2, 2, CHANNEL>(a, s);
 }
 
+template <typename T, int CPT, bool CHANNEL> void launch_decay_any(const DecayScanArgs& a, hipStream_t s) {
+  const unsigned cols = (unsigned)((a.dv + 15) / 16);
+  if (a.segs > 1) {
+    hipLaunchKernelGGL((decay_scan_any_kernel<T, CPT, CHANNEL, true>), dim3((unsigned)(a.B * a.H), cols, (unsigned)(a.segs - 1)), dim3(256), 0, s, a);
+    launch_decay_join(a, s);
+  }
+  hipLaunchKernelGGL((decay_scan_any_kernel<T, CPT, CHANNEL, false>), dim3((unsigned)(a.B * a.H), cols, (unsigned)a.segs), dim3(256), 0, s, a);
+}
+
 template <typename T, bool CHANNEL> void launch_decay_scan_any(const DecayScanArgs& a, hipStream_t s) {
-  const dim3 grid((unsigned)(a.B * a.H), (unsigned)((a.dv + 15) / 16));
-  const int cpt = (a.d + 15) / 16;
-  if (cpt <= 4)
-    hipLaunchKernelGGL((decay_scan_any_kernel<T, 4, CHANNEL>), grid, dim3(256), 0, s, a);
-  else if (cpt <= 8)
-    hipLaunchKernelGGL((decay_scan_any_kernel<T, 8, CHANNEL>), grid, dim3(256), 0, s, a);
+  if (a.d <= 64)
+    launch_decay_any<T, 4, CHANNEL>(a, s);
+  else if (a.d <= 128)
+    launch_decay_any<T, 8, CHANNEL>(a, s);
   else
-    hipLaunchKernelGGL((decay_scan_any_kernel<T, 16, CHANNEL>), grid, dim3(256), 0, s, a);
+    launch_decay_any<T, 16, CHANNEL>(a, s);
 }
 
 template <typename T, int NT, int LPR, int RPT, bool CHANNEL> void launch_decay_step_block(const DecayStepArgs& a, hipStream_t s) {
@@ -933,11 +988,21 @@ static int decay_segments(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV
   return segs < 2 ? 1 : (int)segs;
 }
 
+// The same for the general form: eight workgroups to a compute unit.  Every token but those of the last segment is walked twice, so three
+// segments would gain a third at best, less the launches: from four on (B = 1, H = 12, L = 250: 37 us in four, 77 in one).
+static int decay_any_segments(int64_t B, int64_t L, int64_t H, int64_t DV) {
+  const int64_t chunks = (L + kScanTokens - 1) / kScanTokens, wgs = B * H * ((DV + 15) / 16);
+  int64_t segs = (2048 + wgs - 1) / wgs;
+  if (segs > chunks) segs = chunks;
+  if (segs > 64) segs = 64;
+  return segs < 4 ? 1 : (int)segs;
+}
+
 }  // namespace based
 
 extern "C" BASED_API int64_t based_decay_scan_work(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, int64_t state_row) {
   if (B <= 0 || L <= 0 || H <= 0 || D <= 0 || DV <= 0) return 0;
-  const int64_t segs = based::decay_segments(B, L, H, D, DV);
+  const int64_t mfma = based::decay_segments(B, L, H, D, DV), any = based::decay_any_segments(B, L, H, DV), segs = mfma > any ? mfma : any;
   return segs <= 1 ? 0 : B * H * segs * (DV + 1) * state_row;
 }
 
@@ -966,15 +1031,15 @@ extern "C" BASED_API int based_decay_scan(const void* q, const void* k, const vo
   const bool vec = io_dtype == BASED_BF16 && D <= 128 && D % 4 == 0 && DV % 4 == 0 && q_sb % 4 == 0 && q_sl % 4 == 0 && k_sb % 4 == 0 &&
                    k_sl % 4 == 0 && v_sb % 4 == 0 && v_sl % 4 == 0 && o_sb % 4 == 0 && o_sl % 4 == 0 && aligned_to(q, 8) &&
                    aligned_to(k, 8) && aligned_to(v, 8) && aligned_to(o, 8) && aligned_to(bonus, 8) && aligned_to(channel_log2, 16);
+  const int segs = vec ? decay_segments(B, L, H, D, DV) : work != nullptr ? decay_any_segments(B, L, H, DV) : 1;
+  if (segs > 1) {
+    BASED_REQUIRE(work != nullptr, BASED_ERR_ARG, "decay_scan: no work space");
+    a.seg_chunks = (a.seg_chunks + segs - 1) / segs;
+    a.segs = (int)(((L + kScanTokens - 1) / kScanTokens + a.seg_chunks - 1) / a.seg_chunks);
+    a.seg = work;
+    a.seg_lw = work + B * H * a.segs * DV * state_row;
+  }
   if (vec) {
-    const int segs = decay_segments(B, L, H, D, DV);
-    if (segs > 1) {
-      BASED_REQUIRE(work != nullptr, BASED_ERR_ARG, "decay_scan: no work space");
-      a.seg_chunks = (a.seg_chunks + segs - 1) / segs;
-      a.segs = (int)(((L + kScanTokens - 1) / kScanTokens + a.seg_chunks - 1) / a.seg_chunks);
-      a.seg = work;
-      a.seg_lw = work + B * H * a.segs * DV * state_row;
-    }
     const int rc = channel_log2 != nullptr ? launch_decay_scan_mfma<true>(a, s) : launch_decay_scan_mfma<false>(a, s);
     if (rc != BASED_OK) return rc;
   } else if (io_dtype == BASED_BF16) {

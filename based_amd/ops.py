@@ -1189,10 +1189,8 @@ def decay_scan(q, k, v, state, heads: int, *, channel_log2=None, bonus=None, hea
     else:
         _check_head_decay(head_decay, heads, q.device)
     lib = _lib.lib()
-    work = None
-    if q.dtype == torch.bfloat16:
-        n = lib.based_decay_scan_work(B, L, heads, d, dv, state.shape[3])
-        work = torch.empty(n, dtype=torch.float32, device=q.device) if n else None
+    n = lib.based_decay_scan_work(B, L, heads, d, dv, state.shape[3])
+    work = torch.empty(n, dtype=torch.float32, device=q.device) if n else None
     o = torch.empty(B, L, heads * dv, dtype=q.dtype, device=q.device)
     with _on_device(q.device):
         _lib.check(lib.based_decay_scan(

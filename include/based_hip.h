@@ -629,7 +629,7 @@ BASED_API int based_token_side_step(const void* x, const float* residual_in, flo
  * bonus u (H, D): o_t = (S + diag(u) k v^T)^T q, S <- diag(w) S + k v^T.  Or head_decay (2, H), the log2 of constants w
  * and w itself:
  * S <- w S + k v^T, o = S^T q.  state (B, H, DV, state_row) fp32, by value channel; work: as many floats as
- * based_decay_scan_work says (bf16 only). */
+ * based_decay_scan_work says; without it, what is not bf16 in whole 8-byte pieces is walked in one chain. */
 BASED_API int64_t based_decay_scan_work(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, int64_t state_row);
 BASED_API int based_decay_scan(const void* q, const void* k, const void* v, const float* channel_log2, const float* head_decay,
                                const void* bonus, float* state, float* work, void* o, int64_t B, int64_t L, int64_t H,

@@ -1,0 +1,47 @@
+"""Decaying states over long portions that the matrix form does not take (fp32, odd sizes): cut into segments or in one chain."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("channel", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,L,H,d,dv,start", [(1, 255, 1, 64, 16, 0), (1, 256, 2, 20, 17, 0), (2, 257, 1, 33, 64, 5), (1, 1031, 1, 130, 9, 40),
+                                              (1, 400, 3, 68, 31, 63)])
+def test_decay_scan_segments(dev, B, L, H, d, dv, start, dtype, channel):
+    from based_amd import ops
+
+    g = torch.Generator().manual_seed(L * 7 + d)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype)  # noqa: E731
+    q, k, v, u = rnd(B, L, H, d), rnd(B, L, H, d), rnd(B, L, H, dv), rnd(H, d)
+    lw = -torch.exp(0.5 * torch.randn(B, L, H, d, generator=g) + torch.linspace(-7, 1, d)) / math.log(2)
+    decay = [0.999, 0.0, 0.9][:H]
+    kw = dict(head_decay=ops.head_decays(decay, dev)) if not channel else dict(bonus=u.to(dev))
+    qd, kd, vd = (torch.empty(B, L, t.shape[2] * t.shape[3] + 1, dtype=dtype, device=dev)[..., 1:].copy_(t.flatten(2)) for t in (q, k, v))
+    state = torch.full((B, H, dv, (d + 3) // 4 * 4), float("nan"), device=dev)
+    out = []
+    for s in ([slice(0, start), slice(start, L)] if start else [slice(0, L)]):
+        if channel:
+            kw["channel_log2"] = lw[:, s].flatten(2).contiguous().to(dev)
+        out.append(ops.decay_scan(qd[:, s], kd[:, s], vd[:, s], state, H, fresh=s.start == 0, **kw))
+    out = torch.cat(out, 1).double().cpu().view(B, L, H, dv)
+    S, ref = torch.zeros(B, H, d, dv, dtype=torch.float64), []
+    for t in range(L):
+        qt, kt, vt = (x[:, t].double() for x in (q, k, v))
+        kv = kt[..., None] * vt[:, :, None]
+        if channel:
+            ref.append(((S + u.double()[..., None] * kv) * qt[..., None]).sum(2))
+            S = 2.0 ** lw[:, t].double()[..., None] * S + kv
+        else:
+            S = torch.tensor(decay, dtype=torch.float32).double().view(1, H, 1, 1) * S + kv  # (decays as fp32 holds them)
+            ref.append((S * qt[..., None]).sum(2))
+    ref = torch.stack(ref, 1)
+    rel = lambda a, b: ((a - b).norm() / b.norm()).item()  # noqa: E731
+    # The slowest decays keep a thousand tokens.  Each rounds the decay and the sum by up to 2^-24, independently: 2 * 2^-24 * 1000^0.5 =
+    # 3.8e-6; bf16 outputs add half of 2^-8.
+    tol = 4e-6 if dtype == torch.float32 else 3e-3
+    assert rel(out, ref) < tol and rel(out[:, -8:], ref[:, -8:]) < tol, (rel(out, ref), rel(out[:, -8:], ref[:, -8:]))
+    assert rel(state[..., :d].double().cpu(), S.transpose(2, 3)) < 4e-6
