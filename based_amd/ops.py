@@ -1308,14 +1308,15 @@ def latent_step(q, x, norm_weight, weight, cache, heads: int, dim: int, window: 
         raise ValueError(f"bad shapes q{tuple(q.shape)} weight{tuple(weight.shape)} out{tuple(out.shape)}")
     groups = B * ((heads + 15) // 16)
     splits = max(1, min(LATENT_STEP_TARGET // groups, (min(window, S) + 63) // 64, LATENT_STEP_MAX_SPLITS))
-    f32 = dict(dtype=torch.float32, device=x.device)
-    work_q = torch.empty(B, heads, R + rot, **f32)
-    part, part_ml = torch.empty(B, splits, heads, R, **f32), torch.empty(B, splits, heads, 2, **f32)
+    # queries (B, heads, R + rot), sums (B, splits, heads, R) and their maxima and weights (.., 2) in one allocation, 16-byte pieces each
+    n_q, n_part = (B * heads * (R + rot) + 3) // 4 * 4, (B * splits * heads * R + 3) // 4 * 4
+    work = torch.empty(n_q + n_part + B * splits * heads * 2, dtype=torch.float32, device=x.device)
+    work_q = work.data_ptr()
     pos_ptr, pos_host = _pos_args(pos, B)
     with _on_device(x.device):
         _lib.check(_lib.lib().based_latent_step(
-            q.data_ptr(), x.data_ptr(), norm_weight.data_ptr(), weight.data_ptr(), cache.data_ptr(), work_q.data_ptr(), part.data_ptr(),
-            part_ml.data_ptr(), out.data_ptr(), pos_ptr, pos_host, B, heads, dim, dv, S, R, rot, splits, q.stride(0), x.stride(0),
+            q.data_ptr(), x.data_ptr(), norm_weight.data_ptr(), weight.data_ptr(), cache.data_ptr(), work_q, work_q + 4 * n_q,
+            work_q + 4 * (n_q + n_part), out.data_ptr(), pos_ptr, pos_host, B, heads, dim, dv, S, R, rot, splits, q.stride(0), x.stride(0),
             weight.stride(0), cache.stride(0), cache.stride(1), out.stride(0), int(window), float(scale), float(eps), float(out_scale),
             cos_ptr, sin_ptr, n_pos, half, _dtype_code(x), _stream_ptr(x)))
     return out
