@@ -404,7 +404,7 @@ __global__ __launch_bounds__(256, KC <= 3 && VC <= 2 ? 3 : 1) void window_prefil
 // weights of a lane are what the products with the values take, one each, where product j contracts keys j, 4 + j, 8 + j and 12 + j;
 // keys and queries give up their channels in the same order, so that a lane reads 16 bytes for four products.
 // Bound by the fp32 matrix rate from some thousand rows on and by the chain of one wavefront below.  16 heads on 4, size 64, 129 keys:
-// B = 1, L = 777, with the cache write: 19 us (a wavefront per query on the vector unit: 70); B = 4, L = 2048: 89 us (661).
+// B = 1, L = 777, with the cache write: 19 us (a wavefront per query on the vector unit: 70); B = 4, L = 2048: 81 us (661).
 constexpr int kF32Keys = 32, kF32Rows = 64;
 
 __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
@@ -432,6 +432,36 @@ __device__ __forceinline__ f32x4 turned4(const float* row, int c, int pos, const
     }
   }
   return x;
+}
+
+// The cache write of fp32 rows in 16-byte pieces: 16 lanes per (token, key/value head).  Element by element, a wavefront per head, it was
+// 19.3 us with the attention at B = 1, L = 777, 4 heads of 64, and 88 at B = 4, L = 2048: 18.9 and 81.
+__global__ __launch_bounds__(256) void window_kv_write_f32_kernel(const WindowArgs a) {
+  const long n_items = (long)a.B * a.L * a.G, item0 = (long)blockIdx.x * 16 + (threadIdx.x >> 4);
+  const bool live = item0 < n_items;
+  const long item = live ? item0 : n_items - 1, bl = item / a.G;
+  const int c0 = (threadIdx.x & 15) * 4, g = (int)(item % a.G), l = (int)(bl % a.L), b = (int)(bl / a.L), pos = a.pos_host + l;
+  const float* k = static_cast<const float*>(a.k) + b * a.k_sb + l * a.k_sl + (long)g * a.d;
+  const float* v = static_cast<const float*>(a.v) + b * a.v_sb + l * a.v_sl + (long)g * a.dv;
+  float* out = static_cast<float*>(a.kv) + b * a.kv_sb + pos * a.kv_st + (long)g * (a.d + a.dv);
+  f32x4 x[2], y[2];  // (sizes up to 128)
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = c0 + i * 64;
+    x[i] = turned4(k, c < a.d ? c : 0, pos, a);
+    y[i] = *reinterpret_cast<const f32x4*>(v + (c < a.dv ? c : 0));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) ss = c < a.dv ? __builtin_fmaf(y[i][j], y[i][j], ss) : ss;
+  }
+  const float r = a.norm_v ? 1.0f / sqrtf(sum16(ss) / (float)a.dv + a.eps) : 1.0f;
+  if (!live) return;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = c0 + i * 64;
+    if (c < a.d) *reinterpret_cast<f32x4*>(out + c) = x[i];
+    if (c < a.dv) *reinterpret_cast<f32x4*>(out + a.d + c) = y[i] * r;
+  }
 }
 
 template <int KB, int VB>
@@ -1310,6 +1340,8 @@ extern "C" BASED_API int based_window_attn_prefill(
     widest <= 64 ? launch_kv_write<8>(a, s) : widest <= 128 ? launch_kv_write<16>(a, s) : launch_kv_write<32>(a, s);
   } else if (io_dtype == BASED_BF16)
     hipLaunchKernelGGL(window_kv_write_kernel<__bf16>, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s, a);
+  else if (window_f32(a, io_dtype) && k_sb % 4 == 0 && k_sl % 4 == 0 && v_sb % 4 == 0 && v_sl % 4 == 0 && aligned_to(k, 16) && aligned_to(v, 16))
+    hipLaunchKernelGGL(window_kv_write_f32_kernel, dim3((unsigned)((items + 15) / 16)), dim3(256), 0, s, a);
   else
     hipLaunchKernelGGL(window_kv_write_kernel<float>, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s, a);
   launch_window_attend(a, vec, io_dtype, s);

@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _run(dev, q, k, v, window, scale, start, rope, shift):
-    """The portion from `start` on, the rows before it already in the cache; rows of q and the output `shift` elements off."""
+    """The portion from `start` on, the rows before it already in the cache; rows of q, k, v and the output `shift` elements off."""
     from based_amd import ops
 
     B, L, H, d = q.shape
@@ -24,7 +24,8 @@ def _run(dev, q, k, v, window, scale, start, rope, shift):
         ops.window_attn_prefill(qd[:, :start], kd[:, :start], vd[:, :start], cache, H, G, window, scale, 0,
                                 out=torch.empty(B, start, H * dv, device=dev), **kw)
     qs, out = placed(H * d, L - start).copy_(qd[:, start:]), placed(H * dv, L - start)
-    ops.window_attn_prefill(qs, kd[:, start:], vd[:, start:], cache, H, G, window, scale, start, out=out, **kw)
+    ks, vs = placed(G * d, L - start).copy_(kd[:, start:]), placed(G * dv, L - start).copy_(vd[:, start:])
+    ops.window_attn_prefill(qs, ks, vs, cache, H, G, window, scale, start, out=out, **kw)
     return 2 * out.double().cpu().view(B, L - start, H, dv)
 
 
