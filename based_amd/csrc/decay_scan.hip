@@ -547,7 +547,9 @@ __global__ __launch_bounds__(256) void decay_join_kernel(const DecayScanArgs a) 
   float* st = a.state + (bh * a.dv + col) * a.dp + ch;
   f32x4 S = {0.f, 0.f, 0.f, 0.f};
   if (!a.fresh) S = *reinterpret_cast<const f32x4*>(st);
-  const float head_l2 = a.lw != nullptr ? 0.f : a.head_lw[bh % a.H];
+  // (a decay below zero has no logarithm; segments are whole 64-token pieces, an even power)
+  const float head_w = a.lw != nullptr ? 0.f : a.head_lw[a.H + bh % a.H];
+  const float head_l2 = a.lw != nullptr ? 0.f : head_w < 0.f ? log2f(-head_w) : a.head_lw[bh % a.H];
   for (int s = 0; s < a.segs; ++s) {
     float* p = a.seg + ((bh * a.segs + s) * a.dv + col) * a.dp + ch;
     f32x4 add = {0.f, 0.f, 0.f, 0.f};

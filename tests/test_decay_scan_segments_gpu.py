@@ -45,3 +45,27 @@ def test_decay_scan_segments(dev, B, L, H, d, dv, start, dtype, channel):
     tol = 4e-6 if dtype == torch.float32 else 3e-3
     assert rel(out, ref) < tol and rel(out[:, -8:], ref[:, -8:]) < tol, (rel(out, ref), rel(out[:, -8:], ref[:, -8:]))
     assert rel(state[..., :d].double().cpu(), S.transpose(2, 3)) < 4e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("L", [255, 300, 513])
+def test_head_decays_below_zero(dev, L, dtype):
+    """A decay that changes its sign from token to token has no logarithm, but powers: in segments as in one chain."""
+    from based_amd import ops
+
+    H, d, dv, decay = 3, 20, 17, [-0.9, -0.9995, -1.0]
+    g = torch.Generator().manual_seed(L)
+    q, k, v = (torch.randn(1, L, H * n, generator=g).to(dtype) for n in (d, d, dv))
+    state = torch.randn(1, H, dv, 20, generator=g)
+    S, ref = state.double().transpose(2, 3), []
+    w = torch.tensor(decay, dtype=torch.float32).double().view(1, H, 1, 1)
+    for t in range(L):
+        qt, kt, vt = (x[:, t].double().view(1, H, -1) for x in (q, k, v))
+        S = w * S + kt[..., None] * vt[:, :, None]
+        ref.append((S * qt[..., None]).sum(2).flatten(1))
+    state = state.to(dev)
+    out = ops.decay_scan(q.to(dev), k.to(dev), v.to(dev), state, H, head_decay=ops.head_decays(decay, dev), fresh=False)
+    rel = lambda a, b: ((a.double().cpu() - b).norm() / b.norm()).item()  # noqa: E731
+    # as above: up to five hundred roundings of 2^-24 that lie independently, and half of 2^-8 of bf16 outputs
+    assert rel(out, torch.stack(ref, 1)) < (4e-6 if dtype == torch.float32 else 3e-3)
+    assert rel(state, S.transpose(2, 3)) < 4e-6
