@@ -219,7 +219,8 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
   sq += __shfl_xor(sq, 32, 64), sk += __shfl_xor(sk, 32, 64);
   if (quad == 0) {
     const int t = wave * 16 + l16;
-    s_fq[t] = t < left ? 1.0f / sqrtf((float)((sq + (double)kUnitEps) * (double)a.d)) : 0.f;
+    // (times d only in 64 bits: queries of 1e19 and more have no such product in 32)
+    s_fq[t] = t < left ? (float)(1.0 / sqrt((sq + (double)kUnitEps) * (double)a.d)) : 0.f;
     s_fk[t] = t < left ? 1.0f / sqrtf((float)(sk + (double)kUnitEps)) : 0.f;
   }
   __syncthreads();

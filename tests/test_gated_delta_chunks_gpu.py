@@ -118,3 +118,16 @@ def test_rows_of_no_whole_pieces(dev):
     o, S = run((wide[..., 1:], ab, a_log, dt_bias), H, H, d, dv, state)
     ref, S_ref = reference(x, ab, a_log, dt_bias, H, H, d, dv)
     assert rel_l2(o, ref) < 3e-6 and rel_l2(S, S_ref) < 3e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("scale", [1e-12, 1e17, 1e18])
+def test_long_and_short_queries(dev, dtype, scale):
+    """Queries and keys whose squares' sum fits 32 bits and, times the head size, does not; and those that the constant beside it hides."""
+    L, H, d, dv = 257, 2, 128, 32
+    case = [t.to(dev) for t in make(8, 1, L, H, H, d, dv, dtype)]
+    case[0][..., :2 * H * d] *= scale
+    assert in_chunks(1, L, H, d, dv)
+    o, S = run(case, H, H, d, dv, empty_state(1, H, d, dv, dev))
+    ref, S_ref = reference(*case, H, H, d, dv)
+    assert rel_l2(o, ref) < TOL and rel_l2(S, S_ref) < TOL
