@@ -305,7 +305,9 @@ __global__ __launch_bounds__(256, 2) void lin_prefill_f32_kernel(const PrefillF3
               else
                 p = x[i] * 0.25f;
               z = __builtin_fmaf(p, zt[i], z);
-              o[i & 1] = mma_f32(p, S[t][i], o[i & 1]);
+              // (slots without a feature hold zero times every value, which an infinity made a NaN)
+              const float st = t == 8 ? (quad < 2 || (quad == 2 && i == 0) ? S[t][i] : 0.f) : S[t][i];
+              o[i & 1] = mma_f32(p, st, o[i & 1]);
             }
           }
         }

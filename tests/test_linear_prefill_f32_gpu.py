@@ -91,6 +91,21 @@ def test_no_numbers_stay_behind_their_token(dev, which, value, t):
         assert torch.equal(y[:, :, t + 1:], clean[:, :, t + 1:])
 
 
+@pytest.mark.parametrize("split", [None, False])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf")])
+def test_infinite_values_stay_infinite(dev, value, split):
+    """Every weight is positive: behind an infinite value its channel is that infinity, also where the sum over features has no other
+    sign (queries and keys above zero)."""
+    from based_amd import ops
+
+    q, k, v = make(13, 1, 2, 200, 20)
+    v[:, :, 5, 3] = value
+    y = ops.linear_attn_prefill(*(x.to(dev) for x in (q.abs(), k.abs(), v)), split=split)[0]
+    assert bool((y[:, :, 5:, 3] == value).all())
+    y[:, :, 5:, 3] = 0
+    assert bool(torch.isfinite(y).all())
+
+
 def test_refused_as_before(dev):
     from based_amd import ops
 
