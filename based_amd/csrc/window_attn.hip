@@ -495,6 +495,7 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(const WindowArg
   };
   fetch(lo);
   f32x4 qf[4 * KB];
+  const float sign = a.scale < 0.f ? -1.f : a.scale == 0.f ? 0.f : 1.f;
   {
     const float* q = static_cast<const float*>(a.q) + b * a.q_sb + tok * a.q_sl + (long)head * a.d;
 #pragma unroll
@@ -502,7 +503,7 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(const WindowArg
       const int e = c * 16 + quad * 4;
       qf[c] = turned4(q, e < a.d ? e : 0, pos, a);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) qf[c][j] = e < a.d ? (a.scale < 0.f ? -qf[c][j] : qf[c][j]) : 0.f;
+      for (int j = 0; j < 4; ++j) qf[c][j] = e < a.d ? sign * qf[c][j] : 0.f;
     }
   }
   f32x4 acc[VB][4];  // channels vb * 64 + (quad * 4 + i) * 4 + c of row l16 in [vb][c][i]
@@ -511,9 +512,9 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(const WindowArg
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[vb][c] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_run = 0.f;
-  // Powers of two of the differences, which are exact where they count; the sign is the queries'.  At scale 0 every difference is
-  // all but lost, while a key out of sight stays at minus infinity.
-  const float scale2 = a.scale == 0.f ? 1e-38f : fabsf(a.scale) * 1.4426950408889634f;
+  // Powers of two of the differences, which are exact where they count; the sign is the queries', and so is a scale of zero (a key
+  // out of sight stays at minus infinity, an infinite one is no number).
+  const float scale2 = a.scale == 0.f ? 1.f : fabsf(a.scale) * 1.4426950408889634f;
 
   for (int k0 = lo; k0 <= last; k0 += kF32Keys) {
     __syncthreads();  // every wavefront is done with the tile before

@@ -66,3 +66,19 @@ def test_rows_that_do_not_see_a_key_do_not_take_its_value(dev, bad):
     sees[at:at + window] = True
     assert not out[:, sees][:, :, :2].isfinite().all(-1).any()
     assert torch.allclose(out[:, ~sees], clean[:, ~sees], rtol=1e-5, atol=1e-6) and torch.equal(out[:, :, 2:], clean[:, :, 2:])
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+def test_scale_of_zero(dev, bad, shift):
+    """Zero times an infinite score is no number, whatever its sign, in every row that sees the key and in no other."""
+    B, L, H, G, d, window, at = 1, 150, 4, 2, 64, 40, 70
+    g = torch.Generator().manual_seed(10)
+    q, k, v = (torch.randn(B, L, n, d, generator=g) for n in (H, G, G))
+    k[:, at, 0, 5] = bad
+    out = _run(dev, q, k, v, window, 0.0, 0, None, shift)
+    sees = torch.zeros(L, dtype=torch.bool)
+    sees[at:at + window] = True
+    assert out[:, sees][:, :, :2].isnan().all()
+    mean = torch.stack([v[0, max(0, t - window + 1):t + 1].double().mean(0) for t in range(L)])[None].repeat_interleave(H // G, 2)
+    assert torch.allclose(out[:, ~sees], mean[:, ~sees], rtol=0, atol=1e-6) and torch.allclose(out[:, :, 2:], mean[:, :, 2:], rtol=0, atol=1e-6)
