@@ -127,6 +127,7 @@ SIGNATURES = {
     "based_gated_rms_norm": (C.c_int, [_P] * 4 + [_I64] * 8 + [C.c_float, C.c_float, C.c_int, _P]),
     "based_gated_delta_step": (
         C.c_int, [_P] * 12 + [_I64] * 8 + [C.c_int] + [_I64] * 7 + [C.c_float, C.c_float, C.c_int, _P]),
+    "based_rglru_prefill_work": (_I64, [_P, _P] + [_I64] * 7 + [C.c_int]),
     "based_rglru_prefill": (C.c_int, [_P] * 12 + [_I64] * 10 + [C.c_float, C.c_int, C.c_int, _P]),
     "based_rglru_step": (C.c_int, [_P] * 13 + [_I64] * 4 + [C.c_int] + [_I64] * 4 + [C.c_float, C.c_int, _P]),
     "based_decode_linear_stream": (

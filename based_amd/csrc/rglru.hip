@@ -287,10 +287,30 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
   }
 }
 
-// Rows from the scratch to an output that shares memory with the input.
-template <typename T> __global__ __launch_bounds__(256) void rglru_copy_kernel(const T* src, T* dst, int L, int W, long o_sb, long o_sl) {
-  for (int l = blockIdx.x * kSeg; l < L && l < ((int)blockIdx.x + 1) * kSeg; ++l)
-    for (int w = threadIdx.x; w < W; w += 256) dst[blockIdx.y * o_sb + l * o_sl + w] = src[((long)blockIdx.y * L + l) * W + w];
+// Rows from the scratch to an output that shares memory with the input, V elements at a time; 16 rows of a sequence per workgroup.
+constexpr int kCopyRows = 16;
+template <typename T, int V> __global__ __launch_bounds__(256) void rglru_copy_kernel(const T* src, T* dst, int L, int W, long o_sb, long o_sl) {
+  typedef __attribute__((ext_vector_type(V))) T vec_t;
+  const int l0 = blockIdx.x * kCopyRows, rows = L - l0 < kCopyRows ? L - l0 : kCopyRows;
+  const unsigned pieces = W / V;
+  src += ((long)blockIdx.y * L + l0) * W;
+  dst += blockIdx.y * o_sb + l0 * o_sl;
+  if constexpr (V > 1) {
+    for (unsigned p = threadIdx.x; p < rows * pieces; p += 256) {
+      const unsigned row = p / pieces, e = (p - row * pieces) * V;
+      *reinterpret_cast<vec_t*>(dst + row * o_sl + e) = *reinterpret_cast<const vec_t*>(src + (long)row * W + e);
+    }
+  } else {  // a row per wavefront, eight loads ahead
+    for (int row = threadIdx.x >> 6; row < rows; row += 4)
+      for (int e0 = threadIdx.x & 63; e0 < W; e0 += 8 * 64) {
+        T x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = src[(long)row * W + (e0 + i * 64 < W ? e0 + i * 64 : W - 1)];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (e0 + i * 64 < W) dst[row * o_sl + e0 + i * 64] = x[i];
+      }
+  }
 }
 
 // ---- one token per sequence ----
@@ -473,31 +493,45 @@ template <typename T> void launch_rglru_prefill(const RglruArgs& a, int tiles, T
                        a.ticket_step);
   }
   hipLaunchKernelGGL(rglru_segment_kernel<T>, grid, block, 0, s, t);
-  if (apart)
-    hipLaunchKernelGGL(rglru_copy_kernel<T>, dim3((unsigned)a.segs, (unsigned)a.B), block, 0, s, apart, static_cast<T*>(a.out), a.L, a.W,
-                       a.o_sb, a.o_sl);
+  if (apart) {
+    constexpr int V = Pack<T>::kN;
+    const bool vec = a.W % V == 0 && a.o_sl % V == 0 && a.o_sb % V == 0 && aligned_to(a.out, 16) && aligned_to(apart, 16);
+    hipLaunchKernelGGL((vec ? rglru_copy_kernel<T, V> : rglru_copy_kernel<T, 1>), dim3((unsigned)((a.L + kCopyRows - 1) / kCopyRows), (unsigned)a.B),
+                       block, 0, s, apart, static_cast<T*>(a.out), a.L, a.W, a.o_sb, a.o_sl);
+  }
 }
 
-// whether two (B, L, W) tensors lie in overlapping stretches of memory
-bool rglru_meet(const void* p, int64_t p_sb, int64_t p_sl, const void* q, int64_t q_sb, int64_t q_sl, int64_t B, int64_t L, int64_t W,
-                int64_t size) {
+// Whether two (B, L, W) tensors may share elements: their stretches of memory overlap, and they are not the columns of one matrix next
+// to each other (rows a whole number of row strides apart, W columns that the other does not reach).
+static bool rglru_meet(const void* p, int64_t p_sb, int64_t p_sl, const void* q, int64_t q_sb, int64_t q_sl, int64_t B, int64_t L, int64_t W,
+                       int64_t size) {
   const auto edge = [&](const void* base, int64_t sb, int64_t sl, bool high) {
     int64_t e = high ? W : 0;
     for (const int64_t d : {(B - 1) * sb, (L - 1) * sl}) e += (d > 0) == high ? d : 0;
     return (int64_t)(uintptr_t)base + e * size;
   };
-  return edge(p, p_sb, p_sl, false) < edge(q, q_sb, q_sl, true) && edge(q, q_sb, q_sl, false) < edge(p, p_sb, p_sl, true);
+  if (edge(p, p_sb, p_sl, false) >= edge(q, q_sb, q_sl, true) || edge(q, q_sb, q_sl, false) >= edge(p, p_sb, p_sl, true)) return false;
+  const int64_t row = L > 1 ? p_sl : p_sb, by = (int64_t)(uintptr_t)q - (int64_t)(uintptr_t)p;
+  if ((L > 1 && p_sl != q_sl) || (B > 1 && p_sb != q_sb) || row <= 0 || (B > 1 && p_sb % row != 0) || by % size != 0) return true;
+  const int64_t col = ((by / size) % row + row) % row;
+  return col < W || col + W > row;
 }
 
 }  // namespace based
+
+extern "C" BASED_API int64_t based_rglru_prefill_work(const void* u, const void* out, int64_t B, int64_t L, int64_t W, int64_t u_sb,
+                                                      int64_t u_sl, int64_t o_sb, int64_t o_sl, int io_dtype) {
+  if (B <= 0 || L <= 0 || W <= 0) return 0;
+  const int64_t size = io_dtype == BASED_BF16 ? 2 : 4;
+  return based::rglru_meet(u, u_sb, u_sl, out, o_sb, o_sl, B, L, W, size) ? (B * L * W * size + 3) / 4 : 0;
+}
 
 extern "C" BASED_API int based_rglru_prefill(const void* u, const void* y, const void* ra, const void* rb, const void* ri, const void* ib,
                                              const void* lam, float* work_a, float* work_x, float* work_agg, float* state, void* out,
                                              int64_t B, int64_t L, int64_t W, int64_t blocks, int64_t u_sb, int64_t u_sl, int64_t y_sb,
                                              int64_t y_sl, int64_t o_sb, int64_t o_sl, float c, int fresh, int io_dtype, void* stream) {
   using namespace based;
-  BASED_REQUIRE(u && y && ra && rb && ri && ib && lam && work_a && work_x && work_agg && state && out, BASED_ERR_ARG,
-                "rglru_prefill: null pointer argument");
+  BASED_REQUIRE(u && y && ra && rb && ri && ib && lam && work_agg && state && out, BASED_ERR_ARG, "rglru_prefill: null pointer argument");
   BASED_REQUIRE(B >= 0 && L >= 0 && W > 0 && blocks > 0, BASED_ERR_ARG, "rglru_prefill: bad sizes");
   BASED_REQUIRE(W % blocks == 0, BASED_ERR_SHAPE, "rglru_prefill: %ld channels do not divide into %ld blocks", (long)W, (long)blocks);
   BASED_REQUIRE(io_dtype == BASED_BF16 || io_dtype == BASED_F32, BASED_ERR_DTYPE, "rglru_prefill: bad dtype");
@@ -516,6 +550,7 @@ extern "C" BASED_API int based_rglru_prefill(const void* u, const void* y, const
                     o_sb, o_sl, c, fresh, vec_u, vec_y};
   // A workgroup reads channels of u that others' outputs would replace.
   const bool apart = rglru_meet(u, u_sb, u_sl, out, o_sb, o_sl, B, L, W, size);
+  BASED_REQUIRE(work_x || !apart, BASED_ERR_ARG, "rglru_prefill: no work space for an output that shares memory with the input");
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (io_dtype == BASED_BF16)
     launch_rglru_prefill<__bf16>(a, (int)tiles, apart ? reinterpret_cast<__bf16*>(work_x) : nullptr, s);

@@ -1010,13 +1010,6 @@ def _check_lru(x, y, ra, rb, ri, ib, lam, state, out, rows: int):
     return W, blocks
 
 
-def _stretches_meet(a, b) -> bool:
-    def stretch(t):
-        return t.data_ptr(), t.data_ptr() + (sum((n - 1) * s for n, s in zip(t.shape, t.stride())) + 1) * t.element_size()
-    (a0, a1), (b0, b1) = stretch(a), stretch(b)
-    return a0 < b1 and b0 < a1
-
-
 def rglru_prefill(u, y, ra, rb, ri, ib, lam, state, decay_scale: float, fresh: bool, *, out) -> torch.Tensor:
     """The gated linear recurrence over a portion: u (B, L, W) convolved, y (B, L, W) before its gelu; ra, ri
     (blocks, n, n) as [out, in], rb, ib, lam (W) values; state (B, W) fp32, updated in place, taken as
@@ -1025,12 +1018,15 @@ def rglru_prefill(u, y, ra, rb, ri, ib, lam, state, decay_scale: float, fresh: b
     W, blocks = _check_lru(u, y, ra, rb, ri, ib, lam, state, out, B)
     segs = (L + RGLRU_SEGMENT - 1) // RGLRU_SEGMENT
     agg = torch.empty(B, segs + 1, 2, W, dtype=torch.float32, device=u.device)
-    # only an output that shares memory with u is formed apart from it
-    work = torch.empty(B, L, W, dtype=torch.float32, device=u.device) if _stretches_meet(u, out) else agg
+    lib = _lib.lib()
+    # an output that shares memory with u is formed apart from it
+    n = lib.based_rglru_prefill_work(u.data_ptr(), out.data_ptr(), B, L, W, u.stride(0), u.stride(1), out.stride(0), out.stride(1),
+                                     _dtype_code(u))
+    work = torch.empty(n, dtype=torch.float32, device=u.device) if n else None
     with _on_device(u.device):
-        _lib.check(_lib.lib().based_rglru_prefill(
+        _lib.check(lib.based_rglru_prefill(
             u.data_ptr(), y.data_ptr(), ra.data_ptr(), rb.data_ptr(), ri.data_ptr(), ib.data_ptr(), lam.data_ptr(),
-            work.data_ptr(), work.data_ptr(), agg.data_ptr(), state.data_ptr(), out.data_ptr(), B, L, W, blocks, u.stride(0),
+            None, _ptr(work), agg.data_ptr(), state.data_ptr(), out.data_ptr(), B, L, W, blocks, u.stride(0),
             u.stride(1), y.stride(0), y.stride(1), out.stride(0), out.stride(1), float(decay_scale), int(fresh), _dtype_code(u),
             _stream_ptr(u)))
     return out

@@ -566,8 +566,10 @@ BASED_API int based_gated_delta_step(const void* x, const void* conv_w, void* ri
 /* Real-gated linear recurrent unit over a portion.  u (B, L, W) convolved; ra, ri (blocks, W / blocks,
  * W / blocks) as [out, in]; rb, ib, lam (W).  r = sigmoid(ra u + rb), i = sigmoid(ri u + ib),
  * a = exp(-c r softplus(lam)), S <- a S + sqrt(1 - a^2) i u, out = S * gelu_tanh(y).
- * work_a is not used, work_x, fp32 (B, L, W), only where the stretches of memory that u and out span overlap;
- * work_agg: fp32 (B, ceil(L / 64) + 1, 2, W); state (B, W) fp32. */
+ * work_a is not used and may be NULL; work_x: as many floats as based_rglru_prefill_work says, for an output that may share elements with
+ * u (0 of them: may be NULL); work_agg: fp32 (B, ceil(L / 64) + 1, 2, W); state (B, W) fp32. */
+BASED_API int64_t based_rglru_prefill_work(const void* u, const void* out, int64_t B, int64_t L, int64_t W, int64_t u_sb, int64_t u_sl,
+                                           int64_t o_sb, int64_t o_sl, int io_dtype);
 BASED_API int based_rglru_prefill(const void* u, const void* y, const void* ra, const void* rb, const void* ri, const void* ib,
                                   const void* lam, float* work_a, float* work_x, float* work_agg, float* state, void* out,
                                   int64_t B, int64_t L, int64_t W, int64_t blocks, int64_t u_sb, int64_t u_sl, int64_t y_sb,

@@ -123,3 +123,24 @@ def test_streamed_argument_validation_without_gpu():
     # channels that do not divide into blocks
     assert lib.based_rglru_prefill(*([p] * 12), 1, 1, 10, 3, *([8] * 6), 8.0, 1, 0, None) == 1
     assert b"blocks" in lib.based_hip_last_error()
+
+
+def test_rglru_scratch_wherever_elements_are_shared():
+    """An output that shares an element with the input gets a scratch, columns beside the input's in the same rows get none."""
+    import itertools
+
+    lib = _lib.lib()
+    none = 0
+    for B, L, W, sl, sb, size, code in itertools.product((1, 2), (1, 3), (2, 3), (3, 6, 7), (3, 6, 14, 21, 25), (2, 4), (0, 1)):
+        if size != (2 if code == _lib.BASED_BF16 else 4):
+            continue
+        u = {b * sb + t * sl + w for b in range(B) for t in range(L) for w in range(W)}
+        for at in range(-60, 61):
+            floats = lib.based_rglru_prefill_work(4096, 4096 + at * size, B, L, W, sb, sl, sb, sl, code)
+            meet = any(x + at in u for x in u)
+            assert floats in (0, (B * L * W * size + 3) // 4) and (floats or not meet), (B, L, W, sl, sb, at)
+            none += not floats and min(u) < max(u) + at and max(u) > min(u) + at
+    assert none > 100  # (side by side, stretches of memory overlapping)
+    # other strides: whatever overlaps
+    assert lib.based_rglru_prefill_work(4096, 4096 + 8, 1, 3, 2, 8, 4, 8, 8, 1) > 0
+    assert lib.based_rglru_prefill_work(4096, 4096 + 4 * 64, 1, 3, 2, 8, 4, 8, 8, 1) == 0

@@ -53,3 +53,24 @@ def test_rglru_segments(dev, dtype, L, W, blocks, rows, carry):
     rel = lambda a, b: ((a.double().cpu() - b).norm() / b.norm()).item()  # noqa: E731
     assert rel(state, S) < 2e-6, rel(state, S)
     assert rel(out, ref) < (2e-6 if dtype == torch.float32 else 2.5e-3), rel(out, ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("W,shift", [(72, 0), (72, 8), (72, -3), (33, 0), (33, 1), (128, -128), (128, 128), (120, 128)])
+def test_outputs_in_the_rows_of_the_input(dev, dtype, W, shift):
+    """An output `shift` columns from the input in the same rows (over it, partly over it, beside it) is what it is on its own."""
+    from based_amd import ops
+
+    B, L = 2, 70
+    g = torch.Generator().manual_seed(W + shift)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).to(dev)  # noqa: E731
+    both = rnd(B, L, 3 * 128)
+    u, y, gates = both[..., 128:128 + W], rnd(B, L, W), (rnd(1, W, W) * W ** -0.5, rnd(W), rnd(1, W, W) * W ** -0.5, rnd(W), rnd(W) - 3)
+    want, s0, s1 = torch.empty(B, L, W, dtype=dtype, device=dev), torch.zeros(B, W, device=dev), torch.zeros(B, W, device=dev)
+    ops.rglru_prefill(u.clone(), y, *gates, s0, 8.0, True, out=want)
+    outside = both.clone()
+    out = both[..., 128 + shift:128 + shift + W]
+    ops.rglru_prefill(u, y, *gates, s1, 8.0, True, out=out)
+    assert torch.equal(out, want) and torch.equal(s0, s1)
+    outside[..., 128 + shift:128 + shift + W] = want
+    assert torch.equal(both, outside)
