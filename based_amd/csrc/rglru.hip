@@ -114,6 +114,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
   const float kl = (0.5f * kL) * k2;
   // Token q * 16 + i * 4 + j of the segment stands in row i * 16 + q * 4 + j: element j of product i in the lanes of quad q.
   const auto token_of = [](int row) { return (row >> 2 & 3) * 16 + (row >> 4) * 4 + (row & 3); };
+  // Rows of no whole pieces go element by element: as many columns as are live, rounded up to a power of two (and to `least`).  All 64
+  // columns cost fp32 at B = 4, L = 2048, 7 blocks of 143 channels 180 us (124 now) and 1,024 blocks of one channel at L = 777 233 (167).
+  const auto columns = [](int live, int least) { return 32 - __builtin_clz((live > least ? live : least) * 2 - 1) - 1; };
   constexpr int YP = 64 * 64 / V / 256;
   vec_t yv[YP];
   const T* y = static_cast<const T*>(a.y) + b * a.y_sb + (long)blk * a.n + c0;
@@ -130,6 +133,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
   for (int it = 1, k0 = c0; it <= tiles; ++it) {  // the tile's own channels last: their u stays staged
     k0 = k0 + KT < tiles * KT ? k0 + KT : 0;
     if (it > 1) __syncthreads();
+    const int live = a.n - k0 < KT ? a.n - k0 : KT;
     constexpr int PIECES = 64 * (KT / V) / 256;
     if (a.vec_u) {
       vec_t xu[PIECES], xr[PIECES], xi[PIECES];
@@ -151,10 +155,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
         *reinterpret_cast<vec_t*>(&s_i[row * KS + e]) = xi[i];
       }
     } else {
-      for (int p = tid; p < 64 * KT; p += 256) {
-        const int row = p / KT, e = p % KT;
+      const int sh = columns(live, M::kK);
+#pragma unroll 4
+      for (int p = tid; p < 64 << sh; p += 256) {
+        const int row = p >> sh, e = p - (row << sh);
         const int t = l0 + token_of(row), c = c0 + row < a.n ? c0 + row : a.n - 1;
-        const bool in = k0 + e < a.n;
+        const bool in = e < live;
         const int k = in ? k0 + e : 0;
         const T xu = u[(t < a.L ? t : a.L - 1) * a.u_sl + k], xr = ra[(long)c * a.n + k], xi = ri[(long)c * a.n + k];
         s_u[row * KS + e] = in ? xu : (T)0.0f;
@@ -163,8 +169,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
       }
     }
     __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < KT; kk += M::kK) {
+    const auto product = [&](int kk) {
       const int e = kk + quad * M::kPer;
       const typename M::frag_t fr = *reinterpret_cast<const typename M::frag_t*>(&s_r[(wave * 16 + l16) * KS + e]);
       const typename M::frag_t fi = *reinterpret_cast<const typename M::frag_t*>(&s_i[(wave * 16 + l16) * KS + e]);
@@ -174,6 +179,13 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
         zr[i] = M::run(fu, fr, zr[i]);
         zi[i] = M::run(fu, fi, zi[i]);
       }
+    };
+    if (live == KT) {
+#pragma unroll
+      for (int kk = 0; kk < KT; kk += M::kK) product(kk);
+    } else {
+#pragma unroll 1
+      for (int kk = 0; kk < live; kk += M::kK) product(kk);
     }
   }
   __syncthreads();
@@ -184,8 +196,10 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
       *reinterpret_cast<vec_t*>(&s_y[p / (64 / V) * KS + p % (64 / V) * V]) = yv[i];
     }
   } else {
-    for (int p = tid; p < 64 * 64; p += 256) {
-      const int row = p / 64, e = p % 64, t = l0 + token_of(row);
+    const int sh = columns(a.n - c0 < 64 ? a.n - c0 : 64, 1);
+#pragma unroll 4
+    for (int p = tid; p < 64 << sh; p += 256) {
+      const int row = p >> sh, e = p - (row << sh), t = l0 + token_of(row);
       s_y[row * KS + e] = y[(t < a.L ? t : a.L - 1) * a.y_sl + (c0 + e < a.n ? e : 0)];
     }
   }
@@ -280,15 +294,16 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
       if (t < a.L && c0 + e < a.n) *reinterpret_cast<vec_t*>(out + t * a.o_sl + e) = *reinterpret_cast<const vec_t*>(&s_y[row * KS + e]);
     }
   } else {
-    for (int p = tid; p < 64 * 64; p += 256) {
-      const int row = p / 64, e = p % 64, t = l0 + token_of(row);
+    const int sh = columns(a.n - c0 < 64 ? a.n - c0 : 64, 1);
+    for (int p = tid; p < 64 << sh; p += 256) {
+      const int row = p >> sh, e = p - (row << sh), t = l0 + token_of(row);
       if (t < a.L && c0 + e < a.n) out[t * a.o_sl + e] = s_y[row * KS + e];
     }
   }
 }
 
-// Rows from the scratch to an output that shares memory with the input, V elements at a time; 16 rows of a sequence per workgroup.
-constexpr int kCopyRows = 16;
+// Rows from the scratch to an output that shares memory with the input, V elements at a time; 8 rows of a sequence per workgroup.
+constexpr int kCopyRows = 8;
 template <typename T, int V> __global__ __launch_bounds__(256) void rglru_copy_kernel(const T* src, T* dst, int L, int W, long o_sb, long o_sl) {
   typedef __attribute__((ext_vector_type(V))) T vec_t;
   const int l0 = blockIdx.x * kCopyRows, rows = L - l0 < kCopyRows ? L - l0 : kCopyRows;

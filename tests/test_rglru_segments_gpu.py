@@ -74,3 +74,10 @@ def test_outputs_in_the_rows_of_the_input(dev, dtype, W, shift):
     assert torch.equal(out, want) and torch.equal(s0, s1)
     outside[..., 128 + shift:128 + shift + W] = want
     assert torch.equal(both, outside)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("L,W,blocks", [(70, 40, 40), (66, 14, 7), (130, 15, 5), (65, 96, 24), (64, 48, 4), (100, 100, 1), (129, 65, 1)])
+def test_narrow_blocks(dev, dtype, L, W, blocks):
+    """Tiles with few live channels, of whole pieces and element by element."""
+    test_rglru_segments(dev, dtype, L, W, blocks, "own", True)
