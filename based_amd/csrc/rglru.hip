@@ -13,7 +13,8 @@
 
 namespace based {
 
-constexpr int kSeg = 64;  // tokens per segment
+constexpr int kSeg = 64;    // tokens per segment
+constexpr int kGroup = 64;  // segments whose last one leaves the state behind it
 
 struct RglruArgs {
   const void* u;  // (B, L, W), strides
@@ -81,7 +82,9 @@ __global__ __launch_bounds__(256) void rglru_begin_kernel(unsigned long long* ag
 // A workgroup takes the next segment of its tile and sequence, forms the gates of 64 tokens, leaves what they do to any state that enters
 // them for the segments behind, and takes the state that enters its own from those in front.  It waits for them only after its own is
 // left; they were taken before it by workgroups that run or have run, so each wait ends.  P and X travel in one 64-bit word, which is
-// its own flag.  (Gates as fp32 pairs through memory for a second kernel, 134 of 184 MB at B = 4, L = 2048, W = 1024: 51 us; gates
+// its own flag.  The last of every kGroup segments leaves the state itself (P = 0) once it has it, and nobody reads behind that: at most
+// kGroup words a segment whatever the length (all those in front at 2,048 segments, B = 1, W = 1024: 1,920 us; 664 in groups; 73 and 66 at 16,384 tokens).  A
+// fixed place, not the nearest state that is there: the same sums on every run.  (Gates as fp32 pairs through memory for a second kernel, 134 of 184 MB at B = 4, L = 2048, W = 1024: 51 us; gates
 // formed by two kernels, 43 us: the vector unit is the bound, three exponentials, two reciprocals and a square root an element.)
 // The products lie with 16 consecutive tokens of a channel in one lane, where the recurrence is two instructions an element, and 64 in
 // a wavefront.  B = 4, L = 2048, W = 1024, 8 blocks: 29 us with the kernel in front; B = 8, L = 4096: 111 (237).
@@ -234,20 +237,26 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
   }
   float S = seg == 0 && !a.fresh ? a.state[(long)b * a.W + w] : 0.f;
   unsigned long long* g = a.agg + (long)b * a.segs * a.W + w;
-  if (seg < a.segs - 1 && quad == 3 && ch < a.n) {
+  const auto leave = [&](float pw, float xw) {
+    unsigned int bits = __builtin_bit_cast(unsigned int, pw);
+    bits = bits == ~0u ? 0x7fc00000u : bits;
+    __hip_atomic_store(g + (long)seg * a.W, (unsigned long long)__builtin_bit_cast(unsigned int, xw) << 32 | bits, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  };
+  const bool mine = quad == 3 && ch < a.n, closes = seg % kGroup == kGroup - 1;
+  if (seg < a.segs - 1 && mine && !closes) {
     float xw = __builtin_fmaf(P, before_x, X), pw = P * before_p;
     if (seg == 0) {  // (what enters the call is part of it: the last segment replaces the state)
       xw = __builtin_fmaf(pw, S, xw);
       pw = 0.f;
     }
-    unsigned int bits = __builtin_bit_cast(unsigned int, pw);
-    bits = bits == ~0u ? 0x7fc00000u : bits;
-    __hip_atomic_store(g + (long)seg * a.W, (unsigned long long)__builtin_bit_cast(unsigned int, xw) << 32 | bits, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+    leave(pw, xw);
   }
   if (seg > 0) {
-    // a quarter of the segments in front for each quad
-    const int each = (seg + 3) / 4, first = quad * each;
+    // a quarter of the segments in front for each quad, from the one that closes the group before on
+    const int from = seg < kGroup ? 0 : seg / kGroup * kGroup - 1, count = seg - from;
+    const int each = (count + 3) / 4, first = quad * each;
+    const unsigned long long* in_front = g + (long)from * a.W;
     float p = 1.f, x = 0.f;
     constexpr int U = 4;
     for (int i0 = 0; i0 < each; i0 += U) {
@@ -258,14 +267,14 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
 #pragma unroll
         for (int i = 0; i < U; ++i) {
           const int at = first + i0 + i;
-          v[i] = __hip_atomic_load(g + (long)(at < seg ? at : seg - 1) * a.W, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          v[i] = __hip_atomic_load(in_front + (long)(at < count ? at : count - 1) * a.W, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
 #pragma unroll
         for (int i = 0; i < U; ++i) wait |= (unsigned int)v[i] == ~0u;
       } while (__any(wait));
 #pragma unroll
       for (int i = 0; i < U; ++i) {
-        const bool in = i0 + i < each && first + i0 + i < seg;
+        const bool in = i0 + i < each && first + i0 + i < count;
         const float pi = __builtin_bit_cast(float, (unsigned int)v[i]), xi = __builtin_bit_cast(float, (unsigned int)(v[i] >> 32));
         x = in ? __builtin_fmaf(pi, x, xi) : x;
         p = in ? p * pi : p;
@@ -276,6 +285,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
     for (int q = 1; q < 4; ++q) S = __builtin_fmaf(__shfl(p, q * 16 + l16), S, __shfl(x, q * 16 + l16));
   }
   S = __builtin_fmaf(before_p, S, before_x);
+  if (seg < a.segs - 1 && mine && closes) leave(0.f, __builtin_fmaf(P, S, X));
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -284,7 +294,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
       T* at = &s_y[(i * 16 + quad * 4 + j) * KS + wave * 16 + l16];
       *at = from_f32<T>(S * gelu_tanh_f(to_f32(*at)));
     }
-  if (seg == a.segs - 1 && quad == 3 && ch < a.n) a.state[(long)b * a.W + w] = S;
+  if (seg == a.segs - 1 && mine) a.state[(long)b * a.W + w] = S;
   __syncthreads();
   T* out = static_cast<T*>(a.out) + b * a.o_sb + (long)blk * a.n + c0;
   if (a.vec_y) {

@@ -81,3 +81,9 @@ def test_outputs_in_the_rows_of_the_input(dev, dtype, W, shift):
 def test_narrow_blocks(dev, dtype, L, W, blocks):
     """Tiles with few live channels, of whole pieces and element by element."""
     test_rglru_segments(dev, dtype, L, W, blocks, "own", True)
+
+
+@pytest.mark.parametrize("L", [4095, 4096, 4097, 4160, 4161, 8192, 8193, 12500])
+def test_groups_of_segments(dev, L):
+    """Lengths around one, two and three groups of 64 segments."""
+    test_rglru_segments(dev, torch.float32, L, 20, 1, "own", True)
