@@ -573,9 +573,11 @@ __global__ __launch_bounds__(256) void decay_join_kernel(const DecayScanArgs a) 
 // 16 lanes per value channel, groups of four channels of the key each; 16 value channels per workgroup.  Token by token, so what counts is
 // the length of the chain and the workgroups beside each other: long portions go in segments, as on MFMA.  fp32, B = 1, H = 16,
 // d = dv = 64, channel decays, L = 777: 47 us (one chain, four channels 16 apart to a lane: 230); L = 2048: 86 (715).
-template <typename T, int CPT, bool CHANNEL, bool STATE_ONLY>
+// kTile tokens are staged at once: 16, a barrier pair for each, where all workgroups are on the GPU together anyway, and 8 where keys of
+// more than 128 channels would then keep some waiting for LDS.  fp32, H = 4, d = dv = 256, channel decays, 16 against 8: B = 64, L = 200:
+// 1,078 us, 798; B = 16, L = 300: 435, 300; B = 1, L = 300: 76, 82.
+template <typename T, int CPT, bool CHANNEL, bool STATE_ONLY, int kTile>
 __global__ __launch_bounds__(256) void decay_scan_any_kernel(const DecayScanArgs a) {
-  constexpr int kTile = 16;  // tokens staged at once
   constexpr int CH = 16 * CPT;
   __shared__ __attribute__((aligned(16))) float sq[STATE_ONLY ? 1 : kTile][CH], sk[kTile][CH], sw[CHANNEL ? kTile : 1][CH];
   __shared__ float sv[kTile][16];
@@ -931,13 +933,22 @@ template <bool CHANNEL> int launch_decay_scan_mfma(const DecayScanArgs& a, hipSt
   return launch_decay_mfma<2, 2, CHANNEL>(a, s);
 }
 
-template <typename T, int CPT, bool CHANNEL> void launch_decay_any(const DecayScanArgs& a, hipStream_t s) {
+template <typename T, int CPT, bool CHANNEL, int TOKENS> void launch_decay_any_tile(const DecayScanArgs& a, hipStream_t s) {
   const unsigned cols = (unsigned)((a.dv + 15) / 16);
   if (a.segs > 1) {
-    hipLaunchKernelGGL((decay_scan_any_kernel<T, CPT, CHANNEL, true>), dim3((unsigned)(a.B * a.H), cols, (unsigned)(a.segs - 1)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((decay_scan_any_kernel<T, CPT, CHANNEL, true, TOKENS>), dim3((unsigned)(a.B * a.H), cols, (unsigned)(a.segs - 1)), dim3(256), 0,
+                       s, a);
     launch_decay_join(a, s);
   }
-  hipLaunchKernelGGL((decay_scan_any_kernel<T, CPT, CHANNEL, false>), dim3((unsigned)(a.B * a.H), cols, (unsigned)a.segs), dim3(256), 0, s, a);
+  hipLaunchKernelGGL((decay_scan_any_kernel<T, CPT, CHANNEL, false, TOKENS>), dim3((unsigned)(a.B * a.H), cols, (unsigned)a.segs), dim3(256), 0, s, a);
+}
+
+template <typename T, int CPT, bool CHANNEL> void launch_decay_any(const DecayScanArgs& a, hipStream_t s) {
+  if constexpr (CPT > 8) {
+    // workgroups that the LDS of 256 compute units holds with 16 tokens: three of 49 KB to one, or four of 33 KB
+    if ((long)a.B * a.H * ((a.dv + 15) / 16) * a.segs > (CHANNEL ? 768 : 1024)) return launch_decay_any_tile<T, CPT, CHANNEL, 8>(a, s);
+  }
+  launch_decay_any_tile<T, CPT, CHANNEL, 16>(a, s);
 }
 
 template <typename T, bool CHANNEL> void launch_decay_scan_any(const DecayScanArgs& a, hipStream_t s) {

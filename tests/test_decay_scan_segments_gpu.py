@@ -69,3 +69,34 @@ def test_head_decays_below_zero(dev, L, dtype):
     # as above: up to five hundred roundings of 2^-24 that lie independently, and half of 2^-8 of bf16 outputs
     assert rel(out, torch.stack(ref, 1)) < (4e-6 if dtype == torch.float32 else 3e-3)
     assert rel(state, S.transpose(2, 3)) < 4e-6
+
+
+@pytest.mark.parametrize("B,L,d", [(3, 45, 130), (65, 45, 130), (50, 33, 250)])
+def test_long_keys_in_many_workgroups(dev, B, L, d):
+    """Keys of more than 128 channels: 16 tokens at a time, or 8 where the workgroups are many; whole tiles and a rest."""
+    from based_amd import ops
+
+    H, dv = 2, 128
+    g = torch.Generator().manual_seed(B + L)
+    q, k, v, u = (torch.randn(*s, generator=g) for s in ((B, L, H * d), (B, L, H * d), (B, L, H * dv), (H, d)))
+    lw = -torch.exp(torch.randn(B, L, H * d, generator=g) - 2)
+    decay = [0.9, 0.99]
+    dp = (d + 3) // 4 * 4
+    S0 = torch.randn(B, H, dv, dp, generator=g)
+    for channel in (True, False):
+        kw = dict(channel_log2=lw.to(dev), bonus=u.to(dev)) if channel else dict(head_decay=ops.head_decays(decay, dev))
+        state = S0.to(dev)
+        out = ops.decay_scan(q.to(dev), k.to(dev), v.to(dev), state, H, fresh=False, **kw)
+        S, ref = S0[..., :d].double().transpose(2, 3), []
+        w = torch.tensor(decay, dtype=torch.float32).double().view(1, H, 1, 1)
+        for t in range(L):
+            qt, kt, vt = (x[:, t].double().view(B, H, -1) for x in (q, k, v))
+            kv = kt[..., None] * vt[:, :, None]
+            if channel:
+                ref.append(((S + u.double()[..., None] * kv) * qt[..., None]).sum(2).flatten(1))
+                S = 2.0 ** lw[:, t].double().view(B, H, d, 1) * S + kv
+            else:
+                S = w * S + kv
+                ref.append((S * qt[..., None]).sum(2).flatten(1))
+        rel = lambda a, b: ((a.double().cpu() - b).norm() / b.norm()).item()  # noqa: E731
+        assert rel(out, torch.stack(ref, 1)) < 1e-6 and rel(state[..., :d], S.transpose(2, 3)) < 1e-6  # (some dozens of roundings of 2^-24)
