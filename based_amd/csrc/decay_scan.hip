@@ -1001,21 +1001,28 @@ static int decay_segments(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV
   return segs < 2 ? 1 : (int)segs;
 }
 
-// The same for the general form: eight workgroups to a compute unit.  Every token but those of the last segment is walked twice, so three
-// segments would gain a third at best, less the launches: from four on (B = 1, H = 12, L = 250: 37 us in four, 77 in one).
-static int decay_any_segments(int64_t B, int64_t L, int64_t H, int64_t DV) {
+// The same for the general form: eight workgroups to a compute unit.  Every token but those of the last segment is walked twice, so the
+// chain is two segments long: three segments ask for a third less at best, and the launches.  Segments where four are wanted, of which
+// whole 64-token pieces may leave three.  us in segments against one chain, channel decays: B = 1, H = 12, L = 250: 37 in four, 77; 8 x 16
+// heads of 64, in three, L = 257: 82, 83; L = 320: 86, 103; L = 384: 100, 121.  Keys of more than 64 channels gain only where the two
+// segments are the shorter chain by more than the launches: 16 x 4 heads of 128, L = 257: 127, 114; L = 320: 133, 145; 8 x 4 heads of 256
+// (head decays), L = 257: 181, 158; L = 320: 194, 225.
+static int decay_any_segments(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
   const int64_t chunks = (L + kScanTokens - 1) / kScanTokens, wgs = B * H * ((DV + 15) / 16);
   int64_t segs = (2048 + wgs - 1) / wgs;
   if (segs > chunks) segs = chunks;
   if (segs > 64) segs = 64;
-  return segs < 4 ? 1 : (int)segs;
+  if (segs < 4) return 1;
+  const int64_t each = (chunks + segs - 1) / segs;
+  if (D > 64 && 2 * each * kScanTokens + 16 > L) return 1;
+  return (int)((chunks + each - 1) / each);
 }
 
 }  // namespace based
 
 extern "C" BASED_API int64_t based_decay_scan_work(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, int64_t state_row) {
   if (B <= 0 || L <= 0 || H <= 0 || D <= 0 || DV <= 0) return 0;
-  const int64_t mfma = based::decay_segments(B, L, H, D, DV), any = based::decay_any_segments(B, L, H, DV), segs = mfma > any ? mfma : any;
+  const int64_t mfma = based::decay_segments(B, L, H, D, DV), any = based::decay_any_segments(B, L, H, D, DV), segs = mfma > any ? mfma : any;
   return segs <= 1 ? 0 : B * H * segs * (DV + 1) * state_row;
 }
 
@@ -1044,7 +1051,7 @@ extern "C" BASED_API int based_decay_scan(const void* q, const void* k, const vo
   const bool vec = io_dtype == BASED_BF16 && D <= 128 && D % 4 == 0 && DV % 4 == 0 && q_sb % 4 == 0 && q_sl % 4 == 0 && k_sb % 4 == 0 &&
                    k_sl % 4 == 0 && v_sb % 4 == 0 && v_sl % 4 == 0 && o_sb % 4 == 0 && o_sl % 4 == 0 && aligned_to(q, 8) &&
                    aligned_to(k, 8) && aligned_to(v, 8) && aligned_to(o, 8) && aligned_to(bonus, 8) && aligned_to(channel_log2, 16);
-  const int segs = vec ? decay_segments(B, L, H, D, DV) : work != nullptr ? decay_any_segments(B, L, H, DV) : 1;
+  const int segs = vec ? decay_segments(B, L, H, D, DV) : work != nullptr ? decay_any_segments(B, L, H, D, DV) : 1;
   if (segs > 1) {
     BASED_REQUIRE(work != nullptr, BASED_ERR_ARG, "decay_scan: no work space");
     a.seg_chunks = (a.seg_chunks + segs - 1) / segs;

@@ -100,3 +100,44 @@ def test_long_keys_in_many_workgroups(dev, B, L, d):
                 ref.append((S * qt[..., None]).sum(2).flatten(1))
         rel = lambda a, b: ((a.double().cpu() - b).norm() / b.norm()).item()  # noqa: E731
         assert rel(out, torch.stack(ref, 1)) < 1e-6 and rel(state[..., :d], S.transpose(2, 3)) < 1e-6  # (some dozens of roundings of 2^-24)
+
+
+@pytest.mark.parametrize("channel", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,L,H,d,dv", [(4, 1023, 16, 64, 64), (4, 1025, 16, 64, 64),            # eight or nine segments of two pieces
+                                        (1, 64 * 64 + 70, 1, 20, 17), (2, 64 * 130 + 1, 1, 8, 4),  # 33 of two, 44 of three
+                                        (8, 257, 16, 64, 64), (8, 320, 16, 20, 64),                # three of two, the last of one token or a piece
+                                        (8, 271, 16, 68, 60), (8, 272, 16, 68, 60)])               # one chain, and three
+def test_segments_of_several_pieces(dev, B, L, H, d, dv, dtype, channel):
+    """Segments longer than a 64-token piece, the last one shorter than the others: fresh, and from a state that goes on."""
+    from based_amd import ops
+
+    g = torch.Generator().manual_seed(L + d)
+    dp = (d + 3) // 4 * 4
+    mk = lambda *s: torch.randn(*s, generator=g).to(dtype).to(dev)  # noqa: E731
+    q, k, v, u = mk(B, L, H * d), mk(B, L, H * d), mk(B, L, H * dv), mk(H, d)
+    if dtype == torch.bfloat16:  # rows off an 8-byte address, which the matrix form would take
+        q, k, v = (torch.empty(B, L, t.shape[2] + 1, dtype=dtype, device=dev)[..., 1:].copy_(t) for t in (q, k, v))
+    lw = -torch.exp(0.5 * torch.randn(B, L, H * d, generator=g) - 4).to(dev)
+    decay = torch.linspace(0.9, 0.9995, H).tolist()
+    kw = dict(channel_log2=lw, bonus=u) if channel else dict(head_decay=ops.head_decays(decay, dev))
+    S0 = torch.zeros(B, H, dv, dp)
+    S0[..., :d] = torch.randn(B, H, dv, d, generator=g)
+    rel = lambda a, b: ((a.double() - b).norm() / b.norm()).item()  # noqa: E731
+    for fresh in (True, False):
+        state = torch.full((B, H, dv, dp), float("nan"), device=dev) if fresh else S0.to(dev)
+        out = ops.decay_scan(q, k, v, state, H, fresh=fresh, **kw)
+        S = torch.zeros(B, H, d, dv, dtype=torch.float64, device=dev) if fresh else S0[..., :d].double().transpose(2, 3).to(dev)
+        w = torch.tensor(decay, dtype=torch.float32).double().view(1, H, 1, 1).to(dev)
+        ref = torch.empty(B, L, H * dv, dtype=torch.float64, device=dev)
+        for t in range(L):
+            qt, kt, vt = (x[:, t].double().view(B, H, -1) for x in (q, k, v))
+            kv = kt[..., None] * vt[:, :, None]
+            if channel:
+                ref[:, t] = ((S + u.double()[..., None] * kv) * qt[..., None]).sum(2).flatten(1)
+                S = 2.0 ** lw[:, t].double().view(B, H, d, 1) * S + kv
+            else:
+                S = w * S + kv
+                ref[:, t] = (S * qt[..., None]).sum(2).flatten(1)
+        # decays of 0.99 and 0.9995 keep a hundred to two thousand tokens: 2 * 2^-24 * 2000^0.5 = 5e-6; bf16 outputs add half of 2^-8
+        assert rel(out, ref) < (5e-6 if dtype == torch.float32 else 3e-3) and rel(state[..., :d], S.transpose(2, 3)) < 5e-6
