@@ -1185,9 +1185,13 @@ def decay_scan(q, k, v, state, heads: int, *, channel_log2=None, bonus=None, hea
     else:
         _check_head_decay(head_decay, heads, q.device)
     lib = _lib.lib()
-    n = lib.based_decay_scan_work(B, L, heads, d, dv, state.shape[3])
-    work = torch.empty(n, dtype=torch.float32, device=q.device) if n else None
     o = torch.empty(B, L, heads * dv, dtype=q.dtype, device=q.device)
+    work = None
+    if lib.based_decay_scan_work(B, L, heads, d, dv, state.shape[3]):
+        n = lib.based_decay_scan_work_of(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(channel_log2), _ptr(bonus), o.data_ptr(), B, L, heads, d, dv, state.shape[3],
+            q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1), o.stride(0), o.stride(1), _dtype_code(q))
+        work = torch.empty(n, dtype=torch.float32, device=q.device) if n else None
     with _on_device(q.device):
         _lib.check(lib.based_decay_scan(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(channel_log2), _ptr(head_decay), _ptr(bonus), state.data_ptr(), _ptr(work),

@@ -144,3 +144,21 @@ def test_rglru_scratch_wherever_elements_are_shared():
     # other strides: whatever overlaps
     assert lib.based_rglru_prefill_work(4096, 4096 + 8, 1, 3, 2, 8, 4, 8, 8, 1) > 0
     assert lib.based_rglru_prefill_work(4096, 4096 + 4 * 64, 1, 3, 2, 8, 4, 8, 8, 1) == 0
+
+
+def test_decay_work_is_for_the_form_that_runs():
+    """Aligned bf16 (the matrix form) asks for its own segments, everything else for those of the general form; one number covers both."""
+    lib = _lib.lib()
+
+    def of(B, L, H, D, DV, code, q=4096, row=None, pad=0):
+        row = (D + 3) // 4 * 4
+        x = (L * (H * D + pad), H * D + pad)
+        return lib.based_decay_scan_work_of(q, 8192, 8192, 8192, 8192, 8192, B, L, H, D, DV, row, *x, *x, L * H * DV, H * DV, L * H * DV, H * DV, code)
+
+    floats = lambda segs, B, H, D, DV: B * H * segs * (DV + 1) * ((D + 3) // 4 * 4)  # noqa: E731
+    for B, L, H, D, DV, mfma, general in [(1, 256, 16, 64, 64, 0, 4), (1, 2048, 16, 64, 64, 8, 32), (4, 2048, 16, 64, 64, 8, 8),
+                                          (1, 100, 16, 64, 64, 0, 0), (8, 320, 16, 64, 64, 0, 3), (64, 2048, 16, 64, 64, 0, 0)]:
+        assert of(B, L, H, D, DV, 0) == floats(mfma, B, H, D, DV), (B, L)
+        for other in (dict(code=1), dict(code=0, q=4098), dict(code=0, pad=1)):
+            assert of(B, L, H, D, DV, **other) == floats(general, B, H, D, DV), (B, L, other)
+        assert lib.based_decay_scan_work(B, L, H, D, DV, 64) == floats(max(mfma, general), B, H, D, DV)
