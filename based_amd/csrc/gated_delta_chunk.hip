@@ -559,14 +559,35 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_scan_kernel(const DeltaChu
 // Workspace: the chunks of one launch pair.  Long prompts go through it in spans of chunks, the state carried on in between.
 constexpr int64_t kDcWorkFloats = 64ll << 20;  // 256 MB, which the last-level cache holds between the two launches
 
-// Where chunks are the faster form.  A chunk step of the scan takes 1.7 us (four blocks of 16: 4.8) whatever the number of heads up to
-// two workgroups per compute unit, and costs 20 to 40 ns of preparation per head, 26 times the products of a block's: few heads and
-// more than a few chunks.  us, blocks of 16 against chunks, d = 64, dv = 128 unless said: 1 x 8 heads, L = 64: 22.7, 23.8; 1 x 4, L =
-// 256, dv = 64: 27.6, 24.5; 1 x 4, L = 4096, dv = 64: 295, 118; 4 x 8, L = 2048: 163, 95; 4 x 16, L = 2048, dv = 64: 169, 115; the same
-// with d = dv = 128: 316, 291; 8 x 16, L = 4096, dv = 64: 415, 493; 16 x 16, L = 1024, dv = 64: 170, 285; d = dv = 256, 4 x 4, L = 300:
-// 62.6, 66.0.
+// Where chunks are the faster form: few heads, and enough chunks.  A chunk step of the scan takes 1.5 us (2.7 with heads of more than 64
+// channels, which fill eight tiles whatever their size) where four blocks of 16 take 3.2 to 6.8, by the size of the heads; but both
+// launches together start 8 to 10 us later than those of the blocks, values of many tiles read every chunk's rows once each, and every head
+// adds 20 to 90 ns of preparation a chunk: 26 times a block's products, and more memory than the cache holds at the far end.  us, blocks
+// of 16 against chunks, heads, d x dv:
+//   8, 64 x 64: L = 256: 27.7, 24.0.  32, 64 x 128: L = 256: 29, 28; L = 2048: 161, 91.  64, 64 x 128: L = 256: 33, 35; L = 384: 45, 43.
+//   64, 32 x 128: L = 512: 47, 48; L = 2048: 154, 170.  8, 64 x 512: L = 256: 30, 34; L = 384: 39, 38.
+//   8, 96 x 96: L = 256: 41, 35.  32, 96 x 256: L = 384: 59, 61; L = 1024: 131, 121.  64, 96 x 128: L = 512: 75, 77; L = 2048: 263, 298.
+//   8, 128 x 128: L = 256: 35.0, 35.4; L = 320: 40, 38.  32, 128 x 128: L = 320: 41, 42; L = 384: 47, 45.  16, 128 x 256: L = 384: 45, 47;
+//   L = 512: 56, 52.  More heads: 128, 64 x 64, L = 4096: 415, 493; more channels: 16, 256 x 256, L = 300: 62.6, 66.0.
 static bool dc_faster(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
-  return B * H <= 64 && B * H * ((DV + 15) / 16) <= 512 && L >= 4 * kDc && D <= 128;
+  const int64_t heads = B * H, tiles = (DV + 15) / 16, wgs = heads * tiles;  // (of the scan, two of which a compute unit holds)
+  if (heads > 64 || wgs > 512 || D > 128) return false;
+  const bool crowded = wgs > 256;
+  const int64_t wide = tiles > 16 ? (tiles - 16) / 8 : 0;
+  int64_t chunks;
+  if (D > 96)
+    chunks = 3 + (DV + 127) / 128 + (DV > 128) + (heads > 8 && !crowded);
+  else if (crowded && (D <= 16 || (heads > 32 && (D > 64 || D <= 32))))  // (the blocks' steps are cheap here, and there is much to prepare)
+    return false;
+  else if (D > 64)
+    chunks = crowded ? 10 : 4 + wide;
+  else if (D > 32)
+    chunks = 4 + (D > 48 ? wide : 0) + (wgs > 448) + (wgs > 448 && heads > 32);
+  else if (D > 16)
+    chunks = crowded ? 12 : 4 + wgs / 100 + wide;
+  else
+    chunks = 4 + (wgs < 96 ? wgs / 24 : 4) + (tiles > 8) + 2 * wide;
+  return L >= chunks * kDc;
 }
 
 static int dc_tiles(int64_t D) { return D <= 64 ? 4 : 8; }
@@ -576,7 +597,7 @@ static int64_t dc_span(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
   if (B <= 0 || L <= 0 || H <= 0 || D <= 0 || DV <= 0 || B >= (1ll << 31) || H >= (1ll << 31) || DV >= (1ll << 20) || !dc_faster(B, L, H, D, DV))
     return 0;
   const int64_t chunks = (L + kDc - 1) / kDc, each = B * H * dc_floats(dc_tiles(D), (int)DV);
-  int64_t span = kDcWorkFloats / each;  // (at least 6: 512 value tiles and 64 heads are 10 M floats a chunk at most)
+  int64_t span = kDcWorkFloats / each;  // (at least 29: a chunk of 64 heads and 512 value tiles takes 2.3 M floats at most)
   if (span > chunks) span = chunks;
   // spans of about equal length
   const int64_t n = (chunks + span - 1) / span;

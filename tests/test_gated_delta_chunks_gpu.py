@@ -131,3 +131,17 @@ def test_long_and_short_queries(dev, dtype, scale):
     o, S = run(case, H, H, d, dv, empty_state(1, H, d, dv, dev))
     ref, S_ref = reference(*case, H, H, d, dv)
     assert rel_l2(o, ref) < TOL and rel_l2(S, S_ref) < TOL
+
+
+@pytest.mark.parametrize("B,H,d,dv,first", [(1, 4, 16, 16, 4), (4, 8, 16, 64, 8), (4, 8, 64, 128, 4), (8, 8, 64, 128, 6), (2, 8, 64, 512, 7),
+                                            (4, 8, 96, 256, 10), (8, 8, 96, 128, None), (1, 8, 128, 128, 4), (2, 8, 128, 128, 5),
+                                            (8, 8, 128, 128, 4), (2, 8, 128, 256, 7)])
+def test_where_chunks_begin(dev, B, H, d, dv, first):
+    """The first whole number of chunks that goes in chunks, and a token less: the same numbers on both sides of the line."""
+    edge = 64 * (first or 12)
+    for L in (edge - 1, edge):
+        assert in_chunks(B, L, H, d, dv) == (first is not None and L == edge)
+        case = [t.to(dev) for t in make(L, B, L, H, H, d, dv, torch.float32)]
+        o, S = run(case, H, H, d, dv, empty_state(B, H, d, dv, dev))
+        ref, S_ref = reference(*case, H, H, d, dv)
+        assert rel_l2(o, ref) < 3e-6 and rel_l2(S, S_ref) < 3e-6  # (the tolerance of the blocks)
