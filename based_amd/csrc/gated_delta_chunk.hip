@@ -587,7 +587,7 @@ static bool dc_faster(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
     chunks = crowded ? 12 : 4 + wgs / 100 + wide;
   else
     chunks = 4 + (wgs < 96 ? wgs / 24 : 4) + (tiles > 8) + 2 * wide;
-  return L >= chunks * kDc;
+  return L >= chunks * kDc && L >= BASED_DELTA_CHUNKS_MIN;
 }
 
 static int dc_tiles(int64_t D) { return D <= 64 ? 4 : 8; }
@@ -603,6 +603,12 @@ static int64_t dc_span(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
   const int64_t n = (chunks + span - 1) / span;
   return (chunks + n - 1) / n;
 }
+
+// Rows of queries and keys whose groups of four channels are one load; chunks of more than 64 channels take no others.
+static bool dc_vec(const void* q, const void* k, int64_t B, int64_t D, int64_t x_sb, int64_t x_sl) {
+  return D % 4 == 0 && (B == 1 || x_sb % 4 == 0) && x_sl % 4 == 0 && aligned_to(q, 16) && aligned_to(k, 16);
+}
+static bool dc_near(int64_t H, int64_t DV, int64_t x_sl) { return x_sl >= 0 && x_sl < (1ll << 24) && H * DV < (1ll << 25); }
 
 template <typename T, int RB, int LAY> static int run_delta_chunks(DeltaChunkArgs a, int64_t span, hipStream_t s) {
   const int chunks = (a.L + kDc - 1) / kDc;
@@ -636,6 +642,13 @@ extern "C" BASED_API int64_t based_gated_delta_scan_work(int64_t B, int64_t L, i
   return span == 0 ? 0 : B * H * span * dc_floats(dc_tiles(D), (int)DV);
 }
 
+extern "C" BASED_API int64_t based_gated_delta_scan_work_of(const void* q, const void* k, int64_t B, int64_t L, int64_t H, int64_t D,
+                                                            int64_t DV, int64_t x_sb, int64_t x_sl) {
+  using namespace based;
+  if (!dc_near(H, DV, x_sl) || !(D <= 64 || dc_vec(q, k, B, D, x_sb, x_sl))) return 0;
+  return based_gated_delta_scan_work(B, L, H, D, DV);
+}
+
 extern "C" BASED_API int based_gated_delta_scan_chunks(const void* q, const void* k, const void* v, const void* a_gate, const void* b_gate,
                                                        const void* a_log, const void* dt_bias, float* state, float* work, float* o,
                                                        int64_t B, int64_t L, int64_t H, int64_t G, int64_t D, int64_t DV, int64_t state_row,
@@ -646,21 +659,20 @@ extern "C" BASED_API int based_gated_delta_scan_chunks(const void* q, const void
   BASED_REQUIRE(q && k && v && a_gate && b_gate && a_log && dt_bias && state && work && o, BASED_ERR_ARG, "%s: null pointer argument", who);
   BASED_REQUIRE(B >= 0 && L >= 0 && H > 0 && G > 0 && D > 0 && DV > 0, BASED_ERR_ARG, "%s: bad sizes", who);
   BASED_REQUIRE(H % G == 0, BASED_ERR_SHAPE, "%s: %ld heads do not divide into %ld query/key heads", who, (long)H, (long)G);
-  BASED_REQUIRE(D <= 256, BASED_ERR_SHAPE, "%s: query/key size %ld (at most 256)", who, (long)D);
+  BASED_REQUIRE(D <= 128, BASED_ERR_SHAPE, "%s: query/key size %ld (at most 128 in chunks)", who, (long)D);
   BASED_REQUIRE(state_row >= DV, BASED_ERR_ARG, "%s: state rows of %ld for a value size of %ld", who, (long)state_row, (long)DV);
   BASED_REQUIRE(io_dtype == BASED_BF16 || io_dtype == BASED_F32, BASED_ERR_DTYPE, "%s: bad dtype", who);
   BASED_REQUIRE(B * H < (1ll << 31) && L < (1ll << 31) - kDc && DV < (1ll << 20), BASED_ERR_SHAPE, "%s: grid too large", who);
   if (B == 0 || L == 0) return BASED_OK;
-  BASED_REQUIRE(x_sl >= 0 && x_sl < (1ll << 24) && H * DV < (1ll << 25), BASED_ERR_SHAPE, "%s: rows too long", who);
+  BASED_REQUIRE(dc_near(H, DV, x_sl), BASED_ERR_SHAPE, "%s: rows too long", who);
   BASED_REQUIRE(aligned_to(work, 16), BASED_ERR_ALIGN, "%s: the work space must be 16-byte aligned", who);
   const int64_t span = dc_span(B, L, H, D, DV);
   BASED_REQUIRE(span > 0 && B * H * span < (1ll << 31), BASED_ERR_SHAPE, "%s: the shape is for blocks of 16", who);
-  // groups of four channels as one load
-  const bool vec = D % 4 == 0 && x_sb % 4 == 0 && x_sl % 4 == 0 && aligned_to(q, 16) && aligned_to(k, 16);
+  const bool vec = dc_vec(q, k, B, D, x_sb, x_sl);
   BASED_REQUIRE(vec || D <= 64, BASED_ERR_ALIGN, "%s: chunks of heads of more than 64 channels take rows of whole 16-byte pieces", who);
   const DeltaChunkArgs a{q, k, v, a_gate, b_gate, a_log, dt_bias, state, o, work, (long)dc_floats(dc_tiles(D), (int)DV), (int)B, (int)L, (int)H,
                          (int)G, (int)D, (int)DV, (int)state_row, 0, 0, x_sb, x_sl, g_sb, g_sl, fresh,
-                         DV % 4 == 0 && x_sb % 4 == 0 && x_sl % 4 == 0 && aligned_to(v, 16)};
+                         DV % 4 == 0 && (B == 1 || x_sb % 4 == 0) && x_sl % 4 == 0 && aligned_to(v, 16)};
   hipStream_t s = static_cast<hipStream_t>(stream);
   return io_dtype == BASED_BF16 ? run_delta<__bf16>(a, vec, span, s) : run_delta<float>(a, vec, span, s);
 }

@@ -724,7 +724,7 @@ NORM_RMS, NORM_LAYER, NORM_NONE = 0, 1, 2
 ACT_NONE, ACT_SILU, ACT_SIGMOID = 0, 1, 2
 STREAM_MAX_TAPS = 8  # BASED_STREAM_MAX_TAPS
 DELTA_BLOCK, DELTA_PREP_FLOATS = 16, 592  # tokens per block of based_gated_delta_scan, BASED_DELTA_PREP_FLOATS
-DELTA_CHUNKS_MIN = 256  # tokens from which on the library is asked whether chunks of 64 are the faster form
+DELTA_CHUNKS_MIN = 256  # BASED_DELTA_CHUNKS_MIN: shorter portions are not asked about
 RGLRU_SEGMENT = 64   # tokens per segment of based_rglru_prefill
 
 
@@ -936,9 +936,8 @@ def gated_delta_scan(q, k, v, a_gate, b_gate, a_log, dt_bias, state, heads: int,
     _check_delta(state, B, heads, d, dv)
     o = torch.empty(B, L, heads, dv, dtype=torch.float32, device=q.device)
     lib, floats = _lib.lib(), 0
-    if L >= DELTA_CHUNKS_MIN and q.stride(1) < 1 << 24 and heads * dv < 1 << 25 and (
-            d <= 64 or (d % 4 == 0 and q.stride(0) % 4 == 0 and q.stride(1) % 4 == 0 and q.data_ptr() % 16 == 0 and k.data_ptr() % 16 == 0)):
-        floats = lib.based_gated_delta_scan_work(B, L, heads, d, dv)
+    if L >= DELTA_CHUNKS_MIN:
+        floats = lib.based_gated_delta_scan_work_of(q.data_ptr(), k.data_ptr(), B, L, heads, d, dv, q.stride(0), q.stride(1))
     if floats:
         scan, work = lib.based_gated_delta_scan_chunks, torch.empty(floats, dtype=torch.float32, device=q.device)
     else:

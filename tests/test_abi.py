@@ -162,3 +162,28 @@ def test_decay_work_is_for_the_form_that_runs():
         for other in (dict(code=1), dict(code=0, q=4098), dict(code=0, pad=1)):
             assert of(B, L, H, D, DV, **other) == floats(general, B, H, D, DV), (B, L, other)
         assert lib.based_decay_scan_work(B, L, H, D, DV, 64) == floats(max(mfma, general), B, H, D, DV)
+
+
+def test_delta_chunks_take_the_rows_they_can():
+    """What the library says about tensors is what the chunks' entry takes: no rows off 16 bytes above 64 channels, none too long, and a
+    batch stride counts only where there is a batch."""
+    from based_amd import ops
+
+    lib = _lib.lib()
+
+    def of(B=1, L=640, H=4, D=128, DV=64, q=4096, k=8192, sb=640 * 1280, sl=1280):
+        return lib.based_gated_delta_scan_work_of(q, k, B, L, H, D, DV, sb, sl)
+
+    full = lib.based_gated_delta_scan_work(1, 640, 4, 128, 64)
+    assert of() == full > 0 and of(sb=640 * 1280 + 1) == full and of(B=2) > 0
+    for refused in (dict(B=2, sb=640 * 1280 + 1), dict(sl=1281), dict(q=4100), dict(k=8200), dict(sl=1 << 24), dict(L=100), dict(D=130)):
+        assert of(**refused) == 0, refused
+    assert of(D=64, sl=1281, q=4100) == lib.based_gated_delta_scan_work(1, 640, 4, 64, 64) > 0
+    header = open(os.path.join(ROOT, "include", "based_hip.h")).read()
+    assert int(re.search(r"#define BASED_DELTA_CHUNKS_MIN (\d+)", header).group(1)) == ops.DELTA_CHUNKS_MIN
+    for D in (8, 16, 32, 48, 64, 96, 128):  # what is not asked about would not be taken
+        assert lib.based_gated_delta_scan_work(1, ops.DELTA_CHUNKS_MIN - 1, 1, D, 16) == 0
+    p = ctypes.c_void_p(4096)
+    chunks = lambda L, D, sl: lib.based_gated_delta_scan_chunks(*([p] * 10), 1, L, 4, 4, D, 64, 64, L * sl, sl, 4, 4, 1, 0, None)  # noqa: E731
+    assert chunks(640, 132, 1280) == 1 and chunks(100, 128, 1280) == 1 and chunks(640, 128, 1 << 24) == 1  # BASED_ERR_SHAPE
+    assert chunks(640, 128, 1281) == 3  # BASED_ERR_ALIGN

@@ -145,3 +145,13 @@ def test_where_chunks_begin(dev, B, H, d, dv, first):
         o, S = run(case, H, H, d, dv, empty_state(B, H, d, dv, dev))
         ref, S_ref = reference(*case, H, H, d, dv)
         assert rel_l2(o, ref) < 3e-6 and rel_l2(S, S_ref) < 3e-6  # (the tolerance of the blocks)
+
+
+def test_batch_stride_of_one_sequence(dev):
+    """The stride of a batch of one is any number."""
+    H, d, dv, L = 2, 96, 32, 400
+    x, *gates = (t.to(dev) for t in make(6, 1, L, H, H, d, dv, torch.bfloat16))
+    x = x.as_strided(x.shape, (x.stride(0) + 1, x.stride(1), 1))
+    o, S = run((x, *gates), H, H, d, dv, empty_state(1, H, d, dv, dev))
+    ref, S_ref = reference(x, *gates, H, H, d, dv)
+    assert rel_l2(o, ref) < TOL and rel_l2(S, S_ref) < TOL
