@@ -49,6 +49,7 @@ struct PrefillF32Args {
   float eps;
   long seg_tokens;
   int n_seg, state_vec;
+  int heads, heads_z;  // B H, and those of one blockIdx.z
 };
 
 template <int T> __device__ __forceinline__ float row_ror_f32(float x) {  // value of lane (i - T) mod 16 of each 16
@@ -107,9 +108,10 @@ __global__ __launch_bounds__(256, 2) void lin_prefill_f32_kernel(const PrefillF3
   const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tiles = (a.dv + 15) / 16, groups = (tiles + 3) / 4;
-  const int bh = __builtin_amdgcn_readfirstlane(blockIdx.x / groups);
-  const int ct = (blockIdx.x - bh * groups) * 4 + wave;
-  if (ct >= tiles) return;  // (no barrier in this kernel)
+  const int head = __builtin_amdgcn_readfirstlane(blockIdx.x / groups);
+  const int ct = (blockIdx.x - head * groups) * 4 + wave;
+  const int bh = blockIdx.z * a.heads_z + head;
+  if (ct >= tiles || bh >= a.heads) return;  // (no barrier in this kernel)
   const int b = __builtin_amdgcn_readfirstlane(bh / a.H), h = bh - b * a.H, seg = blockIdx.y;
   const long begin = seg * a.seg_tokens, end = begin + a.seg_tokens < a.L ? begin + a.seg_tokens : a.L;
   const int ch = ct * 16 + l16;
@@ -449,18 +451,22 @@ static bool f32_vec_ok(const void* p, int64_t sb, int64_t sh, int64_t sl, int64_
   return reinterpret_cast<uintptr_t>(p) % (4 * elem) == 0 && sb % 4 == 0 && sh % 4 == 0 && sl % 4 == 0 && f32_near(sl);
 }
 
-template <typename T> static int launch_prefill_f32_as(const PrefillF32Args& a, int64_t BH, bool vec, hipStream_t s, const char* who) {
-  const int tiles = (a.dv + 15) / 16;
-  const unsigned wgs = (unsigned)(BH * ((tiles + 3) / 4));
+template <typename T> static int launch_prefill_f32_as(PrefillF32Args a, int64_t BH, bool vec, hipStream_t s, const char* who) {
+  // the groups of four channel tiles of a head are neighbours (a direction of their own: B = 4, H = 16, L = 1000, dv = 128 181 us, not
+  // 135); heads beyond what a launch has workgroups for in x go on in z
+  const int64_t groups = (a.dv + 63) / 64, most = ((1ll << 24) - 1) / groups;
+  a.heads = (int)BH;
+  a.heads_z = (int)(BH < most ? BH : most);
+  const unsigned wgs = (unsigned)(a.heads_z * groups), more = (unsigned)((BH + a.heads_z - 1) / a.heads_z);
   if (a.n_seg > 1) {
     auto delta = vec ? lin_prefill_f32_kernel<T, true, true> : lin_prefill_f32_kernel<T, false, true>;
-    hipLaunchKernelGGL(delta, dim3(wgs, (unsigned)(a.n_seg - (a.kv_state == nullptr))), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(delta, dim3(wgs, (unsigned)(a.n_seg - (a.kv_state == nullptr)), more), dim3(256), 0, s, a);
     const int rc = check_launch(who);
     if (rc) return rc;
   }
   auto whole = vec ? lin_prefill_f32_kernel<T, true, false> : lin_prefill_f32_kernel<T, false, false>;
   // (one workgroup more per head where the state is wanted: it starts behind the last segment)
-  hipLaunchKernelGGL(whole, dim3(wgs, (unsigned)(a.n_seg + (a.n_seg > 1 && a.kv_state != nullptr))), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(whole, dim3(wgs, (unsigned)(a.n_seg + (a.n_seg > 1 && a.kv_state != nullptr)), more), dim3(256), 0, s, a);
   return check_launch(who);
 }
 
@@ -469,7 +475,6 @@ int launch_prefill_f32(const char* who, const void* q, const void* k, const void
                        int64_t H, int64_t L, int64_t dv, int64_t q_sb, int64_t q_sh, int64_t q_sl, int64_t k_sb, int64_t k_sh, int64_t k_sl,
                        int64_t v_sb, int64_t v_sh, int64_t v_sl, int64_t y_sb, int64_t y_sh, int64_t y_sl, float eps, int io_dtype,
                        int64_t n_seg, float* ws, hipStream_t s) {
-  BASED_REQUIRE(B * H * ((dv + 63) / 64) < (1ll << 31), BASED_ERR_SHAPE, "%s: sizes too large", who);
   const int64_t chunks = (L + kF32Chunk - 1) / kF32Chunk, per = chunks > 0 ? (chunks + n_seg - 1) / n_seg : 1;
   const int64_t elem = io_dtype == BASED_BF16 ? 2 : 4;
   const PrefillF32Args a{q, k, v, y, kv_state, k_state, ws, (int)H, (int)L, (int)dv, q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl,

@@ -106,6 +106,18 @@ def test_infinite_values_stay_infinite(dev, value, split):
     assert bool(torch.isfinite(y).all())
 
 
+def test_as_many_heads_as_a_launch_takes(dev):
+    """2^23 heads of two groups of channel tiles: a single token is its own output."""
+    from based_amd import ops
+
+    B, H, dv = 1 << 19, 16, 65
+    q = torch.randn(B, H, 1, 16, device=dev)
+    v = torch.randn(B, H, 1, dv, device=dev)
+    y = ops.linear_attn_prefill(q, q, v)[0]
+    for part in (slice(0, 64), slice(B // 2 - 32, B // 2 + 32), slice(B - 64, B)):
+        assert rel_l2(y[part], v[part]) < TOL
+
+
 def test_refused_as_before(dev):
     from based_amd import ops
 
