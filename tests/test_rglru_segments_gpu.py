@@ -87,3 +87,43 @@ def test_narrow_blocks(dev, dtype, L, W, blocks):
 def test_groups_of_segments(dev, L):
     """Lengths around one, two and three groups of 64 segments."""
     test_rglru_segments(dev, torch.float32, L, 20, 1, "own", True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("over", [False, True])
+def test_replays(dev, dtype, over):
+    """A recorded portion of two groups of segments: every replay starts its tickets and words anew, with eager portions in between."""
+    from based_amd import ops
+
+    B, L, W, n = 2, 4200, 128, 64
+    g = torch.Generator().manual_seed(77)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).to(dev)  # noqa: E731
+    gates = (rnd(2, n, n) * n ** -0.5, rnd(W), rnd(2, n, n) * n ** -0.5, rnd(W), rnd(W) - 3)
+    inputs = [(rnd(B, L, W), rnd(B, L, W), torch.randn(B, W, generator=g).to(dev)) for _ in range(3)]
+
+    def run(u, y, state, out):
+        return ops.rglru_prefill(u, y, *gates, state, 8.0, False, out=u if over else out)
+
+    want = []
+    for u, y, state in inputs:
+        u, state = u.clone(), state.clone()
+        want.append((run(u, y, state, torch.empty_like(u)).clone(), state))
+    u, y, state, out = torch.empty_like(inputs[0][0]), torch.empty_like(inputs[0][1]), torch.empty(B, W, device=dev), torch.empty_like(inputs[0][0])
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        run(u.zero_(), y.zero_(), state.zero_(), out)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        res = run(u, y, state, out)
+    for i in (0, 1, 2, 0, 2):
+        for t, x in zip((u, y, state), inputs[i]):
+            t.copy_(x)
+        if not over:
+            out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(res, want[i][0]) and torch.equal(state, want[i][1]), i
+        eager = run(inputs[1][0].clone(), inputs[1][1], inputs[1][2].clone(), torch.empty_like(out))
+        assert torch.equal(eager, want[1][0])
