@@ -43,6 +43,9 @@ __device__ __forceinline__ float wave_sum(float x) {
   return x;
 }
 
+// fp32 products and sums on the matrix cores: a (16 x 4), b (4 x 16), c (column = lane % 16, row = 4 (lane / 16) + i)
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
 // Error reporting shared by the C entry points (thread-local last-error string).
 void set_error(const char* fmt, ...);
 

@@ -12,8 +12,6 @@ template <typename T> __device__ __forceinline__ float log_decay_of(float a, con
   return -expf(to_f32(static_cast<const T*>(a_log)[h])) * dt;
 }
 
-__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-
 // 4 consecutive channels of a row of d as they lie in memory.  Fetched without a condition (channels
 // past the end come from the row's start) and cleared where they are used: a load in a branch or
 // in front of a select is waited for on the spot.  LAY: 0 element by element, 1 whole aligned groups, 2 whole

@@ -56,8 +56,6 @@ template <int T> __device__ __forceinline__ float row_ror_f32(float x) {  // val
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x120 + T, 0xf, 0xf, false));
 }
 
-__device__ __forceinline__ f32x4 mma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-
 template <typename T, bool VEC> __device__ __forceinline__ f32x4 load_four(const T* p) {
   typedef __attribute__((ext_vector_type(4))) T t4;
   t4 r;
@@ -191,7 +189,7 @@ __global__ __launch_bounds__(256, 2) void lin_prefill_f32_kernel(const PrefillF3
         psi_key(c.k[kt][i], l16, p);
 #pragma unroll
         for (int t = 0; t < kF32Tiles; ++t) {
-          S[t] = mma_f32(p[t], c.v[kt][i], S[t]);
+          S[t] = mfma_f32(p[t], c.v[kt][i], S[t]);
           zsum[t] += p[t];
         }
       }
@@ -276,7 +274,7 @@ __global__ __launch_bounds__(256, 2) void lin_prefill_f32_kernel(const PrefillF3
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int kt = 0; kt <= m; ++kt) A[kt] = mma_f32(rows[kt][i], x[i], A[kt]);
+          for (int kt = 0; kt <= m; ++kt) A[kt] = mfma_f32(rows[kt][i], x[i], A[kt]);
         float z = 0.f;
 #pragma unroll
         for (int kt = 0; kt <= m; ++kt)
@@ -309,7 +307,7 @@ __global__ __launch_bounds__(256, 2) void lin_prefill_f32_kernel(const PrefillF3
               z = __builtin_fmaf(p, zt[i], z);
               // (slots without a feature hold zero times every value, which an infinity made a NaN)
               const float st = t == 8 ? (quad < 2 || (quad == 2 && i == 0) ? S[t][i] : 0.f) : S[t][i];
-              o[i & 1] = mma_f32(p, st, o[i & 1]);
+              o[i & 1] = mfma_f32(p, st, o[i & 1]);
             }
           }
         }
@@ -338,7 +336,7 @@ __global__ __launch_bounds__(256, 2) void lin_prefill_f32_kernel(const PrefillF3
             }
           } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o[i & 1] = mma_f32(A[kt][i], c.v[kt][i], o[i & 1]);
+            for (int i = 0; i < 4; ++i) o[i & 1] = mfma_f32(A[kt][i], c.v[kt][i], o[i & 1]);
           }
         }
         z += __shfl_xor(z, 16, 64);

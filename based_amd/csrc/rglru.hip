@@ -50,7 +50,7 @@ template <> struct GateMma<float> {
   typedef float frag_t;
   static constexpr int kPer = 1;
   static __device__ __forceinline__ f32x4 run(frag_t a, frag_t b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    return mfma_f32(a, b, c);
   }
 };
 
@@ -80,14 +80,15 @@ __global__ __launch_bounds__(256) void rglru_begin_kernel(unsigned long long* ag
 
 // grid: x = segments of the sequence, y = 64-channel tile within its block (ceil(n / 64) per block), z = sequence.
 // A workgroup takes the next segment of its tile and sequence, forms the gates of 64 tokens, leaves what they do to any state that enters
-// them for the segments behind, and takes the state that enters its own from those in front.  It waits for them only after its own is
-// left; they were taken before it by workgroups that run or have run, so each wait ends.  P and X travel in one 64-bit word, which is
-// its own flag.  The last of every kGroup segments leaves the state itself (P = 0) once it has it, and nobody reads behind that: at most
-// kGroup words a segment whatever the length (all those in front at 2,048 segments, B = 1, W = 1024: 1,920 us; 664 in groups; 73 and 66 at 16,384 tokens).  A
-// fixed place, not the nearest state that is there: the same sums on every run.  (Gates as fp32 pairs through memory for a second kernel, 134 of 184 MB at B = 4, L = 2048, W = 1024: 51 us; gates
-// formed by two kernels, 43 us: the vector unit is the bound, three exponentials, two reciprocals and a square root an element.)
-// The products lie with 16 consecutive tokens of a channel in one lane, where the recurrence is two instructions an element, and 64 in
-// a wavefront.  B = 4, L = 2048, W = 1024, 8 blocks: 29 us with the kernel in front; B = 8, L = 4096: 111 (237).
+// them for the segments behind, and takes the state that enters its own from those in front.  Those were taken before it by workgroups
+// that run or have run and that wait for none behind them, so each wait ends.  P and X travel in one 64-bit word, which is its own flag.
+// The last of every kGroup segments leaves the state itself (P = 0) instead, once it has it, and nobody reads behind that: at most kGroup
+// words a segment whatever the length (all those in front: 1,920 us for the 2,048 segments of B = 1, L = 131072, W = 1024 in bf16; in groups
+// 664; at L = 16384 73 and 66).  A fixed place, not the nearest state that is there: the same sums on every run.
+// Gates as fp32 pairs through memory for a second kernel, 134 of 184 MB at B = 4, L = 2048, W = 1024, 8 blocks, took 51 us; gates formed
+// by two kernels, 43 us: the vector unit is the bound, three exponentials, two reciprocals and a square root an element.  This way 28 us
+// with the kernel in front; B = 8, L = 4096: 92 (218).  The products lie with 16 consecutive tokens of a channel in one lane, where the
+// recurrence is two instructions an element, and 64 in a wavefront.
 template <typename T>
 __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_kernel(const RglruArgs a) {
   typedef GateMma<T> M;

@@ -407,8 +407,6 @@ __global__ __launch_bounds__(256, KC <= 3 && VC <= 2 ? 3 : 1) void window_prefil
 // B = 1, L = 777, with the cache write: 19 us (a wavefront per query on the vector unit: 70); B = 4, L = 2048: 81 us (661).
 constexpr int kF32Keys = 32, kF32Rows = 64;
 
-__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-
 // channels c .. c + 3 of a row, turned; c and the rotary size (its half in half-split pairs) multiples of 4
 __device__ __forceinline__ f32x4 turned4(const float* row, int c, int pos, const WindowArgs& a) {
   f32x4 x = *reinterpret_cast<const f32x4*>(row + c);
