@@ -91,6 +91,7 @@ def test_groups_of_segments(dev, L):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("over", [False, True])
+@torch.inference_mode()  # (torch keeps its generator's graph state in the mode of the process's first recording)
 def test_replays(dev, dtype, over):
     """A recorded portion of two groups of segments: every replay starts its tickets and words anew, with eager portions in between."""
     from based_amd import ops
