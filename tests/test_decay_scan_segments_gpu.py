@@ -141,3 +141,25 @@ def test_segments_of_several_pieces(dev, B, L, H, d, dv, dtype, channel):
                 ref[:, t] = (S * qt[..., None]).sum(2).flatten(1)
         # decays of 0.99 and 0.9995 keep a hundred to two thousand tokens: 2 * 2^-24 * 2000^0.5 = 5e-6; bf16 outputs add half of 2^-8
         assert rel(out, ref) < (5e-6 if dtype == torch.float32 else 3e-3) and rel(state[..., :d], S.transpose(2, 3)) < 5e-6
+
+
+@pytest.mark.parametrize("channel", [True, False])
+def test_infinite_states_outlive_segments(dev, channel):
+    """An infinity times decays that are small, none of them zero, stays one, however small their product; times zero it is no number."""
+    from based_amd import ops
+
+    H, d, dv, L = 2, 20, 17, 300
+    g = torch.Generator().manual_seed(3)
+    q, k, v, u = (torch.randn(*s, generator=g).to(dev) for s in ((1, L, H * d), (1, L, H * d), (1, L, H * dv), (H, d)))
+    lw = torch.full((1, L, H, d), -9.0)
+    lw[:, 100, 1] = float("-inf")
+    kw = dict(channel_log2=lw.flatten(2).to(dev), bonus=u) if channel else dict(head_decay=ops.head_decays([2.0 ** -9, 0.0], dev))
+    state = torch.zeros(1, H, dv, d, device=dev)
+    state[:, :, 3, 5] = float("inf")
+    state[:, :, 4, 5] = float("-inf")
+    out = ops.decay_scan(q, k, v, state, H, fresh=False, **kw).view(1, L, H, dv)
+    assert state[0, 0, 3, 5] == float("inf") and state[0, 0, 4, 5] == float("-inf")
+    assert state[0, 1, 3, 5].isnan() and state[0, 1, 4, 5].isnan()
+    assert out[:, :, 0, 3].isinf().all() and out[:, :, 0, 4].isinf().all() and out[:, 101:, 1, 3].isnan().all()
+    state[:, :, 3:5, 5], out[..., 3:5] = 0, 0
+    assert state.isfinite().all() and out.isfinite().all()
