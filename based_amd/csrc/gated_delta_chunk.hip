@@ -15,8 +15,8 @@
 //
 // Against blocks of 16 (gated_delta_scan_kernel) a chain step takes in four times the tokens with two exchanges instead of one, and
 // nothing but W S0 and k^T U stands in the chain.  Products per 64 tokens, d = 64, dv = 128: 3.9 -> 7.9 M fp32 operations in all, of
-// which 3.9 M in the scan.  4 sequences x 8 heads of 2048 tokens: 163 -> 95 us, 38 of preparation (written back at 2.5 TB/s, matrix pipe
-// a third busy) and 56 of scan (a lone workgroup per compute unit: 2.0 of 4.1 thousand cycles a chunk are products, the rest waits for
+// which 3.9 M in the scan.  4 sequences x 8 heads of 2048 tokens: 161 -> 91 us; traced, 41 of preparation (written back at 2.3 TB/s, matrix
+// pipe a third busy) and 55 of scan (a lone workgroup per compute unit: 2.0 of 4.1 thousand cycles a chunk are products, the rest waits for
 // accumulators, LDS and barriers; eight wavefronts with the outputs apart from the chain take 60).
 #include "gated_delta.hpp"
 
