@@ -1272,7 +1272,8 @@ static bool window_vec(const WindowArgs& a, int n) {
 
 // fp32 rows in 16-byte pieces that are turned whole; 64 rows to a workgroup of 256 threads, of which a launch takes 2^32.
 static bool window_f32(const WindowArgs& a, int io_dtype) {
-  return io_dtype == BASED_F32 && (long)a.L * (a.H / a.G) < (1l << 30) - kF32Rows && a.d <= 128 && a.dv <= 128 && a.rot % (a.half_split ? 8 : 4) == 0 && a.d % 4 == 0 && a.dv % 4 == 0 &&
+  return io_dtype == BASED_F32 && (long)a.L * (a.H / a.G) < (1l << 30) - kF32Rows && a.d <= 128 && a.dv <= 128 &&
+         a.rot % (a.half_split ? 8 : 4) == 0 && a.d % 4 == 0 && a.dv % 4 == 0 &&
          a.q_sb % 4 == 0 && a.q_sl % 4 == 0 && a.o_sb % 4 == 0 && a.o_sl % 4 == 0 && a.kv_sb % 4 == 0 && a.kv_st % 4 == 0 &&
          aligned_to(a.q, 16) && aligned_to(a.kv, 16) && aligned_to(a.o, 16);
 }
