@@ -25,8 +25,6 @@
 //     also what lies between.
 // fp32 numbers enter a bf16 product as pairs (a number rounded to bf16, and the rest rounded to bf16), so
 // an operand keeps 16 bits and the sums 24.
-#include <initializer_list>
-
 #include "stream_common.hpp"
 
 namespace based {
@@ -1024,15 +1022,9 @@ static int decay_any_segments(int64_t B, int64_t L, int64_t H, int64_t D, int64_
   return (int)((chunks + each - 1) / each);
 }
 
-// Whether the MFMA form takes a call: bf16 in whole 8-byte pieces.
-static bool decay_vec(const void* q, const void* k, const void* v, const float* channel_log2, const void* bonus, const void* o, int64_t D,
-                      int64_t DV, std::initializer_list<int64_t> strides, int io_dtype) {
-  if (io_dtype != BASED_BF16 || D > 128 || D % 4 != 0 || DV % 4 != 0 || !aligned_to(channel_log2, 16)) return false;
-  for (const int64_t s : strides)
-    if (s % 4 != 0) return false;
-  for (const void* p : {q, k, v, bonus, o})
-    if (!aligned_to(p, 8)) return false;
-  return true;
+// Whether the MFMA form takes a call: bf16 in whole 8-byte pieces (bits as based_decay_scan_work_of has them).
+static bool decay_vec(int64_t bits, int64_t D, int64_t DV, int io_dtype) {
+  return io_dtype == BASED_BF16 && D <= 128 && D % 4 == 0 && DV % 4 == 0 && bits % 8 == 0;
 }
 
 static int64_t decay_work(int64_t segs, int64_t B, int64_t H, int64_t DV, int64_t state_row) {
@@ -1047,14 +1039,11 @@ extern "C" BASED_API int64_t based_decay_scan_work(int64_t B, int64_t L, int64_t
   return based::decay_work(mfma > any ? mfma : any, B, H, DV, state_row);
 }
 
-extern "C" BASED_API int64_t based_decay_scan_work_of(const void* q, const void* k, const void* v, const float* channel_log2, const void* bonus,
-                                                      const void* o, int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV,
-                                                      int64_t state_row, int64_t q_sb, int64_t q_sl, int64_t k_sb, int64_t k_sl,
-                                                      int64_t v_sb, int64_t v_sl, int64_t o_sb, int64_t o_sl, int io_dtype) {
+extern "C" BASED_API int64_t based_decay_scan_work_of(int64_t bits, int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, int64_t state_row,
+                                                      int io_dtype) {
   using namespace based;
-  if (B <= 0 || L <= 0 || H <= 0 || D <= 0 || DV <= 0) return 0;
-  const bool vec = decay_vec(q, k, v, channel_log2, bonus, o, D, DV, {q_sb, q_sl, k_sb, k_sl, v_sb, v_sl, o_sb, o_sl}, io_dtype);
-  return decay_work(vec ? decay_segments(B, L, H, D, DV) : decay_any_segments(B, L, H, D, DV), B, H, DV, state_row);
+  if (B <= 0 || L < BASED_DECAY_SEGMENTS_MIN || H <= 0 || D <= 0 || DV <= 0) return 0;
+  return decay_work(decay_vec(bits, D, DV, io_dtype) ? decay_segments(B, L, H, D, DV) : decay_any_segments(B, L, H, D, DV), B, H, DV, state_row);
 }
 
 extern "C" BASED_API int based_decay_scan(const void* q, const void* k, const void* v, const float* channel_log2, const float* head_decay,
@@ -1079,7 +1068,9 @@ extern "C" BASED_API int based_decay_scan(const void* q, const void* k, const vo
                   (int)state_row, q_sb, q_sl, k_sb, k_sl, v_sb, v_sl, o_sb, o_sl, 1, (int)((L + kScanTokens - 1) / kScanTokens),
                   activation == BASED_ACT_SILU, fresh};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool vec = decay_vec(q, k, v, channel_log2, bonus, o, D, DV, {q_sb, q_sl, k_sb, k_sl, v_sb, v_sl, o_sb, o_sl}, io_dtype);
+  const auto at = [](const void* p) { return (int64_t)reinterpret_cast<uintptr_t>(p); };
+  const int64_t bits = (at(q) | at(k) | at(v) | at(bonus) | at(o)) | 2 * (q_sb | q_sl | k_sb | k_sl | v_sb | v_sl | o_sb | o_sl) | at(channel_log2) / 2;
+  const bool vec = decay_vec(bits, D, DV, io_dtype);
   const int segs = vec ? decay_segments(B, L, H, D, DV) : work != nullptr ? decay_any_segments(B, L, H, D, DV) : 1;
   if (segs > 1) {
     BASED_REQUIRE(work != nullptr, BASED_ERR_ARG, "decay_scan: no work space");

@@ -725,6 +725,7 @@ ACT_NONE, ACT_SILU, ACT_SIGMOID = 0, 1, 2
 STREAM_MAX_TAPS = 8  # BASED_STREAM_MAX_TAPS
 DELTA_BLOCK, DELTA_PREP_FLOATS = 16, 592  # tokens per block of based_gated_delta_scan, BASED_DELTA_PREP_FLOATS
 DELTA_CHUNKS_MIN = 256  # BASED_DELTA_CHUNKS_MIN: shorter portions are not asked about
+DECAY_SEGMENTS_MIN = 193  # BASED_DECAY_SEGMENTS_MIN, likewise
 RGLRU_SEGMENT = 64   # tokens per segment of based_rglru_prefill
 
 
@@ -1185,17 +1186,20 @@ def decay_scan(q, k, v, state, heads: int, *, channel_log2=None, bonus=None, hea
         _check_head_decay(head_decay, heads, q.device)
     lib = _lib.lib()
     o = torch.empty(B, L, heads * dv, dtype=q.dtype, device=q.device)
+    sizes = (B, L, heads, d, dv, state.shape[3])
+    at = [q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(channel_log2), _ptr(bonus), o.data_ptr()]
+    strides = (*q.stride()[:2], *k.stride()[:2], *v.stride()[:2], L * heads * dv, heads * dv)
     work = None
-    if lib.based_decay_scan_work(B, L, heads, d, dv, state.shape[3]):
-        n = lib.based_decay_scan_work_of(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(channel_log2), _ptr(bonus), o.data_ptr(), B, L, heads, d, dv, state.shape[3],
-            q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1), o.stride(0), o.stride(1), _dtype_code(q))
+    if L >= DECAY_SEGMENTS_MIN:
+        bits = at[0] | at[1] | at[2] | (at[4] or 0) | at[5] | (at[3] or 0) >> 1
+        for x in strides:
+            bits |= 2 * x
+        n = lib.based_decay_scan_work_of(bits, *sizes, _dtype_code(q))
         work = torch.empty(n, dtype=torch.float32, device=q.device) if n else None
     with _on_device(q.device):
         _lib.check(lib.based_decay_scan(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(channel_log2), _ptr(head_decay), _ptr(bonus), state.data_ptr(), _ptr(work),
-            o.data_ptr(), B, L, heads, d, dv, state.shape[3], q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
-            o.stride(0), o.stride(1), int(activation), int(fresh), _dtype_code(q), _stream_ptr(q)))
+            *at[:4], _ptr(head_decay), at[4], state.data_ptr(), _ptr(work), at[5], *sizes, *strides, int(activation), int(fresh),
+            _dtype_code(q), _stream_ptr(q)))
     return o
 
 

@@ -636,12 +636,11 @@ BASED_API int based_token_side_step(const void* x, const float* residual_in, flo
  * and w itself:
  * S <- w S + k v^T, o = S^T q.  state (B, H, DV, state_row) fp32, by value channel; work: as many floats as
  * based_decay_scan_work_of says for the call (0: may be NULL), or based_decay_scan_work for any call of the sizes; without it, what is not
- * bf16 in whole 8-byte pieces is walked in one chain. */
+ * bf16 in whole 8-byte pieces is walked in one chain.  Both are 0 below BASED_DECAY_SEGMENTS_MIN tokens.  bits: the addresses of q, k, v,
+ * bonus and o, twice their strides and half the address of channel_log2, all of them or-ed. */
+#define BASED_DECAY_SEGMENTS_MIN 193
 BASED_API int64_t based_decay_scan_work(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, int64_t state_row);
-BASED_API int64_t based_decay_scan_work_of(const void* q, const void* k, const void* v, const float* channel_log2, const void* bonus,
-                                           const void* o, int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, int64_t state_row,
-                                           int64_t q_sb, int64_t q_sl, int64_t k_sb, int64_t k_sl, int64_t v_sb, int64_t v_sl, int64_t o_sb,
-                                           int64_t o_sl, int io_dtype);
+BASED_API int64_t based_decay_scan_work_of(int64_t bits, int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, int64_t state_row, int io_dtype);
 BASED_API int based_decay_scan(const void* q, const void* k, const void* v, const float* channel_log2, const float* head_decay,
                                const void* bonus, float* state, float* work, void* o, int64_t B, int64_t L, int64_t H,
                                int64_t D, int64_t DV, int64_t state_row, int64_t q_sb, int64_t q_sl, int64_t k_sb,

@@ -150,18 +150,26 @@ def test_decay_work_is_for_the_form_that_runs():
     """Aligned bf16 (the matrix form) asks for its own segments, everything else for those of the general form; one number covers both."""
     lib = _lib.lib()
 
-    def of(B, L, H, D, DV, code, q=4096, row=None, pad=0):
-        row = (D + 3) // 4 * 4
-        x = (L * (H * D + pad), H * D + pad)
-        return lib.based_decay_scan_work_of(q, 8192, 8192, 8192, 8192, 8192, B, L, H, D, DV, row, *x, *x, L * H * DV, H * DV, L * H * DV, H * DV, code)
+    def of(B, L, H, D, DV, code, q=4096, log2=4096, pad=0):
+        bits = q | 8192 | log2 // 2  # the addresses of the tensors, twice their strides
+        for stride in (L * (H * D + pad), H * D + pad, L * H * DV, H * DV):
+            bits |= 2 * stride
+        return lib.based_decay_scan_work_of(bits, B, L, H, D, DV, (D + 3) // 4 * 4, code)
 
     floats = lambda segs, B, H, D, DV: B * H * segs * (DV + 1) * ((D + 3) // 4 * 4)  # noqa: E731
     for B, L, H, D, DV, mfma, general in [(1, 256, 16, 64, 64, 0, 4), (1, 2048, 16, 64, 64, 8, 32), (4, 2048, 16, 64, 64, 8, 8),
                                           (1, 100, 16, 64, 64, 0, 0), (8, 320, 16, 64, 64, 0, 3), (64, 2048, 16, 64, 64, 0, 0)]:
         assert of(B, L, H, D, DV, 0) == floats(mfma, B, H, D, DV), (B, L)
-        for other in (dict(code=1), dict(code=0, q=4098), dict(code=0, pad=1)):
+        for other in (dict(code=1), dict(code=0, q=4098), dict(code=0, q=4100), dict(code=0, log2=4104), dict(code=0, pad=1), dict(code=0, pad=2)):
             assert of(B, L, H, D, DV, **other) == floats(general, B, H, D, DV), (B, L, other)
         assert lib.based_decay_scan_work(B, L, H, D, DV, 64) == floats(max(mfma, general), B, H, D, DV)
+    from based_amd import ops
+
+    header = open(os.path.join(ROOT, "include", "based_hip.h")).read()
+    least = int(re.search(r"#define BASED_DECAY_SEGMENTS_MIN (\d+)", header).group(1))
+    assert least == ops.DECAY_SEGMENTS_MIN
+    for D in (4, 64, 128, 256):  # what is not asked about would take none, and the least that takes some is asked about
+        assert lib.based_decay_scan_work(1, least - 1, 1, D, 4, D) == 0 and lib.based_decay_scan_work(1, least, 1, 64, 4, 64) > 0
 
 
 def test_delta_chunks_take_the_rows_they_can():
