@@ -574,10 +574,12 @@ __global__ __launch_bounds__(256) void decay_join_kernel(const DecayScanArgs a) 
 // ---- any element type and size ----
 // 16 lanes per value channel, groups of four channels of the key each; 16 value channels per workgroup.  Token by token, so what counts is
 // the length of the chain and the workgroups beside each other: long portions go in segments, as on MFMA.  fp32, B = 1, H = 16,
-// d = dv = 64, channel decays, L = 777: 47 us (one chain, four channels 16 apart to a lane: 230); L = 2048: 86 (715).
+// d = dv = 64, channel decays, L = 777: 43 us (one chain: 168); L = 2048: 80 (538).
+// A lane's four channels lie side by side: states are read and written in whole pieces (element by element, four accesses of a quarter
+// of each line: 32 x 4 heads of 256 x 256, L = 2, head decays, 17.8 us; 13.0 in pieces).
 // kTile tokens are staged at once: 16, a barrier pair for each, where all workgroups are on the GPU together anyway, and 8 where keys of
-// more than 128 channels would then keep some waiting for LDS.  fp32, H = 4, d = dv = 256, channel decays, 16 against 8: B = 64, L = 200:
-// 1,078 us, 798; B = 16, L = 300: 435, 300; B = 1, L = 300: 76, 82.
+// more than 128 channels would then keep some waiting for LDS, or where there are no more.  fp32, H = 4, d = dv = 256, channel decays, 16
+// against 8: B = 64, L = 200: 894 us, 710; B = 16, L = 300: 444, 285; B = 1, L = 300: 72, 78.  64 x 12 heads of 128, L = 1: 18.5, 16.3.
 template <typename T, int CPT, bool CHANNEL, bool STATE_ONLY, int kTile>
 __global__ __launch_bounds__(256) void decay_scan_any_kernel(const DecayScanArgs a) {
   constexpr int CH = 16 * CPT;
@@ -599,13 +601,19 @@ __global__ __launch_bounds__(256) void decay_scan_any_kernel(const DecayScanArgs
   static_assert(256 % CH == 0, "a thread stages one channel");
   const float head_w = CHANNEL ? 0.f : a.head_lw[a.H + h];
 #pragma unroll
-  for (int g = 0; g < CPT / 4; ++g)
+  for (int g = 0; g < CPT / 4; ++g) {
+    const int c0 = g * 64 + l16 * 4;
+    S[g] = !zero && col_in && c0 < a.d ? *reinterpret_cast<const f32x4*>(from + c0) : f32x4{0.f, 0.f, 0.f, 0.f};  // (rows are whole pieces)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int c = g * 64 + l16 * 4 + j;
-      S[g][j] = !zero && col_in && c < a.d ? from[c] : 0.f;
-      u[g][j] = CHANNEL && !STATE_ONLY && c < a.d ? to_f32(static_cast<const T*>(a.u)[(long)h * a.d + c]) : 0.f;
-    }
+    for (int j = 0; j < 4; ++j) S[g][j] = c0 + j < a.d ? S[g][j] : 0.f;
+  }
+  if constexpr (CHANNEL && !STATE_ONLY) {  // (rows of any alignment, through LDS)
+    __shared__ __attribute__((aligned(16))) float s_u[CH];
+    if (tid < CH) s_u[tid] = tid < a.d ? to_f32(static_cast<const T*>(a.u)[(long)h * a.d + tid]) : 0.f;
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < CPT / 4; ++g) u[g] = *reinterpret_cast<const f32x4*>(&s_u[g * 64 + l16 * 4]);
+  }
   auto active = [&](T x) { return a.silu ? round_to<T>(silu_exact(to_f32(x))) : to_f32(x); };
   const int begin = sg * a.seg_chunks * kScanTokens;
   const int end = sg < a.segs - 1 ? begin + a.seg_chunks * kScanTokens : a.L;
@@ -657,18 +665,21 @@ __global__ __launch_bounds__(256) void decay_scan_any_kernel(const DecayScanArgs
       }
     }
   }
+  // (what lies behind the last channel is not written)
+  if (STATE_ONLY ? col_in : col_in && sg == a.segs - 1) {
+    float* to = STATE_ONLY ? sgp : st;
 #pragma unroll
-  for (int g = 0; g < CPT / 4; ++g)
+    for (int g = 0; g < CPT / 4; ++g) {
+      const int c = g * 64 + l16 * 4;
+      if (c + 3 < a.d) {
+        *reinterpret_cast<f32x4*>(to + c) = S[g];
+      } else {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int c = g * 64 + l16 * 4 + j;
-      if (c >= a.d) continue;
-      if constexpr (STATE_ONLY) {
-        if (col_in) sgp[c] = S[g][j];
-      } else if (col_in && sg == a.segs - 1) {
-        st[c] = S[g][j];
+        for (int j = 0; j < 3; ++j)
+          if (c + j < a.d) to[c + j] = S[g][j];
       }
     }
+  }
   if constexpr (CHANNEL && STATE_ONLY) {
     // the power of a sum of logarithms loses less than a product of decays that were each rounded
     if (blockIdx.y != 0) return;
@@ -948,10 +959,9 @@ template <typename T, int CPT, bool CHANNEL, int TOKENS> void launch_decay_any_t
 }
 
 template <typename T, int CPT, bool CHANNEL> void launch_decay_any(const DecayScanArgs& a, hipStream_t s) {
-  if constexpr (CPT > 8) {
-    // workgroups that the LDS of 256 compute units holds with 16 tokens: three of 49 KB to one, or four of 33 KB
-    if ((long)a.B * a.H * ((a.dv + 15) / 16) * a.segs > (CHANNEL ? 768 : 1024)) return launch_decay_any_tile<T, CPT, CHANNEL, 8>(a, s);
-  }
+  // workgroups that the LDS of 256 compute units holds with 16 tokens: three of 49 KB to one, or four of 33 KB
+  const bool many = CPT > 8 && (long)a.B * a.H * ((a.dv + 15) / 16) * a.segs > (CHANNEL ? 768 : 1024);
+  if (many || a.L <= 8) return launch_decay_any_tile<T, CPT, CHANNEL, 8>(a, s);
   launch_decay_any_tile<T, CPT, CHANNEL, 16>(a, s);
 }
 
@@ -1007,18 +1017,17 @@ static int decay_segments(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV
 
 // The same for the general form: eight workgroups to a compute unit.  Every token but those of the last segment is walked twice, so the
 // chain is two segments long: three segments ask for a third less at best, and the launches.  Segments where four are wanted, of which
-// whole 64-token pieces may leave three.  us in segments against one chain, channel decays: B = 1, H = 12, L = 250: 37 in four, 77; 8 x 16
-// heads of 64, in three, L = 257: 82, 83; L = 320: 86, 103; L = 384: 100, 121.  Keys of more than 64 channels gain only where the two
-// segments are the shorter chain by more than the launches: 16 x 4 heads of 128, L = 257: 127, 114; L = 320: 133, 145; 8 x 4 heads of 256
-// (head decays), L = 257: 181, 158; L = 320: 194, 225.
-static int decay_any_segments(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
+// whole 64-token pieces may leave three, if the two are the shorter chain by more than the launches.  us in segments against one chain,
+// channel decays: B = 1, H = 12, L = 250: 31 in four, 57; 8 x 16 heads of 64, in three, L = 257: 75, 73; L = 320: 78, 87; L = 384: 91, 105;
+// 16 x 4 heads of 128, in three, L = 290: 121, 123; L = 320: 123, 127; 8 x 4 heads of 256 (head decays), L = 320: 177, 200.
+static int decay_any_segments(int64_t B, int64_t L, int64_t H, int64_t DV) {
   const int64_t chunks = (L + kScanTokens - 1) / kScanTokens, wgs = B * H * ((DV + 15) / 16);
   int64_t segs = (2048 + wgs - 1) / wgs;
   if (segs > chunks) segs = chunks;
   if (segs > 64) segs = 64;
   if (segs < 4) return 1;
   const int64_t each = (chunks + segs - 1) / segs;
-  if (D > 64 && 2 * each * kScanTokens + 16 > L) return 1;
+  if (2 * each * kScanTokens + 16 > L) return 1;
   return (int)((chunks + each - 1) / each);
 }
 
@@ -1035,7 +1044,7 @@ static int64_t decay_work(int64_t segs, int64_t B, int64_t H, int64_t DV, int64_
 
 extern "C" BASED_API int64_t based_decay_scan_work(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, int64_t state_row) {
   if (B <= 0 || L <= 0 || H <= 0 || D <= 0 || DV <= 0) return 0;
-  const int64_t mfma = based::decay_segments(B, L, H, D, DV), any = based::decay_any_segments(B, L, H, D, DV);
+  const int64_t mfma = based::decay_segments(B, L, H, D, DV), any = based::decay_any_segments(B, L, H, DV);
   return based::decay_work(mfma > any ? mfma : any, B, H, DV, state_row);
 }
 
@@ -1043,7 +1052,7 @@ extern "C" BASED_API int64_t based_decay_scan_work_of(int64_t bits, int64_t B, i
                                                       int io_dtype) {
   using namespace based;
   if (B <= 0 || L < BASED_DECAY_SEGMENTS_MIN || H <= 0 || D <= 0 || DV <= 0) return 0;
-  return decay_work(decay_vec(bits, D, DV, io_dtype) ? decay_segments(B, L, H, D, DV) : decay_any_segments(B, L, H, D, DV), B, H, DV, state_row);
+  return decay_work(decay_vec(bits, D, DV, io_dtype) ? decay_segments(B, L, H, D, DV) : decay_any_segments(B, L, H, DV), B, H, DV, state_row);
 }
 
 extern "C" BASED_API int based_decay_scan(const void* q, const void* k, const void* v, const float* channel_log2, const float* head_decay,
@@ -1069,9 +1078,10 @@ extern "C" BASED_API int based_decay_scan(const void* q, const void* k, const vo
                   activation == BASED_ACT_SILU, fresh};
   hipStream_t s = static_cast<hipStream_t>(stream);
   const auto at = [](const void* p) { return (int64_t)reinterpret_cast<uintptr_t>(p); };
-  const int64_t bits = (at(q) | at(k) | at(v) | at(bonus) | at(o)) | 2 * (q_sb | q_sl | k_sb | k_sl | v_sb | v_sl | o_sb | o_sl) | at(channel_log2) / 2;
+  const int64_t strides = q_sb | q_sl | k_sb | k_sl | v_sb | v_sl | o_sb | o_sl;
+  const int64_t bits = at(q) | at(k) | at(v) | at(bonus) | at(o) | 2 * strides | at(channel_log2) / 2;
   const bool vec = decay_vec(bits, D, DV, io_dtype);
-  const int segs = vec ? decay_segments(B, L, H, D, DV) : work != nullptr ? decay_any_segments(B, L, H, D, DV) : 1;
+  const int segs = vec ? decay_segments(B, L, H, D, DV) : work != nullptr ? decay_any_segments(B, L, H, DV) : 1;
   if (segs > 1) {
     BASED_REQUIRE(work != nullptr, BASED_ERR_ARG, "decay_scan: no work space");
     a.seg_chunks = (a.seg_chunks + segs - 1) / segs;

@@ -158,7 +158,7 @@ def test_decay_work_is_for_the_form_that_runs():
 
     floats = lambda segs, B, H, D, DV: B * H * segs * (DV + 1) * ((D + 3) // 4 * 4)  # noqa: E731
     for B, L, H, D, DV, mfma, general in [(1, 256, 16, 64, 64, 0, 4), (1, 2048, 16, 64, 64, 8, 32), (4, 2048, 16, 64, 64, 8, 8),
-                                          (1, 100, 16, 64, 64, 0, 0), (8, 320, 16, 64, 64, 0, 3), (64, 2048, 16, 64, 64, 0, 0)]:
+                                          (1, 100, 16, 64, 64, 0, 0), (8, 257, 16, 64, 64, 0, 0), (8, 320, 16, 64, 64, 0, 3), (64, 2048, 16, 64, 64, 0, 0)]:
         assert of(B, L, H, D, DV, 0) == floats(mfma, B, H, D, DV), (B, L)
         for other in (dict(code=1), dict(code=0, q=4098), dict(code=0, q=4100), dict(code=0, log2=4104), dict(code=0, pad=1), dict(code=0, pad=2)):
             assert of(B, L, H, D, DV, **other) == floats(general, B, H, D, DV), (B, L, other)

@@ -106,7 +106,7 @@ def test_long_keys_in_many_workgroups(dev, B, L, d):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("B,L,H,d,dv", [(4, 1023, 16, 64, 64), (4, 1025, 16, 64, 64),            # eight or nine segments of two pieces
                                         (1, 64 * 64 + 70, 1, 20, 17), (2, 64 * 130 + 1, 1, 8, 4),  # 33 of two, 44 of three
-                                        (8, 257, 16, 64, 64), (8, 320, 16, 20, 64),                # three of two, the last of one token or a piece
+                                        (8, 257, 16, 64, 64), (8, 320, 16, 20, 64),                # one chain, and three of two, the last of a piece
                                         (8, 271, 16, 68, 60), (8, 272, 16, 68, 60)])               # one chain, and three
 def test_segments_of_several_pieces(dev, B, L, H, d, dv, dtype, channel):
     """Segments longer than a 64-token piece, the last one shorter than the others: fresh, and from a state that goes on."""
@@ -163,3 +163,41 @@ def test_infinite_states_outlive_segments(dev, channel):
     assert out[:, :, 0, 3].isinf().all() and out[:, :, 0, 4].isinf().all() and out[:, 101:, 1, 3].isnan().all()
     state[:, :, 3:5, 5], out[..., 3:5] = 0, 0
     assert state.isfinite().all() and out.isfinite().all()
+
+
+@pytest.mark.parametrize("channel", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("L,d", [(1, 3), (1, 17), (8, 64), (9, 66), (8, 101), (9, 128), (1, 130), (8, 255), (9, 256)])
+def test_few_tokens(dev, L, d, dtype, channel):
+    """Portions of one piece of tokens and one more; states in rows of 16-byte pieces whose rest stays as it is, bonuses of any alignment."""
+    from based_amd import ops
+
+    B, H, dv = 2, 3, 21
+    g = torch.Generator().manual_seed(L + d)
+    dp = (d + 3) // 4 * 4
+    q, k, v = (torch.randn(B, L, H * n + 1, generator=g).to(dtype).to(dev)[..., 1:] for n in (d, d, dv))
+    u = torch.randn(H, d, generator=g).to(dtype).to(dev)
+    lw = -torch.exp(torch.randn(B, L, H * d, generator=g) - 2).to(dev)
+    decay = [0.9, 0.99, 0.5]
+    kw = dict(channel_log2=lw, bonus=u) if channel else dict(head_decay=ops.head_decays(decay, dev))
+    S0 = torch.full((B, H, dv, dp), float("nan"))
+    S0[..., :d] = torch.randn(B, H, dv, d, generator=g)
+    rel = lambda a, b: ((a.double() - b).norm() / b.norm()).item()  # noqa: E731
+    for fresh in (True, False):
+        state = S0.to(dev)
+        out = ops.decay_scan(q, k, v, state, H, fresh=fresh, **kw)
+        S = torch.zeros(B, H, d, dv, dtype=torch.float64, device=dev) if fresh else S0[..., :d].double().transpose(2, 3).to(dev)
+        w = torch.tensor(decay, dtype=torch.float32).double().view(1, H, 1, 1).to(dev)
+        ref = torch.empty(B, L, H * dv, dtype=torch.float64, device=dev)
+        for t in range(L):
+            qt, kt, vt = (x[:, t].double().view(B, H, -1) for x in (q, k, v))
+            kv = kt[..., None] * vt[:, :, None]
+            if channel:
+                ref[:, t] = ((S + u.double()[..., None] * kv) * qt[..., None]).sum(2).flatten(1)
+                S = 2.0 ** lw[:, t].double().view(B, H, d, 1) * S + kv
+            else:
+                S = w * S + kv
+                ref[:, t] = (S * qt[..., None]).sum(2).flatten(1)
+        # sums of up to 256 products of 2^-24 each, independent: 16 * 2^-24 = 1e-6; bf16 outputs add half of 2^-8
+        assert rel(out, ref) < (1e-6 if dtype == torch.float32 else 3e-3) and rel(state[..., :d], S.transpose(2, 3)) < 1e-6
+        assert state[..., d:].isnan().all()
