@@ -1278,6 +1278,23 @@ static bool window_f32(const WindowArgs& a, int io_dtype) {
          aligned_to(a.q, 16) && aligned_to(a.kv, 16) && aligned_to(a.o, 16);
 }
 
+// Portions of few rows stay with the general form: a wavefront per query, each on its own way through the keys.  The matrix form takes 68 ns
+// a key whatever the rows and the sizes up to 64 (values above 64 channels, keys above: 20 more each), the general one 36 + 0.45 d (values
+// above 64 channels: 30 more) as long as an L2 holds the keys that it reads, and more with every thousand rows.  General over matrix form,
+// 129 to 2,048 keys, by d x dv: 16 x 16, 300 rows 0.62, 2,600 0.92; 24 x 24, 1,800 0.92; 32 x 32, 300 0.83, 900 0.90, 1,300 0.95, above 4 MB
+// of keys and values 1.2 to 1.6; 48 x 48, 600 0.92, 900 0.98; 64 x 64, 300 0.96, 600 1.00; 16 x 128, 300 0.93, 900 0.99; 32 x 128, 300 0.97,
+// 600 1.00; 64 x 128, 16 1.08; 80 x 80, 600 0.92; 96 x 32, 600 0.88, 900 1.00; 96 x 96, 160 0.97; 128 x 64, 300 0.95; 128 x 128, 160 1.02.
+static bool window_f32_few(const WindowArgs& a) {
+  const long rows = (long)a.B * a.L * a.H, end = (long)a.pos_host + a.L, seen = a.window < end ? a.window : end;
+  const long keys = seen + a.L - 1 < end ? seen + a.L - 1 : end, bytes = keys * a.B * a.G * (a.d + a.dv) * 4;
+  const bool narrow = a.d <= 32 && a.dv <= 32;
+  const long room = a.d <= 16 && a.dv <= 16 ? 32 : rows <= 16 ? 12 : narrow && a.L <= 3 ? 8 : 4;
+  if (bytes > room << 20) return false;
+  if (seen <= 64 && a.d > 64) return rows <= 512;  // (a workgroup's 64 rows span more keys than a row sees: 4 x 96, L = 200, 16 keys: 13.5 us, 15.8)
+  if (a.dv > 64) return rows <= (a.d <= 16 ? 500 : a.d <= 32 ? 250 : a.d <= 64 ? 0 : a.d + a.dv <= 160 ? 512 : a.d + a.dv <= 192 ? 256 : 0);
+  return rows <= (a.d <= 16 ? 2600 : a.d <= 24 ? 2000 : a.d <= 32 ? 1000 : a.d <= 48 ? 700 : a.d <= 64 ? 400 : a.d <= 96 ? 700 : 350);
+}
+
 // The attention of a portion whose keys and values are in place.
 static void launch_window_attend(const WindowArgs& a, bool vec, int io_dtype, hipStream_t s) {
   if (vec) {
@@ -1293,7 +1310,7 @@ static void launch_window_attend(const WindowArgs& a, bool vec, int io_dtype, hi
       launch_window_mfma<4>(a, grid, s);
     else
       launch_window_mfma<8>(a, grid, s);
-  } else if (window_f32(a, io_dtype)) {
+  } else if (window_f32(a, io_dtype) && !window_f32_few(a)) {
     const dim3 grid((unsigned)(((long)a.L * (a.H / a.G) + kF32Rows - 1) / kF32Rows), (unsigned)(a.B * a.G));
     if (a.d <= 64 && a.dv <= 64)
       hipLaunchKernelGGL((window_prefill_f32_kernel<1, 1>), grid, dim3(256), 0, s, a);

@@ -82,3 +82,21 @@ def test_scale_of_zero(dev, bad, shift):
     assert out[:, sees][:, :, :2].isnan().all()
     mean = torch.stack([v[0, max(0, t - window + 1):t + 1].double().mean(0) for t in range(L)])[None].repeat_interleave(H // G, 2)
     assert torch.allclose(out[:, ~sees], mean[:, ~sees], rtol=0, atol=1e-6) and torch.allclose(out[:, :, 2:], mean[:, :, 2:], rtol=0, atol=1e-6)
+
+
+@pytest.mark.parametrize("d,dv,H,G,L,start,window", [
+    (4, 4, 16, 4, 100, 0, 200), (8, 64, 16, 1, 90, 30, 64), (16, 16, 16, 16, 90, 20, 300), (24, 24, 16, 4, 70, 0, 33), (32, 32, 8, 2, 70, 10, 129),
+    (48, 20, 6, 2, 65, 0, 40), (64, 64, 4, 4, 60, 40, 70), (64, 32, 16, 4, 16, 100, 90), (12, 128, 4, 1, 70, 0, 50), (32, 100, 2, 2, 70, 5, 64),
+    (64, 128, 1, 1, 17, 0, 9), (80, 80, 4, 2, 70, 20, 100), (96, 32, 8, 8, 50, 0, 90), (96, 96, 2, 2, 70, 0, 128), (128, 64, 4, 1, 50, 7, 66),
+    (128, 128, 4, 4, 70, 0, 33), (100, 40, 16, 16, 20, 40, 16)])
+def test_both_sides_of_the_rule_for_few_rows(dev, d, dv, H, G, L, start, window):
+    """Batches on either side of the number of rows from which on the matrix form runs: two of them, and eight times as many."""
+    for B in (1, 2, 16):
+        g = torch.Generator().manual_seed(d + dv)
+        q, k, v = (torch.randn(B, start + L, n, m, generator=g) for n, m in ((H, d), (G, d), (G, dv)))
+        out = _run(dev, q, k, v, window, d ** -0.5, start, None, 0)
+        rows = slice(0, B, max(1, B - 1))  # the first and the last sequence
+        ref = torch.stack([O.window_softmax(qq.double(), kk.double(), vv.double(), d ** -0.5, window) for qq, kk, vv in
+                           zip(q[rows], k[rows], v[rows])])[:, start:]
+        err = (out[rows] - ref).norm(dim=-1) / ref.norm(dim=-1)
+        assert float(err.max()) < 3e-6, (B, float(err.max()))  # (scores of up to 5 and sums of 128 products)
