@@ -59,6 +59,9 @@ __device__ __forceinline__ void plan_tiles(const int* counts, int* scan, int* fi
   __syncthreads();
 }
 
+// A score is no less than zero; less is what stays where all that is left to choose from are no numbers, and the choice is none either.
+__device__ __forceinline__ float chosen_score(float best) { return best < 0.f ? __builtin_nanf("") : best; }
+
 // ET: tiles of 16 experts (bf16 MFMA); 0: element by element.  NW wavefronts.  SPLIT: they share 16 TT tokens, a part of the row each;
 // otherwise 16 tokens each.
 template <typename T, int ET, int NW, bool SPLIT, int TT>
@@ -163,7 +166,7 @@ __global__ __launch_bounds__(64 * NW) void expert_route_kernel(const RouteArgs a
       if (sub == 0 && t < n) {
         const long slot = (n0 + t) * a.top + j;
         a.ids[slot] = at;
-        a.scores[slot] = best;
+        a.scores[slot] = chosen_score(best);
         if (a.rank != nullptr) a.rank[slot] = atomicAdd(&hist[at], 1);
       }
     }
@@ -281,7 +284,7 @@ __global__ __launch_bounds__(512) void expert_route_row_kernel(const RouteRowArg
   if (wave != 0) return;
   float mine[kMaxExperts / 64];
 #pragma unroll
-  for (int i = 0; i < kMaxExperts / 64; ++i) mine[i] = i * 64 + lane < E ? s[i * 64 + lane] : -2.f;
+  for (int i = 0; i < kMaxExperts / 64; ++i) mine[i] = i * 64 + lane < E ? s[i * 64 + lane] : -4.f;  // (less than any: never chosen)
   for (int j = 0; j < a.r.top; ++j) {
     float best = -3.f;
     int at = 0;
@@ -298,7 +301,7 @@ __global__ __launch_bounds__(512) void expert_route_row_kernel(const RouteRowArg
     for (int i = 0; i < kMaxExperts / 64; ++i) mine[i] = i * 64 + lane == at ? -2.f : mine[i];
     if (lane == 0) {
       a.r.ids[n * a.r.top + j] = at;
-      a.r.scores[n * a.r.top + j] = best;
+      a.r.scores[n * a.r.top + j] = chosen_score(best);
     }
   }
 }
