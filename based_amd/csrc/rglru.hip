@@ -228,13 +228,17 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
     X = __builtin_fmaf(A[t / 4][t % 4], X, I[t / 4][t % 4]);
     P *= A[t / 4][t % 4];
   }
+  // Where no decay of the channel is zero (2^kl at the least), no product of them is: the smallest number there is, as near as the format
+  // comes, and an infinite state outlives them, as it does token by token.
+  const float least = kl > -126.f ? 0x1p-149f : 0.f;
+  P = fmaxf(P, least);
   // the quads in front of this one
   float before_p = 1.f, before_x = 0.f;
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
     const float p = __shfl(P, q * 16 + l16), x = __shfl(X, q * 16 + l16);
     before_x = q < quad ? __builtin_fmaf(p, before_x, x) : before_x;
-    before_p = q < quad ? p * before_p : before_p;
+    before_p = q < quad ? fmaxf(p * before_p, least) : before_p;
   }
   float S = seg == 0 && !a.fresh ? a.state[(long)b * a.W + w] : 0.f;
   unsigned long long* g = a.agg + (long)b * a.segs * a.W + w;
@@ -246,7 +250,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
   };
   const bool mine = quad == 3 && ch < a.n, closes = seg % kGroup == kGroup - 1;
   if (seg < a.segs - 1 && mine && !closes) {
-    float xw = __builtin_fmaf(P, before_x, X), pw = P * before_p;
+    float xw = __builtin_fmaf(P, before_x, X), pw = fmaxf(P * before_p, least);
     if (seg == 0) {  // (what enters the call is part of it: the last segment replaces the state)
       xw = __builtin_fmaf(pw, S, xw);
       pw = 0.f;
@@ -278,7 +282,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
         const bool in = i0 + i < each && first + i0 + i < count;
         const float pi = __builtin_bit_cast(float, (unsigned int)v[i]), xi = __builtin_bit_cast(float, (unsigned int)(v[i] >> 32));
         x = in ? __builtin_fmaf(pi, x, xi) : x;
-        p = in ? p * pi : p;
+        p = in ? fmaxf(p * pi, least) : p;
       }
     }
     S = __shfl(x, l16);

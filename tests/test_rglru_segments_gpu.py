@@ -128,3 +128,23 @@ def test_replays(dev, dtype, over):
         assert torch.equal(res, want[i][0]) and torch.equal(state, want[i][1]), i
         eager = run(inputs[1][0].clone(), inputs[1][1], inputs[1][2].clone(), torch.empty_like(out))
         assert torch.equal(eager, want[1][0])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("L", [1, 17, 40, 64, 130, 4200, 8300])
+def test_infinite_states_outlive_segments(dev, L, dtype):
+    """An infinity times decays that are small, none of them zero, stays one, however small their product."""
+    from based_amd import ops
+
+    B, W = 2, 24
+    g = torch.Generator().manual_seed(L)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).to(dev)  # noqa: E731
+    u, gates = rnd(B, L, W), (rnd(1, W, W) * W ** -0.5, rnd(W), rnd(1, W, W) * W ** -0.5, rnd(W), rnd(W) + 1)  # decays of 2^-8 and less
+    y = rnd(B, L, W).abs() + 0.1
+    state = torch.zeros(B, W, device=dev)
+    state[0, 3], state[1, 7] = float("inf"), float("-inf")
+    out = ops.rglru_prefill(u, y, *gates, state, 8.0, False, out=torch.empty_like(u))
+    assert (out[0, :, 3] == float("inf")).all() and (out[1, :, 7] == float("-inf")).all()
+    assert state[0, 3] == float("inf") and state[1, 7] == float("-inf")
+    out[0, :, 3], out[1, :, 7], state[0, 3], state[1, 7] = 0, 0, 0, 0
+    assert out.isfinite().all() and state.isfinite().all()
