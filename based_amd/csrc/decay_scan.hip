@@ -561,13 +561,12 @@ __global__ __launch_bounds__(256) void decay_join_kernel(const DecayScanArgs a) 
       l = *reinterpret_cast<const f32x4*>(a.seg_lw + (bh * a.segs + s) * a.dp + ch);
     } else {
       const int lo = s * a.seg_chunks * kScanTokens, hi = (s + 1) * a.seg_chunks * kScanTokens;
-      const float all = __builtin_amdgcn_exp2f(head_l2 * (float)((hi < a.L ? hi : a.L) - lo)), f = all == 0.f && head_w != 0.f ? -0.f : all;
+      const float all = __builtin_amdgcn_exp2f(head_l2 * (float)((hi < a.L ? hi : a.L) - lo)), f = all == 0.f && head_w != 0.f ? 0x1p-149f : all;
       l = f32x4{f, f, f, f};
     }
-    // a product of decays that only the format makes zero comes as minus zero: an infinite state outlives it, as it does token by token
+    // a product of decays that only the format makes zero comes as its smallest number: an infinite state outlives it, as it does token by token
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      S[j] = __builtin_isinf(S[j]) && __builtin_bit_cast(uint32_t, l[j]) == 0x80000000u ? S[j] + add[j] : __builtin_fmaf(S[j], l[j], add[j]);
+    for (int j = 0; j < 4; ++j) S[j] = __builtin_fmaf(S[j], l[j], add[j]);
   }
 }
 
@@ -690,7 +689,7 @@ __global__ __launch_bounds__(256) void decay_scan_any_kernel(const DecayScanArgs
     if (tid >= CH || tid >= a.d) return;
     for (int i = tid + CH; i < 256; i += CH) log2_all += sum[i];
     const float all = exp2f(log2_all);
-    a.seg_lw[(bh * a.segs + sg) * a.dp + tid] = all == 0.f && log2_all > -INFINITY ? -0.f : all;  // (decay_join_kernel)
+    a.seg_lw[(bh * a.segs + sg) * a.dp + tid] = all == 0.f && log2_all > -INFINITY ? 0x1p-149f : all;  // (decay_join_kernel)
   }
 }
 
