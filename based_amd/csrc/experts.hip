@@ -8,11 +8,13 @@
 //   expert_plan     rows of every expert rounded up to tiles, which expert a tile belongs to, and the choices in
 //                   that order
 //   expert_scatter  the last part, where there are too many choices for one workgroup
-//   expert_gemm     MFMA product of a tile of rows with its expert's matrices, gathered and scattered by that
-//                   order: gate and up with the activation behind them, then down
+//   expert_gemm     MFMA product of a tile of 32 rows with its expert's matrices, gathered and scattered by that
+//                   order: gate and up with the activation behind them, then down; expert_gemm_large: of 256 rows
 //   expert_sum      the choices of a token added up (with one choice the product writes the token's row)
 //   expert_route_row  the same for few tokens, with the norm in front of the layer
 //   expert_rows     few tokens, fp32, or rows that are no whole 16-byte pieces: dot products, one choice at a time
+#include <atomic>
+
 #include "stream_common.hpp"
 
 namespace based {
@@ -353,10 +355,8 @@ __device__ __forceinline__ int tile_of_block(int i, int n) {
 }
 
 // BM rows and BN rows of the weights (PAIRED: half of them up, half gate) per workgroup; AHEAD rounds of 64 channels on their
-// way from memory.  They are asked for in front of the products, which the compiler would put between them, with 32-bit offsets: 8192
-// tokens of 1024 channels, 2 of 8 experts of 1024: 106 + 70 us (110 + 72 before).  Then 28 % of the matrix rate; not bound by memory (half the
-// columns to a workgroup, twice the traffic, takes as long) nor helped by rows loaded straight into LDS three rounds deep (120 + 70).
-template <int BM, int BN, int AHEAD, int BUF, bool PAIRED>
+// way from memory.  They are asked for in front of the products, which the compiler would put between them, with 32-bit offsets.
+template <int BM, int BN, int AHEAD, bool PAIRED>
 __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(const ExpertGemmArgs a) {
   // rows of 128 bytes lie side by side, the eight 16-byte pieces of a row turned by half its number: neither the rows that
   // eight lanes write nor the sixteen that a tile reads meet a bank twice
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(const ExpertGemmArg
   auto place = [](int r, int p) { return r * KS + ((p ^ (r >> 1)) & 7) * 8; };
   constexpr int WM = BM >= 128 ? 2 : 1, WN = 4 / WM, MT = BM / 16 / WM, NT = BN / 32 / WN, HALF = BN / 2;
   constexpr int AP = BM / 32, BP = BN / 32;  // 16-byte pieces per thread
-  __shared__ __attribute__((aligned(16))) __bf16 xs[BUF][BM * KS], ws[BUF][BN * KS];
+  __shared__ __attribute__((aligned(16))) __bf16 xs[BM * KS], ws[BN * KS];
   __shared__ int slot_of[BM];
   // bands of kBand row tiles, walked down the rows first: what is in flight on a die shares its rows and its matrices
   const int id = tile_of_block(blockIdx.x, gridDim.x), band = id / (kBand * a.col_tiles), in_band = id % (kBand * a.col_tiles);
@@ -409,24 +409,24 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(const ExpertGemmArg
     for (int i = 0; i < NT; ++i)
 #pragma unroll
       for (int j = 0; j < MT; ++j) acc[p][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto stage = [&](int k0, int buf, const u32x4 (&x)[AP], const u32x4 (&w)[BP]) {
+  auto stage = [&](int k0, const u32x4 (&x)[AP], const u32x4 (&w)[BP]) {
     const bool in = k0 + piece < a.K;
 #pragma unroll
-    for (int i = 0; i < AP; ++i) *reinterpret_cast<u32x4*>(&xs[buf][place(i * 32 + (tid >> 3), tid & 7)]) = in ? x[i] : zero;
+    for (int i = 0; i < AP; ++i) *reinterpret_cast<u32x4*>(&xs[place(i * 32 + (tid >> 3), tid & 7)]) = in ? x[i] : zero;
 #pragma unroll
-    for (int i = 0; i < BP; ++i) *reinterpret_cast<u32x4*>(&ws[buf][place(i * 32 + (tid >> 3), tid & 7)]) = w[i];
+    for (int i = 0; i < BP; ++i) *reinterpret_cast<u32x4*>(&ws[place(i * 32 + (tid >> 3), tid & 7)]) = w[i];
   };
-  auto multiply = [&](int buf) {
+  auto multiply = [&]() {
 #pragma unroll
     for (int kk = 0; kk < kGemmK; kk += 32) {
       bf16x8 xf[MT];
 #pragma unroll
-      for (int j = 0; j < MT; ++j) xf[j] = *reinterpret_cast<const bf16x8*>(&xs[buf][place((wm * MT + j) * 16 + l16, kk / 8 + quad)]);
+      for (int j = 0; j < MT; ++j) xf[j] = *reinterpret_cast<const bf16x8*>(&xs[place((wm * MT + j) * 16 + l16, kk / 8 + quad)]);
 #pragma unroll
       for (int p = 0; p < 2; ++p)
 #pragma unroll
         for (int i = 0; i < NT; ++i) {
-          const bf16x8 wf = *reinterpret_cast<const bf16x8*>(&ws[buf][place(p * HALF + (wn * NT + i) * 16 + l16, kk / 8 + quad)]);
+          const bf16x8 wf = *reinterpret_cast<const bf16x8*>(&ws[place(p * HALF + (wn * NT + i) * 16 + l16, kk / 8 + quad)]);
 #pragma unroll
           for (int j = 0; j < MT; ++j) acc[p][i][j] = expert_mfma(wf, xf[j], acc[p][i][j]);
         }
@@ -435,33 +435,15 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(const ExpertGemmArg
 #pragma unroll
   for (int s = 0; s < AHEAD; ++s) fetch(s * kGemmK, xb[s], wb[s]);
   // (rounds past the end multiply by zeros: every stage of the loops is the same)
-  if constexpr (BUF == 1) {
-    for (int k00 = 0; k00 < a.K; k00 += AHEAD * kGemmK) {
+  for (int k00 = 0; k00 < a.K; k00 += AHEAD * kGemmK) {
 #pragma unroll
-      for (int s = 0; s < AHEAD; ++s) {
-        const int k0 = k00 + s * kGemmK;
-        lds_barrier();
-        stage(k0, 0, xb[s], wb[s]);
-        lds_barrier();
-        fetch(k0 + AHEAD * kGemmK, xb[s], wb[s]);
-        multiply(0);
-      }
-    }
-  } else {
-    // one barrier per round: the next round goes into the other half of LDS while this one is multiplied
-    constexpr int U = AHEAD % 2 == 0 ? AHEAD : 2 * AHEAD;
-    stage(0, 0, xb[0], wb[0]);
-    fetch(AHEAD * kGemmK, xb[0], wb[0]);
-    lds_barrier();
-    for (int k00 = 0; k00 < a.K; k00 += U * kGemmK) {
-#pragma unroll
-      for (int s = 0; s < U; ++s) {
-        const int k1 = k00 + (s + 1) * kGemmK;
-        multiply(s & 1);
-        stage(k1, (s + 1) & 1, xb[(s + 1) % AHEAD], wb[(s + 1) % AHEAD]);
-        fetch(k1 + AHEAD * kGemmK, xb[(s + 1) % AHEAD], wb[(s + 1) % AHEAD]);
-        lds_barrier();
-      }
+    for (int s = 0; s < AHEAD; ++s) {
+      const int k0 = k00 + s * kGemmK;
+      lds_barrier();
+      stage(k0, xb[s], wb[s]);
+      lds_barrier();
+      fetch(k0 + AHEAD * kGemmK, xb[s], wb[s]);
+      multiply();
     }
   }
   // column = row l16 of the tile's rows, rows = features 4 quad + i
@@ -501,19 +483,329 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(const ExpertGemmArg
   }
 }
 
-template <int BM, int BN, int AHEAD, int BUF, bool PAIRED> void launch_expert_gemm(ExpertGemmArgs a, hipStream_t s) {
-  const int cols = PAIRED ? BN / 2 : BN;
-  a.col_tiles = (a.F + cols - 1) / cols;
-  hipLaunchKernelGGL((expert_gemm_kernel<BM, BN, AHEAD, BUF, PAIRED>), dim3((unsigned)(a.col_tiles * a.tiles)), dim3(256), 0, s, a);
+// ---- the same with tiles of 256 rows and 256 rows of the weights (PAIRED: 128 up, 128 gate), rows and weights straight into LDS ----
+// One workgroup of eight wavefronts to a compute unit.  Tiles are dealt to the dies in runs; what is left of a die's run after whole rounds
+// of its compute units goes in parts of 128 or 64 rows where that gives every part a compute unit of its own.
+// 8192 tokens of 1024 channels, 2 of 8 experts of 1024: 77 + 48 us (tiles of 128 x 256 through registers, two workgroups to a compute
+// unit: 106 + 70); without parts 93 + 64.  A whole tile alone takes 29 us: its matrix instructions 22, at the rate that they reach by
+// themselves here (1.6 PFLOP/s), the rest in front of the first and behind the last.
+constexpr int kLargeRows = BASED_EXPERT_TILE_ROWS;
+constexpr int kDies = 8, kDieUnits = 32;
+constexpr int kHalf = 128 * kGemmK;  // elements of 128 rows of a round
+constexpr int kPartSlot = 3 * kHalf, kPartDepth = 3;
+constexpr int kLargeLds = kPartDepth * kPartSlot * 2 + kLargeRows * 4;  // bytes; whole tiles use 8 kHalf of the elements
+
+struct ExpertTile {
+  const __bf16* w;  // matrices of the tile's expert
+  long first;       // first row of the tile among all tiles
+  int rows, f0;     // rows that are there, first feature
+};
+
+// 16 bytes a lane, side by side from dst on.  TAIL: zeros where the lane's piece (from channel c on) is past the last channel; a row has pieces
+// in front of it too, so that the load is always counted.
+template <bool TAIL> __device__ __forceinline__ void load_to_lds(const __bf16* src, __bf16* dst, int c, int channels) {
+  if (TAIL && c >= channels) {
+    *reinterpret_cast<bf16x8*>(dst + (threadIdx.x & 63) * 8) = bf16x8{};
+    return;
+  }
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
 }
 
-template <bool PAIRED> void launch_expert_product(const ExpertGemmArgs& a, int rows, hipStream_t s) {
-  if (rows == BASED_EXPERT_TILE_ROWS_SMALL)
-    launch_expert_gemm<BASED_EXPERT_TILE_ROWS_SMALL, 128, 4, 1, PAIRED>(a, s);
-  else if (a.F >= 256 && (long)a.tiles * a.F >= (PAIRED ? 512 * 128 : 512 * 256))
-    launch_expert_gemm<BASED_EXPERT_TILE_ROWS, 256, 1, 1, PAIRED>(a, s);
-  else
-    launch_expert_gemm<BASED_EXPERT_TILE_ROWS, 128, 2, 1, PAIRED>(a, s);
+// the weights' row (of the expert's matrices) behind row r of a tile's 256
+template <bool PAIRED> __device__ __forceinline__ uint32_t large_w_row(const ExpertGemmArgs& a, int f0, int r) {
+  const int f = f0 + (PAIRED ? r & 127 : r);
+  return (uint32_t)((PAIRED && r >= 128 ? a.F : 0) + (f < a.F ? f : a.F - 1));
+}
+
+template <bool PAIRED> __device__ __forceinline__ const __bf16* large_x_row(const ExpertGemmArgs& a, const ExpertTile& t, const int* slot_of, int r) {
+  return a.x + (PAIRED ? (long)(slot_of[r] / a.top) * a.x_sr : (t.first + (r < t.rows ? r : 0)) * a.x_sr);
+}
+
+// four features of one row from their sums u (PAIRED: of up, and g of gate)
+template <bool PAIRED> __device__ __forceinline__ void large_store(const ExpertGemmArgs& a, __bf16* y, int f, float score, f32x4 u, f32x4 g) {
+  if (f >= a.F) return;
+  bf16x4 o;
+#pragma unroll
+  for (int m = 0; m < 4; ++m) o[m] = PAIRED ? (__bf16)(silu_exact(g[m] * score) * (u[m] * score)) : (__bf16)u[m];
+  *reinterpret_cast<bf16x4*>(y + f) = o;
+}
+
+// A whole tile, two rounds of 64 channels in LDS.  A round is four halves of 128 rows, x0, x1, w0, w1; a wavefront has 64 rows of a half of x
+// and 32 of a half of w, and goes through the products of the halves as phases of 16 matrix instructions
+//   0: x0 w0    1: x0 w1    2: x1 w1    3: x1 w0
+// while it reads from LDS what the next phase multiplies (w1, x1, the next round's x0, its w0) and asks memory for the half whose place
+// became free a phase before (w0, w1, x1 of the round after the next, x0 of the one behind it), seven phases ahead of the phase that reads it.
+// One barrier a phase; the wait in front of it leaves the loads of six phases on their way.  The compiler, which knows of no distance between
+// these loads and reads of LDS, would wait for all of them in front of every read: it does for a static array (148 us where this takes 94), not for one
+// whose extent the launch gives.
+template <bool PAIRED> __device__ __forceinline__ void large_whole_tile(const ExpertGemmArgs& a, const ExpertTile& t, __bf16* lds, const int* slot_of) {
+  constexpr int KS = kGemmK;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, quad = lane >> 4;
+  const int wm = wave & 1, wn = wave >> 1;
+  // a wavefront's two loads of a half: rows 16 wave + 8 i + lane / 8, whose eight pieces lie turned by half the row's number
+  const int row = wave * 16 + (lane >> 3), piece = (lane ^ (lane >> 4)) & 7;  // (i = 1: the piece's bit 2 the other way round)
+  const __bf16* xrow[2][2];
+  uint32_t wrow[2][2];  // bytes
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = h * 128 + row + 8 * i, c = (piece ^ (4 * i)) * 8;
+      xrow[h][i] = large_x_row<PAIRED>(a, t, slot_of, r) + c;
+      wrow[h][i] = (large_w_row<PAIRED>(a, t.f0, r) * (uint32_t)a.K + (uint32_t)c) * 2u;
+    }
+  const int rounds = a.K / KS;
+  auto ask = [&](int half, int at_round) {  // half 0, 1: x; 2, 3: w
+    __bf16* at = lds + (at_round & 1) * 4 * kHalf + half * kHalf + wave * 16 * KS;
+    const int round = at_round < rounds ? at_round : 0;  // (asked for and never read)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      load_to_lds<false>(half < 2 ? xrow[half & 1][i] + round * KS
+                                 : reinterpret_cast<const __bf16*>(reinterpret_cast<const char*>(t.w + round * KS) + wrow[half & 1][i]),
+                        at + i * 8 * KS, 0, 0);
+  };
+  // fragments: rows l16 of a tile of 16, channels 32 kk + 8 quad ..
+  bf16x8 x0[4][2], x1[4][2], wa[2][2], wb[2][2];
+  const int turned = (l16 >> 1) & 7, p0 = (quad ^ turned) * 8, p1 = ((4 + quad) ^ turned) * 8;
+  auto read_x = [&](int round, int h, bf16x8 (&f)[4][2]) {
+    const __bf16* at = lds + (round & 1) * 4 * kHalf + h * kHalf + (wm * 64 + l16) * KS;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f[j][0] = *reinterpret_cast<const bf16x8*>(at + j * 16 * KS + p0);
+      f[j][1] = *reinterpret_cast<const bf16x8*>(at + j * 16 * KS + p1);
+    }
+  };
+  auto read_w = [&](int round, int h, bf16x8 (&f)[2][2]) {
+    const __bf16* at = lds + (round & 1) * 4 * kHalf + (2 + h) * kHalf + (wn * 32 + l16) * KS;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      f[j][0] = *reinterpret_cast<const bf16x8*>(at + j * 16 * KS + p0);
+      f[j][1] = *reinterpret_cast<const bf16x8*>(at + j * 16 * KS + p1);
+    }
+  };
+  f32x4 acc[2][2][2][4];  // [half of x][half of w][16 features][16 rows]
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[h][g][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](const bf16x8 (&x)[4][2], const bf16x8 (&w)[2][2], f32x4 (&c)[2][4], int kk) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) c[i][j] = expert_mfma(w[i][kk], x[j][kk], c[i][j]);
+  };
+  // 16 products with the loads of a half in the middle; then own reads are done and own loads of all but six phases have landed (lgkmcnt 0,
+  // vmcnt 12)
+  auto phase = [&](const bf16x8 (&x)[4][2], const bf16x8 (&w)[2][2], f32x4 (&c)[2][4], int half, int round) {
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(x, w, c, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    ask(half, round);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(x, w, c, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0070 | 12);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // w0 of the round lies in wu; its w1 comes into wv, and the next round's w0 there again
+  auto round_of = [&](int round, bf16x8 (&wu)[2][2], bf16x8 (&wv)[2][2]) {
+    read_w(round, 1, wv);
+    phase(x0, wu, acc[0][0], 2, round + 2);
+    read_x(round, 1, x1);
+    phase(x0, wv, acc[0][1], 3, round + 2);
+    read_x(round + 1, 0, x0);
+    phase(x1, wv, acc[1][1], 1, round + 2);
+    read_w(round + 1, 0, wv);
+    phase(x1, wu, acc[1][0], 0, round + 3);
+  };
+  ask(0, 0), ask(2, 0), ask(3, 0), ask(1, 0), ask(0, 1), ask(2, 1), ask(3, 1), ask(1, 1);
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(0x0070 | 10);  // x0, w0 and w1 of round 0
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  read_x(0, 0, x0);
+  read_w(0, 0, wa);
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt 0
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  ask(0, 2);
+  for (int round = 0; round + 1 < rounds; round += 2) {
+    round_of(round, wa, wb);
+    round_of(round + 1, wb, wa);
+  }
+  if (rounds & 1) round_of(rounds - 1, wa, wb);
+  __builtin_amdgcn_s_waitcnt(0x0070);  // (nothing may come into LDS that is no longer this workgroup's)
+  // column = row l16 of the tile's rows, rows = features 4 quad + i
+  int slot[2][4];
+  float score[2][4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      slot[h][j] = slot_of[h * 128 + wm * 64 + j * 16 + l16];
+      score[h][j] = PAIRED ? a.scores[slot[h][j]] : 1.f;
+    }
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = h * 128 + wm * 64 + j * 16 + l16;
+      if (r >= t.rows) continue;
+      __bf16* y = a.y + (PAIRED ? t.first + r : (long)slot[h][j]) * a.F;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int f = t.f0 + wn * 32 + i * 16 + quad * 4;
+        large_store<PAIRED>(a, y, f, score[h][j], acc[h][0][i][j], acc[h][1][i][j]);
+        if constexpr (!PAIRED) large_store<PAIRED>(a, y, f + 128, score[h][j], acc[h][1][i][j], acc[h][0][i][j]);
+      }
+    }
+}
+
+// R rows from row r0 of a tile on, three rounds of 64 channels in LDS of which two are on their way; a wavefront has all of the rows and 32 rows
+// of the weights.
+template <int R, bool PAIRED, bool TAIL>
+__device__ __forceinline__ void large_part(const ExpertGemmArgs& a, const ExpertTile& t, __bf16* lds, const int* slot_of, int r0) {
+  constexpr int KS = kGemmK, XL = R / 64, WL = 4, MT = R / 16;
+  if (r0 >= t.rows) return;  // (no barrier left)
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, quad = lane >> 4;
+  const int piece = (lane ^ (lane >> 4)) & 7;  // (rows of an odd group of eight: bit 2 the other way round)
+  const __bf16* xrow[XL];
+  uint32_t wrow[WL];  // bytes
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    const int r = (wave * XL + i) * 8 + (lane >> 3);
+    xrow[i] = large_x_row<PAIRED>(a, t, slot_of, r0 + r) + (piece ^ (r >> 1 & 4)) * 8;
+  }
+#pragma unroll
+  for (int i = 0; i < WL; ++i) {
+    const int r = (wave * WL + i) * 8 + (lane >> 3);
+    wrow[i] = (large_w_row<PAIRED>(a, t.f0, r) * (uint32_t)a.K + (uint32_t)((piece ^ (r >> 1 & 4)) * 8)) * 2u;
+  }
+  const int rounds = (a.K + KS - 1) / KS;
+  auto ask = [&](int at_round, int place) {
+    __bf16* at = lds + place * kPartSlot;  // 256 rows of the weights, then the rows
+    const int round = at_round < rounds ? at_round : 0;  // (asked for and never read)
+#pragma unroll
+    for (int i = 0; i < WL; ++i)
+      load_to_lds<TAIL>(reinterpret_cast<const __bf16*>(reinterpret_cast<const char*>(t.w + round * KS) + wrow[i]), at + (wave * WL + i) * 8 * KS,
+                        round * KS + (piece ^ ((wave * WL + i) * 4 & 4)) * 8, a.K);
+#pragma unroll
+    for (int i = 0; i < XL; ++i)
+      load_to_lds<TAIL>(xrow[i] + round * KS, at + 2 * kHalf + (wave * XL + i) * 8 * KS, round * KS + (piece ^ ((wave * XL + i) * 4 & 4)) * 8, a.K);
+  };
+  f32x4 acc[2][MT];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int turned = (l16 >> 1) & 7;
+  ask(0, 0);
+  ask(1, 1);
+  for (int round = 0, place = 0; round < rounds; ++round) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0070 | (XL + WL));  // own reads are done, and all loads but those of the next round
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    ask(round + 2, place == 0 ? 2 : place - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    const __bf16* at = lds + place * kPartSlot + l16 * KS;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int p = ((kk * 4 + quad) ^ turned) * 8;
+      bf16x8 w[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) w[i] = *reinterpret_cast<const bf16x8*>(at + (PAIRED ? i * 128 + wave * 16 : wave * 32 + i * 16) * KS + p);
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        const bf16x8 x = *reinterpret_cast<const bf16x8*>(at + 2 * kHalf + j * 16 * KS + p);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[i][j] = expert_mfma(w[i], x, acc[i][j]);
+      }
+    }
+    place = place == 2 ? 0 : place + 1;
+  }
+  __builtin_amdgcn_s_waitcnt(0x0070);
+  int slot[MT];
+  float score[MT];
+#pragma unroll
+  for (int j = 0; j < MT; ++j) {
+    slot[j] = slot_of[r0 + j * 16 + l16];
+    score[j] = PAIRED ? a.scores[slot[j]] : 1.f;
+  }
+#pragma unroll
+  for (int j = 0; j < MT; ++j) {
+    const int r = r0 + j * 16 + l16;
+    if (r >= t.rows) continue;
+    __bf16* y = a.y + (PAIRED ? t.first + r : (long)slot[j]) * a.F;
+    const int f = t.f0 + wave * (PAIRED ? 16 : 32) + quad * 4;
+    large_store<PAIRED>(a, y, f, score[j], acc[0][j], acc[1][j]);
+    if constexpr (!PAIRED) large_store<PAIRED>(a, y, f + 16, score[j], acc[1][j], acc[0][j]);
+  }
+}
+
+// TAIL: the last round of channels is no whole one, and all tiles go in parts (a whole one would have to spill registers).  Block i is number i / 8 of die i % 8.
+template <bool PAIRED, bool TAIL> __global__ __launch_bounds__(512, 2) void expert_gemm_large_kernel(const ExpertGemmArgs a) {
+  extern __shared__ __attribute__((aligned(16))) __bf16 lds[];
+  int* slot_of = reinterpret_cast<int*>(lds + kPartDepth * kPartSlot);
+  const int row_tiles = a.tile_first[a.E], all = row_tiles * a.col_tiles;
+  const int die = blockIdx.x % kDies, k = blockIdx.x / kDies, more = all % kDies;
+  const int first = die * (all / kDies) + (die < more ? die : more), mine = all / kDies + (die < more ? 1 : 0);
+  const int whole = TAIL ? 0 : mine / kDieUnits * kDieUnits, left = mine - whole;
+  const int parts = left * 4 <= kDieUnits ? 4 : TAIL || left * 2 <= kDieUnits ? 2 : 1;
+  if (k >= whole + left * parts) return;
+  const int id = first + (k < whole ? k : whole + (k - whole) / parts), part = k < whole ? 0 : (k - whole) % parts;
+  // bands of kBand row tiles, walked down the rows first: what is in flight on a die shares its rows and its matrices
+  const int band = id / (kBand * a.col_tiles), in_band = id % (kBand * a.col_tiles);
+  const int deep = row_tiles - band * kBand < kBand ? row_tiles - band * kBand : kBand;
+  const int tile = band * kBand + in_band % deep, e = a.tile_expert[tile], r0 = (tile - a.tile_first[e]) * kLargeRows;
+  ExpertTile t;
+  t.w = a.w + (long)e * (PAIRED ? 2 * a.F : a.F) * a.K;
+  t.first = (long)tile * kLargeRows;
+  t.rows = a.counts[e] - r0 < kLargeRows ? a.counts[e] - r0 : kLargeRows;
+  t.f0 = in_band / deep * (PAIRED ? 128 : 256);
+  if (threadIdx.x < kLargeRows) slot_of[threadIdx.x] = a.order[t.first + ((int)threadIdx.x < t.rows ? (int)threadIdx.x : 0)];
+  __syncthreads();
+  if (k >= whole && parts == 4) return large_part<64, PAIRED, TAIL>(a, t, lds, slot_of, part * 64);
+  if (k >= whole && parts == 2) return large_part<128, PAIRED, TAIL>(a, t, lds, slot_of, part * 128);
+  if constexpr (!TAIL) large_whole_tile<PAIRED>(a, t, lds, slot_of);
+}
+
+constexpr int kMaxDevices = 64;
+
+template <bool PAIRED, bool TAIL> int launch_expert_gemm_large(ExpertGemmArgs a, hipStream_t s) {
+  static std::atomic<bool> allowed[kMaxDevices];
+  int dev = 0;
+  BASED_REQUIRE(hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices, BASED_ERR_LAUNCH, "experts: cannot identify the current device");
+  if (!allowed[dev].load(std::memory_order_acquire)) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(expert_gemm_large_kernel<PAIRED, TAIL>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, kLargeLds);
+    BASED_REQUIRE(e == hipSuccess, BASED_ERR_LAUNCH, "experts: %d bytes of LDS refused: %s", kLargeLds, hipGetErrorString(e));
+    allowed[dev].store(true, std::memory_order_release);
+  }
+  a.col_tiles = PAIRED ? (a.F + 127) / 128 : (a.F + 255) / 256;
+  // (parts beyond the first of a tile: less than one for each of the 32 compute units of a die; TAIL: everything in two)
+  const unsigned per_die = (unsigned)((a.col_tiles * a.tiles + kDies - 1) / kDies * (TAIL ? 2 : 1) + kDieUnits);
+  hipLaunchKernelGGL((expert_gemm_large_kernel<PAIRED, TAIL>), dim3(per_die * kDies), dim3(512), kLargeLds, s, a);
+  return BASED_OK;
+}
+
+template <int BM, int BN, int AHEAD, bool PAIRED> void launch_expert_gemm(ExpertGemmArgs a, hipStream_t s) {
+  const int cols = PAIRED ? BN / 2 : BN;
+  a.col_tiles = (a.F + cols - 1) / cols;
+  hipLaunchKernelGGL((expert_gemm_kernel<BM, BN, AHEAD, PAIRED>), dim3((unsigned)(a.col_tiles * a.tiles)), dim3(256), 0, s, a);
+}
+
+template <bool PAIRED> int launch_expert_product(const ExpertGemmArgs& a, int rows, hipStream_t s) {
+  if (rows == BASED_EXPERT_TILE_ROWS)
+    return a.K % kGemmK == 0 ? launch_expert_gemm_large<PAIRED, false>(a, s) : launch_expert_gemm_large<PAIRED, true>(a, s);
+  launch_expert_gemm<BASED_EXPERT_TILE_ROWS_SMALL, 128, 4, PAIRED>(a, s);
+  return BASED_OK;
 }
 
 // y[n] = sum of the rows of its choices
@@ -700,7 +992,9 @@ static int route_check(const char* who, const RouteArgs& a) {
 }  // namespace based
 
 /* Tiles of BASED_EXPERT_TILE_ROWS or BASED_EXPERT_TILE_ROWS_SMALL rows. */
-static int expert_tile_rows(int64_t slots, int64_t E) { return slots >= 256 * E ? BASED_EXPERT_TILE_ROWS : BASED_EXPERT_TILE_ROWS_SMALL; }
+// The line: 2 of 8 experts of 1024, 354 tokens (88 choices an expert) 41.2 us with large tiles, 40.1 with small ones, 700 tokens 41.8 and 50.0;
+// 1 of 8 of 2048, 900 tokens (112 an expert) 61.8 and 69.2; 4 of 16 of 512, 400 tokens (100) 41.7 and 46.9, 200 tokens (50) 41.5 and 40.7.
+static int expert_tile_rows(int64_t slots, int64_t E) { return slots >= 96 * E ? BASED_EXPERT_TILE_ROWS : BASED_EXPERT_TILE_ROWS_SMALL; }
 
 extern "C" BASED_API int64_t based_expert_tiles(int64_t n, int64_t E, int64_t top) {
   if (n <= 0 || E <= 0 || top <= 0) return 0;
@@ -748,8 +1042,9 @@ extern "C" BASED_API int based_expert_grouped(const void* h, const void* router,
   __bf16* out = static_cast<__bf16*>(top == 1 ? y : work_out);
   const ExpertGemmArgs a2{static_cast<const __bf16*>(work_act), static_cast<const __bf16*>(w2), out, order, counts, tile_first,
                           tile_expert, scores, (long)F, (int)E, (int)D, (int)F, (int)top, 0, (int)tiles};
-  launch_expert_product<true>(a, rows, s);
-  launch_expert_product<false>(a2, rows, s);
+  int done = launch_expert_product<true>(a, rows, s);
+  if (done == BASED_OK) done = launch_expert_product<false>(a2, rows, s);
+  if (done != BASED_OK) return done;
   if (top > 1)
     hipLaunchKernelGGL(expert_sum_kernel, dim3((unsigned)((n * (D / 8) + 255) / 256)), dim3(256), 0, s, out, static_cast<__bf16*>(y), (long)n,
                        (int)D, (int)top);

@@ -694,7 +694,7 @@ BASED_API int based_latent_step(const void* q, const void* x, const void* norm_w
  * tile_expert (tiles), order (tiles * rows), work_act (tiles * rows, F), work_out (n * top, D) with top > 1, tiles and rows from
  * based_expert_tiles / based_expert_tile_rows.  Rows: one choice at a time, for few tokens and any element type; work_act (n * top, F).
  * With norm_weight (D; bf16, D up to 4096) h is the norm of residual_in + mult * x as in based_add_norm, in work_h (n, D). */
-#define BASED_EXPERT_TILE_ROWS 128
+#define BASED_EXPERT_TILE_ROWS 256
 #define BASED_EXPERT_TILE_ROWS_SMALL 32
 BASED_API int64_t based_expert_tiles(int64_t n, int64_t E, int64_t top);
 BASED_API int64_t based_expert_tile_rows(int64_t n, int64_t E, int64_t top);

@@ -534,3 +534,22 @@ def test_refusals(dev):
         ops.experts(z(2, 8), z(3, 8), z(3, 16, 8), z(3, 8, 8), 4)
     with pytest.raises(ValueError, match="mixes"):
         ops.decode_linear(z(2, 64), z(100, 64), prologue=ops.PROLOGUE_STREAM, norm_weight=z(64), mix=(z(5, 64), z(2, 2, 64), 0, 20))
+
+
+@pytest.mark.parametrize("n,D,F,E,top", [(96, 64, 64, 1, 1), (400, 64, 128, 4, 1), (4096, 128, 128, 4, 1), (4100, 384, 264, 3, 1), (2310, 256, 384, 4, 2),
+                                         (5200, 192, 120, 5, 1), (9001, 1024, 256, 8, 2), (6000, 128, 1152, 3, 2)])
+def test_experts_in_large_tiles(dev, n, D, F, E, top):
+    """Tiles of 256 rows: a last one that is partly empty, features that end inside a tile, channels in one round, odd and even numbers of them and
+    a part of one; dies with whole tiles only, with halves and quarters behind them, and with parts alone."""
+    from based_amd import _lib, ops
+
+    assert _lib.lib().based_expert_tile_rows(n, E, top) == 256
+    h, router, w1, w2, w = expert_case(n, D, F, E, top, BF16, seed=n)
+    router[0] = 0.2 * router[0]  # (an expert with few rows)
+    w["m.router"] = router.double()
+    want = O.expert_mlp(h.double(), w, "m", {"router": {"top": top}})
+    got = ops.experts(h.to(dev), router.to(dev), w1.to(dev), w2.to(dev), top).double().cpu()
+    s = O.sigmoid(h.double() @ router.double().T).sort(-1, descending=True).values
+    clear = torch.ones(n, dtype=torch.bool) if top == E else s[:, top - 1] - s[:, top] > 1e-5
+    assert clear.sum() >= 0.98 * n
+    close(got[clear], want[clear], 2 * TOL[BF16])
