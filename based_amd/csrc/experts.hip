@@ -5,9 +5,8 @@
 //
 //   expert_route    scores in fp32, the choice, and for grouped products each choice's place among its
 //                   expert's rows; a single workgroup (up to 32 tokens) also does what the next two do
-//   expert_plan     rows of every expert rounded up to tiles, which expert a tile belongs to, and the choices in
+//   expert_place    rows of every expert rounded up to tiles, which expert a tile belongs to, and the choices in
 //                   that order
-//   expert_scatter  the last part, where there are too many choices for one workgroup
 //   expert_gemm     MFMA product of a tile of 32 rows with its expert's matrices, gathered and scattered by that
 //                   order: gate and up with the activation behind them, then down; expert_gemm_large: of 256 rows
 //   expert_sum      the choices of a token added up (with one choice the product writes the token's row)
@@ -27,7 +26,8 @@ struct RouteArgs {
   int32_t* ids;   // (N, top)
   float* scores;  // (N, top)
   int32_t* rank;  // (N, top) or null
-  int32_t* counts;  // (E), with rank; zero on entry unless one workgroup does everything
+  int32_t* counts;  // (E), with rank; zero on entry unless one workgroup does everything or there is hist
+  int32_t* hist;    // choices of each expert in each workgroup's tokens (workgroups, E): ranks stay those among these tokens; or null
   // one workgroup for all tokens: the plan too
   int32_t* tile_first;
   int32_t* tile_expert;
@@ -55,7 +55,8 @@ __device__ __forceinline__ void plan_tiles(const int* counts, int* scan, int* fi
     const int first = scan[e] - tiles;
     first_of[e] = first;
     tile_first[e] = first;
-    for (int t = 0; t < tiles; ++t) tile_expert[first + t] = e;
+    if (tile_expert != nullptr)
+      for (int t = 0; t < tiles; ++t) tile_expert[first + t] = e;
   }
   if (e == 255) tile_first[E] = scan[255];
   __syncthreads();
@@ -175,6 +176,10 @@ __global__ __launch_bounds__(64 * NW) void expert_route_kernel(const RouteArgs a
   }
   if (a.rank == nullptr) return;
   __syncthreads();
+  if (a.hist != nullptr) {
+    for (int e = tid; e < a.E; e += NT) a.hist[(long)blockIdx.x * a.E + e] = hist[e];
+    return;
+  }
   if (a.order != nullptr) {
     plan_tiles(hist, scan, base, a.tile_first, a.tile_expert, a.E, a.tile_rows);
     for (int e = tid; e < a.E; e += NT) a.counts[e] = hist[e];
@@ -308,27 +313,78 @@ __global__ __launch_bounds__(512) void expert_route_row_kernel(const RouteRowArg
   }
 }
 
-constexpr long kPlanSlots = 8192;  // choices that the planning workgroup puts in order by itself
+constexpr int kPlaceThreads = 512, kPlaceGroups = 8;  // of the routing's workgroups, that one places
+constexpr long kPlaceHist = 1 << 15;                  // entries of hist up to which every workgroup may read all of it
 
-constexpr int kPlanThreads = 1024;
+struct PlaceArgs {
+  int32_t* counts;
+  const int32_t* hist;  // (groups, E); null: counts are there and ranks are those among all choices
+  const int32_t* ids;
+  const int32_t* rank;
+  int32_t* tile_first;
+  int32_t* tile_expert;
+  int32_t* order;
+  long slots;
+  int E, tile_rows, groups, group_slots;
+};
 
-__global__ __launch_bounds__(kPlanThreads) void expert_plan_kernel(const int32_t* counts, const int32_t* __restrict__ ids,
-                                                                   const int32_t* __restrict__ rank, int32_t* tile_first,
-                                                                   int32_t* tile_expert, int32_t* __restrict__ order, long slots, int E,
-                                                                   int tile_rows) {
-  __shared__ int scan[256], first_of[kMaxExperts];
-  plan_tiles(counts, scan, first_of, tile_first, tile_expert, E, tile_rows);
-  if (slots <= kPlanSlots) {
-    // (the loads of the unrolled places are independent of each other)
-#pragma unroll 4
-    for (int i = threadIdx.x; i < (int)slots; i += kPlanThreads) order[(long)first_of[ids[i]] * tile_rows + rank[i]] = i;
+// Workgroup i places the choices of groups kPlaceGroups i ..; each of them plans the tiles for itself, which is less than another launch.
+__global__ __launch_bounds__(kPlaceThreads) void expert_place_kernel(const PlaceArgs a) {
+  __shared__ int scan[256], first_of[kMaxExperts], total[kMaxExperts], base[kPlaceGroups][kMaxExperts];
+  __shared__ int32_t unused[kMaxExperts + 1];
+  const int tid = threadIdx.x, g0 = blockIdx.x * kPlaceGroups;
+  const int mine = a.groups - g0 < kPlaceGroups ? a.groups - g0 : kPlaceGroups;
+  for (int e = tid; e < a.E; e += kPlaceThreads) {
+    total[e] = a.hist != nullptr ? 0 : a.counts[e];
+    for (int g = 0; g < kPlaceGroups; ++g) base[g][e] = 0;
+  }
+  __syncthreads();
+  if (a.hist != nullptr) {
+    int wide = 1;
+    while (wide < a.E) wide <<= 1;
+    const int e = tid & (wide - 1), runs = kPlaceThreads / wide;
+    if (e < a.E) {
+      int before = 0, sum = 0;
+#pragma unroll 8
+      for (int g = tid / wide; g < a.groups; g += runs) {
+        const int c = a.hist[(long)g * a.E + e];
+        sum += c;
+        before += g < g0 ? c : 0;
+      }
+      if (sum != 0) atomicAdd(&total[e], sum);
+      if (before != 0) atomicAdd(&base[0][e], before);
+    }
+    __syncthreads();
+    for (int x = tid; x < a.E; x += kPlaceThreads) {
+      int c[kPlaceGroups], at = base[0][x];
+#pragma unroll
+      for (int g = 0; g < kPlaceGroups; ++g) c[g] = g < mine ? a.hist[(long)(g0 + g) * a.E + x] : 0;
+#pragma unroll
+      for (int g = 0; g < kPlaceGroups; ++g) {
+        base[g][x] = at;
+        at += c[g];
+      }
+    }
+  }
+  if (blockIdx.x == 0) {
+    plan_tiles(total, scan, first_of, a.tile_first, a.tile_expert, a.E, a.tile_rows);
+    if (a.hist != nullptr)
+      for (int e = tid; e < a.E; e += kPlaceThreads) a.counts[e] = total[e];
+  } else {
+    plan_tiles(total, scan, first_of, unused, nullptr, a.E, a.tile_rows);
+  }
+  for (int g = 0; g < mine; ++g) {
+    const long s0 = (long)(g0 + g) * a.group_slots;
+    const int n = a.slots - s0 < a.group_slots ? (int)(a.slots - s0) : a.group_slots;
+    for (int i = tid; i < n; i += kPlaceThreads) {
+      const int e = a.ids[s0 + i];
+      a.order[(long)first_of[e] * a.tile_rows + base[g][e] + a.rank[s0 + i]] = (int32_t)(s0 + i);
+    }
   }
 }
 
-__global__ __launch_bounds__(256) void expert_scatter_kernel(const int32_t* ids, const int32_t* rank, const int32_t* tile_first, int32_t* order,
-                                                             long slots, int tile_rows) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i < slots) order[(long)tile_first[ids[i]] * tile_rows + rank[i]] = (int32_t)i;
+__global__ __launch_bounds__(kMaxExperts) void expert_zero_kernel(int32_t* counts, int E) {
+  if ((int)threadIdx.x < E) counts[threadIdx.x] = 0;
 }
 
 // ---- grouped products ----
@@ -944,19 +1000,27 @@ template <typename T, bool PAIRED> void launch_expert_rows_vec(const ExpertRowsA
 
 constexpr int kRouteOneWg = 32;  // tokens that one workgroup routes, of up to 32 experts (16 of more): it makes the plan too
 
+// Tokens of one workgroup.  Many tokens of few experts: 32, their rows shared out over eight wavefronts (8192 tokens of 1024 channels, 8 experts:
+// 7.2 us without the sums of all workgroups' choices, 10 with them; 16 tokens 11.6, a wavefront to 16 tokens 16.9).
+static int route_group(const RouteArgs& a, bool vec) {
+  const bool many = vec && a.n >= 4096;
+  return !many ? 16 : a.E <= 32 ? 32 : 64;
+}
+
 template <int ET> void launch_route_tiles(const RouteArgs& a, hipStream_t s) {
   const size_t one = (size_t)16 * a.E * sizeof(float);
   constexpr int NW = ET <= 4 ? 8 : 4;
+  const int group = route_group(a, true);
   if constexpr (ET <= 2) {
-    if (a.n > 16 && a.n <= kRouteOneWg) {
-      hipLaunchKernelGGL((expert_route_kernel<__bf16, ET, NW, true, 2>), dim3(1), dim3(64 * NW), 2 * NW * one, s, a);
+    if ((a.n > 16 && a.n <= kRouteOneWg) || group == 32) {
+      hipLaunchKernelGGL((expert_route_kernel<__bf16, ET, NW, true, 2>), dim3((unsigned)((a.n + 31) / 32)), dim3(64 * NW), 2 * NW * one, s, a);
       return;
     }
-  }
-  if (a.n >= 4096)
+  } else if (group == 64) {
     hipLaunchKernelGGL((expert_route_kernel<__bf16, ET, 4, false, 1>), dim3((unsigned)((a.n + 63) / 64)), dim3(256), 4 * one, s, a);
-  else
-    hipLaunchKernelGGL((expert_route_kernel<__bf16, ET, NW, true, 1>), dim3((unsigned)((a.n + 15) / 16)), dim3(64 * NW), NW * one, s, a);
+    return;
+  }
+  hipLaunchKernelGGL((expert_route_kernel<__bf16, ET, NW, true, 1>), dim3((unsigned)((a.n + 15) / 16)), dim3(64 * NW), NW * one, s, a);
 }
 
 static bool route_is_single(const RouteArgs& a, bool vec) { return a.n <= (vec && a.E <= 32 ? kRouteOneWg : 16); }
@@ -1018,7 +1082,7 @@ extern "C" BASED_API int based_expert_grouped(const void* h, const void* router,
   BASED_REQUIRE(aligned_to(h, 16) && aligned_to(w1, 16) && aligned_to(w2, 16) && aligned_to(work_act, 16) && aligned_to(work_out, 16) &&
                     aligned_to(y, 16),
                 BASED_ERR_ALIGN, "expert_grouped: tensors must be 16-byte aligned");
-  RouteArgs r{h, router, ids, scores, rank, counts, tile_first, tile_expert, order, 0, (long)n, (long)h_sr, (int)D, (int)E, (int)top};
+  RouteArgs r{h, router, ids, scores, rank, counts, nullptr, tile_first, tile_expert, order, 0, (long)n, (long)h_sr, (int)D, (int)E, (int)top};
   const int rc = route_check("expert_grouped", r);
   if (rc != BASED_OK) return rc;
   if (n == 0) return BASED_OK;
@@ -1029,13 +1093,22 @@ extern "C" BASED_API int based_expert_grouped(const void* h, const void* router,
   hipStream_t s = static_cast<hipStream_t>(stream);
   r.tile_rows = rows;
   const bool vec = route_vec(r);
+  const int group = route_group(r, vec);
+  const int64_t groups = (n + group - 1) / group;
+  const bool single = route_is_single(r, vec);
+  if (!single) {
+    // the workgroups' counts go where the activations come later; where that has no room for them, or they are too many to be read by
+    // every workgroup that places choices, the workgroups add theirs up (8192 tokens, 8 experts: clearing the counts and placing in two launches
+    // 12.4 us; by the workgroups' counts, in one launch 6.9)
+    if (groups * E <= kPlaceHist && groups * E * 4 <= tiles * rows * F * 2)
+      r.hist = static_cast<int32_t*>(work_act);
+    else
+      hipLaunchKernelGGL(expert_zero_kernel, dim3(1), dim3(kMaxExperts), 0, s, counts, (int)E);
+  }
   launch_route<__bf16>(r, vec, s);
-  if (!route_is_single(r, vec)) {
-    hipLaunchKernelGGL(expert_plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, counts, ids, rank, tile_first, tile_expert, order, (long)slots, (int)E,
-                       rows);
-    if (slots > kPlanSlots)
-      hipLaunchKernelGGL(expert_scatter_kernel, dim3((unsigned)((slots + 255) / 256)), dim3(256), 0, s, ids, rank, tile_first, order,
-                         (long)slots, rows);
+  if (!single) {
+    const PlaceArgs p{counts, r.hist, ids, rank, tile_first, tile_expert, order, (long)slots, (int)E, rows, (int)groups, (int)(group * top)};
+    hipLaunchKernelGGL(expert_place_kernel, dim3((unsigned)((groups + kPlaceGroups - 1) / kPlaceGroups)), dim3(kPlaceThreads), 0, s, p);
   }
   const ExpertGemmArgs a{static_cast<const __bf16*>(h), static_cast<const __bf16*>(w1), static_cast<__bf16*>(work_act), order, counts, tile_first,
                          tile_expert, scores, (long)h_sr, (int)E, (int)F, (int)D, (int)top, 0, (int)tiles};
@@ -1059,7 +1132,7 @@ extern "C" BASED_API int based_expert_rows(const void* x, const float* residual_
   BASED_REQUIRE(x && router && w1 && w2 && ids && scores && work_act && y, BASED_ERR_ARG, "expert_rows: null pointer argument");
   BASED_REQUIRE(F > 0 && D < (1 << 20) && F < (1 << 20), BASED_ERR_SHAPE, "expert_rows: grid too large");
   BASED_REQUIRE(io_dtype == BASED_BF16 || io_dtype == BASED_F32, BASED_ERR_DTYPE, "expert_rows: bad dtype");
-  RouteArgs r{x, router, ids, scores, nullptr, nullptr, nullptr, nullptr, nullptr, 0, (long)n, (long)x_sr, (int)D, (int)E, (int)top};
+  RouteArgs r{x, router, ids, scores, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, (long)n, (long)x_sr, (int)D, (int)E, (int)top};
   const int rc = route_check("expert_rows", r);
   if (rc != BASED_OK) return rc;
   const bool by_row = io_dtype == BASED_BF16 && D % 8 == 0 && D <= kRouteRowMax && x_sr % 8 == 0 && aligned_to(x, 16) && aligned_to(router, 16);

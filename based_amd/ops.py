@@ -1369,7 +1369,7 @@ def experts(h, router, w1, w2, top: int, norm=None) -> torch.Tensor:
         if grouped:
             tiles, rows = lib.based_expert_tiles(n, E, top), lib.based_expert_tile_rows(n, E, top)
             rank = torch.empty(n, top, **i32)
-            counts = (torch.empty if n <= 16 else torch.zeros)(E, **i32)  # (so few tokens are counted by one workgroup)
+            counts = torch.empty(E, **i32)
             plan = torch.empty(E + 1 + tiles + tiles * rows, **i32)
             act = torch.empty(tiles * rows, F, dtype=h2.dtype, device=dev)
             part = torch.empty(n * top, D, dtype=h2.dtype, device=dev) if top > 1 else None

@@ -690,7 +690,7 @@ BASED_API int based_latent_step(const void* q, const void* x, const void* norm_w
 
 /* Mixture of experts: scores = sigmoid(router h) in fp32, the `top` largest of a token into ids and scores (n, top), and
  * y = sum over them of w2_e (silu(gate) * up), [up; gate] = score * w1_e h; router (E, D), w1 (E, 2 F, D), w2 (E, D, F).
- * Grouped (bf16): rows of one expert share its matrices; scratch: rank (n, top), counts (E, zero on entry), tile_first (E + 1),
+ * Grouped (bf16): rows of one expert share its matrices; scratch: rank (n, top), counts (E), tile_first (E + 1),
  * tile_expert (tiles), order (tiles * rows), work_act (tiles * rows, F), work_out (n * top, D) with top > 1, tiles and rows from
  * based_expert_tiles / based_expert_tile_rows.  Rows: one choice at a time, for few tokens and any element type; work_act (n * top, F).
  * With norm_weight (D; bf16, D up to 4096) h is the norm of residual_in + mult * x as in based_add_norm, in work_h (n, D). */

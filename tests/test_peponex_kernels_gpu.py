@@ -553,3 +553,18 @@ def test_experts_in_large_tiles(dev, n, D, F, E, top):
     clear = torch.ones(n, dtype=torch.bool) if top == E else s[:, top - 1] - s[:, top] > 1e-5
     assert clear.sum() >= 0.98 * n
     close(got[clear], want[clear], 2 * TOL[BF16])
+
+
+@pytest.mark.parametrize("n,E,top", [(33, 8, 1), (4095, 8, 2), (4096, 32, 2), (4097, 8, 2), (4100, 33, 2), (4223, 70, 4), (5000, 130, 3), (20000, 64, 2), (40000, 128, 1)])
+def test_places_of_the_choices(dev, n, E, top):
+    """Every choice of a batch goes to the same expert as in batches of few tokens, whose places one workgroup plans: by the workgroups' counts (n E up
+    to a million in 32 tokens), by sums of them (beyond, or no room), with groups that end inside the last workgroup's eight."""
+    from based_amd import ops
+
+    h, router, w1, w2, _ = expert_case(n, 64, 16, E, top, BF16, seed=n)
+    args = [t.to(dev) for t in (router, w1, w2)]
+    whole = ops.experts(h.to(dev), *args, top)
+    rows = torch.randint(0, n, (64,), generator=torch.Generator().manual_seed(n))
+    rows[:2] = torch.tensor([0, n - 1])
+    alone = torch.cat([ops.experts(h[rows[i:i + 16]].to(dev), *args, top) for i in range(0, 64, 16)])
+    assert float((whole[rows.to(dev)].double() - alone.double()).norm() / alone.double().norm()) < 4e-3
