@@ -11,7 +11,8 @@
 //                   order: gate and up with the activation behind them, then down; expert_gemm_large: of 256 rows
 //   expert_sum      the choices of a token added up (with one choice the product writes the token's row)
 //   expert_route_row  the same for few tokens, with the norm in front of the layer
-//   expert_rows     few tokens, fp32, or rows that are no whole 16-byte pieces: dot products, one choice at a time
+//   expert_f32      fp32: 16 choices of one expert at a time on fp32 MFMA
+//   expert_rows     few tokens, or rows that are no whole 16-byte pieces: dot products, one choice at a time
 #include <atomic>
 
 #include "stream_common.hpp"
@@ -213,54 +214,59 @@ struct RouteRowArgs {
 
 constexpr int kRouteRowMax = 4096;  // channels
 
-__global__ __launch_bounds__(512) void expert_route_row_kernel(const RouteRowArgs a) {
-  __shared__ __attribute__((aligned(16))) __bf16 row[kRouteRowMax];
+template <typename T> __global__ __launch_bounds__(512) void expert_route_row_kernel(const RouteRowArgs a) {
+  constexpr int N = Pack<T>::kN;
+  __shared__ __attribute__((aligned(16))) T row[kRouteRowMax];
   __shared__ float s[kMaxExperts], part[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, D = a.r.D, E = a.r.E;
   const long n = blockIdx.x;
-  const __bf16* x = static_cast<const __bf16*>(a.r.h) + n * a.r.h_sr;
-  const int e8 = tid * 8;
-  const bool in = e8 < D;
-  float v[8];
-  load_vec<__bf16, 8>(x + (in ? e8 : 0), v);
-  if (a.norm_w != nullptr) {
-    float w8[8], r8[8];
-    load_vec<__bf16, 8>(a.norm_w + (in ? e8 : 0), w8);
+  const T* x = static_cast<const T*>(a.r.h) + n * a.r.h_sr;
+  if constexpr (sizeof(T) == 2) {
+    const int e8 = tid * 8;
+    const bool in = e8 < D;
+    float v[8];
+    load_vec<__bf16, 8>(x + (in ? e8 : 0), v);
+    if (a.norm_w != nullptr) {
+      float w8[8], r8[8];
+      load_vec<__bf16, 8>(a.norm_w + (in ? e8 : 0), w8);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) r8[i] = 0.f;
-    if (a.res_in != nullptr) load_vec<float, 8>(a.res_in + n * D + (in ? e8 : 0), r8);
-    const float mult = a.res_in != nullptr ? a.mult : 1.0f;
-    float sum = 0.f;
+      for (int i = 0; i < 8; ++i) r8[i] = 0.f;
+      if (a.res_in != nullptr) load_vec<float, 8>(a.res_in + n * D + (in ? e8 : 0), r8);
+      const float mult = a.res_in != nullptr ? a.mult : 1.0f;
+      float sum = 0.f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      v[i] = in ? __builtin_fmaf(mult, v[i], r8[i]) : 0.f;
-      sum += v[i];
+      for (int i = 0; i < 8; ++i) {
+        v[i] = in ? __builtin_fmaf(mult, v[i], r8[i]) : 0.f;
+        sum += v[i];
+      }
+      auto all = [&](float q, int at) {
+        q = sum16(q);
+        q += __shfl_xor(q, 16, 64);
+        q += __shfl_xor(q, 32, 64);
+        if (lane == 0) part[at + wave] = q;
+        __syncthreads();
+        float t = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) t += part[at + i];
+        return t;
+      };
+      if (a.res_out != nullptr && in) store_vec<float, 8>(a.res_out + n * D + e8, v);
+      const float mean = a.kind == BASED_NORM_LAYER ? all(sum, 0) / (float)D : 0.f;
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        v[i] = in ? v[i] - mean : 0.f;
+        ss = __builtin_fmaf(v[i], v[i], ss);
+      }
+      const float rstd = 1.0f / sqrtf(all(ss, 8) / (float)D + a.eps);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] *= rstd * w8[i];
+      if (in) store_vec<__bf16, 8>(a.h_out + n * D + e8, v);
     }
-    auto all = [&](float q, int at) {
-      q = sum16(q);
-      q += __shfl_xor(q, 16, 64);
-      q += __shfl_xor(q, 32, 64);
-      if (lane == 0) part[at + wave] = q;
-      __syncthreads();
-      float t = 0.f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) t += part[at + i];
-      return t;
-    };
-    if (a.res_out != nullptr && in) store_vec<float, 8>(a.res_out + n * D + e8, v);
-    const float mean = a.kind == BASED_NORM_LAYER ? all(sum, 0) / (float)D : 0.f;
-    float ss = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      v[i] = in ? v[i] - mean : 0.f;
-      ss = __builtin_fmaf(v[i], v[i], ss);
-    }
-    const float rstd = 1.0f / sqrtf(all(ss, 8) / (float)D + a.eps);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] *= rstd * w8[i];
-    if (in) store_vec<__bf16, 8>(a.h_out + n * D + e8, v);
+    if (in) store_vec<__bf16, 8>(row + e8, v);
+  } else {
+    for (int c = tid * N; c < D; c += 512 * N) *reinterpret_cast<f32x4*>(row + c) = *reinterpret_cast<const f32x4*>(x + c);
   }
-  if (in) store_vec<__bf16, 8>(row + e8, v);
   __syncthreads();
   constexpr int EU = 4;  // experts whose rows are in flight together
   for (int e0 = wave * EU; e0 < E; e0 += 8 * EU) {
@@ -268,15 +274,15 @@ __global__ __launch_bounds__(512) void expert_route_row_kernel(const RouteRowArg
 #pragma unroll
     for (int u = 0; u < EU; ++u) acc[u] = 0.f;
 #pragma unroll 2
-    for (int c = lane * 8; c < D; c += 512) {
-      float h8[8];
-      load_vec<__bf16, 8>(row + c, h8);
+    for (int c = lane * N; c < D; c += 64 * N) {
+      float h8[N];
+      load_vec<T, N>(row + c, h8);
 #pragma unroll
       for (int u = 0; u < EU; ++u) {
-        float w8[8];
-        load_vec<__bf16, 8>(static_cast<const __bf16*>(a.r.w) + (long)(e0 + u < E ? e0 + u : 0) * D + c, w8);
+        float w8[N];
+        load_vec<T, N>(static_cast<const T*>(a.r.w) + (long)(e0 + u < E ? e0 + u : 0) * D + c, w8);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) acc[u] = __builtin_fmaf(w8[i], h8[i], acc[u]);
+        for (int i = 0; i < N; ++i) acc[u] = __builtin_fmaf(w8[i], h8[i], acc[u]);
       }
     }
 #pragma unroll
@@ -865,22 +871,23 @@ template <bool PAIRED> int launch_expert_product(const ExpertGemmArgs& a, int ro
 }
 
 // y[n] = sum of the rows of its choices
-__global__ __launch_bounds__(256) void expert_sum_kernel(const __bf16* x, __bf16* y, long n, int D, int top) {
-  const int pieces = D / 8;
+template <typename T> __global__ __launch_bounds__(256) void expert_sum_kernel(const T* x, T* y, long n, int D, int top) {
+  constexpr int N = Pack<T>::kN;
+  const int pieces = D / N;
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   if (i >= n * pieces) return;
   const long row = i / pieces;
-  const int c = (int)(i % pieces) * 8;
-  float s[8];
+  const int c = (int)(i % pieces) * N;
+  float s[N];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) s[j] = 0.f;
+  for (int j = 0; j < N; ++j) s[j] = 0.f;
   for (int t = 0; t < top; ++t) {
-    float v[8];
-    load_vec<__bf16, 8>(x + (row * top + t) * D + c, v);
+    float v[N];
+    load_vec<T, N>(x + (row * top + t) * D + c, v);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) s[j] += v[j];
+    for (int j = 0; j < N; ++j) s[j] += v[j];
   }
-  store_vec<__bf16, 8>(y + row * D + c, s);
+  store_vec<T, N>(y + row * D + c, s);
 }
 
 // ---- one choice at a time ----
@@ -998,6 +1005,133 @@ template <typename T, bool PAIRED> void launch_expert_rows_vec(const ExpertRowsA
     launch_expert_rows<T, 1, PAIRED>(a, items, s);
 }
 
+// ---- fp32, rows of one expert on fp32 MFMA ----
+// 16 features (PAIRED: of up and of gate) of one expert per workgroup, which looks its choices up among all and takes 16 of them at a time; its
+// eight wavefronts share the channels, each with its part of the matrices in registers for all of the choices, and add their sums up at the
+// end of each 16.  Bound by reading the matrices, once each, where one choice at a time reads them for every choice: 12 tokens, 4 of 16 experts
+// of 512: 49 us by choices, 54 here; 20 tokens 66 and 54; 140 tokens, 1 of 8 of 2048: 250 and 96; 256 tokens, 4 of 16 of 512: 296 and 117.
+constexpr int kF32Features = 16, kF32Scan = 1024;
+
+struct ExpertF32Args {
+  const float* x;  // PAIRED: (N, K); otherwise (N * top, K)
+  const float* w;  // (E, 2 F, K) / (E, F, K)
+  float* y;        // (N * top, F)
+  const int32_t* ids;
+  const float* scores;
+  long slots, x_sr;
+  int F, K, top;
+};
+
+template <bool PAIRED> __global__ __launch_bounds__(512) void expert_f32_kernel(const ExpertF32Args a) {
+  constexpr int WT = PAIRED ? 2 : 1, S = 16 / WT;  // pieces of 16 channels in registers
+  __shared__ int list[kF32Scan];
+  __shared__ int found[8];
+  __shared__ __attribute__((aligned(16))) float sums[2][8][WT][256];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, quad = lane >> 4;
+  const int e = blockIdx.y, f0 = blockIdx.x * kF32Features;
+  const int pieces = (a.K + 15) / 16, per = (pieces + 7) / 8, p_begin = wave * per, p_end = p_begin + per < pieces ? p_begin + per : pieces;
+  const float* w = a.w + ((long)e * WT * a.F + (f0 + l16 < a.F ? f0 + l16 : a.F - 1)) * a.K;
+  f32x4 wf[WT][S], xf[S];
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  auto channel = [&](int p) { return p * 16 + quad * 4; };
+  auto there = [&](int p) { return p < p_end && channel(p) < a.K; };
+  auto load_w = [&](int p0) {
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+      for (int t = 0; t < WT; ++t) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(w + (long)t * a.F * a.K + (there(p0 + s) ? channel(p0 + s) : 0));
+        wf[t][s] = there(p0 + s) ? v : zero;
+      }
+  };
+  if (per <= S) load_w(p_begin);  // (the caller has several choices for an expert: few of them are not used)
+  int parity = 0;
+  for (long s0 = 0; s0 < a.slots; s0 += kF32Scan) {
+    // this expert's among the next choices, in their order
+    int at = 0, n = 0;
+    bool mine[kF32Scan / 512];
+    int before[kF32Scan / 512];
+#pragma unroll
+    for (int i = 0; i < kF32Scan / 512; ++i) {
+      const long slot = s0 + i * 512 + tid;
+      mine[i] = slot < a.slots && a.ids[slot < a.slots ? slot : 0] == e;
+    }
+#pragma unroll
+    for (int i = 0; i < kF32Scan / 512; ++i) {
+      const uint64_t b = __ballot(mine[i]);
+      before[i] = __popcll(b & ((1ull << lane) - 1));
+      if (lane == 0) found[wave] = __popcll(b);
+      __syncthreads();
+      at = n;
+      for (int v = 0; v < 8; ++v) {
+        if (v < wave) at += found[v];
+        n += found[v];
+      }
+      if (mine[i]) list[at + before[i]] = (int)(s0 + i * 512 + tid);
+      __syncthreads();
+    }
+    for (int r0 = 0; r0 < n; r0 += 16, parity ^= 1) {
+      const int slot = list[r0 + l16 < n ? r0 + l16 : r0];
+      const float* x = a.x + (PAIRED ? slot / a.top : slot) * a.x_sr;
+      f32x4 acc[WT][S];  // (short chains round less)
+#pragma unroll
+      for (int t = 0; t < WT; ++t)
+#pragma unroll
+        for (int s = 0; s < S; ++s) acc[t][s] = zero;
+      for (int p0 = p_begin; p0 < p_begin + per; p0 += S) {
+#pragma unroll
+        for (int s4 = 0; s4 < S; s4 += 4)
+          if (p0 + s4 < p_end) {
+#pragma unroll
+            for (int s = s4; s < s4 + 4; ++s) {
+              const f32x4 v = *reinterpret_cast<const f32x4*>(x + (there(p0 + s) ? channel(p0 + s) : 0));
+              xf[s] = there(p0 + s) ? v : zero;
+            }
+          }
+        if (per > S) load_w(p0);
+#pragma unroll
+        for (int s4 = 0; s4 < S; s4 += 4)
+          if (p0 + s4 < p_end)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+              for (int s = s4; s < s4 + 4; ++s)
+#pragma unroll
+                for (int t = 0; t < WT; ++t) acc[t][s] = mfma_f32(wf[t][s][j], xf[s][j], acc[t][s]);
+      }
+      // column = choice l16, rows = features 4 quad + i
+#pragma unroll
+      for (int t = 0; t < WT; ++t) {
+#pragma unroll
+        for (int m = 1; m < S; m <<= 1)
+#pragma unroll
+          for (int s = 0; s < S; s += 2 * m) acc[t][s] += acc[t][s + m];
+        *reinterpret_cast<f32x4*>(&sums[parity][wave][t][lane * 4]) = acc[t][0];
+      }
+      __syncthreads();  // (the other half of sums is read before this one comes round again)
+      const int r = tid >> 4, f = f0 + l16, i = ((l16 >> 2) * 16 + r) * 4 + (l16 & 3);
+      if (tid < 256 && r0 + r < n && f < a.F) {
+        float z[WT];
+#pragma unroll
+        for (int t = 0; t < WT; ++t) {
+          float q[8];
+#pragma unroll
+          for (int v = 0; v < 8; ++v) q[v] = sums[parity][v][t][i];
+          z[t] = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
+        }
+        const long out = list[r0 + r];
+        if constexpr (PAIRED) {
+          const float score = a.scores[out];
+          a.y[out * a.F + f] = silu_exact(z[1] * score) * (z[0] * score);
+        } else {
+          a.y[out * a.F + f] = z[0];
+        }
+      }
+    }
+    __syncthreads();  // (the list is written again)
+  }
+}
+
 constexpr int kRouteOneWg = 32;  // tokens that one workgroup routes, of up to 32 experts (16 of more): it makes the plan too
 
 // Tokens of one workgroup.  Many tokens of few experts: 32, their rows shared out over eight wavefronts (8192 tokens of 1024 channels, 8 experts:
@@ -1044,6 +1178,19 @@ template <typename T> void launch_route(RouteArgs a, bool vec, hipStream_t s) {
 
 static bool route_vec(const RouteArgs& a) {
   return a.D % 8 == 0 && a.h_sr % 8 == 0 && a.E <= 128 && aligned_to(a.h, 16) && aligned_to(a.w, 16);
+}
+
+static bool route_by_row(const RouteArgs& a, int piece) {
+  return a.D % piece == 0 && a.D <= kRouteRowMax && a.h_sr % piece == 0 && aligned_to(a.h, 16) && aligned_to(a.w, 16);
+}
+
+// A workgroup to each token (element by element, a score to a thread, 12 tokens of 1024 channels took 70 us)
+static void launch_route_f32(const RouteArgs& r, bool by_row, hipStream_t s) {
+  if (by_row)
+    hipLaunchKernelGGL(expert_route_row_kernel<float>, dim3((unsigned)r.n), dim3(512), 0, s,
+                       RouteRowArgs{r, nullptr, nullptr, nullptr, nullptr, 1.f, 0.f, BASED_NORM_RMS});
+  else
+    launch_route<float>(r, false, s);
 }
 
 static int route_check(const char* who, const RouteArgs& a) {
@@ -1119,7 +1266,7 @@ extern "C" BASED_API int based_expert_grouped(const void* h, const void* router,
   if (done == BASED_OK) done = launch_expert_product<false>(a2, rows, s);
   if (done != BASED_OK) return done;
   if (top > 1)
-    hipLaunchKernelGGL(expert_sum_kernel, dim3((unsigned)((n * (D / 8) + 255) / 256)), dim3(256), 0, s, out, static_cast<__bf16*>(y), (long)n,
+    hipLaunchKernelGGL(expert_sum_kernel<__bf16>, dim3((unsigned)((n * (D / 8) + 255) / 256)), dim3(256), 0, s, out, static_cast<__bf16*>(y), (long)n,
                        (int)D, (int)top);
   return check_launch("expert_grouped");
 }
@@ -1135,9 +1282,9 @@ extern "C" BASED_API int based_expert_rows(const void* x, const float* residual_
   RouteArgs r{x, router, ids, scores, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, (long)n, (long)x_sr, (int)D, (int)E, (int)top};
   const int rc = route_check("expert_rows", r);
   if (rc != BASED_OK) return rc;
-  const bool by_row = io_dtype == BASED_BF16 && D % 8 == 0 && D <= kRouteRowMax && x_sr % 8 == 0 && aligned_to(x, 16) && aligned_to(router, 16);
+  const bool by_row = route_by_row(r, io_dtype == BASED_BF16 ? 8 : 4);
   if (norm_weight != nullptr) {
-    BASED_REQUIRE(by_row, BASED_ERR_SHAPE, "expert_rows: the norm takes bf16 rows of a multiple of 8 up to %d channels", kRouteRowMax);
+    BASED_REQUIRE(by_row && io_dtype == BASED_BF16, BASED_ERR_SHAPE, "expert_rows: the norm takes bf16 rows of a multiple of 8 up to %d channels", kRouteRowMax);
     BASED_REQUIRE(work_h && (norm_kind == BASED_NORM_RMS || norm_kind == BASED_NORM_LAYER) && residual_out != residual_in, BASED_ERR_ARG,
                   "expert_rows: bad norm arguments");
     BASED_REQUIRE(aligned_to(norm_weight, 16) && aligned_to(residual_in, 16) && aligned_to(residual_out, 16) && aligned_to(work_h, 16),
@@ -1147,13 +1294,13 @@ extern "C" BASED_API int based_expert_rows(const void* x, const float* residual_
   hipStream_t s = static_cast<hipStream_t>(stream);
   const void* h = norm_weight != nullptr ? work_h : x;
   const int64_t h_sr = norm_weight != nullptr ? D : x_sr;
-  if (norm_weight != nullptr || (by_row && n <= 16)) {
+  if (norm_weight != nullptr || (by_row && io_dtype == BASED_BF16 && n <= 16)) {
     const RouteRowArgs a{r, residual_in, residual_out, static_cast<const __bf16*>(norm_weight), static_cast<__bf16*>(work_h), mult, eps, norm_kind};
-    hipLaunchKernelGGL(expert_route_row_kernel, dim3((unsigned)n), dim3(512), 0, s, a);
+    hipLaunchKernelGGL(expert_route_row_kernel<__bf16>, dim3((unsigned)n), dim3(512), 0, s, a);
   } else if (io_dtype == BASED_BF16) {
     launch_route<__bf16>(r, route_vec(r), s);
   } else {
-    launch_route<float>(r, false, s);
+    launch_route_f32(r, by_row, s);
   }
   const int p = io_dtype == BASED_BF16 ? 8 : 4;
   const bool vec1 = D % p == 0 && h_sr % p == 0 && aligned_to(h, 16) && aligned_to(w1, 16);
@@ -1168,4 +1315,33 @@ extern "C" BASED_API int based_expert_rows(const void* x, const float* residual_
     launch_expert_rows_vec<float, false>(a2, vec2, n, s);
   }
   return check_launch("expert_rows");
+}
+
+extern "C" BASED_API int based_expert_grouped_f32(const float* h, const float* router, const float* w1, const float* w2, int32_t* ids, float* scores,
+                                                  float* work_act, float* work_out, float* y, int64_t n, int64_t D, int64_t F, int64_t E,
+                                                  int64_t top, int64_t h_sr, void* stream) {
+  using namespace based;
+  BASED_REQUIRE(h && router && w1 && w2 && ids && scores && work_act && y, BASED_ERR_ARG, "expert_grouped_f32: null pointer argument");
+  BASED_REQUIRE(F > 0 && D < (1 << 20) && F < (1 << 20), BASED_ERR_SHAPE, "expert_grouped_f32: grid too large");
+  BASED_REQUIRE(top == 1 || work_out != nullptr, BASED_ERR_ARG, "expert_grouped_f32: several choices per token need work_out");
+  BASED_REQUIRE(D % 4 == 0 && F % 4 == 0 && h_sr % 4 == 0, BASED_ERR_SHAPE, "expert_grouped_f32: sizes %ld and %ld must be multiples of 4", (long)D,
+                (long)F);
+  BASED_REQUIRE(aligned_to(h, 16) && aligned_to(w1, 16) && aligned_to(w2, 16) && aligned_to(work_act, 16) && aligned_to(work_out, 16) &&
+                    aligned_to(y, 16),
+                BASED_ERR_ALIGN, "expert_grouped_f32: tensors must be 16-byte aligned");
+  const RouteArgs r{h, router, ids, scores, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, (long)n, (long)h_sr, (int)D, (int)E, (int)top};
+  const int rc = route_check("expert_grouped_f32", r);
+  if (rc != BASED_OK) return rc;
+  if (n == 0) return BASED_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  launch_route_f32(r, route_by_row(r, 4), s);
+  const auto grid = [&](int64_t features) { return dim3((unsigned)((features + kF32Features - 1) / kF32Features), (unsigned)E); };
+  float* out = top == 1 ? y : work_out;
+  hipLaunchKernelGGL(expert_f32_kernel<true>, grid(F), dim3(512), 0, s,
+                     ExpertF32Args{h, w1, work_act, ids, scores, (long)(n * top), (long)h_sr, (int)F, (int)D, (int)top});
+  hipLaunchKernelGGL(expert_f32_kernel<false>, grid(D), dim3(512), 0, s,
+                     ExpertF32Args{work_act, w2, out, ids, scores, (long)(n * top), (long)F, (int)D, (int)F, (int)top});
+  if (top > 1)
+    hipLaunchKernelGGL(expert_sum_kernel<float>, dim3((unsigned)((n * (D / 4) + 255) / 256)), dim3(256), 0, s, out, y, (long)n, (int)D, (int)top);
+  return check_launch("expert_grouped_f32");
 }

@@ -1327,6 +1327,9 @@ def latent_step(q, x, norm_weight, weight, cache, heads: int, dim: int, window: 
 
 # Choices up to which experts are evaluated one choice at a time: beyond, rows of one expert share its matrices.
 EXPERT_ROWS_MAX = 16
+# fp32 choices per expert likewise: 2 of 8 experts of 1024, 6 tokens 30.7 us by rows and 46.8 grouped, 20 tokens 68 and 49; 1 of 8 of 2048, 16 tokens
+# 65 and 80, 24 tokens 88 and 80; 4 of 16 of 512, 12 tokens 48 and 54, 20 tokens 66 and 54.
+EXPERT_ROWS_F32_MAX = 3
 EXPERT_NORM_MAX_DIM = 4096
 
 
@@ -1376,6 +1379,13 @@ def experts(h, router, w1, w2, top: int, norm=None) -> torch.Tensor:
             _lib.check(lib.based_expert_grouped(
                 h2.data_ptr(), router.data_ptr(), w1.data_ptr(), w2.data_ptr(), ids.data_ptr(), scores.data_ptr(), rank.data_ptr(),
                 counts.data_ptr(), plan.data_ptr(), plan[E + 1:].data_ptr(), plan[E + 1 + tiles:].data_ptr(), act.data_ptr(), _ptr(part),
+                y.data_ptr(), n, D, F, E, top, h2.stride(0), _stream_ptr(h2)))
+        elif (h2.dtype == torch.float32 and n * top > EXPERT_ROWS_F32_MAX * E and D % 4 == 0 and F % 4 == 0 and h2.stride(0) % 4 == 0
+              and not (h2.data_ptr() | w1.data_ptr() | w2.data_ptr()) & 15):
+            act = torch.empty(n * top, F, dtype=h2.dtype, device=dev)
+            part = torch.empty(n * top, D, dtype=h2.dtype, device=dev) if top > 1 else None
+            _lib.check(lib.based_expert_grouped_f32(
+                h2.data_ptr(), router.data_ptr(), w1.data_ptr(), w2.data_ptr(), ids.data_ptr(), scores.data_ptr(), act.data_ptr(), _ptr(part),
                 y.data_ptr(), n, D, F, E, top, h2.stride(0), _stream_ptr(h2)))
         else:
             act = torch.empty(n * top, F, dtype=h2.dtype, device=dev)

@@ -693,6 +693,7 @@ BASED_API int based_latent_step(const void* q, const void* x, const void* norm_w
  * Grouped (bf16): rows of one expert share its matrices; scratch: rank (n, top), counts (E), tile_first (E + 1),
  * tile_expert (tiles), order (tiles * rows), work_act (tiles * rows, F), work_out (n * top, D) with top > 1, tiles and rows from
  * based_expert_tiles / based_expert_tile_rows.  Rows: one choice at a time, for few tokens and any element type; work_act (n * top, F).
+ * Grouped, fp32: sizes and h_sr multiples of 4; work_act (n * top, F), work_out (n * top, D) with top > 1.
  * With norm_weight (D; bf16, D up to 4096) h is the norm of residual_in + mult * x as in based_add_norm, in work_h (n, D). */
 #define BASED_EXPERT_TILE_ROWS 256
 #define BASED_EXPERT_TILE_ROWS_SMALL 32
@@ -702,6 +703,9 @@ BASED_API int based_expert_grouped(const void* h, const void* router, const void
                                    int32_t* rank, int32_t* counts, int32_t* tile_first, int32_t* tile_expert, int32_t* order,
                                    void* work_act, void* work_out, void* y, int64_t n, int64_t D, int64_t F, int64_t E, int64_t top,
                                    int64_t h_sr, void* stream);
+BASED_API int based_expert_grouped_f32(const float* h, const float* router, const float* w1, const float* w2, int32_t* ids, float* scores,
+                                       float* work_act, float* work_out, float* y, int64_t n, int64_t D, int64_t F, int64_t E, int64_t top,
+                                       int64_t h_sr, void* stream);
 BASED_API int based_expert_rows(const void* x, const float* residual_in, float* residual_out, const void* norm_weight, void* work_h,
                                 float mult, int norm_kind, float eps, const void* router, const void* w1, const void* w2,
                                 int32_t* ids, float* scores, void* work_act, void* y, int64_t n, int64_t D, int64_t F, int64_t E,
