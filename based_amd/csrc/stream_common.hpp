@@ -90,6 +90,17 @@ __device__ __forceinline__ float sum16(float v) {
   return dpp_move_add<0x140>(v);  // row_mirror
 }
 
+// Largest of the lanes l, l ^ 16, l ^ 32, l ^ 48, in each of them, by exchanges of rows on the vector unit (through LDS a round trip each).
+__device__ __forceinline__ float max_quads(float v) {
+  const unsigned x = __builtin_bit_cast(unsigned, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  const unsigned r0 = r[0], r1 = r[1];
+  const unsigned y = __builtin_bit_cast(unsigned, fmaxf(__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1)));
+  const auto q = __builtin_amdgcn_permlane32_swap(y, y, false, false);
+  const unsigned q0 = q[0], q1 = q[1];
+  return fmaxf(__builtin_bit_cast(float, q0), __builtin_bit_cast(float, q1));
+}
+
 inline bool aligned_to(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
 
 // Sum of w_j x_{t - taps + 1 + j} over the past inputs of one channel of a ring (taps slots, `stride` elements

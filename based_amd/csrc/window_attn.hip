@@ -162,12 +162,16 @@ __global__ __launch_bounds__(256) void window_kv_write_vec_kernel(const WindowAr
 constexpr int kTileKeys = 64;
 constexpr int kTileRows = 128;  // (token, head) rows per workgroup
 
+// Bound by the vector unit and by waiting for the tiles: as many wavefronts as fit.  Sizes up to 64 run in 128 registers, four
+// workgroups to a compute unit (three, with 143, and the maxima of rows exchanged through LDS): 16 heads on 4 of 64 channels, with the cache
+// write, 4 x 2048 tokens and 129 keys 28.9 -> 24.8 us; on 16 44.4 -> 39.5; 6 x 2240 tokens and 513 keys 81.8 -> 73.9; one of 700 26.2 -> 23.1.
+
 __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
 template <int KC, int VC, bool HALF>
-__global__ __launch_bounds__(256, KC <= 3 && VC <= 2 ? 3 : 1) void window_prefill_mfma_kernel(const WindowArgs a) {
+__global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 3 : 1) void window_prefill_mfma_kernel(const WindowArgs a) {
   constexpr int D = KC * 32, DV = VC * 32;
   constexpr int KS = D + 8, VS = kTileKeys + 8;  // LDS row strides: 16-lane reads of 16 bytes meet every bank once
   __shared__ __attribute__((aligned(16))) __bf16 lds_k[kTileKeys * KS];
@@ -184,16 +188,15 @@ __global__ __launch_bounds__(256, KC <= 3 && VC <= 2 ? 3 : 1) void window_prefil
   // queries: lane holds channels quad*8 + 32 c .. of row l16 (+16): the MFMA's second operand.  Turned and
   // rounded after the first tile of keys has been asked for.
   bf16x8 qf[2][KC];
-  int qpos[2], qtok[2], qhead[2];
+  int qpos[2];
   const __bf16* qrow[2];
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
     const int row = row_w + t * 16 + l16;
     const int rr = row < n_rows ? row : n_rows - 1;
-    qtok[t] = rr / qpk;
-    qhead[t] = g * qpk + rr % qpk;
-    qpos[t] = a.pos_host + qtok[t];
-    qrow[t] = static_cast<const __bf16*>(a.q) + b * a.q_sb + qtok[t] * a.q_sl + (long)qhead[t] * a.d;
+    const int tok = rr / qpk;
+    qpos[t] = a.pos_host + tok;
+    qrow[t] = static_cast<const __bf16*>(a.q) + b * a.q_sb + tok * a.q_sl + (long)(g * qpk + rr - tok * qpk) * a.d;
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
       const int e = c * 32 + quad * 8;
@@ -204,23 +207,17 @@ __global__ __launch_bounds__(256, KC <= 3 && VC <= 2 ? 3 : 1) void window_prefil
   const int wave_hi_row = row_w + 31 < n_rows ? row_w + 31 : n_rows - 1;
   const int wave_hi_tok = a.pos_host + wave_hi_row / qpk;
 
-  f32x4 acc[2][2 * VC];
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int i = 0; i < 2 * VC; ++i) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
-  const float scale2 = fabsf(a.scale) * 1.4426950408889634f;  // scores in powers of two; the sign is the queries'
-
   const int first_pos = a.pos_host + r0 / qpk, last_pos = a.pos_host + (r_end - 1) / qpk;
   const int lo = first_pos - a.window + 1 > 0 ? first_pos - a.window + 1 : 0;
 
-  // staging: keys as 16-byte pieces of rows; values as 4 keys x 8 channels, turned on the way
+  // staging: keys as 16-byte pieces of rows; values as VK keys x 8 channels, turned on the way
   constexpr int KP = kTileKeys * (D / 8) / 256;  // pieces per thread
-  constexpr int VP = 16 * (DV / 8) / 256 > 0 ? 16 * (DV / 8) / 256 : 1;
+  constexpr int VK = VC >= 4 ? 4 : 2, VN = kTileKeys / VK;
+  constexpr int VP = VN * (DV / 8) / 256 > 0 ? VN * (DV / 8) / 256 : 1;
+  typedef __attribute__((ext_vector_type(VK))) __bf16 bf16xk;
   typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
   u32x4 kbuf[KP];
-  u32x4 vbuf[VP][4];
+  u32x4 vbuf[VP][VK];
   const u32x4 zero4 = {0u, 0u, 0u, 0u};
   // rows past the last key and channels past the sizes are fetched from valid places and cleared in `stage`
   const int st32 = (int)a.kv_st;
@@ -234,10 +231,10 @@ __global__ __launch_bounds__(256, KC <= 3 && VC <= 2 ? 3 : 1) void window_prefil
     }
 #pragma unroll
     for (int i = 0; i < VP; ++i) {
-      const int p = i * 256 + tid, k4 = p & 15, e = (p >> 4) * 8;
+      const int p = i * 256 + tid, kv0 = p % VN * VK, e = p / VN * 8;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int key = k4 * 4 + r;
+      for (int r = 0; r < VK; ++r) {
+        const int key = kv0 + r;
         vbuf[i][r] = *reinterpret_cast<const u32x4*>(tile + ((key <= last ? key : last) * st32 + a.d + (e < a.dv ? e : 0)));
       }
     }
@@ -250,16 +247,16 @@ __global__ __launch_bounds__(256, KC <= 3 && VC <= 2 ? 3 : 1) void window_prefil
     }
 #pragma unroll
     for (int i = 0; i < VP; ++i) {
-      const int p = i * 256 + tid, k4 = p & 15, e = (p >> 4) * 8;
+      const int p = i * 256 + tid, kv0 = p % VN * VK, e = p / VN * 8;
       if (e < DV) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) vbuf[i][r] = e < a.dv ? vbuf[i][r] : zero4;
+        for (int r = 0; r < VK; ++r) vbuf[i][r] = e < a.dv ? vbuf[i][r] : zero4;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          bf16x4 col;
+          bf16xk col;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) col[r] = __builtin_bit_cast(bf16x8, vbuf[i][r])[j];
-          *reinterpret_cast<bf16x4*>(&lds_v[(e + j) * VS + k4 * 4]) = col;
+          for (int r = 0; r < VK; ++r) col[r] = __builtin_bit_cast(bf16x8, vbuf[i][r])[j];
+          *reinterpret_cast<bf16xk*>(&lds_v[(e + j) * VS + kv0]) = col;
         }
       }
     }
@@ -267,7 +264,7 @@ __global__ __launch_bounds__(256, KC <= 3 && VC <= 2 ? 3 : 1) void window_prefil
 
   fetch(lo);
   if (a.rot > 0) {
-    constexpr int CB = KC == 3 ? 1 : KC < 4 ? KC : 4;
+    constexpr int CB = KC == 3 || (HALF && KC == 2) ? 1 : KC < 4 ? KC : 4;
 #pragma unroll
     for (int c0 = 0; c0 < KC; c0 += CB) {
       Turn8<HALF> turn[2][CB];
@@ -306,6 +303,14 @@ __global__ __launch_bounds__(256, KC <= 3 && VC <= 2 ? 3 : 1) void window_prefil
           for (int j = 0; j < 8; ++j) qf[t][c][j] = (__bf16)0.f;
       }
   }
+  __builtin_amdgcn_sched_barrier(0);  // (the accumulators take their registers from here on)
+  f32x4 acc[2][2 * VC];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int i = 0; i < 2 * VC; ++i) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
+  const float scale2 = fabsf(a.scale) * 1.4426950408889634f;  // scores in powers of two; the sign is the queries'
   for (int k0 = lo; k0 <= last_pos; k0 += kTileKeys) {
     __syncthreads();  // every wavefront is done with the tile before
     stage();
@@ -343,8 +348,7 @@ __global__ __launch_bounds__(256, KC <= 3 && VC <= 2 ? 3 : 1) void window_prefil
             s[t][kt][i] = sc;
             mx = fmaxf(mx, sc);
           }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = max_quads(mx);
         if (__any(mx > m_run[t])) {
           const float m_new = fmaxf(m_run[t], mx);
           // no key seen yet: every weight is 2^-inf = 0
@@ -376,14 +380,17 @@ __global__ __launch_bounds__(256, KC <= 3 && VC <= 2 ? 3 : 1) void window_prefil
       }
     }
   }
+  int row_end = row_w;
+  asm volatile("" : "+v"(row_end));  // (where a row goes is worked out again: kept, it would be a register too many)
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
     float l = l_run[t];
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
     const float inv = a.out_scale / l;
-    if (row_w + t * 16 + l16 < n_rows) {
-      __bf16* op = static_cast<__bf16*>(a.o) + b * a.o_sb + qtok[t] * a.o_sl + (long)qhead[t] * a.dv;
+    const int row = row_end + t * 16 + l16, tok = row / qpk;
+    if (row < n_rows) {
+      __bf16* op = static_cast<__bf16*>(a.o) + b * a.o_sb + tok * a.o_sl + (long)(g * qpk + row - tok * qpk) * a.dv;
 #pragma unroll
       for (int i = 0; i < 2 * VC; ++i) {
         const int e = i * 16 + quad * 4;
@@ -565,8 +572,7 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(const WindowArg
         s[kt][i] = sc;
         mx = fmaxf(mx, sc);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max_quads(mx);
     if (__any(mx > m_run)) {
       const float m_new = fmaxf(m_run, mx);
       // no key seen yet: every weight is 2^-inf = 0
