@@ -11,6 +11,7 @@ import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libbased_hip.so")  # the in-tree build of every kernel
+BINDING_PATH = os.path.join(_HERE, "_binding.so")  # its entry points as Python callables, cheaper to call than through ctypes
 # Builds of some of the sources (based_amd.build.build_part) lie beside it; `use_part` selects one
 # where the whole library has not been built.
 _part_path = None
@@ -202,6 +203,9 @@ class _Entries:
     """The typed entry points of a loaded library."""
 
     def __init__(self, handle, partial: bool):
+        bind = lambda name, fn: fn  # noqa: E731
+        if not partial and os.path.exists(BINDING_PATH):  # (built with the library, of the same header)
+            from ._binding import bind
         for name, (res, args) in SIGNATURES.items():
             if partial and not hasattr(handle, name):
                 setattr(self, name, _absent(name))
@@ -209,7 +213,7 @@ class _Entries:
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
-            setattr(self, name, fn)
+            setattr(self, name, bind(name, fn))
 
 
 def lib():

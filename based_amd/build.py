@@ -12,12 +12,14 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 OBJDIR = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libbased_hip.so")
+BINDING = os.path.join(HERE, "_binding.so")
 
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 FLAGS = [
@@ -84,6 +86,17 @@ def _link(objs, out: str) -> None:
     os.replace(tmp, out)
 
 
+def _build_binding() -> None:
+    """csrc/binding.cpp, the entry points of LIB as Python callables."""
+    tmp = f"{BINDING}.{os.getpid()}.tmp"
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-Wall", "-I", INCLUDE,
+           "-I", sysconfig.get_paths()["include"], os.path.join(CSRC, "binding.cpp"), "-L", HERE, "-l:libbased_hip.so", "-Wl,-rpath,$ORIGIN", "-o", tmp]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"binding build failed:\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, BINDING)
+
+
 def build_part(part: str) -> str:
     """Compiles the sources of one part into a library of its own (based_amd/_lib.py: use_part)."""
     from ._lib import part_path
@@ -116,6 +129,7 @@ def build(verbose: bool = False) -> str:
             if u.get("VGPRs Spill", 0) > 0:
                 sys.stderr.write(f"note: {src}: {name} spills {u['VGPRs Spill']} vector registers\n")
     _link(objs, LIB)
+    _build_binding()
     if verbose:
         print(f"built {LIB} from {len(srcs)} sources")
     return LIB

@@ -34,28 +34,48 @@ def _stream_ptr(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
-class _on_device:
-    """Enters `torch.cuda.device(dev)` only when dev is not already current (entering the context
-    costs microseconds, which matters for single-token steps)."""
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device  # (a tensor is there: so is the runtime)
 
-    __slots__ = ("ctx",)
 
-    def __init__(self, dev: torch.device):
-        self.ctx = None if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
+class _Here:
+    """What `with` wants where nothing is to be done."""
+
+    __slots__ = ()
 
     def __enter__(self):
-        if self.ctx is not None:
-            self.ctx.__enter__()
+        return None
 
     def __exit__(self, *exc):
-        if self.ctx is not None:
-            self.ctx.__exit__(*exc)
         return False
 
 
-# Argument checks of the single-token entry points are done once per distinct combination of
-# shapes, strides, dtypes and device (a decode loop presents the same combination every step).
-_CHECKED: dict = {}
+_HERE = _Here()
+
+
+def _on_device(dev: torch.device):
+    """`torch.cuda.device(dev)` where dev is not already current (entering the context costs microseconds, which matters for
+    single-token steps)."""
+    return _HERE if _current_device() == dev.index else torch.cuda.device(dev)
+
+
+class _Checked(dict):
+    """A dict that starts again when it is full: prompts come in any number of lengths."""
+
+    def __setitem__(self, key, value):
+        if len(self) >= 4096:
+            self.clear()
+        dict.__setitem__(self, key, value)
+
+
+# Argument checks are done once per distinct combination of shapes, strides, dtypes and devices (a decode loop presents the same
+# combination every step, the layers of a prefill the same few), and what the library is told of them is kept with it: 16 heads on 4,
+# 2 x 5 tokens of window attention 17.0 -> 11.1 us a call, most of it the checks and the conversion of forty arguments.
+_CHECKED: dict = _Checked()
+
+
+def _form(*ts):
+    """Everything that the checks look at, of each tensor (or None)."""
+    return tuple([None if t is None else (t.shape, t.stride(), t.dtype, t.device) for t in ts])
 
 
 def _require_cuda(*ts: torch.Tensor) -> None:
@@ -239,6 +259,33 @@ def swa_prefill(q, k, v, w_left: int = 64, scale: Optional[float] = None, rope=N
     (rotated) k and v.  out: None or a (B, L, H, D) tensor (last dim contiguous) to write into.
     impl: None (MFMA kernels), "wide" (the general MFMA kernel also where the 64-channel one would
     do) or "plain" (the one-wavefront-per-query kernel, no rotary: a second statement for tests)."""
+    cos, sin, turned = (None, None, None) if rope is None else (rope[0], rope[1], bool(rope[2]) if len(rope) > 2 else False)
+    key = ("swa_prefill", impl, turned, _form(q, k, v, kv_cache, cos, sin))
+    plan = _CHECKED.get(key)
+    if plan is None:
+        plan = _CHECKED[key] = _swa_prefill_plan(q, k, v, rope, kv_cache, impl)
+    B, L, H, D, name, at, n_pos, rotary, cache_at, code, default_scale = plan
+    scale = default_scale if scale is None else float(scale)
+    if out is None:
+        o = torch.empty(B, L, H, D, dtype=q.dtype, device=q.device)
+    else:
+        o = out
+        if tuple(o.shape) != (B, L, H, D) or o.dtype != q.dtype or o.device != q.device or o.stride(-1) != 1:
+            raise ValueError(f"out must be a ({B}, {L}, {H}, {D}) {q.dtype} tensor on {q.device}")
+    kc_ptr = vc_ptr = None
+    if kv_cache is not None:
+        kc_ptr = kv_cache.data_ptr()
+        vc_ptr = kc_ptr + kv_cache.stride(2) * kv_cache.element_size()
+    run = getattr(_lib.lib(), name)
+    tables = () if rotary is None else (_ptr(cos), _ptr(sin), n_pos, *rotary)
+    with _on_device(q.device):
+        _lib.check(run(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), *at, o.stride(0), o.stride(1), o.stride(2), int(w_left), scale, *tables,
+                       kc_ptr, vc_ptr, *cache_at, code, _stream_ptr(q)))
+    return o
+
+
+def _swa_prefill_plan(q, k, v, rope, kv_cache, impl):
+    """The checked sizes and strides of a swa_prefill call, and the entry that takes it."""
     _require_cuda(q, k, v)
     B, L, H, D = q.shape
     if k.shape != q.shape or v.shape != q.shape:
@@ -246,44 +293,24 @@ def swa_prefill(q, k, v, w_left: int = 64, scale: Optional[float] = None, rope=N
     for t in (q, k, v):
         if t.stride(-1) != 1:
             raise ValueError("innermost dimension must be contiguous")
-    scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
-    cos_ptr, sin_ptr, n_pos, rotary_dim, interleaved = _rope_tables(rope, q.device, L, D)
+    _, _, n_pos, rotary_dim, interleaved = _rope_tables(rope, q.device, L, D)
     if impl == "plain" and rope is not None:
         raise ValueError("the plain kernel has no in-kernel rotary")
-    kc_ptr = vc_ptr = None
-    c_strides, max_seqlen = (0, 0, 0), 0
+    cache_at = (0, 0, 0, 0)
     if kv_cache is not None:
         _require_cuda(q, kv_cache)
         if (kv_cache.dim() != 5 or kv_cache.shape[0] != B or kv_cache.shape[2] != 2
                 or tuple(kv_cache.shape[3:]) != (H, D) or kv_cache.dtype != q.dtype or kv_cache.stride(-1) != 1):
             raise ValueError(f"bad cache {tuple(kv_cache.shape)} {kv_cache.dtype}")
-        kc, vc = kv_cache[:, :, 0], kv_cache[:, :, 1]
-        kc_ptr, vc_ptr = kc.data_ptr(), vc.data_ptr()
-        c_strides, max_seqlen = (kc.stride(0), kc.stride(1), kc.stride(2)), kv_cache.shape[1]
-    if out is None:
-        o = torch.empty(B, L, H, D, dtype=q.dtype, device=q.device)
+        cache_at = (kv_cache.stride(0), kv_cache.stride(1), kv_cache.stride(3), kv_cache.shape[1])
+    if _swa_fast64(D, rotary_dim, interleaved, impl):
+        name, sizes, rotary = "based_swa_prefill", (B, H, L), ()
+    elif impl == "plain":
+        name, sizes, rotary = "based_swa_prefill_anydim", (B, H, L, D), None
     else:
-        o = out
-        if tuple(o.shape) != (B, L, H, D) or o.dtype != q.dtype or o.device != q.device or o.stride(-1) != 1:
-            raise ValueError(f"out must be a ({B}, {L}, {H}, {D}) {q.dtype} tensor on {q.device}")
-    strides = (q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
-               v.stride(0), v.stride(1), v.stride(2), o.stride(0), o.stride(1), o.stride(2))
-    with _on_device(q.device):
-        if _swa_fast64(D, rotary_dim, interleaved, impl):
-            _lib.check(_lib.lib().based_swa_prefill(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), B, H, L, *strides,
-                int(w_left), scale, cos_ptr, sin_ptr, n_pos, kc_ptr, vc_ptr, *c_strides, max_seqlen,
-                _dtype_code(q), _stream_ptr(q)))
-        elif impl == "plain":
-            _lib.check(_lib.lib().based_swa_prefill_anydim(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), B, H, L, D, *strides,
-                int(w_left), scale, kc_ptr, vc_ptr, *c_strides, max_seqlen, _dtype_code(q), _stream_ptr(q)))
-        else:
-            _lib.check(_lib.lib().based_swa_prefill_wide(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), B, H, L, D, *strides,
-                int(w_left), scale, cos_ptr, sin_ptr, n_pos, rotary_dim, int(interleaved), kc_ptr, vc_ptr, *c_strides,
-                max_seqlen, _dtype_code(q), _stream_ptr(q)))
-    return o
+        name, sizes, rotary = "based_swa_prefill_wide", (B, H, L, D), (rotary_dim, int(interleaved))
+    return (B, L, H, D, name, (*sizes, *q.stride()[:3], *k.stride()[:3], *v.stride()[:3]), n_pos, rotary, cache_at, _dtype_code(q),
+            1.0 / math.sqrt(D))
 
 
 def swa_step(q, k_new, v_new, kv_cache, pos, w_left: int = 64, scale: Optional[float] = None, rope=None,
@@ -364,6 +391,31 @@ def linear_attn_prefill(q, k, v, eps: float = 1e-12, return_state: bool = False,
 
     split: None = let the library decide whether to scan each sequence in concurrent segments
     (small batches); False = never; an int > 1 = that many segments."""
+    key = ("linear_attn_prefill", split, type(split), _form(q, k, v))
+    plan = _CHECKED.get(key)
+    if plan is None:
+        plan = _CHECKED[key] = _linear_prefill_plan(q, k, v, split)
+    B, H, L, dv, at, name, n_seg, ws_bytes, code = plan
+    y = torch.empty(B, L, H, dv, dtype=q.dtype, device=q.device).transpose(1, 2)
+    kv_state = k_state = None
+    if return_state:
+        kv_state = torch.empty(B, H, 1, dv, EXPANDED_DIM, dtype=torch.float32, device=q.device)
+        k_state = torch.empty(B, H, 1, 1, EXPANDED_DIM, dtype=torch.float32, device=q.device)
+    run = getattr(_lib.lib(), name)
+    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), y.data_ptr(),
+            kv_state.data_ptr() if return_state else None, k_state.data_ptr() if return_state else None, *at, float(eps), code)
+    with _on_device(q.device):
+        if n_seg > 1:
+            # scratch for the per-segment states; torch's caching allocator makes this cheap
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
+            _lib.check(run(*args, n_seg, ws.data_ptr(), ws_bytes, _stream_ptr(q)))
+        else:
+            _lib.check(run(*args, _stream_ptr(q)))
+    return y, kv_state, k_state
+
+
+def _linear_prefill_plan(q, k, v, split):
+    """The checked sizes and strides of a linear_attn_prefill call, the entry that takes it, its segments and their scratch."""
     _require_cuda(q, k, v)
     B, H, L, d = q.shape
     dv = v.shape[-1]
@@ -374,37 +426,22 @@ def linear_attn_prefill(q, k, v, eps: float = 1e-12, return_state: bool = False,
     for t in (q, k, v):
         if t.stride(-1) != 1:
             raise ValueError("innermost dimension must be contiguous")
-    y = torch.empty(B, L, H, dv, dtype=q.dtype, device=q.device).transpose(1, 2)
-    kv_state = k_state = None
-    if return_state:
-        kv_state = torch.empty(B, H, 1, dv, EXPANDED_DIM, dtype=torch.float32, device=q.device)
-        k_state = torch.empty(B, H, 1, 1, EXPANDED_DIM, dtype=torch.float32, device=q.device)
     lib = _lib.lib()
     n_seg, ws_bytes = ctypes.c_int64(1), ctypes.c_int64(0)
-    run_split = lib.based_linear_attn_prefill_split
-    if split is None and (q.dtype == torch.float32 or dv % 16 != 0):  # fp32 arithmetic
-        _lib.check(lib.based_linear_attn_prefill_f32_plan(B, H, L, dv, ctypes.byref(n_seg), ctypes.byref(ws_bytes)))
-        run_split = lib.based_linear_attn_prefill_f32
-    elif split is not False:
-        _lib.check(lib.based_linear_attn_prefill_plan(B, H, L, dv, _dtype_code(q), ctypes.byref(n_seg),
-                                                      ctypes.byref(ws_bytes)))
-    if isinstance(split, int) and not isinstance(split, bool) and split > 1:
-        n_seg = ctypes.c_int64(split)  # explicit segment count (tests)
-        ws_bytes = ctypes.c_int64(B * H * ((dv + 63) // 64) * split * _lib.PREFILL_SEGMENT_STATE_BYTES)
-    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), y.data_ptr(),
-            kv_state.data_ptr() if return_state else None, k_state.data_ptr() if return_state else None,
-            B, H, L, dv,
-            q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
-            v.stride(0), v.stride(1), v.stride(2), y.stride(0), y.stride(1), y.stride(2),
-            float(eps), _dtype_code(q))
+    name, code = "based_linear_attn_prefill_split", _dtype_code(q)
     with _on_device(q.device):
-        if n_seg.value > 1:
-            # scratch for the per-segment states; torch's caching allocator makes this cheap
-            ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=q.device)
-            _lib.check(run_split(*args, n_seg.value, ws.data_ptr(), ws_bytes.value, _stream_ptr(q)))
-        else:
-            _lib.check(lib.based_linear_attn_prefill(*args, _stream_ptr(q)))
-    return y, kv_state, k_state
+        if split is None and (q.dtype == torch.float32 or dv % 16 != 0):  # fp32 arithmetic
+            _lib.check(lib.based_linear_attn_prefill_f32_plan(B, H, L, dv, ctypes.byref(n_seg), ctypes.byref(ws_bytes)))
+            name = "based_linear_attn_prefill_f32"
+        elif split is not False:
+            _lib.check(lib.based_linear_attn_prefill_plan(B, H, L, dv, code, ctypes.byref(n_seg), ctypes.byref(ws_bytes)))
+    n_seg, ws_bytes = n_seg.value, ws_bytes.value
+    if isinstance(split, int) and not isinstance(split, bool) and split > 1:
+        n_seg, ws_bytes = split, B * H * ((dv + 63) // 64) * split * _lib.PREFILL_SEGMENT_STATE_BYTES  # explicit segment count (tests)
+    if n_seg <= 1:
+        name = "based_linear_attn_prefill"
+    y_at = (L * H * dv, dv, H * dv)  # (B, L, H, dv) as (B, H, L, dv)
+    return B, H, L, dv, (B, H, L, dv, *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *y_at), name, n_seg, ws_bytes, code
 
 
 def gated_conv_prefill(u, weight, bias=None, state=None, gated: bool = True) -> torch.Tensor:
@@ -885,15 +922,22 @@ def window_attn_prefill(q, k, v, kv_cache, heads: int, kv_heads: int, window: in
     included).  q (B, L, H * d), k (B, L, G * d), v (B, L, G * dv); kv_cache (B, S, G, d + dv) receives the
     portion's rotated keys and (normalised, when value_norm_eps is given) values and is attended.
     Written, times out_scale, into out (B, L, H * dv)."""
-    d, dv = _window_shapes(q, k, v, kv_cache, heads, kv_heads, out)
-    cos_ptr, sin_ptr, n_pos, rot, half = _stream_rope(rope, q.device)
-    B, L = q.shape[:2]
+    cos, sin, turned = (None, None, None) if rope is None else rope
+    key = ("window_attn_prefill", heads, kv_heads, bool(turned), _form(q, k, v, kv_cache, out, cos, sin))
+    plan = _CHECKED.get(key)
+    if plan is None:
+        d, dv = _window_shapes(q, k, v, kv_cache, heads, kv_heads, out)
+        rope_at = _stream_rope(rope, q.device)[2:]
+        B, L = q.shape[:2]
+        plan = _CHECKED[key] = (
+            (B, L, heads, kv_heads, d, dv, kv_cache.shape[1], q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
+             out.stride(0), out.stride(1), kv_cache.stride(0), kv_cache.stride(1)), rope_at, _dtype_code(q))
+    at, rope_at, code = plan
     with _on_device(q.device):
         _lib.check(_lib.lib().based_window_attn_prefill(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), kv_cache.data_ptr(), out.data_ptr(), int(start), B, L, heads, kv_heads, d, dv,
-            kv_cache.shape[1], q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1), out.stride(0),
-            out.stride(1), kv_cache.stride(0), kv_cache.stride(1), int(window), float(scale), int(value_norm_eps is not None),
-            float(value_norm_eps or 0.0), float(out_scale), cos_ptr, sin_ptr, n_pos, rot, half, _dtype_code(q), _stream_ptr(q)))
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), kv_cache.data_ptr(), out.data_ptr(), int(start), *at, int(window), float(scale),
+            int(value_norm_eps is not None), float(value_norm_eps or 0.0), float(out_scale), _ptr(cos), _ptr(sin), *rope_at, code,
+            _stream_ptr(q)))
     return out
 
 
@@ -924,21 +968,26 @@ def gated_delta_scan(q, k, v, a_gate, b_gate, a_log, dt_bias, state, heads: int,
     """The gated delta recurrence over a portion.  q, k (B, L, G * d) and v (B, L, H * dv) share their strides
     (slices of one tensor); a_gate, b_gate (B, L, H); state (B, H, d, dv rounded up to 4) fp32, updated in
     place, taken as zero when `fresh`.  Returns o (B, L, H, dv) fp32."""
-    _check_rows(q, k, v, a_gate, b_gate)
-    _check_same_dtype(q, k, v, a_gate, b_gate, a_log, dt_bias)
-    B, L = q.shape[:2]
-    d, dv = q.shape[-1] // kv_heads, v.shape[-1] // heads
-    if q.shape != k.shape or tuple(v.shape[:2]) != (B, L) or q.shape[-1] != kv_heads * d or v.shape[-1] != heads * dv:
-        raise ValueError(f"bad shapes q{tuple(q.shape)} k{tuple(k.shape)} v{tuple(v.shape)}")
-    if not (q.stride() == k.stride() == v.stride()) or a_gate.stride() != b_gate.stride():
-        raise ValueError("q, k and v must share their strides, and the two gates theirs")
-    if tuple(a_gate.shape) != (B, L, heads) or b_gate.shape != a_gate.shape:
-        raise ValueError(f"gates must be ({B}, {L}, {heads})")
-    _check_delta(state, B, heads, d, dv)
+    key = ("gated_delta_scan", heads, kv_heads, _form(q, k, v, a_gate, b_gate, a_log, dt_bias, state))
+    plan = _CHECKED.get(key)
+    if plan is None:
+        _check_rows(q, k, v, a_gate, b_gate)
+        _check_same_dtype(q, k, v, a_gate, b_gate, a_log, dt_bias)
+        B, L = q.shape[:2]
+        d, dv = q.shape[-1] // kv_heads, v.shape[-1] // heads
+        if q.shape != k.shape or tuple(v.shape[:2]) != (B, L) or q.shape[-1] != kv_heads * d or v.shape[-1] != heads * dv:
+            raise ValueError(f"bad shapes q{tuple(q.shape)} k{tuple(k.shape)} v{tuple(v.shape)}")
+        if not (q.stride() == k.stride() == v.stride()) or a_gate.stride() != b_gate.stride():
+            raise ValueError("q, k and v must share their strides, and the two gates theirs")
+        if tuple(a_gate.shape) != (B, L, heads) or b_gate.shape != a_gate.shape:
+            raise ValueError(f"gates must be ({B}, {L}, {heads})")
+        _check_delta(state, B, heads, d, dv)
+        plan = _CHECKED[key] = (B, L, d, dv, state.shape[3], q.stride(0), q.stride(1), a_gate.stride(0), a_gate.stride(1), _dtype_code(q))
+    B, L, d, dv, state_row, x_sb, x_sl, g_sb, g_sl, code = plan
     o = torch.empty(B, L, heads, dv, dtype=torch.float32, device=q.device)
     lib, floats = _lib.lib(), 0
     if L >= DELTA_CHUNKS_MIN:
-        floats = lib.based_gated_delta_scan_work_of(q.data_ptr(), k.data_ptr(), B, L, heads, d, dv, q.stride(0), q.stride(1))
+        floats = lib.based_gated_delta_scan_work_of(q.data_ptr(), k.data_ptr(), B, L, heads, d, dv, x_sb, x_sl)
     if floats:
         scan, work = lib.based_gated_delta_scan_chunks, torch.empty(floats, dtype=torch.float32, device=q.device)
     else:
@@ -948,8 +997,8 @@ def gated_delta_scan(q, k, v, a_gate, b_gate, a_log, dt_bias, state, heads: int,
     with _on_device(q.device):
         _lib.check(scan(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), a_gate.data_ptr(), b_gate.data_ptr(), a_log.data_ptr(), dt_bias.data_ptr(),
-            state.data_ptr(), work.data_ptr(), o.data_ptr(), B, L, heads, kv_heads, d, dv, state.shape[3], q.stride(0), q.stride(1),
-            a_gate.stride(0), a_gate.stride(1), int(fresh), _dtype_code(q), _stream_ptr(q)))
+            state.data_ptr(), work.data_ptr(), o.data_ptr(), B, L, heads, kv_heads, d, dv, state_row, x_sb, x_sl, g_sb, g_sl, int(fresh), code,
+            _stream_ptr(q)))
     return o
 
 
@@ -1014,21 +1063,24 @@ def rglru_prefill(u, y, ra, rb, ri, ib, lam, state, decay_scale: float, fresh: b
     """The gated linear recurrence over a portion: u (B, L, W) convolved, y (B, L, W) before its gelu; ra, ri
     (blocks, n, n) as [out, in], rb, ib, lam (W) values; state (B, W) fp32, updated in place, taken as
     zero when `fresh`.  out (B, L, W) = S * gelu_tanh(y)."""
-    B, L, _ = u.shape
-    W, blocks = _check_lru(u, y, ra, rb, ri, ib, lam, state, out, B)
+    key = ("rglru_prefill", _form(u, y, ra, rb, ri, ib, lam, state, out))
+    plan = _CHECKED.get(key)
+    if plan is None:
+        B, L, _ = u.shape
+        W, blocks = _check_lru(u, y, ra, rb, ri, ib, lam, state, out, B)
+        plan = _CHECKED[key] = ((B, L, W, blocks), (u.stride(0), u.stride(1)), (y.stride(0), y.stride(1)), (out.stride(0), out.stride(1)), _dtype_code(u))
+    sizes, u_at, y_at, o_at, code = plan
+    B, L, W, _ = sizes
     segs = (L + RGLRU_SEGMENT - 1) // RGLRU_SEGMENT
     agg = torch.empty(B, segs + 1, 2, W, dtype=torch.float32, device=u.device)
-    lib = _lib.lib()
+    lib, u_ptr, out_ptr = _lib.lib(), u.data_ptr(), out.data_ptr()
     # an output that shares memory with u is formed apart from it
-    n = lib.based_rglru_prefill_work(u.data_ptr(), out.data_ptr(), B, L, W, u.stride(0), u.stride(1), out.stride(0), out.stride(1),
-                                     _dtype_code(u))
+    n = lib.based_rglru_prefill_work(u_ptr, out_ptr, B, L, W, *u_at, *o_at, code)
     work = torch.empty(n, dtype=torch.float32, device=u.device) if n else None
     with _on_device(u.device):
         _lib.check(lib.based_rglru_prefill(
-            u.data_ptr(), y.data_ptr(), ra.data_ptr(), rb.data_ptr(), ri.data_ptr(), ib.data_ptr(), lam.data_ptr(),
-            None, _ptr(work), agg.data_ptr(), state.data_ptr(), out.data_ptr(), B, L, W, blocks, u.stride(0),
-            u.stride(1), y.stride(0), y.stride(1), out.stride(0), out.stride(1), float(decay_scale), int(fresh), _dtype_code(u),
-            _stream_ptr(u)))
+            u_ptr, y.data_ptr(), ra.data_ptr(), rb.data_ptr(), ri.data_ptr(), ib.data_ptr(), lam.data_ptr(), None, _ptr(work), agg.data_ptr(),
+            state.data_ptr(), out_ptr, *sizes, *u_at, *y_at, *o_at, float(decay_scale), int(fresh), code, _stream_ptr(u)))
     return out
 
 
@@ -1170,36 +1222,42 @@ def decay_scan(q, k, v, state, heads: int, *, channel_log2=None, bonus=None, hea
     """Linear attention with decaying states over a portion: q, k (B, L, H * d), v (B, L, H * dv) -> o (B, L, H * dv); state (B, H, dv,
     d rounded up to 4) fp32, updated in place, taken as zero when `fresh`.  channel_log2 (B, L, H * d) fp32 with bonus (H, d):
     o_t = (S + diag(u) k v^T)^T q, S <- diag(w) S + k v^T; head_decay (2, H) of `head_decays`: S <- w S + k v^T, o = S^T q."""
-    _check_rows(q, k, v)
-    _check_same_dtype(q, k, v, bonus)
-    B, L = q.shape[:2]
-    d, dv = q.shape[-1] // heads, v.shape[-1] // heads
-    if q.shape != k.shape or tuple(q.shape) != (B, L, heads * d) or tuple(v.shape) != (B, L, heads * dv):
-        raise ValueError(f"bad shapes q{tuple(q.shape)} k{tuple(k.shape)} v{tuple(v.shape)}")
-    _check_decay_state(state, B, heads, d, dv)
-    if channel_log2 is not None:
-        if tuple(channel_log2.shape) != (B, L, heads * d) or channel_log2.dtype != torch.float32 or not channel_log2.is_contiguous() \
-                or bonus is None or tuple(bonus.shape) != (heads, d) or not bonus.is_contiguous():
-            raise ValueError(f"channel decays must be contiguous float32 ({B}, {L}, {heads * d}) with a bonus ({heads}, {d})")
-        _require_cuda(q, channel_log2, bonus)
-    else:
-        _check_head_decay(head_decay, heads, q.device)
-    lib = _lib.lib()
-    o = torch.empty(B, L, heads * dv, dtype=q.dtype, device=q.device)
-    sizes = (B, L, heads, d, dv, state.shape[3])
-    at = [q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(channel_log2), _ptr(bonus), o.data_ptr()]
-    strides = (*q.stride()[:2], *k.stride()[:2], *v.stride()[:2], L * heads * dv, heads * dv)
-    work = None
-    if L >= DECAY_SEGMENTS_MIN:
-        bits = at[0] | at[1] | at[2] | (at[4] or 0) | at[5] | (at[3] or 0) >> 1
+    key = ("decay_scan", heads, _form(q, k, v, state, channel_log2, bonus, head_decay))
+    plan = _CHECKED.get(key)
+    if plan is None:
+        _check_rows(q, k, v)
+        _check_same_dtype(q, k, v, bonus)
+        B, L = q.shape[:2]
+        d, dv = q.shape[-1] // heads, v.shape[-1] // heads
+        if q.shape != k.shape or tuple(q.shape) != (B, L, heads * d) or tuple(v.shape) != (B, L, heads * dv):
+            raise ValueError(f"bad shapes q{tuple(q.shape)} k{tuple(k.shape)} v{tuple(v.shape)}")
+        _check_decay_state(state, B, heads, d, dv)
+        if channel_log2 is not None:
+            if tuple(channel_log2.shape) != (B, L, heads * d) or channel_log2.dtype != torch.float32 or not channel_log2.is_contiguous() \
+                    or bonus is None or tuple(bonus.shape) != (heads, d) or not bonus.is_contiguous():
+                raise ValueError(f"channel decays must be contiguous float32 ({B}, {L}, {heads * d}) with a bonus ({heads}, {d})")
+            _require_cuda(q, channel_log2, bonus)
+        else:
+            _check_head_decay(head_decay, heads, q.device)
+        strides = (*q.stride()[:2], *k.stride()[:2], *v.stride()[:2], L * heads * dv, heads * dv)
+        bits = 0
         for x in strides:
             bits |= 2 * x
-        n = lib.based_decay_scan_work_of(bits, *sizes, _dtype_code(q))
+        plan = _CHECKED[key] = ((B, L, heads, d, dv, state.shape[3]), strides, bits, _dtype_code(q))
+    sizes, strides, stride_bits, code = plan
+    B, L, _, d, dv, _ = sizes
+    lib = _lib.lib()
+    o = torch.empty(B, L, heads * dv, dtype=q.dtype, device=q.device)
+    at = [q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(channel_log2), _ptr(bonus), o.data_ptr()]
+    work = None
+    if L >= DECAY_SEGMENTS_MIN:
+        bits = at[0] | at[1] | at[2] | (at[4] or 0) | at[5] | (at[3] or 0) >> 1 | stride_bits
+        n = lib.based_decay_scan_work_of(bits, *sizes, code)
         work = torch.empty(n, dtype=torch.float32, device=q.device) if n else None
     with _on_device(q.device):
         _lib.check(lib.based_decay_scan(
             *at[:4], _ptr(head_decay), at[4], state.data_ptr(), _ptr(work), at[5], *sizes, *strides, int(activation), int(fresh),
-            _dtype_code(q), _stream_ptr(q)))
+            code, _stream_ptr(q)))
     return o
 
 
@@ -1301,27 +1359,34 @@ def latent_step(q, x, norm_weight, weight, cache, heads: int, dim: int, window: 
     """One token per sequence on a latent cache: q (B, H * (rot + d)) with a head's rotated channels first, x (B, R + rot) the token's own
     row before norm and rotation, weight (H * (rot + d + dv), >= R): of each head rot rows that are not read, uk, uv.
     Written, times out_scale, into out (B, H * dv)."""
-    R, rot, cos_ptr, sin_ptr, n_pos, half = _latent_rows(x, norm_weight, cache, rope)
-    _check_rows(q, weight, out)
-    _check_same_dtype(x, q, weight, out)
-    B, S = x.shape[0], cache.shape[1]
-    dv = out.shape[-1] // heads
-    if tuple(q.shape) != (B, heads * (rot + dim)) or tuple(out.shape) != (B, heads * dv) or weight.shape[0] != heads * (rot + dim + dv) \
-            or weight.shape[1] < R:
-        raise ValueError(f"bad shapes q{tuple(q.shape)} weight{tuple(weight.shape)} out{tuple(out.shape)}")
-    groups = B * ((heads + 15) // 16)
-    splits = max(1, min(LATENT_STEP_TARGET // groups, (min(window, S) + 63) // 64, LATENT_STEP_MAX_SPLITS))
-    # queries (B, heads, R + rot), sums (B, splits, heads, R) and their maxima and weights (.., 2) in one allocation, 16-byte pieces each
-    n_q, n_part = (B * heads * (R + rot) + 3) // 4 * 4, (B * splits * heads * R + 3) // 4 * 4
-    work = torch.empty(n_q + n_part + B * splits * heads * 2, dtype=torch.float32, device=x.device)
+    cos, sin, turned = (None, None, None) if rope is None else rope
+    key = ("latent_step", heads, dim, window, bool(turned), _form(q, x, norm_weight, weight, cache, out, cos, sin))
+    plan = _CHECKED.get(key)
+    if plan is None:
+        R, rot, _, _, n_pos, half = _latent_rows(x, norm_weight, cache, rope)
+        _check_rows(q, weight, out)
+        _check_same_dtype(x, q, weight, out)
+        B, S = x.shape[0], cache.shape[1]
+        dv = out.shape[-1] // heads
+        if tuple(q.shape) != (B, heads * (rot + dim)) or tuple(out.shape) != (B, heads * dv) or weight.shape[0] != heads * (rot + dim + dv) \
+                or weight.shape[1] < R:
+            raise ValueError(f"bad shapes q{tuple(q.shape)} weight{tuple(weight.shape)} out{tuple(out.shape)}")
+        groups = B * ((heads + 15) // 16)
+        splits = max(1, min(LATENT_STEP_TARGET // groups, (min(window, S) + 63) // 64, LATENT_STEP_MAX_SPLITS))
+        # queries (B, heads, R + rot), sums (B, splits, heads, R) and their maxima and weights (.., 2) in one allocation, 16-byte pieces each
+        n_q, n_part = (B * heads * (R + rot) + 3) // 4 * 4, (B * splits * heads * R + 3) // 4 * 4
+        plan = _CHECKED[key] = (
+            4 * n_q, 4 * (n_q + n_part), n_q + n_part + B * splits * heads * 2, n_pos, half, _dtype_code(x),
+            (B, heads, dim, dv, S, R, rot, splits, q.stride(0), x.stride(0), weight.stride(0), cache.stride(0), cache.stride(1), out.stride(0)))
+    at_part, at_ml, floats, n_pos, half, code, sizes = plan
+    work = torch.empty(floats, dtype=torch.float32, device=x.device)
     work_q = work.data_ptr()
-    pos_ptr, pos_host = _pos_args(pos, B)
+    pos_ptr, pos_host = _pos_args(pos, sizes[0])
     with _on_device(x.device):
         _lib.check(_lib.lib().based_latent_step(
-            q.data_ptr(), x.data_ptr(), norm_weight.data_ptr(), weight.data_ptr(), cache.data_ptr(), work_q, work_q + 4 * n_q,
-            work_q + 4 * (n_q + n_part), out.data_ptr(), pos_ptr, pos_host, B, heads, dim, dv, S, R, rot, splits, q.stride(0), x.stride(0),
-            weight.stride(0), cache.stride(0), cache.stride(1), out.stride(0), int(window), float(scale), float(eps), float(out_scale),
-            cos_ptr, sin_ptr, n_pos, half, _dtype_code(x), _stream_ptr(x)))
+            q.data_ptr(), x.data_ptr(), norm_weight.data_ptr(), weight.data_ptr(), cache.data_ptr(), work_q, work_q + at_part, work_q + at_ml,
+            out.data_ptr(), pos_ptr, pos_host, *sizes, int(window), float(scale), float(eps), float(out_scale), _ptr(cos), _ptr(sin), n_pos, half,
+            code, _stream_ptr(x)))
     return out
 
 
@@ -1337,21 +1402,13 @@ def experts(h, router, w1, w2, top: int, norm=None) -> torch.Tensor:
     """y = sum over the `top` experts of a token with the largest sigmoid(router h) of w2_e (silu(gate) * up), [up; gate] = score * w1_e h.
     h (..., D), router (E, D), w1 (E, 2 F, D) up rows first, w2 (E, D, F).  norm = (residual fp32 or None, residual_out fp32 or None, weight,
     eps, kind, mult): h is the input of `add_norm` with these and the layer reads its norm."""
-    D = h.shape[-1]
-    E, F = w2.shape[0], w2.shape[2]
-    h2 = h.reshape(-1, D)
-    _check_rows(h2, router, w1, w2)
-    _check_same_dtype(h2, router, w1, w2)
-    if tuple(router.shape) != (E, D) or tuple(w1.shape) != (E, 2 * F, D) or tuple(w2.shape) != (E, D, F):
-        raise ValueError(f"bad shapes router{tuple(router.shape)} w1{tuple(w1.shape)} w2{tuple(w2.shape)}")
-    if not (router.is_contiguous() and w1.is_contiguous() and w2.is_contiguous()):
-        raise ValueError("expert weights must be contiguous")
-    if not 1 <= top <= E:
-        raise ValueError(f"{top} of {E} experts")
-    n, dev = h2.shape[0], h2.device
+    key = ("experts", top, _form(h, router, w1, w2))
+    plan = _CHECKED.get(key)
+    if plan is None:
+        plan = _CHECKED[key] = _experts_plan(h, router, w1, w2, top)
+    n, D, F, E, grouped, vec_f32, tiles, (at_ids, at_rank, at_counts, at_first, at_tiles, at_order, at_act, at_part, ints), code = plan
+    h2, dev = h.reshape(-1, D), h.device
     lib = _lib.lib()
-    grouped = h2.dtype == torch.bfloat16 and n * top > EXPERT_ROWS_MAX and D % 8 == 0 and F % 8 == 0 and h2.stride(0) % 8 == 0
-    i32 = dict(dtype=torch.int32, device=dev)
     norm_args = (None, None, None, None, 1.0, NORM_RMS, 0.0)
     if norm is not None:
         residual, residual_out, weight, eps, kind, mult = norm
@@ -1366,33 +1423,55 @@ def experts(h, router, w1, w2, top: int, norm=None) -> torch.Tensor:
                 raise ValueError(f"the norm's weight must be a contiguous ({D},) on the device")
             normed = torch.empty_like(h2)
             norm_args = (_ptr(residual), _ptr(residual_out), weight.data_ptr(), normed.data_ptr(), float(mult), int(kind), float(eps))
-    ids, scores = torch.empty(n, top, **i32), torch.empty(n, top, dtype=torch.float32, device=dev)
     y = torch.empty(n, D, dtype=h2.dtype, device=dev)
+    work = torch.empty(ints, dtype=torch.int32, device=dev)  # all that a call keeps between its launches
+    at = work.data_ptr()
+    h_ptr, w1_ptr, w2_ptr = h2.data_ptr(), w1.data_ptr(), w2.data_ptr()
+    # (scores in front of the choices)
+    part = at + at_part if top > 1 else None
     with _on_device(dev):
         if grouped:
-            tiles, rows = lib.based_expert_tiles(n, E, top), lib.based_expert_tile_rows(n, E, top)
-            rank = torch.empty(n, top, **i32)
-            counts = torch.empty(E, **i32)
-            plan = torch.empty(E + 1 + tiles + tiles * rows, **i32)
-            act = torch.empty(tiles * rows, F, dtype=h2.dtype, device=dev)
-            part = torch.empty(n * top, D, dtype=h2.dtype, device=dev) if top > 1 else None
             _lib.check(lib.based_expert_grouped(
-                h2.data_ptr(), router.data_ptr(), w1.data_ptr(), w2.data_ptr(), ids.data_ptr(), scores.data_ptr(), rank.data_ptr(),
-                counts.data_ptr(), plan.data_ptr(), plan[E + 1:].data_ptr(), plan[E + 1 + tiles:].data_ptr(), act.data_ptr(), _ptr(part),
-                y.data_ptr(), n, D, F, E, top, h2.stride(0), _stream_ptr(h2)))
-        elif (h2.dtype == torch.float32 and n * top > EXPERT_ROWS_F32_MAX * E and D % 4 == 0 and F % 4 == 0 and h2.stride(0) % 4 == 0
-              and not (h2.data_ptr() | w1.data_ptr() | w2.data_ptr()) & 15):
-            act = torch.empty(n * top, F, dtype=h2.dtype, device=dev)
-            part = torch.empty(n * top, D, dtype=h2.dtype, device=dev) if top > 1 else None
+                h_ptr, router.data_ptr(), w1_ptr, w2_ptr, at + at_ids, at, at + at_rank, at + at_counts, at + at_first, at + at_tiles, at + at_order,
+                at + at_act, part, y.data_ptr(), n, D, F, E, top, h2.stride(0), _stream_ptr(h2)))
+        elif vec_f32 and h2.stride(0) % 4 == 0 and not (h_ptr | w1_ptr | w2_ptr) & 15:
             _lib.check(lib.based_expert_grouped_f32(
-                h2.data_ptr(), router.data_ptr(), w1.data_ptr(), w2.data_ptr(), ids.data_ptr(), scores.data_ptr(), act.data_ptr(), _ptr(part),
-                y.data_ptr(), n, D, F, E, top, h2.stride(0), _stream_ptr(h2)))
+                h_ptr, router.data_ptr(), w1_ptr, w2_ptr, at + at_ids, at, at + at_act, part, y.data_ptr(), n, D, F, E, top, h2.stride(0),
+                _stream_ptr(h2)))
         else:
-            act = torch.empty(n * top, F, dtype=h2.dtype, device=dev)
-            _lib.check(lib.based_expert_rows(h2.data_ptr(), *norm_args, router.data_ptr(), w1.data_ptr(), w2.data_ptr(), ids.data_ptr(),
-                                             scores.data_ptr(), act.data_ptr(), y.data_ptr(), n, D, F, E, top, h2.stride(0), _dtype_code(h2),
-                                             _stream_ptr(h2)))
+            _lib.check(lib.based_expert_rows(h_ptr, *norm_args, router.data_ptr(), w1_ptr, w2_ptr, at + at_ids, at, at + at_act, y.data_ptr(), n, D, F, E,
+                                             top, h2.stride(0), code, _stream_ptr(h2)))
     return y.view(h.shape)
+
+
+def _experts_plan(h, router, w1, w2, top: int):
+    """The checked sizes of an `experts` call, whether rows of one expert share its matrices, and where what lies in its work space (bytes; 32-bit
+    words in all): scores, choices, their ranks, counts, the plan of the tiles, activations, the choices' outputs."""
+    D = h.shape[-1]
+    E, F = w2.shape[0], w2.shape[2]
+    h2 = h.reshape(-1, D)
+    _check_rows(h2, router, w1, w2)
+    _check_same_dtype(h2, router, w1, w2)
+    if tuple(router.shape) != (E, D) or tuple(w1.shape) != (E, 2 * F, D) or tuple(w2.shape) != (E, D, F):
+        raise ValueError(f"bad shapes router{tuple(router.shape)} w1{tuple(w1.shape)} w2{tuple(w2.shape)}")
+    if not (router.is_contiguous() and w1.is_contiguous() and w2.is_contiguous()):
+        raise ValueError("expert weights must be contiguous")
+    if not 1 <= top <= E:
+        raise ValueError(f"{top} of {E} experts")
+    n, lib = h2.shape[0], _lib.lib()
+    slots = n * top
+    grouped = h2.dtype == torch.bfloat16 and slots > EXPERT_ROWS_MAX and D % 8 == 0 and F % 8 == 0 and h2.stride(0) % 8 == 0
+    vec_f32 = h2.dtype == torch.float32 and slots > EXPERT_ROWS_F32_MAX * E and D % 4 == 0 and F % 4 == 0
+    tiles, rows = (lib.based_expert_tiles(n, E, top), lib.based_expert_tile_rows(n, E, top)) if grouped else (0, 0)
+    at, ends = 0, []
+    act_rows = tiles * rows if grouped else slots
+    parts = slots * D if top > 1 and (grouped or vec_f32) else 0
+    size = h2.element_size()
+    for nbytes in (4 * slots, 4 * slots, 4 * slots if grouped else 0, 4 * E if grouped else 0, 4 * (E + 1) if grouped else 0, 4 * tiles,
+                   4 * tiles * rows, act_rows * F * size, parts * size):
+        at += (nbytes + 15) // 16 * 16  # (whole 16-byte pieces each)
+        ends.append(at)
+    return n, D, F, E, grouped, vec_f32, tiles, (*ends[:8], ends[8] // 4), _dtype_code(h2)
 
 
 # Rows up to which the streamed-input prologue is evaluated inside the projection.  Every workgroup of it

@@ -215,3 +215,31 @@ def test_gated_mlp_variants_construct_like_the_reference():
     assert base.fc1.weight.shape == (4096, 1024) and base.fc2.weight.shape == (1024, 2048)
     with pytest.raises(NotImplementedError):
         GatedMlp(64, activation="gelu_new")
+
+
+def test_binding_reads_what_ctypes_reads():
+    """The callables of csrc/binding.cpp against the ctypes entries they stand for: numbers, None, truth values, and what goes to ctypes after all."""
+    import ctypes
+
+    from based_amd import _lib
+
+    lib, handle = _lib.lib(), ctypes.CDLL(_lib.LIB_PATH)
+    for name, calls in {"based_expert_tiles": [(100, 8, 2), (0, 8, 2), (True, 1, 1), (ctypes.c_int64(300), 4, 1)],
+                        "based_decay_scan_work_of": [(0, 4, 2048, 16, 64, 64, 64, 0), (8, 1, 300, 12, 64, 64, 64, 1), (1 << 40, 1, 300, 12, 64, 64, 64, 1)],
+                        "based_swiglu": [(None, None, 1, 8, 16, 8, 0, None), (None, None, 1, 8, 16, 8, 0, 0)]}.items():
+        fn = getattr(handle, name)
+        fn.restype, fn.argtypes = _lib.SIGNATURES[name]
+        for args in calls:
+            assert getattr(lib, name)(*args) == fn(*args), (name, args)
+    for bad in ((1, 2), (1, 2, "3"), (1.5, 2, 3)):
+        with pytest.raises((TypeError, ctypes.ArgumentError)):
+            lib.based_expert_tiles(*bad)
+
+
+def test_remembered_checks_are_bounded():
+    from based_amd import ops
+
+    kept = ops._Checked()
+    for i in range(10000):
+        kept[i] = i
+    assert len(kept) <= 4096 and kept[9999] == 9999
