@@ -45,7 +45,7 @@ struct DecayScanArgs {
   int B, L, H, d, dv, dp;
   long q_sb, q_sl, k_sb, k_sl, v_sb, v_sl, o_sb, o_sl;
   int segs, seg_chunks;  // segments, and 64-token pieces in each
-  int silu, fresh;
+  int silu, fresh, fold;
 };
 
 template <int CTRL> __device__ __forceinline__ float row_moved(float x) {  // lanes without a source receive 0
@@ -112,6 +112,14 @@ __device__ __forceinline__ void store_pair(__bf16* p, __bf16* q, uint32_t x) {
   *reinterpret_cast<uint16_t*>(q) = (uint16_t)(x >> 16);
 }
 
+// Decay of a head over a segment that is not the last: whole 64-token pieces, an even power (a decay below zero has no logarithm).  A product of
+// decays that only the format makes zero comes as its smallest number: an infinite state outlives it, as it does token by token.
+__device__ __forceinline__ float decay_of_segment(const DecayScanArgs& a, int h) {
+  const float w = a.head_lw[a.H + h], l2 = w < 0.f ? log2f(-w) : a.head_lw[h];
+  const float all = __builtin_amdgcn_exp2f(l2 * (float)(a.seg_chunks * kScanTokens));
+  return all == 0.f && w != 0.f ? 0x1p-149f : all;
+}
+
 // HALVES wavefronts (1 or 2) share the key channels of 16 tokens, DT 32-channel pieces each (d <= 32 DT HALVES, d % 4 == 0), so
 // that what a lane holds of a token stays in registers; their parts of P are added through LDS.  Channels of a piece are held by the lanes in the
 // order of the accumulators: element e < 4 of a lane in 16-lane row `quad` is channel 4 quad + e, e >= 4
@@ -161,13 +169,53 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
   // state: tile ct holds key channels 16 ct + 4 quad + i of value channel dv0 + l16
   f32x4 S[2 * DA];
   {
-    const float* from = a.segs > 1 ? a.seg + ((bh * a.segs + sg) * a.dv + (col_in ? dv0 + l16 : 0)) * a.dp : st;
-    const bool zero = STATE_ONLY || (a.segs == 1 && a.fresh);
+    const long seg_row = (col_in ? dv0 + l16 : 0), seg_step = (long)a.dv * a.dp;
+    const float* segs = a.seg + (bh * a.segs * a.dv + seg_row) * a.dp;
+    // folded: what the segments in front have added is put together here, the state that enters the call from the last one's place, where
+    // the state pass has left it (the last segment replaces it)
+    const bool fold = !STATE_ONLY && a.segs > 1 && a.fold;
+    const float* from = a.segs > 1 ? segs + (fold ? a.segs - 1 : sg) * seg_step : st;
+    const bool zero = STATE_ONLY || ((a.segs == 1 || fold) && a.fresh);
 #pragma unroll
     for (int ct = 0; ct < 2 * DA; ++ct) {
       const int ch = ct * 16 + quad * 4;
       S[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (!zero && col_in && ch < a.d) S[ct] = *reinterpret_cast<const f32x4*>(from + ch);
+    }
+    if constexpr (STATE_ONLY) {
+      if (a.fold && !a.fresh && sg == 0 && col_in) {
+        float* keep = a.seg + ((bh * a.segs + a.segs - 1) * a.dv + seg_row) * a.dp;
+#pragma unroll
+        for (int ct = 0; ct < 2 * DA; ++ct) {
+          const int ch = ct * 16 + quad * 4;
+          if (ch < a.d) *reinterpret_cast<f32x4*>(keep + ch) = *reinterpret_cast<const f32x4*>(st + ch);
+        }
+      }
+    } else if (fold) {
+      const float seg_decay = CHANNEL ? 0.f : decay_of_segment(a, h);  // (all in front of the last are of one length)
+      constexpr int U = HALVES == 1 ? 4 : 2;  // segments asked for together
+      for (int s0 = 0; s0 < sg; s0 += U) {
+        f32x4 add[U][2 * DA], l[U][2 * DA];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int ct = 0; ct < 2 * DA; ++ct) {
+            const int ch = ct * 16 + quad * 4 < a.d ? ct * 16 + quad * 4 : 0, s = s0 + u < sg ? s0 + u : sg - 1;
+            add[u][ct] = *reinterpret_cast<const f32x4*>(segs + s * seg_step + ch);
+            if constexpr (CHANNEL) l[u][ct] = *reinterpret_cast<const f32x4*>(a.seg_lw + (bh * a.segs + s) * a.dp + ch);
+          }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (s0 + u >= sg) break;  // (uniform)
+#pragma unroll
+          for (int ct = 0; ct < 2 * DA; ++ct)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const float sum = __builtin_fmaf(S[ct][j], CHANNEL ? l[u][ct][j] : seg_decay, add[u][ct][j]);
+              S[ct][j] = col_in && ct * 16 + quad * 4 < a.d ? sum : 0.f;
+            }
+        }
+      }
     }
   }
   float seg_total = 1.f;  // (state pass, channel decays) decay of the segment so far, of the channel that is this thread's number
@@ -547,9 +595,7 @@ __global__ __launch_bounds__(256) void decay_join_kernel(const DecayScanArgs a) 
   float* st = a.state + (bh * a.dv + col) * a.dp + ch;
   f32x4 S = {0.f, 0.f, 0.f, 0.f};
   if (!a.fresh) S = *reinterpret_cast<const f32x4*>(st);
-  // (a decay below zero has no logarithm; segments are whole 64-token pieces, an even power)
-  const float head_w = a.lw != nullptr ? 0.f : a.head_lw[a.H + bh % a.H];
-  const float head_l2 = a.lw != nullptr ? 0.f : head_w < 0.f ? log2f(-head_w) : a.head_lw[bh % a.H];
+  const float head = a.lw != nullptr ? 0.f : decay_of_segment(a, (int)(bh % a.H));
   for (int s = 0; s < a.segs; ++s) {
     float* p = a.seg + ((bh * a.segs + s) * a.dv + col) * a.dp + ch;
     f32x4 add = {0.f, 0.f, 0.f, 0.f};
@@ -560,11 +606,8 @@ __global__ __launch_bounds__(256) void decay_join_kernel(const DecayScanArgs a) 
     if (a.lw != nullptr) {
       l = *reinterpret_cast<const f32x4*>(a.seg_lw + (bh * a.segs + s) * a.dp + ch);
     } else {
-      const int lo = s * a.seg_chunks * kScanTokens, hi = (s + 1) * a.seg_chunks * kScanTokens;
-      const float all = __builtin_amdgcn_exp2f(head_l2 * (float)((hi < a.L ? hi : a.L) - lo)), f = all == 0.f && head_w != 0.f ? 0x1p-149f : all;
-      l = f32x4{f, f, f, f};
+      l = f32x4{head, head, head, head};
     }
-    // a product of decays that only the format makes zero comes as its smallest number: an infinite state outlives it, as it does token by token
 #pragma unroll
     for (int j = 0; j < 4; ++j) S[j] = __builtin_fmaf(S[j], l[j], add[j]);
   }
@@ -935,7 +978,7 @@ template <int DT, int HALVES, bool CHANNEL> int launch_decay_mfma(const DecaySca
     dim3 all_but_last = grid;
     all_but_last.z -= 1;
     hipLaunchKernelGGL((decay_scan_mfma_kernel<DT, HALVES, CHANNEL, true>), all_but_last, dim3(256 * HALVES), bytes, s, a);
-    launch_decay_join(a, s);
+    if (!a.fold) launch_decay_join(a, s);
   }
   hipLaunchKernelGGL((decay_scan_mfma_kernel<DT, HALVES, CHANNEL, false>), grid, dim3(256 * HALVES), bytes, s, a);
   return BASED_OK;
@@ -1004,6 +1047,11 @@ template <typename T, bool CHANNEL> void launch_decay_step(const DecayStepArgs& 
   else
     launch_decay_step_rows<T, 64, CHANNEL>(a, s);
 }
+
+// Segments up to which those of the scan put the ones in front of them together themselves, heads of up to 64 channels: a launch less, and memory's
+// answer to four segments at a time in front of the scan.  4 x 2048 tokens, 16 heads of 64 (8 segments): 74.6 us with decay_join_kernel,
+// 72.2; 12 x 960 (3) 124.2, 121.2; 1 x 2000, 12 heads (8) 53.6, 53.5; 1 x 4096 (16) 57.6, 60.1; 1 x 2000, 8 heads of 128 87.4, 96.0.
+constexpr int kFoldSegments = 8;
 
 // Segments of a scan: enough workgroups to give every SIMD two wavefronts, none shorter than four pieces of 64 tokens.
 static int decay_segments(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
@@ -1087,6 +1135,7 @@ extern "C" BASED_API int based_decay_scan(const void* q, const void* k, const vo
     a.segs = (int)(((L + kScanTokens - 1) / kScanTokens + a.seg_chunks - 1) / a.seg_chunks);
     a.seg = work;
     a.seg_lw = work + B * H * a.segs * DV * state_row;
+    a.fold = vec && D <= 64 && a.segs <= kFoldSegments;
   }
   if (vec) {
     const int rc = channel_log2 != nullptr ? launch_decay_scan_mfma<true>(a, s) : launch_decay_scan_mfma<false>(a, s);

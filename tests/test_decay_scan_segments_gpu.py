@@ -201,3 +201,31 @@ def test_few_tokens(dev, L, d, dtype, channel):
         # sums of up to 256 products of 2^-24 each, independent: 16 * 2^-24 = 1e-6; bf16 outputs add half of 2^-8
         assert rel(out, ref) < (1e-6 if dtype == torch.float32 else 3e-3) and rel(state[..., :d], S.transpose(2, 3)) < 1e-6
         assert state[..., d:].isnan().all()
+
+
+@pytest.mark.parametrize("channel", [True, False])
+@pytest.mark.parametrize("fresh", [True, False])
+@pytest.mark.parametrize("L,d,dv", [(512, 64, 64), (577, 20, 36), (1100, 64, 100), (2048, 60, 64), (2304, 64, 64), (2500, 36, 16), (700, 72, 64)])
+def test_segments_of_the_matrix_form(dev, L, d, dv, fresh, channel):
+    """Two segments to ten of bf16 portions, put together by those behind them or by a launch of its own, against one chain of portions that
+    are too short for segments."""
+    from based_amd import ops
+
+    B, H = 1, 2
+    g = torch.Generator().manual_seed(L + d)
+    q, k, v = (torch.randn(B, L, H * n, generator=g).bfloat16().to(dev) for n in (d, d, dv))
+    dp = (d + 3) // 4 * 4
+    start = torch.zeros(B, H, dv, dp) if fresh else torch.randn(B, H, dv, dp, generator=g)
+    state = torch.full((B, H, dv, dp), float("nan"), device=dev) if fresh else start.to(dev)
+    lw = (-torch.exp(0.5 * torch.randn(B, L, H, d, generator=g) + torch.linspace(-7, 1, d)) / math.log(2)).flatten(2).to(dev)
+    kw = dict(head_decay=ops.head_decays([0.9995, 0.9], dev)) if not channel else dict(bonus=torch.randn(H, d, generator=g).bfloat16().to(dev))
+    part = lambda s: dict(channel_log2=lw[:, s].contiguous()) if channel else {}  # noqa: E731
+    whole = ops.decay_scan(q, k, v, state, H, fresh=fresh, **kw, **part(slice(0, L)))
+    chain, pieces = start.to(dev), []
+    for at in range(0, L, 192):
+        s = slice(at, min(at + 192, L))
+        pieces.append(ops.decay_scan(q[:, s], k[:, s], v[:, s], chain, H, fresh=False, **kw, **part(s)))
+    rel = lambda a, b: ((a.double() - b.double()).norm() / b.double().norm()).item()  # noqa: E731
+    # outputs: one rounding to bf16 that falls another way, 2^-8 of few values; states: 32-bit sums in another order over up to 2500 tokens
+    assert rel(whole, torch.cat(pieces, 1)) < 1e-3
+    assert rel(state[..., :d], chain[..., :d]) < 1e-5
