@@ -283,10 +283,15 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
     }
 
     if constexpr (HALVES > 1) __builtin_amdgcn_sched_barrier(0);
-    f32x4 diag = {0.f, 0.f, 0.f, 0.f};  // the weights inside the 16 tokens: column t, rows s = 4 quad + i
+    // The weights inside the 16 tokens.  BACK: token t with the one 4 g + quad back in [g], zero where that is none of the 16, four sums
+    // added up over the channels' lanes at once without LDS (two exchanges through LDS a sum, 16 heads of 64, 12 x 960 tokens: 121.2 us ->
+    // 117.1; 12 heads, 1 x 1000: 50.2 -> 47.8); otherwise column t, rows s = 4 quad + i (128 channels: 104.9 us, 107.5 with BACK, which spills
+    // more).
+    constexpr bool BACK = CHANNEL && HALVES == 1;
+    f32x4 diag = {0.f, 0.f, 0.f, 0.f};
     if constexpr (CHANNEL && !STATE_ONLY) {
       const int rel = l16 - quad * 4;  // row i is j tokens back where rel = j + i
-      float sum = 0.f;
+      float sum = 0.f, four[4];
 #pragma unroll
       for (int g = 0; g < 2 * DT; ++g) {
         const int ch = chan(g >> 1, g & 1) < a.d ? chan(g >> 1, g & 1) : 0;
@@ -294,16 +299,19 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
 #pragma unroll
         for (int j = 0; j < 4; ++j) sum = __builtin_fmaf(q[g * 4 + j] * to_f32(u[j]), k[g * 4 + j], sum);
       }
-      sum = quad_rows_sum(sum);
+      four[0] = sum;
+      if constexpr (!BACK) {
+        sum = quad_rows_sum(sum);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) diag[i] = rel == i ? sum : diag[i];
+        for (int i = 0; i < 4; ++i) diag[i] = rel == i ? sum : diag[i];
+      }
       float x[E], before[E];
 #pragma unroll
       for (int i = 0; i < E; ++i) {
         x[i] = row_moved<0x111>(k[i]);
         before[i] = row_moved<0x111>(w[i]);  // of the token before
       }
-      constexpr int kUnroll = 3;  // (few steps in flight: registers are scarce)
+      constexpr int kUnroll = BACK ? 15 : 3;  // (few steps in flight: registers are scarce)
 #pragma unroll kUnroll
       for (int j = 1; j < 16; ++j) {
         sum = 0.f;
@@ -312,9 +320,18 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
           sum = __builtin_fmaf(q[i], x[i], sum);
           x[i] = row_moved<0x111>(x[i]) * before[i];
         }
-        sum = quad_rows_sum(sum);
+        if constexpr (BACK) {
+          four[j % 4] = sum;
+          if (j % 4 == 3) {
+            sum = sum_quads4(four[0], four[1], four[2], four[3]);
+            diag[j / 4] = j - 3 + quad <= l16 ? sum : 0.f;
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        } else {
+          sum = quad_rows_sum(sum);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) diag[i] = rel == j + i ? sum : diag[i];
+          for (int i = 0; i < 4; ++i) diag[i] = rel == j + i ? sum : diag[i];
+        }
       }
     }
 
@@ -498,7 +515,14 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
           split2(P[j][2 * i], P[j][2 * i + 1], x, y);
           hi[i] = x, lo[i] = y;
         }
-        if (half == 0 && j <= (blk | 1)) {
+        if (CHANNEL && HALVES == 1 && j == blk) {  // as diag has them
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const int s0 = t * TS + j * 16 + ((l16 - 8 * i - quad) & 15), s1 = t * TS + j * 16 + ((l16 - 8 * i - 4 - quad) & 15);
+            store_pair(&lds.p.hi[s0], &lds.p.hi[s1], hi[i]);
+            store_pair(&lds.p.lo[s0], &lds.p.lo[s1], lo[i]);
+          }
+        } else if (half == 0 && j <= (blk | 1)) {
           *reinterpret_cast<u32x2*>(&lds.p.hi[t * TS + j * 16 + quad * 4]) = hi;
           *reinterpret_cast<u32x2*>(&lds.p.lo[t * TS + j * 16 + quad * 4]) = lo;
         }

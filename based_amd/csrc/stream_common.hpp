@@ -101,6 +101,17 @@ __device__ __forceinline__ float max_quads(float v) {
   return fmaxf(__builtin_bit_cast(float, q0), __builtin_bit_cast(float, q1));
 }
 
+// Sums of four values over the lanes l, l ^ 16, l ^ 32, l ^ 48: the 16-lane row r receives that of value r.  All 64 lanes are on.
+__device__ __forceinline__ float sum_quads4(float a, float b, float c, float d) {
+  const auto ab = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  const auto cd = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, c), __builtin_bit_cast(unsigned, d), false, false);
+  const unsigned ab0 = ab[0], ab1 = ab[1], cd0 = cd[0], cd1 = cd[1];
+  const float lo = __builtin_bit_cast(float, ab0) + __builtin_bit_cast(float, ab1), hi = __builtin_bit_cast(float, cd0) + __builtin_bit_cast(float, cd1);
+  const auto all = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, lo), __builtin_bit_cast(unsigned, hi), false, false);
+  const unsigned x = all[0], y = all[1];
+  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+}
+
 inline bool aligned_to(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
 
 // Sum of w_j x_{t - taps + 1 + j} over the past inputs of one channel of a ring (taps slots, `stride` elements
