@@ -36,7 +36,7 @@ struct DecayScanArgs {
   const void* k;
   const void* v;
   const float* lw;       // (B, L, H * d) contiguous: log2 of the channel decays, or null
-  const float* head_lw;  // (2, H): log2 of the head decays, then the decays, or null
+  const float* head_lw;  // (2, H): log2 of the sizes of the head decays, then the decays, or null
   const void* u;         // (H, d)
   float* state;          // (B, H, dv, dp)
   float* seg;            // (B, H, segs, dv, dp) work, null with one segment
@@ -112,13 +112,16 @@ __device__ __forceinline__ void store_pair(__bf16* p, __bf16* q, uint32_t x) {
   *reinterpret_cast<uint16_t*>(q) = (uint16_t)(x >> 16);
 }
 
-// Decay of a head over a segment that is not the last: whole 64-token pieces, an even power (a decay below zero has no logarithm).  A product of
-// decays that only the format makes zero comes as its smallest number: an infinite state outlives it, as it does token by token.
-__device__ __forceinline__ float decay_of_segment(const DecayScanArgs& a, int h) {
-  const float w = a.head_lw[a.H + h], l2 = w < 0.f ? log2f(-w) : a.head_lw[h];
-  const float all = __builtin_amdgcn_exp2f(l2 * (float)(a.seg_chunks * kScanTokens));
-  return all == 0.f && w != 0.f ? 0x1p-149f : all;
-}
+// Powers of a head's decay w, without their signs, from the logarithm of its size.  (Nothing is worked out from the two in front of the first
+// tokens' loads, which would wait for them.)
+struct HeadPowers {
+  float l2, w;
+  __device__ __forceinline__ HeadPowers(const DecayScanArgs& a, int h) : l2(a.head_lw[h]), w(a.head_lw[a.H + h]) {}
+  __device__ __forceinline__ float operator()(int n) const { return __builtin_amdgcn_exp2f(l2 * (float)n); }
+  // What a state is multiplied by.  A product of decays that only the format makes zero comes as the smallest number: an infinite state outlives it,
+  // as it does token by token.
+  __device__ __forceinline__ float of_state(int n) const { return fmaxf((*this)(n), w != 0.f ? 0x1p-149f : 0.f); }
+};
 
 // HALVES wavefronts (1 or 2) share the key channels of 16 tokens, DT 32-channel pieces each (d <= 32 DT HALVES, d % 4 == 0), so
 // that what a lane holds of a token stays in registers; their parts of P are added through LDS.  Channels of a piece are held by the lanes in the
@@ -158,7 +161,10 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
   const __bf16* kp = static_cast<const __bf16*>(a.k) + b * a.k_sb + (long)h * a.d;
   const __bf16* vp = static_cast<const __bf16*>(a.v) + b * a.v_sb + (long)h * a.dv;
   const float* lwp = CHANNEL ? a.lw + ((long)b * a.L) * a.H * a.d + (long)h * a.d : nullptr;
-  const float head_l2 = CHANNEL ? 0.f : a.head_lw[h];
+  const auto powers = [&] {
+    if constexpr (CHANNEL) return nullptr;
+    else return HeadPowers(a, h);
+  }();
   const long bh = (long)b * a.H + h;
   float* st = a.state + (bh * a.dv + (col_in ? dv0 + l16 : 0)) * a.dp;
 
@@ -192,7 +198,8 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
         }
       }
     } else if (fold) {
-      const float seg_decay = CHANNEL ? 0.f : decay_of_segment(a, h);  // (all in front of the last are of one length)
+      float seg_decay = 0.f;  // (all in front of the last are of one length)
+      if constexpr (!CHANNEL) seg_decay = powers.of_state(a.seg_chunks * kScanTokens);
       constexpr int U = HALVES == 1 ? 4 : 2;  // segments asked for together
       for (int s0 = 0; s0 < sg; s0 += U) {
         f32x4 add[U][2 * DA], l[U][2 * DA];
@@ -254,6 +261,15 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
   constexpr bool LATE = CHANNEL && !STATE_ONLY && HALVES > 1;
   Stage cur;
   if (first < last) fetch(cur, first);
+  // A head decay below zero: with w's sign s, s^t v_t in the place of v_t, s S in that of the state and s^t o_t in that of o_t, the powers are
+  // those of |w| (4 x 2048 tokens, 16 heads of 64: 43.4 us, without signs at all 43.4; on the weights themselves 44.2, the state turned
+  // in front of the first tokens 43.8).
+  uint32_t odd_sign = 0u;  // of two halves, where this lane's token has an odd number
+  auto turn_state = [&](bool turn) {
+#pragma unroll
+    for (int ct = 0; ct < 2 * DA; ++ct) S[ct] = turn ? -S[ct] : S[ct];
+  };
+  if constexpr (!CHANNEL) odd_sign = powers.w < 0.f && (l16 & 1) ? 0x80008000u : 0u;
   for (int chunk = first; chunk < last; ++chunk) {
     const int left = a.L - chunk * kScanTokens, n = left < kScanTokens ? left : kScanTokens;
     const int t = blk * 16 + l16;  // this lane's token
@@ -349,7 +365,7 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
       for (int f = 0; f < 4; ++f) {
         const bool in = live && col_base + half * 64 + quad * 16 + f * 4 < a.dv;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) vv[f * 2 + j] = in ? pack_bf16(v[f * 4 + 2 * j], v[f * 4 + 2 * j + 1]) : 0u;
+        for (int j = 0; j < 2; ++j) vv[f * 2 + j] = in ? pack_bf16(v[f * 4 + 2 * j], v[f * 4 + 2 * j + 1]) ^ odd_sign : 0u;
       }
     }
     if (!LATE && chunk + 1 < last) fetch(cur, chunk + 1);
@@ -384,7 +400,7 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
         }
       }
     } else {
-      const float f = __builtin_amdgcn_exp2f(head_l2 * (float)(n - 1 - t > 0 ? n - 1 - t : 0));
+      const float f = powers(n - 1 - t > 0 ? n - 1 - t : 0);
 #pragma unroll
       for (int i = 0; i < E; i += 2) {
         uint32_t hi, lo;
@@ -488,7 +504,7 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int dist = t - (j * 16 + quad * 4 + i);
-          P[j][i] = dist >= 0 ? P[j][i] * __builtin_amdgcn_exp2f(head_l2 * (float)dist) : 0.f;
+          P[j][i] = dist >= 0 ? P[j][i] * powers(dist) : 0.f;
         }
       }
     }
@@ -535,11 +551,27 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
 #pragma unroll
       for (int g = 0; g < 2; ++g) v8[g] = *reinterpret_cast<const bf16x8*>(&lds.vt[(wave * 16 + l16) * TS + g * 32 + quad * 8]);
       if constexpr (!STATE_ONLY) {
+        if constexpr (!CHANNEL) {
+          if (chunk == first && powers.w < 0.f) turn_state(true);  // (no sooner: the state is on its way until here)
+        }
         bf16x8 sh[DA], sl[DA];
 #pragma unroll
         for (int c = 0; c < DA; ++c) {
           const float x[8] = {S[2 * c][0], S[2 * c][1], S[2 * c][2], S[2 * c][3], S[2 * c + 1][0], S[2 * c + 1][1], S[2 * c + 1][2], S[2 * c + 1][3]};
           split8(x, sh[c], sl[c]);
+        }
+        if constexpr (!CHANNEL) {  // (rounding leaves nothing of an infinity: the difference of two is no number)
+          float most = 0.f;
+#pragma unroll
+          for (int ct = 0; ct < 2 * DA; ++ct)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) most = fmaxf(most, fabsf(S[ct][j]));
+          if (__any(most == INFINITY)) {
+#pragma unroll
+            for (int ct = 0; ct < 2 * DA; ++ct)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) sl[ct / 2][ct % 2 * 4 + j] = fabsf(S[ct][j]) == INFINITY ? (__bf16)0.f : sl[ct / 2][ct % 2 * 4 + j];
+          }
         }
 #pragma unroll
         for (int tb = 0; tb < 4; ++tb) {
@@ -556,7 +588,7 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
               acc = mfma_16(sh[c], ql, acc);
             }
           }
-          if constexpr (!CHANNEL) acc *= __builtin_amdgcn_exp2f(head_l2 * (float)(tok + 1));
+          if constexpr (!CHANNEL) acc *= powers.of_state(tok + 1);
 #pragma unroll
           for (int g = 0; g < 2; ++g) {
             if (g * 2 > tb) continue;
@@ -566,10 +598,9 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
             acc = mfma_16(v8[g], pl, acc);
           }
           if (tok < n && dv0 + quad * 4 < a.dv) {
-            bf16x4 out;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) out[i] = (__bf16)acc[i];
-            *reinterpret_cast<bf16x4*>(static_cast<__bf16*>(a.o) + b * a.o_sb + (long)(chunk * kScanTokens + tok) * a.o_sl +
+            typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+            const u32x2 out = {pack_bf16(acc[0], acc[1]) ^ odd_sign, pack_bf16(acc[2], acc[3]) ^ odd_sign};
+            *reinterpret_cast<u32x2*>(static_cast<__bf16*>(a.o) + b * a.o_sb + (long)(chunk * kScanTokens + tok) * a.o_sl +
                                        (long)h * a.dv + dv0 + quad * 4) = out;
           }
         }
@@ -581,7 +612,7 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
         if constexpr (CHANNEL) {
           S[ct] *= *reinterpret_cast<const f32x4*>(&lds.all[ct * 16 + quad * 4]);
         } else {
-          S[ct] *= __builtin_amdgcn_exp2f(head_l2 * (float)n);
+          S[ct] *= powers.of_state(n);
         }
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
@@ -597,6 +628,7 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
     if (blockIdx.y == 0 && threadIdx.x < a.d) a.seg_lw[(bh * a.segs + sg) * a.dp + threadIdx.x] = seg_total;
   }
   if (!has_cols) return;
+  if constexpr (!CHANNEL) turn_state(powers.w < 0.f && !(last == chunks && (a.L & 1)));  // (of an odd number of tokens the signs are turned already)
   float* to = st;
   if constexpr (STATE_ONLY) to = a.seg + ((bh * a.segs + sg) * a.dv + (col_in ? dv0 + l16 : 0)) * a.dp;
   if (STATE_ONLY || sg == a.segs - 1) {
@@ -619,7 +651,7 @@ __global__ __launch_bounds__(256) void decay_join_kernel(const DecayScanArgs a) 
   float* st = a.state + (bh * a.dv + col) * a.dp + ch;
   f32x4 S = {0.f, 0.f, 0.f, 0.f};
   if (!a.fresh) S = *reinterpret_cast<const f32x4*>(st);
-  const float head = a.lw != nullptr ? 0.f : decay_of_segment(a, (int)(bh % a.H));
+  const float head = a.lw != nullptr ? 0.f : HeadPowers(a, (int)(bh % a.H)).of_state(a.seg_chunks * kScanTokens);
   for (int s = 0; s < a.segs; ++s) {
     float* p = a.seg + ((bh * a.segs + s) * a.dv + col) * a.dp + ch;
     f32x4 add = {0.f, 0.f, 0.f, 0.f};

@@ -1204,10 +1204,10 @@ def _check_decay_state(state, rows: int, heads: int, d: int, dv: int) -> None:
 
 
 def head_decays(decay, device) -> torch.Tensor:
-    """(2, H) fp32 for the head form of decay_scan and decay_step: base-2 logarithms of the decays as fp32 holds them, and the decays.
-    A decay of zero is one whose powers are zero (0 * -inf would not be a number)."""
+    """(2, H) fp32 for the head form of decay_scan and decay_step: base-2 logarithms of the sizes of the decays as fp32 holds them,
+    and the decays.  A decay of zero is one whose powers are zero (0 * -inf would not be a number)."""
     value = torch.tensor(list(decay), dtype=torch.float32)
-    log2 = torch.where(value > 0, value.double().log2(), torch.full_like(value, -1e4).double()).float()
+    log2 = torch.where(value != 0, value.double().abs().log2(), torch.full_like(value, -1e4).double()).float()
     return torch.stack([log2, value]).to(device)
 
 

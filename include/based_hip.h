@@ -632,8 +632,8 @@ BASED_API int based_token_side_step(const void* x, const float* residual_in, flo
 
 /* Linear attention with decaying states over a portion; q, k (B, L, H * D), v, o (B, L, H * DV), silu on q, k
  * and v first with BASED_ACT_SILU.  channel_log2 (B, L, H * D) contiguous, the log2 of a decay w per key channel, with
- * bonus u (H, D): o_t = (S + diag(u) k v^T)^T q, S <- diag(w) S + k v^T.  Or head_decay (2, H), the log2 of constants w
- * and w itself:
+ * bonus u (H, D): o_t = (S + diag(u) k v^T)^T q, S <- diag(w) S + k v^T.  Or head_decay (2, H), the log2 of the size of
+ * constants w (of zero a number whose powers are zero) and w itself:
  * S <- w S + k v^T, o = S^T q.  state (B, H, DV, state_row) fp32, by value channel; work: as many floats as
  * based_decay_scan_work_of says for the call (0: may be NULL), or based_decay_scan_work for any call of the sizes; without it, what is not
  * bf16 in whole 8-byte pieces is walked in one chain.  Both are 0 below BASED_DECAY_SEGMENTS_MIN tokens.  bits: the addresses of q, k, v,

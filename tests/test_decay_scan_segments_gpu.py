@@ -229,3 +229,71 @@ def test_segments_of_the_matrix_form(dev, L, d, dv, fresh, channel):
     # outputs: one rounding to bf16 that falls another way, 2^-8 of few values; states: 32-bit sums in another order over up to 2500 tokens
     assert rel(whole, torch.cat(pieces, 1)) < 1e-3
     assert rel(state[..., :d], chain[..., :d]) < 1e-5
+
+
+def _head_decays_in_64_bits(q, k, v, w, state):
+    """o (B, L, H, dv) and the state (B, H, dv, d) behind a portion, token by token."""
+    B, L, H, d = q.shape
+    S, o = state.double().transpose(2, 3), []
+    for t in range(L):
+        S = w.double().view(1, H, 1, 1) * S + k[:, t].double()[..., None] * v[:, t].double()[:, :, None]
+        o.append((S * q[:, t].double()[..., None]).sum(2))
+    return torch.stack(o, 1), S.transpose(2, 3)
+
+
+@pytest.mark.parametrize("L,d,dv", [(100, 64, 64), (301, 20, 36), (513, 64, 64), (577, 32, 16), (1100, 64, 100), (2048, 60, 64), (2500, 36, 16),
+                                    (200, 72, 64), (1030, 128, 64)])
+def test_signs_of_head_decays_in_the_matrix_form(dev, L, d, dv):
+    """Decays below zero, zero and above, bf16: one chain, two segments to eight that put the ones in front together themselves, ten, and heads of
+    more than 64 channels."""
+    from based_amd import ops
+
+    B, decay = 2, [-0.9, -0.9995, -1.0, 0.0, 0.999, -2.0 ** -9]
+    H, g = len(decay), torch.Generator().manual_seed(L + d)
+    q, k, v = (torch.randn(B, L, H, n, generator=g).bfloat16() for n in (d, d, dv))
+    S0 = torch.randn(B, H, dv, d, generator=g)
+    state = S0.to(dev)
+    got = ops.decay_scan(*(x.flatten(2).to(dev) for x in (q, k, v)), state, H, head_decay=ops.head_decays(decay, dev), fresh=False)
+    want, S = _head_decays_in_64_bits(q, k, v, torch.tensor(decay), S0)
+    got, state = got.double().cpu().view(B, L, H, dv), state.double().cpu()
+    for h in range(H):  # each head by itself: they differ in size by up to fifty times
+        rel = lambda a, b: ((a[..., h, :] - b[..., h, :]).norm() / b[..., h, :].norm()).item()  # noqa: E731
+        # bf16 outputs: half of 2^-8 at most, 2^-9 / 3^0.5 = 1.1e-3 evenly spread; weights keep 16 bits
+        assert rel(got, want) < 3e-3 and rel(got[:, -8:], want[:, -8:]) < 3e-3, (decay[h], rel(got, want))
+        rel = lambda a, b: ((a[:, h] - b[:, h]).norm() / b[:, h].norm()).item()  # noqa: E731
+        # a sum's terms keep 16 bits each, 2^-17 / 3^0.5 = 4.4e-6 evenly spread, signs independent
+        assert rel(state, S) < 2e-5, (decay[h], rel(state, S))
+
+
+@pytest.mark.parametrize("L", [60, 150, 513, 1100, 2500])
+def test_infinite_states_in_the_matrix_form(dev, L):
+    """An infinite part of the state that enters, head decays, bf16, one chain to ten segments: infinite and no numbers where they are token by token."""
+    from based_amd import ops
+
+    decay, d, dv = [-0.9, 2.0 ** -9, 0.0, 0.999, -2.0 ** -9], 64, 64
+    H, g = len(decay), torch.Generator().manual_seed(L)
+    q, k, v = (torch.randn(1, L, H, n, generator=g).bfloat16() for n in (d, d, dv))
+    S0 = torch.randn(1, H, dv, d, generator=g)
+    S0[:, :, 3, 5], S0[:, :, 40, 63] = float("inf"), float("-inf")
+    state = S0.to(dev)
+    got = ops.decay_scan(*(x.flatten(2).to(dev) for x in (q, k, v)), state, H, head_decay=ops.head_decays(decay, dev), fresh=False)
+    want, S = _head_decays_in_64_bits(q, k, v, torch.tensor(decay), S0)
+    for a, b in ((got.cpu().view(1, L, H, dv), want), (state.cpu(), S)):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf()) and torch.equal(a[a.isinf()] > 0, b[b.isinf()] > 0)
+
+
+@pytest.mark.parametrize("L", [60, 513, 1100, 2500])
+def test_infinite_states_and_channel_decays_in_the_matrix_form(dev, L):
+    """The same with channel decays: the state's part stays infinite, and what does not meet it stays a number."""
+    from based_amd import ops
+
+    H, d, dv, g = 2, 64, 64, torch.Generator().manual_seed(L)
+    q, k, v, u = (torch.randn(*s, generator=g).bfloat16().to(dev) for s in ((1, L, H * d), (1, L, H * d), (1, L, H * dv), (H, d)))
+    lw = torch.full((1, L, H * d), -2.0 ** -5, device=dev)  # (2^-2 over 64 tokens, 2^-79 over all)
+    state = torch.randn(1, H, dv, d, generator=g).to(dev)
+    state[:, :, 3, 5], state[:, :, 40, 63] = float("inf"), float("-inf")
+    out = ops.decay_scan(q, k, v, state, H, channel_log2=lw, bonus=u, fresh=False).view(1, L, H, dv)
+    assert (state[:, :, 3, 5] == float("inf")).all() and (state[:, :, 40, 63] == float("-inf")).all()
+    assert not out[..., [3, 40]].isfinite().any()
+    state[:, :, 3, 5], state[:, :, 40, 63], out[..., [3, 40]] = 0, 0, 0
+    assert state.isfinite().all() and out.isfinite().all()
