@@ -1191,9 +1191,11 @@ static bool route_by_row(const RouteArgs& a, int piece) {
   return a.D % piece == 0 && a.D <= kRouteRowMax && a.h_sr % piece == 0 && aligned_to(a.h, 16) && aligned_to(a.w, 16);
 }
 
-// A workgroup to each token (element by element, a score to a thread, 12 tokens of 1024 channels took 70 us)
+// A workgroup to each token, or a score to a thread (element by element: 12 tokens of 1024 channels take 70 us) where the tokens are so many that
+// workgroups cost more than channels: calls of 8 experts of ff 64 with 64 channels, 1024 tokens 18.3 us by rows and 19.7 by scores, 4096 tokens 51.6
+// and 45.7; 256 channels, 4096 tokens 113 and 117; 64 experts, 32 channels, 1024 tokens 17.0 and 26.4, 4096 tokens 46.9 and 39.1.
 static void launch_route_f32(const RouteArgs& r, bool by_row, hipStream_t s) {
-  if (by_row)
+  if (by_row && r.n <= (long)16 * r.D * ((r.E + 15) / 16))
     hipLaunchKernelGGL(expert_route_row_kernel<float>, dim3((unsigned)r.n), dim3(512), 0, s,
                        RouteRowArgs{r, nullptr, nullptr, nullptr, nullptr, 1.f, 0.f, BASED_NORM_RMS});
   else

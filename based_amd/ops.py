@@ -1395,6 +1395,11 @@ EXPERT_ROWS_MAX = 16
 # fp32 choices per expert likewise: 2 of 8 experts of 1024, 6 tokens 30.7 us by rows and 46.8 grouped, 20 tokens 68 and 49; 1 of 8 of 2048, 16 tokens
 # 65 and 80, 24 tokens 88 and 80; 4 of 16 of 512, 12 tokens 48 and 54, 20 tokens 66 and 54.
 EXPERT_ROWS_F32_MAX = 3
+# Channels and features from which on, and features of all experts (a sixteenth of the workgroups of the first product).  Small matrices stay in the
+# caches for every choice, and few workgroups leave the GPU idle.  2 of 8 experts, 1024 tokens, us by rows and grouped: 64 x 64 18 and 74,
+# 256 x 256 87 and 103, 512 x 512 250 and 104; 64 experts, 256 x 256 101 and 102, 256 x 64 43 and 60; one expert of 512 136 and 319, one of four
+# (2048 features in all) 145 and 98; one of 2048 x 512 482 and 1088, one of four 493 and 341.
+EXPERT_GROUPED_F32_SIZE_MIN, EXPERT_GROUPED_F32_FEATURES_MIN = 512, 2048
 EXPERT_NORM_MAX_DIM = 4096
 
 
@@ -1444,6 +1449,11 @@ def experts(h, router, w1, w2, top: int, norm=None) -> torch.Tensor:
     return y.view(h.shape)
 
 
+def _experts_f32_grouped(slots: int, D: int, F: int, E: int) -> bool:
+    """Whether fp32 rows of one expert share its matrices."""
+    return slots > EXPERT_ROWS_F32_MAX * E and min(D, F) >= EXPERT_GROUPED_F32_SIZE_MIN and E * F >= EXPERT_GROUPED_F32_FEATURES_MIN
+
+
 def _experts_plan(h, router, w1, w2, top: int):
     """The checked sizes of an `experts` call, whether rows of one expert share its matrices, and where what lies in its work space (bytes; 32-bit
     words in all): scores, choices, their ranks, counts, the plan of the tiles, activations, the choices' outputs."""
@@ -1461,7 +1471,7 @@ def _experts_plan(h, router, w1, w2, top: int):
     n, lib = h2.shape[0], _lib.lib()
     slots = n * top
     grouped = h2.dtype == torch.bfloat16 and slots > EXPERT_ROWS_MAX and D % 8 == 0 and F % 8 == 0 and h2.stride(0) % 8 == 0
-    vec_f32 = h2.dtype == torch.float32 and slots > EXPERT_ROWS_F32_MAX * E and D % 4 == 0 and F % 4 == 0
+    vec_f32 = h2.dtype == torch.float32 and D % 4 == 0 and F % 4 == 0 and _experts_f32_grouped(slots, D, F, E)
     tiles, rows = (lib.based_expert_tiles(n, E, top), lib.based_expert_tile_rows(n, E, top)) if grouped else (0, 0)
     at, ends = 0, []
     act_rows = tiles * rows if grouped else slots

@@ -243,3 +243,15 @@ def test_remembered_checks_are_bounded():
     for i in range(10000):
         kept[i] = i
     assert len(kept) <= 4096 and kept[9999] == 9999
+
+
+def test_fp32_experts_share_matrices_only_where_that_is_faster():
+    """Measured on both sides: many tokens of small matrices, or few experts of small ones, took up to 22 times as long with the matrices shared."""
+    from based_amd import ops
+
+    shared = ops._experts_f32_grouped
+    for slots, D, F, E in ((20000, 32, 32, 4), (16384, 64, 64, 8), (16384, 128, 256, 8), (32768, 64, 64, 256), (300, 4104, 64, 3), (1024, 512, 512, 1),
+                           (4096, 256, 256, 256), (24, 1024, 1024, 8), (4096, 512, 512, 3)):
+        assert not shared(slots, D, F, E), (slots, D, F, E)
+    for slots, D, F, E in ((25, 1024, 1024, 8), (140, 2048, 2048, 8), (49, 512, 512, 16), (16384, 512, 512, 8), (1024, 512, 512, 4), (256, 2048, 512, 64)):
+        assert shared(slots, D, F, E), (slots, D, F, E)

@@ -572,16 +572,35 @@ def test_places_of_the_choices(dev, n, E, top):
 
 @pytest.mark.parametrize("n,D,F,E,top", [(4, 64, 64, 1, 1), (17, 1024, 20, 3, 1), (70, 1028, 260, 4, 2), (33, 2052, 1040, 2, 2), (600, 132, 2048, 5, 2), (1100, 64, 4100, 6, 1),
                                          (300, 4104, 36, 3, 1)])
-def test_experts_grouped_fp32(dev, n, D, F, E, top):
+def test_experts_grouped_fp32(dev, n, D, F, E, top, monkeypatch):
     """One choice in a tile of 16 and more than one tile; channels in one part of a wavefront's registers, in all and beyond them, and a part
     of a piece; more choices than are looked up at once; rows that the routing by rows does not take."""
     from based_amd import ops
 
-    assert n * top > ops.EXPERT_ROWS_F32_MAX * E
+    monkeypatch.setattr(ops, "_CHECKED", ops._Checked())
+    monkeypatch.setattr(ops, "EXPERT_GROUPED_F32_SIZE_MIN", 0)  # (the line is about time: the form takes all of them)
+    monkeypatch.setattr(ops, "EXPERT_GROUPED_F32_FEATURES_MIN", 0)
+    assert ops._experts_f32_grouped(n * top, D, F, E)
     h, router, w1, w2, w = expert_case(n, D, F, E, top, torch.float32, seed=n)
     want = O.expert_mlp(h.double(), w, "m", {"router": {"top": top}})
     got = ops.experts(h.to(dev), router.to(dev), w1.to(dev), w2.to(dev), top).double().cpu()
     s = O.sigmoid(h.double() @ router.double().T).sort(-1, descending=True).values
     clear = torch.ones(n, dtype=torch.bool) if top == E else s[:, top - 1] - s[:, top] > 1e-5
+    assert clear.sum() >= 0.98 * n
+    close(got[clear], want[clear], 2 * TOL[torch.float32])
+
+
+@pytest.mark.parametrize("n,D,F,E,top", [(512, 32, 16, 3, 2), (513, 32, 16, 3, 2), (1025, 64, 64, 16, 1), (2049, 64, 20, 17, 3), (9000, 32, 32, 250, 1), (4096, 512, 512, 4, 1)])
+def test_experts_of_many_tokens_fp32(dev, n, D, F, E, top):
+    """Scores by workgroups of tokens up to where scores by threads are faster, and beyond; small matrices, by choices however many those are, and
+    the smallest that choices share."""
+    from based_amd import ops
+
+    assert ops._experts_f32_grouped(n * top, D, F, E) == (D == 512)
+    h, router, w1, w2, w = expert_case(n, D, F, E, top, torch.float32, seed=n)
+    want = O.expert_mlp(h.double(), w, "m", {"router": {"top": top}})
+    got = ops.experts(h.to(dev), router.to(dev), w1.to(dev), w2.to(dev), top).double().cpu()
+    s = O.sigmoid(h.double() @ router.double().T).sort(-1, descending=True).values
+    clear = s[:, top - 1] - s[:, top] > 1e-5
     assert clear.sum() >= 0.98 * n
     close(got[clear], want[clear], 2 * TOL[torch.float32])
