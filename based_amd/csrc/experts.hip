@@ -403,7 +403,8 @@ struct ExpertGemmArgs {
   __bf16* y;             // PAIRED: (tiles * rows, F); otherwise (slots, F) scattered by order
   const int32_t* order;
   const int32_t* tile_first;
-  const int32_t* tile_expert;
+  const int32_t* tile_expert;  // or null (small tiles): from tile_first and counts
+  const int32_t* counts;
   const float* scores;   // (slots), PAIRED
   long x_sr;
   int E, F, K, top, col_tiles, tiles;
@@ -436,7 +437,17 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(const ExpertGemmArg
   const int tile = band * kBand + in_band % deep, f0 = in_band / deep * (PAIRED ? HALF : BN);
   if (tile >= a.tile_first[a.E]) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4, wm = wave % WM, wn = wave / WM;
-  const int what = a.tile_expert[tile], e = what & 255, rows = what >> 8;
+  int e, rows;
+  if (a.tile_expert != nullptr) {
+    const int what = a.tile_expert[tile];
+    e = what & 255, rows = what >> 8;
+  } else {
+    e = 0;
+    for (int x0 = 0; x0 < a.E; x0 += 64) e += __popcll(__ballot(x0 + lane < a.E && a.tile_first[x0 + lane < a.E ? x0 + lane + 1 : 0] <= tile));
+    e = __builtin_amdgcn_readfirstlane(e);
+    rows = a.counts[e] - (tile - a.tile_first[e]) * BM;
+    rows = rows < BM ? rows : BM;
+  }
   for (int i = tid; i < BM; i += 256) slot_of[i] = a.order[(long)tile * BM + (i < rows ? i : 0)];
   lds_barrier();
   typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
@@ -1216,10 +1227,17 @@ static int route_check(const char* who, const RouteArgs& a) {
 // 1 of 8 of 2048, 900 tokens (112 an expert) 61.8 and 69.2; 4 of 16 of 512, 400 tokens (100) 41.7 and 46.9, 200 tokens (50) 41.5 and 40.7.
 static int expert_tile_rows(int64_t slots, int64_t E) { return slots >= 96 * E ? BASED_EXPERT_TILE_ROWS : BASED_EXPERT_TILE_ROWS_SMALL; }
 
+static int64_t expert_tiles(int64_t slots, int64_t E, int64_t rows) { return slots / rows + (E < slots ? E : slots); }
+
+// Few large tiles leave most of the GPU idle: such a call goes in small ones all the same, in the scratch of the large ones.  Choices in all at which both
+// take the same time, whether of one expert or of sixteen: 256 x 256 4,000, 512 x 512 2,000, 768 x 768 1,250, 1024 x 1024 900, 2048 x 2048 450, 1024
+// channels x 64 2,000, 64 x 1024 1,050, 512 x 2048 1,300, 1024 x 512 1,000, 4096 x 1024 450; 128 x 128 the same at any number.  100 tokens, one
+// expert of 1024: 33.2 us in large ones, 27.9 in small ones; 200, 1 of 2 of 2048 x 2048 54.0 and 41.7; 400, 2 of 8 of 1024 42.6 and 46.3.
+static bool expert_large_products(int64_t slots, int64_t D, int64_t F) { return D + F <= 256 || (double)slots * (D + F) >= 1.6e6; }
+
 extern "C" BASED_API int64_t based_expert_tiles(int64_t n, int64_t E, int64_t top) {
   if (n <= 0 || E <= 0 || top <= 0) return 0;
-  const int64_t rows = expert_tile_rows(n * top, E);
-  return n * top / rows + (E < n * top ? E : n * top);
+  return expert_tiles(n * top, E, expert_tile_rows(n * top, E));
 }
 
 extern "C" BASED_API int64_t based_expert_tile_rows(int64_t n, int64_t E, int64_t top) { return expert_tile_rows(n * top, E); }
@@ -1238,16 +1256,20 @@ extern "C" BASED_API int based_expert_grouped(const void* h, const void* router,
   BASED_REQUIRE(aligned_to(h, 16) && aligned_to(w1, 16) && aligned_to(w2, 16) && aligned_to(work_act, 16) && aligned_to(work_out, 16) &&
                     aligned_to(y, 16),
                 BASED_ERR_ALIGN, "expert_grouped: tensors must be 16-byte aligned");
-  RouteArgs r{h, router, ids, scores, rank, counts, nullptr, tile_first, tile_expert, order, 0, (long)n, (long)h_sr, (int)D, (int)E, (int)top};
+  RouteArgs r{h, router, ids, scores, rank, counts, nullptr, tile_first, nullptr, order, 0, (long)n, (long)h_sr, (int)D, (int)E, (int)top};
   const int rc = route_check("expert_grouped", r);
   if (rc != BASED_OK) return rc;
   if (n == 0) return BASED_OK;
   const int64_t slots = n * top;
-  const int rows = expert_tile_rows(slots, E);
-  const int64_t tiles = based_expert_tiles(n, E, top);
+  int rows = expert_tile_rows(slots, E);
+  if (rows == BASED_EXPERT_TILE_ROWS && !expert_large_products(slots, D, F)) {
+    rows = BASED_EXPERT_TILE_ROWS_SMALL;  // (rows of all tiles together are no more, 32 - 1 to an expert in place of 256 - 1; the tiles are)
+    tile_expert = nullptr;
+  }
+  const int64_t tiles = expert_tiles(slots, E, rows);
   BASED_REQUIRE(tiles * ((F > D ? F : D) / 64 + 1) < (1ll << 31), BASED_ERR_SHAPE, "expert_grouped: too many rows");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  r.tile_rows = rows;
+  r.tile_rows = rows, r.tile_expert = tile_expert;
   const bool vec = route_vec(r);
   const int group = route_group(r, vec);
   const int64_t groups = (n + group - 1) / group;
@@ -1267,10 +1289,10 @@ extern "C" BASED_API int based_expert_grouped(const void* h, const void* router,
     hipLaunchKernelGGL(expert_place_kernel, dim3((unsigned)((groups + kPlaceGroups - 1) / kPlaceGroups)), dim3(kPlaceThreads), 0, s, p);
   }
   const ExpertGemmArgs a{static_cast<const __bf16*>(h), static_cast<const __bf16*>(w1), static_cast<__bf16*>(work_act), order, tile_first,
-                         tile_expert, scores, (long)h_sr, (int)E, (int)F, (int)D, (int)top, 0, (int)tiles};
+                         tile_expert, counts, scores, (long)h_sr, (int)E, (int)F, (int)D, (int)top, 0, (int)tiles};
   __bf16* out = static_cast<__bf16*>(top == 1 ? y : work_out);
   const ExpertGemmArgs a2{static_cast<const __bf16*>(work_act), static_cast<const __bf16*>(w2), out, order, tile_first,
-                          tile_expert, scores, (long)F, (int)E, (int)D, (int)F, (int)top, 0, (int)tiles};
+                          tile_expert, counts, scores, (long)F, (int)E, (int)D, (int)F, (int)top, 0, (int)tiles};
   int done = launch_expert_product<true>(a, rows, s);
   if (done == BASED_OK) done = launch_expert_product<false>(a2, rows, s);
   if (done != BASED_OK) return done;

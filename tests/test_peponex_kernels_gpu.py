@@ -604,3 +604,24 @@ def test_experts_of_many_tokens_fp32(dev, n, D, F, E, top):
     clear = s[:, top - 1] - s[:, top] > 1e-5
     assert clear.sum() >= 0.98 * n
     close(got[clear], want[clear], 2 * TOL[torch.float32])
+
+
+@pytest.mark.parametrize("n,D,F,E,top", [(96, 264, 136, 1, 1), (255, 136, 128, 1, 1), (500, 1024, 520, 1, 1), (511, 512, 512, 2, 1), (380, 1024, 1024, 4, 2),
+                                         (6050, 128, 136, 63, 1), (4990, 160, 160, 5, 1), (5010, 160, 160, 5, 1)])
+def test_experts_of_few_large_tiles(dev, n, D, F, E, top):
+    """Batches planned in tiles of 256 rows and multiplied in tiles of 32, which find their expert themselves: one expert to 63, one of them
+    chosen by nobody; scratch that is just enough; both sides of the line."""
+    from based_amd import _lib, ops
+
+    assert _lib.lib().based_expert_tile_rows(n, E, top) == 256
+    h, router, w1, w2, w = expert_case(n, D, F, E, top, BF16, seed=n)
+    if E > 4:
+        h = (h + 1).to(BF16)
+        router[E // 2] = -0.5  # (a score of sigmoid(-D / 2): among the last of every token)
+    w["m.router"] = router.double()
+    want = O.expert_mlp(h.double(), w, "m", {"router": {"top": top}})
+    got = ops.experts(h.to(dev), router.to(dev), w1.to(dev), w2.to(dev), top).double().cpu()
+    s = O.sigmoid(h.double() @ router.double().T).sort(-1, descending=True).values
+    clear = torch.ones(n, dtype=torch.bool) if top == E else s[:, top - 1] - s[:, top] > 1e-5
+    assert clear.sum() >= 0.9 * n
+    close(got[clear], want[clear], 2 * TOL[BF16])
