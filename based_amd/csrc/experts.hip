@@ -612,7 +612,10 @@ template <bool PAIRED> __device__ __forceinline__ void large_store(const ExpertG
 // One barrier a phase; the wait in front of it leaves the loads of six phases on their way.  The compiler, which knows of no distance between
 // these loads and reads of LDS, would wait for all of them in front of every read: it does for a static array (148 us where this takes 94), not for one
 // whose extent the launch gives.
-template <bool PAIRED> __device__ __forceinline__ void large_whole_tile(const ExpertGemmArgs& a, const ExpertTile& t, __bf16* lds, const int* slot_of) {
+// TAIL: the last round of channels is no whole one.  It comes by itself behind the others, nothing else on its way any more.  8192 tokens, 2 of 8 experts,
+// 1000 channels and features: 159 us a call, everything in parts of 128 or 64 rows 204; 32,768 tokens, 1032 channels, 520 features 363 and 465.
+template <bool PAIRED, bool TAIL>
+__device__ __forceinline__ void large_whole_tile(const ExpertGemmArgs& a, const ExpertTile& t, __bf16* lds, const int* slot_of) {
   constexpr int KS = kGemmK;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, quad = lane >> 4;
   const int wm = wave & 1, wn = wave >> 1;
@@ -624,7 +627,9 @@ template <bool PAIRED> __device__ __forceinline__ void large_whole_tile(const Ex
   for (int h = 0; h < 2; ++h)
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const int r = h * 128 + row + 8 * i, c = (piece ^ (4 * i)) * 8;
+      const int r = h * 128 + row + 8 * i;
+      int c = (piece ^ (4 * i)) * 8;
+      if (TAIL && c >= a.K) c = 0;  // (no whole round: what is asked for in its place lies in the row)
       xrow[h][i] = large_x_row<PAIRED>(a, t, slot_of, r) + c;
       wrow[h][i] = (large_w_row<PAIRED>(a, t.f0, r) * (uint32_t)a.K + (uint32_t)c) * 2u;
     }
@@ -715,6 +720,35 @@ template <bool PAIRED> __device__ __forceinline__ void large_whole_tile(const Ex
   }
   if (rounds & 1) round_of(rounds - 1, wa, wb);
   __builtin_amdgcn_s_waitcnt(0x0070);  // (nothing may come into LDS that is no longer this workgroup's)
+  if constexpr (TAIL) {
+    __builtin_amdgcn_s_barrier();  // every wavefront's loads have landed
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int half = 0; half < 4; ++half)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        load_to_lds<true>(half < 2 ? xrow[half & 1][i] + rounds * KS
+                                   : reinterpret_cast<const __bf16*>(reinterpret_cast<const char*>(t.w + rounds * KS) + wrow[half & 1][i]),
+                          lds + half * kHalf + (wave * 16 + i * 8) * KS, rounds * KS + (piece ^ (4 * i)) * 8, a.K);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    read_x(0, 0, x0);
+    read_w(0, 0, wa);
+    read_w(0, 1, wb);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      multiply(x0, wa, acc[0][0], kk);
+      multiply(x0, wb, acc[0][1], kk);
+    }
+    read_x(0, 1, x1);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      multiply(x1, wb, acc[1][1], kk);
+      multiply(x1, wa, acc[1][0], kk);
+    }
+  }
   // column = row l16 of the tile's rows, rows = features 4 quad + i
   int slot[2][4];
   float score[2][4];
@@ -823,15 +857,15 @@ __device__ __forceinline__ void large_part(const ExpertGemmArgs& a, const Expert
   }
 }
 
-// TAIL: the last round of channels is no whole one, and all tiles go in parts (a whole one would have to spill registers).  Block i is number i / 8 of die i % 8.
+// TAIL: the last round of channels is no whole one.  Block i is number i / 8 of die i % 8.
 template <bool PAIRED, bool TAIL> __global__ __launch_bounds__(512, 2) void expert_gemm_large_kernel(const ExpertGemmArgs a) {
   extern __shared__ __attribute__((aligned(16))) __bf16 lds[];
   int* slot_of = reinterpret_cast<int*>(lds + kPartDepth * kPartSlot);
   const int row_tiles = a.tile_first[a.E], all = row_tiles * a.col_tiles;
   const int die = blockIdx.x % kDies, k = blockIdx.x / kDies, more = all % kDies;
   const int first = die * (all / kDies) + (die < more ? die : more), mine = all / kDies + (die < more ? 1 : 0);
-  const int whole = TAIL ? 0 : mine / kDieUnits * kDieUnits, left = mine - whole;
-  const int parts = left * 4 <= kDieUnits ? 4 : TAIL || left * 2 <= kDieUnits ? 2 : 1;
+  const int whole = mine / kDieUnits * kDieUnits, left = mine - whole;
+  const int parts = left * 4 <= kDieUnits ? 4 : left * 2 <= kDieUnits ? 2 : 1;
   if (k >= whole + left * parts) return;
   const int id = first + (k < whole ? k : whole + (k - whole) / parts), part = k < whole ? 0 : (k - whole) % parts;
   // bands of kBand row tiles, walked down the rows first: what is in flight on a die shares its rows and its matrices
@@ -853,7 +887,7 @@ template <bool PAIRED, bool TAIL> __global__ __launch_bounds__(512, 2) void expe
   __syncthreads();
   if (k >= whole && parts == 4) return large_part<64, PAIRED, TAIL>(a, t, lds, slot_of, part * 64);
   if (k >= whole && parts == 2) return large_part<128, PAIRED, TAIL>(a, t, lds, slot_of, part * 128);
-  if constexpr (!TAIL) large_whole_tile<PAIRED>(a, t, lds, slot_of);
+  large_whole_tile<PAIRED, TAIL>(a, t, lds, slot_of);
 }
 
 constexpr int kMaxDevices = 64;
@@ -869,8 +903,8 @@ template <bool PAIRED, bool TAIL> int launch_expert_gemm_large(ExpertGemmArgs a,
     allowed[dev].store(true, std::memory_order_release);
   }
   a.col_tiles = PAIRED ? (a.F + 127) / 128 : (a.F + 255) / 256;
-  // (parts beyond the first of a tile: less than one for each of the 32 compute units of a die; TAIL: everything in two)
-  const unsigned per_die = (unsigned)((a.col_tiles * a.tiles + kDies - 1) / kDies * (TAIL ? 2 : 1) + kDieUnits);
+  // (parts beyond the first of a tile: less than one for each of the 32 compute units of a die)
+  const unsigned per_die = (unsigned)((a.col_tiles * a.tiles + kDies - 1) / kDies + kDieUnits);
   hipLaunchKernelGGL((expert_gemm_large_kernel<PAIRED, TAIL>), dim3(per_die * kDies), dim3(512), kLargeLds, s, a);
   return BASED_OK;
 }

@@ -625,3 +625,17 @@ def test_experts_of_few_large_tiles(dev, n, D, F, E, top):
     clear = torch.ones(n, dtype=torch.bool) if top == E else s[:, top - 1] - s[:, top] > 1e-5
     assert clear.sum() >= 0.9 * n
     close(got[clear], want[clear], 2 * TOL[BF16])
+
+
+@pytest.mark.parametrize("n,D,F,E,top", [(9000, 56, 520, 3, 1), (9000, 72, 520, 3, 1), (16000, 264, 264, 4, 2), (9600, 200, 712, 2, 1), (5000, 120, 1032, 4, 2)])
+def test_experts_in_whole_large_tiles_with_a_part_of_a_round(dev, n, D, F, E, top):
+    """Channels that are no whole rounds of 64, so many rows that tiles of 256 go whole: no whole round, one, an even and an odd number of them."""
+    from based_amd import ops
+
+    h, router, w1, w2, w = expert_case(n, D, F, E, top, BF16, seed=n)
+    want = O.expert_mlp(h.double(), w, "m", {"router": {"top": top}})
+    got = ops.experts(h.to(dev), router.to(dev), w1.to(dev), w2.to(dev), top).double().cpu()
+    s = O.sigmoid(h.double() @ router.double().T).sort(-1, descending=True).values
+    clear = s[:, top - 1] - s[:, top] > 1e-5
+    assert clear.sum() >= 0.98 * n
+    close(got[clear], want[clear], 2 * TOL[BF16])
