@@ -403,7 +403,7 @@ struct ExpertGemmArgs {
   __bf16* y;             // PAIRED: (tiles * rows, F); otherwise (slots, F) scattered by order
   const int32_t* order;
   const int32_t* tile_first;
-  const int32_t* tile_expert;  // or null (small tiles): from tile_first and counts
+  const int32_t* tile_expert;  // null: there is one expert (small tiles)
   const int32_t* counts;
   const float* scores;   // (slots), PAIRED
   long x_sr;
@@ -437,15 +437,11 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(const ExpertGemmArg
   const int tile = band * kBand + in_band % deep, f0 = in_band / deep * (PAIRED ? HALF : BN);
   if (tile >= a.tile_first[a.E]) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4, wm = wave % WM, wn = wave / WM;
-  int e, rows;
+  int e = 0, rows = a.counts[0] - tile * BM;  // (of one expert)
   if (a.tile_expert != nullptr) {
     const int what = a.tile_expert[tile];
     e = what & 255, rows = what >> 8;
   } else {
-    e = 0;
-    for (int x0 = 0; x0 < a.E; x0 += 64) e += __popcll(__ballot(x0 + lane < a.E && a.tile_first[x0 + lane < a.E ? x0 + lane + 1 : 0] <= tile));
-    e = __builtin_amdgcn_readfirstlane(e);
-    rows = a.counts[e] - (tile - a.tile_first[e]) * BM;
     rows = rows < BM ? rows : BM;
   }
   for (int i = tid; i < BM; i += 256) slot_of[i] = a.order[(long)tile * BM + (i < rows ? i : 0)];
@@ -1297,8 +1293,13 @@ extern "C" BASED_API int based_expert_grouped(const void* h, const void* router,
   const int64_t slots = n * top;
   int rows = expert_tile_rows(slots, E);
   if (rows == BASED_EXPERT_TILE_ROWS && !expert_large_products(slots, D, F)) {
-    rows = BASED_EXPERT_TILE_ROWS_SMALL;  // (rows of all tiles together are no more, 32 - 1 to an expert in place of 256 - 1; the tiles are)
-    tile_expert = nullptr;
+    // Rows of all tiles together are no more, less than 32 added to an expert in place of 256; the tiles are, and theirs goes behind the order.
+    const int64_t small = expert_tiles(slots, E, BASED_EXPERT_TILE_ROWS_SMALL), at = small * BASED_EXPERT_TILE_ROWS_SMALL;
+    const bool room = at + small <= expert_tiles(slots, E, BASED_EXPERT_TILE_ROWS) * BASED_EXPERT_TILE_ROWS;
+    if (room || E == 1) {
+      rows = BASED_EXPERT_TILE_ROWS_SMALL;
+      tile_expert = room ? order + at : nullptr;
+    }
   }
   const int64_t tiles = expert_tiles(slots, E, rows);
   BASED_REQUIRE(tiles * ((F > D ? F : D) / 64 + 1) < (1ll << 31), BASED_ERR_SHAPE, "expert_grouped: too many rows");
