@@ -1183,24 +1183,27 @@ template <bool PAIRED> __global__ __launch_bounds__(512) void expert_f32_kernel(
 constexpr int kRouteOneWg = 32;  // tokens that one workgroup routes, of up to 32 experts (16 of more): it makes the plan too
 
 // Tokens of one workgroup.  Many tokens of few experts: 32, their rows shared out over eight wavefronts (8192 tokens of 1024 channels, 8 experts:
-// 7.2 us without the sums of all workgroups' choices, 10 with them; 16 tokens 11.6, a wavefront to 16 tokens 16.9).
+// 7.2 us without the sums of all workgroups' choices, 10 with them; 16 tokens 11.6, a wavefront to 16 tokens 16.9).  So many that every
+// wavefront has enough of its own: 64, fewer workgroups whose choices are added up (calls of 16 experts of 16 features, 256 channels: 65,536 tokens
+// 113.9 -> 98.8 us, 16,384 49.8 and 49.1, 8192 39.0 and 42.0; 768 channels, 65,536 tokens 232.5 and 234.3, of 4 experts 104.3 and 100.2).
 static int route_group(const RouteArgs& a, bool vec) {
   const bool many = vec && a.n >= 4096;
-  return !many ? 16 : a.E <= 32 ? 32 : 64;
+  return !many ? 16 : a.E <= 32 && (a.n < 32768 || a.D > 768) ? 32 : 64;
 }
 
 template <int ET> void launch_route_tiles(const RouteArgs& a, hipStream_t s) {
   const size_t one = (size_t)16 * a.E * sizeof(float);
   constexpr int NW = ET <= 4 ? 8 : 4;
   const int group = route_group(a, true);
+  if (group == 64) {
+    hipLaunchKernelGGL((expert_route_kernel<__bf16, ET, 4, false, 1>), dim3((unsigned)((a.n + 63) / 64)), dim3(256), 4 * one, s, a);
+    return;
+  }
   if constexpr (ET <= 2) {
     if ((a.n > 16 && a.n <= kRouteOneWg) || group == 32) {
       hipLaunchKernelGGL((expert_route_kernel<__bf16, ET, NW, true, 2>), dim3((unsigned)((a.n + 31) / 32)), dim3(64 * NW), 2 * NW * one, s, a);
       return;
     }
-  } else if (group == 64) {
-    hipLaunchKernelGGL((expert_route_kernel<__bf16, ET, 4, false, 1>), dim3((unsigned)((a.n + 63) / 64)), dim3(256), 4 * one, s, a);
-    return;
   }
   hipLaunchKernelGGL((expert_route_kernel<__bf16, ET, NW, true, 1>), dim3((unsigned)((a.n + 15) / 16)), dim3(64 * NW), NW * one, s, a);
 }

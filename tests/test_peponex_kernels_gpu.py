@@ -555,7 +555,7 @@ def test_experts_in_large_tiles(dev, n, D, F, E, top):
     close(got[clear], want[clear], 2 * TOL[BF16])
 
 
-@pytest.mark.parametrize("n,E,top", [(33, 8, 1), (4095, 8, 2), (4096, 32, 2), (4097, 8, 2), (4100, 33, 2), (4223, 70, 4), (5000, 130, 3), (20000, 64, 2), (40000, 128, 1)])
+@pytest.mark.parametrize("n,E,top", [(33, 8, 1), (4095, 8, 2), (4096, 32, 2), (4097, 8, 2), (4100, 33, 2), (4223, 70, 4), (5000, 130, 3), (20000, 64, 2), (40000, 128, 1), (32767, 8, 2), (32768, 8, 2), (33000, 30, 1)])
 def test_places_of_the_choices(dev, n, E, top):
     """Every choice of a batch goes to the same expert as in batches of few tokens, whose places one workgroup plans: by the workgroups' counts (n E up
     to a million in 32 tokens), by sums of them (beyond, or no room), with groups that end inside the last workgroup's eight."""
