@@ -45,7 +45,7 @@ struct DecayScanArgs {
   int B, L, H, d, dv, dp;
   long q_sb, q_sl, k_sb, k_sl, v_sb, v_sl, o_sb, o_sl;
   int segs, seg_chunks;  // segments, and 64-token pieces in each
-  int silu, fresh, fold;
+  int silu, fresh;
 };
 
 template <int CTRL> __device__ __forceinline__ float row_moved(float x) {  // lanes without a source receive 0
@@ -146,7 +146,7 @@ template <int DT, int HALVES, bool CHANNEL> struct ScanLds {
   float total[4][CH], all[CH];                   // decay over each 16 tokens, and over the 64
 };
 
-template <int DT, int HALVES, bool CHANNEL, bool STATE_ONLY>
+template <int DT, int HALVES, bool CHANNEL, bool STATE_ONLY, bool FOLD>
 __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const DecayScanArgs a) {
   typedef ScanLds<DT, HALVES, CHANNEL> Lds;
   constexpr int RS = Lds::RS, TS = Lds::TS, E = DT * 8, DA = DT * HALVES;
@@ -177,9 +177,9 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
   {
     const long seg_row = (col_in ? dv0 + l16 : 0), seg_step = (long)a.dv * a.dp;
     const float* segs = a.seg + (bh * a.segs * a.dv + seg_row) * a.dp;
-    // folded: what the segments in front have added is put together here, the state that enters the call from the last one's place, where
-    // the state pass has left it (the last segment replaces it)
-    const bool fold = !STATE_ONLY && a.segs > 1 && a.fold;
+    // FOLD: what the segments in front have added is put together here, the state that enters the call from the last one's place, where
+    // the state pass has left it (the last segment replaces it).  Kernels of their own: the others have registers for what they do.
+    constexpr bool fold = FOLD && !STATE_ONLY;
     const float* from = a.segs > 1 ? segs + (fold ? a.segs - 1 : sg) * seg_step : st;
     const bool zero = STATE_ONLY || ((a.segs == 1 || fold) && a.fresh);
 #pragma unroll
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
       if (!zero && col_in && ch < a.d) S[ct] = *reinterpret_cast<const f32x4*>(from + ch);
     }
     if constexpr (STATE_ONLY) {
-      if (a.fold && !a.fresh && sg == 0 && col_in) {
+      if (FOLD && !a.fresh && sg == 0 && col_in) {
         float* keep = a.seg + ((bh * a.segs + a.segs - 1) * a.dv + seg_row) * a.dp;
 #pragma unroll
         for (int ct = 0; ct < 2 * DA; ++ct) {
@@ -197,10 +197,10 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
           if (ch < a.d) *reinterpret_cast<f32x4*>(keep + ch) = *reinterpret_cast<const f32x4*>(st + ch);
         }
       }
-    } else if (fold) {
+    } else if constexpr (FOLD) {
       float seg_decay = 0.f;  // (all in front of the last are of one length)
       if constexpr (!CHANNEL) seg_decay = powers.of_state(a.seg_chunks * kScanTokens);
-      constexpr int U = HALVES == 1 ? 4 : 2;  // segments asked for together
+      constexpr int U = 4;  // segments asked for together
       for (int s0 = 0; s0 < sg; s0 += U) {
         f32x4 add[U][2 * DA], l[U][2 * DA];
 #pragma unroll
@@ -1016,14 +1016,14 @@ void launch_decay_join(const DecayScanArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(decay_join_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, a);
 }
 
-template <int DT, int HALVES, bool CHANNEL> int launch_decay_mfma(const DecayScanArgs& a, hipStream_t s) {
+template <int DT, int HALVES, bool CHANNEL, bool FOLD> int launch_decay_mfma(const DecayScanArgs& a, hipStream_t s) {
   const size_t bytes = sizeof(ScanLds<DT, HALVES, CHANNEL>);
   if (bytes > 64 * 1024) {
     static const hipError_t once = [&] {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(decay_scan_mfma_kernel<DT, HALVES, CHANNEL, false>),
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(decay_scan_mfma_kernel<DT, HALVES, CHANNEL, false, FOLD>),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
       if (e != hipSuccess) return e;
-      return hipFuncSetAttribute(reinterpret_cast<const void*>(decay_scan_mfma_kernel<DT, HALVES, CHANNEL, true>),
+      return hipFuncSetAttribute(reinterpret_cast<const void*>(decay_scan_mfma_kernel<DT, HALVES, CHANNEL, true, FOLD>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     }();
     BASED_REQUIRE(once == hipSuccess, BASED_ERR_LAUNCH, "decay_scan: %zu bytes of LDS refused: %s", bytes, hipGetErrorString(once));
@@ -1033,17 +1033,17 @@ template <int DT, int HALVES, bool CHANNEL> int launch_decay_mfma(const DecaySca
   if (a.segs > 1) {
     dim3 all_but_last = grid;
     all_but_last.z -= 1;
-    hipLaunchKernelGGL((decay_scan_mfma_kernel<DT, HALVES, CHANNEL, true>), all_but_last, dim3(256 * HALVES), bytes, s, a);
-    if (!a.fold) launch_decay_join(a, s);
+    hipLaunchKernelGGL((decay_scan_mfma_kernel<DT, HALVES, CHANNEL, true, FOLD>), all_but_last, dim3(256 * HALVES), bytes, s, a);
+    if (!FOLD) launch_decay_join(a, s);
   }
-  hipLaunchKernelGGL((decay_scan_mfma_kernel<DT, HALVES, CHANNEL, false>), grid, dim3(256 * HALVES), bytes, s, a);
+  hipLaunchKernelGGL((decay_scan_mfma_kernel<DT, HALVES, CHANNEL, false, FOLD>), grid, dim3(256 * HALVES), bytes, s, a);
   return BASED_OK;
 }
 
-template <bool CHANNEL> int launch_decay_scan_mfma(const DecayScanArgs& a, hipStream_t s) {
-  if (a.d <= 32) return launch_decay_mfma<1, 1, CHANNEL>(a, s);
-  if (a.d <= 64) return launch_decay_mfma<2, 1, CHANNEL>(a, s);
-  return launch_decay_mfma<2, 2, CHANNEL>(a, s);
+template <bool CHANNEL> int launch_decay_scan_mfma(const DecayScanArgs& a, bool fold, hipStream_t s) {
+  if (a.d <= 32) return fold ? launch_decay_mfma<1, 1, CHANNEL, true>(a, s) : launch_decay_mfma<1, 1, CHANNEL, false>(a, s);
+  if (a.d <= 64) return fold ? launch_decay_mfma<2, 1, CHANNEL, true>(a, s) : launch_decay_mfma<2, 1, CHANNEL, false>(a, s);
+  return launch_decay_mfma<2, 2, CHANNEL, false>(a, s);
 }
 
 template <typename T, int CPT, bool CHANNEL, int TOKENS> void launch_decay_any_tile(const DecayScanArgs& a, hipStream_t s) {
@@ -1191,10 +1191,10 @@ extern "C" BASED_API int based_decay_scan(const void* q, const void* k, const vo
     a.segs = (int)(((L + kScanTokens - 1) / kScanTokens + a.seg_chunks - 1) / a.seg_chunks);
     a.seg = work;
     a.seg_lw = work + B * H * a.segs * DV * state_row;
-    a.fold = vec && D <= 64 && a.segs <= kFoldSegments;
   }
+  const bool fold = vec && D <= 64 && a.segs > 1 && a.segs <= kFoldSegments;
   if (vec) {
-    const int rc = channel_log2 != nullptr ? launch_decay_scan_mfma<true>(a, s) : launch_decay_scan_mfma<false>(a, s);
+    const int rc = channel_log2 != nullptr ? launch_decay_scan_mfma<true>(a, fold, s) : launch_decay_scan_mfma<false>(a, fold, s);
     if (rc != BASED_OK) return rc;
   } else if (io_dtype == BASED_BF16) {
     channel_log2 != nullptr ? launch_decay_scan_any<__bf16, true>(a, s) : launch_decay_scan_any<__bf16, false>(a, s);
