@@ -302,8 +302,10 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
     // The weights inside the 16 tokens.  BACK: token t with the one 4 g + quad back in [g], zero where that is none of the 16, four sums
     // added up over the channels' lanes at once without LDS (two exchanges through LDS a sum, 16 heads of 64, 12 x 960 tokens: 121.2 us ->
     // 117.1; 12 heads, 1 x 1000: 50.2 -> 47.8); otherwise column t, rows s = 4 quad + i (128 channels: 104.9 us, 107.5 with BACK, which spills
-    // more).
-    constexpr bool BACK = CHANNEL && HALVES == 1;
+    // more; up to 32 channels where there are no segments to put together, so more workgroups than are on the GPU at once: 147 registers and three
+    // wavefronts on a SIMD, with BACK 174 and two.  24 x 512 tokens, 32 heads of 32: 70 us, 81 with BACK; 16 x 1024, 48 heads of 16: 114, 154; in
+    // segments 1 x 1000, 12 heads of 32: 30.1, 28.9).
+    constexpr bool BACK = CHANNEL && HALVES == 1 && (DT == 2 || FOLD);
     f32x4 diag = {0.f, 0.f, 0.f, 0.f};
     if constexpr (CHANNEL && !STATE_ONLY) {
       const int rel = l16 - quad * 4;  // row i is j tokens back where rel = j + i
@@ -531,7 +533,7 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
           split2(P[j][2 * i], P[j][2 * i + 1], x, y);
           hi[i] = x, lo[i] = y;
         }
-        if (CHANNEL && HALVES == 1 && j == blk) {  // as diag has them
+        if (BACK && j == blk) {  // as diag has them
 #pragma unroll
           for (int i = 0; i < 2; ++i) {
             const int s0 = t * TS + j * 16 + ((l16 - 8 * i - quad) & 15), s1 = t * TS + j * 16 + ((l16 - 8 * i - 4 - quad) & 15);
