@@ -1107,9 +1107,11 @@ template <typename T, bool CHANNEL> void launch_decay_step(const DecayStepArgs& 
 }
 
 // Segments up to which those of the scan put the ones in front of them together themselves, heads of up to 64 channels: a launch less, and memory's
-// answer to four segments at a time in front of the scan.  4 x 2048 tokens, 16 heads of 64 (8 segments): 74.6 us with decay_join_kernel,
-// 72.2; 12 x 960 (3) 124.2, 121.2; 1 x 2000, 12 heads (8) 53.6, 53.5; 1 x 4096 (16) 57.6, 60.1; 1 x 2000, 8 heads of 128 87.4, 96.0.
-constexpr int kFoldSegments = 8;
+// answer to four segments at a time in front of the scan, with channel decays also the segments' decays.  us with decay_join_kernel and without, 16 heads of 64,
+// channel decays: 4 x 2048 tokens (8 segments) 74.6, 72.9; 12 x 960 (3) 118.6, 110.7; 1 x 2304 (9) 53.0, 50.7; 1 x 2560 (10) 53.6, 52.3; 1 x 2816 (11)
+// 54.1, 55.0; 1 x 4096 (16) 57.3, 59.9.  Head decays: 1 x 2560 32.3, 28.7; 1 x 3584 (14) 34.5, 32.5; 1 x 4096 35.3, 34.0.  Heads of 128, channel
+// decays, 1 x 2000, 8 heads: 87.4, 96.0.
+constexpr int kFoldSegmentsChannel = 10, kFoldSegmentsHead = 16;
 
 // Segments of a scan: enough workgroups to give every SIMD two wavefronts, none shorter than four pieces of 64 tokens.
 static int decay_segments(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
@@ -1194,7 +1196,7 @@ extern "C" BASED_API int based_decay_scan(const void* q, const void* k, const vo
     a.seg = work;
     a.seg_lw = work + B * H * a.segs * DV * state_row;
   }
-  const bool fold = vec && D <= 64 && a.segs > 1 && a.segs <= kFoldSegments;
+  const bool fold = vec && D <= 64 && a.segs > 1 && a.segs <= (channel_log2 != nullptr ? kFoldSegmentsChannel : kFoldSegmentsHead);
   if (vec) {
     const int rc = channel_log2 != nullptr ? launch_decay_scan_mfma<true>(a, fold, s) : launch_decay_scan_mfma<false>(a, fold, s);
     if (rc != BASED_OK) return rc;

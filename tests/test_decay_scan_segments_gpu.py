@@ -205,20 +205,22 @@ def test_few_tokens(dev, L, d, dtype, channel):
 
 @pytest.mark.parametrize("channel", [True, False])
 @pytest.mark.parametrize("fresh", [True, False])
-@pytest.mark.parametrize("L,d,dv", [(512, 64, 64), (577, 20, 36), (1100, 64, 100), (2048, 60, 64), (2304, 64, 64), (2500, 36, 16), (700, 72, 64)])
+@pytest.mark.parametrize("L,d,dv", [(512, 64, 64), (577, 20, 36), (1100, 64, 100), (2048, 60, 64), (2304, 64, 64), (2500, 36, 16), (700, 72, 64),
+                                    (2817, 20, 16), (4100, 36, 16), (4353, 64, 16)])
 def test_segments_of_the_matrix_form(dev, L, d, dv, fresh, channel):
-    """Two segments to ten of bf16 portions, put together by those behind them or by a launch of its own, against one chain of portions that
-    are too short for segments."""
+    """Two segments to seventeen of bf16 portions, put together by those behind them (up to ten with channel decays, sixteen with head decays) or by
+    a launch of its own, against 64-bit sums token by token and against one chain of portions that are too short for segments."""
     from based_amd import ops
 
-    B, H = 1, 2
+    B, H, decay = 1, 2, [0.9995, 0.9]
     g = torch.Generator().manual_seed(L + d)
     q, k, v = (torch.randn(B, L, H * n, generator=g).bfloat16().to(dev) for n in (d, d, dv))
     dp = (d + 3) // 4 * 4
     start = torch.zeros(B, H, dv, dp) if fresh else torch.randn(B, H, dv, dp, generator=g)
     state = torch.full((B, H, dv, dp), float("nan"), device=dev) if fresh else start.to(dev)
     lw = (-torch.exp(0.5 * torch.randn(B, L, H, d, generator=g) + torch.linspace(-7, 1, d)) / math.log(2)).flatten(2).to(dev)
-    kw = dict(head_decay=ops.head_decays([0.9995, 0.9], dev)) if not channel else dict(bonus=torch.randn(H, d, generator=g).bfloat16().to(dev))
+    u = torch.randn(H, d, generator=g).bfloat16().to(dev)
+    kw = dict(head_decay=ops.head_decays(decay, dev)) if not channel else dict(bonus=u)
     part = lambda s: dict(channel_log2=lw[:, s].contiguous()) if channel else {}  # noqa: E731
     whole = ops.decay_scan(q, k, v, state, H, fresh=fresh, **kw, **part(slice(0, L)))
     chain, pieces = start.to(dev), []
@@ -226,9 +228,21 @@ def test_segments_of_the_matrix_form(dev, L, d, dv, fresh, channel):
         s = slice(at, min(at + 192, L))
         pieces.append(ops.decay_scan(q[:, s], k[:, s], v[:, s], chain, H, fresh=False, **kw, **part(s)))
     rel = lambda a, b: ((a.double() - b.double()).norm() / b.double().norm()).item()  # noqa: E731
-    # outputs: one rounding to bf16 that falls another way, 2^-8 of few values; states: 32-bit sums in another order over up to 2500 tokens
+    # outputs: one rounding to bf16 that falls another way, 2^-8 of few values; states: 32-bit sums in another order over up to 4400 tokens
     assert rel(whole, torch.cat(pieces, 1)) < 1e-3
     assert rel(state[..., :d], chain[..., :d]) < 1e-5
+    S, ref = start[..., :d].double().transpose(2, 3).to(dev), torch.empty(B, L, H, dv, dtype=torch.float64, device=dev)
+    w = 2.0 ** lw.double().view(B, L, H, d, 1) if channel else torch.tensor(decay, device=dev).double().view(1, 1, H, 1, 1).expand(B, L, H, 1, 1)
+    qd, kd, vd = (x.double().view(B, L, H, -1) for x in (q, k, v))
+    for t in range(L):
+        kv = kd[:, t, :, :, None] * vd[:, t, :, None]
+        if channel:
+            ref[:, t] = ((S + u.double()[..., None] * kv) * qd[:, t, ..., None]).sum(2)
+        S = w[:, t] * S + kv
+        if not channel:
+            ref[:, t] = (S * qd[:, t, ..., None]).sum(2)
+    # bf16 outputs: half of 2^-8 at most, 2^-9 / 3^0.5 = 1.1e-3 evenly spread; a state's terms keep 16 bits each, 2^-17 / 3^0.5 = 4.4e-6
+    assert rel(whole.view(B, L, H, dv), ref) < 3e-3 and rel(state[..., :d], S.transpose(2, 3)) < 2e-5
 
 
 def _head_decays_in_64_bits(q, k, v, w, state):
