@@ -6,12 +6,17 @@ the first use raises, so a GPU run can never silently go through something else.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
+import sysconfig
 import threading
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libbased_hip.so")  # the in-tree build of every kernel
-BINDING_PATH = os.path.join(_HERE, "_binding.so")  # its entry points as Python callables, cheaper to call than through ctypes
+# Its entry points as Python callables, cheaper to call than through ctypes.
+BINDING_PATH = os.path.join(_HERE, "_binding" + sysconfig.get_config_var("EXT_SUFFIX"))
 # Builds of some of the sources (based_amd.build.build_part) lie beside it; `use_part` selects one
 # where the whole library has not been built.
 _part_path = None
@@ -34,6 +39,7 @@ class StreamExtras(C.Structure):
 # name -> (restype, argtypes); must list every symbol declared in include/based_hip.h
 SIGNATURES = {
     "based_hip_version": (C.c_int, []),
+    "based_hip_interface": (_I64, []),
     "based_hip_last_error": (C.c_char_p, []),
     "based_linear_attn_step": (
         C.c_int,
@@ -199,13 +205,29 @@ def _absent(name):
     return refuse
 
 
+def _binding(path: str, number: int):
+    """bind(name, address, ctypes entry) -> callable of the binding at `path`, or None (with a warning where one is there and does not fit): built of
+    another header it would read arguments that the library does not take."""
+    if not os.path.exists(path):
+        return None
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("_binding", path)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_binding", loader))
+        loader.exec_module(module)
+    except ImportError as e:
+        warnings.warn(f"{path} cannot be loaded, calls go through ctypes: {e}")
+        return None
+    if module.interface() != number or number == 0:
+        warnings.warn(f"{path} was built of another include/based_hip.h than the library, calls go through ctypes: python -m based_amd.build")
+        return None
+    return module.bind
+
+
 class _Entries:
     """The typed entry points of a loaded library."""
 
     def __init__(self, handle, partial: bool):
-        bind = lambda name, fn: fn  # noqa: E731
-        if not partial and os.path.exists(BINDING_PATH):  # (built with the library, of the same header)
-            from ._binding import bind
+        bind = None
         for name, (res, args) in SIGNATURES.items():
             if partial and not hasattr(handle, name):
                 setattr(self, name, _absent(name))
@@ -213,7 +235,13 @@ class _Entries:
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
-            setattr(self, name, bind(name, fn))
+            setattr(self, name, fn)
+        if not partial:
+            bind = _binding(BINDING_PATH, self.based_hip_interface())
+        if bind is not None:
+            for name in SIGNATURES:
+                fn = getattr(self, name)
+                setattr(self, name, bind(name, C.cast(fn, C.c_void_p).value, fn))
 
 
 def lib():

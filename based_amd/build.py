@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import concurrent.futures as cf
 import glob
+import hashlib
 import json
 import os
 import re
@@ -19,7 +20,7 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 OBJDIR = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libbased_hip.so")
-BINDING = os.path.join(HERE, "_binding.so")
+BINDING = os.path.join(HERE, "_binding" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 FLAGS = [
@@ -45,10 +46,16 @@ _REMARK = re.compile(r"remark:\s+(Function Name|VGPRs|AGPRs|VGPRs Spill|SGPRs Sp
 _SNIPPET = re.compile(r"^\s*\d*\s*\|")   # the source lines clang shows under a remark
 
 
+def interface() -> int:
+    """The number of include/based_hip.h that everything built of it carries (never 0)."""
+    with open(os.path.join(INCLUDE, "based_hip.h"), "rb") as f:
+        return int.from_bytes(hashlib.sha256(f.read()).digest()[:8], "little") >> 1 | 1
+
+
 def _compile(src: str):
     """Compiles one source; returns (object file, {kernel: resource figures the compiler reports})."""
     obj = os.path.join(OBJDIR, os.path.basename(src).rsplit(".", 1)[0] + ".o")
-    cmd = [HIPCC, *FLAGS, "-Rpass-analysis=kernel-resource-usage", "-c", src, "-o", obj]
+    cmd = [HIPCC, *FLAGS, f"-DBASED_HIP_INTERFACE={interface()}LL", "-Rpass-analysis=kernel-resource-usage", "-c", src, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stdout}\n{r.stderr}")
@@ -86,15 +93,24 @@ def _link(objs, out: str) -> None:
     os.replace(tmp, out)
 
 
-def _build_binding() -> None:
-    """csrc/binding.cpp, the entry points of LIB as Python callables."""
-    tmp = f"{BINDING}.{os.getpid()}.tmp"
-    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-Wall", "-I", INCLUDE,
-           "-I", sysconfig.get_paths()["include"], os.path.join(CSRC, "binding.cpp"), "-L", HERE, "-l:libbased_hip.so", "-Wl,-rpath,$ORIGIN", "-o", tmp]
-    r = subprocess.run(cmd, capture_output=True, text=True)
+def _build_binding(out: str = BINDING, number: int | None = None, compiler: str = "g++") -> bool:
+    """csrc/binding.cpp, the entry points of LIB as Python callables.  Without a compiler or Python's headers there is none, and calls go
+    through ctypes."""
+    if os.path.exists(out):
+        os.remove(out)
+    tmp = f"{out}.{os.getpid()}.tmp"
+    cmd = [compiler, "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-Wall", "-I", INCLUDE, "-I", sysconfig.get_paths()["include"],
+           f"-DBASED_HIP_INTERFACE={interface() if number is None else number}LL", os.path.join(CSRC, "binding.cpp"), "-L", HERE, "-l:libbased_hip.so",
+           "-Wl,-rpath,$ORIGIN", "-o", tmp]
+    try:
+        r = subprocess.run(cmd, capture_output=True, text=True)
+    except OSError as e:
+        r = subprocess.CompletedProcess(cmd, 1, "", str(e))
     if r.returncode != 0:
-        raise RuntimeError(f"binding build failed:\n{r.stdout}\n{r.stderr}")
-    os.replace(tmp, BINDING)
+        sys.stderr.write(f"note: no binding was built, calls go through ctypes:\n{r.stdout}{r.stderr}\n")
+        return False
+    os.replace(tmp, out)
+    return True
 
 
 def build_part(part: str) -> str:
@@ -128,6 +144,8 @@ def build(verbose: bool = False) -> str:
         for name, u in kernels.items():
             if u.get("VGPRs Spill", 0) > 0:
                 sys.stderr.write(f"note: {src}: {name} spills {u['VGPRs Spill']} vector registers\n")
+    if os.path.exists(BINDING):  # (one of a library before must not lie beside this one)
+        os.remove(BINDING)
     _link(objs, LIB)
     _build_binding()
     if verbose:

@@ -54,8 +54,14 @@ template <typename R, typename... A, R (*F)(A...)> struct Entry<F> {
   }
 };
 
-#define BASED_ENTRY(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&Entry<&name>::call)), METH_FASTCALL, nullptr}
-PyMethodDef kEntries[] = {
+struct Listed {
+  PyMethodDef def;
+  void (*entry)();
+};
+#define BASED_ENTRY(name)                                                                                                  \
+  {{#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&Entry<&name>::call)), METH_FASTCALL, nullptr}, \
+   reinterpret_cast<void (*)()>(&name)}
+Listed kEntries[] = {
     BASED_ENTRY(based_linear_attn_step),
     BASED_ENTRY(based_linear_attn_step_deferred),
     BASED_ENTRY(based_linear_attn_prefill),
@@ -107,18 +113,29 @@ PyMethodDef kEntries[] = {
     BASED_ENTRY(based_expert_rows),
 };
 
-// bind(name, entry): the callable for an entry point that is listed, the ctypes entry itself for others.
+#ifndef BASED_HIP_INTERFACE
+#define BASED_HIP_INTERFACE 0
+#endif
+
+// bind(name, address, entry): the callable for an entry point that is listed, the ctypes entry itself for others and for those of another library
+// than the one that this is linked to.
 PyObject* bind(PyObject*, PyObject* args) {
   const char* name;
+  unsigned long long address;
   PyObject* general;
-  if (!PyArg_ParseTuple(args, "sO", &name, &general)) return nullptr;
-  for (PyMethodDef& e : kEntries)
-    if (!std::strcmp(e.ml_name, name)) return PyCFunction_New(&e, general);
+  if (!PyArg_ParseTuple(args, "sKO", &name, &address, &general)) return nullptr;
+  for (Listed& e : kEntries)
+    if (!std::strcmp(e.def.ml_name, name) && reinterpret_cast<uintptr_t>(e.entry) == address) return PyCFunction_New(&e.def, general);
   Py_INCREF(general);
   return general;
 }
 
-PyMethodDef kModule[] = {{"bind", bind, METH_VARARGS, "bind(name, ctypes entry) -> callable"}, {nullptr, nullptr, 0, nullptr}};
+// interface(): the number of the header that this was built of
+PyObject* interface(PyObject*, PyObject*) { return PyLong_FromLongLong(BASED_HIP_INTERFACE); }
+
+PyMethodDef kModule[] = {{"bind", bind, METH_VARARGS, "bind(name, address, ctypes entry) -> callable"},
+                         {"interface", interface, METH_NOARGS, "interface() -> int"},
+                         {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kDef = {PyModuleDef_HEAD_INIT, "_binding", nullptr, -1, kModule, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -19,4 +19,9 @@ void set_error(const char* fmt, ...) {
 
 extern "C" BASED_API int based_hip_version(void) { return 1; }
 
+#ifndef BASED_HIP_INTERFACE
+#define BASED_HIP_INTERFACE 0
+#endif
+extern "C" BASED_API int64_t based_hip_interface(void) { return BASED_HIP_INTERFACE; }
+
 extern "C" BASED_API const char* based_hip_last_error(void) { return based::g_last_error; }

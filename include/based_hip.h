@@ -43,6 +43,8 @@ enum { BASED_BF16 = 0, BASED_F32 = 1 };
 #define BASED_EXPANDED_DIM 273
 
 BASED_API int based_hip_version(void);
+/* A number of this header's text, the same in all that was built of it with based_amd/build.py (0: built otherwise). */
+BASED_API int64_t based_hip_interface(void);
 BASED_API const char* based_hip_last_error(void);
 
 /*

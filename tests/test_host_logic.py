@@ -1,5 +1,7 @@
 """Host-side logic that needs no GPU: module construction and parameter names, cache
 shapes, config routing, sampling, and loud failure when tensors are not on a HIP device."""
+import os
+
 import pytest
 import torch
 
@@ -217,23 +219,90 @@ def test_gated_mlp_variants_construct_like_the_reference():
         GatedMlp(64, activation="gelu_new")
 
 
+# Entries that stay with ctypes: asked for once a plan or a process, or with arguments by reference.
+CTYPES_ENTRIES = {"based_hip_version", "based_hip_interface", "based_hip_last_error", "based_linear_attn_flush_deferred", "based_linear_attn_prefill_plan",
+                  "based_linear_attn_prefill_f32_plan", "based_linear_attn_prefill_split_static", "based_swa_prefill_anydim", "based_swa_step_anydim",
+                  "based_gated_delta_scan_work", "based_decay_scan_work", "based_decode_linear_extras"}
+
+
+def test_binding_lists_every_other_entry():
+    import types
+
+    from based_amd import _lib
+
+    lib = _lib.lib()
+    assert os.path.exists(_lib.BINDING_PATH), "no binding was built: calls go through ctypes"
+    native = {name for name in _lib.SIGNATURES if isinstance(getattr(lib, name), types.BuiltinFunctionType)}
+    assert native == set(_lib.SIGNATURES) - CTYPES_ENTRIES
+
+
 def test_binding_reads_what_ctypes_reads():
-    """The callables of csrc/binding.cpp against the ctypes entries they stand for: numbers, None, truth values, and what goes to ctypes after all."""
+    """The callables of csrc/binding.cpp against the ctypes entries they stand for: numbers, None, truth values, and what goes to ctypes after all.  Every
+    listed entry refuses a call of nothing but zeros (without a kernel's launch), with the same code and message from both sides."""
     import ctypes
+    import types
 
     from based_amd import _lib
 
     lib, handle = _lib.lib(), ctypes.CDLL(_lib.LIB_PATH)
-    for name, calls in {"based_expert_tiles": [(100, 8, 2), (0, 8, 2), (True, 1, 1), (ctypes.c_int64(300), 4, 1)],
-                        "based_decay_scan_work_of": [(0, 4, 2048, 16, 64, 64, 64, 0), (8, 1, 300, 12, 64, 64, 64, 1), (1 << 40, 1, 300, 12, 64, 64, 64, 1)],
-                        "based_swiglu": [(None, None, 1, 8, 16, 8, 0, None), (None, None, 1, 8, 16, 8, 0, 0)]}.items():
-        fn = getattr(handle, name)
+    last = handle.based_hip_last_error
+    last.restype = ctypes.c_char_p
+
+    def same(name, args):
+        ours, fn = getattr(lib, name), getattr(handle, name)
+        assert isinstance(ours, types.BuiltinFunctionType), name
         fn.restype, fn.argtypes = _lib.SIGNATURES[name]
+        results = []
+        for f in (ours, fn):
+            code = f(*args)
+            results.append((code, last() if isinstance(code, int) and code else b""))
+        assert results[0] == results[1], (name, args, results)
+        return results[0]
+
+    for name, calls in {"based_expert_tiles": [(100, 8, 2), (0, 8, 2), (True, 1, 1), (ctypes.c_int64(300), 4, 1), (-1, 8, 2)],
+                        "based_decay_scan_work_of": [(0, 4, 2048, 16, 64, 64, 64, 0), (8, 1, 300, 12, 64, 64, 64, 1), (1 << 40, 1, 300, 12, 64, 64, 64, 1),
+                                                     (-8, 1, 300, 12, 64, 64, 64, 1), (0, 4, 2048, 16, 64, 64, 64, 1 << 32),  # (an int cut to 32 bits)
+                                                     (0, 4, 2048, 16, 64, 64, 64, -(1 << 31))],
+                        "based_swiglu": [(None, None, 1, 8, 16, 8, 0, None), (None, None, 1, 8, 16, 8, 0, 0), (-1, None, 1, 8, 16, 8, 0, None),
+                                         ((1 << 63) + 8, None, 1, 8, 16, 8, 0, None), (None, None, 1, 8, 16, 8, False, None)],
+                        "based_softcap": [(64, 8, 0.0, 0, None), (64, 8, -1.0, 0, None), (64, 8, 0, 0, None), (64, 8, float("nan"), 0, None), (None, 8, 1.0, 0, None)]}.items():
         for args in calls:
-            assert getattr(lib, name)(*args) == fn(*args), (name, args)
+            same(name, args)
+    zero = {ctypes.c_void_p: None, ctypes.c_int64: 0, ctypes.c_int: 0, ctypes.c_float: 0.0}
+    for name in sorted(set(_lib.SIGNATURES) - CTYPES_ENTRIES):
+        res, types_ = _lib.SIGNATURES[name]
+        assert all(t in zero for t in types_), name
+        same(name, [zero[t] for t in types_])
     for bad in ((1, 2), (1, 2, "3"), (1.5, 2, 3)):
         with pytest.raises((TypeError, ctypes.ArgumentError)):
             lib.based_expert_tiles(*bad)
+
+
+def test_binding_that_does_not_fit_is_not_used(tmp_path, capsys):
+    """A binding of another header, one that does not load, one of another library, and none: calls go through ctypes."""
+    import ctypes
+
+    from based_amd import _lib, build
+
+    number = _lib.lib().based_hip_interface()
+    assert number == build.interface() != 0
+    suffix = os.path.basename(_lib.BINDING_PATH)[len("_binding"):]
+    assert _lib._binding(str(tmp_path / f"_binding{suffix}"), number) is None
+    torn = tmp_path / f"torn{suffix}"
+    torn.write_bytes(b"no library")
+    with pytest.warns(UserWarning, match="cannot be loaded"):
+        assert _lib._binding(str(torn), number) is None
+    with pytest.warns(UserWarning, match="another include/based_hip.h"):
+        assert _lib._binding(_lib.BINDING_PATH, number + 2) is None
+    with pytest.warns(UserWarning, match="another include/based_hip.h"):
+        assert _lib._binding(_lib.BINDING_PATH, 0) is None
+    entry = ctypes.CDLL(_lib.LIB_PATH).based_expert_tiles
+    assert _lib._binding(_lib.BINDING_PATH, number)("based_expert_tiles", 64, entry) is entry
+    # a build without a compiler leaves none behind, not even the one of a build before
+    out = tmp_path / f"old{suffix}"
+    out.write_bytes(b"of a build before")
+    assert not build._build_binding(str(out), compiler="/nonexistent/g++") and not out.exists()
+    assert "ctypes" in capsys.readouterr().err
 
 
 def test_remembered_checks_are_bounded():
