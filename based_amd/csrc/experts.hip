@@ -411,6 +411,7 @@ struct ExpertGemmArgs {
 };
 
 constexpr int kGemmK = 64;
+constexpr int kSmallWeights = 128;
 constexpr int kBand = 8;
 
 // Workgroups are dealt to the eight dies in turn: those of one die take neighbouring tiles, which share rows and matrices.
@@ -419,15 +420,14 @@ __device__ __forceinline__ int tile_of_block(int i, int n) {
   return die * per + (die < more ? die : more) + k;
 }
 
-// BM rows and BN rows of the weights (PAIRED: half of them up, half gate) per workgroup; AHEAD rounds of 64 channels on their
-// way from memory.  They are asked for in front of the products, which the compiler would put between them, with 32-bit offsets.
-template <int BM, int BN, int AHEAD, bool PAIRED>
-__global__ __launch_bounds__(256, 2) void expert_gemm_kernel(const ExpertGemmArgs a) {
+// 32 rows and 128 rows of the weights (PAIRED: half of them up, half gate) per workgroup, a wavefront 16 rows of each half of the weights; four rounds of
+// 64 channels on their way from memory.  They are asked for in front of the products, which the compiler would put between them, with
+// 32-bit offsets.
+template <bool PAIRED> __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(const ExpertGemmArgs a) {
   // rows of 128 bytes lie side by side, the eight 16-byte pieces of a row turned by half its number: neither the rows that
   // eight lanes write nor the sixteen that a tile reads meet a bank twice
-  constexpr int KS = kGemmK;
+  constexpr int BM = BASED_EXPERT_TILE_ROWS_SMALL, BN = kSmallWeights, AHEAD = 4, KS = kGemmK, MT = BM / 16, HALF = BN / 2;
   auto place = [](int r, int p) { return r * KS + ((p ^ (r >> 1)) & 7) * 8; };
-  constexpr int WM = BM >= 128 ? 2 : 1, WN = 4 / WM, MT = BM / 16 / WM, NT = BN / 32 / WN, HALF = BN / 2;
   constexpr int AP = BM / 32, BP = BN / 32;  // 16-byte pieces per thread
   __shared__ __attribute__((aligned(16))) __bf16 xs[BM * KS], ws[BN * KS];
   __shared__ int slot_of[BM];
@@ -436,7 +436,7 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(const ExpertGemmArg
   const int deep = a.tiles - band * kBand < kBand ? a.tiles - band * kBand : kBand;
   const int tile = band * kBand + in_band % deep, f0 = in_band / deep * (PAIRED ? HALF : BN);
   if (tile >= a.tile_first[a.E]) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4, wm = wave % WM, wn = wave / WM;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4;
   int e = 0, rows = a.counts[0] - tile * BM;  // (of one expert)
   if (a.tile_expert != nullptr) {
     const int what = a.tile_expert[tile];
@@ -472,13 +472,11 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(const ExpertGemmArg
     for (int i = 0; i < BP; ++i) w[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(wbase) + (wrow[i] + (uint32_t)c * 2u));
     __builtin_amdgcn_sched_barrier(0);  // (the products would otherwise be put in front of most of them)
   };
-  f32x4 acc[2][NT][MT];
+  f32x4 acc[2][MT];
 #pragma unroll
   for (int p = 0; p < 2; ++p)
 #pragma unroll
-    for (int i = 0; i < NT; ++i)
-#pragma unroll
-      for (int j = 0; j < MT; ++j) acc[p][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < MT; ++j) acc[p][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   auto stage = [&](int k0, const u32x4 (&x)[AP], const u32x4 (&w)[BP]) {
     const bool in = k0 + piece < a.K;
 #pragma unroll
@@ -491,15 +489,13 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(const ExpertGemmArg
     for (int kk = 0; kk < kGemmK; kk += 32) {
       bf16x8 xf[MT];
 #pragma unroll
-      for (int j = 0; j < MT; ++j) xf[j] = *reinterpret_cast<const bf16x8*>(&xs[place((wm * MT + j) * 16 + l16, kk / 8 + quad)]);
+      for (int j = 0; j < MT; ++j) xf[j] = *reinterpret_cast<const bf16x8*>(&xs[place(j * 16 + l16, kk / 8 + quad)]);
 #pragma unroll
-      for (int p = 0; p < 2; ++p)
+      for (int p = 0; p < 2; ++p) {
+        const bf16x8 wf = *reinterpret_cast<const bf16x8*>(&ws[place(p * HALF + wave * 16 + l16, kk / 8 + quad)]);
 #pragma unroll
-        for (int i = 0; i < NT; ++i) {
-          const bf16x8 wf = *reinterpret_cast<const bf16x8*>(&ws[place(p * HALF + (wn * NT + i) * 16 + l16, kk / 8 + quad)]);
-#pragma unroll
-          for (int j = 0; j < MT; ++j) acc[p][i][j] = expert_mfma(wf, xf[j], acc[p][i][j]);
-        }
+        for (int j = 0; j < MT; ++j) acc[p][j] = expert_mfma(wf, xf[j], acc[p][j]);
+      }
     }
   };
 #pragma unroll
@@ -519,36 +515,29 @@ __global__ __launch_bounds__(256, 2) void expert_gemm_kernel(const ExpertGemmArg
   // column = row l16 of the tile's rows, rows = features 4 quad + i
 #pragma unroll
   for (int j = 0; j < MT; ++j) {
-    const int r = (wm * MT + j) * 16 + l16;
+    const int r = j * 16 + l16;
     if (r >= rows) continue;
     const int slot = slot_of[r];
     if constexpr (PAIRED) {
       const float s = a.scores[slot];
-      __bf16* y = a.y + ((long)tile * BM + r) * a.F;
+      const int f = f0 + wave * 16 + quad * 4;
+      if (f < a.F) {
+        bf16x4 o;
 #pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        const int f = f0 + (wn * NT + i) * 16 + quad * 4;
+        for (int m = 0; m < 4; ++m) o[m] = (__bf16)(silu_exact(acc[1][j][m] * s) * (acc[0][j][m] * s));
+        *reinterpret_cast<bf16x4*>(a.y + ((long)tile * BM + r) * a.F + f) = o;
+      }
+    } else {
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int f = f0 + p * HALF + wave * 16 + quad * 4;
         if (f < a.F) {
           bf16x4 o;
 #pragma unroll
-          for (int m = 0; m < 4; ++m) o[m] = (__bf16)(silu_exact(acc[1][i][j][m] * s) * (acc[0][i][j][m] * s));
-          *reinterpret_cast<bf16x4*>(y + f) = o;
+          for (int m = 0; m < 4; ++m) o[m] = (__bf16)acc[p][j][m];
+          *reinterpret_cast<bf16x4*>(a.y + (long)slot * a.F + f) = o;
         }
       }
-    } else {
-      __bf16* y = a.y + (long)slot * a.F;
-#pragma unroll
-      for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int i = 0; i < NT; ++i) {
-          const int f = f0 + p * HALF + (wn * NT + i) * 16 + quad * 4;
-          if (f < a.F) {
-            bf16x4 o;
-#pragma unroll
-            for (int m = 0; m < 4; ++m) o[m] = (__bf16)acc[p][i][j][m];
-            *reinterpret_cast<bf16x4*>(y + f) = o;
-          }
-        }
     }
   }
 }
@@ -905,16 +894,16 @@ template <bool PAIRED, bool TAIL> int launch_expert_gemm_large(ExpertGemmArgs a,
   return BASED_OK;
 }
 
-template <int BM, int BN, int AHEAD, bool PAIRED> void launch_expert_gemm(ExpertGemmArgs a, hipStream_t s) {
-  const int cols = PAIRED ? BN / 2 : BN;
+template <bool PAIRED> void launch_expert_gemm(ExpertGemmArgs a, hipStream_t s) {
+  const int cols = PAIRED ? kSmallWeights / 2 : kSmallWeights;
   a.col_tiles = (a.F + cols - 1) / cols;
-  hipLaunchKernelGGL((expert_gemm_kernel<BM, BN, AHEAD, PAIRED>), dim3((unsigned)(a.col_tiles * a.tiles)), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(expert_gemm_kernel<PAIRED>, dim3((unsigned)(a.col_tiles * a.tiles)), dim3(256), 0, s, a);
 }
 
 template <bool PAIRED> int launch_expert_product(const ExpertGemmArgs& a, int rows, hipStream_t s) {
   if (rows == BASED_EXPERT_TILE_ROWS)
     return a.K % kGemmK == 0 ? launch_expert_gemm_large<PAIRED, false>(a, s) : launch_expert_gemm_large<PAIRED, true>(a, s);
-  launch_expert_gemm<BASED_EXPERT_TILE_ROWS_SMALL, 128, 4, PAIRED>(a, s);
+  launch_expert_gemm<PAIRED>(a, s);
   return BASED_OK;
 }
 

@@ -1411,7 +1411,7 @@ def experts(h, router, w1, w2, top: int, norm=None) -> torch.Tensor:
     plan = _CHECKED.get(key)
     if plan is None:
         plan = _CHECKED[key] = _experts_plan(h, router, w1, w2, top)
-    n, D, F, E, grouped, vec_f32, tiles, (at_ids, at_rank, at_counts, at_first, at_tiles, at_order, at_act, at_part, ints), code = plan
+    n, D, F, E, grouped, vec_f32, (at_ids, at_rank, at_counts, at_first, at_tiles, at_order, at_act, at_part, ints), code = plan
     h2, dev = h.reshape(-1, D), h.device
     lib = _lib.lib()
     norm_args = (None, None, None, None, 1.0, NORM_RMS, 0.0)
@@ -1481,7 +1481,7 @@ def _experts_plan(h, router, w1, w2, top: int):
                    4 * tiles * rows, act_rows * F * size, parts * size):
         at += (nbytes + 15) // 16 * 16  # (whole 16-byte pieces each)
         ends.append(at)
-    return n, D, F, E, grouped, vec_f32, tiles, (*ends[:8], ends[8] // 4), _dtype_code(h2)
+    return n, D, F, E, grouped, vec_f32, (*ends[:8], ends[8] // 4), _dtype_code(h2)
 
 
 # Rows up to which the streamed-input prologue is evaluated inside the projection.  Every workgroup of it
