@@ -558,11 +558,26 @@ def test_experts_in_large_tiles(dev, n, D, F, E, top):
 @pytest.mark.parametrize("n,E,top", [(33, 8, 1), (4095, 8, 2), (4096, 32, 2), (4097, 8, 2), (4100, 33, 2), (4223, 70, 4), (5000, 130, 3), (20000, 64, 2), (40000, 128, 1), (32767, 8, 2), (32768, 8, 2), (33000, 30, 1)])
 def test_places_of_the_choices(dev, n, E, top):
     """Every choice of a batch goes to the same expert as in batches of few tokens, whose places one workgroup plans: by the workgroups' counts (n E up
-    to a million in 32 tokens), by sums of them (beyond, or no room), with groups that end inside the last workgroup's eight."""
+    to a million in 32 tokens), by sums of them (beyond), with groups that end inside the last workgroup's eight."""
+    check_places(dev, n, E, top, 16)
+
+
+@pytest.mark.parametrize("E", [120, 121])
+def test_places_of_the_choices_without_room_for_counts(dev, E):
+    """4305 tokens in workgroups of 16 (a router that is not 16-byte aligned) leave 270 E counts, 4 bytes each: of 121 experts 130,680 bytes, more than
+    the 130,560 of the activations; of 120 they fit."""
+    n, F = 4305, 8
+    counts, rows = -(-n // 16) * E, 32 * (n // 32 + E)  # (tiles of 32: less than 96 choices an expert)
+    assert counts <= 32768 and (counts * 4 > rows * F * 2) == (E == 121)
+    check_places(dev, n, E, 1, F, router_offset=1)
+
+
+def check_places(dev, n, E, top, F, router_offset=0):
     from based_amd import ops
 
-    h, router, w1, w2, _ = expert_case(n, 64, 16, E, top, BF16, seed=n)
-    args = [t.to(dev) for t in (router, w1, w2)]
+    h, router, w1, w2, _ = expert_case(n, 64, F, E, top, BF16, seed=n)
+    moved = torch.empty(router.numel() + router_offset, dtype=BF16, device=dev)[router_offset:].view_as(router).copy_(router)
+    args = [moved, w1.to(dev), w2.to(dev)]
     whole = ops.experts(h.to(dev), *args, top)
     rows = torch.randint(0, n, (64,), generator=torch.Generator().manual_seed(n))
     rows[:2] = torch.tensor([0, n - 1])
