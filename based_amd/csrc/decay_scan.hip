@@ -11,7 +11,7 @@
 //   decay_scan_mfma   bf16: walks 64 tokens at a time with the state in MFMA accumulators, 16 value channels
 //                     per wavefront.  Long sequences are cut into segments: a first pass leaves what every
 //                     segment adds to the state, `decay_join` turns that into the state at every segment's
-//                     start, and the second pass starts there.
+//                     start, and the second pass starts there; few segments it puts together itself.
 //   decay_scan_any    any element type and size, in segments too: a thread holds some key channels of one value channel.
 //   decay_step        one token per sequence; for channel decays with the low-rank decay in front and the
 //                     head norm and gate behind.

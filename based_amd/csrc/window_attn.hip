@@ -163,8 +163,9 @@ constexpr int kTileKeys = 64;
 constexpr int kTileRows = 128;  // (token, head) rows per workgroup
 
 // Bound by the vector unit and by waiting for the tiles: as many wavefronts as fit.  Sizes up to 64 run in 128 registers, four
-// workgroups to a compute unit (three, with 143, and the maxima of rows exchanged through LDS): 16 heads on 4 of 64 channels, with the cache
-// write, 4 x 2048 tokens and 129 keys 28.9 -> 24.8 us; on 16 44.4 -> 39.5; 6 x 2240 tokens and 513 keys 81.8 -> 73.9; one of 700 26.2 -> 23.1.
+// workgroups to a compute unit (three, with 143, and the maxima of rows exchanged through LDS; 2.3 wavefronts on a SIMD on average, 1.9): 16 heads on
+// 4 of 64 channels, with the cache write, 4 x 2048 tokens and 129 keys 28.9 -> 24.8 us; on 16 44.4 -> 39.5; 6 x 2240 tokens and 513 keys 81.8 ->
+// 73.9; one of 700 26.2 -> 23.1.
 
 __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
