@@ -7,27 +7,34 @@
 //                        would lose digits to cancellation), the others from them block by block.
 //   delta_chunk_scan     walks the chunks: U = Uv + W S0, S1 = G_64 S0 + sum_s k_s (G_64 / G_s) u_s^T, and beside the chain
 //                        o_t = G_t S0^T q_t + sum_{s <= t} P_ts u_s.  A workgroup of four wavefronts carries 16 value channels of a
-//                        head; wavefront w has the 16 tokens w of every chunk and the state rows w, w + 4, ..; S0 and U go round
+//                        head; wavefront w has 16 tokens of every chunk and the state tiles w, w + 4, ..; S0 and U go round
 //                        through LDS, two barriers per chunk.
-// Everything is fp32 MFMA (v_mfma_f32_16x16x4_f32).  The accumulator layout (column = lane % 16, row = 4 (lane / 16) + i) is the operand
-// of instruction i of a product contracted over rows {i, 4 + i, 8 + i, 12 + i}, so accumulators become operands as they stand, and
-// what delta_chunk_prepare leaves lies as the scan's lanes want it: whole wavefronts of 16-byte pieces.
+// Products run on bf16 MFMA (16 x 16 x 32, sixteen times the rate of fp32), with 32 bits of every operand: a number of 32 bits enters as
+// the sum of three of bf16 (each what the ones before leave, rounded: 24 bits and a sign between them), and of the nine products of two such
+// sums the six that reach 2^-24 of the result are taken.  Inputs of bf16 are one part as they are, scaled by row or behind the product, so
+// their products are exact.  Sums are the matrix unit's, in 32 bits; the small products have an accumulator of their own.
+//
+// Operand layout of a lane (l16 = lane % 16, quad = lane / 16): row or column l16, contracted elements 8 quad .. 8 quad + 7; results: column
+// l16, rows 4 quad + i.  What a result feeds next is contracted over its rows, so the rows of the tiles 2 n and 2 n + 1 are dealt out in turn:
+// row 4 quad + i of tile 2 n + p is element 32 n + 8 quad + 4 p + i, and the four results of a lane in both tiles are one operand.  State
+// tiles (channels), U (tokens) and the tiles of W and Uv that make it are dealt so; outputs are not.
 //
 // Against blocks of 16 (gated_delta_scan_kernel) a chain step takes in four times the tokens with two exchanges instead of one, and
-// nothing but W S0 and k^T U stands in the chain.  Products per 64 tokens, d = 64, dv = 128: 3.9 -> 7.9 M fp32 operations in all, of
-// which 3.9 M in the scan.  4 sequences x 8 heads of 2048 tokens: 161 -> 91 us; traced, 41 of preparation (written back at 2.3 TB/s, matrix
-// pipe a third busy) and 55 of scan (a lone workgroup per compute unit: 2.0 of 4.1 thousand cycles a chunk are products, the rest waits for
-// accumulators, LDS and barriers; eight wavefronts with the outputs apart from the chain take 60).
+// nothing but W S0 and k^T U stands in the chain.  4 sequences x 8 heads of 2048 tokens, d = 64, dv = 128, bf16: 161 us in blocks, 91 with
+// fp32 products (41 of preparation, 55 of scan, 2.0 of whose 4.1 thousand cycles a chunk were products), now 67: preparation 24, bound by
+// what it writes (92 MB at 3.8 TB/s), and scan 41, 3.1 thousand cycles a chunk: 2.0 of the chain itself, the rest waits for the chunk's 62 KB
+// (without those loads 27 us, with all of them from L2 37).  d = 128: 226 -> 131 us (1 x 4096, 16 heads), fp32 232 -> 188.  Errors against
+// 64 bits: 1.9e-7 -> 1.4e-7.
 #include "gated_delta.hpp"
 
 namespace based {
 
-constexpr int kDc = 64;           // tokens per chunk
-constexpr int kDcPairs = 10;      // lower-triangular pairs of 16-token tiles
-// pairs (0, 0), (1, 0), (1, 1), (2, 0) ..: a digit each, in registers (a table would be read from memory)
-__host__ __device__ constexpr int pair_t(int p) { return (int)(0x3333222110ull >> (4 * p)) & 15; }
-__host__ __device__ constexpr int pair_s(int p) { return (int)(0x3210210100ull >> (4 * p)) & 15; }
-__host__ __device__ constexpr int pair_of(int t, int s) { return t * (t + 1) / 2 + s; }
+constexpr int kDc = 64;        // tokens per chunk
+constexpr int kDcRow = 72;     // a row of 64 in LDS, bf16: 16-byte pieces of 16 rows meet every bank once
+// Products of a tile of 16 tokens with the tokens up to its end, by 32: a tile and a piece of 32 for each of six
+__host__ __device__ constexpr int unit_t(int u) { return (int)(0x332210u >> (4 * u)) & 15; }
+__host__ __device__ constexpr int unit_s(int u) { return (int)(0x101000u >> (4 * u)) & 15; }
+__host__ __device__ constexpr int unit_of(int t) { return t < 2 ? t : 2 * t - 2; }
 
 struct DeltaChunkArgs {
   const void* q;
@@ -48,14 +55,14 @@ struct DeltaChunkArgs {
   int fresh, v_vec;
 };
 
-// What a chunk leaves in the workspace, in tiles of 256 floats, a lane's four next to each other: W and q by (token tile, channel
-// tile), k G_64 / G_t by (channel tile, token tile), P by pair, Uv by (value tile, token tile); then fq G of every token, and G_64.
-// (q and k in bf16 would halve their bytes, and cost the scan a conversion in front of every product: 56 -> 68 us.)
-template <int RB> struct DcAt {
-  static constexpr long kW = 0, kQ = (long)4 * RB * 256, kK = 2 * kQ, kP = 3 * kQ, kUv = kP + kDcPairs * 256;
+// What a chunk leaves in the workspace, in operands of 1 KB (16 bytes a lane): W (token tile, 32 channels, part), q (token tile, 32
+// channels; as they are, 8 of bf16 or of fp32 a lane), k transposed (channel tile, 32 tokens, part), P (unit, part), and Uv (value tile, token tile) in 32 bits; then, by token,
+// fq G of the queries and what a token's value is multiplied by at the chunk's end, and G_64.  NP: parts of an element of q and k.
+template <int RB, int NP> struct DcAt {
+  static constexpr long kW = 0, kQ = (long)6 * RB * 256, kK = kQ + 2 * RB * (NP == 1 ? 1 : 2) * 256, kP = kK + 2 * RB * NP * 256, kUv = kP + 18 * 256;
 };
-__host__ __device__ inline long dc_vec_at(int rb, int dv) { return ((long)12 * rb + kDcPairs + (long)((dv + 15) / 16) * 4) * 256; }
-__host__ __device__ inline long dc_floats(int rb, int dv) { return dc_vec_at(rb, dv) + kDc + 4; }
+__host__ __device__ inline long dc_vec_at(int rb, int np, int dv) { return ((long)(np == 1 ? 10 : 16) * rb + 18 + (long)((dv + 15) / 16) * 4) * 256; }
+__host__ __device__ inline long dc_floats(int rb, int np, int dv) { return dc_vec_at(rb, np, dv) + 2 * kDc + 4; }
 
 // exp of a sum of log decays held in 64 bits, which as a float would lose |x| 2^-24 of the result
 __device__ __forceinline__ float exp_of(double x) {
@@ -63,27 +70,62 @@ __device__ __forceinline__ float exp_of(double x) {
   return __builtin_fmaf(e, (float)(x - (double)hi), e);
 }
 
-// Four channels of a row in LDS.
-template <typename T> __device__ __forceinline__ f32x4 four_at(const T* p) {
-  typedef __attribute__((ext_vector_type(4))) T t4;
-  const t4 r = *reinterpret_cast<const t4*>(p);
-  return f32x4{to_f32(r[0]), to_f32(r[1]), to_f32(r[2]), to_f32(r[3])};
+typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+
+// Two numbers as three packed pairs of bf16: rounded, what that left rounded, and what is left.
+__device__ __forceinline__ void parts2(float a, float b, uint32_t (&o)[3]) {
+#pragma unroll
+  for (int n = 0; n < 3; ++n) {
+    o[n] = pack_bf16(a, b);
+    a -= __builtin_bit_cast(float, o[n] << 16);
+    b -= __builtin_bit_cast(float, o[n] & 0xffff0000u);
+  }
+}
+__device__ __forceinline__ void parts4(const f32x4& x, u32x2 (&o)[3]) {
+  uint32_t a[3], b[3];
+  parts2(x[0], x[1], a);
+  parts2(x[2], x[3], b);
+#pragma unroll
+  for (int n = 0; n < 3; ++n) o[n] = u32x2{a[n], b[n]};
+}
+__device__ __forceinline__ void parts8(const f32x4& x, const f32x4& y, bf16x8 (&o)[3]) {
+  u32x2 a[3], b[3];
+  parts4(x, a);
+  parts4(y, b);
+#pragma unroll
+  for (int n = 0; n < 3; ++n) o[n] = __builtin_bit_cast(bf16x8, u32x4{a[n][0], a[n][1], b[n][0], b[n][1]});
+}
+
+__device__ __forceinline__ bf16x4 read_transposed(const __bf16* p) {
+  typedef __attribute__((address_space(3))) bf16x4 shared4;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((shared4*)p);
+}
+
+__device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+
+// x y added to sum[0], the products that are at most 2^-8 of it to sum[1]: NX and NY parts.
+template <int NX, int NY> __device__ __forceinline__ void product(const bf16x8 (&x)[NX], const bf16x8 (&y)[NY], f32x4 (&sum)[2]) {
+#pragma unroll
+  for (int n = NX + NY - 2 < 2 ? NX + NY - 2 : 2; n > 0; --n)
+#pragma unroll
+    for (int i = 0; i < NX; ++i)
+      if (n - i >= 0 && n - i < NY) sum[1] = mfma_bf16(x[i], y[n - i], sum[1]);
+  sum[0] = mfma_bf16(x[0], y[0], sum[0]);
 }
 
 // RB: 16-channel tiles of queries and keys.  LAY as for Four.  Rows go through LDS 64 channels at a time: a lane's operands lie in 16
-// rows, and asked for one by one they cost 16 lines of cache per instruction (20 of 44 thousand cycles of a lone workgroup).
+// rows, and asked for one by one they cost 16 lines of cache per instruction.
 template <typename T, int LAY, int RB>
-__global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const DeltaChunkArgs a) {
-  constexpr int kRow = kDc + 4, kSlabs = RB / 4;
+__global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void delta_chunk_prepare_kernel(const DeltaChunkArgs a) {
+  constexpr int NP = sizeof(T) == 2 ? 1 : 3, KC = RB / 2, kSlabs = RB / 4;
   constexpr bool kAhead = LAY != 0 && sizeof(T) == 2;  // slabs of queries and keys asked for one ahead (others do not fit the registers)
-  typedef DcAt<RB> At;
+  typedef DcAt<RB, NP> At;
   typedef __attribute__((ext_vector_type(4))) T t4;
-  __shared__ __attribute__((aligned(16))) float s_a[kDc][kRow], s_t[kDc][kRow];
-  __shared__ __attribute__((aligned(16))) T s_x[2][kDc][kRow];
+  __shared__ __attribute__((aligned(16))) __bf16 s_x[2][NP][kDc][kDcRow];
+  __shared__ __attribute__((aligned(16))) float s_a[kDc][kDc + 4];  // A, then T
   __shared__ double s_lc[kDc];
-  __shared__ __attribute__((aligned(16))) float s_beta[kDc], s_bg[kDc], s_tail[kDc], s_fq[kDc], s_fk[kDc];
-  // (in the place of T, which comes later: three workgroups share a compute unit's LDS for bf16)
-  float *s_e1k = &s_t[0][0], *s_e1q = s_e1k + kDc, *s_e2 = s_e1q + kDc;  // s_e2[4][kDc]
+  __shared__ __attribute__((aligned(16))) float s_beta[kDc], s_bg[kDc], s_fq[kDc], s_fk[kDc], s_e1k[kDc], s_e1q[kDc], s_e2[4 * kDc];
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int bh = __builtin_amdgcn_readfirstlane(blockIdx.x / a.span), c = a.c0 + (int)(blockIdx.x - bh * a.span);
@@ -94,10 +136,21 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
   const T* k = static_cast<const T*>(a.k) + b * a.x_sb + (long)t0 * a.x_sl + (long)hk * a.d;
   const T* v = static_cast<const T*>(a.v) + b * a.x_sb + (long)t0 * a.x_sl + (long)h * a.dv;
   float* ws = a.work + (long)blockIdx.x * a.per;
+  const int dealt = (l16 >> 2) * 8 + (l16 & 3);  // (+ 4 p: row l16 of tile p of a pair)
 
   // 64 channels from `e0` on of the chunk's rows: thread t has 4 channels of rows t / 16 + 16 j.  Rows past the last token are fetched
   // from it: gates of zero keep them out.
   const int piece = (tid & 15) * 4, row0 = tid >> 4;
+  auto keep = [&](int buf, int row, const t4& x) {
+    if constexpr (NP == 1) {
+      *reinterpret_cast<t4*>(&s_x[buf][0][row][piece]) = x;
+    } else {
+      u32x2 p[3];
+      parts4(f32x4{x[0], x[1], x[2], x[3]}, p);
+#pragma unroll
+      for (int n = 0; n < 3; ++n) *reinterpret_cast<u32x2*>(&s_x[buf][n][row][piece]) = p[n];
+    }
+  };
   auto fetch_slab = [&](Four<T, LAY> (&x)[4], const T* src, int e0, int lim) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -111,7 +164,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
       t4 r = x[j].r;
 #pragma unroll
       for (int i = 0; i < 4; ++i) r[i] = e0 + piece + i < lim ? r[i] : (T)0.0f;
-      *reinterpret_cast<t4*>(&s_x[buf][row0 + j * 16][piece]) = r;
+      keep(buf, row0 + j * 16, r);
     }
   };
   // values: any alignment
@@ -134,9 +187,23 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
       t4 r = x[j];
 #pragma unroll
       for (int i = 0; i < 4; ++i) r[i] = e0 + piece + i < a.dv ? r[i] : (T)0.0f;
-      *reinterpret_cast<t4*>(&s_x[buf][row0 + j * 16][piece]) = r;
+      keep(buf, row0 + j * 16, r);
     }
   };
+  auto row_operand = [&](int buf, int row, int e, bf16x8 (&x)[NP]) {
+#pragma unroll
+    for (int n = 0; n < NP; ++n) x[n] = *reinterpret_cast<const bf16x8*>(&s_x[buf][n][row][e]);
+  };
+  // tokens 32 ks + 8 quad .. of channel l16 of four pieces of 4 channels, EACH channels apart, from `e` on: a transposing read gives lane l16
+  // element l16 of the four rows whose 8 bytes each its group of 16 lanes names (24.6 -> 23.9 us)
+  auto column_operand = [&](int buf, int ks, int e, int each, bf16x8 (&x)[NP]) {
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+      const __bf16* at = &s_x[buf][n][ks * 32 + quad * 8 + (l16 >> 2)][e + (l16 & 3) * each];
+      x[n] = __builtin_shufflevector(read_transposed(at), read_transposed(at + 4 * kDcRow), 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+  };
+  auto put = [&](long at, const bf16x8& x) { *reinterpret_cast<bf16x8*>(ws + at * 256 + lane * 4) = x; };
 
   Four<T, LAY> kr[4], qr[4];
   fetch_slab(kr, k, 0, a.d);
@@ -144,18 +211,15 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
   const long gate = b * a.g_sb + (long)(t0 + (lane < left ? lane : left - 1)) * a.g_sl + h;
   const T gate_a = static_cast<const T*>(a.a)[gate], gate_b = static_cast<const T*>(a.bt)[gate];
   const T a_log = static_cast<const T*>(a.a_log)[h], dt_bias = static_cast<const T*>(a.dt_bias)[h];
-  // Products of keys with keys and with queries, transposed (column = token t, row = token s): seven of the twenty tiles for each of
-  // wavefronts 1 to 3, while wavefront 0 works the decays out.
-  constexpr int kMine = 7;
-  f32x4 acc[kMine][2];
-  int ri[kMine], ci[kMine];
+  const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+  // Products of keys with keys and with queries, transposed (column = token t, rows = the tokens s of a pair of tiles): four of the twelve
+  // units for each of wavefronts 1 to 3, while wavefront 0 works the decays out.
+  constexpr int kMine = 4;
+  f32x4 acc[kMine][2][2];
 #pragma unroll
-  for (int j = 0; j < kMine; ++j) {
-    const int p = (wave > 0 ? wave - 1 : 0) * kMine + j, pair = p < kDcPairs ? p : p < 2 * kDcPairs ? p - kDcPairs : 0;
-    acc[j][0] = acc[j][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-    ri[j] = pair_s(pair) * 16 + l16;
-    ci[j] = pair_t(pair) * 16 + l16;
-  }
+  for (int j = 0; j < kMine; ++j)
+#pragma unroll
+    for (int p = 0; p < 2; ++p) acc[j][p][0] = acc[j][p][1] = none;
   double sq = 0.0, sk = 0.0;  // (the squares' sums scale whole rows: an error in them does not average out)
 #pragma unroll 1
   for (int sl = 0; sl < kSlabs; ++sl) {
@@ -175,17 +239,19 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
     __syncthreads();
     if (wave > 0) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int e = r * 16 + quad * 4;
-        __builtin_amdgcn_sched_barrier(0);  // (a quarter of the operands in registers at a time)
+      for (int r = 0; r < 2; ++r)
 #pragma unroll
         for (int j = 0; j < kMine; ++j) {
-          const int p = (wave - 1) * kMine + j;
-          const f32x4 xf = four_at<T>(&s_x[0][ri[j]][e]), yf = four_at<T>(&s_x[p < kDcPairs ? 0 : 1][ci[j]][e]);
+          const int u = (wave - 1) * kMine + j, unit = u < 6 ? u : u - 6;
+          bf16x8 y[NP];
+          row_operand(u < 6 ? 0 : 1, unit_t(unit) * 16 + l16, r * 32 + quad * 8, y);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[j][i & 1] = mfma_f32(xf[i], yf[i], acc[j][i & 1]);
+          for (int p = 0; p < 2; ++p) {
+            bf16x8 x[NP];
+            row_operand(0, unit_s(unit) * 32 + dealt + 4 * p, r * 32 + quad * 8, x);
+            product(x, y, acc[j][p]);
+          }
         }
-      }
     } else if (sl == 0) {
       // log G in 64 bits: behind a token that forgets nearly everything the differences of these sums still have to carry the
       // ordinary decays
@@ -201,12 +267,27 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
       s_lc[lane] = lc;
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int e = r * 16 + quad * 4;
-      const f32x4 qf = four_at<T>(&s_x[1][wave * 16 + l16][e]), kf = four_at<T>(&s_x[0][wave * 16 + l16][e]);
-      sq += (double)(qf[0] * qf[0] + qf[1] * qf[1]) + (double)(qf[2] * qf[2] + qf[3] * qf[3]);
-      sk += (double)(kf[0] * kf[0] + kf[1] * kf[1]) + (double)(kf[2] * kf[2] + kf[3] * kf[3]);
-      *reinterpret_cast<f32x4*>(ws + At::kQ + ((long)wave * RB + sl * 4 + r) * 256 + lane * 4) = qf;
+    for (int r = 0; r < 2; ++r) {
+      bf16x8 x[2][NP];
+#pragma unroll
+      for (int n = 0; n < 2; ++n) row_operand(n, wave * 16 + l16, r * 32 + quad * 8, x[n]);
+      float f[2][8];
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[n][j] = NP == 1 ? to_f32(x[n][0][j]) : to_f32(x[n][0][j]) + (to_f32(x[n][NP > 1][j]) + to_f32(x[n][NP - 1][j]));
+#pragma unroll
+      for (int j = 0; j < 8; j += 4) {
+        sk += (double)(f[0][j] * f[0][j] + f[0][j + 1] * f[0][j + 1]) + (double)(f[0][j + 2] * f[0][j + 2] + f[0][j + 3] * f[0][j + 3]);
+        sq += (double)(f[1][j] * f[1][j] + f[1][j + 1] * f[1][j + 1]) + (double)(f[1][j + 2] * f[1][j + 2] + f[1][j + 3] * f[1][j + 3]);
+      }
+      const long at = At::kQ / 256 + (wave * KC + sl * 2 + r) * (NP == 1 ? 1 : 2);
+      if constexpr (NP == 1) {
+        put(at, x[1][0]);
+      } else {
+#pragma unroll
+        for (int n = 0; n < 2; ++n) *reinterpret_cast<f32x4*>(ws + (at + n) * 256 + lane * 4) = f32x4{f[1][4 * n], f[1][4 * n + 1], f[1][4 * n + 2], f[1][4 * n + 3]};
+      }
     }
   }
   // the next slab: the first of the keys again, or, where that one is still in LDS, the first of the values
@@ -235,10 +316,11 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
     if (wave == 0) {
       const double end = s_lc[kDc - 1];
       const float G = exp_of(lc);
+      float* vec = ws + dc_vec_at(RB, NP, a.dv);
       s_bg[lane] = -s_beta[lane] * G * fk;
-      s_tail[lane] = fk * exp_of(end - lc < 0.0 ? end - lc : 0.0);
-      ws[dc_vec_at(RB, a.dv) + lane] = s_fq[lane] * G;
-      if (lane == 63) ws[dc_vec_at(RB, a.dv) + kDc] = G;
+      vec[lane] = s_fq[lane] * G;
+      vec[kDc + lane] = fk * exp_of(end - lc < 0.0 ? end - lc : 0.0);
+      if (lane == 63) vec[2 * kDc] = G;
       s_e2[lane] = fk * exp_of(lc_front - lc);
     } else {
       const double ref = s_lc[wave * 16 - 1];
@@ -251,36 +333,47 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
   if (wave > 0) {
 #pragma unroll
     for (int j = 0; j < kMine; ++j) {
-      const int p = (wave - 1) * kMine + j;
-      if (p >= 2 * kDcPairs) break;  // (uniform)
-      const bool keys = p < kDcPairs;
-      const int pair = keys ? p : p - kDcPairs, tt = pair_t(pair), t = ci[j], s0 = pair_s(pair) * 16 + quad * 4;
-      f32x4 out = acc[j][0] + acc[j][1];
+      const int u = (wave - 1) * kMine + j;
+      const bool keys = u < 6;
+      const int unit = keys ? u : u - 6, tt = unit_t(unit), t = tt * 16 + l16, s0 = unit_s(unit) * 32 + quad * 8, ts = s0 >> 4;
       const float e1 = keys ? s_e1k[t] : s_e1q[t];
-      if (pair_s(pair) != tt) {  // (uniform)
-        out *= *reinterpret_cast<const f32x4*>(&s_e2[tt * kDc + s0]) * e1;
-      } else {
-        const double lc_t = s_lc[t], fall = (tt > 0 ? s_lc[tt > 0 ? tt * 16 - 1 : 0] : 0.0) - s_lc[tt * 16 + 15];
-        f32x4 f = *reinterpret_cast<const f32x4*>(&s_e2[s0]) * e1;
-        if (fall > 60.0) {
-          const float ft = keys ? s_fk[t] * s_beta[t] : s_fq[t];
+      const float* e2 = &s_e2[(ts == tt ? 0 : tt) * kDc + s0];
+      f32x4 out[2];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) out[p] = acc[j][p][0] + acc[j][p][1];
+      f32x4 f[2] = {*reinterpret_cast<const f32x4*>(e2) * e1, *reinterpret_cast<const f32x4*>(e2 + 4) * e1};
+      const double fall = (tt > 0 ? s_lc[tt > 0 ? tt * 16 - 1 : 0] : 0.0) - s_lc[tt * 16 + 15];
+      if (fall > 60.0 && ts == tt) {
+        const double lc_t = s_lc[t];
+        const float ft = keys ? s_fk[t] * s_beta[t] : s_fq[t];
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const double diff = lc_t - s_lc[s0 + i];
-            f[i] = ft * s_fk[s0 + i] * exp_of(diff < 0.0 ? diff : 0.0);
+            const double diff = lc_t - s_lc[s0 + 4 * p + i];
+            f[p][i] = ft * s_fk[s0 + 4 * p + i] * exp_of(diff < 0.0 ? diff : 0.0);
           }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) out[i] = s0 + i < t || (s0 + i == t && !keys) ? out[i] * f[i] : 0.f;
       }
-      if (keys)
-        *reinterpret_cast<f32x4*>(&s_a[t][s0]) = out;
-      else
-        *reinterpret_cast<f32x4*>(ws + At::kP + pair * 256 + lane * 4) = out;
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int s = s0 + 4 * p + i;
+          out[p][i] = s < t || (s == t && !keys) ? out[p][i] * f[p][i] : 0.f;
+        }
+      if (keys) {
+        *reinterpret_cast<f32x4*>(&s_a[t][s0]) = out[0];
+        *reinterpret_cast<f32x4*>(&s_a[t][s0 + 4]) = out[1];
+      } else {
+        bf16x8 x[3];
+        parts8(out[0], out[1], x);
+#pragma unroll
+        for (int n = 0; n < 3; ++n) put(At::kP / 256 + unit * 3 + n, x[n]);
+      }
     }
   }
   __syncthreads();
-  // T: the diagonal blocks, one per wavefront; column l16: x_t = [t = l16] - sum_{s<t} A_ts x_s
+  // T, in the place of A: the diagonal blocks, one per wavefront; column l16: x_t = [t = l16] - sum_{s<t} A_ts x_s
   {
     const int at = wave * 16;
     float x[16];
@@ -298,20 +391,18 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
     }
     if (quad == 0) {
 #pragma unroll
-      for (int t = 0; t < 16; ++t) s_t[at + t][at + l16] = x[t];
+      for (int t = 0; t < 16; ++t) s_a[at + t][at + l16] = x[t];
     }
   }
   __syncthreads();
   // the blocks below them, a column of blocks per wavefront: T_ij = -T_ii sum_{j <= k < i} A_ik T_kj
-  const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+  f32x4 col[4] = {none, none, none, none};
   if (wave < 3) {
-    f32x4 col[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      col[i] = none;
       if (i == wave) {
 #pragma unroll
-        for (int x = 0; x < 4; ++x) col[i][x] = s_t[i * 16 + quad * 4 + x][i * 16 + l16];
+        for (int x = 0; x < 4; ++x) col[i][x] = s_a[i * 16 + quad * 4 + x][i * 16 + l16];
       } else if (i > wave) {
         f32x4 sum[2] = {none, none};
 #pragma unroll
@@ -321,14 +412,12 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
 #pragma unroll
             for (int x = 0; x < 4; ++x) sum[x & 1] = mfma_f32(row[x], col[kb][x], sum[x & 1]);
           }
-        const f32x4 row = *reinterpret_cast<const f32x4*>(&s_t[i * 16 + l16][i * 16 + quad * 4]);
+        const f32x4 row = *reinterpret_cast<const f32x4*>(&s_a[i * 16 + l16][i * 16 + quad * 4]);
         const f32x4 y = sum[0] + sum[1];
         f32x4 res[2] = {none, none};
 #pragma unroll
         for (int x = 0; x < 4; ++x) res[x & 1] = mfma_f32(row[x], y[x], res[x & 1]);
         col[i] = -(res[0] + res[1]);
-#pragma unroll
-        for (int x = 0; x < 4; ++x) s_t[i * 16 + quad * 4 + x][wave * 16 + l16] = col[i][x];
       }
     }
   }
@@ -336,46 +425,75 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
     store_slab(0, kr, 0, a.d);
   else
     store_v(1, vr, 0);
+  __syncthreads();  // everybody has read A
+  if (wave < 3) {
+#pragma unroll
+    for (int i = 1; i < 4; ++i)
+      if (i > wave) {
+#pragma unroll
+        for (int x = 0; x < 4; ++x) s_a[i * 16 + quad * 4 + x][wave * 16 + l16] = col[i][x];
+      }
+  }
   __syncthreads();
-  f32x4 tm[kDcPairs];
+  // Every wavefront has two of the four (dealt) token tiles, one of the first 32 tokens and one of the others, and half of the channels.
+  const int half = wave & 1, m_of[2] = {wave >> 1, 3 - (wave >> 1)};
+  bf16x8 tm[3][3];  // T with its columns scaled: tokens 0 .. 31 for the first tile, then both halves for the second
+  auto scaled = [&](const float* by) {
 #pragma unroll
-  for (int p = 0; p < kDcPairs; ++p) tm[p] = *reinterpret_cast<const f32x4*>(&s_t[pair_t(p) * 16 + l16][pair_s(p) * 16 + quad * 4]);
-  auto column = [&](int buf, int s, int i) { return to_f32(s_x[buf][s * 16 + quad * 4 + i][wave * 16 + l16]); };
-  // W^T (row = channel, column = token: the scan's operand) and the scaled keys of a slab's channel tile `wave`
-  auto keys_tile = [&](int buf, int tile) {
-    f32x4 out[4] = {none, none, none, none};
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const f32x4 f = *reinterpret_cast<const f32x4*>(&s_bg[s * 16 + quad * 4]), g = *reinterpret_cast<const f32x4*>(&s_tail[s * 16 + quad * 4]);
-      f32x4 kf;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float x = column(buf, s, i), xf = x * f[i];
-        kf[i] = x * g[i];
-#pragma unroll
-        for (int m = s; m < 4; ++m) out[m] = mfma_f32(xf, tm[pair_of(m, s)][i], out[m]);
-      }
-      *reinterpret_cast<f32x4*>(ws + At::kK + ((long)tile * 4 + s) * 256 + lane * 4) = kf;
+    for (int n = 0; n < 3; ++n) {
+      const int m = m_of[n > 0], ks = n == 2, t = (m >> 1) * 32 + dealt + 4 * (m & 1), s0 = ks * 32 + quad * 8;
+      const f32x4* row = reinterpret_cast<const f32x4*>(&s_a[t][s0]);
+      const f32x4* f = reinterpret_cast<const f32x4*>(by + s0);
+      parts8(row[0] * f[0], row[1] * f[1], tm[n]);
     }
-#pragma unroll
-    for (int m = 0; m < 4; ++m) *reinterpret_cast<f32x4*>(ws + At::kW + ((long)m * RB + tile) * 256 + lane * 4) = out[m];
   };
-  // Uv (row = token, column = channel: the scan's accumulator) of a slab's value tile `wave`
-  auto values_tile = [&](int buf, int tile) {
-    f32x4 out[4] = {none, none, none, none};
+  // W (row = token, contracted over channels in the scan: here transposed) and the keys of 32 channels of a slab
+  auto keys_tile = [&](int buf, int kc) {
+    bf16x8 kx[2][2][NP];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const f32x4 f = *reinterpret_cast<const f32x4*>(&s_beta[s * 16 + quad * 4]);
+    for (int p = 0; p < 2; ++p)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float xf = column(buf, s, i) * f[i];
+      for (int ks = 0; ks < 2; ++ks) column_operand(buf, ks, half * 32 + 4 * p, 8, kx[p][ks]);
+    const int mine = wave >> 1;
 #pragma unroll
-        for (int m = s; m < 4; ++m) out[m] = mfma_f32(tm[pair_of(m, s)][i], xf, out[m]);
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int n = 0; n < NP; ++n) put(At::kK / 256 + ((kc * 2 + mine) * 2 + ks) * NP + n, mine ? kx[1][ks][n] : kx[0][ks][n]);
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      f32x4 out[2];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        f32x4 sum[2] = {none, none};
+#pragma unroll
+        for (int ks = 0; ks <= m; ++ks) product(kx[p][ks], tm[m + ks], sum);
+        out[p] = sum[0] + sum[1];
+      }
+      bf16x8 x[3];
+      parts8(out[0], out[1], x);
+#pragma unroll
+      for (int n = 0; n < 3; ++n) put(At::kW / 256 + (m_of[m] * KC + kc) * 3 + n, x[n]);
+    }
+  };
+  // Uv (rows = tokens, column = channel: the scan's accumulator) of two of a slab's value tiles
+  auto values_tile = [&](int buf, int tile0) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const int tile = tile0 + half * 2 + x;
+      if (tile * 16 >= a.dv) break;  // (uniform)
+      bf16x8 vx[2][NP];
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) column_operand(buf, ks, (half * 2 + x) * 16, 4, vx[ks]);
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        f32x4 sum[2] = {none, none};
+#pragma unroll
+        for (int ks = 0; ks <= m; ++ks) product(tm[m + ks], vx[ks], sum);
+        *reinterpret_cast<f32x4*>(ws + At::kUv + ((long)tile * 4 + m_of[m]) * 256 + lane * 4) = sum[0] + sum[1];
       }
     }
-#pragma unroll
-    for (int m = 0; m < 4; ++m) *reinterpret_cast<f32x4*>(ws + At::kUv + ((long)tile * 4 + m) * 256 + lane * 4) = out[m];
   };
+  scaled(s_bg);
   int buf = 0;  // the slab in LDS; the next one goes into the other buffer, which everybody has left behind at the barrier before
   if constexpr (kSlabs > 1) {
 #pragma unroll 1
@@ -387,7 +505,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
           fetch_v(vr, 0);
       };
       if (kAhead) fetch();
-      keys_tile(buf, sl * 4 + wave);
+      keys_tile(buf, sl * 2 + half);
       if (!kAhead) fetch();
       buf ^= 1;
       if (sl + 1 < kSlabs)
@@ -397,14 +515,15 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
       __syncthreads();
     }
   } else {
-    keys_tile(0, wave);
+    keys_tile(0, half);
     buf = 1;
   }
+  scaled(s_beta);
 #pragma unroll 1
   for (int e0 = 0; e0 < a.dv; e0 += 64) {
     const bool more = e0 + 64 < a.dv;
     if (more) fetch_v(vr, e0 + 64);
-    if (e0 + wave * 16 < a.dv) values_tile(buf, e0 / 16 + wave);
+    values_tile(buf, e0 / 16);
     if (!more) break;
     buf ^= 1;
     if (kSlabs == 1 && e0 == 0) __syncthreads();  // (a slower wavefront may still read the keys there)
@@ -413,157 +532,227 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_prepare_kernel(const Delta
   }
 }
 
-// grid: x = (sequence, head), y = 16 value channels
-template <int RB>
-__global__ __launch_bounds__(256, 2) void delta_chunk_scan_kernel(const DeltaChunkArgs a) {
-  static_assert(RB % 4 == 0, "every wavefront has state rows");
-  constexpr int RBW = RB / 4;
-  typedef DcAt<RB> At;
-  __shared__ __attribute__((aligned(16))) f32x4 s_s[RB][64], s_u[2][4][64];
+// Whether a workgroup of the scan has more registers than two of them find on a compute unit.
+__host__ __device__ constexpr bool dc_lone(int rb) { return rb == 8; }
+
+// grid: x = (sequence, head), y = 16 value channels.  Wavefronts 0 .. 3 carry the state, 4 .. 7 form the outputs, a chunk behind with the
+// products of P: four wavefronts that do both take 44 us for 41 above and 118 for 105 with keys of 128.  Two barriers a chunk:
+//   state there   state: U = Uv + W S0, its scaled parts to LDS.  outputs: parts of S0 and of the U before are read, q S0 and P U formed
+//   U there       state: S1 = G S0 + k U, its parts to LDS, and those of U.  outputs: stored, the next operands asked for
+template <int RB, int NP>
+__global__ __launch_bounds__(512, dc_lone(RB) ? 2 : 4) void delta_chunk_scan_kernel(const DeltaChunkArgs a) {
+  static_assert(RB % 4 == 0, "every wavefront has state tiles");
+  constexpr int RBW = RB / 4, KC = RB / 2;
+  typedef DcAt<RB, NP> At;
+  // operands of three parts: the state by 32 channels; U by 32 tokens, as the outputs take it and scaled to the chunk's end
+  __shared__ __attribute__((aligned(16))) bf16x8 s_s[KC][3][64], s_u[2][3][64], s_us[2][3][64];
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int role = __builtin_amdgcn_readfirstlane(tid >> 8), wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
   const int bh = blockIdx.x, b = __builtin_amdgcn_readfirstlane(bh / a.H), h = bh - b * a.H;
   const int ct = blockIdx.y, col = ct * 16 + l16;
   const bool col_in = col < a.dv;
-  const float* ws = a.work + (long)bh * a.span * a.per;
-  const long vec_at = dc_vec_at(RB, a.dv);
-  float* st = a.state + (long)bh * a.d * a.dvp + (col_in ? col : 0);
-  const int o_sl = a.H * a.dv;
-  float* o = a.o + ((long)b * a.L * a.H + h) * a.dv + (long)a.c0 * kDc * o_sl;
+  const char* ws = reinterpret_cast<const char*>(a.work + (long)bh * a.span * a.per);
+  const long per = a.per * 4, vec_at = dc_vec_at(RB, NP, a.dv) * 4;
   const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+  const unsigned at_lane = (unsigned)lane * 16u;
+  auto operand_at = [&](const char* p, int n) { return *reinterpret_cast<const bf16x8*>(p + n * 1024 + at_lane); };
 
-  f32x4 S[RBW];  // rows 16 (wave + 4 x) ..
+  if (role == 0) {
+    __builtin_amdgcn_s_setprio(2);
+    const int dealt = (wave >> 1) * 32 + quad * 8 + (wave & 1) * 4;  // first of the tokens (channels + 64 x) of this lane's four rows
+    // half of a lane's operand, where this wavefront's tile of a pair goes
+    auto put = [&](bf16x8 (&to)[3][64], const f32x4& x) {
+      u32x2 p[3];
+      parts4(x, p);
 #pragma unroll
-  for (int x = 0; x < RBW; ++x) {
-    const int r = wave + 4 * x;
+      for (int n = 0; n < 3; ++n) reinterpret_cast<u32x2*>(&to[n][lane])[wave & 1] = p[n];
+    };
+    float* st = a.state + (long)bh * a.d * a.dvp + (col_in ? col : 0);
+    f32x4 S[RBW];  // tiles wave + 4 x
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = r * 16 + quad * 4 + i;
-      const bool in = !a.fresh && col_in && row < a.d;
-      S[x][i] = in ? st[(long)row * a.dvp] : 0.f;
+    for (int x = 0; x < RBW; ++x) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = x * 64 + dealt + i;
+        const bool in = !a.fresh && col_in && row < a.d;
+        S[x][i] = in ? st[(long)row * a.dvp] : 0.f;
+      }
+      put(s_s[(wave >> 1) + 2 * x], S[x]);
     }
-    s_s[r][lane] = S[x];
-  }
-
-  // What a chunk needs from memory: one set of registers, each part asked for anew as soon as its last use has been issued, in the
-  // order of the uses, so that a part travels for the rest of the chunk.
-  f32x4 w[RB], p[4], uv, gq, qx[RB], kt[RBW][4];
-  float last;
-  auto tile_at = [&](int n, long at) { return *reinterpret_cast<const f32x4*>(ws + (long)n * a.per + at + lane * 4); };
-  auto rows_at = [&](int n, long at) { return *reinterpret_cast<const f32x4*>(ws + (long)n * a.per + at + wave * 16 + quad * 4); };
-  auto fetch_w = [&](int n) {
+    // What a chunk needs from memory: a set of registers, each part asked for anew as soon as its last use has been issued.
+    bf16x8 w[KC][3], kt[RBW][2][NP];
+    f32x4 uv, tail;
+    float last;
+    const char *pw = ws + At::kW * 4 + wave * KC * 3072, *pu = ws + At::kUv * 4 + (ct * 4 + wave) * 1024;
+    const char *pk = ws + At::kK * 4 + wave * 2 * NP * 1024, *pv = ws + vec_at;
+    auto fetch_w = [&] {
 #pragma unroll
-    for (int r = 0; r < RB; ++r) w[r] = tile_at(n, At::kW + (wave * RB + r) * 256);
-    uv = tile_at(n, At::kUv + (ct * 4 + wave) * 256);
-  };
-  auto fetch_q = [&](int n) {
+      for (int r = 0; r < KC; ++r)
 #pragma unroll
-    for (int r = 0; r < RB; ++r) qx[r] = tile_at(n, At::kQ + (wave * RB + r) * 256);
-  };
-  auto fetch_k = [&](int n) {
+        for (int j = 0; j < 3; ++j) w[r][j] = operand_at(pw, r * 3 + j);
+      uv = *reinterpret_cast<const f32x4*>(pu + at_lane);
+      tail = *reinterpret_cast<const f32x4*>(pv + kDc * 4 + (unsigned)dealt * 4u);
+    };
+    auto fetch_k = [&] {
+#pragma unroll
+      for (int x = 0; x < RBW; ++x)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int j = 0; j < NP; ++j) kt[x][s][j] = operand_at(pk, (x * 8 + s) * NP + j);
+      last = *reinterpret_cast<const float*>(pv + kDc * 8);
+    };
+    fetch_w();
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_k();
+    for (int n = 0; n < a.span; ++n) {
+      const long step = n + 1 < a.span ? per : 0;
+      pw += step, pu += step, pk += step, pv += step;
+      lds_barrier();  // the state is there
+      bf16x8 s0[KC][3];
+#pragma unroll
+      for (int r = 0; r < KC; ++r)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) s0[r][j] = s_s[r][j][lane];
+      // (what is added to a sum that starts from the large term loses its last digits sixteen times: added at the end, once)
+      f32x4 u[2][2] = {{none, none}, {none, none}};
+#pragma unroll
+      for (int r = 0; r < KC; ++r) product(w[r], s0[r], u[r & 1]);
+      const f32x4 un = uv + ((u[0][1] + u[1][1]) + (u[0][0] + u[1][0]));
+      put(s_us[wave >> 1], un * tail);
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_w();
+      __builtin_amdgcn_sched_barrier(0);
+      lds_barrier();  // U is there
+      bf16x8 us[2][3];
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) us[s][j] = s_us[s][j][lane];
+      put(s_u[wave >> 1], un);
+#pragma unroll
+      for (int x = 0; x < RBW; ++x) {
+        f32x4 sum[2][2] = {{none, none}, {none, none}};
+#pragma unroll
+        for (int s = 0; s < 2; ++s) product(kt[x][s], us[s], sum[s]);
+        S[x] = S[x] * last + ((sum[0][1] + sum[1][1]) + (sum[0][0] + sum[1][0]));
+        put(s_s[(wave >> 1) + 2 * x], S[x]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_k();
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    lds_barrier();  // the last U is there
 #pragma unroll
     for (int x = 0; x < RBW; ++x)
 #pragma unroll
-      for (int s = 0; s < 4; ++s) kt[x][s] = tile_at(n, At::kK + ((wave + 4 * x) * 4 + s) * 256);
-    last = ws[(long)n * a.per + vec_at + kDc];
-  };
-  auto fetch_p = [&](int n) {
-    gq = rows_at(n, vec_at);
-#pragma unroll
-    for (int s = 0; s < 4; ++s)  // (tiles behind the wavefront's own tokens: its own again, not used)
-      p[s] = tile_at(n, At::kP + (wave * (wave + 1) / 2 + (s <= wave ? s : wave)) * 256);
-  };
-
-  fetch_w(0);
-  __builtin_amdgcn_sched_barrier(0);
-  fetch_q(0);
-  __builtin_amdgcn_sched_barrier(0);
-  fetch_k(0);
-  __builtin_amdgcn_sched_barrier(0);
-  fetch_p(0);
-  unsigned mine = (unsigned)((wave * 16 + quad * 4) * o_sl + (col_in ? col : 0)) * 4u;
-  for (int n = 0; n < a.span; ++n) {
-    const int next = n + 1 < a.span ? n + 1 : n, buf = n & 1;
-    lds_barrier();  // S0 is there
-    f32x4 s0[RB];
-#pragma unroll
-    for (int r = 0; r < RB; ++r) s0[r] = s_s[r][lane];
-    // (what is added to a sum that starts from the large term loses its last digits sixteen times: added at the end, once)
-    f32x4 u[4] = {none, none, none, none};
-#pragma unroll
-    for (int r = 0; r < RB; ++r)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) u[i] = mfma_f32(w[r][i], s0[r][i], u[i]);
-    s_u[buf][wave][lane] = uv + ((u[0] + u[1]) + (u[2] + u[3]));
-    __builtin_amdgcn_sched_barrier(0);
-    fetch_w(next);
-    __builtin_amdgcn_sched_barrier(0);
-    // the queries' product with the state fills the wait for the other wavefronts
-    f32x4 oo[2] = {none, none};
-#pragma unroll
-    for (int r = 0; r < RB; ++r)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) oo[i & 1] = mfma_f32(qx[r][i], s0[r][i], oo[i & 1]);
-    __builtin_amdgcn_sched_barrier(0);
-    fetch_q(next);
-    lds_barrier();  // U is there
-    f32x4 us[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) us[s] = s_u[buf][s][lane];
-#pragma unroll
-    for (int x = 0; x < RBW; ++x) {
-      f32x4 sum[4] = {none, none, none, none};
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int s = 0; s < 4; ++s) sum[s] = mfma_f32(kt[x][s][i], us[s][i], sum[s]);
-      S[x] = S[x] * last + ((sum[0] + sum[1]) + (sum[2] + sum[3]));
-      s_s[wave + 4 * x][lane] = S[x];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    fetch_k(next);
-    __builtin_amdgcn_sched_barrier(0);
-    oo[0] = gq * (oo[0] + oo[1]);
-    oo[1] = none;
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-      if (s <= wave) {  // (uniform)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) oo[i & 1] = mfma_f32(p[s][i], us[s][i], oo[i & 1]);
+      for (int i = 0; i < 4; ++i) {
+        const int row = x * 64 + dealt + i;
+        if (col_in && row < a.d) st[(long)row * a.dvp] = S[x][i];
       }
-    const f32x4 out = oo[0] + oo[1];
-    __builtin_amdgcn_sched_barrier(0);
-    fetch_p(next);
-    char* ob = reinterpret_cast<char*>(o + (long)n * kDc * o_sl);
-    const int left = a.L - (a.c0 + n) * kDc;
-    if (col_in) {
-      if (left >= kDc) {  // (uniform)
+  } else {
+    const int o_sl = a.H * a.dv * 4;  // bytes
+    char* o = reinterpret_cast<char*>(a.o + ((long)b * a.L * a.H + h) * a.dv) + (long)a.c0 * kDc * o_sl;
+    const unsigned mine = (unsigned)((wave * 16 + quad * 4) * o_sl + (col_in ? col : 0) * 4);
+    const int pieces = wave >> 1;  // of 32 tokens in front of the last one that the wavefront's own reach
+    constexpr int NQ = NP == 1 ? 1 : 2;  // (queries of fp32 are taken apart here: their parts would be half as much again to write and to read)
+    bf16x8 p[2][3], qx[KC][NQ];
+    f32x4 gq, on = none;  // on: queries' product with the state of the chunk before
+    const char *pq = ws + At::kQ * 4 + wave * KC * NQ * 1024, *pp = ws + At::kP * 4 + unit_of(wave) * 3072, *pv = ws + vec_at;
+    auto fetch_q = [&] {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) *reinterpret_cast<float*>(ob + (long)i * o_sl * 4 + mine) = out[i];
-      } else {
+      for (int r = 0; r < KC; ++r)
+#pragma unroll
+        for (int j = 0; j < NQ; ++j) qx[r][j] = operand_at(pq, r * NQ + j);
+      gq = *reinterpret_cast<const f32x4*>(pv + (unsigned)(wave * 16 + quad * 4) * 4u);
+    };
+    auto fetch_p = [&] {
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        if (s <= pieces) {  // (uniform)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) p[s][j] = operand_at(pp, s * 3 + j);
+        }
+    };
+    bf16x8 us[2][3];
+    auto read_u = [&] {
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        if (s <= pieces) {  // (uniform)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) us[s][j] = s_u[s][j][lane];
+        }
+    };
+    // P U behind `on`
+    auto finish = [&] {
+      f32x4 sum[2] = {on, none};
+      product(p[0], us[0], sum);
+      if (pieces > 0) product(p[1], us[1], sum);  // (uniform)
+      return sum[0] + sum[1];
+    };
+    auto store = [&](int n, const f32x4& out) {
+      const int left = a.L - (a.c0 + n) * kDc;
+      char* ob = o + (long)n * kDc * o_sl;
+      if (col_in) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          if (wave * 16 + quad * 4 + i < left) *reinterpret_cast<float*>(ob + (long)i * o_sl * 4 + mine) = out[i];
+          if (left >= kDc || wave * 16 + quad * 4 + i < left) *reinterpret_cast<float*>(ob + (long)i * o_sl + mine) = out[i];
       }
+    };
+    // The workgroups of a head, which share an L2 where the heads are a multiple of the dies, ask together for every line of the chunk after
+    // next, a word each: what the registers hold ahead is less than the way from memory takes (fp32, d = 128: 243 -> 206 us).
+    const int lines = (int)((per + 127) / 128), first = (ct * 4 + wave) * 64 + lane, every = (int)gridDim.y * 256;
+    unsigned seen = 0;
+    auto touch = [&](int n) {
+      if (n >= a.span) return;  // (uniform)
+      const char* chunk = ws + (long)n * per;
+      for (int line = first; line < lines; line += every) seen = *reinterpret_cast<const unsigned*>(chunk + (unsigned)line * 128u);
+    };
+    fetch_q();
+    for (int n = 0; n < a.span; ++n) {
+      asm volatile("" ::"v"(seen));
+      touch(n + 2);
+      lds_barrier();  // the state is there, and the U of the chunk before
+      bf16x8 s0[KC][3];
+#pragma unroll
+      for (int r = 0; r < KC; ++r)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) s0[r][j] = s_s[r][j][lane];
+      if (n > 0) read_u();
+      f32x4 oo[2] = {none, none};
+#pragma unroll
+      for (int r = 0; r < KC; ++r) {
+        bf16x8 x[NP];
+        if constexpr (NP == 1)
+          x[0] = qx[r][0];
+        else
+          parts8(__builtin_bit_cast(f32x4, qx[r][0]), __builtin_bit_cast(f32x4, qx[r][1]), x);
+        product(x, s0[r], oo);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      lds_barrier();  // (the state and U may be written)
+      if (n > 0) store(n - 1, finish());
+      on = gq * (oo[0] + oo[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_p();
+      pp += per, pq += n + 1 < a.span ? per : 0, pv += n + 1 < a.span ? per : 0;
+      fetch_q();
+      __builtin_amdgcn_sched_barrier(0);
     }
+    lds_barrier();  // the last U is there
+    read_u();
+    store(a.span - 1, finish());
   }
-#pragma unroll
-  for (int x = 0; x < RBW; ++x)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = (wave + 4 * x) * 16 + quad * 4 + i;
-      if (col_in && row < a.d) st[(long)row * a.dvp] = S[x][i];
-    }
 }
 
 // Workspace: the chunks of one launch pair.  Long prompts go through it in spans of chunks, the state carried on in between.
 constexpr int64_t kDcWorkFloats = 64ll << 20;  // 256 MB, which the last-level cache holds between the two launches
 
-// Where chunks are the faster form: few heads, and enough chunks.  A chunk step of the scan takes 1.5 us (2.7 with heads of more than 64
+// Where chunks are the faster form: few heads, and enough chunks.  A chunk step of the scan takes 1.3 us (1.6 with heads of more than 64
 // channels, which fill eight tiles whatever their size) where four blocks of 16 take 3.2 to 6.8, by the size of the heads; but both
 // launches together start 8 to 10 us later than those of the blocks, values of many tiles read every chunk's rows once each, and every head
 // adds 20 to 90 ns of preparation a chunk: 26 times a block's products, and more memory than the cache holds at the far end.  us, blocks
-// of 16 against chunks, heads, d x dv:
+// of 16 against chunks as they were with fp32 products (bf16 chunks take 0.57 to 0.83 of that since, fp32 0.8 to 1.02), heads, d x dv:
 //   8, 64 x 64: L = 256: 27.7, 24.0.  32, 64 x 128: L = 256: 29, 28; L = 2048: 161, 91.  64, 64 x 128: L = 256: 33, 35; L = 384: 45, 43.
 //   64, 32 x 128: L = 512: 47, 48; L = 2048: 154, 170.  8, 64 x 512: L = 256: 30, 34; L = 384: 39, 38.
 //   8, 96 x 96: L = 256: 41, 35.  32, 96 x 256: L = 384: 59, 61; L = 1024: 131, 121.  64, 96 x 128: L = 512: 75, 77; L = 2048: 263, 298.
@@ -596,7 +785,7 @@ static int dc_tiles(int64_t D) { return D <= 64 ? 4 : 8; }
 static int64_t dc_span(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
   if (B <= 0 || L <= 0 || H <= 0 || D <= 0 || DV <= 0 || B >= (1ll << 31) || H >= (1ll << 31) || DV >= (1ll << 20) || !dc_faster(B, L, H, D, DV))
     return 0;
-  const int64_t chunks = (L + kDc - 1) / kDc, each = B * H * dc_floats(dc_tiles(D), (int)DV);
+  const int64_t chunks = (L + kDc - 1) / kDc, each = B * H * dc_floats(dc_tiles(D), 3, (int)DV);
   int64_t span = kDcWorkFloats / each;  // (at least 29: a chunk of 64 heads and 512 value tiles takes 2.3 M floats at most)
   if (span > chunks) span = chunks;
   // spans of about equal length
@@ -611,12 +800,13 @@ static bool dc_vec(const void* q, const void* k, int64_t B, int64_t D, int64_t x
 static bool dc_near(int64_t H, int64_t DV, int64_t x_sl) { return x_sl >= 0 && x_sl < (1ll << 24) && H * DV < (1ll << 25); }
 
 template <typename T, int RB, int LAY> static int run_delta_chunks(DeltaChunkArgs a, int64_t span, hipStream_t s) {
+  constexpr int NP = sizeof(T) == 2 ? 1 : 3;
   const int chunks = (a.L + kDc - 1) / kDc;
   for (int c = 0; c < chunks; c += (int)span) {
     a.c0 = c;
     a.span = chunks - c < span ? chunks - c : (int)span;
     hipLaunchKernelGGL((delta_chunk_prepare_kernel<T, LAY, RB>), dim3((unsigned)((long)a.B * a.H * a.span)), dim3(256), 0, s, a);
-    hipLaunchKernelGGL((delta_chunk_scan_kernel<RB>), dim3((unsigned)(a.B * a.H), (unsigned)((a.dv + 15) / 16)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((delta_chunk_scan_kernel<RB, NP>), dim3((unsigned)(a.B * a.H), (unsigned)((a.dv + 15) / 16)), dim3(512), 0, s, a);
     const int rc = check_launch("gated_delta_scan_chunks");
     if (rc) return rc;
     a.fresh = 0;
@@ -639,7 +829,7 @@ template <typename T> static int run_delta(const DeltaChunkArgs& a, bool vec, in
 extern "C" BASED_API int64_t based_gated_delta_scan_work(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
   using namespace based;
   const int64_t span = dc_span(B, L, H, D, DV);
-  return span == 0 ? 0 : B * H * span * dc_floats(dc_tiles(D), (int)DV);
+  return span == 0 ? 0 : B * H * span * dc_floats(dc_tiles(D), 3, (int)DV);
 }
 
 extern "C" BASED_API int64_t based_gated_delta_scan_work_of(const void* q, const void* k, int64_t B, int64_t L, int64_t H, int64_t D,
@@ -670,7 +860,7 @@ extern "C" BASED_API int based_gated_delta_scan_chunks(const void* q, const void
   BASED_REQUIRE(span > 0 && B * H * span < (1ll << 31), BASED_ERR_SHAPE, "%s: the shape is for blocks of 16", who);
   const bool vec = dc_vec(q, k, B, D, x_sb, x_sl);
   BASED_REQUIRE(vec || D <= 64, BASED_ERR_ALIGN, "%s: chunks of heads of more than 64 channels take rows of whole 16-byte pieces", who);
-  const DeltaChunkArgs a{q, k, v, a_gate, b_gate, a_log, dt_bias, state, o, work, (long)dc_floats(dc_tiles(D), (int)DV), (int)B, (int)L, (int)H,
+  const DeltaChunkArgs a{q, k, v, a_gate, b_gate, a_log, dt_bias, state, o, work, (long)dc_floats(dc_tiles(D), io_dtype == BASED_BF16 ? 1 : 3, (int)DV), (int)B, (int)L, (int)H,
                          (int)G, (int)D, (int)DV, (int)state_row, 0, 0, x_sb, x_sl, g_sb, g_sl, fresh,
                          DV % 4 == 0 && (B == 1 || x_sb % 4 == 0) && x_sl % 4 == 0 && aligned_to(v, 16)};
   hipStream_t s = static_cast<hipStream_t>(stream);

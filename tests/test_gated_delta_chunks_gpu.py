@@ -155,3 +155,24 @@ def test_batch_stride_of_one_sequence(dev):
     o, S = run((x, *gates), H, H, d, dv, empty_state(1, H, d, dv, dev))
     ref, S_ref = reference(x, *gates, H, H, d, dv)
     assert rel_l2(o, ref) < TOL and rel_l2(S, S_ref) < TOL
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d,dv", [(64, 64), (128, 40)])
+@pytest.mark.parametrize("scale", [1e-24, 1e24])
+def test_parts_of_small_and_large_values(dev, dtype, d, dv, scale):
+    """32 bits of a state and of values whose smallest parts (2^-16 of them) are near the ends of the format, an element of 64 in 1,000 times
+    the others; states that go on."""
+    L, H = 330, 3
+    x, *gates = make(9, 2, L, H, H, d, dv, dtype)
+    x[..., 2 * H * d:] *= scale
+    x[..., 2 * H * d::64] *= 1000
+    case = [t.to(dev) for t in (x, *gates)]
+    assert in_chunks(2, L, H, d, dv)
+    state = empty_state(2, H, d, dv, dev)
+    S_ref = None
+    for fresh in (True, False):
+        o, S = run(case, H, H, d, dv, state, fresh=fresh)
+        ref, S_ref = reference(*case, H, H, d, dv, S_ref)
+        # (norms of 1e-24 have no squares in 32 bits)
+        assert rel_l2(o.double() / scale, ref / scale) < TOL and rel_l2(S.double() / scale, S_ref / scale) < TOL
