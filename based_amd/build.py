@@ -78,8 +78,8 @@ def _compile(src: str):
 
 # Sources a group of models needs, for a machine that serves nothing else: `build_part`.
 PARTS = {
-    "streaming": ("capi", "decay_scan", "decode_linear", "experts", "gated_conv", "gated_delta", "gated_delta_chunk", "greedy", "latent_attn", "rglru",
-                  "stream_norm_conv", "token_mix", "window_attn"),
+    "streaming": ("capi", "decay_scan", "decode_linear", "experts", "gated_conv", "gated_delta", "gated_delta_chunk", "greedy", "latent_attn",
+                  "prompt_linear", "rglru", "stream_norm_conv", "token_mix", "window_attn"),
 }
 
 

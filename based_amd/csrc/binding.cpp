@@ -77,6 +77,7 @@ Listed kEntries[] = {
     BASED_ENTRY(based_short_conv_step),
     BASED_ENTRY(based_add_rms_norm),
     BASED_ENTRY(based_swiglu),
+    BASED_ENTRY(based_prompt_linear),
     BASED_ENTRY(based_greedy_step),
     BASED_ENTRY(based_decode_linear),
     BASED_ENTRY(based_decode_linear_stream),

@@ -8,6 +8,8 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
+from ..linear import Linear
+
 
 class ShortConvolution(nn.Module):
     def __init__(self, d_model: int, kernel_size: int, layer_idx=None, conv_bias: bool = False,
@@ -68,8 +70,8 @@ class BaseConv(nn.Module):
         self.l_max = l_max
         self.layer_idx = layer_idx
         self.d_inner = expand_proj * d_model // 2
-        self.in_proj = nn.Linear(d_model, expand_proj * d_model, bias=use_bias, device=device, dtype=dtype)
-        self.out_proj = nn.Linear(self.d_inner, d_model, bias=use_bias, device=device, dtype=dtype)
+        self.in_proj = Linear(d_model, expand_proj * d_model, bias=use_bias, device=device, dtype=dtype)
+        self.out_proj = Linear(self.d_inner, d_model, bias=use_bias, device=device, dtype=dtype)
         self.conv = ShortConvolution(self.d_inner, kernel_size=kernel_size, layer_idx=(layer_idx, "conv"),
                                      device=device, dtype=dtype)
 

@@ -8,9 +8,9 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from .. import ops
+from ..linear import linear
 from .streaming import cached, portion_start
 from .window_attention import _ExactRotary
 
@@ -80,7 +80,7 @@ class LatentAttention(nn.Module):
         ops.latent_write(x, self.norm_weight, cache, start, self.norm_eps, rope)
         # keys and values of every row that the portion sees; positions count from the first of them
         lo = max(0, start - self.window + 1)
-        kv = F.linear(cache[:, lo:start + L], self.expand).view(B, start + L - lo, self.heads, -1)
+        kv = linear(cache[:, lo:start + L], self.expand).view(B, start + L - lo, self.heads, -1)
         if rope is not None:
             rope = (rope[0][lo:], rope[1][lo:], rope[2])
         ops.window_attn_attend(q, kv, self.heads, self.heads, self.rot_dim + self.dim, self.window, self.scale, start - lo, rope, out_scale,

@@ -16,6 +16,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import ops
+from ..linear import Linear
 from ..generation import InferenceParams
 
 
@@ -101,10 +102,10 @@ class LinearAttention(nn.Module):
                 "the HIP kernels implement the TaylorExp feature map with feature_dim=16 only")
         self.feature_map = feature_map
 
-        self.proj_q = nn.Linear(self.d_model, self.feature_dim * self.num_heads, bias=False, **factory_kwargs)
-        self.proj_k = nn.Linear(self.d_model, self.feature_dim * self.num_heads, bias=False, **factory_kwargs)
-        self.proj_v = nn.Linear(self.d_model, self.num_heads * self.head_dim, bias=False, **factory_kwargs)
-        self.out_proj = nn.Linear(self.num_heads * self.head_dim, self.d_model, bias=False, **factory_kwargs)
+        self.proj_q = Linear(self.d_model, self.feature_dim * self.num_heads, bias=False, **factory_kwargs)
+        self.proj_k = Linear(self.d_model, self.feature_dim * self.num_heads, bias=False, **factory_kwargs)
+        self.proj_v = Linear(self.d_model, self.num_heads * self.head_dim, bias=False, **factory_kwargs)
+        self.out_proj = Linear(self.num_heads * self.head_dim, self.d_model, bias=False, **factory_kwargs)
 
     def forward(self, hidden_states: torch.Tensor, inference_params: InferenceParams = None, *args, **kwargs):
         """hidden_states (b, l, d_model) -> (b, l, d_model)."""

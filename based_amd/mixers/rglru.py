@@ -7,6 +7,7 @@ import torch
 import torch.nn as nn
 
 from .. import ops
+from ..linear import Linear
 from .streaming import StreamConv, cached, portion_start, project, round_up
 
 
@@ -20,7 +21,7 @@ class RGLRU(nn.Module):
         self.width, self.blocks, self.decay_scale, self.layer_idx = width, blocks, decay_scale, layer_idx
         self.x_off = round_up(width)  # rows of in_proj: y, then x
         n = width // blocks
-        self.in_proj = nn.Linear(d_model, 2 * self.x_off, bias=bias, **fk)
+        self.in_proj = Linear(d_model, 2 * self.x_off, bias=bias, **fk)
         self.conv = StreamConv(width, conv_taps, bias=bias, layer_idx=layer_idx, name="conv", **fk)
         self.gate_r = nn.Parameter(torch.empty(blocks, n, n, **fk))   # [out, in]
         self.gate_i = nn.Parameter(torch.empty(blocks, n, n, **fk))
@@ -29,7 +30,7 @@ class RGLRU(nn.Module):
         self.bias_r = nn.Parameter(torch.zeros(width, **fk))
         self.bias_i = nn.Parameter(torch.zeros(width, **fk))
         self.lam = nn.Parameter(torch.full((width,), -3.0, **fk))
-        self.out_proj = nn.Linear(self.x_off, d_model, bias=False, **fk)
+        self.out_proj = Linear(self.x_off, d_model, bias=False, **fk)
 
     def allocate_state(self, batch_size: int, max_seqlen: int = 0, dtype=None):
         return torch.zeros(batch_size, self.width, device=self.lam.device, dtype=torch.float32)

@@ -10,6 +10,7 @@ import torch
 import torch.nn as nn
 
 from .. import ops
+from ..linear import Linear
 from .streaming import project, round_up
 
 
@@ -37,8 +38,8 @@ class SideBySide(nn.Module):
             self.out_cols.append((col, core.out_features))
             col += round_up(core.out_features)
         self._gaps = any(core.out_features % 8 for core in self.cores)
-        self.in_proj = nn.Linear(d_model, row, bias=False, **fk)
-        self.out_proj = nn.Linear(col, d_model, bias=False, **fk)
+        self.in_proj = Linear(d_model, row, bias=False, **fk)
+        self.out_proj = Linear(col, d_model, bias=False, **fk)
 
     def allocate_inference_cache(self, batch_size: int, max_seqlen: int, dtype=None, **kwargs):
         return {name: make(batch_size, max_seqlen) for core in self.cores for name, make in core.allocations().items()}

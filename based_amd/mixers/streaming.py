@@ -10,9 +10,9 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from .. import ops
+from ..linear import linear as linear_of
 
 
 def round_up(n: int, to: int = 8) -> int:
@@ -20,7 +20,7 @@ def round_up(n: int, to: int = 8) -> int:
 
 
 def project(x, linear: nn.Linear):
-    return F.linear(x, linear.weight, linear.bias)
+    return linear_of(x, linear.weight, linear.bias)
 
 
 def portion_start(inference_params, batch: int, seqlen: int):

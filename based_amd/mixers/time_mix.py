@@ -5,9 +5,9 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from .. import ops
+from ..linear import Linear, linear
 from .streaming import cached, portion_start, project, round_up
 
 
@@ -26,12 +26,12 @@ class TimeMix(nn.Module):
         self.width = heads * dim
         self.segment = round_up(self.width, self.SEGMENT)
         self.mu = nn.Parameter(torch.full((len(self.MIXES), d_model), 0.5, **fk))
-        self.in_proj = nn.Linear(d_model, 4 * self.segment + round_up(rank), bias=False, **fk)
+        self.in_proj = Linear(d_model, 4 * self.segment + round_up(rank), bias=False, **fk)
         self.w2 = nn.Parameter(torch.empty(self.width, rank, **fk).normal_(std=0.1))
         self.w0 = nn.Parameter(torch.full((self.width,), -3.0, **fk))
         self.bonus = nn.Parameter(torch.zeros(heads, dim, **fk))
         self.norm_weight = nn.Parameter(torch.ones(self.width, **fk))
-        self.out_proj = nn.Linear(round_up(self.width), d_model, bias=False, **fk)
+        self.out_proj = Linear(round_up(self.width), d_model, bias=False, **fk)
 
     def allocate_state(self, batch_size: int, max_seqlen: int = 0, dtype=None):
         return torch.zeros(batch_size, self.heads, self.dim, round_up(self.dim, 4), device=self.mu.device, dtype=torch.float32)
@@ -80,7 +80,7 @@ class TimeMix(nn.Module):
         start, step = portion_start(inference_params, B, L)
         state, ring = self._cached(inference_params, B)
         mixed = ops.token_mix(x, self.mu, ring, start)
-        r, k, v, g, hidden = (F.linear(mixed[i], self.in_proj.weight[self._rows(i)]) for i in range(len(self.MIXES)))
+        r, k, v, g, hidden = (linear(mixed[i], self.in_proj.weight[self._rows(i)]) for i in range(len(self.MIXES)))
         if step:
             return project(self._step(r[:, 0], k[:, 0], v[:, 0], g[:, 0], hidden[:, 0], state, start), self.out_proj).unsqueeze(1)
         decay = ops.channel_decay(hidden, self.w2, self.w0)

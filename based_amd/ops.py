@@ -567,8 +567,13 @@ def add_rms_norm(x, residual, weight, eps: float = 1e-5, residual_in_fp32: bool 
     return y.view(x.shape), (out.view(x.shape) if out is not None else None)
 
 
-def swiglu(u) -> torch.Tensor:
-    """u (..., 2F) -> u[..., :F] * silu(u[..., F:]), one pass."""
+def swiglu(u, weight=None, bias=None) -> torch.Tensor:
+    """u (..., 2F) -> u[..., :F] * silu(u[..., F:]), one pass.  weight (2F, K) (and bias): u (..., K) goes through that projection first, in the
+    same launch where `prompt_linear` is the faster form."""
+    if weight is not None:
+        if linear_form(u, weight, bias) == LINEAR_PROMPT and weight.shape[0] % 8 == 0:
+            return _prompt_linear(u, weight, bias, weight.shape[0] // 2, True)
+        u = linear(u, weight, bias)
     _require_cuda(u)
     F2 = u.shape[-1]
     if F2 % 2 != 0:
@@ -582,6 +587,80 @@ def swiglu(u) -> torch.Tensor:
         _lib.check(_lib.lib().based_swiglu(u2.data_ptr(), out.data_ptr(), u2.shape[0], F, u2.stride(0), out.stride(0),
                                            _dtype_code(u), _stream_ptr(u)))
     return out.view(*u.shape[:-1], F)
+
+
+LINEAR_LIBRARY, LINEAR_PROMPT, LINEAR_ROWS = 0, 1, 2
+PROMPT_LINEAR_MAX_ROWS = 512
+
+
+def linear_form(x, weight, bias=None) -> int:
+    """Which of its forms `linear` takes.  The library's call costs the host 19 to 21 us, the two others 7.5, and a prompt of a few hundred tokens
+    waits for the host; us on the GPU, weights from memory, library against prompt_linear, N x K: 4096 x 1024, 33 to 512 rows 11 - 13 against 6.8 - 11.9
+    (777 rows: 14.5, 20.7); 1024 x 1024 8.1 - 8.5, 6.1 - 6.6; 1024 x 2048 8.1 - 9.5, 8.6 - 9.1; 3072 x 768 7.0 - 9.4, 5.6 - 9.5; 50280 x 1024, 64 rows
+    26, 36: one tile for each of the 256 compute units at most.  Up to 8 rows the kernel of the single-token steps (4096 x 1024, 4 rows: 7.6, 6.6, here
+    4.3; 50280 x 1024, 4 rows 23.7, here 23.3, 8 rows 23.7, here 25.6)."""
+    key = ("linear", x.shape, x.stride(), x.dtype, x.device, weight.shape, weight.stride(), weight.dtype, weight.device,
+           None if bias is None else (bias.shape, bias.stride(), bias.dtype, bias.device))
+    form = _CHECKED.get(key)
+    if form is None:
+        form = LINEAR_LIBRARY
+        if (x.is_cuda and x.dim() > 1 and x.dtype == weight.dtype == torch.bfloat16 and weight.dim() == 2 and x.shape[-1] == weight.shape[1]
+                and x.device == weight.device and weight.stride(1) == 1 and weight.stride(0) % 8 == 0
+                and weight.stride(0) >= weight.shape[1]
+                and (bias is None or (bias.dtype == torch.bfloat16 and bias.device == x.device and bias.is_contiguous()
+                                      and tuple(bias.shape) == weight.shape[:1]))):
+            N, K = weight.shape
+            M = x.numel() // K if K else 0
+            one_each = x.dim() == 3 and x.shape[1] == 1 and x.stride(2) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= K  # (the last tokens)
+            if 0 < M <= 8 and (x.is_contiguous() or one_each) and K % 8 == 0 and K <= 4096 and 0 < N and (M <= 4 or N <= 16384):
+                form = LINEAR_ROWS
+            elif x.is_contiguous() and 0 < M <= PROMPT_LINEAR_MAX_ROWS and N % 4 == 0 and K % 128 == 0 and K <= 2048 and -(-M // 128) * -(-N // 64) <= 256:
+                form = LINEAR_PROMPT
+        _CHECKED[key] = form
+    if form != LINEAR_LIBRARY and ((x.data_ptr() | weight.data_ptr()) & 15 or (bias is not None and bias.data_ptr() & 7)):
+        return LINEAR_LIBRARY
+    return form
+
+
+def linear(x, weight, bias=None) -> torch.Tensor:
+    """torch.nn.functional.linear without a gradient: few rows of bf16 by the kernels here, everything else by the library."""
+    form = linear_form(x, weight, bias)
+    if form == LINEAR_LIBRARY:
+        return torch.nn.functional.linear(x, weight, bias)
+    N, K = weight.shape
+    if form == LINEAR_PROMPT:
+        return _prompt_linear(x, weight, bias, N, False)
+    y = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=x.device)
+    with _on_device(x.device):
+        _lib.check(_lib.lib().based_decode_linear(
+            x.data_ptr(), K if x.is_contiguous() else x.stride(0), None, 0, weight.data_ptr(), weight.stride(0), None if bias is None else bias.data_ptr(),
+            y.data_ptr(), N, x.numel() // K, N, K, PROLOGUE_NONE, None, 0, None, 0, None, 0.0, EPILOGUE_NONE, None, 0, None, None, 0, _stream_ptr(x)))
+    return y
+
+
+def _prompt_linear(x, weight, bias, N: int, gated: bool) -> torch.Tensor:
+    K = weight.shape[1]
+    y = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=x.device)
+    with _on_device(x.device):
+        _lib.check(_lib.lib().based_prompt_linear(x.data_ptr(), K, weight.data_ptr(), weight.stride(0), None if bias is None else bias.data_ptr(),
+                                                  y.data_ptr(), N, x.numel() // K, N, K, int(gated), _stream_ptr(x)))
+    return y
+
+
+def prompt_linear(x, weight, bias=None, gated: bool = False) -> torch.Tensor:
+    """x (..., K) bf16 through weight (N, K) (+ bias), as torch.nn.functional.linear; gated: weight (2F, K), and `swiglu` of the result.
+    K a multiple of 128, N (F) of 4."""
+    key = ("prompt_linear", gated, _form(x, weight, bias))
+    if key not in _CHECKED:
+        _require_cuda(x, weight, *(() if bias is None else (bias,)))
+        if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.dim() != 2 or weight.stride(1) != 1 or x.shape[-1:] != weight.shape[1:]:
+            raise ValueError(f"x {tuple(x.shape)} and weight {tuple(weight.shape)} must be bfloat16 rows of the contraction length")
+        if bias is not None and (tuple(bias.shape) != tuple(weight.shape[:1]) or bias.dtype != torch.bfloat16 or not bias.is_contiguous()):
+            raise ValueError(f"bias must be a contiguous bfloat16 ({weight.shape[0]},)")
+        if gated and weight.shape[0] % 2:
+            raise ValueError("a gated projection has as many gates as values")
+        _CHECKED[key] = True
+    return _prompt_linear(x.contiguous(), weight, bias, weight.shape[0] // 2 if gated else weight.shape[0], gated)
 
 
 def greedy_step(logits, next_ids, lengths, sequences=None, position_ids=None, vocab_size=None) -> None:

@@ -4,9 +4,10 @@ Just enough of based/models/gpt.py (create_mixer_cls :64-96, create_block :347-3
 :463-485, GPTModel :510-736, GPTLMHeadModel :739-827), block.py (:114-163), mlp.py (GatedMlp
 :99-157) and the RMSNorm closed form (based/ops/triton/layer_norm.py:117-118) to run the
 27-layer Based-360m shape end to end: embeddings -> [prenorm Block(mixer, SwiGLU MLP)] x N ->
-final norm -> tied LM head, with the generation cache threaded through.  The GEMMs and the
-embedding lookup are ordinary torch (hipBLASLt); mixers, add + RMSNorm and the SwiGLU gate are
-the HIP kernels, and there is no host-tensor path.
+final norm -> tied LM head, with the generation cache threaded through.  The GEMMs of
+more than a few hundred tokens and the embedding lookup are ordinary torch (hipBLASLt); those of fewer
+(`based_amd.linear`), mixers, add + RMSNorm and the SwiGLU gate are the HIP kernels, and there is no
+host-tensor path.
 """
 from __future__ import annotations
 
@@ -23,6 +24,7 @@ import torch.nn.functional as F
 from . import ops
 
 from .generation import GenerationMixin
+from .linear import Linear, swiglu
 from .mixers.convolution import BaseConv, ShortConvolution
 from .mixers.decay_attention import DecayAttention
 from .mixers.gated_delta import GatedDeltaRule
@@ -308,19 +310,19 @@ class GatedMlp(nn.Module):
         if mlp_type == "base":
             hidden_features = hidden_features if hidden_features is not None else int(8 * in_features / 3)
             hidden_features = (hidden_features + multiple_of - 1) // multiple_of * multiple_of
-            self.fc1 = nn.Linear(in_features, 2 * hidden_features, bias=bias1, **fk)
+            self.fc1 = Linear(in_features, 2 * hidden_features, bias=bias1, **fk)
         else:
             hidden_features = int(2 * in_features * ff_mult / 3)
             hidden_features = (hidden_features + multiple_of - 1) // multiple_of * multiple_of
-            self.fc1 = nn.Linear(in_features, hidden_features, bias=bias1, **fk)
-            self.fc3 = nn.Linear(in_features, hidden_features, bias=bias1, **fk)
-        self.fc2 = nn.Linear(hidden_features, in_features, bias=bias2, **fk)
+            self.fc1 = Linear(in_features, hidden_features, bias=bias1, **fk)
+            self.fc3 = Linear(in_features, hidden_features, bias=bias1, **fk)
+        self.fc2 = Linear(hidden_features, in_features, bias=bias2, **fk)
 
     def forward(self, x):
         if self.mlp_type != "base":
             return self.fc2(_GATE_ACTIVATIONS[self.activation](self.fc1(x)) * self.fc3(x))
         if self.activation == "swiglu":
-            return self.fc2(ops.swiglu(self.fc1(x)))
+            return self.fc2(swiglu(self.fc1, x))
         y, gate = self.fc1(x).chunk(2, dim=-1)
         return self.fc2(y * _GATE_ACTIVATIONS[self.activation](gate))
 
@@ -354,8 +356,8 @@ class TokenSide(nn.Module):
         super().__init__()
         fk = {"device": device, "dtype": dtype}
         self.dim, self.first = dim, layer_idx * dim
-        self.gate = nn.Linear(d_model, dim, bias=False, **fk)
-        self.proj = nn.Linear(dim, d_model, bias=False, **fk)
+        self.gate = Linear(d_model, dim, bias=False, **fk)
+        self.proj = Linear(dim, d_model, bias=False, **fk)
         self.norm = StreamNorm(d_model, eps=eps, kind="rms", **fk)
 
     def table(self, side_table):
@@ -665,7 +667,7 @@ class GPTLMHeadModel(nn.Module, GenerationMixin):
         self.config = config
         self.transformer = GPTModel(config, device=device, dtype=dtype)
         vocab = self.transformer.embeddings.word_embeddings.num_embeddings
-        self.lm_head = nn.Linear(config.n_embd, vocab, bias=False, device=device, dtype=dtype)
+        self.lm_head = Linear(config.n_embd, vocab, bias=False, device=device, dtype=dtype)
         self.apply(partial(_init_weights, n_layer=config.num_hidden_layers,
                            initializer_range=config.initializer_range))
         if config.tie_word_embeddings:

@@ -337,6 +337,12 @@ BASED_API int based_add_rms_norm(const void* x, const void* residual_in, const v
 BASED_API int based_swiglu(const void* u, void* out, int64_t rows, int64_t F, int64_t u_sr, int64_t o_sr,
                  int io_dtype, void* stream);
 
+/* Projections of a short prompt: y = x w^T (+ bias) in bf16 with fp32 sums, x (M, K), w (N, K), y (M, N).  gated: w is (2N, K), bias (2N) and
+ * y[:, f] = p[:, f] silu(p[:, N + f]) of p = x w^T + bias rounded to bf16, as based_swiglu gives it.  K a multiple of 128, N of 4; rows of x and w
+ * in whole 16-byte pieces; bias may be null. */
+BASED_API int based_prompt_linear(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride, const void* bias, void* y,
+                                  int64_t y_row_stride, int64_t M, int64_t N, int64_t K, int gated, void* stream);
+
 /*
  * A projection of a single-token step, with the element-wise operation in front of it:
  *
