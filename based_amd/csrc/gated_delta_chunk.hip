@@ -97,11 +97,6 @@ __device__ __forceinline__ void parts8(const f32x4& x, const f32x4& y, bf16x8 (&
   for (int n = 0; n < 3; ++n) o[n] = __builtin_bit_cast(bf16x8, u32x4{a[n][0], a[n][1], b[n][0], b[n][1]});
 }
 
-__device__ __forceinline__ bf16x4 read_transposed(const __bf16* p) {
-  typedef __attribute__((address_space(3))) bf16x4 shared4;
-  return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((shared4*)p);
-}
-
 __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
 // x y added to sum[0], the products that are at most 2^-8 of it to sum[1]: NX and NY parts.

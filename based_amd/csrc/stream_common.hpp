@@ -112,6 +112,12 @@ __device__ __forceinline__ float sum_quads4(float a, float b, float c, float d) 
   return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
 }
 
+// Four rows of 16 elements in LDS, whose 8-byte pieces the lanes of each group of 16 name in turn: lane l receives element l of every row.
+__device__ __forceinline__ bf16x4 read_transposed(const __bf16* p) {
+  typedef __attribute__((address_space(3))) bf16x4 shared4;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((shared4*)p);
+}
+
 inline bool aligned_to(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
 
 // Sum of w_j x_{t - taps + 1 + j} over the past inputs of one channel of a ring (taps slots, `stride` elements

@@ -36,6 +36,7 @@ struct WindowArgs {
   long kv_sb, kv_st;
   int rot, half_split, window, norm_v;
   float scale, eps, out_scale;
+  uint32_t heads_inv;  // 2^32 / (H / G), rounded down (window_prefill_mfma)
 };
 
 // partner and sign of channel c in the rotation: x'_c = x_c cos + sgn * x_partner sin
@@ -161,54 +162,53 @@ __global__ __launch_bounds__(256) void window_kv_write_vec_kernel(const WindowAr
 // channels past the real sizes are zeros).
 constexpr int kTileKeys = 64;
 constexpr int kTileRows = 128;  // (token, head) rows per workgroup
+constexpr int kDirectTile = kTileKeys * 128;  // elements of a tile of keys and values of 64 channels
 
-// Bound by the vector unit and by waiting for the tiles: as many wavefronts as fit.  Sizes up to 64 run in 128 registers, four
-// workgroups to a compute unit (three, with 143, and the maxima of rows exchanged through LDS; 2.3 wavefronts on a SIMD on average, 1.9): 16 heads on
-// 4 of 64 channels, with the cache write, 4 x 2048 tokens and 129 keys 28.9 -> 24.8 us; on 16 44.4 -> 39.5; 6 x 2240 tokens and 513 keys 81.8 ->
-// 73.9; one of 700 26.2 -> 23.1.
+// Bound by the vector unit, and in short windows by a workgroup's own start (queries, tables, first tile: 11 of 30 thousand cycles where all
+// workgroups run together).  As many wavefronts as fit: sizes up to 64 run in 128 registers, four workgroups to a compute unit (three, with
+// 143: 28.9 us where four take 24.8).  What a wavefront sees is worked out on the scalar unit, so that only tiles at the edges of a window are
+// masked; the lanes of a row look for their largest score together only where one of them has found a larger; weights are summed on the matrix unit;
+// and rows of 64 channels go straight into LDS.  Kernels alone, 16 heads of 64 channels, with the cache write, without and with these: on 4, 4 x 2048
+// tokens and 129 keys 31.7 / 30.1 us; 6 x 2240 and 513 keys 77.3 / 64.8; on 2, 4 x 4096 and 1,024 keys 140 / 112; on 16, 1 x 2048 and 1,024 keys
+// 47.4 / 38.4; 1 x 700 12.4 / 11.3.
 
 __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-template <int KC, int VC, bool HALF>
+// DIRECT: keys and values of 64 channels each, straight into LDS, the next tile while one is worked on.  Piece p (16 bytes) of row r lies at
+// p ^ (r / 2 % 8), of values at p ^ (r / 2 % 4 * 2), so that reads of 16 rows (transposing reads of 8) meet every bank once; one barrier a tile.
+template <int KC, int VC, bool HALF, bool DIRECT>
 __global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 3 : 1) void window_prefill_mfma_kernel(const WindowArgs a) {
   constexpr int D = KC * 32, DV = VC * 32;
   constexpr int KS = D + 8, VS = kTileKeys + 8;  // LDS row strides: 16-lane reads of 16 bytes meet every bank once
-  __shared__ __attribute__((aligned(16))) __bf16 lds_k[kTileKeys * KS];
-  __shared__ __attribute__((aligned(16))) __bf16 lds_v[DV * VS];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4;
-  const int bg = blockIdx.y, b = bg / a.G, g = bg % a.G;
-  const int qpk = a.H / a.G;
+  static_assert(!DIRECT || (KC == 2 && VC == 2), "rows of 64 channels");
+  __shared__ __attribute__((aligned(16))) __bf16 lds_k[DIRECT ? 8 : kTileKeys * KS];
+  __shared__ __attribute__((aligned(16))) __bf16 lds_v[DIRECT ? 8 : DV * VS];
+  // (an array whose extent the launch gives: in front of every read of a static one the compiler waits for all loads that go to LDS)
+  extern __shared__ __attribute__((aligned(16))) __bf16 lds_tiles[];
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (what a wavefront sees is worked out once for it, on the scalar unit)
+  const int g = blockIdx.y, b = blockIdx.z;
+  const int qpk = (int)((uint32_t)a.H / (uint32_t)a.G);
   const int n_rows = a.L * qpk;
+  // token of a (token, head) row, and the head: a product with the rounded inverse is the quotient or one less
+  const auto token_of = [&](int row, int* head) {
+    uint32_t tok = __umulhi((uint32_t)row, a.heads_inv), rest = (uint32_t)row - tok * (uint32_t)qpk;
+    if (rest >= (uint32_t)qpk) ++tok, rest -= (uint32_t)qpk;
+    if (head) *head = (int)rest;
+    return (int)tok;
+  };
   const int r0 = blockIdx.x * kTileRows;
   const int r_end = r0 + kTileRows < n_rows ? r0 + kTileRows : n_rows;
   const int row_w = r0 + wave * 32;  // first row of this wavefront
   const __bf16* kv = static_cast<const __bf16*>(a.kv) + b * a.kv_sb + (long)g * (a.d + a.dv);
 
-  // queries: lane holds channels quad*8 + 32 c .. of row l16 (+16): the MFMA's second operand.  Turned and
-  // rounded after the first tile of keys has been asked for.
-  bf16x8 qf[2][KC];
-  int qpos[2];
-  const __bf16* qrow[2];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int row = row_w + t * 16 + l16;
-    const int rr = row < n_rows ? row : n_rows - 1;
-    const int tok = rr / qpk;
-    qpos[t] = a.pos_host + tok;
-    qrow[t] = static_cast<const __bf16*>(a.q) + b * a.q_sb + tok * a.q_sl + (long)(g * qpk + rr - tok * qpk) * a.d;
-#pragma unroll
-    for (int c = 0; c < KC; ++c) {
-      const int e = c * 32 + quad * 8;
-      qf[t][c] = *reinterpret_cast<const bf16x8*>(qrow[t] + (e < a.d ? e : 0));
-    }
-  }
-  const int wave_lo_tok = a.pos_host + (row_w < n_rows ? row_w : n_rows - 1) / qpk;
+  const int wave_lo_tok = a.pos_host + token_of(row_w < n_rows ? row_w : n_rows - 1, nullptr);
   const int wave_hi_row = row_w + 31 < n_rows ? row_w + 31 : n_rows - 1;
-  const int wave_hi_tok = a.pos_host + wave_hi_row / qpk;
+  const int wave_hi_tok = a.pos_host + token_of(wave_hi_row, nullptr);
 
-  const int first_pos = a.pos_host + r0 / qpk, last_pos = a.pos_host + (r_end - 1) / qpk;
+  const int first_pos = a.pos_host + token_of(r0, nullptr), last_pos = a.pos_host + token_of(r_end - 1, nullptr);
   const int lo = first_pos - a.window + 1 > 0 ? first_pos - a.window + 1 : 0;
 
   // staging: keys as 16-byte pieces of rows; values as VK keys x 8 channels, turned on the way
@@ -217,11 +217,23 @@ __global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 
   constexpr int VP = VN * (DV / 8) / 256 > 0 ? VN * (DV / 8) / 256 : 1;
   typedef __attribute__((ext_vector_type(VK))) __bf16 bf16xk;
   typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
-  u32x4 kbuf[KP];
-  u32x4 vbuf[VP][VK];
+  u32x4 kbuf[DIRECT ? 1 : KP];
+  u32x4 vbuf[DIRECT ? 1 : VP][VK];
   const u32x4 zero4 = {0u, 0u, 0u, 0u};
   // rows past the last key and channels past the sizes are fetched from valid places and cleared in `stage`
   const int st32 = (int)a.kv_st;
+  auto ask = [&](int k0, int place) {
+    const __bf16* tile = kv + (long)k0 * a.kv_st;
+    const int last = last_pos - k0;
+    __bf16* to = lds_tiles + place * kDirectTile;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int group = wave * 4 + i, row = (group & 7) * 8 + (lane >> 3);  // 8 rows; keys, then values
+      const int piece = group < 8 ? (lane & 7) ^ (row >> 1 & 7) : 8 + ((lane & 7) ^ (row >> 1 & 3) * 2);
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(tile + ((row <= last ? row : last) * st32 + piece * 8)),
+                                       (__attribute__((address_space(3))) void*)(to + group * 512), 16, 0, 0);
+    }
+  };
   auto fetch = [&](int k0) {
     const __bf16* tile = kv + (long)k0 * a.kv_st;
     const int last = last_pos - k0;
@@ -263,7 +275,27 @@ __global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 
     }
   };
 
-  fetch(lo);
+  if constexpr (DIRECT) ask(lo, 0);
+  // queries: lane holds channels quad*8 + 32 c .. of row l16 (+16): the MFMA's second operand.  Turned and
+  // rounded after the first tile of keys has been asked for.
+  bf16x8 qf[2][KC];
+  int qpos[2];
+  const __bf16* qrow[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int row = row_w + t * 16 + l16;
+    const int rr = row < n_rows ? row : n_rows - 1;
+    int head;
+    const int tok = token_of(rr, &head);
+    qpos[t] = a.pos_host + tok;
+    qrow[t] = static_cast<const __bf16*>(a.q) + b * a.q_sb + tok * a.q_sl + (long)(g * qpk + head) * a.d;
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      const int e = c * 32 + quad * 8;
+      qf[t][c] = *reinterpret_cast<const bf16x8*>(qrow[t] + (e < a.d ? e : 0));
+    }
+  }
+  if constexpr (!DIRECT) fetch(lo);
   if (a.rot > 0) {
     constexpr int CB = KC == 3 || (HALF && KC == 2) ? 1 : KC < 4 ? KC : 4;
 #pragma unroll
@@ -310,19 +342,38 @@ __global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int i = 0; i < 2 * VC; ++i) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
+  float m_run[2] = {-INFINITY, -INFINITY};
+  // Sums of the weights as they enter the products, on the matrix unit too: rows of ones times the weights.  A weight's rounding then moves both and
+  // leaves the mean of the values in place (errors against 64 bits 3.098e-3 -> 3.090e-3), and the vector unit, which bounds the kernel, adds nothing.
+  f32x4 l_run[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+  bf16x8 ones;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) ones[j] = (__bf16)1.f;
   const float scale2 = fabsf(a.scale) * 1.4426950408889634f;  // scores in powers of two; the sign is the queries'
+  int place = 0;
   for (int k0 = lo; k0 <= last_pos; k0 += kTileKeys) {
-    __syncthreads();  // every wavefront is done with the tile before
-    stage();
-    __syncthreads();
-    if (k0 + kTileKeys <= last_pos) fetch(k0 + kTileKeys);
+    if constexpr (DIRECT) {
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(0x0070);  // own loads are there, own reads of the tile before are done
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      if (k0 + kTileKeys <= last_pos) ask(k0 + kTileKeys, place ^ 1);
+      __builtin_amdgcn_sched_barrier(0);
+    } else {
+      __syncthreads();  // every wavefront is done with the tile before
+      stage();
+      __syncthreads();
+      if (k0 + kTileKeys <= last_pos) fetch(k0 + kTileKeys);
+    }
+    const __bf16* tile_k = lds_tiles + place * kDirectTile;
+    const __bf16* tile_v = tile_k + kTileKeys * 64;
+    place ^= 1;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       // 32 keys at a time: does any row of this wavefront see one of them, does every row see all?
       const int kh = k0 + h * 32;
       if (kh > wave_hi_tok || kh + 31 <= wave_lo_tok - a.window) continue;
-      const bool all = kh + 31 <= wave_lo_tok && kh > wave_hi_tok - a.window;
+      const bool late = kh + 31 > wave_lo_tok, early = kh <= wave_hi_tok - a.window;  // (of some row)
       f32x4 s[2][2];
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt) {
@@ -330,7 +381,8 @@ __global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 
         for (int t = 0; t < 2; ++t) s[t][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
-          const bf16x8 kf = *reinterpret_cast<const bf16x8*>(&lds_k[(h * 32 + kt * 16 + l16) * KS + c * 32 + quad * 8]);
+          const bf16x8 kf = DIRECT ? *reinterpret_cast<const bf16x8*>(&tile_k[(h * 32 + kt * 16 + l16) * 64 + ((c * 4 + quad) ^ (l16 >> 1 & 7)) * 8])
+                                   : *reinterpret_cast<const bf16x8*>(&lds_k[(h * 32 + kt * 16 + l16) * KS + c * 32 + quad * 8]);
 #pragma unroll
           for (int t = 0; t < 2; ++t) s[t][kt] = mfma_bf16(kf, qf[t][c], s[t][kt]);
         }
@@ -338,43 +390,56 @@ __global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 
       bf16x8 pf[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        float mx = -INFINITY;
+        // (a score out of sight is minus infinity)
         const int d0 = qpos[t] - kh - quad * 4;
+        if (late) {
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+          for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            float sc = s[t][kt][i];
-            if (!all) sc = (unsigned)(d0 - kt * 16 - i) < (unsigned)a.window ? sc : -INFINITY;
-            s[t][kt][i] = sc;
-            mx = fmaxf(mx, sc);
-          }
-        mx = max_quads(mx);
-        if (__any(mx > m_run[t])) {
+            for (int i = 0; i < 4; ++i) s[t][kt][i] = d0 >= kt * 16 + i ? s[t][kt][i] : -INFINITY;
+        }
+        if (early) {
+          const int w0 = d0 - a.window;
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[t][kt][i] = w0 < kt * 16 + i ? s[t][kt][i] : -INFINITY;
+        }
+        float mx = s[t][0][0];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) mx = fmaxf(mx, s[t][i >> 2][i & 3]);
+        if (__any(mx > m_run[t])) {  // (2^8 of slack would save 3 to 10 % of the time, and round the heaviest weight, which is one, like the others)
+          mx = max_quads(mx);
           const float m_new = fmaxf(m_run[t], mx);
           // no key seen yet: every weight is 2^-inf = 0
           const float alpha = __builtin_amdgcn_exp2f((m_run[t] - (m_new == -INFINITY ? 0.f : m_new)) * scale2);
           m_run[t] = m_new;
-          l_run[t] *= alpha;
+          l_run[t][0] *= alpha;  // (the others are the same sum, and not used)
 #pragma unroll
           for (int i = 0; i < 2 * VC; ++i) acc[t][i] *= alpha;
         }
         const float m2 = m_run[t] == -INFINITY ? 0.f : m_run[t] * scale2;
-        float sum = 0.f;
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][kt][i], scale2, -m2));
-            sum += p;
             pf[t][kt * 4 + i] = (__bf16)p;
           }
-        l_run[t] += sum;  // this lane's keys; the four lane groups are added at the end
+        l_run[t] = mfma_bf16(ones, pf[t], l_run[t]);
       }
 #pragma unroll
       for (int i = 0; i < 2 * VC; ++i) {
-        const __bf16* vp = &lds_v[(i * 16 + l16) * VS + h * 32 + quad * 4];
-        const bf16x4 v0 = *reinterpret_cast<const bf16x4*>(vp), v1 = *reinterpret_cast<const bf16x4*>(vp + 16);
+        bf16x4 v0, v1;
+        if constexpr (DIRECT) {
+          // lane l16 receives channel l16 of the four keys whose 8 bytes each its group of 16 lanes names
+          const int row = quad * 4 + (l16 >> 2);
+          const __bf16* vp = &tile_v[(h * 32 + row) * 64 + ((i * 2 + (l16 >> 1 & 1)) ^ (row >> 1 & 3) * 2) * 8 + (l16 & 1) * 4];
+          v0 = read_transposed(vp), v1 = read_transposed(vp + 16 * 64);
+        } else {
+          const __bf16* vp = &lds_v[(i * 16 + l16) * VS + h * 32 + quad * 4];
+          v0 = *reinterpret_cast<const bf16x4*>(vp), v1 = *reinterpret_cast<const bf16x4*>(vp + 16);
+        }
         const bf16x8 vf = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
         for (int t = 0; t < 2; ++t) acc[t][i] = mfma_bf16(vf, pf[t], acc[t][i]);
@@ -385,13 +450,12 @@ __global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 
   asm volatile("" : "+v"(row_end));  // (where a row goes is worked out again: kept, it would be a register too many)
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
-    float l = l_run[t];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
-    const float inv = a.out_scale / l;
-    const int row = row_end + t * 16 + l16, tok = row / qpk;
+    const float inv = a.out_scale / l_run[t][0];
+    const int row = row_end + t * 16 + l16;
+    int head;
+    const int tok = token_of(row, &head);
     if (row < n_rows) {
-      __bf16* op = static_cast<__bf16*>(a.o) + b * a.o_sb + tok * a.o_sl + (long)(g * qpk + row - tok * qpk) * a.dv;
+      __bf16* op = static_cast<__bf16*>(a.o) + b * a.o_sb + tok * a.o_sl + (long)(g * qpk + head) * a.dv;
 #pragma unroll
       for (int i = 0; i < 2 * VC; ++i) {
         const int e = i * 16 + quad * 4;
@@ -1237,23 +1301,24 @@ template <int LPI> void launch_kv_write(const WindowArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((window_kv_write_vec_kernel<LPI, false>), grid, dim3(256), 0, s, a);
 }
 
-template <int KC, int VC> void launch_window_mfma_pairs(const WindowArgs& a, dim3 grid, hipStream_t s) {
+template <int KC, int VC, bool DIRECT> void launch_window_mfma_pairs(const WindowArgs& a, dim3 grid, hipStream_t s) {
+  constexpr unsigned lds = DIRECT ? 2 * kDirectTile * sizeof(__bf16) : 0;
   if (a.half_split)
-    hipLaunchKernelGGL((window_prefill_mfma_kernel<KC, VC, true>), grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL((window_prefill_mfma_kernel<KC, VC, true, DIRECT>), grid, dim3(256), lds, s, a);
   else
-    hipLaunchKernelGGL((window_prefill_mfma_kernel<KC, VC, false>), grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL((window_prefill_mfma_kernel<KC, VC, false, DIRECT>), grid, dim3(256), lds, s, a);
 }
 
 template <int KC> void launch_window_mfma(const WindowArgs& a, dim3 grid, hipStream_t s) {
   const int vc = (a.dv + 31) / 32;
   if (vc <= 1)
-    launch_window_mfma_pairs<KC, 1>(a, grid, s);
+    launch_window_mfma_pairs<KC, 1, false>(a, grid, s);
   else if (vc <= 2)
-    launch_window_mfma_pairs<KC, 2>(a, grid, s);
+    launch_window_mfma_pairs<KC, 2, false>(a, grid, s);
   else if (vc <= 4)
-    launch_window_mfma_pairs<KC, 4>(a, grid, s);
+    launch_window_mfma_pairs<KC, 4, false>(a, grid, s);
   else
-    launch_window_mfma_pairs<KC, 8>(a, grid, s);
+    launch_window_mfma_pairs<KC, 8, false>(a, grid, s);
 }
 
 static int window_check(const char* who, const WindowArgs& a, int64_t n_rope, int io_dtype, int64_t last) {
@@ -1303,11 +1368,15 @@ static bool window_f32_few(const WindowArgs& a) {
 }
 
 // The attention of a portion whose keys and values are in place.
-static void launch_window_attend(const WindowArgs& a, bool vec, int io_dtype, hipStream_t s) {
+static void launch_window_attend(WindowArgs a, bool vec, int io_dtype, hipStream_t s) {
   if (vec) {
-    const dim3 grid((unsigned)(((long)a.L * (a.H / a.G) + kTileRows - 1) / kTileRows), (unsigned)(a.B * a.G));
+    const uint32_t qpk = (uint32_t)(a.H / a.G);
+    a.heads_inv = qpk == 1 ? ~0u : (uint32_t)((1ull << 32) / qpk);
+    const dim3 grid((unsigned)(((long)a.L * qpk + kTileRows - 1) / kTileRows), (unsigned)a.G, (unsigned)a.B);
     const int kc = (int)((a.d + 31) / 32);
-    if (kc <= 1)
+    if (a.d == 64 && a.dv == 64)
+      launch_window_mfma_pairs<2, 2, true>(a, grid, s);
+    else if (kc <= 1)
       launch_window_mfma<1>(a, grid, s);
     else if (kc <= 2)
       launch_window_mfma<2>(a, grid, s);

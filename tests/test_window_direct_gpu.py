@@ -1,0 +1,51 @@
+"""Window attention over bf16 prompts of 64-channel heads (keys and values straight into LDS, weights summed as they enter the products)
+against 64 bits: portions, windows and heads around tiles of 64 keys and 128 rows, either sign of the scale, and scores that climb."""
+import pytest
+import torch
+
+from oracle import sozilix_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def run(dev, q, k, v, window, scale, start, shift=0):
+    from based_amd import ops
+
+    B, L, H, d = q.shape
+    G = k.shape[2]
+    wide = torch.full((B, L + 3, G, 2 * d + 8 * shift), float("nan"), dtype=torch.bfloat16, device=dev)  # (rows of a wider cache)
+    cache = wide[..., :2 * d] if shift == 0 else torch.as_strided(wide, (B, L + 3, G, 2 * d), (wide.stride(0), wide.stride(1), 2 * d, 1))
+    out = torch.empty(B, L, H * d, dtype=torch.bfloat16, device=dev)
+    for lo, hi in ((0, start), (start, L)):
+        if hi > lo:
+            s = slice(lo, hi)
+            ops.window_attn_prefill(*(t[:, s].to(dev).flatten(2) for t in (q, k, v)), cache, H, G, window, scale, lo, out=out[:, s])
+    return out.double().cpu().view(B, L, H, d)
+
+
+def error(out, q, k, v, window, scale):
+    ref = torch.stack([O.window_softmax(a.double(), b.double(), c.double(), scale, window) for a, b, c in zip(q, k, v)])
+    return float(((out - ref).norm(dim=-1) / ref.norm(dim=-1)).max())
+
+
+@pytest.mark.parametrize("H,G,L,start,window", [(1, 1, 1, 0, 1), (4, 1, 31, 0, 129), (3, 1, 43, 0, 20), (16, 4, 65, 0, 64), (16, 4, 97, 33, 33), (5, 1, 128, 0, 1),
+                                                (2, 2, 129, 64, 63), (16, 2, 200, 0, 65), (16, 16, 257, 0, 129), (12, 4, 321, 100, 128), (7, 1, 130, 1, 500),
+                                                (8, 8, 640, 0, 513), (2, 1, 700, 690, 129)])
+@pytest.mark.parametrize("scale", [0.125, -0.3])
+def test_portions_windows_and_heads(dev, H, G, L, start, window, scale):
+    g = torch.Generator().manual_seed(L + window)
+    q, k, v = (torch.randn(2, L, n, 64, generator=g).bfloat16() for n in (H, G, G))
+    # bf16 weights and outputs: 2^-9 each, of rows whose values partly cancel
+    assert error(run(dev, q, k, v, window, scale, start, L % 2), q, k, v, window, scale) < 2e-2
+
+
+@pytest.mark.parametrize("step", [0.02, 0.2, 3.0, -0.2])
+def test_scores_that_climb(dev, step):
+    """Scores that grow (or fall) by `step` powers of two from key to key: a new largest one in every tile, or none."""
+    L, window = 300, 129
+    g = torch.Generator().manual_seed(1)
+    q, k, v = (0.05 * torch.randn(1, L, 2, 64, generator=g) for _ in range(3))
+    q[..., 0] = 1.0
+    k[..., 0] = (step / 1.4426950408889634) * torch.arange(L)[None, :, None]
+    q, k, v = (t.bfloat16() for t in (q, k, 20 * v))
+    assert error(run(dev, q, k, v, window, 1.0, 0), q, k, v, window, 1.0) < 2e-2
