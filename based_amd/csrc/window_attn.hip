@@ -476,8 +476,43 @@ __global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 
 // weights of a lane are what the products with the values take, one each, where product j contracts keys j, 4 + j, 8 + j and 12 + j;
 // keys and queries give up their channels in the same order, so that a lane reads 16 bytes for four products.
 // Bound by the fp32 matrix rate from some thousand rows on and by the chain of one wavefront below.  16 heads on 4, size 64, 129 keys:
-// B = 1, L = 777, with the cache write: 19 us (a wavefront per query on the vector unit: 70); B = 4, L = 2048: 81 us (661).
+// B = 1, L = 777, with the cache write: 17.7 us (a wavefront per query on the vector unit: 70); B = 4, L = 2048: 77 us (661).
 constexpr int kF32Keys = 32, kF32Rows = 64;
+
+// What turns channels c .. c + 3 of a row (as Turn8, for either kind of pairs): loaded without a condition, applied later.
+struct Turn4 {
+  f32x4 cs, sn, partner;  // (interleaved pairs: two angles)
+  __device__ __forceinline__ void load(const float* row, int c, int pos, const WindowArgs& a) {
+    const bool in = c < a.rot;
+    const int half = a.rot / 2;
+    const float *cos_t = a.rot > 0 ? a.cos_t : static_cast<const float*>(a.kv), *sin_t = a.rot > 0 ? a.sin_t : static_cast<const float*>(a.kv);
+    if (a.half_split) {  // (uniform)
+      const long t = in ? (long)pos * half + (c < half ? c : c - half) : 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) cs[j] = cos_t[t + j], sn[j] = sin_t[t + j];
+      partner = *reinterpret_cast<const f32x4*>(row + (in ? (c < half ? c + half : c - half) : 0));
+    } else {
+      const long t = in ? (long)pos * half + c / 2 : 0;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) cs[j] = cos_t[t + j], sn[j] = sin_t[t + j];
+    }
+  }
+  __device__ __forceinline__ void apply(f32x4& x, int c, const WindowArgs& a) const {
+    if (c >= a.rot) return;
+    if (a.half_split) {
+      const float sgn = c < a.rot / 2 ? -1.f : 1.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = x[j] * cs[j] + sgn * partner[j] * sn[j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const float u = x[2 * j], v = x[2 * j + 1];
+        x[2 * j] = u * cs[j] - v * sn[j];
+        x[2 * j + 1] = v * cs[j] + u * sn[j];
+      }
+    }
+  }
+};
 
 // channels c .. c + 3 of a row, turned; c and the rotary size (its half in half-split pairs) multiples of 4
 __device__ __forceinline__ f32x4 turned4(const float* row, int c, int pos, const WindowArgs& a) {
@@ -534,14 +569,19 @@ __global__ __launch_bounds__(256) void window_kv_write_f32_kernel(const WindowAr
   }
 }
 
-template <int KB, int VB>
-__global__ __launch_bounds__(256) void window_prefill_f32_kernel(const WindowArgs a) {
-  constexpr int D = KB * 64, DV = VB * 64, KS = D + 4, VS = DV + 4;
-  __shared__ __attribute__((aligned(16))) float lds_k[kF32Keys * KS], lds_v[kF32Keys * VS];
-  __shared__ int s_odd[4];  // values of this tile that are not finite, by the wavefront that staged them
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4;
+// KH: wavefronts to the same 16 rows, which take 32 keys of a tile each and add up what they have in the end.
+// FILL: the portion's keys and values are taken as they come, turned and normed on their way to LDS, and left in the cache by the workgroups
+// whose tokens they are; nobody reads there what is written.
+template <int KB, int VB, int KH, bool FILL>
+__global__ __launch_bounds__(256 * KH) void window_prefill_f32_kernel(const WindowArgs a) {
+  constexpr int D = KB * 64, DV = VB * 64, KS = D + 4, VS = DV + 4, NT = 256 * KH, KEYS = kF32Keys * KH;
+  __shared__ __attribute__((aligned(16))) float lds[KEYS * (KS + VS)];
+  float *lds_k = lds, *lds_v = lds + KEYS * KS;
+  __shared__ int s_odd[4 * KH];  // values of this tile that are not finite, by the wavefront that staged them
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), part = wave >> 2;
   const int b = blockIdx.y / a.G, g = blockIdx.y % a.G, qpk = a.H / a.G, n_rows = a.L * qpk;
-  const int r0 = blockIdx.x * kF32Rows, row_w = r0 + wave * 16;
+  const int r0 = blockIdx.x * kF32Rows, row_w = r0 + (wave & 3) * 16;
   const auto token_of = [&](int row) { return (row < n_rows ? row : n_rows - 1) / qpk; };
   const float* kv = static_cast<const float*>(a.kv) + b * a.kv_sb + (long)g * (a.d + a.dv);
   const int tok = token_of(row_w + l16), pos = a.pos_host + tok;
@@ -551,16 +591,54 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(const WindowArg
   const int lo = first - a.window + 1 > 0 ? first - a.window + 1 : 0;
 
   f32x4 kbuf[2 * KB], vbuf[2 * VB];
+  Turn4 turn[FILL ? 2 * KB : 1];
+  const float* fresh_k = static_cast<const float*>(a.k) + b * a.k_sb + (long)g * a.d;
+  const float* fresh_v = static_cast<const float*>(a.v) + b * a.v_sb + (long)g * a.dv;
   const auto fetch = [&](int k0) {
 #pragma unroll
     for (int i = 0; i < 2 * KB; ++i) {
-      const int p = i * 256 + tid, key = p / (D / 4), e = p % (D / 4) * 4;
-      kbuf[i] = *reinterpret_cast<const f32x4*>(kv + (long)(k0 + key <= last ? k0 + key : last) * a.kv_st + (e < a.d ? e : 0));
+      const int p = i * NT + tid, e = p % (D / 4) * 4, c = e < a.d ? e : 0;
+      const int key = k0 + p / (D / 4) <= last ? k0 + p / (D / 4) : last;
+      const float* row = kv + (long)key * a.kv_st;
+      if constexpr (FILL) {
+        row = key < a.pos_host ? row : fresh_k + (long)(key - a.pos_host) * a.k_sl;
+        turn[i].load(row, c, key, a);
+      }
+      kbuf[i] = *reinterpret_cast<const f32x4*>(row + c);
     }
 #pragma unroll
     for (int i = 0; i < 2 * VB; ++i) {
-      const int p = i * 256 + tid, key = p / (DV / 4), e = p % (DV / 4) * 4;
-      vbuf[i] = *reinterpret_cast<const f32x4*>(kv + (long)(k0 + key <= last ? k0 + key : last) * a.kv_st + a.d + (e < a.dv ? e : 0));
+      const int p = i * NT + tid, e = p % (DV / 4) * 4, c = e < a.dv ? e : 0;
+      const int key = k0 + p / (DV / 4) <= last ? k0 + p / (DV / 4) : last;
+      const float* row = kv + (long)key * a.kv_st + a.d;
+      if constexpr (FILL) row = key < a.pos_host ? row : fresh_v + (long)(key - a.pos_host) * a.v_sl;
+      vbuf[i] = *reinterpret_cast<const f32x4*>(row + c);
+    }
+  };
+  // what `fetch` brought of the tile at k0, as the cache has it
+  const auto settle = [&](int k0) {
+    if constexpr (FILL) {
+      float* fill = const_cast<float*>(kv);
+#pragma unroll
+      for (int i = 0; i < 2 * KB; ++i) {
+        const int p = i * NT + tid, e = p % (D / 4) * 4, key = k0 + p / (D / 4);
+        if (key >= a.pos_host && e < a.d) {
+          turn[i].apply(kbuf[i], e, a);
+          if (key >= first && key <= last) *reinterpret_cast<f32x4*>(fill + (long)key * a.kv_st + e) = kbuf[i];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 2 * VB; ++i) {
+        const int p = i * NT + tid, e = p % (DV / 4) * 4, key = k0 + p / (DV / 4);
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ss = e < a.dv ? __builtin_fmaf(vbuf[i][j], vbuf[i][j], ss) : ss;
+        ss = sum16(ss);
+        if (VB == 2) ss += __shfl_xor(ss, 16, 64);
+        const float r = a.norm_v && key >= a.pos_host ? 1.0f / sqrtf(ss / (float)a.dv + a.eps) : 1.0f;
+        vbuf[i] *= r;
+        if (key >= first && key <= last && e < a.dv) *reinterpret_cast<f32x4*>(fill + (long)key * a.kv_st + a.d + e) = vbuf[i];
+      }
     }
   };
   fetch(lo);
@@ -586,17 +664,18 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(const WindowArg
   // out of sight stays at minus infinity, an infinite one is no number).
   const float scale2 = a.scale == 0.f ? 1.f : fabsf(a.scale) * 1.4426950408889634f;
 
-  for (int k0 = lo; k0 <= last; k0 += kF32Keys) {
+  for (int t0 = lo; t0 <= last; t0 += KEYS) {
+    settle(t0);
     __syncthreads();  // every wavefront is done with the tile before
     bool odd = false;
 #pragma unroll
     for (int i = 0; i < 2 * KB; ++i) {
-      const int p = i * 256 + tid, key = p / (D / 4), e = p % (D / 4) * 4;
+      const int p = i * NT + tid, key = p / (D / 4), e = p % (D / 4) * 4;
       *reinterpret_cast<f32x4*>(&lds_k[key * KS + e]) = e < a.d ? kbuf[i] : f32x4{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
     for (int i = 0; i < 2 * VB; ++i) {
-      const int p = i * 256 + tid, key = p / (DV / 4), e = p % (DV / 4) * 4;
+      const int p = i * NT + tid, key = p / (DV / 4), e = p % (DV / 4) * 4;
       const f32x4 x = vbuf[i];
       const float zero = (x[0] * 0.f + x[1] * 0.f) + (x[2] * 0.f + x[3] * 0.f);
       odd |= !(zero == 0.f);
@@ -605,7 +684,9 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(const WindowArg
     odd = __any(odd);
     if (lane == 0) s_odd[wave] = odd;
     __syncthreads();
-    if (k0 + kF32Keys <= last) fetch(k0 + kF32Keys);
+    if (t0 + KEYS <= last) fetch(t0 + KEYS);
+    const int k0 = t0 + part * kF32Keys;
+    const float *tile_k = lds_k + part * kF32Keys * KS, *tile_v = lds_v + part * kF32Keys * VS;
     if (k0 > wave_hi || k0 + kF32Keys - 1 <= wave_lo - a.window) continue;
     const bool all = k0 + kF32Keys - 1 <= wave_lo && k0 > wave_hi - a.window;  // does every row see every key?
     const bool kt_in[2] = {k0 + 15 > wave_lo - a.window, k0 + 16 <= wave_hi};  // does any see one of these 16?
@@ -616,8 +697,8 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(const WindowArg
         f32x4 half = {0.f, 0.f, 0.f, 0.f};  // (two sums of half the channels each round less than one)
 #pragma unroll
         for (int c = 0; c < 4 * KB; c += 2) {
-          const f32x4 k0f = *reinterpret_cast<const f32x4*>(&lds_k[(kt * 16 + l16) * KS + c * 16 + quad * 4]);
-          const f32x4 k1f = *reinterpret_cast<const f32x4*>(&lds_k[(kt * 16 + l16) * KS + (c + 1) * 16 + quad * 4]);
+          const f32x4 k0f = *reinterpret_cast<const f32x4*>(&tile_k[(kt * 16 + l16) * KS + c * 16 + quad * 4]);
+          const f32x4 k1f = *reinterpret_cast<const f32x4*>(&tile_k[(kt * 16 + l16) * KS + (c + 1) * 16 + quad * 4]);
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             s[kt] = mfma_f32(k0f[j], qf[c][j], s[kt]);
@@ -659,7 +740,10 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(const WindowArg
         sum += s[kt][i];
       }
     l_run += sum;  // this lane's keys; the four quads are added at the end
-    if (all || !(s_odd[0] | s_odd[1] | s_odd[2] | s_odd[3])) {
+    int odd_any = 0;
+#pragma unroll
+    for (int w = 0; w < 4 * KH; ++w) odd_any |= s_odd[w];
+    if (all || !odd_any) {
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
         if (kt_in[kt]) {
@@ -667,7 +751,7 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(const WindowArg
           for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int vb = 0; vb < VB; ++vb) {
-              const f32x4 vf = *reinterpret_cast<const f32x4*>(&lds_v[(kt * 16 + quad * 4 + j) * VS + vb * 64 + l16 * 4]);
+              const f32x4 vf = *reinterpret_cast<const f32x4*>(&tile_v[(kt * 16 + quad * 4 + j) * VS + vb * 64 + l16 * 4]);
 #pragma unroll
               for (int c = 0; c < 4; ++c) acc[vb][c] = mfma_f32(vf[c], s[kt][j], acc[vb][c]);
             }
@@ -686,10 +770,29 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(const WindowArg
             for (int c = 0; c < 4; ++c)
 #pragma unroll
               for (int i = 0; i < 4; ++i)
-                acc[vb][c][i] = __builtin_fmaf(p, lds_v[key * VS + vb * 64 + (quad * 4 + i) * 4 + c], acc[vb][c][i]);
+                acc[vb][c][i] = __builtin_fmaf(p, tile_v[key * VS + vb * 64 + (quad * 4 + i) * 4 + c], acc[vb][c][i]);
         }
       }
     }
+  }
+  if constexpr (KH > 1) {
+    // the other wavefront's sums of the same rows, both taken to the larger of their largest scores
+    constexpr int N = 16 * VB + 2;
+    static_assert(KH == 2 && N * 256 <= KEYS * (KS + VS), "room for one half");
+    __syncthreads();
+    float* at = lds + (wave & 3) * 64 + lane;
+    if (part == 1) {
+      at[0] = m_run, at[256] = l_run;
+#pragma unroll
+      for (int n = 0; n < 16 * VB; ++n) at[(n + 2) * 256] = acc[n / 16][n / 4 % 4][n % 4];
+    }
+    __syncthreads();
+    if (part == 1) return;
+    const float other = at[0], m = fmaxf(m_run, other), m0 = m == -INFINITY ? 0.f : m;
+    const float mine = __builtin_amdgcn_exp2f((m_run - m0) * scale2), theirs = __builtin_amdgcn_exp2f((other - m0) * scale2);
+    l_run = l_run * mine + at[256] * theirs;
+#pragma unroll
+    for (int n = 0; n < 16 * VB; ++n) acc[n / 16][n / 4 % 4][n % 4] = acc[n / 16][n / 4 % 4][n % 4] * mine + at[(n + 2) * 256] * theirs;
   }
   float l = l_run;
   l += __shfl_xor(l, 16, 64);
@@ -1367,8 +1470,54 @@ static bool window_f32_few(const WindowArgs& a) {
   return rows <= (a.d <= 16 ? 2600 : a.d <= 24 ? 2000 : a.d <= 32 ? 1000 : a.d <= 48 ? 700 : a.d <= 64 ? 400 : a.d <= 96 ? 700 : 350);
 }
 
-// The attention of a portion whose keys and values are in place.
-static void launch_window_attend(WindowArgs a, bool vec, int io_dtype, hipStream_t s) {
+// Two wavefronts to the same rows where the workgroups are no more than the compute units, or the way through the keys is long; in the first case,
+// where that way is short, the cache filled as well (every workgroup turns the keys that it sees: with 1,024 of them 104 us become 158).  us, 16
+// heads of 64 channels, one wavefront and a launch for the cache / two / cache filled: on 4, 129 keys, 1 x 777 (196 workgroups) 19.8 / 18.7 / 17.7;
+// 1 x 100 13.8 / 12.7 / 11.9; 1 x 2048 (512) 30.5 / 30.4 / -; 4 x 2048 (2,048) 77 / 80 / -; on 16, 1,024 keys, 1 x 2048 (512) 115 / 104 / 158; on 2, 513
+// keys, 2 x 500 (252) 39.2 / 32.5 / 37.7.
+static bool window_f32_small(const WindowArgs& a) { return ((long)a.L * (a.H / a.G) + kF32Rows - 1) / kF32Rows * a.B * a.G <= 256; }
+static long window_f32_keys(const WindowArgs& a) {
+  const long end = (long)a.pos_host + a.L;
+  return (a.window < end ? a.window : end) + kF32Rows / (a.H / a.G);
+}
+
+template <int KB, int VB> void launch_window_f32(const WindowArgs& a, dim3 grid, bool fill, hipStream_t s) {
+  if constexpr (KB + VB < 4) {
+    if (fill) {
+      hipLaunchKernelGGL((window_prefill_f32_kernel<KB, VB, 2, true>), grid, dim3(512), 0, s, a);
+      return;
+    }
+    if (window_f32_small(a) || window_f32_keys(a) > 256) {
+      hipLaunchKernelGGL((window_prefill_f32_kernel<KB, VB, 2, false>), grid, dim3(512), 0, s, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((window_prefill_f32_kernel<KB, VB, 1, false>), grid, dim3(256), 0, s, a);
+}
+
+// Whether memory that rows of `width` elements at these strides span overlaps.
+static bool rows_meet(const WindowArgs& a, const void* x, long x_sb, long x_sl, long x_width, const void* y, long y_sb, long y_sl, long y_width) {
+  const auto bytes = [&](long sb, long sl, long width) { return ((a.B - 1) * sb + (a.L - 1) * sl + width) * 4; };
+  const uintptr_t p = reinterpret_cast<uintptr_t>(x), q = reinterpret_cast<uintptr_t>(y);
+  return p < q + bytes(y_sb, y_sl, y_width) && q < p + bytes(x_sb, x_sl, x_width);
+}
+
+// Whether the fp32 form fills the cache itself: keys and values are read by every workgroup that sees them, so that nothing else may be written
+// there, and in 16-byte pieces.
+static bool window_f32_fills(const WindowArgs& a) {
+  if (!window_f32_small(a) || window_f32_keys(a) > 256 || (a.d > 64 && a.dv > 64)) return false;
+  if (a.k_sb % 4 || a.k_sl % 4 || a.v_sb % 4 || a.v_sl % 4 || !aligned_to(a.k, 16) || !aligned_to(a.v, 16)) return false;
+  if (a.k_sb < 0 || a.k_sl < 0 || a.v_sb < 0 || a.v_sl < 0 || a.o_sb < 0 || a.o_sl < 0 || a.kv_sb < 0 || a.kv_st < 0) return false;
+  const long kw = (long)a.G * a.d, vw = (long)a.G * a.dv, row = kw + vw;
+  const float* cache = static_cast<const float*>(a.kv) + (long)a.pos_host * a.kv_st;
+  const auto apart = [&](const void* x, long sb, long sl, long width) {
+    return !rows_meet(a, x, sb, sl, width, cache, a.kv_sb, a.kv_st, row) && !rows_meet(a, x, sb, sl, width, a.o, a.o_sb, a.o_sl, (long)a.H * a.dv);
+  };
+  return apart(a.k, a.k_sb, a.k_sl, kw) && apart(a.v, a.v_sb, a.v_sl, vw);
+}
+
+// The attention of a portion whose keys and values are in place (fill: it puts them there itself; `window_f32_fills`).
+static void launch_window_attend(WindowArgs a, bool vec, int io_dtype, bool fill, hipStream_t s) {
   if (vec) {
     const uint32_t qpk = (uint32_t)(a.H / a.G);
     a.heads_inv = qpk == 1 ? ~0u : (uint32_t)((1ull << 32) / qpk);
@@ -1389,13 +1538,13 @@ static void launch_window_attend(WindowArgs a, bool vec, int io_dtype, hipStream
   } else if (window_f32(a, io_dtype) && !window_f32_few(a)) {
     const dim3 grid((unsigned)(((long)a.L * (a.H / a.G) + kF32Rows - 1) / kF32Rows), (unsigned)(a.B * a.G));
     if (a.d <= 64 && a.dv <= 64)
-      hipLaunchKernelGGL((window_prefill_f32_kernel<1, 1>), grid, dim3(256), 0, s, a);
+      launch_window_f32<1, 1>(a, grid, fill, s);
     else if (a.d <= 64)
-      hipLaunchKernelGGL((window_prefill_f32_kernel<1, 2>), grid, dim3(256), 0, s, a);
+      launch_window_f32<1, 2>(a, grid, fill, s);
     else if (a.dv <= 64)
-      hipLaunchKernelGGL((window_prefill_f32_kernel<2, 1>), grid, dim3(256), 0, s, a);
+      launch_window_f32<2, 1>(a, grid, fill, s);
     else
-      hipLaunchKernelGGL((window_prefill_f32_kernel<2, 2>), grid, dim3(256), 0, s, a);
+      launch_window_f32<2, 2>(a, grid, fill, s);
   } else {
     const dim3 grid((unsigned)a.L, (unsigned)a.H, (unsigned)a.B);
     if (io_dtype == BASED_BF16)
@@ -1428,16 +1577,19 @@ extern "C" BASED_API int based_window_attn_prefill(
   const bool vec = io_dtype == BASED_BF16 && D <= 256 && DV <= 256 && rotary_dim % (half_split ? 16 : 8) == 0 && window_vec(a, 8);
   const int64_t items = B * L * G;
   BASED_REQUIRE(items < (1ll << 32), BASED_ERR_SHAPE, "window_attn_prefill: grid too large");
+  const bool fill = window_f32(a, io_dtype) && !window_f32_few(a) && window_f32_fills(a);
   if (vec) {
     const int64_t widest = D > DV ? D : DV;
     widest <= 64 ? launch_kv_write<8>(a, s) : widest <= 128 ? launch_kv_write<16>(a, s) : launch_kv_write<32>(a, s);
   } else if (io_dtype == BASED_BF16)
     hipLaunchKernelGGL(window_kv_write_kernel<__bf16>, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s, a);
+  else if (fill)
+    ;
   else if (window_f32(a, io_dtype) && k_sb % 4 == 0 && k_sl % 4 == 0 && v_sb % 4 == 0 && v_sl % 4 == 0 && aligned_to(k, 16) && aligned_to(v, 16))
     hipLaunchKernelGGL(window_kv_write_f32_kernel, dim3((unsigned)((items + 15) / 16)), dim3(256), 0, s, a);
   else
     hipLaunchKernelGGL(window_kv_write_kernel<float>, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s, a);
-  launch_window_attend(a, vec, io_dtype, s);
+  launch_window_attend(a, vec, io_dtype, fill, s);
   return check_launch("window_attn_prefill");
 }
 
@@ -1459,7 +1611,7 @@ extern "C" BASED_API int based_window_attn_attend(const void* q, const void* kv,
   BASED_REQUIRE(B * G < 65536 && B < 65536 && H < 65536, BASED_ERR_SHAPE, "window_attn_attend: grid too large");
   if (B == 0 || L == 0) return BASED_OK;
   const bool vec = io_dtype == BASED_BF16 && D <= 256 && DV <= 256 && rotary_dim % (half_split ? 16 : 8) == 0 && window_vec(a, 8);
-  launch_window_attend(a, vec, io_dtype, static_cast<hipStream_t>(stream));
+  launch_window_attend(a, vec, io_dtype, false, static_cast<hipStream_t>(stream));
   return check_launch("window_attn_attend");
 }
 

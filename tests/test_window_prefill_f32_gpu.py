@@ -100,3 +100,45 @@ def test_both_sides_of_the_rule_for_few_rows(dev, d, dv, H, G, L, start, window)
                            zip(q[rows], k[rows], v[rows])])[:, start:]
         err = (out[rows] - ref).norm(dim=-1) / ref.norm(dim=-1)
         assert float(err.max()) < 3e-6, (B, float(err.max()))  # (scores of up to 5 and sums of 128 products)
+
+
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("H,G,d,dv,B,L,start,window,rot,half", [
+    (16, 4, 64, 64, 1, 777, 0, 129, 32, False), (16, 4, 64, 64, 1, 300, 77, 129, 32, True), (6, 2, 60, 36, 3, 190, 0, 20, 8, False),
+    (16, 16, 64, 64, 1, 130, 1, 64, 64, False), (12, 4, 64, 100, 1, 200, 40, 200, 16, True), (8, 1, 100, 64, 2, 128, 0, 65, 4, False),
+    (16, 2, 64, 64, 2, 500, 0, 513, 32, False)])
+def test_cache_that_the_attention_fills(dev, H, G, d, dv, B, L, start, window, rot, half, norm):
+    """Rows of the cache behind a portion, and what a second portion makes of them: written by the attention itself, or in front of it where the
+    portion's own keys lie in the output's rows."""
+    from based_amd import ops
+    from based_amd.mixers.window_attention import _ExactRotary
+
+    g = torch.Generator().manual_seed(L)
+    n = L + start
+    rope = _ExactRotary(rot, base=100.0, interleaved=not half).tables(n, dev)
+    x = torch.randn(B, n, H * d + G * (d + dv), generator=g).to(dev)
+    q, k, v = x[..., :H * d], x[..., H * d:(H + G) * d], x[..., (H + G) * d:]
+    kw = dict(rope=rope, value_norm_eps=1e-5 if norm else None)
+
+    def run(inside):
+        cache = torch.full((B, n + 2, G, d + dv), float("nan"), device=dev)
+        room = x.clone() if inside else torch.full((B, n, H * dv), float("nan"), device=dev)
+        kk, vv = (room[..., H * d:(H + G) * d], room[..., (H + G) * d:]) if inside else (k, v)
+        out = room[..., :H * dv] if inside and dv <= d else torch.empty(B, n, H * dv, device=dev) if inside else room
+        qq = q
+        for lo, hi in ((0, start), (start, n)):
+            if hi > lo:
+                s = slice(lo, hi)
+                ops.window_attn_prefill(qq[:, s], kk[:, s], vv[:, s], cache, H, G, window, d ** -0.5, lo, out=out[:, s], **kw)
+        return out.clone(), cache
+
+    out, cache = run(False)
+    ref, rows = run(True)
+    # (a rotation's two products are added in one order or the other: 2^-24 of the larger)
+    assert float((cache[:, :n] - rows[:, :n]).abs().max()) <= 2 ** -23 * float(rows[:, :n].abs().max()) and cache[:, n:].isnan().all()
+    # (two forms of the same sums of up to 513 weights: a few roundings of 2^-24)
+    assert float((out - ref).norm() / ref.norm()) < 1e-6
+    want = v.view(B, n, G, dv).double()
+    if norm:
+        want = want / (want.square().mean(-1, keepdim=True) + 1e-5).sqrt()
+    assert float((cache[:, :n, :, d:].double() - want).norm() / want.norm()) < 2e-7
