@@ -875,18 +875,124 @@ template <bool PAIRED, bool TAIL> __global__ __launch_bounds__(512, 2) void expe
   large_whole_tile<PAIRED, TAIL>(a, t, lds, slot_of);
 }
 
+// The same tiles of 32 rows with 64 rows of the weights (PAIRED: 32 up, 32 gate), rows and weights straight into LDS, rounds of 128 channels three
+// deep: a few rows an expert wait for its matrices to come from memory, which asks for many loads on their way and many workgroups.  A wavefront
+// takes 32 channels of a round and the whole tile; the four sums of an element are added through LDS in the end.  Channels in whole 128.
+constexpr int kDirectWeights = 64, kDirectRows = BASED_EXPERT_TILE_ROWS_SMALL + kDirectWeights;
+constexpr int kDirectSlab = kDirectRows * 64, kDirectRound = 2 * kDirectSlab, kDirectDepth = 3;  // elements; a slab: 64 channels of every row
+constexpr int kDirectLds = kDirectDepth * kDirectRound * 2 + BASED_EXPERT_TILE_ROWS_SMALL * 4;   // bytes
+
+template <bool PAIRED> __global__ __launch_bounds__(256, 2) void expert_gemm_direct_kernel(const ExpertGemmArgs a) {
+  constexpr int BM = BASED_EXPERT_TILE_ROWS_SMALL, BN = kDirectWeights, COLS = PAIRED ? BN / 2 : BN, LOADS = kDirectRows / 16;
+  extern __shared__ __attribute__((aligned(16))) __bf16 lds[];
+  int* slot_of = reinterpret_cast<int*>(lds + kDirectDepth * kDirectRound);
+  const int id = tile_of_block(blockIdx.x, gridDim.x), band = id / (kBand * a.col_tiles), in_band = id % (kBand * a.col_tiles);
+  const int deep = a.tiles - band * kBand < kBand ? a.tiles - band * kBand : kBand;
+  const int tile = band * kBand + in_band % deep, f0 = in_band / deep * COLS;
+  if (tile >= a.tile_first[a.E]) return;
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int e = 0, rows = a.counts[0] - tile * BM;  // (of one expert)
+  if (a.tile_expert != nullptr) {
+    const int what = a.tile_expert[tile];
+    e = what & 255, rows = what >> 8;
+  } else {
+    rows = rows < BM ? rows : BM;
+  }
+  if (tid < BM) slot_of[tid] = a.order[(long)tile * BM + (tid < rows ? tid : 0)];
+  lds_barrier();
+  // 8 rows of a slab to a load; piece p (16 bytes) of a row lies at p ^ (row / 2 % 8), so that reads of 16 rows meet every bank once
+  const char* src[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int group = wave * LOADS + i, slab = group / (kDirectRows / 8), row = group % (kDirectRows / 8) * 8 + (lane >> 3);
+    const __bf16* at;
+    if (row < BM) {
+      at = a.x + (PAIRED ? (long)(slot_of[row] / a.top) * a.x_sr : ((long)tile * BM + (row < rows ? row : 0)) * a.x_sr);
+    } else {
+      const int r = row - BM, f = f0 + r % COLS;
+      at = a.w + ((long)e * (PAIRED ? 2 * a.F : a.F) + (PAIRED && r >= COLS ? a.F : 0) + (f < a.F ? f : a.F - 1)) * a.K;
+    }
+    src[i] = reinterpret_cast<const char*>(at + slab * 64 + ((lane & 7) ^ (row >> 1 & 7)) * 8);
+  }
+  const int rounds = a.K / 128;
+  auto ask = [&](int round, int place) {
+    const long from = (long)(round < rounds ? round : 0) * 256;  // (past the end: asked for and never read, the count of loads stays)
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + from),
+                                       (__attribute__((address_space(3))) void*)(lds + place * kDirectRound + (wave * LOADS + i) * 512), 16, 0, 0);
+  };
+  f32x4 acc[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i][0] = acc[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  ask(0, 0);
+  ask(1, 1);
+  const int turned = l16 >> 1 & 7, step = (wave >> 1) * kDirectSlab + (((wave & 1) * 4 + quad) ^ turned) * 8 + l16 * 64;
+  for (int round = 0, place = 0; round < rounds; ++round) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0070 | LOADS);  // own reads are done, and all loads but those of the next round
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    ask(round + 2, place == 0 ? 2 : place - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    const __bf16* at = lds + place * kDirectRound + step;
+    bf16x8 x[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) x[j] = *reinterpret_cast<const bf16x8*>(at + j * 16 * 64);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bf16x8 w = *reinterpret_cast<const bf16x8*>(at + (BM + i * 16) * 64);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] = expert_mfma(w, x[j], acc[i][j]);
+    }
+    place = place == 2 ? 0 : place + 1;
+  }
+  __builtin_amdgcn_s_waitcnt(0x0070);  // (nothing may come into LDS that is no longer the loads')
+  __builtin_amdgcn_s_barrier();
+  f32x4* sums = reinterpret_cast<f32x4*>(lds);  // [wave][feature tile][row tile][lane]
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) sums[((wave * 4 + i) * 2 + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  // two feature tiles (PAIRED: up and gate) of 16 rows to a wavefront
+  const int half = wave & 1, r = (wave >> 1) * 16 + l16;
+  f32x4 out[2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const f32x4* at = sums + ((p * 2 + half) * 2 + (wave >> 1)) * 64 + lane;
+    out[p] = (at[0] + at[512]) + (at[1024] + at[1536]);
+  }
+  if (r >= rows) return;
+  const int slot = slot_of[r];
+  if constexpr (PAIRED) {
+    large_store<true>(a, a.y + ((long)tile * BM + r) * a.F, f0 + half * 16 + quad * 4, a.scores[slot], out[0], out[1]);
+  } else {
+    __bf16* y = a.y + (long)slot * a.F;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) large_store<false>(a, y, f0 + (p * 2 + half) * 16 + quad * 4, 1.f, out[p], out[p]);
+  }
+}
+
 constexpr int kMaxDevices = 64;
 
-template <bool PAIRED, bool TAIL> int launch_expert_gemm_large(ExpertGemmArgs a, hipStream_t s) {
-  static std::atomic<bool> allowed[kMaxDevices];
+// Lets a kernel have `bytes` of LDS, once for each device.
+static int allow_lds(const void* kernel, int bytes, std::atomic<bool> (&allowed)[kMaxDevices]) {
   int dev = 0;
   BASED_REQUIRE(hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices, BASED_ERR_LAUNCH, "experts: cannot identify the current device");
   if (!allowed[dev].load(std::memory_order_acquire)) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(expert_gemm_large_kernel<PAIRED, TAIL>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, kLargeLds);
-    BASED_REQUIRE(e == hipSuccess, BASED_ERR_LAUNCH, "experts: %d bytes of LDS refused: %s", kLargeLds, hipGetErrorString(e));
+    const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    BASED_REQUIRE(e == hipSuccess, BASED_ERR_LAUNCH, "experts: %d bytes of LDS refused: %s", bytes, hipGetErrorString(e));
     allowed[dev].store(true, std::memory_order_release);
   }
+  return BASED_OK;
+}
+
+template <bool PAIRED, bool TAIL> int launch_expert_gemm_large(ExpertGemmArgs a, hipStream_t s) {
+  static std::atomic<bool> allowed[kMaxDevices];
+  const int rc = allow_lds(reinterpret_cast<const void*>(expert_gemm_large_kernel<PAIRED, TAIL>), kLargeLds, allowed);
+  if (rc != BASED_OK) return rc;
   a.col_tiles = PAIRED ? (a.F + 127) / 128 : (a.F + 255) / 256;
   // (parts beyond the first of a tile: less than one for each of the 32 compute units of a die)
   const unsigned per_die = (unsigned)((a.col_tiles * a.tiles + kDies - 1) / kDies + kDieUnits);
@@ -894,17 +1000,31 @@ template <bool PAIRED, bool TAIL> int launch_expert_gemm_large(ExpertGemmArgs a,
   return BASED_OK;
 }
 
-template <bool PAIRED> void launch_expert_gemm(ExpertGemmArgs a, hipStream_t s) {
-  const int cols = PAIRED ? kSmallWeights / 2 : kSmallWeights;
+// Straight into LDS where tiles of 128 rows of the weights are fewer than half of the compute units and a tile's way is long.  Whole calls, kernels alone,
+// us, without and with (both products, the second alone): 2 of 8 experts of 1024, 12 tokens (128 and 64 workgroups) 27.3 / 23.7 / 24.9, 30 (144, 72) 28.4
+// / 27.0 / 26.2, 100 (224, 112) 33.9 / 32.7 / 32.5, 164 (288, 144) 37.6 / 36.5 / 38.0; 1 of 8 of 2048, 30 tokens (256, 64) 34.4 / 29.9 / 29.3, 260 (512,
+// 128) 42.8 / 39.4 / 38.3; 4 of 16 of 512, 30 tokens (152, 152; 512 channels) 29.2 / 30.9 / 30.1.
+template <bool PAIRED> int launch_expert_gemm(ExpertGemmArgs a, hipStream_t s) {
+  const int before = PAIRED ? kSmallWeights / 2 : kSmallWeights;
+  const bool direct = a.K % 128 == 0 && a.K >= 1024 && (long)((a.F + before - 1) / before) * a.tiles <= 128;
+  const int weights = direct ? kDirectWeights : kSmallWeights, cols = PAIRED ? weights / 2 : weights;
   a.col_tiles = (a.F + cols - 1) / cols;
-  hipLaunchKernelGGL(expert_gemm_kernel<PAIRED>, dim3((unsigned)(a.col_tiles * a.tiles)), dim3(256), 0, s, a);
+  const dim3 grid((unsigned)(a.col_tiles * a.tiles));
+  if (!direct) {
+    hipLaunchKernelGGL(expert_gemm_kernel<PAIRED>, grid, dim3(256), 0, s, a);
+    return BASED_OK;
+  }
+  static std::atomic<bool> allowed[kMaxDevices];
+  const int rc = allow_lds(reinterpret_cast<const void*>(expert_gemm_direct_kernel<PAIRED>), kDirectLds, allowed);
+  if (rc != BASED_OK) return rc;
+  hipLaunchKernelGGL(expert_gemm_direct_kernel<PAIRED>, grid, dim3(256), kDirectLds, s, a);
+  return BASED_OK;
 }
 
 template <bool PAIRED> int launch_expert_product(const ExpertGemmArgs& a, int rows, hipStream_t s) {
   if (rows == BASED_EXPERT_TILE_ROWS)
     return a.K % kGemmK == 0 ? launch_expert_gemm_large<PAIRED, false>(a, s) : launch_expert_gemm_large<PAIRED, true>(a, s);
-  launch_expert_gemm<PAIRED>(a, s);
-  return BASED_OK;
+  return launch_expert_gemm<PAIRED>(a, s);
 }
 
 // y[n] = sum of the rows of its choices

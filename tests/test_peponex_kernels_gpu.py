@@ -654,3 +654,21 @@ def test_experts_in_whole_large_tiles_with_a_part_of_a_round(dev, n, D, F, E, to
     clear = s[:, top - 1] - s[:, top] > 1e-5
     assert clear.sum() >= 0.98 * n
     close(got[clear], want[clear], 2 * TOL[BF16])
+
+
+@pytest.mark.parametrize("n,D,F,E,top", [(34, 1024, 1024, 1, 1), (100, 1024, 1024, 1, 1), (40, 1024, 1032, 2, 1), (50, 1000, 1024, 4, 2), (60, 72, 2048, 8, 1),
+                                         (33, 1280, 8, 5, 2), (90, 1152, 1408, 3, 2), (128, 2048, 1024, 2, 1), (17, 1024, 1024, 8, 2)])
+def test_experts_straight_into_lds(dev, n, D, F, E, top):
+    """Tiles of 32 rows and 64 of the weights: one expert and several, of which one has few rows; features that end inside a tile; either product
+    alone and both; an odd and an even number of rounds."""
+    from based_amd import ops
+
+    h, router, w1, w2, w = expert_case(n, D, F, E, top, BF16, seed=n)
+    router[0] = 0.2 * router[0]
+    w["m.router"] = router.double()
+    want = O.expert_mlp(h.double(), w, "m", {"router": {"top": top}})
+    got = ops.experts(h.to(dev), router.to(dev), w1.to(dev), w2.to(dev), top).double().cpu()
+    s = O.sigmoid(h.double() @ router.double().T).sort(-1, descending=True).values
+    clear = torch.ones(n, dtype=torch.bool) if top == E else s[:, top - 1] - s[:, top] > 1e-5
+    assert clear.sum() >= 0.9 * n
+    close(got[clear], want[clear], 2 * TOL[BF16])
