@@ -15,7 +15,10 @@
 
 namespace based {
 
-constexpr int kConvTokens = 8;   // tokens per thread in the prefill kernel
+// Tokens per thread in the prefill kernel: few where more would leave compute units without a workgroup, whose threads then wait for one round of loads in
+// place of two.  us, bf16, 2048 channels with the state, 8 tokens and 2 (and the state's stores in pieces): 4 x 128 tokens (64 workgroups) 9.6 -> 4.7, 1 x 30 7.9 ->
+// 3.4, 8 x 128 10.9 -> 6.1, 16 x 128 (256) 12.9 -> 8.8; in pieces alone 8 x 2048 41.7 -> 39.8.
+constexpr int kConvTokens = 8, kConvTokensFew = 2;
 constexpr int kConvMaxK = 4;      // supported kernel sizes: 2..4
 
 template <typename T> struct Vec16;
@@ -43,7 +46,7 @@ __device__ __forceinline__ void store_dyn(void* p, long i, int dtype, float x) {
     reinterpret_cast<float*>(p)[i] = x;
 }
 
-template <typename T, int K>
+template <typename T, int K, int TOK>
 __global__ __launch_bounds__(256) void gated_conv_prefill_kernel(
     const T* __restrict__ u, const T* __restrict__ weight, const T* __restrict__ bias, T* __restrict__ y,
     void* __restrict__ state, int L, int D, long u_sb, long u_sl, long y_sb, long y_sl, int state_dtype, int gated) {
@@ -51,7 +54,7 @@ __global__ __launch_bounds__(256) void gated_conv_prefill_kernel(
   typedef typename Vec16<T>::type vec_t;
   const int c0 = (blockIdx.x * 256 + threadIdx.x) * N;  // first channel of this thread
   if (c0 >= D) return;
-  const int l0 = blockIdx.y * kConvTokens;
+  const int l0 = blockIdx.y * TOK;
   const int b = blockIdx.z;
   const T* u1 = u + b * u_sb + c0;
   const T* u2 = u1 + D;
@@ -93,11 +96,11 @@ __global__ __launch_bounds__(256) void gated_conv_prefill_kernel(
     for (int c = 0; c < N; ++c) win[j][c] = to_f32(x[c]);
   }
 
-  const int ntok = L - l0 < kConvTokens ? L - l0 : kConvTokens;
+  const int ntok = L - l0 < TOK ? L - l0 : TOK;
   const T* gate_src = gated ? u2 : u1;  // without a gate the second operand is fetched and ignored
-  constexpr int kBatch = 4;  // tokens whose loads are in flight together
+  constexpr int kBatch = TOK < 4 ? TOK : 4;  // tokens whose loads are in flight together
 #pragma unroll
-  for (int t0 = 0; t0 < kConvTokens; t0 += kBatch) {
+  for (int t0 = 0; t0 < TOK; t0 += kBatch) {
     vec_t x1[kBatch], x2[kBatch];
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
@@ -126,16 +129,37 @@ __global__ __launch_bounds__(256) void gated_conv_prefill_kernel(
 
   // rolling state for decoding: the last K inputs of every channel, oldest first
   if (state != nullptr && l0 + ntok == L) {
+    // after the last token the window holds inputs L-K+1 .. L-1 in win[0..K-2]; input L-K is
+    // gone from it, so it is read again (it exists only if L >= K)
+    const vec_t oldest = keep_if(*reinterpret_cast<const vec_t*>(u1 + (long)(L >= K ? L - K : 0) * u_sl), L >= K);
+    float run[N * K];
 #pragma unroll
     for (int c = 0; c < N; ++c) {
-      const long base = ((long)b * D + c0 + c) * K;
-      // after the last token the window holds inputs L-K+1 .. L-1 in win[0..K-2]; input L-K is
-      // gone from it, so re-read it (it exists only if L >= K)
-      float oldest = 0.0f;
-      if (L - K >= 0) oldest = to_f32(u1[(long)(L - K) * u_sl + c]);
-      store_dyn(state, base, state_dtype, oldest);
+      run[c * K] = to_f32(oldest[c]);
 #pragma unroll
-      for (int j = 1; j < K; ++j) store_dyn(state, base + j, state_dtype, win[j - 1][c]);
+      for (int j = 1; j < K; ++j) run[c * K + j] = win[j - 1][c];
+    }
+    const long base = ((long)b * D + c0) * K;
+    // (one by one the stores of the last tokens' threads outlast the others': 24 of two bytes each, bf16)
+    if (state_dtype == BASED_BF16) {
+      __bf16* at = static_cast<__bf16*>(state) + base;
+      if (reinterpret_cast<uintptr_t>(state) % 8 == 0) {
+#pragma unroll
+        for (int i = 0; i < N * K / 4; ++i)
+          *reinterpret_cast<bf16x4*>(at + i * 4) = bf16x4{(__bf16)run[i * 4], (__bf16)run[i * 4 + 1], (__bf16)run[i * 4 + 2], (__bf16)run[i * 4 + 3]};
+      } else {
+#pragma unroll
+        for (int i = 0; i < N * K; ++i) at[i] = (__bf16)run[i];
+      }
+    } else {
+      float* at = static_cast<float*>(state) + base;
+      if (reinterpret_cast<uintptr_t>(state) % 16 == 0) {
+#pragma unroll
+        for (int i = 0; i < N * K / 4; ++i) *reinterpret_cast<f32x4*>(at + i * 4) = f32x4{run[i * 4], run[i * 4 + 1], run[i * 4 + 2], run[i * 4 + 3]};
+      } else {
+#pragma unroll
+        for (int i = 0; i < N * K; ++i) at[i] = run[i];
+      }
     }
   }
 }
@@ -230,12 +254,20 @@ int launch_gated_conv_prefill(const void* u, const void* weight, const void* bia
                               int64_t B, int64_t L, int64_t D, int K, int64_t u_sb, int64_t u_sl,
                               int64_t y_sb, int64_t y_sl, int state_dtype, int gated, hipStream_t stream) {
   constexpr int N = Vec16<T>::kN;
-  dim3 grid((unsigned)((D / N + 255) / 256), (unsigned)((L + kConvTokens - 1) / kConvTokens), (unsigned)B), block(256);
-#define BASED_CONV_CASE(KK)                                                                               \
-  case KK:                                                                                                \
-    hipLaunchKernelGGL((gated_conv_prefill_kernel<T, KK>), grid, block, 0, stream, (const T*)u,            \
-                       (const T*)weight, (const T*)bias, (T*)y, state, (int)L, (int)D, u_sb, u_sl, y_sb,   \
-                       y_sl, state_dtype, gated);                                                         \
+  const int64_t across = (D / N + 255) / 256;
+  const bool few = across * ((L + kConvTokens - 1) / kConvTokens) * B <= 256;
+  const int tokens = few ? kConvTokensFew : kConvTokens;
+  dim3 grid((unsigned)across, (unsigned)((L + tokens - 1) / tokens), (unsigned)B), block(256);
+#define BASED_CONV_CASE(KK)                                                                                \
+  case KK:                                                                                                 \
+    if (few)                                                                                               \
+      hipLaunchKernelGGL((gated_conv_prefill_kernel<T, KK, kConvTokensFew>), grid, block, 0, stream, (const T*)u, \
+                         (const T*)weight, (const T*)bias, (T*)y, state, (int)L, (int)D, u_sb, u_sl, y_sb,  \
+                         y_sl, state_dtype, gated);                                                        \
+    else                                                                                                   \
+      hipLaunchKernelGGL((gated_conv_prefill_kernel<T, KK, kConvTokens>), grid, block, 0, stream, (const T*)u, \
+                         (const T*)weight, (const T*)bias, (T*)y, state, (int)L, (int)D, u_sb, u_sl, y_sb,  \
+                         y_sl, state_dtype, gated);                                                        \
     break;
   switch (K) {
     BASED_CONV_CASE(2)

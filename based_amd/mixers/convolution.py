@@ -33,7 +33,7 @@ class ShortConvolution(nn.Module):
         if inference_params.seqlen_offset > 0:
             state = self._get_state(inference_params)
             return ops.gated_conv_step(x, state[: x.shape[0]], weight, bias, gated=False)
-        self._init_state(inference_params)
+        self._init_state(inference_params, x)
         state = self._get_state(inference_params)
         return ops.gated_conv_prefill(x, weight, bias, state=state[: x.shape[0]], gated=False)
 
@@ -41,9 +41,10 @@ class ShortConvolution(nn.Module):
         return torch.zeros(batch_size, self.d_model, self.kernel_size, device=self.conv.weight.device,
                            dtype=self.conv.weight.dtype if dtype is None else dtype)
 
-    def _init_state(self, inference_params):
+    def _init_state(self, inference_params, x=None):
         """Creates the state if it does not exist, zeroes it otherwise (a pre-allocated state may
-        be larger than the running batch; it is cleared whole)."""
+        be larger than the running batch; it is cleared whole, but for the rows that the
+        convolution over x (b, l, ..) leaves complete anyway)."""
         outer, inner = self.layer_idx if isinstance(self.layer_idx, tuple) else (self.layer_idx, None)
         d = inference_params.key_value_memory_dict
         outer = inference_params.layer_key(outer)
@@ -51,7 +52,9 @@ class ShortConvolution(nn.Module):
             d = d.setdefault(outer, {})
         key = outer if inner is None else inner
         if key in d:
-            d[key].zero_()
+            written = x.shape[0] if x is not None and x.shape[1] > 0 else 0
+            if written < d[key].shape[0]:
+                d[key][written:].zero_()
         else:
             d[key] = self.allocate_inference_cache(inference_params.max_batch_size, inference_params.max_seqlen)
 
@@ -111,7 +114,7 @@ class BaseConv(nn.Module):
         if inference_params.seqlen_offset > 0:
             state = self.conv._get_state(inference_params)
             return ops.gated_conv_step(u, state[: u.shape[0]], weight, bias)
-        self.conv._init_state(inference_params)
+        self.conv._init_state(inference_params, u)
         state = self.conv._get_state(inference_params)
         return ops.gated_conv_prefill(u, weight, bias, state=state[: u.shape[0]])
 

@@ -123,3 +123,23 @@ def test_convolution_alone_prefill_and_steps(dev, K, dtype):
     for t in range(L, L + T):
         yt = ops.gated_conv_step(xd[:, t:t + 1], state, wd, None, gated=False)
         assert rel_l2(yt.float(), ref[:, t:t + 1]) < tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("state_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,L,D,K", [(1, 1, 64, 3), (2, 2, 72, 4), (3, 3, 64, 2), (2, 9, 2048, 3), (1, 31, 264, 4), (5, 160, 1024, 3), (40, 33, 2048, 2)])
+def test_few_and_many_tokens_a_thread_and_the_state(dev, B, L, D, K, dtype, state_dtype):
+    """Prompts on either side of the line, whole pairs of tokens and one more or less; states on and off 16 bytes, of either type."""
+    from based_amd import ops
+
+    g = torch.Generator().manual_seed(L * D + K)
+    u, w, b = (torch.randn(*s, generator=g).to(dtype).to(dev) for s in ((B, L, 2 * D), (D, 1, K), (D,)))
+    x = torch.nn.functional.pad(u[..., :D].double(), (0, 0, K, 0))
+    conv = sum(x[:, j + 1:j + 1 + L] * w.double()[:, 0, j] for j in range(K)) + b.double()
+    want = torch.nn.functional.silu(conv) * u[..., D:].double()
+    for off in (0, 1):
+        state = torch.full((B * D * K + 1,), float("nan"), dtype=state_dtype, device=dev)[off:off + B * D * K].view(B, D, K)
+        y = ops.gated_conv_prefill(u, w, b, state=state)
+        # one rounding of bf16 (2^-9), or a few of fp32
+        assert float((y.double() - want).norm() / want.norm()) < (4e-3 if dtype == torch.bfloat16 else 1e-6)
+        assert torch.equal(state, x[:, -K:].transpose(1, 2).to(dtype).to(state_dtype))
