@@ -132,6 +132,7 @@ SIGNATURES = {
     "based_gated_delta_scan": (C.c_int, [_P] * 10 + [_I64] * 11 + [C.c_int, C.c_int, _P]),
     "based_gated_delta_scan_work": (_I64, [_I64] * 5),
     "based_gated_delta_scan_work_of": (_I64, [_P, _P] + [_I64] * 7),
+    "based_gated_delta_scan_work_as": (_I64, [_P, _P] + [_I64] * 7 + [C.c_int]),
     "based_gated_delta_scan_chunks": (C.c_int, [_P] * 10 + [_I64] * 11 + [C.c_int, C.c_int, _P]),
     "based_gated_rms_norm": (C.c_int, [_P] * 4 + [_I64] * 8 + [C.c_float, C.c_float, C.c_int, _P]),
     "based_gated_delta_step": (

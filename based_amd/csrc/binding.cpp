@@ -90,6 +90,7 @@ Listed kEntries[] = {
     BASED_ENTRY(based_window_attn_step),
     BASED_ENTRY(based_gated_delta_scan),
     BASED_ENTRY(based_gated_delta_scan_work_of),
+    BASED_ENTRY(based_gated_delta_scan_work_as),
     BASED_ENTRY(based_gated_delta_scan_chunks),
     BASED_ENTRY(based_gated_rms_norm),
     BASED_ENTRY(based_gated_delta_step),

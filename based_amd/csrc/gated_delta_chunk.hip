@@ -753,8 +753,21 @@ constexpr int64_t kDcWorkFloats = 64ll << 20;  // 256 MB, which the last-level c
 //   8, 96 x 96: L = 256: 41, 35.  32, 96 x 256: L = 384: 59, 61; L = 1024: 131, 121.  64, 96 x 128: L = 512: 75, 77; L = 2048: 263, 298.
 //   8, 128 x 128: L = 256: 35.0, 35.4; L = 320: 40, 38.  32, 128 x 128: L = 320: 41, 42; L = 384: 47, 45.  16, 128 x 256: L = 384: 45, 47;
 //   L = 512: 56, 52.  More heads: 128, 64 x 64, L = 4096: 415, 493; more channels: 16, 256 x 256, L = 300: 62.6, 66.0.
-static bool dc_faster(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
+// More heads than 64, in bf16 alone, which takes a third of the products of fp32, and of the sizes that were measured, which fill their
+// tiles.  us, blocks of 16 against chunks, heads, d x dv:
+//   72, 64 x 64: L = 256: 38.5, 29.8; L = 1500: 167, 87.  72, 64 x 128: 46.4, 34.6; 206, 130.  72, 128 x 128: 92, 50; 444, 204.
+//   112, L = 800: 64 x 64: 102, 68; 64 x 128: 120, 98; 128 x 64: 132, 110; 128 x 128: 254, 164.
+//   128, 64 x 64: L = 256: 38.7, 31.8; L = 2048: 210, 188.  128, 64 x 128: L = 256: 47.9, 42.3; L = 512: 80, 68; L = 1024: 146, 175.
+//   128, 128 x 64: L = 256: 55.5, 45; L = 2048: 341, 322.  128, 128 x 128: 85.8, 66.8; 575, 474.
+//   256, L = 256: 64 x 64: 54, 52; 64 x 128: 76, 81; 128 x 128: 160, 179; L = 1024: 64 x 64: 170, 247.  fp32, 128, 64 x 128: L = 512: 78, 105.
+static bool dc_faster_many(int64_t heads, int64_t L, int64_t D, int64_t DV) {
+  if (heads > 128 || L < BASED_DELTA_CHUNKS_MIN || DV < 64 || DV > 128) return false;
+  if (D > 48 && D <= 64) return DV <= 64 || heads <= 112 || L <= 512;
+  return D > 112 && D <= 128;
+}
+static bool dc_faster(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, bool bf16) {
   const int64_t heads = B * H, tiles = (DV + 15) / 16, wgs = heads * tiles;  // (of the scan, two of which a compute unit holds)
+  if (bf16 && heads > 64) return dc_faster_many(heads, L, D, DV);
   if (heads > 64 || wgs > 512 || D > 128) return false;
   const bool crowded = wgs > 256;
   const int64_t wide = tiles > 16 ? (tiles - 16) / 8 : 0;
@@ -777,8 +790,8 @@ static bool dc_faster(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
 static int dc_tiles(int64_t D) { return D <= 64 ? 4 : 8; }
 
 // chunks per span, 0 where blocks of 16 are for the shape
-static int64_t dc_span(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
-  if (B <= 0 || L <= 0 || H <= 0 || D <= 0 || DV <= 0 || B >= (1ll << 31) || H >= (1ll << 31) || DV >= (1ll << 20) || !dc_faster(B, L, H, D, DV))
+static int64_t dc_span(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, bool bf16) {
+  if (B <= 0 || L <= 0 || H <= 0 || D <= 0 || DV <= 0 || B >= (1ll << 31) || H >= (1ll << 31) || DV >= (1ll << 20) || !dc_faster(B, L, H, D, DV, bf16))
     return 0;
   const int64_t chunks = (L + kDc - 1) / kDc, each = B * H * dc_floats(dc_tiles(D), 3, (int)DV);
   int64_t span = kDcWorkFloats / each;  // (at least 29: a chunk of 64 heads and 512 value tiles takes 2.3 M floats at most)
@@ -823,7 +836,7 @@ template <typename T> static int run_delta(const DeltaChunkArgs& a, bool vec, in
 
 extern "C" BASED_API int64_t based_gated_delta_scan_work(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
   using namespace based;
-  const int64_t span = dc_span(B, L, H, D, DV);
+  const int64_t span = dc_span(B, L, H, D, DV, false);
   return span == 0 ? 0 : B * H * span * dc_floats(dc_tiles(D), 3, (int)DV);
 }
 
@@ -832,6 +845,14 @@ extern "C" BASED_API int64_t based_gated_delta_scan_work_of(const void* q, const
   using namespace based;
   if (!dc_near(H, DV, x_sl) || !(D <= 64 || dc_vec(q, k, B, D, x_sb, x_sl))) return 0;
   return based_gated_delta_scan_work(B, L, H, D, DV);
+}
+
+extern "C" BASED_API int64_t based_gated_delta_scan_work_as(const void* q, const void* k, int64_t B, int64_t L, int64_t H, int64_t D,
+                                                            int64_t DV, int64_t x_sb, int64_t x_sl, int io_dtype) {
+  using namespace based;
+  if (!dc_near(H, DV, x_sl) || !(D <= 64 || dc_vec(q, k, B, D, x_sb, x_sl))) return 0;
+  const int64_t span = dc_span(B, L, H, D, DV, io_dtype == BASED_BF16);
+  return span == 0 ? 0 : B * H * span * dc_floats(dc_tiles(D), 3, (int)DV);
 }
 
 extern "C" BASED_API int based_gated_delta_scan_chunks(const void* q, const void* k, const void* v, const void* a_gate, const void* b_gate,
@@ -851,7 +872,7 @@ extern "C" BASED_API int based_gated_delta_scan_chunks(const void* q, const void
   if (B == 0 || L == 0) return BASED_OK;
   BASED_REQUIRE(dc_near(H, DV, x_sl), BASED_ERR_SHAPE, "%s: rows too long", who);
   BASED_REQUIRE(aligned_to(work, 16), BASED_ERR_ALIGN, "%s: the work space must be 16-byte aligned", who);
-  const int64_t span = dc_span(B, L, H, D, DV);
+  const int64_t span = dc_span(B, L, H, D, DV, io_dtype == BASED_BF16);
   BASED_REQUIRE(span > 0 && B * H * span < (1ll << 31), BASED_ERR_SHAPE, "%s: the shape is for blocks of 16", who);
   const bool vec = dc_vec(q, k, B, D, x_sb, x_sl);
   BASED_REQUIRE(vec || D <= 64, BASED_ERR_ALIGN, "%s: chunks of heads of more than 64 channels take rows of whole 16-byte pieces", who);

@@ -1066,7 +1066,7 @@ def gated_delta_scan(q, k, v, a_gate, b_gate, a_log, dt_bias, state, heads: int,
     o = torch.empty(B, L, heads, dv, dtype=torch.float32, device=q.device)
     lib, floats = _lib.lib(), 0
     if L >= DELTA_CHUNKS_MIN:
-        floats = lib.based_gated_delta_scan_work_of(q.data_ptr(), k.data_ptr(), B, L, heads, d, dv, x_sb, x_sl)
+        floats = lib.based_gated_delta_scan_work_as(q.data_ptr(), k.data_ptr(), B, L, heads, d, dv, x_sb, x_sl, code)
     if floats:
         scan, work = lib.based_gated_delta_scan_chunks, torch.empty(floats, dtype=torch.float32, device=q.device)
     else:

@@ -176,3 +176,18 @@ def test_parts_of_small_and_large_values(dev, dtype, d, dv, scale):
         ref, S_ref = reference(*case, H, H, d, dv, S_ref)
         # (norms of 1e-24 have no squares in 32 bits)
         assert rel_l2(o.double() / scale, ref / scale) < TOL and rel_l2(S.double() / scale, S_ref / scale) < TOL
+
+
+@pytest.mark.parametrize("B,L,H,d,dv,chunks", [(5, 256, 13, 64, 64, True), (13, 257, 5, 128, 128, True), (8, 512, 16, 64, 128, True),
+                                               (8, 513, 16, 64, 128, False), (5, 300, 13, 112, 64, False), (43, 256, 3, 64, 64, False)])
+def test_many_heads(dev, B, L, H, d, dv, chunks):
+    """More than 64 heads: chunks in bf16 where they are the faster form, blocks in fp32 and in front of and behind it."""
+    from based_amd import _lib
+
+    x, ab, a_log, dt_bias = (t.to(dev) for t in make(B + L, B, L, H, H, d, dv, torch.bfloat16))
+    at = lambda dtype: _lib.lib().based_gated_delta_scan_work_as(x.data_ptr(), x.data_ptr(), B, L, H, d, dv, *x.stride()[:2], dtype) > 0
+    assert at(_lib.BASED_BF16) == chunks and not at(_lib.BASED_F32) and not in_chunks(B, L, H, d, dv)
+    got, S = run((x, ab, a_log, dt_bias), H, H, d, dv, empty_state(B, H, d, dv, dev))
+    want, T = reference(x, ab, a_log, dt_bias, H, H, d, dv)
+    tol = TOL if chunks else 3e-6  # (blocks: as above)
+    assert rel_l2(got, want) < tol and rel_l2(S, T) < tol
