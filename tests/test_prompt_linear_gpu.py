@@ -92,6 +92,21 @@ def test_modules_that_are_watched(dev):
     assert mlp.fc1.weight.grad is not None
 
 
+def test_module_with_a_forward_of_its_own(dev):
+    """A wrapper that replaces the projection's forward (to move weights, to add a term) is called in front of the gate, too."""
+    from based_amd.stack import GatedMlp
+
+    mlp = GatedMlp(256, hidden_features=512, device=dev, dtype=torch.bfloat16)
+    x = torch.randn(2, 40, 256, device=dev).bfloat16()
+    inner = mlp.fc1.forward
+    with torch.no_grad():
+        plain = mlp(x)
+        mlp.fc1.forward = lambda x: inner(x) * 0
+        assert not mlp(x).any()
+        del mlp.fc1.forward
+        assert torch.equal(mlp(x), plain)
+
+
 @torch.inference_mode()
 def test_in_a_recorded_graph(dev):
     """Recorded in the mode the models record in."""
