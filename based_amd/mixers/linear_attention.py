@@ -3,7 +3,7 @@
 Drop-in for based/models/mixers/linear_attention.py of the reference: same constructor
 arguments, parameter names (proj_q / proj_k / proj_v / out_proj), forward /
 recurrent_forward / allocate_inference_cache signatures and cache layout.  The q/k/v and
-output projections stay ordinary nn.Linear GEMMs; everything between them (feature map,
+output projections are nn.Linear GEMMs (of few tokens by kernels here); everything between them (feature map,
 causal product, normaliser, decode-state construction and update) is one HIP kernel call.
 There is no non-HIP path: tensors must live on the GPU.
 """
