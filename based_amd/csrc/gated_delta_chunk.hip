@@ -743,31 +743,44 @@ __global__ __launch_bounds__(512, dc_lone(RB) ? 2 : 4) void delta_chunk_scan_ker
 // Workspace: the chunks of one launch pair.  Long prompts go through it in spans of chunks, the state carried on in between.
 constexpr int64_t kDcWorkFloats = 64ll << 20;  // 256 MB, which the last-level cache holds between the two launches
 
-// Where chunks are the faster form: few heads, and enough chunks.  A chunk step of the scan takes 1.3 us (1.6 with heads of more than 64
+// In bf16 chunks take 0.57 to 0.83 of the times that the rule for fp32, below, was made of.  They are slower only where channels are few,
+// which makes the blocks' steps cheap, and where workgroups are many, each of which reads what is formed ahead.  us, blocks of 16 against chunks, heads, d x dv (in 900 shapes, 0.24 to 1.03 of the time where the rule takes them):
+//   1, 64 x 16: L = 256: 27, 17.  24, 34 x 332: L = 700: 160, 45.  32, 64 x 512: L = 1024: 146, 93.  64, 128 x 256: L = 256: 81, 57; L = 1024: 269, 172.
+//   64, 32 x 128: L = 256: 29, 30; L = 320: 34, 31; L = 1024: 85, 56.  48, 32 x 256: L = 1024: 113, 80.  64, 32 x 256: L = 1024: 90, 98.
+//   4, 16 x 512: L = 256: 23, 24; L = 384: 30, 28.  64, 16 x 64: L = 320: 28, 27.  64, 16 x 128: L = 384: 34, 34; L = 512: 41, 37.  48, 16 x 256: L = 512: 41, 50.
+//   72, 64 x 128: L = 1500: 206, 130.  112, 48 x 128: L = 1024: 117, 129.  112, 64 x 128: L = 800: 120, 98.  112, 80 x 16: L = 1024: 141, 102; 80 x 64: 143, 147.
+//   80, 96 x 128: L = 256: 64, 50.  128, 48 x 64: L = 1024: 116, 88.  128, 64 x 128: L = 256: 48, 42; L = 512: 80, 68; L = 1024: 146, 175.
+//   128, 128 x 64: L = 2048: 341, 322.  128, 128 x 128: L = 256: 86, 67; L = 2048: 575, 474.
+//   256, L = 256: 64 x 64: 54, 52; 64 x 128: 76, 81; 128 x 128: 160, 179.  256, 64 x 64: L = 1024: 170, 247.
+//   Long prompts take several launches, for what is formed ahead is 256 MB at most: 64, 48 x 256: L = 1024: 114, 99; L = 4096: 402, 454.
+//   128, 112 x 128: L = 1024: 275, 253; L = 4096: 1,011, 1,051; 128 x 128: 1,167, 992.  112, 64 x 128, L = 4096: 586, 504.
+static bool dc_faster_bf16(int64_t heads, int64_t L, int64_t D, int64_t DV) {
+  const int64_t tiles = (DV + 15) / 16, wgs = heads * tiles;
+  if (heads > 128 || wgs > 1024 || D > 128 || L < BASED_DELTA_CHUNKS_MIN) return false;
+  if (heads > 64) {
+    if (DV > 128 || D <= 32) return false;
+    if (D <= 64) return DV <= 64 || heads <= 80 || (D > 48 && (heads <= 112 || L <= 512));
+    if (heads > 112 && D > 104 && (D <= 112 || DV <= 32)) return L <= 1024;
+    return D > 104 || heads <= 80 || DV <= 16;
+  }
+  if (D > 32) return D > 48 || wgs <= 768 || L <= 1024;
+  if (D > 16) return wgs <= 768 && L >= (wgs <= 448 ? 4 : tiles <= 16 ? 5 : 6) * kDc;
+  return wgs <= 512 && L >= (wgs > 256 ? 8 : wgs > 128 || heads > 48 || tiles > 16 ? 6 : 4) * kDc;
+}
+
+// Where chunks are the faster form in fp32: few heads, and enough chunks.  A chunk step of the scan takes 1.3 us (1.6 with heads of more than 64
 // channels, which fill eight tiles whatever their size) where four blocks of 16 take 3.2 to 6.8, by the size of the heads; but both
 // launches together start 8 to 10 us later than those of the blocks, values of many tiles read every chunk's rows once each, and every head
 // adds 20 to 90 ns of preparation a chunk: 26 times a block's products, and more memory than the cache holds at the far end.  us, blocks
-// of 16 against chunks as they were with fp32 products (bf16 chunks take 0.57 to 0.83 of that since, fp32 0.8 to 1.02), heads, d x dv:
+// of 16 against chunks as they were with products on fp32 MFMA (they take 0.8 to 1.02 of that since), heads, d x dv:
 //   8, 64 x 64: L = 256: 27.7, 24.0.  32, 64 x 128: L = 256: 29, 28; L = 2048: 161, 91.  64, 64 x 128: L = 256: 33, 35; L = 384: 45, 43.
 //   64, 32 x 128: L = 512: 47, 48; L = 2048: 154, 170.  8, 64 x 512: L = 256: 30, 34; L = 384: 39, 38.
 //   8, 96 x 96: L = 256: 41, 35.  32, 96 x 256: L = 384: 59, 61; L = 1024: 131, 121.  64, 96 x 128: L = 512: 75, 77; L = 2048: 263, 298.
 //   8, 128 x 128: L = 256: 35.0, 35.4; L = 320: 40, 38.  32, 128 x 128: L = 320: 41, 42; L = 384: 47, 45.  16, 128 x 256: L = 384: 45, 47;
 //   L = 512: 56, 52.  More heads: 128, 64 x 64, L = 4096: 415, 493; more channels: 16, 256 x 256, L = 300: 62.6, 66.0.
-// More heads than 64, in bf16 alone, which takes a third of the products of fp32, and of the sizes that were measured, which fill their
-// tiles.  us, blocks of 16 against chunks, heads, d x dv:
-//   72, 64 x 64: L = 256: 38.5, 29.8; L = 1500: 167, 87.  72, 64 x 128: 46.4, 34.6; 206, 130.  72, 128 x 128: 92, 50; 444, 204.
-//   112, L = 800: 64 x 64: 102, 68; 64 x 128: 120, 98; 128 x 64: 132, 110; 128 x 128: 254, 164.
-//   128, 64 x 64: L = 256: 38.7, 31.8; L = 2048: 210, 188.  128, 64 x 128: L = 256: 47.9, 42.3; L = 512: 80, 68; L = 1024: 146, 175.
-//   128, 128 x 64: L = 256: 55.5, 45; L = 2048: 341, 322.  128, 128 x 128: 85.8, 66.8; 575, 474.
-//   256, L = 256: 64 x 64: 54, 52; 64 x 128: 76, 81; 128 x 128: 160, 179; L = 1024: 64 x 64: 170, 247.  fp32, 128, 64 x 128: L = 512: 78, 105.
-static bool dc_faster_many(int64_t heads, int64_t L, int64_t D, int64_t DV) {
-  if (heads > 128 || L < BASED_DELTA_CHUNKS_MIN || DV < 64 || DV > 128) return false;
-  if (D > 48 && D <= 64) return DV <= 64 || heads <= 112 || L <= 512;
-  return D > 112 && D <= 128;
-}
 static bool dc_faster(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, bool bf16) {
   const int64_t heads = B * H, tiles = (DV + 15) / 16, wgs = heads * tiles;  // (of the scan, two of which a compute unit holds)
-  if (bf16 && heads > 64) return dc_faster_many(heads, L, D, DV);
+  if (bf16) return dc_faster_bf16(heads, L, D, DV);
   if (heads > 64 || wgs > 512 || D > 128) return false;
   const bool crowded = wgs > 256;
   const int64_t wide = tiles > 16 ? (tiles - 16) / 8 : 0;
@@ -794,7 +807,7 @@ static int64_t dc_span(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, b
   if (B <= 0 || L <= 0 || H <= 0 || D <= 0 || DV <= 0 || B >= (1ll << 31) || H >= (1ll << 31) || DV >= (1ll << 20) || !dc_faster(B, L, H, D, DV, bf16))
     return 0;
   const int64_t chunks = (L + kDc - 1) / kDc, each = B * H * dc_floats(dc_tiles(D), 3, (int)DV);
-  int64_t span = kDcWorkFloats / each;  // (at least 29: a chunk of 64 heads and 512 value tiles takes 2.3 M floats at most)
+  int64_t span = kDcWorkFloats / each;  // (at least 11: a chunk of 128 heads of 128 channels and 8 value tiles takes 5.9 M floats at most)
   if (span > chunks) span = chunks;
   // spans of about equal length
   const int64_t n = (chunks + span - 1) / span;

@@ -179,9 +179,11 @@ def test_parts_of_small_and_large_values(dev, dtype, d, dv, scale):
 
 
 @pytest.mark.parametrize("B,L,H,d,dv,chunks", [(5, 256, 13, 64, 64, True), (13, 257, 5, 128, 128, True), (8, 512, 16, 64, 128, True),
-                                               (8, 513, 16, 64, 128, False), (5, 300, 13, 112, 64, False), (43, 256, 3, 64, 64, False)])
+                                               (8, 513, 16, 64, 128, False), (7, 300, 13, 80, 64, False), (43, 256, 3, 64, 64, False),
+                                               (4, 256, 16, 128, 256, True), (4, 257, 12, 18, 52, True), (4, 511, 16, 16, 128, False),
+                                               (4, 512, 16, 16, 128, True), (4, 256, 16, 32, 252, False), (3, 320, 16, 32, 256, True)])
 def test_many_heads(dev, B, L, H, d, dv, chunks):
-    """More than 64 heads: chunks in bf16 where they are the faster form, blocks in fp32 and in front of and behind it."""
+    """Many heads, and few channels: chunks in bf16 where they are the faster form, blocks in fp32 and in front of and behind it."""
     from based_amd import _lib
 
     x, ab, a_log, dt_bias = (t.to(dev) for t in make(B + L, B, L, H, H, d, dv, torch.bfloat16))
