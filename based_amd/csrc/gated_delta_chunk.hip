@@ -744,7 +744,7 @@ __global__ __launch_bounds__(512, dc_lone(RB) ? 2 : 4) void delta_chunk_scan_ker
 constexpr int64_t kDcWorkFloats = 64ll << 20;  // 256 MB, which the last-level cache holds between the two launches
 
 // In bf16 chunks take 0.57 to 0.83 of the times that the rule for fp32, below, was made of.  They are slower only where channels are few,
-// which makes the blocks' steps cheap, and where workgroups are many, each of which reads what is formed ahead.  us, blocks of 16 against chunks, heads, d x dv (in 900 shapes, 0.24 to 1.03 of the time where the rule takes them):
+// which makes the blocks' steps cheap, and where workgroups are many, each of which reads what is formed ahead.  us, blocks of 16 against chunks, heads, d x dv (in 970 shapes, 0.24 to 1.00 of the time where the rule takes them):
 //   1, 64 x 16: L = 256: 27, 17.  24, 34 x 332: L = 700: 160, 45.  32, 64 x 512: L = 1024: 146, 93.  64, 128 x 256: L = 256: 81, 57; L = 1024: 269, 172.
 //   64, 32 x 128: L = 256: 29, 30; L = 320: 34, 31; L = 1024: 85, 56.  48, 32 x 256: L = 1024: 113, 80.  64, 32 x 256: L = 1024: 90, 98.
 //   4, 16 x 512: L = 256: 23, 24; L = 384: 30, 28.  64, 16 x 64: L = 320: 28, 27.  64, 16 x 128: L = 384: 34, 34; L = 512: 41, 37.  48, 16 x 256: L = 512: 41, 50.
