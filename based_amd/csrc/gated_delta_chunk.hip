@@ -780,7 +780,7 @@ static bool dc_faster_bf16(int64_t heads, int64_t L, int64_t D, int64_t DV) {
 //   L = 512: 56, 52.  More heads: 128, 64 x 64, L = 4096: 415, 493; more channels: 16, 256 x 256, L = 300: 62.6, 66.0.
 static bool dc_faster(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, bool bf16) {
   const int64_t heads = B * H, tiles = (DV + 15) / 16, wgs = heads * tiles;  // (of the scan, two of which a compute unit holds)
-  if (bf16) return dc_faster_bf16(heads, L, D, DV);
+  if (bf16 && dc_faster_bf16(heads, L, D, DV)) return true;  // (and what follows: a work space asked for without a type is for either)
   if (heads > 64 || wgs > 512 || D > 128) return false;
   const bool crowded = wgs > 256;
   const int64_t wide = tiles > 16 ? (tiles - 16) / 8 : 0;

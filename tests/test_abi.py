@@ -195,3 +195,23 @@ def test_delta_chunks_take_the_rows_they_can():
     chunks = lambda L, D, sl: lib.based_gated_delta_scan_chunks(*([p] * 10), 1, L, 4, 4, D, 64, 64, L * sl, sl, 4, 4, 1, 0, None)  # noqa: E731
     assert chunks(640, 132, 1280) == 1 and chunks(100, 128, 1280) == 1 and chunks(640, 128, 1 << 24) == 1  # BASED_ERR_SHAPE
     assert chunks(640, 128, 1281) == 3  # BASED_ERR_ALIGN
+
+
+def test_delta_work_of_no_type_serves_either_type():
+    """A shape that the queries without a type send through chunks of 64 tokens goes through them in either type, in no more work space: few
+    and many heads, channels and values on both sides of every tile count, lengths on both sides of the first chunks."""
+    lib = _lib.lib()
+    taken = 0
+    for B, H in [(1, 1), (1, 2), (1, 3), (2, 4), (1, 16), (3, 8), (4, 8), (6, 8), (4, 16), (5, 16), (8, 16), (9, 16)]:
+        for D in (8, 16, 17, 32, 33, 48, 49, 64, 65, 96, 97, 112, 128, 129):
+            for DV in (16, 17, 64, 128, 129, 256, 257, 272, 368, 369, 400, 512, 1024):
+                for L in (255, 256, 319, 320, 383, 384, 447, 448, 512, 640, 1024, 1025, 2048, 4096):
+                    floats = lib.based_gated_delta_scan_work(B, L, H, D, DV)
+                    of = lib.based_gated_delta_scan_work_of(None, None, B, L, H, D, DV, 0, 8 * 128)
+                    assert of == (floats if D <= 64 or D % 4 == 0 else 0)  # (rows of whole pieces above 64)
+                    if of > 0:
+                        taken += 1
+                        for dtype in (_lib.BASED_BF16, _lib.BASED_F32):
+                            own = lib.based_gated_delta_scan_work_as(None, None, B, L, H, D, DV, 0, 8 * 128, dtype)
+                            assert 0 < own <= floats, (B, H, D, DV, L, dtype)
+    assert taken > 2000
