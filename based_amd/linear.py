@@ -10,13 +10,17 @@ from torch.nn.modules import module as nn_module
 from . import ops
 
 
+def _watched() -> bool:
+    """Something watches or rewrites torch's operations here: a gradient of either mode, autocast, tracing, compiling, vmap (of which the weight or
+    the bias may be mapped and x not), a mode."""
+    return (torch.is_grad_enabled() or torch.compiler.is_compiling() or forward_ad._current_level >= 0 or torch.is_autocast_enabled("cuda")
+            or torch._C._is_tracing() or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0)
+
+
 def _plain(x, weight) -> bool:
-    """Nothing watches or rewrites torch's operations here: no gradient of either mode, no autocast, no tracing, compiling or vmap, no subclass
-    of a tensor."""
-    return (type(x) is torch.Tensor and type(weight) in (torch.Tensor, nn.Parameter) and not torch.compiler.is_compiling()
-            and not torch.is_grad_enabled() and x.is_cuda and forward_ad._current_level < 0 and not torch.is_autocast_enabled("cuda")
-            and not torch._C._is_tracing() and not torch._C._functorch.is_functorch_wrapped_tensor(x)
-            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0)
+    """Tensors on the GPU, no subclasses of them, and nothing that watches."""
+    return type(x) is torch.Tensor and type(weight) in (torch.Tensor, nn.Parameter) and x.is_cuda and not _watched()
 
 
 def linear(x, weight, bias=None):

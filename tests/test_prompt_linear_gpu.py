@@ -92,6 +92,26 @@ def test_modules_that_are_watched(dev):
     assert mlp.fc1.weight.grad is not None
 
 
+@pytest.mark.parametrize("M", [4, 40])
+def test_stacked_weights(dev, M):
+    """An ensemble: torch.vmap over weights, over biases and over both, the rows the same for all; each as the library takes it alone."""
+    from torch.func import functional_call
+
+    from based_amd.linear import Linear
+
+    torch.manual_seed(1)
+    fc = Linear(256, 1024, device=dev, dtype=torch.bfloat16)
+    x = torch.randn(2, M // 2, 256, device=dev).bfloat16()
+    stacked = {"weight": torch.randn(3, 1024, 256, device=dev).mul(1 / 16).bfloat16(), "bias": torch.randn(3, 1024, device=dev).bfloat16()}
+    with torch.no_grad():
+        for names in (("weight",), ("bias",), ("weight", "bias")):
+            mapped = {n: stacked[n] for n in names}
+            got = torch.vmap(lambda p: functional_call(fc, p, (x,)))(mapped)
+            for i in range(3):
+                w, b = (mapped[n][i] if n in mapped else getattr(fc, n).detach() for n in ("weight", "bias"))
+                assert rel_l2(got[i], reference(x.view(M, 256), w, b).view_as(got[i])) < 2.5e-3
+
+
 def test_module_with_a_forward_of_its_own(dev):
     """A wrapper that replaces the projection's forward (to move weights, to add a term) is called in front of the gate, too."""
     from based_amd.stack import GatedMlp
