@@ -19,12 +19,18 @@
 // row 4 quad + i of tile 2 n + p is element 32 n + 8 quad + 4 p + i, and the four results of a lane in both tiles are one operand.  State
 // tiles (channels), U (tokens) and the tiles of W and Uv that make it are dealt so; outputs are not.
 //
+// Products take 32 tokens at a time and hold zeros where a token does not see another.  What is no finite number stays out of the tiles of 16 tokens in
+// front of its own all the same, as in blocks: the first 16 of such 32 are formed a second time without the others, and the outputs'
+// wavefronts read zeros in their place (0 to 2 % of a call, 0.7 in the mean of 20 shapes).
+//
 // Against blocks of 16 (gated_delta_scan_kernel) a chain step takes in four times the tokens with two exchanges instead of one, and
 // nothing but W S0 and k^T U stands in the chain.  4 sequences x 8 heads of 2048 tokens, d = 64, dv = 128, bf16: 161 us in blocks, 91 with
 // fp32 products (41 of preparation, 55 of scan, 2.0 of whose 4.1 thousand cycles a chunk were products), now 67: preparation 24, bound by
 // what it writes (92 MB at 3.8 TB/s), and scan 41, 3.1 thousand cycles a chunk: 2.0 of the chain itself, the rest waits for the chunk's 62 KB
 // (without those loads 27 us, with all of them from L2 37).  d = 128: 226 -> 131 us (1 x 4096, 16 heads), fp32 232 -> 188.  Errors against
 // 64 bits: 1.9e-7 -> 1.4e-7.
+#include <type_traits>
+
 #include "gated_delta.hpp"
 
 namespace based {
@@ -109,6 +115,12 @@ template <int NX, int NY> __device__ __forceinline__ void product(const bf16x8 (
   sum[0] = mfma_bf16(x[0], y[0], sum[0]);
 }
 
+// The operand's first 16 of 32 contracted elements.
+template <int N> __device__ __forceinline__ void first_half(const bf16x8 (&x)[N], bf16x8 (&y)[N], int quad) {
+#pragma unroll
+  for (int n = 0; n < N; ++n) y[n] = quad < 2 ? x[n] : bf16x8{};
+}
+
 // RB: 16-channel tiles of queries and keys.  LAY as for Four.  Rows go through LDS 64 channels at a time: a lane's operands lie in 16
 // rows, and asked for one by one they cost 16 lines of cache per instruction.
 template <typename T, int LAY, int RB>
@@ -120,6 +132,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
   __shared__ __attribute__((aligned(16))) __bf16 s_x[2][NP][kDc][kDcRow];
   __shared__ __attribute__((aligned(16))) float s_a[kDc][kDc + 4];  // A, then T
   __shared__ double s_lc[kDc];
+  // what is no finite number, by the wavefront that saw it: values in either slab, keys
+  __shared__ __attribute__((aligned(16))) int s_odd[3][4];
   __shared__ __attribute__((aligned(16))) float s_beta[kDc], s_bg[kDc], s_fq[kDc], s_fk[kDc], s_e1k[kDc], s_e1q[kDc], s_e2[4 * kDc];
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -132,6 +146,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
   const T* v = static_cast<const T*>(a.v) + b * a.x_sb + (long)t0 * a.x_sl + (long)h * a.dv;
   float* ws = a.work + (long)blockIdx.x * a.per;
   const int dealt = (l16 >> 2) * 8 + (l16 & 3);  // (+ 4 p: row l16 of tile p of a pair)
+  const f32x4 none = {0.f, 0.f, 0.f, 0.f};
 
   // 64 channels from `e0` on of the chunk's rows: thread t has 4 channels of rows t / 16 + 16 j.  Rows past the last token are fetched
   // from it: gates of zero keep them out.
@@ -177,13 +192,22 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
     }
   };
   auto store_v = [&](int buf, const t4 (&x)[4], int e0) {
+    float zero = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       t4 r = x[j];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) r[i] = e0 + piece + i < a.dv ? r[i] : (T)0.0f;
+      for (int i = 0; i < 4; ++i) {
+        r[i] = e0 + piece + i < a.dv ? r[i] : (T)0.0f;
+        zero = __builtin_fmaf(to_f32(r[i]), 0.f, zero);
+      }
       keep(buf, row0 + j * 16, r);
     }
+    const bool odd = __any(!(zero == 0.f));
+    if (lane == 0) s_odd[buf][wave] = odd;
+  };
+  auto any_of = [&](const int (&x)[4]) {
+    return __builtin_amdgcn_readfirstlane(x[0] | x[1] | x[2] | x[3]) != 0;
   };
   auto row_operand = [&](int buf, int row, int e, bf16x8 (&x)[NP]) {
 #pragma unroll
@@ -199,6 +223,24 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
     }
   };
   auto put = [&](long at, const bf16x8& x) { *reinterpret_cast<bf16x8*>(ws + at * 256 + lane * 4) = x; };
+  // Sums over the tokens that a tile of (dealt) tokens sees, 32 at a time: `one` adds 32 of them, its own behind those in front.  Zeros stand for the
+  // tokens that a token does not see, and zero times what is no finite number is none: where there is one (ODD), the first 16 of the 32 (`first`: this
+  // lane's results are theirs) are formed without the others, by a second pass over what the first has left.
+  auto tokens_product = [&](auto odd, int m, bool first, const auto& one) {
+    f32x4 sum[2] = {none, none};
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      if (ks <= m) one(ks, false, sum);
+    f32x4 out = sum[0] + sum[1];
+    if constexpr (decltype(odd)::value) {
+      f32x4 less[2] = {none, none};
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+        if (ks <= m) one(ks, ks == m, less);
+      if (first) out = less[0] + less[1];
+    }
+    return out;
+  };
 
   Four<T, LAY> kr[4], qr[4];
   fetch_slab(kr, k, 0, a.d);
@@ -206,7 +248,6 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
   const long gate = b * a.g_sb + (long)(t0 + (lane < left ? lane : left - 1)) * a.g_sl + h;
   const T gate_a = static_cast<const T*>(a.a)[gate], gate_b = static_cast<const T*>(a.bt)[gate];
   const T a_log = static_cast<const T*>(a.a_log)[h], dt_bias = static_cast<const T*>(a.dt_bias)[h];
-  const f32x4 none = {0.f, 0.f, 0.f, 0.f};
   // Products of keys with keys and with queries, transposed (column = token t, rows = the tokens s of a pair of tiles): four of the twelve
   // units for each of wavefronts 1 to 3, while wavefront 0 works the decays out.
   constexpr int kMine = 4;
@@ -299,6 +340,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
     s_fq[t] = t < left ? (float)(1.0 / sqrt((sq + (double)kUnitEps) * (double)a.d)) : 0.f;
     s_fk[t] = t < left ? 1.0f / sqrtf((float)(sk + (double)kUnitEps)) : 0.f;
   }
+  const bool odd_k = __any(!((float)sk < INFINITY));
+  if (lane == 0) s_odd[2][wave] = odd_k;
   __syncthreads();
   // Quotients of decays as products of two, over the token in front of the later tile: a few exponentials a token in place of one for
   // every pair.  Between tiles both are at most one; inside a tile the second is at least one, and is not used where the tile forgets
@@ -439,11 +482,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
       const int m = m_of[n > 0], ks = n == 2, t = (m >> 1) * 32 + dealt + 4 * (m & 1), s0 = ks * 32 + quad * 8;
       const f32x4* row = reinterpret_cast<const f32x4*>(&s_a[t][s0]);
       const f32x4* f = reinterpret_cast<const f32x4*>(by + s0);
-      parts8(row[0] * f[0], row[1] * f[1], tm[n]);
+      const bool unseen = n != 1 && l16 < 8 && quad >= 2;  // (zero, whatever it is scaled by)
+      parts8(row[0] * (unseen ? none : f[0]), row[1] * (unseen ? none : f[1]), tm[n]);
     }
   };
   // W (row = token, contracted over channels in the scan: here transposed) and the keys of 32 channels of a slab
-  auto keys_tile = [&](int buf, int kc) {
+  auto keys_tile = [&](auto odd, int buf, int kc) {
     bf16x8 kx[2][2][NP];
 #pragma unroll
     for (int p = 0; p < 2; ++p)
@@ -459,10 +503,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
       f32x4 out[2];
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
-        f32x4 sum[2] = {none, none};
-#pragma unroll
-        for (int ks = 0; ks <= m; ++ks) product(kx[p][ks], tm[m + ks], sum);
-        out[p] = sum[0] + sum[1];
+        out[p] = tokens_product(odd, m, l16 < 8, [&](int ks, bool half_only, f32x4 (&sum)[2]) {
+          if (!half_only) return product(kx[p][ks], tm[m + ks], sum);
+          bf16x8 x[NP];
+          first_half(kx[p][ks], x, quad);
+          product(x, tm[m + ks], sum);
+        });
       }
       bf16x8 x[3];
       parts8(out[0], out[1], x);
@@ -471,7 +517,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
     }
   };
   // Uv (rows = tokens, column = channel: the scan's accumulator) of two of a slab's value tiles
-  auto values_tile = [&](int buf, int tile0) {
+  auto values_tile = [&](auto odd, int buf, int tile0) {
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
       const int tile = tile0 + half * 2 + x;
@@ -481,14 +527,18 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
       for (int ks = 0; ks < 2; ++ks) column_operand(buf, ks, (half * 2 + x) * 16, 4, vx[ks]);
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
-        f32x4 sum[2] = {none, none};
-#pragma unroll
-        for (int ks = 0; ks <= m; ++ks) product(tm[m + ks], vx[ks], sum);
-        *reinterpret_cast<f32x4*>(ws + At::kUv + ((long)tile * 4 + m_of[m]) * 256 + lane * 4) = sum[0] + sum[1];
+        const f32x4 uv = tokens_product(odd, m, quad < 2, [&](int ks, bool half_only, f32x4 (&sum)[2]) {
+          if (!half_only) return product(tm[m + ks], vx[ks], sum);
+          bf16x8 x[NP];
+          first_half(vx[ks], x, quad);
+          product(tm[m + ks], x, sum);
+        });
+        *reinterpret_cast<f32x4*>(ws + At::kUv + ((long)tile * 4 + m_of[m]) * 256 + lane * 4) = uv;
       }
     }
   };
   scaled(s_bg);
+  const bool odd_keys = any_of(s_odd[2]);
   int buf = 0;  // the slab in LDS; the next one goes into the other buffer, which everybody has left behind at the barrier before
   if constexpr (kSlabs > 1) {
 #pragma unroll 1
@@ -500,7 +550,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
           fetch_v(vr, 0);
       };
       if (kAhead) fetch();
-      keys_tile(buf, sl * 2 + half);
+      keys_tile(std::false_type(), buf, sl * 2 + half);
+      if (odd_keys) keys_tile(std::true_type(), buf, sl * 2 + half);
       if (!kAhead) fetch();
       buf ^= 1;
       if (sl + 1 < kSlabs)
@@ -510,7 +561,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
       __syncthreads();
     }
   } else {
-    keys_tile(0, half);
+    keys_tile(std::false_type(), 0, half);
+    if (odd_keys) keys_tile(std::true_type(), 0, half);
     buf = 1;
   }
   scaled(s_beta);
@@ -518,7 +570,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
   for (int e0 = 0; e0 < a.dv; e0 += 64) {
     const bool more = e0 + 64 < a.dv;
     if (more) fetch_v(vr, e0 + 64);
-    values_tile(buf, e0 / 16);
+    values_tile(std::false_type(), buf, e0 / 16);
+    if (any_of(s_odd[buf])) values_tile(std::true_type(), buf, e0 / 16);
     if (!more) break;
     buf ^= 1;
     if (kSlabs == 1 && e0 == 0) __syncthreads();  // (a slower wavefront may still read the keys there)
@@ -540,7 +593,7 @@ __global__ __launch_bounds__(512, dc_lone(RB) ? 2 : 4) void delta_chunk_scan_ker
   constexpr int RBW = RB / 4, KC = RB / 2;
   typedef DcAt<RB, NP> At;
   // operands of three parts: the state by 32 channels; U by 32 tokens, as the outputs take it and scaled to the chunk's end
-  __shared__ __attribute__((aligned(16))) bf16x8 s_s[KC][3][64], s_u[2][3][64], s_us[2][3][64];
+  __shared__ __attribute__((aligned(16))) bf16x8 s_s[KC][3][64], s_u[2][3][64], s_us[2][3][64], s_none[3][64];
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4;
   const int role = __builtin_amdgcn_readfirstlane(tid >> 8), wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
   const int bh = blockIdx.x, b = __builtin_amdgcn_readfirstlane(bh / a.H), h = bh - b * a.H;
@@ -670,12 +723,19 @@ __global__ __launch_bounds__(512, dc_lone(RB) ? 2 : 4) void delta_chunk_scan_ker
         }
     };
     bf16x8 us[2][3];
+    // (zeros for those tokens of the last piece that the wavefront's own do not see: what is there may be no finite number)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) s_none[j][lane] = bf16x8{};
+    const bool behind = (wave & 1) == 0 && quad >= 2;
+    const bf16x8* from[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) from[s] = behind && s == pieces ? &s_none[0][lane] : &s_u[s][0][lane];
     auto read_u = [&] {
 #pragma unroll
       for (int s = 0; s < 2; ++s)
         if (s <= pieces) {  // (uniform)
 #pragma unroll
-          for (int j = 0; j < 3; ++j) us[s][j] = s_u[s][j][lane];
+          for (int j = 0; j < 3; ++j) us[s][j] = from[s][j * 64];
         }
     };
     // P U behind `on`

@@ -193,3 +193,32 @@ def test_many_heads(dev, B, L, H, d, dv, chunks):
     want, T = reference(x, ab, a_log, dt_bias, H, H, d, dv)
     tol = TOL if chunks else 3e-6  # (blocks: as above)
     assert rel_l2(got, want) < tol and rel_l2(S, T) < tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d,dv", [(64, 64), (128, 40)])
+@pytest.mark.parametrize("what", ["value", "key", "gate"])
+@pytest.mark.parametrize("at", [16, 20, 31, 40, 63, 64 + 50, 299])
+def test_a_number_that_is_none(dev, dtype, d, dv, what, at):
+    """A value, a key or a gate that is not finite stays out of the tokens in front of its tile of 16, of the other value channels and of the other
+    heads, to the last bit: products take 32 tokens at a time, and zero times infinity is no zero."""
+    B, L, H = 2, 300, 3
+    clean = [t.to(dev) for t in make(5, B, L, H, H, d, dv, dtype)]
+    assert in_chunks(B, L, H, d, dv)
+    want, S_want = run(clean, H, H, d, dv, empty_state(B, H, d, dv, dev))
+    for bad in (float("nan"), float("inf")):
+        x, ab = clean[0].clone(), clean[1].clone()
+        if what == "gate":
+            if bad == float("inf"):
+                continue  # (a gate of one)
+            ab[1, at, H + 1] = bad
+        else:
+            x[1, at, (H * d + d + 5) if what == "key" else (2 * H * d + dv + 5)] = bad
+        o, S = run((x, ab, *clean[2:]), H, H, d, dv, empty_state(B, H, d, dv, dev))
+        assert not o[1, at, 1, 5].isfinite() and not S[1, 1, :, 5].isfinite().any()
+        free = torch.ones(B, L, H, dv, dtype=torch.bool, device=dev)
+        free[1, at // 16 * 16:, 1, slice(5, 6) if what == "value" else slice(None)] = False
+        assert torch.equal(o[free], want[free])
+        kept = torch.ones_like(S, dtype=torch.bool)
+        kept[1, 1, :, slice(5, 6) if what == "value" else slice(None)] = False
+        assert torch.equal(S[kept], S_want[kept])
