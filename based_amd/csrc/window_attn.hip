@@ -166,7 +166,8 @@ constexpr int kDirectTile = kTileKeys * 128;  // elements of a tile of keys and 
 
 // Bound by the vector unit, and in short windows by a workgroup's own start (queries, tables, first tile: 11 of 30 thousand cycles where all
 // workgroups run together).  As many wavefronts as fit: sizes up to 64 run in 128 registers, four workgroups to a compute unit (three, with
-// 143: 28.9 us where four take 24.8).  What a wavefront sees is worked out on the scalar unit, so that only tiles at the edges of a window are
+// 143: 28.9 us where four take 24.8); keys of up to 96 channels with values of 65 to 128 in 256, two (one, with 268, which the compiler takes where it
+// may: 16 heads on 4, 96 x 96, 4 x 2048 tokens and 129 keys 62 us for 42).  What a wavefront sees is worked out on the scalar unit, so that only tiles at the edges of a window are
 // masked; the lanes of a row look for their largest score together only where one of them has found a larger; weights are summed on the matrix unit;
 // and rows of 64 channels go straight into LDS.  Kernels alone, 16 heads of 64 channels, with the cache write, without and with these: on 4, 4 x 2048
 // tokens and 129 keys 31.7 / 30.1 us; 6 x 2240 and 513 keys 77.3 / 64.8; on 2, 4 x 4096 and 1,024 keys 140 / 112; on 16, 1 x 2048 and 1,024 keys
@@ -179,7 +180,7 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
 // DIRECT: keys and values of 64 channels each, straight into LDS, the next tile while one is worked on.  Piece p (16 bytes) of row r lies at
 // p ^ (r / 2 % 8), of values at p ^ (r / 2 % 4 * 2), so that reads of 16 rows (transposing reads of 8) meet every bank once; one barrier a tile.
 template <int KC, int VC, bool HALF, bool DIRECT>
-__global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 3 : 1) void window_prefill_mfma_kernel(const WindowArgs a) {
+__global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 3 : KC <= 3 && VC <= 4 ? 2 : 1) void window_prefill_mfma_kernel(const WindowArgs a) {
   constexpr int D = KC * 32, DV = VC * 32;
   constexpr int KS = D + 8, VS = kTileKeys + 8;  // LDS row strides: 16-lane reads of 16 bytes meet every bank once
   static_assert(!DIRECT || (KC == 2 && VC == 2), "rows of 64 channels");

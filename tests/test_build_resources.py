@@ -26,3 +26,13 @@ def test_hot_kernels_do_not_spill_vector_registers():
                 continue
             assert u.get("VGPRs Spill", 0) == 0, f"{src}: {name} spills {u['VGPRs Spill']} vector registers"
     assert seen > 50   # the report covers every source
+
+
+def test_window_kernels_share_a_compute_unit():
+    """Prefill of bf16 windows, keys of up to 96 channels and values of up to 128: two workgroups or more."""
+    if not os.path.exists(build.RESOURCES):
+        pytest.skip("no build in this tree yet (python -m based_amd.build writes the report)")
+    usage = json.load(open(build.RESOURCES))["window_attn.hip"]
+    waves = {n: u["Occupancy [waves/SIMD]"] for n, u in usage.items() if "window_prefill_mfma_kernel" in n
+             and any(f"ILi{kc}ELi{vc}E" in n for kc in (1, 2, 3) for vc in (1, 2, 4))}
+    assert len(waves) == 20 and min(waves.values()) >= 2, waves
