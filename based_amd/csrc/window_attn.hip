@@ -1476,19 +1476,30 @@ static bool window_f32_few(const WindowArgs& a) {
 // heads of 64 channels, one wavefront and a launch for the cache / two / cache filled: on 4, 129 keys, 1 x 777 (196 workgroups) 19.8 / 18.7 / 17.7;
 // 1 x 100 13.8 / 12.7 / 11.9; 1 x 2048 (512) 30.5 / 30.4 / -; 4 x 2048 (2,048) 77 / 80 / -; on 16, 1,024 keys, 1 x 2048 (512) 115 / 104 / 158; on 2, 513
 // keys, 2 x 500 (252) 39.2 / 32.5 / 37.7.
-static bool window_f32_small(const WindowArgs& a) { return ((long)a.L * (a.H / a.G) + kF32Rows - 1) / kF32Rows * a.B * a.G <= 256; }
+// A compute unit holds two workgroups of two wavefronts to a row, and three of one: between 512 and 768 of them the first take a second round that
+// the others do not.  Time of two as a part of one's, values of up to 64, by workgroups: 300 keys, 350 0.95, 500 0.96, 600 1.13, 750 1.13, 780 1.08, 900
+// 0.87, 1,030 0.84, 1,530 1.01; 1,024 keys, 350 0.92, 500 0.89, 600 0.86, 750 1.16, 900 0.94, 1,030 0.84, 2,040 0.92; 260 keys, 1,300 to 3,000 1.00 to
+// 1.05.  Values of 65 to 128, of whose workgroups there is room for one and two: 270 0.80 to 0.87, 350 to 3,000 1.00 to 1.25 with 200 to 513 keys.  Keys of 65
+// to 128: never, 50 to 1,000 workgroups 1.00 to 1.08.
+static long window_f32_groups(const WindowArgs& a) { return ((long)a.L * (a.H / a.G) + kF32Rows - 1) / kF32Rows * a.B * a.G; }
+static bool window_f32_small(const WindowArgs& a) { return window_f32_groups(a) <= 256; }
 static long window_f32_keys(const WindowArgs& a) {
   const long end = (long)a.pos_host + a.L;
   return (a.window < end ? a.window : end) + kF32Rows / (a.H / a.G);
 }
+static bool window_f32_twice(const WindowArgs& a) {
+  const long groups = window_f32_groups(a), keys = window_f32_keys(a);
+  if (a.dv > 64) return groups <= 300;
+  return groups <= 256 || (groups <= 512 ? keys > 256 : groups > 800 && keys > 300);
+}
 
 template <int KB, int VB> void launch_window_f32(const WindowArgs& a, dim3 grid, bool fill, hipStream_t s) {
-  if constexpr (KB + VB < 4) {
+  if constexpr (KB == 1) {
     if (fill) {
       hipLaunchKernelGGL((window_prefill_f32_kernel<KB, VB, 2, true>), grid, dim3(512), 0, s, a);
       return;
     }
-    if (window_f32_small(a) || window_f32_keys(a) > 256) {
+    if (window_f32_twice(a)) {
       hipLaunchKernelGGL((window_prefill_f32_kernel<KB, VB, 2, false>), grid, dim3(512), 0, s, a);
       return;
     }
@@ -1506,7 +1517,7 @@ static bool rows_meet(const WindowArgs& a, const void* x, long x_sb, long x_sl, 
 // Whether the fp32 form fills the cache itself: keys and values are read by every workgroup that sees them, so that nothing else may be written
 // there, and in 16-byte pieces.
 static bool window_f32_fills(const WindowArgs& a) {
-  if (!window_f32_small(a) || window_f32_keys(a) > 256 || (a.d > 64 && a.dv > 64)) return false;
+  if (!window_f32_small(a) || window_f32_keys(a) > 256 || a.d > 64) return false;
   if (a.k_sb % 4 || a.k_sl % 4 || a.v_sb % 4 || a.v_sl % 4 || !aligned_to(a.k, 16) || !aligned_to(a.v, 16)) return false;
   if (a.k_sb < 0 || a.k_sl < 0 || a.v_sb < 0 || a.v_sl < 0 || a.o_sb < 0 || a.o_sl < 0 || a.kv_sb < 0 || a.kv_st < 0) return false;
   const long kw = (long)a.G * a.d, vw = (long)a.G * a.dv, row = kw + vw;

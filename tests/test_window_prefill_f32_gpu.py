@@ -102,6 +102,19 @@ def test_both_sides_of_the_rule_for_few_rows(dev, d, dv, H, G, L, start, window)
         assert float(err.max()) < 3e-6, (B, float(err.max()))  # (scores of up to 5 and sums of 128 products)
 
 
+@pytest.mark.parametrize("d,dv,H,G,B,L,window", [
+    (64, 64, 16, 16, 1, 1024, 300), (64, 64, 16, 16, 1, 1025, 300), (32, 64, 16, 4, 1, 3200, 290), (32, 64, 16, 4, 1, 3201, 290), (64, 48, 16, 4, 1, 2048, 240),
+    (64, 48, 16, 4, 1, 2048, 241), (64, 128, 15, 3, 4, 320, 200), (64, 128, 15, 3, 4, 321, 200), (128, 64, 16, 4, 1, 300, 129), (96, 32, 4, 4, 1, 1500, 513)])
+def test_both_sides_of_the_rule_for_two_wavefronts(dev, d, dv, H, G, B, L, window):
+    """512 workgroups and more, 800 and more, 256 keys and more, 300 workgroups and more with wide values; wide keys."""
+    g = torch.Generator().manual_seed(L)
+    q, k, v = (torch.randn(B, L, n, m, generator=g) for n, m in ((H, d), (G, d), (G, dv)))
+    out = _run(dev, q, k, v, window, d ** -0.5, 0, None, 0)[-1]
+    ref = O.window_softmax(q[-1].double(), k[-1].double(), v[-1].double(), d ** -0.5, window)
+    err = (out - ref).norm(dim=-1) / ref.norm(dim=-1)
+    assert float(err.max()) < 3e-6, float(err.max())  # (scores of up to 5 and sums of 128 products)
+
+
 @pytest.mark.parametrize("norm", [False, True])
 @pytest.mark.parametrize("H,G,d,dv,B,L,start,window,rot,half", [
     (16, 4, 64, 64, 1, 777, 0, 129, 32, False), (16, 4, 64, 64, 1, 300, 77, 129, 32, True), (6, 2, 60, 36, 3, 190, 0, 20, 8, False),
