@@ -801,31 +801,37 @@ __global__ __launch_bounds__(512, dc_lone(RB) ? 2 : 4) void delta_chunk_scan_ker
 }
 
 // Workspace: the chunks of one launch pair.  Long prompts go through it in spans of chunks, the state carried on in between.
-constexpr int64_t kDcWorkFloats = 64ll << 20;  // 256 MB, which the last-level cache holds between the two launches
+// 192 MB, which the last-level cache (256 MB) holds between the two launches beside what they read and write otherwise: work spaces of 224 to 256 MB in one
+// launch pair, 1.00; in two of half as much, 0.82 to 0.86 of the time; more pairs of up to 160, 192 and 224 MB in place of 256, in 635 long prompts of bf16 0.92, 0.93
+// and 0.96; 160 MB cost 2 to 3 % where 192 take the call in one pair.
+constexpr int64_t kDcWorkFloats = 48ll << 20;
 
-// In bf16 chunks take 0.57 to 0.83 of the times that the rule for fp32, below, was made of.  They are slower only where channels are few,
-// which makes the blocks' steps cheap, and where workgroups are many, each of which reads what is formed ahead.  us, blocks of 16 against chunks, heads, d x dv (in 970 shapes, 0.24 to 1.00 of the time where the rule takes them):
-//   1, 64 x 16: L = 256: 27, 17.  24, 34 x 332: L = 700: 160, 45.  32, 64 x 512: L = 1024: 146, 93.  64, 128 x 256: L = 256: 81, 57; L = 1024: 269, 172.
-//   64, 32 x 128: L = 256: 29, 30; L = 320: 34, 31; L = 1024: 85, 56.  48, 32 x 256: L = 1024: 113, 80.  64, 32 x 256: L = 1024: 90, 98.
-//   4, 16 x 512: L = 256: 23, 24; L = 384: 30, 28.  64, 16 x 64: L = 320: 28, 27.  64, 16 x 128: L = 384: 34, 34; L = 512: 41, 37.  48, 16 x 256: L = 512: 41, 50.
-//   72, 64 x 128: L = 1500: 206, 130.  112, 48 x 128: L = 1024: 117, 129.  112, 64 x 128: L = 800: 120, 98.  112, 80 x 16: L = 1024: 141, 102; 80 x 64: 143, 147.
-//   80, 96 x 128: L = 256: 64, 50.  128, 48 x 64: L = 1024: 116, 88.  128, 64 x 128: L = 256: 48, 42; L = 512: 80, 68; L = 1024: 146, 175.
-//   128, 128 x 64: L = 2048: 341, 322.  128, 128 x 128: L = 256: 86, 67; L = 2048: 575, 474.
-//   256, L = 256: 64 x 64: 54, 52; 64 x 128: 76, 81; 128 x 128: 160, 179.  256, 64 x 64: L = 1024: 170, 247.
-//   Long prompts take several launches, for what is formed ahead is 256 MB at most: 64, 48 x 256: L = 1024: 114, 99; L = 4096: 402, 454.
-//   128, 112 x 128: L = 1024: 275, 253; L = 4096: 1,011, 1,051; 128 x 128: 1,167, 992.  112, 64 x 128, L = 4096: 586, 504.
+// In bf16 chunks take 0.57 to 0.83 of the times that the rule for fp32, below, was made of.  Three things make them the slower form.  A step of the
+// blocks costs by 16 channels of keys, chunks fill 64 or 128: few channels (up to 16, 32, 48), and 65 to 112, whose blocks leave out what chunks
+// multiply.  Two workgroups of the scan fit a compute unit (one above 64 channels): beyond 512 to 1,024 of them they take turns, each reads all that
+// is formed ahead, and every head adds preparation.  And short prompts pay for two launches.  us, blocks of 16 against chunks, heads, d x dv (in 5,658 shapes 0.35
+// to 1.04 of the blocks' time where the rule takes them, 0.69 in the mean):
+//   1, 64 x 16: L = 256: 27, 17.  24, 34 x 332: L = 700: 160, 45.  32, 64 x 512: L = 1024: 158, 96.  64, 128 x 256: L = 256: 85, 61; L = 1024: 281, 175.
+//   Up to 16 channels: 64, 16 x 64: L = 320: 30, 30.  64, 16 x 128: L = 512: 43, 41; L = 1024: 73, 62; L = 2048: 130, 139.  48, 16 x 256: L = 512: 44, 55.
+//   4, 16 x 512: L = 256: 24, 27; L = 320: 28, 28.
+//   Up to 32: 64, 32 x 128: L = 256: 30, 32; L = 320: 37, 35; L = 1024: 90, 63.  48, 32 x 256: L = 1024: 120, 85; L = 4096: 423, 387.  64, 32 x 256: L = 1024: 96, 100.
+//   Up to 48: 64, 48 x 256: L = 1024: 120, 102; L = 4096: 411, 493.  80, 48 x 128: L = 2048: 224, 206.  96, 48 x 128: L = 4096: 439, 486.
+//   Up to 64: 120, 64 x 128: L = 2048: 310, 309.  128, 64 x 128: L = 512: 86, 73; L = 1024: 158, 172.
+//   Up to 96: 80, 96 x 64: L = 4096: 485, 438.  112, 96 x 64: L = 4096: 515, 571.  112, 96 x 16: L = 4096: 530, 392.
+//   Up to 112: 112, 112 x 64: L = 4096: 662, 592.  128, 112 x 64: L = 1024: 179, 169; L = 4096: 674, 737.
+//   Up to 128: 128, 128 x 128: L = 4096: 1,161, 963.  128, 128 x 32: L = 4096: 479, 496.
+//   256 heads: 64 x 64: L = 256: 56, 56; L = 1024: 177, 249.  128 x 128: L = 256: 170, 183.
 static bool dc_faster_bf16(int64_t heads, int64_t L, int64_t D, int64_t DV) {
   const int64_t tiles = (DV + 15) / 16, wgs = heads * tiles;
   if (heads > 128 || wgs > 1024 || D > 128 || L < BASED_DELTA_CHUNKS_MIN) return false;
-  if (heads > 64) {
-    if (DV > 128 || D <= 32) return false;
-    if (D <= 64) return DV <= 64 || heads <= 80 || (D > 48 && (heads <= 112 || L <= 512));
-    if (heads > 112 && D > 104 && (D <= 112 || DV <= 32)) return L <= 1024;
-    return D > 104 || heads <= 80 || DV <= 16;
-  }
-  if (D > 32) return D > 48 || wgs <= 768 || L <= 1024;
+  if (D > 112) return true;
+  if (D > 96) return heads <= 112 || L <= 1024;
+  if (D > 64) return heads <= 80 || tiles == 1;
+  if (D > 48) return heads <= 64 || wgs <= 960 || L <= 512;
+  if (D > 32) return heads <= 64 ? wgs <= 768 || L <= 1024 : wgs <= 640;
+  if (heads > 64) return false;
   if (D > 16) return wgs <= 768 && L >= (wgs <= 448 ? 4 : tiles <= 16 ? 5 : 6) * kDc;
-  return wgs <= 512 && L >= (wgs > 256 ? 8 : wgs > 128 || heads > 48 || tiles > 16 ? 6 : 4) * kDc;
+  return wgs <= (heads <= 48 || L <= 1024 ? 512 : 256) && L >= (wgs > 256 ? 8 : wgs > 128 || heads > 48 || tiles > 16 ? 6 : 4) * kDc;
 }
 
 // Where chunks are the faster form in fp32: few heads, and enough chunks.  A chunk step of the scan takes 1.3 us (1.6 with heads of more than 64
@@ -862,16 +868,24 @@ static bool dc_faster(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, bo
 
 static int dc_tiles(int64_t D) { return D <= 64 ? 4 : 8; }
 
+// parts of an element of queries and keys
+static int dc_parts(bool bf16) { return bf16 ? 1 : 3; }
+
 // chunks per span, 0 where blocks of 16 are for the shape
 static int64_t dc_span(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, bool bf16) {
   if (B <= 0 || L <= 0 || H <= 0 || D <= 0 || DV <= 0 || B >= (1ll << 31) || H >= (1ll << 31) || DV >= (1ll << 20) || !dc_faster(B, L, H, D, DV, bf16))
     return 0;
-  const int64_t chunks = (L + kDc - 1) / kDc, each = B * H * dc_floats(dc_tiles(D), 3, (int)DV);
-  int64_t span = kDcWorkFloats / each;  // (at least 11: a chunk of 128 heads of 128 channels and 8 value tiles takes 5.9 M floats at most)
+  const int64_t chunks = (L + kDc - 1) / kDc, each = B * H * dc_floats(dc_tiles(D), dc_parts(bf16), (int)DV);
+  int64_t span = kDcWorkFloats / each;  // (at least 11: a chunk of 128 heads of 128 channels and 8 value tiles takes 4.3 M floats)
   if (span > chunks) span = chunks;
   // spans of about equal length
   const int64_t n = (chunks + span - 1) / span;
   return (chunks + n - 1) / n;
+}
+
+static int64_t dc_work(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, bool bf16) {
+  const int64_t span = dc_span(B, L, H, D, DV, bf16);
+  return span == 0 ? 0 : B * H * span * dc_floats(dc_tiles(D), dc_parts(bf16), (int)DV);
 }
 
 // Rows of queries and keys whose groups of four channels are one load; chunks of more than 64 channels take no others.
@@ -909,8 +923,9 @@ template <typename T> static int run_delta(const DeltaChunkArgs& a, bool vec, in
 
 extern "C" BASED_API int64_t based_gated_delta_scan_work(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
   using namespace based;
-  const int64_t span = dc_span(B, L, H, D, DV, false);
-  return span == 0 ? 0 : B * H * span * dc_floats(dc_tiles(D), 3, (int)DV);
+  // (a span of bf16 may hold more chunks, and all of them more than fewer of fp32)
+  const int64_t wide = dc_work(B, L, H, D, DV, false), narrow = dc_work(B, L, H, D, DV, true);
+  return wide == 0 || wide > narrow ? wide : narrow;
 }
 
 extern "C" BASED_API int64_t based_gated_delta_scan_work_of(const void* q, const void* k, int64_t B, int64_t L, int64_t H, int64_t D,
@@ -924,8 +939,7 @@ extern "C" BASED_API int64_t based_gated_delta_scan_work_as(const void* q, const
                                                             int64_t DV, int64_t x_sb, int64_t x_sl, int io_dtype) {
   using namespace based;
   if (!dc_near(H, DV, x_sl) || !(D <= 64 || dc_vec(q, k, B, D, x_sb, x_sl))) return 0;
-  const int64_t span = dc_span(B, L, H, D, DV, io_dtype == BASED_BF16);
-  return span == 0 ? 0 : B * H * span * dc_floats(dc_tiles(D), 3, (int)DV);
+  return dc_work(B, L, H, D, DV, io_dtype == BASED_BF16);
 }
 
 extern "C" BASED_API int based_gated_delta_scan_chunks(const void* q, const void* k, const void* v, const void* a_gate, const void* b_gate,
@@ -949,9 +963,9 @@ extern "C" BASED_API int based_gated_delta_scan_chunks(const void* q, const void
   BASED_REQUIRE(span > 0 && B * H * span < (1ll << 31), BASED_ERR_SHAPE, "%s: the shape is for blocks of 16", who);
   const bool vec = dc_vec(q, k, B, D, x_sb, x_sl);
   BASED_REQUIRE(vec || D <= 64, BASED_ERR_ALIGN, "%s: chunks of heads of more than 64 channels take rows of whole 16-byte pieces", who);
-  const DeltaChunkArgs a{q, k, v, a_gate, b_gate, a_log, dt_bias, state, o, work, (long)dc_floats(dc_tiles(D), io_dtype == BASED_BF16 ? 1 : 3, (int)DV), (int)B, (int)L, (int)H,
-                         (int)G, (int)D, (int)DV, (int)state_row, 0, 0, x_sb, x_sl, g_sb, g_sl, fresh,
-                         DV % 4 == 0 && (B == 1 || x_sb % 4 == 0) && x_sl % 4 == 0 && aligned_to(v, 16)};
+  const long per = (long)dc_floats(dc_tiles(D), dc_parts(io_dtype == BASED_BF16), (int)DV);
+  const DeltaChunkArgs a{q, k, v, a_gate, b_gate, a_log, dt_bias, state, o, work, per, (int)B, (int)L, (int)H, (int)G, (int)D, (int)DV, (int)state_row, 0, 0,
+                         x_sb, x_sl, g_sb, g_sl, fresh, DV % 4 == 0 && (B == 1 || x_sb % 4 == 0) && x_sl % 4 == 0 && aligned_to(v, 16)};
   hipStream_t s = static_cast<hipStream_t>(stream);
   return io_dtype == BASED_BF16 ? run_delta<__bf16>(a, vec, span, s) : run_delta<float>(a, vec, span, s);
 }

@@ -215,3 +215,14 @@ def test_delta_work_of_no_type_serves_either_type():
                             own = lib.based_gated_delta_scan_work_as(None, None, B, L, H, D, DV, 0, 8 * 128, dtype)
                             assert 0 < own <= floats, (B, H, D, DV, L, dtype)
     assert taken > 2000
+
+
+def test_delta_work_is_what_a_type_takes():
+    """Queries and keys of bf16 are one part of three of fp32's, in the work space too."""
+    lib = _lib.lib()
+    for B, L, H, D, DV in [(4, 2048, 8, 64, 128), (1, 300, 8, 128, 128), (1, 512, 2, 64, 16)]:
+        narrow, wide = (lib.based_gated_delta_scan_work_as(None, None, B, L, H, D, DV, 0, 4096, t) for t in (_lib.BASED_BF16, _lib.BASED_F32))
+        chunks, tiles, values = B * H * ((L + 63) // 64), 4 if D <= 64 else 8, (DV + 15) // 16
+        # operands of 1 KB: W (6 a tile of channels), queries, keys and outputs' weights in their parts, values in 32 bits; a row of factors
+        assert narrow == chunks * (((6 + 2 + 2) * tiles + 18 + 4 * values) * 256 + 132)
+        assert wide == chunks * (((6 + 4 + 6) * tiles + 18 + 4 * values) * 256 + 132)

@@ -222,3 +222,32 @@ def test_a_number_that_is_none(dev, dtype, d, dv, what, at):
         kept = torch.ones_like(S, dtype=torch.bool)
         kept[1, 1, :, slice(5, 6) if what == "value" else slice(None)] = False
         assert torch.equal(S[kept], S_want[kept])
+
+
+@pytest.mark.parametrize("B,L,H,d,dv,chunks", [(8, 1025, 16, 116, 32, True), (8, 1024, 16, 112, 32, True), (8, 1025, 16, 112, 32, False), (7, 1025, 16, 104, 48, True),
+                                               (5, 300, 16, 96, 64, True), (27, 300, 3, 96, 64, False), (27, 300, 3, 72, 16, True), (8, 513, 15, 64, 128, True),
+                                               (5, 300, 16, 48, 128, True), (27, 300, 3, 48, 128, False), (4, 1024, 16, 48, 256, True),
+                                               (4, 1025, 16, 48, 256, False), (4, 1025, 16, 16, 128, False), (6, 1025, 8, 16, 160, True)])
+def test_both_sides_of_the_lines_for_bf16(dev, B, L, H, d, dv, chunks):
+    """Every line of the rule for bf16: channels, heads, workgroups, and prompts that are long for them."""
+    test_many_heads(dev, B, L, H, d, dv, chunks)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,L,H,d,dv", [(4, 2500, 16, 64, 64), (4, 1600, 16, 128, 128)])
+def test_work_space_of_a_long_prompt(dev, dtype, B, L, H, d, dv):
+    """In a work space of exactly what was asked for, whatever lies behind it stays as it is; several launch pairs."""
+    from based_amd import _lib, ops
+
+    x, ab, a_log, dt_bias = (t.to(dev) for t in make(11, B, L, H, H, d, dv, dtype))
+    lib, s = _lib.lib(), ops._stream_ptr(x)
+    q, k, v, a, b = (x[..., :H * d], x[..., H * d:2 * H * d], x[..., 2 * H * d:], ab[..., :H], ab[..., H:])
+    code = _lib.BASED_BF16 if dtype == torch.bfloat16 else _lib.BASED_F32
+    floats = lib.based_gated_delta_scan_work_as(q.data_ptr(), k.data_ptr(), B, L, H, d, dv, *x.stride()[:2], code)
+    assert 0 < floats <= 48 << 20
+    room = torch.full((floats + 4096,), 7.0, device=dev)
+    o, S = torch.empty(B, L, H, dv, device=dev), torch.empty(B, H, d, dv, device=dev)
+    _lib.check(lib.based_gated_delta_scan_chunks(q.data_ptr(), k.data_ptr(), v.data_ptr(), a.data_ptr(), b.data_ptr(), a_log.data_ptr(), dt_bias.data_ptr(),
+                                                 S.data_ptr(), room.data_ptr(), o.data_ptr(), B, L, H, H, d, dv, dv, *x.stride()[:2], *ab.stride()[:2], 1, code, s))
+    want, T = run((x, ab, a_log, dt_bias), H, H, d, dv, empty_state(B, H, d, dv, dev))
+    assert torch.equal(o, want) and torch.equal(S, T) and (room[floats:] == 7).all()
