@@ -671,4 +671,39 @@ def test_experts_straight_into_lds(dev, n, D, F, E, top):
     s = O.sigmoid(h.double() @ router.double().T).sort(-1, descending=True).values
     clear = torch.ones(n, dtype=torch.bool) if top == E else s[:, top - 1] - s[:, top] > 1e-5
     assert clear.sum() >= 0.9 * n
-    close(got[clear], want[clear], 2 * TOL[BF16])
+    # three roundings to bf16 one behind the other (activations, a choice's row, the sum of the choices), each 2^-9 of a value at most and 1.1e-3 in the
+    # mean of squares: 2e-3, and as much again
+    close(got[clear], want[clear], 4e-3)
+
+
+def test_which_products_go_straight_into_lds():
+    """The kernels that run, by name: both products, either one alone (channels that are no whole 128; too few; too many tiles), neither.  In a process of its
+    own, which the trace ends with."""
+    import json
+    import os
+    import subprocess
+    import sys
+
+    cases = {(34, 1024, 1024, 1, 1): "both", (100, 1024, 1024, 1, 1): "both", (50, 1000, 1024, 4, 2): "second", (60, 72, 2048, 8, 1): "second",
+             (33, 1280, 8, 5, 2): "first", (17, 1024, 1024, 8, 2): "second", (30, 1024, 512, 16, 4): "neither"}
+    code = """
+import json, sys, torch
+from torch.profiler import ProfilerActivity, profile
+from based_amd import ops
+for n, D, F, E, top in json.loads(sys.argv[1]):
+    h, r, w1, w2 = (torch.randn(*s, device="cuda").bfloat16() for s in ((n, D), (E, D), (E, 2 * F, D), (E, D, F)))
+    ops.experts(h, r, w1, w2, top)
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        ops.experts(h, r, w1, w2, top)
+        torch.cuda.synchronize()
+    print("ran", json.dumps([e.name for e in p.events() if "expert_gemm" in e.name]), flush=True)
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    done = subprocess.run([sys.executable, "-c", code, json.dumps(list(cases))], cwd=root, capture_output=True, text=True, timeout=100)
+    assert done.returncode == 0, done.stderr[-2000:]
+    ran = [json.loads(line[4:]) for line in done.stdout.splitlines() if line.startswith("ran ")]
+    assert len(ran) == len(cases)
+    for (case, which), names in zip(cases.items(), ran):
+        direct = ["expert_gemm_direct_kernel" in n for n in names]
+        assert direct == [which in ("both", "first"), which in ("both", "second")], (case, names)
