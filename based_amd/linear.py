@@ -18,13 +18,18 @@ def _watched() -> bool:
             or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0)
 
 
-def _plain(x, weight) -> bool:
-    """Tensors on the GPU, no subclasses of them, and nothing that watches."""
-    return type(x) is torch.Tensor and type(weight) in (torch.Tensor, nn.Parameter) and x.is_cuda and not _watched()
+def _ordinary(t) -> bool:
+    """A tensor with rows: no subclass, not sparse, not nested."""
+    return type(t) in (torch.Tensor, nn.Parameter) and t.layout is torch.strided and not t.is_nested
+
+
+def _plain(x, weight, bias) -> bool:
+    """Tensors on the GPU, and nothing that watches."""
+    return _ordinary(x) and _ordinary(weight) and (bias is None or _ordinary(bias)) and x.is_cuda and not _watched()
 
 
 def linear(x, weight, bias=None):
-    return ops.linear(x, weight, bias) if _plain(x, weight) else F.linear(x, weight, bias)
+    return ops.linear(x, weight, bias) if _plain(x, weight, bias) else F.linear(x, weight, bias)
 
 
 class Linear(nn.Linear):
@@ -35,6 +40,6 @@ class Linear(nn.Linear):
 def swiglu(fc: nn.Linear, x):
     """`ops.swiglu` of fc(x), in one launch where nothing wants to see what lies between or has put a forward of its own into fc."""
     if (type(fc) is Linear and "forward" not in fc.__dict__ and not (fc._forward_hooks or fc._forward_pre_hooks or nn_module._global_forward_hooks
-                                    or nn_module._global_forward_pre_hooks) and _plain(x, fc.weight)):
+                                    or nn_module._global_forward_pre_hooks) and _plain(x, fc.weight, fc.bias)):
         return ops.swiglu(x, fc.weight, fc.bias)
     return ops.swiglu(fc(x))

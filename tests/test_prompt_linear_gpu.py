@@ -112,6 +112,28 @@ def test_stacked_weights(dev, M):
                 assert rel_l2(got[i], reference(x.view(M, 256), w, b).view_as(got[i])) < 2.5e-3
 
 
+def test_tensors_without_rows_of_their_own(dev):
+    """A sparse weight, a nested batch and a bias of another class are torch's own."""
+    from based_amd.linear import linear
+
+    class Marked(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    x, w, b = make(dev, 40, 256, 128, True)
+    plain = torch.nn.functional.linear(x, w, b)
+    with torch.no_grad():
+        few = w * (torch.arange(128, device=dev) % 16 == 0)
+        sparse = few.float().to_sparse_csr()
+        assert rel_l2(linear(x.float(), sparse), x.float() @ few.float().T) < 1e-5
+        nested = torch.nested.nested_tensor([x[:12], x[12:]])
+        assert torch.equal(torch.cat(list(linear(nested, w, b).unbind())), plain)
+        seen = []
+        assert rel_l2(linear(x, w, b.as_subclass(Marked)).as_subclass(torch.Tensor), plain) < 1e-2 and seen
+
+
 def test_module_with_a_forward_of_its_own(dev):
     """A wrapper that replaces the projection's forward (to move weights, to add a term) is called in front of the gate, too."""
     from based_amd.stack import GatedMlp
