@@ -10,12 +10,25 @@ from torch.nn.modules import module as nn_module
 from . import ops
 
 
+def _questions(c=torch._C, ad=forward_ad):
+    """What tells whether torch's operations are watched, and has no public name; None where a torch build lacks one of them."""
+    try:
+        ad._current_level
+        return c._is_tracing, c._functorch.peek_interpreter_stack, c._len_torch_dispatch_stack, c._len_torch_function_stack
+    except AttributeError:
+        return None
+
+
+_QUESTIONS = _questions()
+
+
 def _watched() -> bool:
     """Something watches or rewrites torch's operations here: a gradient of either mode, autocast, tracing, compiling, vmap (of which the weight or
-    the bias may be mapped and x not), a mode."""
-    return (torch.is_grad_enabled() or torch.compiler.is_compiling() or forward_ad._current_level >= 0 or torch.is_autocast_enabled("cuda")
-            or torch._C._is_tracing() or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0)
+    the bias may be mapped and x not), a mode.  Or it cannot be told."""
+    if torch.is_grad_enabled() or _QUESTIONS is None or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda"):
+        return True
+    tracing, transform, dispatch_modes, function_modes = _QUESTIONS
+    return forward_ad._current_level >= 0 or tracing() or transform() is not None or dispatch_modes() > 0 or function_modes() > 0
 
 
 def _ordinary(t) -> bool:

@@ -16,3 +16,45 @@ def test_mapped_weights_are_seen():
     with torch.no_grad():
         torch.vmap(f)(torch.ones(2, 3))
         assert seen == [True, True] and not linear._watched()
+
+
+def test_modes_and_tracing_are_seen():
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class SeenToo(TorchFunctionMode):
+        pass
+
+    with torch.no_grad():
+        assert not linear._watched()
+        for mode in (Seen(), SeenToo(), torch.enable_grad(), torch.autograd.forward_ad.dual_level()):
+            with mode:
+                assert linear._watched()
+        traced = []
+        torch.jit.trace(lambda x: traced.append(linear._watched()) or x + 1, torch.ones(2), check_trace=False)
+        assert traced == [True] and not linear._watched()
+
+
+def test_a_torch_that_cannot_be_asked(monkeypatch):
+    """A build without one of the private names: everything is torch's own."""
+    from types import SimpleNamespace
+
+    whole = linear._questions()
+    assert whole is not None
+    names = {"_is_tracing": 1, "_functorch": SimpleNamespace(peek_interpreter_stack=1), "_len_torch_dispatch_stack": 1, "_len_torch_function_stack": 1}
+    ad = SimpleNamespace(_current_level=-1)
+    assert linear._questions(SimpleNamespace(**names), ad) == (1, 1, 1, 1)
+    for gone in names:
+        assert linear._questions(SimpleNamespace(**{n: v for n, v in names.items() if n != gone}), ad) is None
+    assert linear._questions(SimpleNamespace(**{**names, "_functorch": SimpleNamespace()}), ad) is None
+    assert linear._questions(SimpleNamespace(**names), SimpleNamespace()) is None
+    with torch.no_grad():
+        assert not linear._watched()
+        monkeypatch.setattr(linear, "_QUESTIONS", None)
+        assert linear._watched()
+        x, w = torch.randn(3, 8), torch.randn(4, 8)
+        assert torch.equal(linear.linear(x, w), torch.nn.functional.linear(x, w))
