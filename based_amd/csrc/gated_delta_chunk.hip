@@ -599,10 +599,13 @@ __global__ __launch_bounds__(512, dc_lone(RB) ? 2 : 4) void delta_chunk_scan_ker
   // The workgroups of a head run on one die, whose L2 then has its chunks once.  Workgroup i is number i / 8 of die i % 8: heads in whole eights lie side
   // by side, others one behind the other, tile by tile, a run of them to a die (spread over all dies 61 heads of 40 x 160, 4,677 tokens took 676 us
   // for 413, and the blocks 499; runs for whole eights as well: 24 heads of 24 x 256, 4,096 tokens 200 for 184).
-  const int tiles = (a.dv + 15) >> 4, heads = a.B * a.H, i = (int)blockIdx.x, die = i & 7, more = (int)gridDim.x & 7;
-  const int run = die * (int)(gridDim.x >> 3) + (die < more ? die : more) + (i >> 3);
-  const int bh = __builtin_amdgcn_readfirstlane(heads % 8 ? run / tiles : i % heads), b = __builtin_amdgcn_readfirstlane(bh / a.H), h = bh - b * a.H;
-  const int ct = __builtin_amdgcn_readfirstlane(heads % 8 ? run - bh * tiles : i / heads), col = ct * 16 + l16;
+  int head = (int)blockIdx.x, ct = (int)blockIdx.y;
+  if (gridDim.x % 8 != 0) {
+    const int i = ct * (int)gridDim.x + head, n = (int)(gridDim.x * gridDim.y), die = i & 7, more = n & 7;
+    const int at = die * (n >> 3) + (die < more ? die : more) + (i >> 3);
+    head = __builtin_amdgcn_readfirstlane(at / (int)gridDim.y), ct = __builtin_amdgcn_readfirstlane(at - head * (int)gridDim.y);
+  }
+  const int bh = head, b = __builtin_amdgcn_readfirstlane(bh / a.H), h = bh - b * a.H, col = ct * 16 + l16;
   const bool col_in = col < a.dv;
   const char* ws = reinterpret_cast<const char*>(a.work + (long)bh * a.span * a.per);
   const long per = a.per * 4, vec_at = dc_vec_at(RB, NP, a.dv) * 4;
@@ -761,7 +764,7 @@ __global__ __launch_bounds__(512, dc_lone(RB) ? 2 : 4) void delta_chunk_scan_ker
     };
     // The workgroups of a head, which share an L2 where the heads are a multiple of the dies, ask together for every line of the chunk after
     // next, a word each: what the registers hold ahead is less than the way from memory takes (fp32, d = 128: 243 -> 206 us).
-    const int lines = (int)((per + 127) / 128), first = (ct * 4 + wave) * 64 + lane, every = tiles * 256;
+    const int lines = (int)((per + 127) / 128), first = (ct * 4 + wave) * 64 + lane, every = (int)gridDim.y * 256;
     unsigned seen = 0;
     auto touch = [&](int n) {
       if (n >= a.span) return;  // (uniform)
@@ -906,7 +909,7 @@ template <typename T, int RB, int LAY> static int run_delta_chunks(DeltaChunkArg
     a.c0 = c;
     a.span = chunks - c < span ? chunks - c : (int)span;
     hipLaunchKernelGGL((delta_chunk_prepare_kernel<T, LAY, RB>), dim3((unsigned)((long)a.B * a.H * a.span)), dim3(256), 0, s, a);
-    hipLaunchKernelGGL((delta_chunk_scan_kernel<RB, NP>), dim3((unsigned)(a.B * a.H) * (unsigned)((a.dv + 15) / 16)), dim3(512), 0, s, a);
+    hipLaunchKernelGGL((delta_chunk_scan_kernel<RB, NP>), dim3((unsigned)(a.B * a.H), (unsigned)((a.dv + 15) / 16)), dim3(512), 0, s, a);
     const int rc = check_launch("gated_delta_scan_chunks");
     if (rc) return rc;
     a.fresh = 0;
