@@ -47,6 +47,8 @@ def linear(x, weight, bias=None):
 
 class Linear(nn.Linear):
     def forward(self, x):
+        if torch.jit.is_scripting():
+            return F.linear(x, self.weight, self.bias)
         return linear(x, self.weight, self.bias)
 
 

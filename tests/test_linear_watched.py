@@ -58,3 +58,13 @@ def test_a_torch_that_cannot_be_asked(monkeypatch):
         assert linear._watched()
         x, w = torch.randn(3, 8), torch.randn(4, 8)
         assert torch.equal(linear.linear(x, w), torch.nn.functional.linear(x, w))
+
+
+def test_scripted_exported_and_traced():
+    """A projection by itself goes where torch.nn.Linear goes."""
+    fc, x = linear.Linear(8, 4), torch.randn(3, 8)
+    want = fc(x)
+    for other in (torch.jit.script(fc), torch.jit.trace(fc, x), torch.export.export(fc, (x,)).module(), torch.compile(fc, backend="eager", fullgraph=True)):
+        assert torch.equal(other(x), want)
+        with torch.no_grad():
+            assert torch.equal(other(x), want)
