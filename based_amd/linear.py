@@ -14,7 +14,7 @@ def _questions(c=torch._C, ad=forward_ad):
     """What tells whether torch's operations are watched, and has no public name; None where a torch build lacks one of them."""
     try:
         ad._current_level
-        return c._is_tracing, c._functorch.peek_interpreter_stack, c._len_torch_dispatch_stack, c._len_torch_function_stack
+        return c._functorch.peek_interpreter_stack, c._len_torch_dispatch_stack, c._len_torch_function_stack
     except AttributeError:
         return None
 
@@ -22,13 +22,22 @@ def _questions(c=torch._C, ad=forward_ad):
 _QUESTIONS = _questions()
 
 
+_is_tracing = getattr(torch._C, "_is_tracing", torch.jit.is_tracing)
+
+
+def _beyond(x, weight) -> bool:
+    """Torch's own for certain: a gradient, a compiler or a trace wants it, or there are too many rows.  Asked in front of everything else, for prompts that
+    the library takes wait for the host as well (the 360M model, 1 x 600 tokens: 4.8 ms, 5.1 where each projection's form was looked up first)."""
+    return torch.is_grad_enabled() or torch.compiler.is_compiling() or _is_tracing() or x.numel() > ops.PROMPT_LINEAR_MAX_ROWS * weight.size(-1)
+
+
 def _watched() -> bool:
-    """Something watches or rewrites torch's operations here: a gradient of either mode, autocast, tracing, compiling, vmap (of which the weight or
-    the bias may be mapped and x not), a mode.  Or it cannot be told."""
-    if torch.is_grad_enabled() or _QUESTIONS is None or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda"):
+    """Something else watches or rewrites torch's operations: autocast, forward mode, vmap (of which the weight or the bias may be mapped and x not), a
+    mode.  Or it cannot be told."""
+    if _QUESTIONS is None or forward_ad._current_level >= 0 or torch.is_autocast_enabled("cuda"):
         return True
-    tracing, transform, dispatch_modes, function_modes = _QUESTIONS
-    return forward_ad._current_level >= 0 or tracing() or transform() is not None or dispatch_modes() > 0 or function_modes() > 0
+    transform, dispatch_modes, function_modes = _QUESTIONS
+    return transform() is not None or dispatch_modes() > 0 or function_modes() > 0
 
 
 def _ordinary(t) -> bool:
@@ -37,24 +46,43 @@ def _ordinary(t) -> bool:
 
 
 def _plain(x, weight, bias) -> bool:
-    """Tensors on the GPU, and nothing that watches."""
+    """Tensors on the GPU, and nothing that watches (behind `_beyond`)."""
     return _ordinary(x) and _ordinary(weight) and (bias is None or _ordinary(bias)) and x.is_cuda and not _watched()
 
 
 def linear(x, weight, bias=None):
-    return ops.linear(x, weight, bias) if _plain(x, weight, bias) else F.linear(x, weight, bias)
+    if _beyond(x, weight) or not _plain(x, weight, bias):
+        return F.linear(x, weight, bias)
+    return ops.linear(x, weight, bias)
 
 
 class Linear(nn.Linear):
+    def _operands(self):
+        own = self._parameters  # (`self.weight` looks through Module.__getattr__ first, half a microsecond)
+        try:
+            return own["weight"], own["bias"]
+        except KeyError:  # (something else stands in for them)
+            return self.weight, self.bias
+
     def forward(self, x):
         if torch.jit.is_scripting():
             return F.linear(x, self.weight, self.bias)
-        return linear(x, self.weight, self.bias)
+        weight, bias = self._operands()
+        if _beyond(x, weight) or not _plain(x, weight, bias):
+            return F.linear(x, weight, bias)
+        return ops.linear(x, weight, bias)
+
+
+def _alone(fc) -> bool:
+    """A projection without hooks, of which nothing has put a forward of its own into it."""
+    return type(fc) is Linear and "forward" not in fc.__dict__ and not (
+        fc._forward_hooks or fc._forward_pre_hooks or nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks)
 
 
 def swiglu(fc: nn.Linear, x):
-    """`ops.swiglu` of fc(x), in one launch where nothing wants to see what lies between or has put a forward of its own into fc."""
-    if (type(fc) is Linear and "forward" not in fc.__dict__ and not (fc._forward_hooks or fc._forward_pre_hooks or nn_module._global_forward_hooks
-                                    or nn_module._global_forward_pre_hooks) and _plain(x, fc.weight, fc.bias)):
-        return ops.swiglu(x, fc.weight, fc.bias)
+    """`ops.swiglu` of fc(x), in one launch where nothing wants to see what lies between."""
+    if _alone(fc):
+        weight, bias = fc._operands()
+        if not _beyond(x, weight) and _plain(x, weight, bias):
+            return ops.swiglu(x, weight, bias)
     return ops.swiglu(fc(x))

@@ -571,9 +571,10 @@ def swiglu(u, weight=None, bias=None) -> torch.Tensor:
     """u (..., 2F) -> u[..., :F] * silu(u[..., F:]), one pass.  weight (2F, K) (and bias): u (..., K) goes through that projection first, in the
     same launch where `prompt_linear` is the faster form."""
     if weight is not None:
-        if linear_form(u, weight, bias) == LINEAR_PROMPT and weight.shape[0] % 8 == 0:
+        form = linear_form(u, weight, bias)
+        if form == LINEAR_PROMPT and weight.shape[0] % 8 == 0:
             return _prompt_linear(u, weight, bias, weight.shape[0] // 2, True)
-        u = linear(u, weight, bias)
+        u = _linear_as(form, u, weight, bias)
     _require_cuda(u)
     F2 = u.shape[-1]
     if F2 % 2 != 0:
@@ -624,7 +625,10 @@ def linear_form(x, weight, bias=None) -> int:
 
 def linear(x, weight, bias=None) -> torch.Tensor:
     """torch.nn.functional.linear without a gradient: few rows of bf16 by the kernels here, everything else by the library."""
-    form = linear_form(x, weight, bias)
+    return _linear_as(linear_form(x, weight, bias), x, weight, bias)
+
+
+def _linear_as(form: int, x, weight, bias) -> torch.Tensor:
     if form == LINEAR_LIBRARY:
         return torch.nn.functional.linear(x, weight, bias)
     N, K = weight.shape

@@ -4,18 +4,23 @@ import torch
 from based_amd import linear
 
 
+def watched():
+    few = torch.ones(1, 8)
+    return linear._beyond(few, few) or linear._watched()
+
+
 def test_mapped_weights_are_seen():
     """Under torch.vmap the weight or the bias may be mapped and x not."""
     seen = []
 
     def f(w):
-        seen.append(linear._watched())
+        seen.append(watched())
         return w.sum()
 
     torch.vmap(f)(torch.ones(2, 3))
     with torch.no_grad():
         torch.vmap(f)(torch.ones(2, 3))
-        assert seen == [True, True] and not linear._watched()
+        assert seen == [True, True] and not watched()
 
 
 def test_modes_and_tracing_are_seen():
@@ -27,16 +32,17 @@ def test_modes_and_tracing_are_seen():
             return func(*args, **(kwargs or {}))
 
     class SeenToo(TorchFunctionMode):
-        pass
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
 
     with torch.no_grad():
-        assert not linear._watched()
+        assert not watched()
         for mode in (Seen(), SeenToo(), torch.enable_grad(), torch.autograd.forward_ad.dual_level()):
             with mode:
-                assert linear._watched()
+                assert watched()
         traced = []
-        torch.jit.trace(lambda x: traced.append(linear._watched()) or x + 1, torch.ones(2), check_trace=False)
-        assert traced == [True] and not linear._watched()
+        torch.jit.trace(lambda x: traced.append(watched()) or x + 1, torch.ones(2), check_trace=False)
+        assert traced == [True] and not watched()
 
 
 def test_a_torch_that_cannot_be_asked(monkeypatch):
@@ -45,17 +51,17 @@ def test_a_torch_that_cannot_be_asked(monkeypatch):
 
     whole = linear._questions()
     assert whole is not None
-    names = {"_is_tracing": 1, "_functorch": SimpleNamespace(peek_interpreter_stack=1), "_len_torch_dispatch_stack": 1, "_len_torch_function_stack": 1}
+    names = {"_functorch": SimpleNamespace(peek_interpreter_stack=1), "_len_torch_dispatch_stack": 1, "_len_torch_function_stack": 1}
     ad = SimpleNamespace(_current_level=-1)
-    assert linear._questions(SimpleNamespace(**names), ad) == (1, 1, 1, 1)
+    assert linear._questions(SimpleNamespace(**names), ad) == (1, 1, 1)
     for gone in names:
         assert linear._questions(SimpleNamespace(**{n: v for n, v in names.items() if n != gone}), ad) is None
     assert linear._questions(SimpleNamespace(**{**names, "_functorch": SimpleNamespace()}), ad) is None
     assert linear._questions(SimpleNamespace(**names), SimpleNamespace()) is None
     with torch.no_grad():
-        assert not linear._watched()
+        assert not watched()
         monkeypatch.setattr(linear, "_QUESTIONS", None)
-        assert linear._watched()
+        assert watched()
         x, w = torch.randn(3, 8), torch.randn(4, 8)
         assert torch.equal(linear.linear(x, w), torch.nn.functional.linear(x, w))
 
@@ -68,3 +74,21 @@ def test_scripted_exported_and_traced():
         assert torch.equal(other(x), want)
         with torch.no_grad():
             assert torch.equal(other(x), want)
+
+
+def test_parameters_that_something_stands_in_for():
+    """Pruned, parametrised and replaced weights, by whatever way torch.nn.Linear finds them."""
+    from torch.func import functional_call
+    from torch.nn.utils import parametrize, prune
+
+    x = torch.randn(3, 8)
+    fc = linear.Linear(8, 4)
+    prune.random_unstructured(fc, "weight", 0.5)
+    assert torch.equal(fc(x), torch.nn.functional.linear(x, fc.weight, fc.bias)) and (fc.weight == 0).any()
+    fc = linear.Linear(8, 4, bias=False)
+    parametrize.register_parametrization(fc, "weight", torch.nn.ReLU())
+    assert torch.equal(fc(x), x @ fc.weight.T) and (fc.weight >= 0).all()
+    fc, other = linear.Linear(8, 4), torch.randn(4, 8)
+    assert torch.equal(functional_call(fc, {"weight": other}, (x,)), torch.nn.functional.linear(x, other, fc.bias))
+    fc.weight.data = other
+    assert torch.equal(fc(x), torch.nn.functional.linear(x, other, fc.bias))

@@ -134,6 +134,19 @@ def test_tensors_without_rows_of_their_own(dev):
         assert rel_l2(linear(x, w, b.as_subclass(Marked)).as_subclass(torch.Tensor), plain) < 1e-2 and seen
 
 
+def test_many_rows_are_not_looked_at(dev, monkeypatch):
+    """More rows than either kernel takes: nothing but the library's call, of the projection and of the gate's."""
+    from based_amd import ops
+    from based_amd.stack import GatedMlp
+
+    mlp = GatedMlp(256, hidden_features=512, device=dev, dtype=torch.bfloat16)
+    monkeypatch.setattr(ops, "linear_form", lambda *a: pytest.fail("looked up"))
+    with torch.no_grad():
+        assert mlp(torch.randn(1, 513, 256, device=dev).bfloat16()).shape == (1, 513, 256)
+        with pytest.raises(pytest.fail.Exception):
+            mlp(torch.randn(1, 512, 256, device=dev).bfloat16())
+
+
 def test_module_with_a_forward_of_its_own(dev):
     """A wrapper that replaces the projection's forward (to move weights, to add a term) is called in front of the gate, too."""
     from based_amd.stack import GatedMlp
