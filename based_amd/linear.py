@@ -26,9 +26,13 @@ _is_tracing = getattr(torch._C, "_is_tracing", torch.jit.is_tracing)
 
 
 def _beyond(x, weight) -> bool:
-    """Torch's own for certain: a gradient, a compiler or a trace wants it, or there are too many rows.  Asked in front of everything else, for prompts that
-    the library takes wait for the host as well (the 360M model, 1 x 600 tokens: 4.8 ms, 5.1 where each projection's form was looked up first)."""
-    return torch.is_grad_enabled() or torch.compiler.is_compiling() or _is_tracing() or x.numel() > ops.PROMPT_LINEAR_MAX_ROWS * weight.size(-1)
+    """Torch's own for certain: a gradient, a compiler or a trace wants it, it is not in bf16 or there are too many rows.  Asked in front of everything
+    else, for what the library takes waits for the host as well (the 360M model, 1 x 600 tokens: 4.8 ms, 5.1 where each projection's form was looked
+    up first)."""
+    if torch.is_grad_enabled() or torch.compiler.is_compiling() or _is_tracing() or x.dtype is not torch.bfloat16:
+        return True
+    K = weight.size(-1)
+    return x.numel() > ops.linear_max_rows(K) * K
 
 
 def _watched() -> bool:

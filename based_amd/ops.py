@@ -591,7 +591,12 @@ def swiglu(u, weight=None, bias=None) -> torch.Tensor:
 
 
 LINEAR_LIBRARY, LINEAR_PROMPT, LINEAR_ROWS = 0, 1, 2
-PROMPT_LINEAR_MAX_ROWS = 512
+PROMPT_LINEAR_MAX_ROWS, STEP_LINEAR_MAX_ROWS = 512, 8
+
+
+def linear_max_rows(K: int) -> int:
+    """Rows of K channels beyond which `linear` is the library's call whatever else they are."""
+    return PROMPT_LINEAR_MAX_ROWS if K % 128 == 0 and K <= 2048 else STEP_LINEAR_MAX_ROWS
 
 
 def linear_form(x, weight, bias=None) -> int:
@@ -613,9 +618,9 @@ def linear_form(x, weight, bias=None) -> int:
             N, K = weight.shape
             M = x.numel() // K if K else 0
             one_each = x.dim() == 3 and x.shape[1] == 1 and x.stride(2) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= K  # (the last tokens)
-            if 0 < M <= 8 and (x.is_contiguous() or one_each) and K % 8 == 0 and K <= 4096 and 0 < N and (M <= 4 or N <= 16384):
+            if 0 < M <= STEP_LINEAR_MAX_ROWS and (x.is_contiguous() or one_each) and K % 8 == 0 and K <= 4096 and 0 < N and (M <= 4 or N <= 16384):
                 form = LINEAR_ROWS
-            elif x.is_contiguous() and 0 < M <= PROMPT_LINEAR_MAX_ROWS and N % 4 == 0 and K % 128 == 0 and K <= 2048 and -(-M // 128) * -(-N // 64) <= 256:
+            elif x.is_contiguous() and STEP_LINEAR_MAX_ROWS < linear_max_rows(K) >= M > 0 and N % 4 == 0 and -(-M // 128) * -(-N // 64) <= 256:
                 form = LINEAR_PROMPT
         _CHECKED[key] = form
     if form != LINEAR_LIBRARY and ((x.data_ptr() | weight.data_ptr()) & 15 or (bias is not None and bias.data_ptr() & 7)):

@@ -5,7 +5,7 @@ from based_amd import linear
 
 
 def watched():
-    few = torch.ones(1, 8)
+    few = torch.ones(1, 8, dtype=torch.bfloat16)
     return linear._beyond(few, few) or linear._watched()
 
 

@@ -134,17 +134,20 @@ def test_tensors_without_rows_of_their_own(dev):
         assert rel_l2(linear(x, w, b.as_subclass(Marked)).as_subclass(torch.Tensor), plain) < 1e-2 and seen
 
 
-def test_many_rows_are_not_looked_at(dev, monkeypatch):
-    """More rows than either kernel takes: nothing but the library's call, of the projection and of the gate's."""
+@pytest.mark.parametrize("dtype,rows,width,hidden,looked_up", [
+    (torch.bfloat16, 512, 256, 512, True), (torch.bfloat16, 513, 256, 512, False), (torch.float32, 40, 256, 512, False), (torch.bfloat16, 8, 200, 200, True),
+    (torch.bfloat16, 9, 200, 200, False), (torch.bfloat16, 9, 2176, 128, True), (torch.bfloat16, 9, 2176, 2176, False)])
+def test_what_is_not_looked_at(dev, monkeypatch, dtype, rows, width, hidden, looked_up):
+    """More rows than either kernel takes, other types and channels: nothing but the library's call, of the projections and of the gate's."""
     from based_amd import ops
     from based_amd.stack import GatedMlp
 
-    mlp = GatedMlp(256, hidden_features=512, device=dev, dtype=torch.bfloat16)
-    monkeypatch.setattr(ops, "linear_form", lambda *a: pytest.fail("looked up"))
+    mlp = GatedMlp(width, hidden_features=hidden, multiple_of=8, device=dev, dtype=dtype)
+    seen, form = [], ops.linear_form
+    monkeypatch.setattr(ops, "linear_form", lambda *a: seen.append(1) or form(*a))
     with torch.no_grad():
-        assert mlp(torch.randn(1, 513, 256, device=dev).bfloat16()).shape == (1, 513, 256)
-        with pytest.raises(pytest.fail.Exception):
-            mlp(torch.randn(1, 512, 256, device=dev).bfloat16())
+        assert mlp(torch.randn(1, rows, width, device=dev).to(dtype)).shape == (1, rows, width)
+    assert bool(seen) == looked_up
 
 
 def test_module_with_a_forward_of_its_own(dev):
