@@ -9,18 +9,22 @@
 //                        o_t = G_t S0^T q_t + sum_{s <= t} P_ts u_s.  A workgroup of four wavefronts carries 16 value channels of a
 //                        head; wavefront w has 16 tokens of every chunk and the state tiles w, w + 4, ..; S0 and U go round
 //                        through LDS, two barriers per chunk.
-// Products run on bf16 MFMA (16 x 16 x 32, sixteen times the rate of fp32), with 32 bits of every operand: a number of 32 bits enters as
-// the sum of three of bf16 (each what the ones before leave, rounded: 24 bits and a sign between them), and of the nine products of two such
-// sums the six that reach 2^-24 of the result are taken.  Inputs of bf16 are one part as they are, scaled by row or behind the product, so
-// their products are exact.  Sums are the matrix unit's, in 32 bits; the small products have an accumulator of their own.
+// Products run on bf16 MFMA (16 x 16 x 32, sixteen times the rate of fp32), with 24 bits of every operand: a number of 32 bits enters as
+// the sum of three of bf16 (each what the ones before leave, rounded; as in Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial
+// Intelligence Datatype For Higher-Precision Computations"), and of the nine products of two such sums the six that reach 2^-24 of the result
+// are taken.  Inputs of bf16 are one part as they are, scaled by row or behind the product, so their products are exact.  Sums are the matrix
+// unit's, in 32 bits; the small products have an accumulator of their own.
+// The parts hold what they should from 1e-32 to 3.39e38 in size.  Below, the last of them fall among the subnormals and are lost: values of 1e-33,
+// 1e-35 and 1e-37 have errors of 3e-7, 3e-5 and 3e-3 (products on fp32 MFMA: 1.4e-7, 1.4e-7, 1.4e-6).  What bf16 rounds to infinity, and infinity
+// itself, which leaves no number when it is taken off itself, makes every product that it enters no number.
 //
 // Operand layout of a lane (l16 = lane % 16, quad = lane / 16): row or column l16, contracted elements 8 quad .. 8 quad + 7; results: column
 // l16, rows 4 quad + i.  What a result feeds next is contracted over its rows, so the rows of the tiles 2 n and 2 n + 1 are dealt out in turn:
 // row 4 quad + i of tile 2 n + p is element 32 n + 8 quad + 4 p + i, and the four results of a lane in both tiles are one operand.  State
 // tiles (channels), U (tokens) and the tiles of W and Uv that make it are dealt so; outputs are not.
 //
-// Products take 32 tokens at a time and hold zeros where a token does not see another.  What is no finite number stays out of the tiles of 16 tokens in
-// front of its own all the same, as in blocks: the first 16 of such 32 are formed a second time without the others, and the outputs'
+// Products take 32 tokens at a time and hold zeros where a token does not see another.  What is no finite number stays out of the tiles of 16 tokens
+// in front of its own all the same, as in blocks: the first 16 of such 32 are formed a second time without the others, and the outputs'
 // wavefronts read zeros in their place (0 to 2 % of a call, 0.7 in the mean of 20 shapes).
 //
 // Against blocks of 16 (gated_delta_scan_kernel) a chain step takes in four times the tokens with two exchanges instead of one, and
@@ -62,8 +66,9 @@ struct DeltaChunkArgs {
 };
 
 // What a chunk leaves in the workspace, in operands of 1 KB (16 bytes a lane): W (token tile, 32 channels, part), q (token tile, 32
-// channels; as they are, 8 of bf16 or of fp32 a lane), k transposed (channel tile, 32 tokens, part), P (unit, part), and Uv (value tile, token tile) in 32 bits; then, by token,
-// fq G of the queries and what a token's value is multiplied by at the chunk's end, and G_64.  NP: parts of an element of q and k.
+// channels; as they are, 8 of bf16 or of fp32 a lane), k transposed (channel tile, 32 tokens, part), P (unit, part), and Uv (value tile,
+// token tile) in 32 bits; then, by token, fq G of the queries and what a token's value is multiplied by at the chunk's end, and G_64.  NP: parts of
+// an element of q and k.
 template <int RB, int NP> struct DcAt {
   static constexpr long kW = 0, kQ = (long)6 * RB * 256, kK = kQ + 2 * RB * (NP == 1 ? 1 : 2) * 256, kP = kK + 2 * RB * NP * 256, kUv = kP + 18 * 256;
 };
@@ -224,8 +229,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
   };
   auto put = [&](long at, const bf16x8& x) { *reinterpret_cast<bf16x8*>(ws + at * 256 + lane * 4) = x; };
   // Sums over the tokens that a tile of (dealt) tokens sees, 32 at a time: `one` adds 32 of them, its own behind those in front.  Zeros stand for the
-  // tokens that a token does not see, and zero times what is no finite number is none: where there is one (ODD), the first 16 of the 32 (`first`: this
-  // lane's results are theirs) are formed without the others, by a second pass over what the first has left.
+  // tokens that a token does not see, and zero times what is no finite number is none: where there is one (ODD), the first 16 of the 32 (`first`:
+  // this lane's results are theirs) are formed without the others, by a second pass over what the first has left.
   auto tokens_product = [&](auto odd, int m, bool first, const auto& one) {
     f32x4 sum[2] = {none, none};
 #pragma unroll
@@ -322,7 +327,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RB == 4 ? 4 : 3) : 2) void d
         put(at, x[1][0]);
       } else {
 #pragma unroll
-        for (int n = 0; n < 2; ++n) *reinterpret_cast<f32x4*>(ws + (at + n) * 256 + lane * 4) = f32x4{f[1][4 * n], f[1][4 * n + 1], f[1][4 * n + 2], f[1][4 * n + 3]};
+        for (int n = 0; n < 2; ++n)
+          *reinterpret_cast<f32x4*>(ws + (at + n) * 256 + lane * 4) =
+              f32x4{f[1][4 * n], f[1][4 * n + 1], f[1][4 * n + 2], f[1][4 * n + 3]};
       }
     }
   }
@@ -596,9 +603,9 @@ __global__ __launch_bounds__(512, dc_lone(RB) ? 2 : 4) void delta_chunk_scan_ker
   __shared__ __attribute__((aligned(16))) bf16x8 s_s[KC][3][64], s_u[2][3][64], s_us[2][3][64], s_none[3][64];
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4;
   const int role = __builtin_amdgcn_readfirstlane(tid >> 8), wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
-  // The workgroups of a head run on one die, whose L2 then has its chunks once.  Workgroup i is number i / 8 of die i % 8: heads in whole eights lie side
-  // by side, others one behind the other, tile by tile, a run of them to a die (spread over all dies 61 heads of 40 x 160, 4,677 tokens took 676 us
-  // for 413, and the blocks 499; runs for whole eights as well: 24 heads of 24 x 256, 4,096 tokens 200 for 184).
+  // The workgroups of a head run on one die, whose L2 then has its chunks once.  Workgroup i is number i / 8 of die i % 8: heads in whole eights lie
+  // side by side, others one behind the other, tile by tile, a run of them to a die (spread over all dies 61 heads of 40 x 160, 4,677 tokens took 676
+  // us for 413, and the blocks 499; runs for whole eights as well: 24 heads of 24 x 256, 4,096 tokens 200 for 184).
   int head = (int)blockIdx.x, ct = (int)blockIdx.y;
   if (gridDim.x % 8 != 0) {
     const int i = ct * (int)gridDim.x + head, n = (int)(gridDim.x * gridDim.y), die = i & 7, more = n & 7;
@@ -809,20 +816,22 @@ __global__ __launch_bounds__(512, dc_lone(RB) ? 2 : 4) void delta_chunk_scan_ker
 }
 
 // Workspace: the chunks of one launch pair.  Long prompts go through it in spans of chunks, the state carried on in between.
-// 192 MB, which the last-level cache (256 MB) holds between the two launches beside what they read and write otherwise: work spaces of 224 to 256 MB in one
-// launch pair, 1.00; in two of half as much, 0.82 to 0.86 of the time; more pairs of up to 160, 192 and 224 MB in place of 256, in 635 long prompts of bf16 0.92, 0.93
-// and 0.96; 160 MB cost 2 to 3 % where 192 take the call in one pair.
+// 192 MB, which the last-level cache (256 MB) holds between the two launches beside what they read and write otherwise: work spaces of 224 to 256 MB
+// in one launch pair, 1.00; in two of half as much, 0.82 to 0.86 of the time; more pairs of up to 160, 192 and 224 MB in place of 256, in 635 long
+// prompts of bf16 0.92, 0.93 and 0.96; 160 MB cost 2 to 3 % where 192 take the call in one pair.
 constexpr int64_t kDcWorkFloats = 48ll << 20;
 
 // In bf16 chunks take 0.57 to 0.83 of the times that the rule for fp32, below, was made of.  Three things make them the slower form.  A step of the
 // blocks costs by 16 channels of keys, chunks fill 64 or 128: few channels (up to 16, 32, 48), and 65 to 112, whose blocks leave out what chunks
 // multiply.  Two workgroups of the scan fit a compute unit (one above 64 channels): beyond 512 to 1,024 of them they take turns, each reads all that
-// is formed ahead, and every head adds preparation.  And short prompts pay for two launches.  us, blocks of 16 against chunks, heads, d x dv (in 5,658 shapes 0.35
-// to 1.04 of the blocks' time where the rule takes them, 0.69 in the mean):
-//   1, 64 x 16: L = 256: 27, 17.  24, 34 x 332: L = 700: 160, 45.  32, 64 x 512: L = 1024: 158, 96.  64, 128 x 256: L = 256: 85, 61; L = 1024: 281, 175.
-//   Up to 16 channels: 64, 16 x 64: L = 320: 30, 30.  64, 16 x 128: L = 512: 43, 41; L = 1024: 73, 62; L = 2048: 130, 139.  48, 16 x 256: L = 512: 44, 55.
+// is formed ahead, and every head adds preparation.  And short prompts pay for two launches.  us, blocks of 16 against chunks, heads, d x dv (in
+// 5,658 shapes 0.24 to 1.04 of the blocks' time where the rule takes them, 0.57 in the mean; in 1,500 of any size at most 1.03):
+//   24, 34 x 332: L = 700: 160, 45.  32, 64 x 512: L = 1024: 158, 96.  64, 128 x 256: L = 256: 85, 61; L = 1024: 281, 175.
+//   Up to 16 channels: 64, 16 x 64: L = 320: 30, 30.  64, 16 x 128: L = 512: 43, 41; L = 1024: 73, 62; L = 2048: 130, 139.  48, 16 x 256: L = 512:
+//   44, 55.
 //   4, 16 x 512: L = 256: 24, 27; L = 320: 28, 28.
-//   Up to 32: 64, 32 x 128: L = 256: 30, 32; L = 320: 37, 35; L = 1024: 90, 63.  48, 32 x 256: L = 1024: 120, 85; L = 4096: 423, 387.  64, 32 x 256: L = 1024: 96, 100.
+//   Up to 32: 64, 32 x 128: L = 256: 30, 32; L = 320: 37, 35; L = 1024: 90, 63.  48, 32 x 256: L = 1024: 120, 85; L = 4096: 423, 387.  64, 32 x 256:
+//   L = 1024: 96, 100.
 //   Up to 48: 64, 48 x 256: L = 1024: 120, 102; L = 4096: 411, 493.  80, 48 x 128: L = 2048: 224, 206.  96, 48 x 128: L = 4096: 439, 486.
 //   Up to 64: 120, 64 x 128: L = 2048: 310, 309.  128, 64 x 128: L = 512: 86, 73; L = 1024: 158, 172.
 //   Up to 96: 80, 96 x 64: L = 4096: 485, 438.  112, 96 x 64: L = 4096: 515, 571.  112, 96 x 16: L = 4096: 530, 392.
@@ -881,8 +890,8 @@ static int dc_parts(bool bf16) { return bf16 ? 1 : 3; }
 
 // chunks per span, 0 where blocks of 16 are for the shape
 static int64_t dc_span(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, bool bf16) {
-  if (B <= 0 || L <= 0 || H <= 0 || D <= 0 || DV <= 0 || B >= (1ll << 31) || H >= (1ll << 31) || DV >= (1ll << 20) || !dc_faster(B, L, H, D, DV, bf16))
-    return 0;
+  if (B <= 0 || L <= 0 || H <= 0 || D <= 0 || DV <= 0 || B >= (1ll << 31) || H >= (1ll << 31) || DV >= (1ll << 20)) return 0;
+  if (!dc_faster(B, L, H, D, DV, bf16)) return 0;
   const int64_t chunks = (L + kDc - 1) / kDc, each = B * H * dc_floats(dc_tiles(D), dc_parts(bf16), (int)DV);
   int64_t span = kDcWorkFloats / each;  // (at least 11: a chunk of 128 heads of 128 channels and 8 value tiles takes 4.3 M floats)
   if (span > chunks) span = chunks;
@@ -972,8 +981,9 @@ extern "C" BASED_API int based_gated_delta_scan_chunks(const void* q, const void
   const bool vec = dc_vec(q, k, B, D, x_sb, x_sl);
   BASED_REQUIRE(vec || D <= 64, BASED_ERR_ALIGN, "%s: chunks of heads of more than 64 channels take rows of whole 16-byte pieces", who);
   const long per = (long)dc_floats(dc_tiles(D), dc_parts(io_dtype == BASED_BF16), (int)DV);
-  const DeltaChunkArgs a{q, k, v, a_gate, b_gate, a_log, dt_bias, state, o, work, per, (int)B, (int)L, (int)H, (int)G, (int)D, (int)DV, (int)state_row, 0, 0,
-                         x_sb, x_sl, g_sb, g_sl, fresh, DV % 4 == 0 && (B == 1 || x_sb % 4 == 0) && x_sl % 4 == 0 && aligned_to(v, 16)};
+  const int v_vec = DV % 4 == 0 && (B == 1 || x_sb % 4 == 0) && x_sl % 4 == 0 && aligned_to(v, 16);
+  const DeltaChunkArgs a{q,      k,      v,       a_gate,         b_gate, a_log, dt_bias, state, o,    work,  per,  (int)B, (int)L, (int)H,
+                         (int)G, (int)D, (int)DV, (int)state_row, 0,      0,     x_sb,    x_sl,  g_sb, g_sl, fresh, v_vec};
   hipStream_t s = static_cast<hipStream_t>(stream);
   return io_dtype == BASED_BF16 ? run_delta<__bf16>(a, vec, span, s) : run_delta<float>(a, vec, span, s);
 }

@@ -178,6 +178,20 @@ def test_parts_of_small_and_large_values(dev, dtype, d, dv, scale):
         assert rel_l2(o.double() / scale, ref / scale) < TOL and rel_l2(S.double() / scale, S_ref / scale) < TOL
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("scale", [1e-32, 3e37])
+def test_ends_of_the_range_of_the_parts(dev, dtype, scale):
+    """The smallest and the largest values that keep all of their 24 bits."""
+    L, H, d, dv = 330, 3, 64, 64
+    x, *gates = make(9, 2, L, H, H, d, dv, torch.float32)
+    x[..., 2 * H * d:] *= scale
+    case = [t.to(dtype).to(dev) for t in (x, *gates)]
+    assert in_chunks(2, L, H, d, dv)
+    o, S = run(case, H, H, d, dv, empty_state(2, H, d, dv, dev))
+    ref, S_ref = reference(*case, H, H, d, dv)
+    assert rel_l2(o.double() / scale, ref / scale) < TOL and rel_l2(S.double() / scale, S_ref / scale) < TOL
+
+
 @pytest.mark.parametrize("B,L,H,d,dv,chunks", [(5, 256, 13, 64, 64, True), (13, 257, 5, 128, 128, True), (8, 512, 16, 64, 128, True),
                                                (8, 513, 16, 64, 128, False), (7, 300, 13, 80, 64, False), (43, 256, 3, 64, 64, False),
                                                (4, 256, 16, 128, 256, True), (4, 257, 12, 18, 52, True), (4, 511, 16, 16, 128, False),
