@@ -1000,10 +1000,10 @@ template <bool PAIRED, bool TAIL> int launch_expert_gemm_large(ExpertGemmArgs a,
   return BASED_OK;
 }
 
-// Straight into LDS where tiles of 128 rows of the weights are fewer than half of the compute units and a tile's way is long.  Whole calls, kernels alone,
-// us, without and with (both products, the second alone): 2 of 8 experts of 1024, 12 tokens (128 and 64 workgroups) 27.3 / 23.7 / 24.9, 30 (144, 72) 28.4
-// / 27.0 / 26.2, 100 (224, 112) 33.9 / 32.7 / 32.5, 164 (288, 144) 37.6 / 36.5 / 38.0; 1 of 8 of 2048, 30 tokens (256, 64) 34.4 / 29.9 / 29.3, 260 (512,
-// 128) 42.8 / 39.4 / 38.3; 4 of 16 of 512, 30 tokens (152, 152; 512 channels) 29.2 / 30.9 / 30.1.
+// Straight into LDS where tiles of 128 rows of the weights are fewer than half of the compute units and a tile's way is long.  Whole calls, kernels
+// alone, us, without and with (both products, the second alone): 2 of 8 experts of 1024, 12 tokens (128 and 64 workgroups) 27.3 / 23.7 / 24.9, 30
+// (144, 72) 28.4 / 27.0 / 26.2, 100 (224, 112) 33.9 / 32.7 / 32.5, 164 (288, 144) 37.6 / 36.5 / 38.0; 1 of 8 of 2048, 30 tokens (256, 64) 34.4 / 29.9
+// / 29.3, 260 (512, 128) 42.8 / 39.4 / 38.3; 4 of 16 of 512, 30 tokens (152, 152; 512 channels) 29.2 / 30.9 / 30.1.
 template <bool PAIRED> int launch_expert_gemm(ExpertGemmArgs a, hipStream_t s) {
   const int before = PAIRED ? kSmallWeights / 2 : kSmallWeights;
   const bool direct = a.K % 128 == 0 && a.K >= 1024 && (long)((a.F + before - 1) / before) * a.tiles <= 128;

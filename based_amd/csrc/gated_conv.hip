@@ -15,9 +15,9 @@
 
 namespace based {
 
-// Tokens per thread in the prefill kernel: few where more would leave compute units without a workgroup, whose threads then wait for one round of loads in
-// place of two.  us, bf16, 2048 channels with the state, 8 tokens and 2 (and the state's stores in pieces): 4 x 128 tokens (64 workgroups) 9.6 -> 4.7, 1 x 30 7.9 ->
-// 3.4, 8 x 128 10.9 -> 6.1, 16 x 128 (256) 12.9 -> 8.8; in pieces alone 8 x 2048 41.7 -> 39.8.
+// Tokens per thread in the prefill kernel: few where more would leave compute units without a workgroup, whose threads then wait for one round of
+// loads in place of two.  us, bf16, 2048 channels with the state, 8 tokens and 2 (and the state's stores in pieces): 4 x 128 tokens (64 workgroups)
+// 9.6 -> 4.7, 1 x 30 7.9 -> 3.4, 8 x 128 10.9 -> 6.1, 16 x 128 (256) 12.9 -> 8.8; in pieces alone 8 x 2048 41.7 -> 39.8.
 constexpr int kConvTokens = 8, kConvTokensFew = 2;
 constexpr int kConvMaxK = 4;      // supported kernel sizes: 2..4
 

@@ -7,9 +7,9 @@
 // loaded there directly; four wavefronts of 64 tokens x 32 features each, side by side or, in the smaller tiles, on different channels of
 // the same tile, their sums added through LDS in the end.  The tile is the one whose rounds over the chip's 256 compute units bring the fewest rows
 // and columns to one of them; tiles that share columns of the matrix run on the same die.  us, weights from memory, the library (and the gate's own
-// launch) before: 4096 x 1024 with the gate, 64 / 128 / 512 rows 13.9 / 14.9 / 16.9 -> 7.4 / 7.5 / 11.5; 1024 x 1024 8.5 / 8.1 / 8.4 -> 6.4 / 6.5 / 6.6;
-// 1024 x 2048 8.2 / 8.6 / 9.3 -> 8.9 / 8.9 / 9.0; of the host 20 (28) -> 7.5.  Rounds of 64 channels for the tile of 64 x 64: 1024 x 1024, 1000 rows
-// 9.1 for 8.2.
+// launch) before: 4096 x 1024 with the gate, 64 / 128 / 512 rows 13.9 / 14.9 / 16.9 -> 7.4 / 7.5 / 11.5; 1024 x 1024 8.5 / 8.1 / 8.4 -> 6.4 / 6.5 /
+// 6.6; 1024 x 2048 8.2 / 8.6 / 9.3 -> 8.9 / 8.9 / 9.0; of the host 20 (28) -> 7.5.  Rounds of 64 channels for the tile of 64 x 64: 1024 x 1024, 1000
+// rows 9.1 for 8.2.
 #include <atomic>
 
 #include "stream_common.hpp"
@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256, 1) void prompt_linear_kernel(const PromptLinea
 #pragma unroll
     for (int i = 0; i < P::LOADS; ++i)
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + (long)from * P::KS * 2),
-                                       (__attribute__((address_space(3))) void*)(pl_lds + place * P::ROUND + (wave * P::LOADS + i) * 8 * 64), 16, 0, 0);
+                                       (__attribute__((address_space(3))) void*)(pl_lds + place * P::ROUND + (wave * P::LOADS + i) * 512), 16, 0, 0);
   };
   f32x4 acc[2][4];
 #pragma unroll
@@ -173,7 +173,8 @@ template <int WM, int WN, int WK, bool GATED> static int launch_prompt_linear(Pr
   typedef PlTile<WM, WN, WK> P;
   static std::atomic<bool> allowed[kPlMaxDevices];
   int dev = 0;
-  BASED_REQUIRE(hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kPlMaxDevices, BASED_ERR_LAUNCH, "prompt_linear: cannot identify the current device");
+  BASED_REQUIRE(hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kPlMaxDevices, BASED_ERR_LAUNCH,
+                "prompt_linear: cannot identify the current device");
   if (!allowed[dev].load(std::memory_order_acquire)) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(prompt_linear_kernel<WM, WN, WK, GATED>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, P::LDS);
@@ -208,12 +209,13 @@ extern "C" BASED_API int based_prompt_linear(const void* x, int64_t x_row_stride
                                              void* y, int64_t y_row_stride, int64_t M, int64_t N, int64_t K, int gated, void* stream) {
   using namespace based;
   BASED_REQUIRE(x && w && y, BASED_ERR_ARG, "prompt_linear: null pointer argument");
-  BASED_REQUIRE(M >= 0 && N > 0 && K > 0 && M < (1 << 24) && N < (1 << 24) && K < (1 << 24), BASED_ERR_SHAPE, "prompt_linear: bad sizes (%ld, %ld, %ld)",
-                (long)M, (long)N, (long)K);
-  BASED_REQUIRE(K % 128 == 0 && N % 4 == 0, BASED_ERR_SHAPE, "prompt_linear: channels in whole 128 and features in whole 4 (%ld, %ld)", (long)K, (long)N);
+  BASED_REQUIRE(M >= 0 && N > 0 && K > 0 && M < (1 << 24) && N < (1 << 24) && K < (1 << 24), BASED_ERR_SHAPE,
+                "prompt_linear: bad sizes (%ld, %ld, %ld)", (long)M, (long)N, (long)K);
+  BASED_REQUIRE(K % 128 == 0 && N % 4 == 0, BASED_ERR_SHAPE, "prompt_linear: channels in whole 128 and features in whole 4 (%ld, %ld)", (long)K,
+                (long)N);
   BASED_REQUIRE(x_row_stride >= K && w_row_stride >= K && y_row_stride >= N, BASED_ERR_ARG, "prompt_linear: rows overlap");
-  BASED_REQUIRE(aligned_to(x, 16) && aligned_to(w, 16) && x_row_stride % 8 == 0 && w_row_stride % 8 == 0 && aligned_to(y, 8) && y_row_stride % 4 == 0 &&
-                    (!bias || aligned_to(bias, 8)),
+  BASED_REQUIRE(aligned_to(x, 16) && aligned_to(w, 16) && x_row_stride % 8 == 0 && w_row_stride % 8 == 0 && aligned_to(y, 8) &&
+                    y_row_stride % 4 == 0 && (!bias || aligned_to(bias, 8)),
                 BASED_ERR_ALIGN, "prompt_linear: rows in whole 16-byte pieces");
   if (M == 0) return BASED_OK;
   const PromptLinearArgs a{static_cast<const __bf16*>(x), static_cast<const __bf16*>(w), static_cast<const __bf16*>(bias), static_cast<__bf16*>(y),

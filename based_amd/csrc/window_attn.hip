@@ -166,12 +166,12 @@ constexpr int kDirectTile = kTileKeys * 128;  // elements of a tile of keys and 
 
 // Bound by the vector unit, and in short windows by a workgroup's own start (queries, tables, first tile: 11 of 30 thousand cycles where all
 // workgroups run together).  As many wavefronts as fit: sizes up to 64 run in 128 registers, four workgroups to a compute unit (three, with
-// 143: 28.9 us where four take 24.8); keys of up to 96 channels with values of 65 to 128 in 256, two (one, with 268, which the compiler takes where it
-// may: 16 heads on 4, 96 x 96, 4 x 2048 tokens and 129 keys 62 us for 42).  What a wavefront sees is worked out on the scalar unit, so that only tiles at the edges of a window are
-// masked; the lanes of a row look for their largest score together only where one of them has found a larger; weights are summed on the matrix unit;
-// and rows of 64 channels go straight into LDS.  Kernels alone, 16 heads of 64 channels, with the cache write, without and with these: on 4, 4 x 2048
-// tokens and 129 keys 31.7 / 30.1 us; 6 x 2240 and 513 keys 77.3 / 64.8; on 2, 4 x 4096 and 1,024 keys 140 / 112; on 16, 1 x 2048 and 1,024 keys
-// 47.4 / 38.4; 1 x 700 12.4 / 11.3.
+// 143: 28.9 us where four take 24.8); keys of up to 96 channels with values of 65 to 128 in 256, two (one, with 268, which the compiler takes where
+// it may: 16 heads on 4, 96 x 96, 4 x 2048 tokens and 129 keys 62 us for 42).  What a wavefront sees is worked out on the scalar unit, so that only
+// tiles at the edges of a window are masked; the lanes of a row look for their largest score together only where one of them has found a larger;
+// weights are summed on the matrix unit; and rows of 64 channels go straight into LDS.  Kernels alone, 16 heads of 64 channels, with the cache write,
+// without and with these: on 4, 4 x 2048 tokens and 129 keys 31.7 / 30.1 us; 6 x 2240 and 513 keys 77.3 / 64.8; on 2, 4 x 4096 and 1,024 keys 140 /
+// 112; on 16, 1 x 2048 and 1,024 keys 47.4 / 38.4; 1 x 700 12.4 / 11.3.
 
 __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -180,7 +180,8 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
 // DIRECT: keys and values of 64 channels each, straight into LDS, the next tile while one is worked on.  Piece p (16 bytes) of row r lies at
 // p ^ (r / 2 % 8), of values at p ^ (r / 2 % 4 * 2), so that reads of 16 rows (transposing reads of 8) meet every bank once; one barrier a tile.
 template <int KC, int VC, bool HALF, bool DIRECT>
-__global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 3 : KC <= 3 && VC <= 4 ? 2 : 1) void window_prefill_mfma_kernel(const WindowArgs a) {
+__global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 3 : KC <= 3 && VC <= 4 ? 2 : 1)
+void window_prefill_mfma_kernel(const WindowArgs a) {
   constexpr int D = KC * 32, DV = VC * 32;
   constexpr int KS = D + 8, VS = kTileKeys + 8;  // LDS row strides: 16-lane reads of 16 bytes meet every bank once
   static_assert(!DIRECT || (KC == 2 && VC == 2), "rows of 64 channels");
@@ -1474,13 +1475,13 @@ static bool window_f32_few(const WindowArgs& a) {
 // Two wavefronts to the same rows where the workgroups are no more than the compute units, or the way through the keys is long; in the first case,
 // where that way is short, the cache filled as well (every workgroup turns the keys that it sees: with 1,024 of them 104 us become 158).  us, 16
 // heads of 64 channels, one wavefront and a launch for the cache / two / cache filled: on 4, 129 keys, 1 x 777 (196 workgroups) 19.8 / 18.7 / 17.7;
-// 1 x 100 13.8 / 12.7 / 11.9; 1 x 2048 (512) 30.5 / 30.4 / -; 4 x 2048 (2,048) 77 / 80 / -; on 16, 1,024 keys, 1 x 2048 (512) 115 / 104 / 158; on 2, 513
-// keys, 2 x 500 (252) 39.2 / 32.5 / 37.7.
+// 1 x 100 13.8 / 12.7 / 11.9; 1 x 2048 (512) 30.5 / 30.4 / -; 4 x 2048 (2,048) 77 / 80 / -; on 16, 1,024 keys, 1 x 2048 (512) 115 / 104 / 158; on 2,
+// 513 keys, 2 x 500 (252) 39.2 / 32.5 / 37.7.
 // A compute unit holds two workgroups of two wavefronts to a row, and three of one: between 512 and 768 of them the first take a second round that
-// the others do not.  Time of two as a part of one's, values of up to 64, by workgroups: 300 keys, 350 0.95, 500 0.96, 600 1.13, 750 1.13, 780 1.08, 900
-// 0.87, 1,030 0.84, 1,530 1.01; 1,024 keys, 350 0.92, 500 0.89, 600 0.86, 750 1.16, 900 0.94, 1,030 0.84, 2,040 0.92; 260 keys, 1,300 to 3,000 1.00 to
-// 1.05.  Values of 65 to 128, of whose workgroups there is room for one and two: 270 0.80 to 0.87, 350 to 3,000 1.00 to 1.25 with 200 to 513 keys.  Keys of 65
-// to 128: never, 50 to 1,000 workgroups 1.00 to 1.08.
+// the others do not.  Time of two as a part of one's, values of up to 64, by workgroups: 300 keys, 350 0.95, 500 0.96, 600 1.13, 750 1.13, 780 1.08,
+// 900 0.87, 1,030 0.84, 1,530 1.01; 1,024 keys, 350 0.92, 500 0.89, 600 0.86, 750 1.16, 900 0.94, 1,030 0.84, 2,040 0.92; 260 keys, 1,300 to 3,000
+// 1.00 to 1.05.  Values of 65 to 128, of whose workgroups there is room for one and two: 270 0.80 to 0.87, 350 to 3,000 1.00 to 1.25 with 200 to 513
+// keys.  Keys of 65 to 128: never, 50 to 1,000 workgroups 1.00 to 1.08.
 static long window_f32_groups(const WindowArgs& a) { return ((long)a.L * (a.H / a.G) + kF32Rows - 1) / kF32Rows * a.B * a.G; }
 static bool window_f32_small(const WindowArgs& a) { return window_f32_groups(a) <= 256; }
 static long window_f32_keys(const WindowArgs& a) {
