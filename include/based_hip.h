@@ -549,10 +549,10 @@ BASED_API int based_gated_delta_scan(const void* q, const void* k, const void* v
                                      int64_t x_sl, int64_t g_sb, int64_t g_sl, int fresh, int io_dtype, void* stream);
 
 /* The same in chunks of 64 tokens, which is faster for few heads and long portions; D up to 128, strides x_sl below 2^24, H * DV below
- * 2^25, and 16-byte pieces in the rows of q and k where D is above 64.  work: as many floats, 16-byte aligned, at most 256 MB, as
+ * 2^25, and 16-byte pieces in the rows of q and k where D is above 64.  work: as many floats, 16-byte aligned, at most 192 MB, as
  * based_gated_delta_scan_work says for the sizes; 0 of them: the shape is for based_gated_delta_scan.  based_gated_delta_scan_work_of
  * says it for the tensors: 0 also where their rows are for based_gated_delta_scan.  Both are 0 below BASED_DELTA_CHUNKS_MIN tokens, and
- * what they say goes for either type; based_gated_delta_scan_work_as says it for one: more shapes of bf16 than of fp32 are faster so. */
+ * what they say goes for either type; based_gated_delta_scan_work_as says it for one: fewer floats in bf16, and more shapes are faster so. */
 #define BASED_DELTA_CHUNKS_MIN 256
 BASED_API int64_t based_gated_delta_scan_work(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV);
 BASED_API int64_t based_gated_delta_scan_work_of(const void* q, const void* k, int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV,
