@@ -168,10 +168,11 @@ constexpr int kDirectTile = kTileKeys * 128;  // elements of a tile of keys and 
 // workgroups run together).  As many wavefronts as fit: sizes up to 64 run in 128 registers, four workgroups to a compute unit (three, with
 // 143: 28.9 us where four take 24.8); keys of up to 96 channels with values of 65 to 128 in 256, two (one, with 268, which the compiler takes where
 // it may: 16 heads on 4, 96 x 96, 4 x 2048 tokens and 129 keys 62 us for 42).  What a wavefront sees is worked out on the scalar unit, so that only
-// tiles at the edges of a window are masked; the lanes of a row look for their largest score together only where one of them has found a larger;
-// weights are summed on the matrix unit; and rows of 64 channels go straight into LDS.  Kernels alone, 16 heads of 64 channels, with the cache write,
-// without and with these: on 4, 4 x 2048 tokens and 129 keys 31.7 / 30.1 us; 6 x 2240 and 513 keys 77.3 / 64.8; on 2, 4 x 4096 and 1,024 keys 140 /
-// 112; on 16, 1 x 2048 and 1,024 keys 47.4 / 38.4; 1 x 700 12.4 / 11.3.
+// tiles at the edges of a window are masked; the lanes of a row look for their largest score together only where one of them has found a larger; and
+// rows of 64 channels go straight into LDS.  Kernels alone, 16 heads of 64 channels, with the cache write, without and with these: on 4, 4 x 2048
+// tokens and 129 keys 30.8 / 28.6 us; 6 x 2240 and 513 keys 80 / 67.6; on 2, 4 x 4096 and 1,024 keys 138 / 112; on 16, 1 x 2048 and 1,024 keys
+// 45.7 / 36.9; on 4, 1 x 700 and 129 keys 12.0 / 10.8.  Weights are summed in 32 bits, as they are before the products take them rounded: sums of the
+// rounded ones, by products with ones, take 0.99 of that (4 x 4096 110 for 112) and 1.03 above 64 channels (128 x 128 68.0 for 66.0).
 
 __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -344,13 +345,7 @@ void window_prefill_mfma_kernel(const WindowArgs a) {
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int i = 0; i < 2 * VC; ++i) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run[2] = {-INFINITY, -INFINITY};
-  // Sums of the weights as they enter the products, on the matrix unit too: rows of ones times the weights.  A weight's rounding then moves both and
-  // leaves the mean of the values in place (errors against 64 bits 3.098e-3 -> 3.090e-3), and the vector unit, which bounds the kernel, adds nothing.
-  f32x4 l_run[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-  bf16x8 ones;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) ones[j] = (__bf16)1.f;
+  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
   const float scale2 = fabsf(a.scale) * 1.4426950408889634f;  // scores in powers of two; the sign is the queries'
   int place = 0;
   for (int k0 = lo; k0 <= last_pos; k0 += kTileKeys) {
@@ -416,19 +411,21 @@ void window_prefill_mfma_kernel(const WindowArgs a) {
           // no key seen yet: every weight is 2^-inf = 0
           const float alpha = __builtin_amdgcn_exp2f((m_run[t] - (m_new == -INFINITY ? 0.f : m_new)) * scale2);
           m_run[t] = m_new;
-          l_run[t][0] *= alpha;  // (the others are the same sum, and not used)
+          l_run[t] *= alpha;
 #pragma unroll
           for (int i = 0; i < 2 * VC; ++i) acc[t][i] *= alpha;
         }
         const float m2 = m_run[t] == -INFINITY ? 0.f : m_run[t] * scale2;
+        float sum = 0.f;
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][kt][i], scale2, -m2));
+            sum += p;
             pf[t][kt * 4 + i] = (__bf16)p;
           }
-        l_run[t] = mfma_bf16(ones, pf[t], l_run[t]);
+        l_run[t] += sum;  // this lane's keys, their weights in 32 bits; the four lane groups are added at the end
       }
 #pragma unroll
       for (int i = 0; i < 2 * VC; ++i) {
@@ -452,7 +449,10 @@ void window_prefill_mfma_kernel(const WindowArgs a) {
   asm volatile("" : "+v"(row_end));  // (where a row goes is worked out again: kept, it would be a register too many)
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
-    const float inv = a.out_scale / l_run[t][0];
+    float l = l_run[t];
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    const float inv = a.out_scale / l;
     const int row = row_end + t * 16 + l16;
     int head;
     const int tok = token_of(row, &head);

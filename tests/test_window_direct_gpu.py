@@ -1,5 +1,7 @@
-"""Window attention over bf16 prompts of 64-channel heads (keys and values straight into LDS, weights summed as they enter the products)
+"""Window attention over bf16 prompts of 64-channel heads (keys and values straight into LDS) and of others
 against 64 bits: portions, windows and heads around tiles of 64 keys and 128 rows, either sign of the scale, and scores that climb."""
+import math
+
 import pytest
 import torch
 
@@ -49,3 +51,18 @@ def test_scores_that_climb(dev, step):
     k[..., 0] = (step / 1.4426950408889634) * torch.arange(L)[None, :, None]
     q, k, v = (t.bfloat16() for t in (q, k, 20 * v))
     assert error(run(dev, q, k, v, window, 1.0, 0), q, k, v, window, 1.0) < 2e-2
+
+
+@pytest.mark.parametrize("d", [48, 64, 96])
+def test_weights_are_summed_in_32_bits(dev, d):
+    """One key of weight one and of the only value, the others all of a weight 0.96 * 2^-8 above 0.5, of which bf16 leaves 0.5: their sum has the
+    whole of it where it is of 32-bit weights.  Means over channels and tokens, of outputs rounded by 2^-9 at most."""
+    L, window = 100, 129
+    weight = 0.5 * (1 + 0.96 * 2.0 ** -8)
+    q, k, v = (torch.zeros(1, L, 1, d, dtype=torch.bfloat16) for _ in range(3))
+    q[..., 0], k[:, 0, :, 0] = 1.0, 1.0
+    v[:, 0] = 1.0 + torch.rand(1, 1, d, generator=torch.Generator().manual_seed(2)).bfloat16()
+    out = run(dev, q, k, v, window, -math.log(weight), 0)[0, 20:, 0]
+    ref = O.window_softmax(q[0].double(), k[0].double(), v[0].double(), -math.log(weight), window)[20:, 0]
+    # (with weights of 0.5 the outputs 1 / (1 + n w) are 0.9 to 1.0 of 3.7e-3 too large)
+    assert abs(float((out / ref - 1).mean())) < 5e-4
