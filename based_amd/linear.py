@@ -21,24 +21,27 @@ def _questions(c=torch._C, ad=forward_ad):
 
 _QUESTIONS = _questions()
 
-
+# Names of this module for what a model asks 119 times a prompt: with them, and the channels by the module, 2.2 us a projection for 3.0.
 _is_tracing = getattr(torch._C, "_is_tracing", torch.jit.is_tracing)
+_is_grad_enabled, _is_compiling, _is_autocast_enabled = torch.is_grad_enabled, torch.compiler.is_compiling, torch.is_autocast_enabled
+_BF16, _STRIDED, _TENSORS = torch.bfloat16, torch.strided, (torch.Tensor, nn.Parameter)
 
 
-def _beyond(x, weight) -> bool:
-    """Torch's own for certain: a gradient, a compiler or a trace wants it, it is not in bf16 or there are too many rows.  Asked in front of everything
-    else, for what the library takes waits for the host as well (the 360M model, 1 x 600 tokens: 4.8 ms, 5.1 where each projection's form was looked
-    up first)."""
-    if torch.is_grad_enabled() or torch.compiler.is_compiling() or _is_tracing() or x.dtype is not torch.bfloat16:
+def _beyond(x, weight, K=None) -> bool:
+    """Torch's own for certain: a gradient, a compiler or a trace wants it, it is not in bf16 or there are too many rows.  Asked in front of
+    everything else, for what the library takes waits for the host as well (the 360M model, 1 x 600 tokens: 4.8 ms, 5.1 where each projection's form
+    was looked up first)."""
+    if _is_grad_enabled() or _is_compiling() or _is_tracing() or x.dtype is not _BF16:
         return True
-    K = weight.size(-1)
+    if K is None:
+        K = weight.size(-1)
     return x.numel() > ops.linear_max_rows(K) * K
 
 
 def _watched() -> bool:
-    """Something else watches or rewrites torch's operations: autocast, forward mode, vmap (of which the weight or the bias may be mapped and x not), a
-    mode.  Or it cannot be told."""
-    if _QUESTIONS is None or forward_ad._current_level >= 0 or torch.is_autocast_enabled("cuda"):
+    """Something else watches or rewrites torch's operations: autocast (of the GPU), forward mode, vmap (of which the weight or the bias may be mapped
+    and x not), a mode.  Or it cannot be told."""
+    if _QUESTIONS is None or forward_ad._current_level >= 0 or _is_autocast_enabled():
         return True
     transform, dispatch_modes, function_modes = _QUESTIONS
     return transform() is not None or dispatch_modes() > 0 or function_modes() > 0
@@ -46,7 +49,7 @@ def _watched() -> bool:
 
 def _ordinary(t) -> bool:
     """A tensor with rows: no subclass, not sparse, not nested."""
-    return type(t) in (torch.Tensor, nn.Parameter) and t.layout is torch.strided and not t.is_nested
+    return type(t) in _TENSORS and t.layout is _STRIDED and not t.is_nested
 
 
 def _plain(x, weight, bias) -> bool:
@@ -72,7 +75,7 @@ class Linear(nn.Linear):
         if torch.jit.is_scripting():
             return F.linear(x, self.weight, self.bias)
         weight, bias = self._operands()
-        if _beyond(x, weight) or not _plain(x, weight, bias):
+        if _beyond(x, weight, self.in_features) or not _plain(x, weight, bias):
             return F.linear(x, weight, bias)
         return ops.linear(x, weight, bias)
 
@@ -87,6 +90,6 @@ def swiglu(fc: nn.Linear, x):
     """`ops.swiglu` of fc(x), in one launch where nothing wants to see what lies between."""
     if _alone(fc):
         weight, bias = fc._operands()
-        if not _beyond(x, weight) and _plain(x, weight, bias):
+        if not _beyond(x, weight, fc.in_features) and _plain(x, weight, bias):
             return ops.swiglu(x, weight, bias)
     return ops.swiglu(fc(x))
