@@ -623,7 +623,8 @@ def linear_form(x, weight, bias=None) -> int:
             one_each = x.dim() == 3 and x.shape[1] == 1 and x.stride(2) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= K  # (the last tokens)
             if 0 < M <= STEP_LINEAR_MAX_ROWS and (x.is_contiguous() or one_each) and K % 8 == 0 and K <= 4096 and 0 < N and (M <= 4 or N <= 16384):
                 form = LINEAR_ROWS
-            elif x.is_contiguous() and STEP_LINEAR_MAX_ROWS < linear_max_rows(K) >= M > 0 and N % 4 == 0 and -(-M // 128) * -(-N // 64) <= 256:
+            elif (x.is_contiguous() and M > 0 and N > 0 and STEP_LINEAR_MAX_ROWS < linear_max_rows(K) >= M and N % 4 == 0
+                  and -(-M // 128) * -(-N // 64) <= 256):
                 form = LINEAR_PROMPT
         _CHECKED[key] = form
     if form != LINEAR_LIBRARY and ((x.data_ptr() | weight.data_ptr()) & 15 or (bias is not None and bias.data_ptr() & 7)):

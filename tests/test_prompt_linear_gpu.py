@@ -62,6 +62,14 @@ def test_which_calls_take_them(dev, M, N, K, form):
     assert rel_l2(ops.linear(x.view(1, M, K), w, b)[0], reference(x, w, b)) < 2.5e-3
 
 
+@pytest.mark.parametrize("M", [4, 40])
+def test_no_features(dev, M):
+    from based_amd.linear import Linear
+
+    with torch.no_grad():
+        assert Linear(256, 0, device=dev, dtype=torch.bfloat16)(torch.randn(M, 256, device=dev).bfloat16()).shape == (M, 0)
+
+
 def test_modules_that_are_watched(dev):
     """Gradients, hooks and modes see torch's own operations; the last tokens of a prompt are rows of a wider tensor."""
     from based_amd import ops
