@@ -572,7 +572,7 @@ def swiglu(u, weight=None, bias=None) -> torch.Tensor:
     same launch where `prompt_linear` is the faster form."""
     if weight is not None:
         form = linear_form(u, weight, bias)
-        if form == LINEAR_PROMPT and weight.shape[0] % 8 == 0:
+        if form == LINEAR_PROMPT and weight.shape[0] % 16 == 0:  # (gates in whole eights, as without a weight)
             return _prompt_linear(u, weight, bias, weight.shape[0] // 2, True)
         u = _linear_as(form, u, weight, bias)
     _require_cuda(u)

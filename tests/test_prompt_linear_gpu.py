@@ -70,6 +70,22 @@ def test_no_features(dev, M):
         assert Linear(256, 0, device=dev, dtype=torch.bfloat16)(torch.randn(M, 256, device=dev).bfloat16()).shape == (M, 0)
 
 
+def test_gates_in_whole_eights(dev):
+    """Any number of rows: others are refused, as by the gate's kernel."""
+    from based_amd.stack import GatedMlp
+
+    with torch.no_grad():
+        for hidden in (16, 20):
+            mlp = GatedMlp(256, hidden_features=hidden, multiple_of=4, device=dev, dtype=torch.bfloat16)
+            for rows in (4, 40, 600):
+                x = torch.randn(1, rows, 256, device=dev).bfloat16()
+                if hidden == 16:
+                    assert mlp(x).shape == x.shape
+                else:
+                    with pytest.raises((ValueError, RuntimeError), match="width must be a multiple of 8"):
+                        mlp(x)
+
+
 def test_modules_that_are_watched(dev):
     """Gradients, hooks and modes see torch's own operations; the last tokens of a prompt are rows of a wider tensor."""
     from based_amd import ops
