@@ -63,6 +63,11 @@ def linear(x, weight, bias=None):
     return ops.linear(x, weight, bias)
 
 
+def linear_like(x, K: int):
+    """`linear` for several products of as many rows of K channels as x has, whose sizes are then asked once where torch has them."""
+    return F.linear if _beyond(x, None, K) else linear
+
+
 class Linear(nn.Linear):
     def _operands(self):
         own = self._parameters  # (`self.weight` looks through Module.__getattr__ first, half a microsecond)
@@ -80,16 +85,16 @@ class Linear(nn.Linear):
         return ops.linear(x, weight, bias)
 
 
-def _alone(fc) -> bool:
+def _alone(fc: Linear) -> bool:
     """A projection without hooks, of which nothing has put a forward of its own into it."""
-    return type(fc) is Linear and "forward" not in fc.__dict__ and not (
+    return "forward" not in fc.__dict__ and not (
         fc._forward_hooks or fc._forward_pre_hooks or nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks)
 
 
 def swiglu(fc: nn.Linear, x):
     """`ops.swiglu` of fc(x), in one launch where nothing wants to see what lies between."""
-    if _alone(fc):
+    if type(fc) is Linear and not _beyond(x, None, fc.in_features) and _alone(fc):
         weight, bias = fc._operands()
-        if not _beyond(x, weight, fc.in_features) and _plain(x, weight, bias):
+        if _plain(x, weight, bias):
             return ops.swiglu(x, weight, bias)
     return ops.swiglu(fc(x))

@@ -12,6 +12,7 @@ import torch
 import torch.nn as nn
 
 from .. import ops
+from ..linear import Linear
 from ..linear import linear as linear_of
 
 
@@ -20,6 +21,9 @@ def round_up(n: int, to: int = 8) -> int:
 
 
 def project(x, linear: nn.Linear):
+    """The product itself: neither hooks nor a forward that something has put into the projection."""
+    if isinstance(linear, Linear):
+        return Linear.forward(linear, x)
     return linear_of(x, linear.weight, linear.bias)
 
 

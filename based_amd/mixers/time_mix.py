@@ -7,7 +7,7 @@ import torch
 import torch.nn as nn
 
 from .. import ops
-from ..linear import Linear, linear
+from ..linear import Linear, linear_like
 from .streaming import cached, portion_start, project, round_up
 
 
@@ -80,7 +80,8 @@ class TimeMix(nn.Module):
         start, step = portion_start(inference_params, B, L)
         state, ring = self._cached(inference_params, B)
         mixed = ops.token_mix(x, self.mu, ring, start)
-        r, k, v, g, hidden = (linear(mixed[i], self.in_proj.weight[self._rows(i)]) for i in range(len(self.MIXES)))
+        weight, linear = self.in_proj.weight, linear_like(x, x.shape[2])
+        r, k, v, g, hidden = (linear(mixed[i], weight[self._rows(i)]) for i in range(len(self.MIXES)))
         if step:
             return project(self._step(r[:, 0], k[:, 0], v[:, 0], g[:, 0], hidden[:, 0], state, start), self.out_proj).unsqueeze(1)
         decay = ops.channel_decay(hidden, self.w2, self.w0)
