@@ -601,10 +601,11 @@ def linear_max_rows(K: int) -> int:
 
 def linear_form(x, weight, bias=None) -> int:
     """Which of its forms `linear` takes.  The library's call costs the host 19 to 21 us, the two others 7.5, and a prompt of a few hundred tokens
-    waits for the host; us on the GPU, weights from memory, library against prompt_linear, N x K: 4096 x 1024, 33 to 512 rows 10 - 11 against 6.8 - 11.7;
-    1024 x 1024 8.1 - 8.8, 6.1 - 7.0; 1024 x 2048 8.1 - 9.7, 8.6 - 9.5; 3072 x 768 7.0 - 9.4, 5.6 - 9.7; up to 256 features of 1024 channels 4.2 - 5.4,
-    5.5 - 6.2; 50280 x 1024, 64 rows 26, 36: one tile for each of the 256 compute units at most.  Up to 8 rows the kernel of the single-token steps
-    (4096 x 1024, 4 rows: 7.6, 6.6, here 4.3; 50280 x 1024, 4 rows 23.7, here 23.3, 8 rows 23.7, here 25.6).
+    waits for the host; us on the GPU, weights from memory, library against prompt_linear, N x K: 4096 x 1024, 33 to 512 rows 11 - 13 against
+    6.9 - 11.9; 1024 x 1024 8.1 - 8.8, 6.1 - 7.0; 1024 x 2048 8.1 - 9.7, 8.6 - 9.5; 3072 x 768 7.0 - 9.4, 5.6 - 9.7; few features of many channels, whose
+    few tiles go over all of them, 64 x 1024 4.1 - 8.3, 5.5 - 5.9; 64 x 2048 5.2 - 8.1, 8.1 - 8.8; 16 x 2048 5.0 - 5.4, 7.9 - 8.0 (in 236 of 16 to 16,384
+    features and 128 to 2,048 channels 0.90 in the mean); 50280 x 1024, 64 rows 26, 36: one tile for each of the 256 compute units at most.  Up to 8 rows
+    the kernel of the single-token steps (4096 x 1024, 4 rows: 7.6, 6.6, here 4.3; 50280 x 1024, 4 rows 23.7, here 23.3, 8 rows 23.7, here 25.6).
     512 rows: from there on tiles of the wider matrices take a second round (513 rows: 4096 x 1024 13.3, 20.7, with the gate 17.3, 21.4; 2048 x 1024
     9.9, 11.2; 1024 x 2048 10.7, 12.1; 1024 x 1024 9.0, 8.3), which a recorded step of so many sequences would pay for.  A prompt that waits for the
     host would still gain: 4 x 129 to 4 x 512 tokens of the 360M model 4.8 ms here, 4.3 without this line, 4 x 128 3.1."""
