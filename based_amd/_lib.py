@@ -155,6 +155,8 @@ SIGNATURES = {
     "based_decay_scan_work": (_I64, [_I64] * 6),
     "based_decay_scan_work_of": (_I64, [_I64] * 7 + [C.c_int]),
     "based_decay_scan": (C.c_int, [_P] * 9 + [_I64] * 14 + [C.c_int, C.c_int, C.c_int, _P]),
+    "based_decay_scan_channels_work": (_I64, [_I64] * 7 + [C.c_int]),
+    "based_decay_scan_channels": (C.c_int, [_P] * 8 + [_I64] * 14 + [C.c_int, C.c_int, C.c_int, _P]),
     "based_decay_step": (C.c_int, [_P] * 13 + [_I64] * 13 + [C.c_int, C.c_float, C.c_int, _P]),
     "based_group_norm_gate": (C.c_int, [_P] * 4 + [_I64] * 10 + [C.c_float, C.c_float, C.c_int, C.c_int, _P]),
     "based_window_attn_attend": (

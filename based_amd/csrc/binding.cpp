@@ -104,6 +104,8 @@ Listed kEntries[] = {
     BASED_ENTRY(based_softcap),
     BASED_ENTRY(based_decay_scan_work_of),
     BASED_ENTRY(based_decay_scan),
+    BASED_ENTRY(based_decay_scan_channels_work),
+    BASED_ENTRY(based_decay_scan_channels),
     BASED_ENTRY(based_decay_step),
     BASED_ENTRY(based_group_norm_gate),
     BASED_ENTRY(based_latent_write),

@@ -25,6 +25,8 @@
 //     also what lies between.
 // fp32 numbers enter a bf16 product as pairs (a number rounded to bf16, and the rest rounded to bf16), so
 // an operand keeps 16 bits and the sums 24.
+#include <type_traits>
+
 #include "stream_common.hpp"
 
 namespace based {
@@ -46,6 +48,7 @@ struct DecayScanArgs {
   long q_sb, q_sl, k_sb, k_sl, v_sb, v_sl, o_sb, o_sl;
   int segs, seg_chunks;  // segments, and 64-token pieces in each
   int silu, fresh;
+  int wide;              // rows of q, k, v and o in whole 16-byte pieces (channel decays, bf16)
 };
 
 template <int CTRL> __device__ __forceinline__ float row_moved(float x) {  // lanes without a source receive 0
@@ -67,12 +70,6 @@ template <int CTRL> __device__ __forceinline__ float row_moved(float x) {  // la
   "v_mul_f32_dpp %5, %1, %5 " ctrl " row_mask:0xf bank_mask:0xf\n\t" \
   "v_mul_f32_dpp %6, %2, %6 " ctrl " row_mask:0xf bank_mask:0xf\n\t" \
   "v_mul_f32_dpp %7, %3, %7 " ctrl " row_mask:0xf bank_mask:0xf"
-__device__ __forceinline__ void row_prefix4(float* prefix, float* before) {
-  asm volatile("s_nop 1\n\t" BASED_ROW_STEP("row_shr:1") BASED_ROW_STEP("row_shr:2") BASED_ROW_STEP("row_shr:4")
-               BASED_ROW_STEP("row_shr:8") BASED_ROW_LAST("row_shr:1")
-               : "+v"(prefix[0]), "+v"(prefix[1]), "+v"(prefix[2]), "+v"(prefix[3]), "+v"(before[0]), "+v"(before[1]), "+v"(before[2]),
-                 "+v"(before[3]));
-}
 __device__ __forceinline__ void row_suffix4(float* suffix, float* after) {
   asm volatile("s_nop 1\n\t" BASED_ROW_STEP("row_shl:1") BASED_ROW_STEP("row_shl:2") BASED_ROW_STEP("row_shl:4")
                BASED_ROW_STEP("row_shl:8") BASED_ROW_LAST("row_shl:1")
@@ -123,19 +120,528 @@ struct HeadPowers {
   __device__ __forceinline__ float of_state(int n) const { return fmaxf((*this)(n), w != 0.f ? 0x1p-149f : 0.f); }
 };
 
+// ---- channel decays, bf16 ----
+// HALVES groups of four wavefronts (1 or 2) share the key channels, 32 DT each (d <= 32 DT HALVES, d % 4 == 0); a wavefront has 16 of the 64 tokens, a
+// lane 8 DT channels of one of them that lie side by side, so that rows come in 16-byte pieces.  In a product the lanes of a 16-lane row bring
+// eight channels of a piece of 32 each; every contraction over channels has that order on both sides.
+//
+// Inside 16 tokens the weights are found by halves: with b = 1, 2, 4, 8, tokens of the second half of each 2 b meet those of its first half, queries
+// decayed from the middle to their token, keys from theirs to the middle, so that one operand x (a query or a key, by the lane's half) times itself
+// holds all of them; the products of decays double with b on the way.  (Keys passed from token to token on the vector unit were 610 of a
+// wavefront's 1,500 instructions to 64 tokens.  x in fp32 on the fp32 matrix unit, which takes the vector unit's issue with it: 4 x 2048 tokens, 16 heads of
+// 64, 58.7 us for 55.5; the error against 64 bits is that of the rounding of o to bf16 either way, 1.659e-3.)
+// Across 16 tokens the keys wait in LDS, decayed to the end of theirs, for the queries decayed from the start of their own and what lies between;
+// the state takes the same keys, decayed itself by what each 16 tokens leave of it.  Outputs belong to the wavefronts of their tokens, so that neither
+// weights nor queries go through LDS, the state's tiles of 16 value channels to a wavefront each: two barriers to 64 tokens, one behind what is written
+// of each piece and one behind what is read.
+//
+// What bounds it: a wavefront issues an instruction in five cycles, whatever it waits for, so 64 tokens are a chain of 11,000 to 14,000 cycles; wavefronts
+// beside each other on a SIMD take next to nothing from one another up to three.  So channels are dealt to more wavefronts where heads are few, prompts
+// are cut into segments of a piece where that leaves compute units idle (decay_channel_segments), and nothing is kept in memory inside the loop:
+// a value fetched back from there waits for the tokens that were asked for before it (17 of them: 68.6 us for 62.9).
+// us before (tokens passed along, four barriers, segments of four pieces) and now: 4 x 2048 tokens, 16 heads of 64: 70.7, 54.6; 2 x 768: 46.7, 22.7;
+// 30 x 513: 123, 71; 2 x 27, 12 heads: 10.2, 8.3; 4 x 2048, 8 heads of 128: 100, 91; 16 x 1024: 184, 113; 2 x 133: 42.4, 24.8.
+template <int DT, int HALVES, int COLS> struct ChannelLds {
+  static constexpr int CH = 32 * DT * HALVES, RS = CH + 8, VS = COLS + 8;
+  static constexpr int OT = COLS / 16, OF = OT / HALVES;  // tiles of 16 value channels, and those a group of wavefronts finishes
+  __bf16 k_hi[kScanTokens * RS], k_lo[kScanTokens * RS];  // k decayed to the end of its 16 tokens, [token][channel as the lanes have them]
+  __bf16 v[kScanTokens * VS];
+  float total[4][CH];                                     // decay over each 16 tokens, by channel
+  // (from here on not in the state pass)
+  float u[CH];
+  __bf16 s_hi[COLS * RS], s_lo[COLS * RS];                // the state in front of the 64 tokens, [value channel][channel as the lanes have them]
+  f32x4 part[HALVES > 1 ? 4 * HALVES * (HALVES - 1) * OF * 64 : 1];  // what the other groups' channels add to an output
+};
+
+// q[i] *= decays of the half in front, k[i] *= those of the half behind, t[i] (the decay over a half) over both; two channels at a time.  Lanes without such
+// a half meet a one, or keep theirs by the bank mask.  (A register must not be read through DPP in the two issue slots behind its writing: the s_nop.)
+#define BASED_HALF_STEP(ctrl, qa, qb, qbank, ka, kb, kbank) \
+  "s_nop 1\n\t" \
+  "v_mul_f32_dpp %0, " qa ", %0 " ctrl " row_mask:0xf bank_mask:" qbank "\n\t" \
+  "v_mul_f32_dpp %1, " qb ", %1 " ctrl " row_mask:0xf bank_mask:" qbank "\n\t" \
+  "v_mul_f32_dpp %2, " ka ", %2 " ctrl " row_mask:0xf bank_mask:" kbank "\n\t" \
+  "v_mul_f32_dpp %3, " kb ", %3 " ctrl " row_mask:0xf bank_mask:" kbank "\n\t" \
+  "v_mul_f32_dpp %4, %4, %4 " ctrl " row_mask:0xf bank_mask:0xf\n\t" \
+  "v_mul_f32_dpp %5, %5, %5 " ctrl " row_mask:0xf bank_mask:0xf"
+#define BASED_HALF_REGS "+&v"(q[0]), "+&v"(q[1]), "+&v"(k[0]), "+&v"(k[1]), "+&v"(t[0]), "+&v"(t[1])
+template <int B> __device__ __forceinline__ void join_halves2(float* q, float* k, float* t, bool second) {
+  if constexpr (B < 4) {
+    const float f0 = second ? 1.f : t[0], f1 = second ? 1.f : t[1];  // decays of lanes of a first half, a one in the others
+    const float s0 = second ? t[0] : 1.f, s1 = second ? t[1] : 1.f;  // of a second half
+    if constexpr (B == 1)
+      asm(BASED_HALF_STEP("quad_perm:[1,0,3,2]", "%6", "%7", "0xf", "%8", "%9", "0xf") : BASED_HALF_REGS : "v"(f0), "v"(f1), "v"(s0), "v"(s1));
+    else
+      asm(BASED_HALF_STEP("quad_perm:[2,3,0,1]", "%6", "%7", "0xf", "%8", "%9", "0xf") : BASED_HALF_REGS : "v"(f0), "v"(f1), "v"(s0), "v"(s1));
+  } else if constexpr (B == 4) {
+    asm(BASED_HALF_STEP("row_half_mirror", "%4", "%5", "0xa", "%4", "%5", "0x5") : BASED_HALF_REGS);
+  } else {
+    asm(BASED_HALF_STEP("row_mirror", "%4", "%5", "0xc", "%4", "%5", "0x3") : BASED_HALF_REGS);
+  }
+}
+#undef BASED_HALF_STEP
+#undef BASED_HALF_REGS
+
+__device__ __forceinline__ f32x4 mfma_16_half(bf16x4 a, bf16x4 b, f32x4 c) {
+  typedef __attribute__((ext_vector_type(4))) short s16x4;
+  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ void split4(f32x4 x, bf16x4& hi, bf16x4& lo) {
+  typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+  uint32_t h0, h1, l0, l1;
+  split2(x[0], x[1], h0, l0);
+  split2(x[2], x[3], h1, l1);
+  hi = __builtin_bit_cast(bf16x4, u32x2{h0, h1});
+  lo = __builtin_bit_cast(bf16x4, u32x2{l0, l1});
+}
+
+constexpr int channel_waves(int dt, int halves) { return halves == 1 ? 3 : dt == 1 ? 4 : 2; }  // wavefronts on a SIMD that registers are left for
+
+template <int DT, int HALVES, int COLS, bool STATE_ONLY, bool FOLD>
+__global__ __launch_bounds__(256 * HALVES, channel_waves(DT, HALVES)) void decay_channel_kernel(const DecayScanArgs a) {
+  typedef ChannelLds<DT, HALVES, COLS> Lds;
+  constexpr int RS = Lds::RS, VS = Lds::VS, E = DT * 8, OT = Lds::OT, OF = Lds::OF;
+  constexpr int VC = COLS / HALVES / 4;                           // value channels that a lane brings of its token
+  constexpr int SP = DT * HALVES * OT / (4 * HALVES);             // 32-channel pieces of the state that a wavefront has of its 16 value channels
+  extern __shared__ __attribute__((aligned(16))) char scan_lds[];
+  Lds& lds = *reinterpret_cast<Lds*>(scan_lds);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, quad = lane >> 4;
+  // This wavefront's key channels, and its 16 tokens of 64: later ones have more in front of them, so that the wavefronts of a SIMD take turns.
+  const int half = wave >> 2, ch0 = half * 32 * DT, blk = half & 1 ? 3 - ((wave + blockIdx.x) & 3) : (wave + blockIdx.x) & 3;
+  const int tile = wave % OT, piece0 = wave / OT * SP;  // its value channels and pieces of the state
+  const int b = blockIdx.x / a.H, h = blockIdx.x % a.H, sg = blockIdx.z;
+  const int col_base = blockIdx.y * COLS, dv0 = col_base + tile * 16;
+  const bool has_cols = dv0 < a.dv, col_in = dv0 + l16 < a.dv;
+  const __bf16* qp = static_cast<const __bf16*>(a.q) + b * a.q_sb + (long)h * a.d;
+  const __bf16* kp = static_cast<const __bf16*>(a.k) + b * a.k_sb + (long)h * a.d;
+  const __bf16* vp = static_cast<const __bf16*>(a.v) + b * a.v_sb + (long)h * a.dv;
+  const float* lwp = a.lw + ((long)b * a.L) * a.H * a.d + (long)h * a.d;
+  const long bh = (long)b * a.H + h;
+  float* st = a.state + (bh * a.dv + (col_in ? dv0 + l16 : 0)) * a.dp;
+
+  // channel of element 4 f of piece c, and of element i; of the state's tile ct
+  auto chan = [&](int c, int f, int quad) { return ch0 + quad * E + c * 8 + f * 4; };
+  auto chan_of = [&](int i, int quad) { return ch0 + quad * E + i; };
+  auto state_chan = [&](int ct, int quad) { return (piece0 + ct / 2) / DT * 32 * DT + quad * E + (piece0 + ct / 2) % DT * 8 + ct % 2 * 4; };
+
+  struct Stage {
+    bf16x4 q[STATE_ONLY ? 1 : 2 * DT], k[2 * DT], v[VC / 4];
+    f32x4 lw[2 * DT];
+  };
+  const int first = sg * a.seg_chunks, chunks = (a.L + kScanTokens - 1) / kScanTokens;
+  const int last = first + a.seg_chunks < chunks ? first + a.seg_chunks : chunks;
+  // The rows of this wavefront's 16 tokens, unconditionally (places past the end are cleared at use): the place of the 64 tokens is the same for all
+  // lanes, and what lies behind it (in front of it, where a stride is below zero) fits 32 bits.
+  const int q_back = a.q_sl < 0 ? (int)a.q_sl * (kScanTokens - 1) : 0, k_back = a.k_sl < 0 ? (int)a.k_sl * (kScanTokens - 1) : 0,
+            v_back = a.v_sl < 0 ? (int)a.v_sl * (kScanTokens - 1) : 0;
+  auto pieces = [](bf16x8 x, bf16x4& lo, bf16x4& hi) {
+    lo = __builtin_shufflevector(x, x, 0, 1, 2, 3), hi = __builtin_shufflevector(x, x, 4, 5, 6, 7);
+  };
+  // (parts: 1 keys, 2 decays, 4 queries, 8 values)
+  auto fetch = [&](Stage& s, int chunk, int l16, int quad, auto parts) {
+    constexpr int kParts = decltype(parts)::value;
+    const int left = a.L - chunk * kScanTokens, mine = blk * 16 + l16, t = mine < left ? mine : left - 1;
+    const long t0 = (long)chunk * kScanTokens;
+    auto rows = [&](const __bf16* p, long sl, int back, bf16x4* to) {  // key channels
+      const char* p0 = reinterpret_cast<const char*>(p + t0 * sl + back);
+      const uint32_t at = (uint32_t)(t * (int)sl - back);
+      if (a.wide) {  // (uniform)
+#pragma unroll
+        for (int c = 0; c < DT; ++c)
+          pieces(*reinterpret_cast<const bf16x8*>(p0 + (at + (chan(c, 0, quad) < a.d ? chan(c, 0, quad) : 0)) * 2u), to[2 * c], to[2 * c + 1]);
+      } else {
+#pragma unroll
+        for (int g = 0; g < 2 * DT; ++g)
+          to[g] = *reinterpret_cast<const bf16x4*>(p0 + (at + (chan(g >> 1, g & 1, quad) < a.d ? chan(g >> 1, g & 1, quad) : 0)) * 2u);
+      }
+    };
+    if constexpr ((kParts & 1) != 0) rows(kp, a.k_sl, k_back, s.k);
+    if constexpr ((kParts & 2) != 0) {
+      const char* w0 = reinterpret_cast<const char*>(lwp + t0 * a.H * a.d);
+      const uint32_t at = (uint32_t)t * (uint32_t)(a.H * a.d);
+#pragma unroll
+      for (int g = 0; g < 2 * DT; ++g)
+        s.lw[g] = *reinterpret_cast<const f32x4*>(w0 + (at + (chan(g >> 1, g & 1, quad) < a.d ? chan(g >> 1, g & 1, quad) : 0)) * 4u);
+    }
+    if constexpr (!STATE_ONLY && (kParts & 4) != 0) rows(qp, a.q_sl, q_back, s.q);
+    if constexpr ((kParts & 8) != 0) {
+      const char* v0 = reinterpret_cast<const char*>(vp + t0 * a.v_sl + v_back);
+      const uint32_t at = (uint32_t)(t * (int)a.v_sl - v_back);
+      const int col = col_base + half * (COLS / HALVES) + quad * VC;
+      if (VC >= 8 && a.wide) {
+#pragma unroll
+        for (int f = 0; f < VC / 8; ++f)
+          pieces(*reinterpret_cast<const bf16x8*>(v0 + (at + (uint32_t)(col + f * 8 < a.dv ? col + f * 8 : 0)) * 2u), s.v[2 * f], s.v[2 * f + 1]);
+      } else {
+#pragma unroll
+        for (int f = 0; f < VC / 4; ++f) s.v[f] = *reinterpret_cast<const bf16x4*>(v0 + (at + (uint32_t)(col + f * 4 < a.dv ? col + f * 4 : 0)) * 2u);
+      }
+    }
+  };
+  Stage cur;
+  if (first < last) fetch(cur, first, l16, quad, std::integral_constant<int, 15>{});
+  if constexpr (!STATE_ONLY) {
+    const int ch = threadIdx.x;
+    if (ch < Lds::CH) lds.u[ch] = ch < a.d ? to_f32(static_cast<const __bf16*>(a.u)[(long)h * a.d + ch]) : 0.f;
+  }
+
+  // state: tile ct holds key channels 16 ct + 4 quad + i of value channel dv0 + l16
+  f32x4 S[2 * SP];
+  {
+    const long seg_row = (col_in ? dv0 + l16 : 0), seg_step = (long)a.dv * a.dp;
+    const float* segs = a.seg + (bh * a.segs * a.dv + seg_row) * a.dp;
+    // FOLD: what the segments in front have added is put together here, the state that enters the call from the last one's place, where
+    // the state pass has left it (the last segment replaces it).  Kernels of their own: the others have registers for what they do.
+    const bool fold = FOLD && !STATE_ONLY && a.segs > 1;
+    const float* from = a.segs > 1 ? segs + (fold ? a.segs - 1 : sg) * seg_step : st;
+    const bool zero = STATE_ONLY || ((a.segs == 1 || fold) && a.fresh);
+#pragma unroll
+    for (int ct = 0; ct < 2 * SP; ++ct) {
+      const int ch = state_chan(ct, quad);
+      S[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (!zero && col_in && ch < a.d) S[ct] = *reinterpret_cast<const f32x4*>(from + ch);
+    }
+    if constexpr (STATE_ONLY) {
+      if (FOLD && !a.fresh && sg == 0 && col_in) {
+        float* keep = a.seg + ((bh * a.segs + a.segs - 1) * a.dv + seg_row) * a.dp;
+#pragma unroll
+        for (int ct = 0; ct < 2 * SP; ++ct) {
+          const int ch = state_chan(ct, quad);
+          if (ch < a.d) *reinterpret_cast<f32x4*>(keep + ch) = *reinterpret_cast<const f32x4*>(st + ch);
+        }
+      }
+    } else if (fold) {
+      constexpr int U = SP > 2 ? 2 : 4;  // segments asked for together
+      for (int s0 = 0; s0 < sg; s0 += U) {
+        f32x4 add[U][2 * SP], l[U][2 * SP];
+#pragma unroll
+        for (int n = 0; n < U; ++n)
+#pragma unroll
+          for (int ct = 0; ct < 2 * SP; ++ct) {
+            const int ch = state_chan(ct, quad) < a.d ? state_chan(ct, quad) : 0, s = s0 + n < sg ? s0 + n : sg - 1;
+            add[n][ct] = *reinterpret_cast<const f32x4*>(segs + s * seg_step + ch);
+            l[n][ct] = *reinterpret_cast<const f32x4*>(a.seg_lw + (bh * a.segs + s) * a.dp + ch);
+          }
+#pragma unroll
+        for (int n = 0; n < U; ++n) {
+          if (s0 + n >= sg) break;  // (uniform)
+#pragma unroll
+          for (int ct = 0; ct < 2 * SP; ++ct)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const float sum = __builtin_fmaf(S[ct][j], l[n][ct][j], add[n][ct][j]);
+              S[ct][j] = col_in && state_chan(ct, quad) < a.d ? sum : 0.f;
+            }
+        }
+      }
+    }
+  }
+  if constexpr (!STATE_ONLY) lds_barrier();  // (the bonus)
+  int apart = 0;  // byte i: the half length at which row s = 4 quad + i meets this lane's token, 0 where it does not
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int s = quad * 4 + i, z = l16 ^ s;
+    apart |= (s >= l16 ? 0 : 0x80000000u >> __builtin_clz(z | 1)) << i * 8;
+  }
+  float seg_total = 1.f;  // (state pass) decay of the segment so far, of the channel that is this thread's number
+
+  for (int chunk = first; chunk < last; ++chunk) {
+    // (What follows from the lane is worked out anew each time: kept in front of the loop, it went to memory, and every value fetched back waited
+    // for the next tokens as well.)
+    int here = lane;
+    asm volatile("" : "+v"(here));
+    const int l16 = here & 15, quad = here >> 4;
+    const int tr_row = l16 >> 2, tr_piece = (l16 & 3) * 4;  // what a lane names of a transposed read: a token of four, and four channels of 16
+    const int left = a.L - chunk * kScanTokens, n = left < kScanTokens ? left : kScanTokens;
+    const int t = blk * 16 + l16;  // this lane's token
+    const bool live = t < n;
+    float q[STATE_ONLY ? 1 : E], k[E], w[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      if constexpr (!STATE_ONLY) q[i] = to_f32(cur.q[i >> 2][i & 3]);
+      k[i] = to_f32(cur.k[i >> 2][i & 3]);
+      w[i] = __builtin_amdgcn_exp2f(cur.lw[i >> 2][i & 3]);
+    }
+    if (a.silu) {  // (one branch for all of them)
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+        if constexpr (!STATE_ONLY) q[i] = round_to<__bf16>(silu_exact(q[i]));
+        k[i] = round_to<__bf16>(silu_exact(k[i]));
+      }
+    }
+    if (n < kScanTokens || a.d < Lds::CH) {  // (uniform)
+#pragma unroll
+      for (int g = 0; g < 2 * DT; ++g) {
+        const bool in = live && chan(g >> 1, g & 1, quad) < a.d;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if constexpr (!STATE_ONLY) q[g * 4 + j] = in ? q[g * 4 + j] : 0.f;
+          k[g * 4 + j] = in ? k[g * 4 + j] : 0.f;
+          w[g * 4 + j] = in ? w[g * 4 + j] : 1.f;
+        }
+      }
+    }
+    typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+    u32x2 vv[VC / 4];
+#pragma unroll
+    for (int f = 0; f < VC / 4; ++f) vv[f] = __builtin_bit_cast(u32x2, cur.v[f]);
+    if (a.silu) {
+#pragma unroll
+      for (int f = 0; f < VC / 4; ++f)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) vv[f][j] = pack_bf16(silu_exact(to_f32(cur.v[f][2 * j])), silu_exact(to_f32(cur.v[f][2 * j + 1])));
+    }
+    if (n < kScanTokens || col_base + COLS > a.dv) {
+#pragma unroll
+      for (int f = 0; f < VC / 4; ++f)
+        if (!(live && col_base + half * (COLS / HALVES) + quad * VC + f * 4 < a.dv)) vv[f] = u32x2{0u, 0u};
+    }
+#pragma unroll
+    for (int f = 0; f < VC / 4; ++f) *reinterpret_cast<u32x2*>(&lds.v[t * VS + half * (COLS / HALVES) + quad * VC + f * 4]) = vv[f];
+    const bool more = chunk + 1 < last;
+    auto ask = [&](auto parts) {  // (the memory unit takes rows of 16 tokens a lane at a time: a few requests here and there, none of which waits for its turn)
+      if (more) fetch(cur, chunk + 1, l16, quad, parts);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // the weights inside the 16 tokens: column t, rows s = 4 quad + i
+    f32x4 diag = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (!STATE_ONLY) {
+      float bonus = 0.f;
+#pragma unroll
+      for (int i = 0; i < E; i += 4) {
+        const f32x4 u = *reinterpret_cast<const f32x4*>(&lds.u[chan_of(i, quad)]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bonus = __builtin_fmaf(q[i + j] * u[j], k[i + j], bonus);
+      }
+      bonus = sum_quads4(bonus, bonus, bonus, bonus);  // (in every lane of the token)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) diag[i] = quad * 4 + i == l16 ? bonus : 0.f;
+      auto meet = [&](int half_len, f32x4 acc) {  // rows of the first half of this lane's second half
+#pragma unroll
+        for (int i = 0; i < 4; ++i) diag[i] = (apart >> i * 8 & 0xff) == half_len ? acc[i] : diag[i];
+      };
+      {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < DT; ++c) {  // (neighbours: no decay lies between, the operands are what came in)
+          u32x4 x;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            x[e] = pack_bf16(l16 & 1 ? q[c * 8 + 2 * e] : k[c * 8 + 2 * e], l16 & 1 ? q[c * 8 + 2 * e + 1] : k[c * 8 + 2 * e + 1]);
+          acc = mfma_16(__builtin_bit_cast(bf16x8, x), __builtin_bit_cast(bf16x8, x), acc);
+        }
+#pragma unroll
+        for (int i = 0; i < E; i += 2) join_halves2<1>(q + i, k + i, w + i, l16 & 1);
+        meet(1, acc);
+      }
+      auto level = [&](auto half_len) {
+        constexpr int HB = decltype(half_len)::value;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < DT; ++c) {
+          float x[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) x[i] = l16 & HB ? q[c * 8 + i] : k[c * 8 + i];
+          bf16x8 hi, lo;
+          split8(x, hi, lo);
+          acc = mfma_16(hi, hi, acc);
+          acc = mfma_16(lo, hi, acc);
+          acc = mfma_16(hi, lo, acc);
+        }
+#pragma unroll
+        for (int i = 0; i < E; i += 2) join_halves2<HB>(q + i, k + i, w + i, l16 & HB);
+        meet(HB, acc);
+      };
+      ask(std::integral_constant<int, 1>{});
+      level(std::integral_constant<int, 2>{});
+      ask(std::integral_constant<int, 2>{});
+      level(std::integral_constant<int, 4>{});
+      ask(std::integral_constant<int, 4>{});
+      level(std::integral_constant<int, 8>{});
+      ask(std::integral_constant<int, 8>{});
+      // q is decayed from the start of the 16 tokens now, k to their end, w the decay over all of them
+    } else {
+#pragma unroll
+      for (int i = 0; i < E; i += 4) row_suffix4(w + i, k + i);  // (the product over all 16 is lane 0's)
+      ask(std::integral_constant<int, 15>{});
+    }
+
+#pragma unroll
+    for (int c = 0; c < DT; ++c) {
+      bf16x8 hi, lo;
+      split8(k + c * 8, hi, lo);
+      *reinterpret_cast<bf16x8*>(&lds.k_hi[t * RS + ch0 + c * 32 + quad * 8]) = hi;
+      *reinterpret_cast<bf16x8*>(&lds.k_lo[t * RS + ch0 + c * 32 + quad * 8]) = lo;
+    }
+    if (l16 == 0) {
+#pragma unroll
+      for (int i = 0; i < E; i += 4) *reinterpret_cast<f32x4*>(&lds.total[blk][chan_of(i, quad)]) = f32x4{w[i], w[i + 1], w[i + 2], w[i + 3]};
+    }
+    if constexpr (!STATE_ONLY) {
+      if (has_cols) {
+        const int s_row = tile / 4 * 64 + (l16 >> 2) * 16 + tile % 4 * 4 + (l16 & 3);  // in the order of the outputs' rows
+#pragma unroll
+        for (int c = 0; c < SP; ++c) {
+          bf16x8 hi, lo;
+          const float x[8] = {S[2 * c][0], S[2 * c][1], S[2 * c][2], S[2 * c][3], S[2 * c + 1][0], S[2 * c + 1][1], S[2 * c + 1][2], S[2 * c + 1][3]};
+          split8(x, hi, lo);
+          *reinterpret_cast<bf16x8*>(&lds.s_hi[s_row * RS + (piece0 + c) * 32 + quad * 8]) = hi;
+          *reinterpret_cast<bf16x8*>(&lds.s_lo[s_row * RS + (piece0 + c) * 32 + quad * 8]) = lo;
+        }
+      }
+    }
+    lds_barrier();
+
+    f32x4 o[STATE_ONLY ? 1 : OT];  // column t, rows: value channels 16 quad + 4 g + i of each 64
+    if constexpr (!STATE_ONLY) {
+#pragma unroll
+      for (int g = 0; g < OT; ++g) o[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+      f32x4 P = diag;  // column t, rows s of 16 tokens j
+      for (int j = blk;;) {
+        // (all of a round's reads in front of it)
+        bf16x4 v4[OT], ph, pl;
+        bf16x8 kh[DT], kl[DT], hi[DT], lo[DT];
+        const int before = j > 0 ? j - 1 : 0;
+#pragma unroll
+        for (int g = 0; g < OT; ++g) v4[g] = read_transposed(&lds.v[(j * 16 + quad * 4 + tr_row) * VS + g / 4 * 64 + tr_piece * 4 + g % 4 * 4]);
+#pragma unroll
+        for (int c = 0; c < DT; ++c) {
+          kh[c] = *reinterpret_cast<const bf16x8*>(&lds.k_hi[(before * 16 + l16) * RS + ch0 + c * 32 + quad * 8]);
+          kl[c] = *reinterpret_cast<const bf16x8*>(&lds.k_lo[(before * 16 + l16) * RS + ch0 + c * 32 + quad * 8]);
+        }
+        split4(P, ph, pl);
+#pragma unroll
+        for (int g = 0; g < OT; ++g) {
+          o[g] = mfma_16_half(v4[g], ph, o[g]);
+          o[g] = mfma_16_half(v4[g], pl, o[g]);
+        }
+#pragma unroll
+        for (int c = 0; c < DT; ++c) split8(q + c * 8, hi[c], lo[c]);
+        if (--j < 0) {  // q is scaled to the start of the 64 tokens
+#pragma unroll
+          for (int g = 0; g < OT; ++g)
+#pragma unroll
+            for (int c = 0; c < DT; ++c) {
+              const bf16x8 sh = *reinterpret_cast<const bf16x8*>(&lds.s_hi[(g * 16 + l16) * RS + ch0 + c * 32 + quad * 8]);
+              const bf16x8 sl = *reinterpret_cast<const bf16x8*>(&lds.s_lo[(g * 16 + l16) * RS + ch0 + c * 32 + quad * 8]);
+              o[g] = mfma_16(sh, hi[c], o[g]);
+              o[g] = mfma_16(sl, hi[c], o[g]);
+              o[g] = mfma_16(sh, lo[c], o[g]);
+            }
+          break;
+        }
+        P = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < DT; ++c) {
+          P = mfma_16(kh[c], hi[c], P);
+          P = mfma_16(kl[c], hi[c], P);
+          P = mfma_16(kh[c], lo[c], P);
+        }
+#pragma unroll
+        for (int i = 0; i < E; i += 4) {
+          const f32x4 f = *reinterpret_cast<const f32x4*>(&lds.total[j][chan_of(i, quad)]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) q[i + e] *= f[e];
+        }
+      }
+    }
+    auto store = [&](const f32x4* x) {  // the tiles that this group finishes: 4 OF value channels side by side of each lane
+      const int col = col_base + half * OF / 4 * 64 + quad * 16 + half * OF % 4 * 4;
+      __bf16* to = static_cast<__bf16*>(a.o) + b * a.o_sb + (long)(chunk * kScanTokens + t) * a.o_sl + (long)h * a.dv + col;
+      uint32_t y[2 * OF];
+#pragma unroll
+      for (int i = 0; i < 2 * OF; ++i) y[i] = pack_bf16(x[i / 2][i % 2 * 2], x[i / 2][i % 2 * 2 + 1]);
+      if (!live) return;
+      if constexpr (OF > 1) {
+        if (a.wide) {
+#pragma unroll
+          for (int f = 0; f < OF / 2; ++f)
+            if (col + f * 8 < a.dv) *reinterpret_cast<u32x4*>(to + f * 8) = u32x4{y[f * 4], y[f * 4 + 1], y[f * 4 + 2], y[f * 4 + 3]};
+          return;
+        }
+      }
+#pragma unroll
+      for (int f = 0; f < OF; ++f)
+        if (col + f * 4 < a.dv) *reinterpret_cast<u32x2*>(to + f * 4) = u32x2{y[f * 2], y[f * 2 + 1]};
+    };
+    if constexpr (!STATE_ONLY) {
+      if constexpr (HALVES == 1) {
+        store(o);
+      } else {
+#pragma unroll
+        for (int other = 0; other < HALVES; ++other) {  // (of each group the tiles that it finishes; the others' parts in order of their groups)
+          if (other == half) continue;
+#pragma unroll
+          for (int g = 0; g < OF; ++g)
+            lds.part[(((blk * HALVES + other) * (HALVES - 1) + (half < other ? half : half - 1)) * OF + g) * 64 + here] = o[other * OF + g];
+        }
+      }
+    }
+
+    if constexpr (STATE_ONLY) {
+      const int ch = threadIdx.x;
+      if (ch < Lds::CH) seg_total *= (lds.total[0][ch] * lds.total[1][ch]) * (lds.total[2][ch] * lds.total[3][ch]);
+    }
+    if (has_cols) {  // the state behind the 64 tokens: what each 16 add, by themselves, and then one behind the other
+      bf16x4 v4[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v4[j] = read_transposed(&lds.v[(j * 16 + quad * 4 + tr_row) * VS + tile * 16 + tr_piece]);
+#pragma unroll
+      for (int ct = 0; ct < 2 * SP; ++ct) {
+        f32x4 add[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int at = (j * 16 + quad * 4 + tr_row) * RS + (piece0 + (ct >> 1)) * 32 + (ct & 1) * 4 + tr_piece * 2;
+          add[j] = mfma_16_half(read_transposed(&lds.k_hi[at]), v4[j], f32x4{0.f, 0.f, 0.f, 0.f});
+          add[j] = mfma_16_half(read_transposed(&lds.k_lo[at]), v4[j], add[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const f32x4 f = *reinterpret_cast<const f32x4*>(&lds.total[j][state_chan(ct, quad)]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) S[ct][i] = __builtin_fmaf(S[ct][i], f[i], add[j][i]);
+        }
+      }
+    }
+    lds_barrier();
+    if constexpr (!STATE_ONLY && HALVES > 1) {
+      f32x4 x[OF];
+#pragma unroll
+      for (int g = 0; g < OF; ++g) {
+        x[g] = o[g];
+#pragma unroll
+        for (int own = 1; own < HALVES; ++own) x[g] = own == half ? o[own * OF + g] : x[g];
+#pragma unroll
+        for (int m = 0; m < HALVES - 1; ++m) x[g] += lds.part[(((blk * HALVES + half) * (HALVES - 1) + m) * OF + g) * 64 + here];
+      }
+      store(x);
+    }
+  }
+  if constexpr (STATE_ONLY) {
+    if (blockIdx.y == 0 && threadIdx.x < a.d) a.seg_lw[(bh * a.segs + sg) * a.dp + threadIdx.x] = seg_total;
+  }
+  if (!has_cols) return;
+  float* to = st;
+  if constexpr (STATE_ONLY) to = a.seg + ((bh * a.segs + sg) * a.dv + (col_in ? dv0 + l16 : 0)) * a.dp;
+  if (STATE_ONLY || sg == a.segs - 1) {
+#pragma unroll
+    for (int ct = 0; ct < 2 * SP; ++ct) {
+      const int ch = state_chan(ct, quad);
+      if (col_in && ch < a.d) *reinterpret_cast<f32x4*>(to + ch) = S[ct];
+    }
+  }
+}
+
+// ---- head decays, bf16 ----
 // HALVES wavefronts (1 or 2) share the key channels of 16 tokens, DT 32-channel pieces each (d <= 32 DT HALVES, d % 4 == 0), so
 // that what a lane holds of a token stays in registers; their parts of P are added through LDS.  Channels of a piece are held by the lanes in the
 // order of the accumulators: element e < 4 of a lane in 16-lane row `quad` is channel 4 quad + e, e >= 4
 // channel 16 + 4 quad + e - 4; every contraction over channels uses that order on both sides.
-template <int DT, int HALVES, bool CHANNEL> struct ScanLds {
+template <int DT, int HALVES> struct HeadLds {
   static constexpr int CH = 32 * DT * HALVES, RS = CH + 8, TS = kScanTokens + 8;
-  __bf16 q_hi[kScanTokens * RS];                 // q scaled to the start of the 64 tokens; head decays: q itself
-  __bf16 q_lo[CHANNEL ? kScanTokens * RS : 8];
+  __bf16 q[kScanTokens * RS];
   union {
-    struct {
-      __bf16 hi[kScanTokens * RS];               // k decayed to the end of its 16 tokens; head decays: k itself
-      __bf16 lo[CHANNEL ? kScanTokens * RS : 8];
-    } k;
+    __bf16 k[kScanTokens * RS];
     struct {
       __bf16 hi[kScanTokens * TS], lo[kScanTokens * TS];  // P, [t][s]
       f32x4 part[HALVES > 1 ? 4 * 4 * 64 : 1];            // the second half's part of P, as its lanes hold it
@@ -143,12 +649,11 @@ template <int DT, int HALVES, bool CHANNEL> struct ScanLds {
   };
   __bf16 kt_hi[CH * TS], kt_lo[CH * TS];         // k decayed to the end of the 64 tokens, [channel][token]
   __bf16 vt[64 * HALVES * TS];                            // v, [channel][token]
-  float total[4][CH], all[CH];                   // decay over each 16 tokens, and over the 64
 };
 
-template <int DT, int HALVES, bool CHANNEL, bool STATE_ONLY, bool FOLD>
-__global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const DecayScanArgs a) {
-  typedef ScanLds<DT, HALVES, CHANNEL> Lds;
+template <int DT, int HALVES, bool STATE_ONLY, bool FOLD>
+__global__ __launch_bounds__(256 * HALVES, 2) void decay_head_kernel(const DecayScanArgs a) {
+  typedef HeadLds<DT, HALVES> Lds;
   constexpr int RS = Lds::RS, TS = Lds::TS, E = DT * 8, DA = DT * HALVES;
   extern __shared__ __attribute__((aligned(16))) char scan_lds[];
   Lds& lds = *reinterpret_cast<Lds*>(scan_lds);
@@ -160,11 +665,7 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
   const __bf16* qp = static_cast<const __bf16*>(a.q) + b * a.q_sb + (long)h * a.d;
   const __bf16* kp = static_cast<const __bf16*>(a.k) + b * a.k_sb + (long)h * a.d;
   const __bf16* vp = static_cast<const __bf16*>(a.v) + b * a.v_sb + (long)h * a.dv;
-  const float* lwp = CHANNEL ? a.lw + ((long)b * a.L) * a.H * a.d + (long)h * a.d : nullptr;
-  const auto powers = [&] {
-    if constexpr (CHANNEL) return nullptr;
-    else return HeadPowers(a, h);
-  }();
+  const HeadPowers powers(a, h);
   const long bh = (long)b * a.H + h;
   float* st = a.state + (bh * a.dv + (col_in ? dv0 + l16 : 0)) * a.dp;
 
@@ -179,7 +680,6 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
     const float* segs = a.seg + (bh * a.segs * a.dv + seg_row) * a.dp;
     // FOLD: what the segments in front have added is put together here, the state that enters the call from the last one's place, where
     // the state pass has left it (the last segment replaces it).  Kernels of their own: the others have registers for what they do.
-    // (Always so in these; but without the branch the compiler lays the loads out worse: 1 x 2000 tokens, 12 heads of 64, 50.8 us, with it 49.7.)
     const bool fold = FOLD && !STATE_ONLY && a.segs > 1;
     const float* from = a.segs > 1 ? segs + (fold ? a.segs - 1 : sg) * seg_step : st;
     const bool zero = STATE_ONLY || ((a.segs == 1 || fold) && a.fresh);
@@ -199,18 +699,16 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
         }
       }
     } else if (fold) {
-      float seg_decay = 0.f;  // (all in front of the last are of one length)
-      if constexpr (!CHANNEL) seg_decay = powers.of_state(a.seg_chunks * kScanTokens);
+      const float seg_decay = powers.of_state(a.seg_chunks * kScanTokens);  // (all in front of the last are of one length)
       constexpr int U = 4;  // segments asked for together
       for (int s0 = 0; s0 < sg; s0 += U) {
-        f32x4 add[U][2 * DA], l[U][2 * DA];
+        f32x4 add[U][2 * DA];
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
           for (int ct = 0; ct < 2 * DA; ++ct) {
             const int ch = ct * 16 + quad * 4 < a.d ? ct * 16 + quad * 4 : 0, s = s0 + u < sg ? s0 + u : sg - 1;
             add[u][ct] = *reinterpret_cast<const f32x4*>(segs + s * seg_step + ch);
-            if constexpr (CHANNEL) l[u][ct] = *reinterpret_cast<const f32x4*>(a.seg_lw + (bh * a.segs + s) * a.dp + ch);
           }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -219,18 +717,15 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
           for (int ct = 0; ct < 2 * DA; ++ct)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-              const float sum = __builtin_fmaf(S[ct][j], CHANNEL ? l[u][ct][j] : seg_decay, add[u][ct][j]);
+              const float sum = __builtin_fmaf(S[ct][j], seg_decay, add[u][ct][j]);
               S[ct][j] = col_in && ct * 16 + quad * 4 < a.d ? sum : 0.f;
             }
         }
       }
     }
   }
-  float seg_total = 1.f;  // (state pass, channel decays) decay of the segment so far, of the channel that is this thread's number
-
   struct Stage {
     bf16x4 q[STATE_ONLY ? 1 : 2 * DT], k[2 * DT], v[4];
-    f32x4 lw[CHANNEL ? 2 * DT : 1];
   };
   const int first = sg * a.seg_chunks, chunks = (a.L + kScanTokens - 1) / kScanTokens;
   const int last = first + a.seg_chunks < chunks ? first + a.seg_chunks : chunks;
@@ -242,14 +737,12 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
     const __bf16* q0 = qp + t0 * a.q_sl;
     const __bf16* k0 = kp + t0 * a.k_sl;
     const __bf16* v0 = vp + t0 * a.v_sl;
-    const float* w0 = CHANNEL ? lwp + t0 * a.H * a.d : nullptr;
-    const int tq = t * (int)a.q_sl, tk = t * (int)a.k_sl, tv = t * (int)a.v_sl, tw = t * a.H * a.d;
+    const int tq = t * (int)a.q_sl, tk = t * (int)a.k_sl, tv = t * (int)a.v_sl;
 #pragma unroll
     for (int g = 0; g < 2 * DT; ++g) {
       const int ch = chan(g >> 1, g & 1) < a.d ? chan(g >> 1, g & 1) : 0;
       if constexpr (!STATE_ONLY) s.q[g] = *reinterpret_cast<const bf16x4*>(q0 + (tq + ch));
       s.k[g] = *reinterpret_cast<const bf16x4*>(k0 + (tk + ch));
-      if constexpr (CHANNEL) s.lw[g] = *reinterpret_cast<const f32x4*>(w0 + (tw + ch));
     }
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
@@ -258,8 +751,6 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
     }
   };
 
-  // the next 64 tokens are asked for as soon as these are in registers, or where those are scarce behind P
-  constexpr bool LATE = CHANNEL && !STATE_ONLY && HALVES > 1;
   Stage cur;
   if (first < last) fetch(cur, first);
   // A head decay below zero: with w's sign s, s^t v_t in the place of v_t, s S in that of the state and s^t o_t in that of o_t, the powers are
@@ -270,12 +761,12 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
 #pragma unroll
     for (int ct = 0; ct < 2 * DA; ++ct) S[ct] = turn ? -S[ct] : S[ct];
   };
-  if constexpr (!CHANNEL) odd_sign = powers.w < 0.f && (l16 & 1) ? 0x80008000u : 0u;
+  odd_sign = powers.w < 0.f && (l16 & 1) ? 0x80008000u : 0u;
   for (int chunk = first; chunk < last; ++chunk) {
     const int left = a.L - chunk * kScanTokens, n = left < kScanTokens ? left : kScanTokens;
     const int t = blk * 16 + l16;  // this lane's token
     const bool live = t < n;
-    float q[STATE_ONLY ? 1 : E], k[E], w[CHANNEL ? E : 1];
+    float q[STATE_ONLY ? 1 : E], k[E];
 #pragma unroll
     for (int i = 0; i < E; ++i) {
       if constexpr (!STATE_ONLY) q[i] = to_f32(cur.q[i >> 2][i & 3]);
@@ -295,62 +786,6 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
       for (int j = 0; j < 4; ++j) {
         if constexpr (!STATE_ONLY) q[g * 4 + j] = in ? q[g * 4 + j] : 0.f;
         k[g * 4 + j] = in ? k[g * 4 + j] : 0.f;
-        if constexpr (CHANNEL) w[g * 4 + j] = in ? __builtin_amdgcn_exp2f(cur.lw[g][j]) : 1.f;
-      }
-    }
-
-    if constexpr (HALVES > 1) __builtin_amdgcn_sched_barrier(0);
-    // The weights inside the 16 tokens.  BACK: token t with the one 4 g + quad back in [g], zero where that is none of the 16, four sums
-    // added up over the channels' lanes at once without LDS (two exchanges through LDS a sum, 16 heads of 64, 12 x 960 tokens: 121.2 us ->
-    // 117.1; 12 heads, 1 x 1000: 50.2 -> 47.8); otherwise column t, rows s = 4 quad + i (128 channels: 104.9 us, 107.5 with BACK, which spills
-    // more; up to 32 channels where there are no segments to put together, so more workgroups than are on the GPU at once: 147 registers and three
-    // wavefronts on a SIMD, with BACK 174 and two.  24 x 512 tokens, 32 heads of 32: 70 us, 81 with BACK; 16 x 1024, 48 heads of 16: 114, 154; in
-    // segments 1 x 1000, 12 heads of 32: 30.1, 28.9).
-    constexpr bool BACK = CHANNEL && HALVES == 1 && (DT == 2 || FOLD);
-    f32x4 diag = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (CHANNEL && !STATE_ONLY) {
-      const int rel = l16 - quad * 4;  // row i is j tokens back where rel = j + i
-      float sum = 0.f, four[4];
-#pragma unroll
-      for (int g = 0; g < 2 * DT; ++g) {
-        const int ch = chan(g >> 1, g & 1) < a.d ? chan(g >> 1, g & 1) : 0;
-        const bf16x4 u = *reinterpret_cast<const bf16x4*>(static_cast<const __bf16*>(a.u) + (long)h * a.d + ch);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sum = __builtin_fmaf(q[g * 4 + j] * to_f32(u[j]), k[g * 4 + j], sum);
-      }
-      four[0] = sum;
-      if constexpr (!BACK) {
-        sum = quad_rows_sum(sum);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) diag[i] = rel == i ? sum : diag[i];
-      }
-      float x[E], before[E];
-#pragma unroll
-      for (int i = 0; i < E; ++i) {
-        x[i] = row_moved<0x111>(k[i]);
-        before[i] = row_moved<0x111>(w[i]);  // of the token before
-      }
-      constexpr int kUnroll = BACK ? 15 : 3;  // (few steps in flight: registers are scarce)
-#pragma unroll kUnroll
-      for (int j = 1; j < 16; ++j) {
-        sum = 0.f;
-#pragma unroll
-        for (int i = 0; i < E; ++i) {
-          sum = __builtin_fmaf(q[i], x[i], sum);
-          x[i] = row_moved<0x111>(x[i]) * before[i];
-        }
-        if constexpr (BACK) {
-          four[j % 4] = sum;
-          if (j % 4 == 3) {
-            sum = sum_quads4(four[0], four[1], four[2], four[3]);
-            diag[j / 4] = j - 3 + quad <= l16 ? sum : 0.f;
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        } else {
-          sum = quad_rows_sum(sum);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) diag[i] = rel == j + i ? sum : diag[i];
-        }
       }
     }
 
@@ -371,38 +806,12 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
         for (int j = 0; j < 2; ++j) vv[f * 2 + j] = in ? pack_bf16(v[f * 4 + 2 * j], v[f * 4 + 2 * j + 1]) ^ odd_sign : 0u;
       }
     }
-    if (!LATE && chunk + 1 < last) fetch(cur, chunk + 1);
+    if (chunk + 1 < last) fetch(cur, chunk + 1);
     lds_barrier();  // every wavefront is done with the 64 tokens before
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       store_pair(&lds.vt[(half * 64 + quad * 16 + 2 * j) * TS + t], &lds.vt[(half * 64 + quad * 16 + 2 * j + 1) * TS + t], vv[j]);
-    if constexpr (CHANNEL) {
-      if constexpr (HALVES > 1) __builtin_amdgcn_sched_barrier(0);
-      // q decayed from the start of these 16 tokens, k to their end
-      if constexpr (!STATE_ONLY) {
-        float prefix[E];
-#pragma unroll
-        for (int i = 0; i < E; ++i) prefix[i] = w[i];
-#pragma unroll
-        for (int i = 0; i < E; i += 4) row_prefix4(prefix + i, q + i);
-      }
-#pragma unroll
-      for (int i = 0; i < E; i += 4) row_suffix4(w + i, k + i);
-      // (the product over all 16 is lane 0's suffix)
-      if (l16 == 0) {
-#pragma unroll
-        for (int i = 0; i < E; i += 4) *reinterpret_cast<f32x4*>(&lds.total[blk][chan_of(i)]) = f32x4{w[i], w[i + 1], w[i + 2], w[i + 3]};
-      }
-      if constexpr (!STATE_ONLY) {
-#pragma unroll
-        for (int c = 0; c < DT; ++c) {
-          bf16x8 hi, lo;
-          split8(k + c * 8, hi, lo);
-          *reinterpret_cast<bf16x8*>(&lds.k.hi[t * RS + ch0 + c * 32 + quad * 8]) = hi;
-          *reinterpret_cast<bf16x8*>(&lds.k.lo[t * RS + ch0 + c * 32 + quad * 8]) = lo;
-        }
-      }
-    } else {
+    {
       const float f = powers(n - 1 - t > 0 ? n - 1 - t : 0);
 #pragma unroll
       for (int i = 0; i < E; i += 2) {
@@ -420,88 +829,23 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
             q4[e] = pack_bf16(q[c * 8 + 2 * e], q[c * 8 + 2 * e + 1]);
             k4[e] = pack_bf16(k[c * 8 + 2 * e], k[c * 8 + 2 * e + 1]);
           }
-          *reinterpret_cast<u32x4*>(&lds.k.hi[t * RS + ch0 + c * 32 + quad * 8]) = k4;
-          *reinterpret_cast<u32x4*>(&lds.q_hi[t * RS + ch0 + c * 32 + quad * 8]) = q4;
+          *reinterpret_cast<u32x4*>(&lds.k[t * RS + ch0 + c * 32 + quad * 8]) = k4;
+          *reinterpret_cast<u32x4*>(&lds.q[t * RS + ch0 + c * 32 + quad * 8]) = q4;
         }
       }
     }
     lds_barrier();
 
-    if constexpr (CHANNEL) {
-      const int ch = threadIdx.x;
-      if (ch < Lds::CH) {
-        const float all = (lds.total[0][ch] * lds.total[1][ch]) * (lds.total[2][ch] * lds.total[3][ch]);
-        lds.all[ch] = all;
-        if constexpr (STATE_ONLY) seg_total *= all;
-      }
-    }
     f32x4 P[STATE_ONLY ? 1 : 4];  // P^T tiles: column t of this wavefront's 16 tokens, rows s of 16 tokens j
-    if constexpr (CHANNEL) {
-#pragma unroll
-      for (int i = 0; i < E; i += 4) {
-        f32x4 x = {k[i], k[i + 1], k[i + 2], k[i + 3]};
-#pragma unroll
-        for (int m = 1; m < 4; ++m)  // the 16-token groups behind this one
-          if (m > blk) x *= *reinterpret_cast<const f32x4*>(&lds.total[m][chan_of(i)]);
-#pragma unroll
-        for (int e = 0; e < 4; e += 2) {
-          const int ch = chan_of(i) + e;
-          uint32_t hi, lo;
-          split2(x[e], x[e + 1], hi, lo);
-          store_pair(&lds.kt_hi[ch * TS + t], &lds.kt_hi[(ch + 1) * TS + t], hi);
-          store_pair(&lds.kt_lo[ch * TS + t], &lds.kt_lo[(ch + 1) * TS + t], lo);
-        }
-      }
-      if constexpr (!STATE_ONLY) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) P[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        // q scaled to the start of its own 16 tokens, then by the groups in between, nearest first
-#pragma unroll
-        for (int step = 1; step <= 4; ++step) {
-          __builtin_amdgcn_sched_barrier(0);
-          const int j = blk - step;  // the last round scales to the start of the 64 tokens
-          if (j < -1) break;
-          bf16x8 hi[DT], lo[DT];
-#pragma unroll
-          for (int c = 0; c < DT; ++c) split8(q + c * 8, hi[c], lo[c]);
-          if (j >= 0) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int c = 0; c < DT; ++c) {
-              const bf16x8 kh = *reinterpret_cast<const bf16x8*>(&lds.k.hi[(j * 16 + l16) * RS + ch0 + c * 32 + quad * 8]);
-              const bf16x8 kl = *reinterpret_cast<const bf16x8*>(&lds.k.lo[(j * 16 + l16) * RS + ch0 + c * 32 + quad * 8]);
-              acc = mfma_16(kh, hi[c], acc);
-              acc = mfma_16(kl, hi[c], acc);
-              acc = mfma_16(kh, lo[c], acc);
-            }
-#pragma unroll
-            for (int m = 0; m < 3; ++m) P[m] = m == j ? acc : P[m];
-#pragma unroll
-            for (int i = 0; i < E; i += 4) {
-              const f32x4 f = *reinterpret_cast<const f32x4*>(&lds.total[j][chan_of(i)]);
-#pragma unroll
-              for (int e = 0; e < 4; ++e) q[i + e] *= f[e];
-            }
-          } else {
-#pragma unroll
-            for (int c = 0; c < DT; ++c) {
-              *reinterpret_cast<bf16x8*>(&lds.q_hi[t * RS + ch0 + c * 32 + quad * 8]) = hi[c];
-              *reinterpret_cast<bf16x8*>(&lds.q_lo[t * RS + ch0 + c * 32 + quad * 8]) = lo[c];
-            }
-          }
-        }
-#pragma unroll
-        for (int m = 0; m < 4; ++m) P[m] = m == blk ? diag : P[m];
-      }
-    } else if constexpr (!STATE_ONLY) {
+    if constexpr (!STATE_ONLY) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         P[j] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (j > blk) continue;
 #pragma unroll
         for (int c = 0; c < DT; ++c) {
-          const bf16x8 k8 = *reinterpret_cast<const bf16x8*>(&lds.k.hi[(j * 16 + l16) * RS + ch0 + c * 32 + quad * 8]);
-          const bf16x8 q8 = *reinterpret_cast<const bf16x8*>(&lds.q_hi[t * RS + ch0 + c * 32 + quad * 8]);
+          const bf16x8 k8 = *reinterpret_cast<const bf16x8*>(&lds.k[(j * 16 + l16) * RS + ch0 + c * 32 + quad * 8]);
+          const bf16x8 q8 = *reinterpret_cast<const bf16x8*>(&lds.q[t * RS + ch0 + c * 32 + quad * 8]);
           P[j] = mfma_16(k8, q8, P[j]);
         }
 #pragma unroll
@@ -534,36 +878,26 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
           split2(P[j][2 * i], P[j][2 * i + 1], x, y);
           hi[i] = x, lo[i] = y;
         }
-        if (BACK && j == blk) {  // as diag has them
-#pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            const int s0 = t * TS + j * 16 + ((l16 - 8 * i - quad) & 15), s1 = t * TS + j * 16 + ((l16 - 8 * i - 4 - quad) & 15);
-            store_pair(&lds.p.hi[s0], &lds.p.hi[s1], hi[i]);
-            store_pair(&lds.p.lo[s0], &lds.p.lo[s1], lo[i]);
-          }
-        } else if (half == 0 && j <= (blk | 1)) {
+        if (half == 0 && j <= (blk | 1)) {
           *reinterpret_cast<u32x2*>(&lds.p.hi[t * TS + j * 16 + quad * 4]) = hi;
           *reinterpret_cast<u32x2*>(&lds.p.lo[t * TS + j * 16 + quad * 4]) = lo;
         }
       }
       lds_barrier();
     }
-    if (LATE && chunk + 1 < last) fetch(cur, chunk + 1);
     if (has_cols) {
       bf16x8 v8[2];
 #pragma unroll
       for (int g = 0; g < 2; ++g) v8[g] = *reinterpret_cast<const bf16x8*>(&lds.vt[(wave * 16 + l16) * TS + g * 32 + quad * 8]);
       if constexpr (!STATE_ONLY) {
-        if constexpr (!CHANNEL) {
-          if (chunk == first && powers.w < 0.f) turn_state(true);  // (no sooner: the state is on its way until here)
-        }
+        if (chunk == first && powers.w < 0.f) turn_state(true);  // (no sooner: the state is on its way until here)
         bf16x8 sh[DA], sl[DA];
 #pragma unroll
         for (int c = 0; c < DA; ++c) {
           const float x[8] = {S[2 * c][0], S[2 * c][1], S[2 * c][2], S[2 * c][3], S[2 * c + 1][0], S[2 * c + 1][1], S[2 * c + 1][2], S[2 * c + 1][3]};
           split8(x, sh[c], sl[c]);
         }
-        if constexpr (!CHANNEL) {  // (rounding leaves nothing of an infinity: the difference of two is no number)
+        {  // (rounding leaves nothing of an infinity: the difference of two is no number)
           float most = 0.f;
 #pragma unroll
           for (int ct = 0; ct < 2 * DA; ++ct)
@@ -583,15 +917,11 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
           f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int c = 0; c < DA; ++c) {
-            const bf16x8 qh = *reinterpret_cast<const bf16x8*>(&lds.q_hi[tok * RS + c * 32 + quad * 8]);
+            const bf16x8 qh = *reinterpret_cast<const bf16x8*>(&lds.q[tok * RS + c * 32 + quad * 8]);
             acc = mfma_16(sh[c], qh, acc);
             acc = mfma_16(sl[c], qh, acc);
-            if constexpr (CHANNEL) {
-              const bf16x8 ql = *reinterpret_cast<const bf16x8*>(&lds.q_lo[tok * RS + c * 32 + quad * 8]);
-              acc = mfma_16(sh[c], ql, acc);
-            }
           }
-          if constexpr (!CHANNEL) acc *= powers.of_state(tok + 1);
+          acc *= powers.of_state(tok + 1);
 #pragma unroll
           for (int g = 0; g < 2; ++g) {
             if (g * 2 > tb) continue;
@@ -612,11 +942,7 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
 #pragma unroll
       for (int ct = 0; ct < 2 * DA; ++ct) {
         if (HALVES > 1 && ct % 2 == 0) __builtin_amdgcn_sched_barrier(0);
-        if constexpr (CHANNEL) {
-          S[ct] *= *reinterpret_cast<const f32x4*>(&lds.all[ct * 16 + quad * 4]);
-        } else {
-          S[ct] *= powers.of_state(n);
-        }
+        S[ct] *= powers.of_state(n);
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
           const bf16x8 kh = *reinterpret_cast<const bf16x8*>(&lds.kt_hi[(ct * 16 + l16) * TS + g * 32 + quad * 8]);
@@ -627,11 +953,8 @@ __global__ __launch_bounds__(256 * HALVES, 2) void decay_scan_mfma_kernel(const 
       }
     }
   }
-  if constexpr (CHANNEL && STATE_ONLY) {
-    if (blockIdx.y == 0 && threadIdx.x < a.d) a.seg_lw[(bh * a.segs + sg) * a.dp + threadIdx.x] = seg_total;
-  }
   if (!has_cols) return;
-  if constexpr (!CHANNEL) turn_state(powers.w < 0.f && !(last == chunks && (a.L & 1)));  // (of an odd number of tokens the signs are turned already)
+  turn_state(powers.w < 0.f && !(last == chunks && (a.L & 1)));  // (of an odd number of tokens the signs are turned already)
   float* to = st;
   if constexpr (STATE_ONLY) to = a.seg + ((bh * a.segs + sg) * a.dv + (col_in ? dv0 + l16 : 0)) * a.dp;
   if (STATE_ONLY || sg == a.segs - 1) {
@@ -1019,34 +1342,65 @@ void launch_decay_join(const DecayScanArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(decay_join_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, a);
 }
 
-template <int DT, int HALVES, bool CHANNEL, bool FOLD> int launch_decay_mfma(const DecayScanArgs& a, hipStream_t s) {
-  const size_t bytes = sizeof(ScanLds<DT, HALVES, CHANNEL>);
-  if (bytes > 64 * 1024) {
-    static const hipError_t once = [&] {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(decay_scan_mfma_kernel<DT, HALVES, CHANNEL, false, FOLD>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-      if (e != hipSuccess) return e;
-      return hipFuncSetAttribute(reinterpret_cast<const void*>(decay_scan_mfma_kernel<DT, HALVES, CHANNEL, true, FOLD>),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    }();
-    BASED_REQUIRE(once == hipSuccess, BASED_ERR_LAUNCH, "decay_scan: %zu bytes of LDS refused: %s", bytes, hipGetErrorString(once));
-  }
-  const int cols = 64 * HALVES;
-  dim3 grid((unsigned)(a.B * a.H), (unsigned)((a.dv + cols - 1) / cols), (unsigned)a.segs);
-  if (a.segs > 1) {
-    dim3 all_but_last = grid;
-    all_but_last.z -= 1;
-    hipLaunchKernelGGL((decay_scan_mfma_kernel<DT, HALVES, CHANNEL, true, FOLD>), all_but_last, dim3(256 * HALVES), bytes, s, a);
-    if (!FOLD) launch_decay_join(a, s);
-  }
-  hipLaunchKernelGGL((decay_scan_mfma_kernel<DT, HALVES, CHANNEL, false, FOLD>), grid, dim3(256 * HALVES), bytes, s, a);
+template <typename Kernel> int allow_lds(Kernel kernel, size_t bytes) {
+  if (bytes <= 64 * 1024) return BASED_OK;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  BASED_REQUIRE(e == hipSuccess, BASED_ERR_LAUNCH, "decay_scan: %zu bytes of LDS refused: %s", bytes, hipGetErrorString(e));
   return BASED_OK;
 }
 
-template <bool CHANNEL> int launch_decay_scan_mfma(const DecayScanArgs& a, bool fold, hipStream_t s) {
-  if (a.d <= 32) return fold ? launch_decay_mfma<1, 1, CHANNEL, true>(a, s) : launch_decay_mfma<1, 1, CHANNEL, false>(a, s);
-  if (a.d <= 64) return fold ? launch_decay_mfma<2, 1, CHANNEL, true>(a, s) : launch_decay_mfma<2, 1, CHANNEL, false>(a, s);
-  return launch_decay_mfma<2, 2, CHANNEL, false>(a, s);
+template <int DT, int HALVES, int COLS, bool CHANNEL, bool FOLD> int launch_decay_mfma(const DecayScanArgs& a, hipStream_t s) {
+  void (*scan)(DecayScanArgs);
+  void (*states)(DecayScanArgs);
+  size_t bytes, state_bytes;
+  if constexpr (CHANNEL) {
+    typedef ChannelLds<DT, HALVES, COLS> Lds;
+    scan = decay_channel_kernel<DT, HALVES, COLS, false, FOLD>, states = decay_channel_kernel<DT, HALVES, COLS, true, FOLD>;
+    bytes = sizeof(Lds), state_bytes = offsetof(Lds, u);
+  } else {
+    static_assert(COLS == 64 * HALVES, "a wavefront has 16 value channels");
+    scan = decay_head_kernel<DT, HALVES, false, FOLD>, states = decay_head_kernel<DT, HALVES, true, FOLD>;
+    bytes = state_bytes = sizeof(HeadLds<DT, HALVES>);
+  }
+  static const int allowed = [&] {
+    const int rc = allow_lds(scan, bytes);
+    return rc != BASED_OK ? rc : allow_lds(states, state_bytes);
+  }();
+  if (allowed != BASED_OK) return allowed;
+  dim3 grid((unsigned)(a.B * a.H), (unsigned)((a.dv + COLS - 1) / COLS), (unsigned)a.segs);
+  if (a.segs > 1) {
+    dim3 all_but_last = grid;
+    all_but_last.z -= 1;
+    hipLaunchKernelGGL(states, all_but_last, dim3(256 * HALVES), state_bytes, s, a);
+    if (!FOLD) launch_decay_join(a, s);
+  }
+  hipLaunchKernelGGL(scan, grid, dim3(256 * HALVES), bytes, s, a);
+  return BASED_OK;
+}
+
+// Channel decays.  Up to 64 channels: two wavefronts to the same 16 tokens, half of the channels each, where a SIMD would otherwise have fewer than
+// two; beyond that one, which adds nothing up across wavefronts.
+static bool channel_split(int64_t B, int64_t H, int64_t DV, int64_t segs, int64_t seg_chunks) {
+  return B * H * ((DV + 63) / 64) * segs <= 384 || seg_chunks == 1;
+}
+// More channels: workgroups of 64 value channels where the 98 KB of each find a compute unit of their own, of 128 beyond that.
+static bool channel_narrow(int64_t B, int64_t H, int64_t DV) { return B * H * ((DV + 63) / 64) <= 256; }
+
+int launch_decay_head(const DecayScanArgs& a, bool fold, hipStream_t s) {
+  if (a.d <= 32) return fold ? launch_decay_mfma<1, 1, 64, false, true>(a, s) : launch_decay_mfma<1, 1, 64, false, false>(a, s);
+  if (a.d <= 64) return fold ? launch_decay_mfma<2, 1, 64, false, true>(a, s) : launch_decay_mfma<2, 1, 64, false, false>(a, s);
+  return launch_decay_mfma<2, 2, 128, false, false>(a, s);
+}
+
+int launch_decay_channel(const DecayScanArgs& a, bool fold, hipStream_t s) {
+  if (a.d <= 32) return fold ? launch_decay_mfma<1, 1, 64, true, true>(a, s) : launch_decay_mfma<1, 1, 64, true, false>(a, s);
+  if (a.d <= 64) {
+    if (channel_split(a.B, a.H, a.dv, a.segs, a.seg_chunks))
+      return fold ? launch_decay_mfma<1, 2, 64, true, true>(a, s) : launch_decay_mfma<1, 2, 64, true, false>(a, s);
+    return fold ? launch_decay_mfma<2, 1, 64, true, true>(a, s) : launch_decay_mfma<2, 1, 64, true, false>(a, s);
+  }
+  if (channel_narrow(a.B, a.H, a.dv)) return fold ? launch_decay_mfma<2, 2, 64, true, true>(a, s) : launch_decay_mfma<2, 2, 64, true, false>(a, s);
+  return launch_decay_mfma<2, 2, 128, true, false>(a, s);
 }
 
 template <typename T, int CPT, bool CHANNEL, int TOKENS> void launch_decay_any_tile(const DecayScanArgs& a, hipStream_t s) {
@@ -1123,6 +1477,28 @@ static int decay_segments(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV
   return segs < 2 ? 1 : (int)segs;
 }
 
+// Those of a call that has work space by the rule of channel decays.  A piece of 64 tokens takes the scan about 4.5 us and the state pass 2, a launch
+// and the folding of some segments 3: pieces by themselves pay from four of them on (2 x 440 tokens, 12 heads of 64, us in segments of 1, 2 and
+// 4 pieces or in one: 16.2, 24.8, 34.9 (7 pieces); 5 x 320, 16 heads: 20.4, 25.1, 26.3), as long as the segments need no launch of their own to be put
+// together or are of four pieces anyway (1 x 4096, 16 heads: 42.6 in 16 of four, 47.9 in 32 of two).  Not where there are workgroups for
+// every compute unit without them: every token but those of the last segment is walked twice (30 x 513, 16 heads: 70.4, in two 83.0).
+static int decay_channel_segments(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
+  if (L < BASED_DECAY_SEGMENTS_MIN) return 1;
+  const int64_t chunks = (L + kScanTokens - 1) / kScanTokens;
+  int64_t segs, most = chunks;
+  if (D <= 64) {
+    const int64_t wgs = B * H * ((DV + 63) / 64);
+    segs = wgs <= 256 ? 768 / wgs : 1;
+    most = chunks / 4 > kFoldSegmentsChannel ? chunks / 4 : kFoldSegmentsChannel;
+  } else {  // (one workgroup to a compute unit.  1 x 2000, 8 heads of 128: 41.9 in 16 of two pieces, 55 in eight of four)
+    segs = 256 / (B * H * (channel_narrow(B, H, DV) ? (DV + 63) / 64 : (DV + 127) / 128));
+  }
+  if (segs > most) segs = most;
+  if (segs > chunks) segs = chunks;
+  if (segs > 64) segs = 64;
+  return segs < 2 ? 1 : (int)segs;
+}
+
 // The same for the general form: eight workgroups to a compute unit.  Every token but those of the last segment is walked twice, so the
 // chain is two segments long: three segments ask for a third less at best, and the launches.  Segments where four are wanted, of which
 // whole 64-token pieces may leave three, if the two are the shorter chain by more than the launches.  us in segments against one chain,
@@ -1163,11 +1539,11 @@ extern "C" BASED_API int64_t based_decay_scan_work_of(int64_t bits, int64_t B, i
   return decay_work(decay_vec(bits, D, DV, io_dtype) ? decay_segments(B, L, H, D, DV) : decay_any_segments(B, L, H, DV), B, H, DV, state_row);
 }
 
-extern "C" BASED_API int based_decay_scan(const void* q, const void* k, const void* v, const float* channel_log2, const float* head_decay,
-                                          const void* bonus, float* state, float* work, void* o, int64_t B, int64_t L, int64_t H,
-                                          int64_t D, int64_t DV, int64_t state_row, int64_t q_sb, int64_t q_sl, int64_t k_sb,
-                                          int64_t k_sl, int64_t v_sb, int64_t v_sl, int64_t o_sb, int64_t o_sl, int activation, int fresh,
-                                          int io_dtype, void* stream) {
+// by_channel: the work space is of based_decay_scan_channels_work
+static int decay_scan_call(bool by_channel, const void* q, const void* k, const void* v, const float* channel_log2, const float* head_decay,
+                           const void* bonus, float* state, float* work, void* o, int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV,
+                           int64_t state_row, int64_t q_sb, int64_t q_sl, int64_t k_sb, int64_t k_sl, int64_t v_sb, int64_t v_sl, int64_t o_sb,
+                           int64_t o_sl, int activation, int fresh, int io_dtype, void* stream) {
   using namespace based;
   BASED_REQUIRE(q && k && v && state && o, BASED_ERR_ARG, "decay_scan: null pointer argument");
   BASED_REQUIRE((channel_log2 != nullptr) != (head_decay != nullptr), BASED_ERR_ARG, "decay_scan: decays per channel or per head");
@@ -1183,13 +1559,13 @@ extern "C" BASED_API int based_decay_scan(const void* q, const void* k, const vo
   if (B == 0 || L == 0) return BASED_OK;
   DecayScanArgs a{q,    k,    v,    channel_log2, head_decay, bonus, state, nullptr, nullptr, o,    (int)B, (int)L, (int)H, (int)D, (int)DV,
                   (int)state_row, q_sb, q_sl, k_sb, k_sl, v_sb, v_sl, o_sb, o_sl, 1, (int)((L + kScanTokens - 1) / kScanTokens),
-                  activation == BASED_ACT_SILU, fresh};
+                  activation == BASED_ACT_SILU, fresh, 0};
   hipStream_t s = static_cast<hipStream_t>(stream);
   const auto at = [](const void* p) { return (int64_t)reinterpret_cast<uintptr_t>(p); };
   const int64_t strides = q_sb | q_sl | k_sb | k_sl | v_sb | v_sl | o_sb | o_sl;
   const int64_t bits = at(q) | at(k) | at(v) | at(bonus) | at(o) | 2 * strides | at(channel_log2) / 2;
   const bool vec = decay_vec(bits, D, DV, io_dtype);
-  const int segs = vec ? decay_segments(B, L, H, D, DV) : work != nullptr ? decay_any_segments(B, L, H, DV) : 1;
+  const int segs = vec ? (by_channel ? decay_channel_segments : decay_segments)(B, L, H, D, DV) : work != nullptr ? decay_any_segments(B, L, H, DV) : 1;
   if (segs > 1) {
     BASED_REQUIRE(work != nullptr, BASED_ERR_ARG, "decay_scan: no work space");
     a.seg_chunks = (a.seg_chunks + segs - 1) / segs;
@@ -1197,9 +1573,10 @@ extern "C" BASED_API int based_decay_scan(const void* q, const void* k, const vo
     a.seg = work;
     a.seg_lw = work + B * H * a.segs * DV * state_row;
   }
-  const bool fold = vec && D <= 64 && a.segs > 1 && a.segs <= (channel_log2 != nullptr ? kFoldSegmentsChannel : kFoldSegmentsHead);
+  const bool fold = vec && (D <= 64 || (channel_log2 != nullptr && channel_narrow(B, H, DV))) && a.segs > 1 && a.segs <= (channel_log2 != nullptr ? kFoldSegmentsChannel : kFoldSegmentsHead);
+  a.wide = bits % 16 == 0 && D % 8 == 0 && DV % 8 == 0;
   if (vec) {
-    const int rc = channel_log2 != nullptr ? launch_decay_scan_mfma<true>(a, fold, s) : launch_decay_scan_mfma<false>(a, fold, s);
+    const int rc = channel_log2 != nullptr ? launch_decay_channel(a, fold, s) : launch_decay_head(a, fold, s);
     if (rc != BASED_OK) return rc;
   } else if (io_dtype == BASED_BF16) {
     channel_log2 != nullptr ? launch_decay_scan_any<__bf16, true>(a, s) : launch_decay_scan_any<__bf16, false>(a, s);
@@ -1207,6 +1584,31 @@ extern "C" BASED_API int based_decay_scan(const void* q, const void* k, const vo
     channel_log2 != nullptr ? launch_decay_scan_any<float, true>(a, s) : launch_decay_scan_any<float, false>(a, s);
   }
   return check_launch("decay_scan");
+}
+
+extern "C" BASED_API int based_decay_scan(const void* q, const void* k, const void* v, const float* channel_log2, const float* head_decay,
+                                          const void* bonus, float* state, float* work, void* o, int64_t B, int64_t L, int64_t H,
+                                          int64_t D, int64_t DV, int64_t state_row, int64_t q_sb, int64_t q_sl, int64_t k_sb,
+                                          int64_t k_sl, int64_t v_sb, int64_t v_sl, int64_t o_sb, int64_t o_sl, int activation, int fresh,
+                                          int io_dtype, void* stream) {
+  return decay_scan_call(false, q, k, v, channel_log2, head_decay, bonus, state, work, o, B, L, H, D, DV, state_row, q_sb, q_sl, k_sb, k_sl, v_sb,
+                         v_sl, o_sb, o_sl, activation, fresh, io_dtype, stream);
+}
+
+extern "C" BASED_API int64_t based_decay_scan_channels_work(int64_t bits, int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV,
+                                                            int64_t state_row, int io_dtype) {
+  using namespace based;
+  if (B <= 0 || L < BASED_DECAY_SEGMENTS_MIN || H <= 0 || D <= 0 || DV <= 0) return 0;
+  return decay_work(decay_vec(bits, D, DV, io_dtype) ? decay_channel_segments(B, L, H, D, DV) : decay_any_segments(B, L, H, DV), B, H, DV, state_row);
+}
+
+extern "C" BASED_API int based_decay_scan_channels(const void* q, const void* k, const void* v, const float* channel_log2, const void* bonus,
+                                                   float* state, float* work, void* o, int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV,
+                                                   int64_t state_row, int64_t q_sb, int64_t q_sl, int64_t k_sb, int64_t k_sl, int64_t v_sb,
+                                                   int64_t v_sl, int64_t o_sb, int64_t o_sl, int activation, int fresh, int io_dtype,
+                                                   void* stream) {
+  return decay_scan_call(true, q, k, v, channel_log2, nullptr, bonus, state, work, o, B, L, H, D, DV, state_row, q_sb, q_sl, k_sb, k_sl, v_sb, v_sl,
+                         o_sb, o_sl, activation, fresh, io_dtype, stream);
 }
 
 extern "C" BASED_API int based_decay_step(const void* q, const void* k, const void* v, const float* head_decay, const void* bonus,

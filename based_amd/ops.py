@@ -1342,15 +1342,17 @@ def decay_scan(q, k, v, state, heads: int, *, channel_log2=None, bonus=None, hea
     lib = _lib.lib()
     o = torch.empty(B, L, heads * dv, dtype=q.dtype, device=q.device)
     at = [q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(channel_log2), _ptr(bonus), o.data_ptr()]
-    work = None
+    work, by_channel = None, channel_log2 is not None and head_decay is None
     if L >= DECAY_SEGMENTS_MIN:
         bits = at[0] | at[1] | at[2] | (at[4] or 0) | at[5] | (at[3] or 0) >> 1 | stride_bits
-        n = lib.based_decay_scan_work_of(bits, *sizes, code)
+        n = (lib.based_decay_scan_channels_work if by_channel else lib.based_decay_scan_work_of)(bits, *sizes, code)
         work = torch.empty(n, dtype=torch.float32, device=q.device) if n else None
     with _on_device(q.device):
-        _lib.check(lib.based_decay_scan(
-            *at[:4], _ptr(head_decay), at[4], state.data_ptr(), _ptr(work), at[5], *sizes, *strides, int(activation), int(fresh),
-            code, _stream_ptr(q)))
+        tail = (state.data_ptr(), _ptr(work), at[5], *sizes, *strides, int(activation), int(fresh), code, _stream_ptr(q))
+        if by_channel:
+            _lib.check(lib.based_decay_scan_channels(*at[:5], *tail))
+        else:
+            _lib.check(lib.based_decay_scan(*at[:4], _ptr(head_decay), at[4], *tail))
     return o
 
 

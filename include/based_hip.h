@@ -658,6 +658,14 @@ BASED_API int based_decay_scan(const void* q, const void* k, const void* v, cons
                                int64_t k_sl, int64_t v_sb, int64_t v_sl, int64_t o_sb, int64_t o_sl, int activation,
                                int fresh, int io_dtype, void* stream);
 
+/* The same over channel decays alone, with work space as based_decay_scan_channels_work says (bits as above): short prompts of few heads come in
+ * segments there, which take some. */
+BASED_API int64_t based_decay_scan_channels_work(int64_t bits, int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, int64_t state_row, int io_dtype);
+BASED_API int based_decay_scan_channels(const void* q, const void* k, const void* v, const float* channel_log2, const void* bonus, float* state,
+                                        float* work, void* o, int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV, int64_t state_row,
+                                        int64_t q_sb, int64_t q_sl, int64_t k_sb, int64_t k_sl, int64_t v_sb, int64_t v_sl, int64_t o_sb,
+                                        int64_t o_sl, int activation, int fresh, int io_dtype, void* stream);
+
 /* One token of it.  With `hidden` (B, R), w2, w0 as in based_channel_decay the channel form, its output divided by its
  * RMS per head, times norm_w (H, DV) and silu(gate) (B, H * DV); otherwise the head form, its output as it is. */
 BASED_API int based_decay_step(const void* q, const void* k, const void* v, const float* head_decay, const void* bonus,

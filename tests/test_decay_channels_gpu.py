@@ -1,0 +1,62 @@
+"""Channel decays over prompts in bf16, against the recurrence in 64 bits: every split of heads and channels over wavefronts, at the edges of pieces of
+64 tokens, of segments, and of rows in whole 16-byte pieces or not."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+CASES = [(2, 70, 3, 20, 12),        # up to 32 channels
+         (1, 1, 1, 64, 64), (2, 16, 2, 64, 64), (1, 17, 3, 64, 64), (3, 128, 2, 64, 64),  # one piece and two, two wavefronts to the same tokens
+         (2, 130, 5, 44, 36),       # rows of 8-byte pieces
+         (2, 65, 3, 64, 72),        # value channels of two workgroups
+         (30, 129, 14, 64, 64), (30, 66, 14, 60, 44),  # many heads: one wavefront
+         (1, 193, 2, 64, 64), (3, 704, 2, 64, 64), (1, 705, 1, 52, 20), (65, 260, 6, 64, 64),  # segments: four of a piece, ten and more, none
+         (2, 133, 2, 128, 128), (1, 64, 3, 96, 68), (2, 700, 2, 128, 64), (1, 1100, 1, 72, 128),  # workgroups of 64 value channels
+         (33, 66, 4, 128, 128), (34, 130, 4, 100, 132)]  # of 128
+
+
+@pytest.mark.parametrize("silu", [False, True])
+@pytest.mark.parametrize("fresh", [True, False])
+@pytest.mark.parametrize("B,L,H,d,dv", CASES)
+def test_channel_decays(dev, B, L, H, d, dv, fresh, silu):
+    from based_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(L * 7 + d + B)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    x = rnd(B, L, H * (2 * d + dv)).bfloat16()
+    q, k, v = x[..., :H * d], x[..., H * d:2 * H * d], x[..., 2 * H * d:]
+    u = rnd(H, d).bfloat16()
+    lw = -torch.exp(rnd(B, L, H * d) + 2 * rnd(H * d) - 3) / math.log(2)
+    dp = (d + 3) // 4 * 4
+    state = rnd(B, H, dv, dp)
+    S = torch.zeros(B, H, d, dv, dtype=torch.float64, device=dev) if fresh else state[..., :d].double().transpose(2, 3)
+    act = ops.ACT_SILU if silu else ops.ACT_NONE
+    out = ops.decay_scan(q, k, v, state, H, channel_log2=lw, bonus=u, activation=act, fresh=fresh)
+    f = lambda t, n: (torch.nn.functional.silu(t.double()).bfloat16() if silu else t).double().view(B, L, H, n)  # noqa: E731
+    qd, kd, vd, w, ref = f(q, d), f(k, d), f(v, dv), 2.0 ** lw.double().view(B, L, H, d), []
+    for t in range(L):
+        kv = kd[:, t, :, :, None] * vd[:, t, :, None]
+        ref.append(((S + u.double()[..., None] * kv) * qd[:, t, :, :, None]).sum(2).flatten(1))
+        S = w[:, t, :, :, None] * S + kv
+    ref = torch.stack(ref, 1)
+    rel = lambda a, b: ((a.double() - b).norm() / b.norm()).item()  # noqa: E731
+    # outputs: half of the 2^-8 of bf16 at most.  Keys enter the state as pairs of bf16 (within 2^-18 of themselves), decayed by products of up to a
+    # few hundred factors of 2^-24 each: 2^-17 together; a silu that falls the other way in bf16 moves one key or value in some thousands by 2^-8.
+    assert rel(out, ref) < 3.9e-3 and rel(out[:, -1:], ref[:, -1:]) < 3.9e-3
+    assert rel(state[..., :d], S.transpose(2, 3)) < (1e-4 if silu else 7.7e-6)
+
+
+def test_work_space_of_channel_decays():
+    """Segments by the rule of channel decays for aligned bf16, those of the general form for everything else; none for short prompts."""
+    from based_amd import _lib
+
+    lib = _lib.lib()
+    floats = lambda segs, B, H, D, DV: B * H * segs * (DV + 1) * D  # noqa: E731
+    for B, L, H, D, segs in [(1, 192, 16, 64, 0), (1, 193, 16, 64, 4), (5, 320, 16, 64, 5), (4, 2048, 16, 64, 10), (1, 4096, 16, 64, 16), (30, 513, 16, 64, 0),
+                             (2, 500, 8, 128, 8), (4, 2048, 8, 128, 4), (16, 1024, 8, 128, 0), (30, 500, 8, 128, 0)]:
+        sizes = (B, L, H, D, D, D)
+        assert lib.based_decay_scan_channels_work(0, *sizes, 0) == floats(segs, B, H, D, D), (B, L, H, D)
+        assert lib.based_decay_scan_channels_work(4, *sizes, 0) == lib.based_decay_scan_work_of(4, *sizes, 0)  # (off 8 bytes)
+        assert lib.based_decay_scan_channels_work(0, *sizes, 1) == lib.based_decay_scan_work_of(0, *sizes, 1)
