@@ -17,6 +17,8 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libbased_hip.so")  # the in-tree build of every kernel
 # Its entry points as Python callables, cheaper to call than through ctypes.
 BINDING_PATH = os.path.join(_HERE, "_binding" + sysconfig.get_config_var("EXT_SUFFIX"))
+# What a call asks of its tensors (csrc/tensors.cpp), likewise.
+TENSORS_PATH = os.path.join(_HERE, "_tensors" + sysconfig.get_config_var("EXT_SUFFIX"))
 # Builds of some of the sources (based_amd.build.build_part) lie beside it; `use_part` selects one
 # where the whole library has not been built.
 _part_path = None
@@ -225,6 +227,26 @@ def _binding(path: str, number: int):
         warnings.warn(f"{path} was built of another include/based_hip.h than the library, calls go through ctypes: python -m based_amd.build")
         return None
     return module.bind
+
+
+def tensor_calls(form, empty):
+    """(form, empty) of csrc/tensors.cpp, which leave to the given two what they do not take; the given two themselves where that is not built, or was
+    built against another torch (with a warning)."""
+    if not os.path.exists(TENSORS_PATH):
+        return form, empty
+    import torch
+
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("_tensors", TENSORS_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_tensors", loader))
+        loader.exec_module(module)
+    except ImportError as e:
+        warnings.warn(f"{TENSORS_PATH} cannot be loaded, tensors are asked from Python: {e}")
+        return form, empty
+    if module.torch_version() != torch.__version__.split("+")[0]:
+        warnings.warn(f"{TENSORS_PATH} was built against torch {module.torch_version()}, tensors are asked from Python: python -m based_amd.build")
+        return form, empty
+    return module.bind(form, empty)
 
 
 class _Entries:

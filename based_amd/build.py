@@ -21,6 +21,7 @@ INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 OBJDIR = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libbased_hip.so")
 BINDING = os.path.join(HERE, "_binding" + sysconfig.get_config_var("EXT_SUFFIX"))
+TENSORS = os.path.join(HERE, "_tensors" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 FLAGS = [
@@ -113,6 +114,30 @@ def _build_binding(out: str = BINDING, number: int | None = None, compiler: str 
     return True
 
 
+def _build_tensors(out: str = TENSORS, compiler: str = "g++") -> bool:
+    """csrc/tensors.cpp, against the torch that is installed.  Without a compiler or the headers there is none, and tensors are asked from Python."""
+    if os.path.exists(out):
+        os.remove(out)
+    tmp = f"{out}.{os.getpid()}.tmp"
+    try:
+        import torch
+        from torch.utils import cpp_extension
+
+        headers = [x for path in cpp_extension.include_paths() for x in ("-isystem", path)]
+        libraries = [x for path in cpp_extension.library_paths()[:1] for x in ("-L", path)]
+        cmd = [compiler, "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+               *headers, "-I", sysconfig.get_paths()["include"], os.path.join(CSRC, "tensors.cpp"), *libraries, "-ltorch_python", "-ltorch_cpu", "-lc10",
+               "-o", tmp]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+    except (OSError, ImportError, AttributeError) as e:
+        r = subprocess.CompletedProcess([], 1, "", str(e))
+    if r.returncode != 0:
+        sys.stderr.write(f"note: tensors are asked from Python:\n{r.stdout}{r.stderr}\n")
+        return False
+    os.replace(tmp, out)
+    return True
+
+
 def build_part(part: str) -> str:
     """Compiles the sources of one part into a library of its own (based_amd/_lib.py: use_part)."""
     from ._lib import part_path
@@ -132,7 +157,9 @@ def build(verbose: bool = False) -> str:
     if not srcs:
         raise RuntimeError("no HIP sources found")
     with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+        tensors = ex.submit(_build_tensors)
         done = list(ex.map(_compile, srcs))
+        tensors.result()
     objs = [o for o, _ in done]
     # what the compiler says each kernel needs (registers, spills, LDS): kept beside the objects; a
     # kernel that spills vector registers is named, because a few spilled registers in a loop have

@@ -73,9 +73,17 @@ class _Checked(dict):
 _CHECKED: dict = _Checked()
 
 
-def _form(*ts):
-    """Everything that the checks look at, of each tensor (or None)."""
+def _form_of(*ts):
     return tuple([None if t is None else (t.shape, t.stride(), t.dtype, t.device) for t in ts])
+
+
+def _empty_of(like, dtype, *sizes):
+    return torch.empty(sizes, dtype=dtype, device=like.device)
+
+
+# _form(*tensors): everything that the checks look at, of each tensor (or None), as a key.  _empty(like, dtype, *sizes): a tensor beside `like`.
+# Native where that is built (csrc/tensors.cpp, which leaves what is no ordinary tensor to these two).
+_form, _empty = _lib.tensor_calls(_form_of, _empty_of)
 
 
 def _require_cuda(*ts: torch.Tensor) -> None:
@@ -91,10 +99,9 @@ def linear_attn_step(q, k, v, kv_state, k_state, eps: float = 1e-12, out: Option
     """One decode step.  q, k: (B, H, 1, 16) raw; v: (B, H, 1, dv); kv_state (B,H,1,dv,273)
     and k_state (B,H,1,1,273) fp32 contiguous, updated in place.  Returns y (B, H, 1, dv)
     (written into `out` when given)."""
-    key = ("lin_step", q.shape, q.stride(), k.shape, k.stride(), v.shape, v.stride(), kv_state.shape, kv_state.stride(),
-           k_state.shape, k_state.stride(), q.dtype, k.dtype, v.dtype, kv_state.dtype, k_state.dtype, q.device,
-           k.device, v.device, kv_state.device, k_state.device)
-    if key not in _CHECKED:
+    key = ("lin_step", _form(q, k, v, kv_state, k_state))
+    plan = _CHECKED.get(key)
+    if plan is None:
         _require_cuda(q, k, v, kv_state, k_state)
         B, H, l, d = q.shape
         assert l == 1, f"q.shape is {tuple(q.shape)} but should be ({B}, {H}, 1, {d})"
@@ -112,23 +119,18 @@ def linear_attn_step(q, k, v, kv_state, k_state, eps: float = 1e-12, out: Option
         for t in (q, k, v):
             if t.stride(-1) != 1:
                 raise ValueError("innermost dimension must be contiguous")
-        _dtype_code(q)
-        _CHECKED[key] = True
-    B, H, _, _ = q.shape
-    dv = v.shape[-1]
+        plan = _CHECKED[key] = (B, H, dv, (q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1)), _dtype_code(q))
+    B, H, dv, at, code = plan
     if out is None:
-        y = torch.empty(B, H, 1, dv, dtype=q.dtype, device=q.device)
+        y, y_at = _empty(q, q.dtype, B, H, 1, dv), (H * dv, dv)
     else:
-        y = out
+        y, y_at = out, (out.stride(0), out.stride(1))
         if tuple(y.shape) != (B, H, 1, dv) or y.dtype != q.dtype or y.device != q.device or y.stride(-1) != 1:
             raise ValueError(f"out must be a ({B}, {H}, 1, {dv}) {q.dtype} tensor on {q.device}")
     with _on_device(q.device):
         _lib.check(_lib.lib().based_linear_attn_step(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), kv_state.data_ptr(), k_state.data_ptr(), y.data_ptr(),
-            B, H, dv,
-            q.stride(0), q.stride(1), k.stride(0), k.stride(1),
-            v.stride(0), v.stride(1), y.stride(0), y.stride(1),
-            float(eps), _dtype_code(q), _stream_ptr(q)))
+            B, H, dv, *at, *y_at, float(eps), code, _stream_ptr(q)))
     return y
 
 
@@ -267,7 +269,7 @@ def swa_prefill(q, k, v, w_left: int = 64, scale: Optional[float] = None, rope=N
     B, L, H, D, name, at, n_pos, rotary, cache_at, code, default_scale = plan
     scale = default_scale if scale is None else float(scale)
     if out is None:
-        o = torch.empty(B, L, H, D, dtype=q.dtype, device=q.device)
+        o = _empty(q, q.dtype, B, L, H, D)
     else:
         o = out
         if tuple(o.shape) != (B, L, H, D) or o.dtype != q.dtype or o.device != q.device or o.stride(-1) != 1:
@@ -396,18 +398,18 @@ def linear_attn_prefill(q, k, v, eps: float = 1e-12, return_state: bool = False,
     if plan is None:
         plan = _CHECKED[key] = _linear_prefill_plan(q, k, v, split)
     B, H, L, dv, at, name, n_seg, ws_bytes, code = plan
-    y = torch.empty(B, L, H, dv, dtype=q.dtype, device=q.device).transpose(1, 2)
+    y = _empty(q, q.dtype, B, L, H, dv).transpose(1, 2)
     kv_state = k_state = None
     if return_state:
-        kv_state = torch.empty(B, H, 1, dv, EXPANDED_DIM, dtype=torch.float32, device=q.device)
-        k_state = torch.empty(B, H, 1, 1, EXPANDED_DIM, dtype=torch.float32, device=q.device)
+        kv_state = _empty(q, torch.float32, B, H, 1, dv, EXPANDED_DIM)
+        k_state = _empty(q, torch.float32, B, H, 1, 1, EXPANDED_DIM)
     run = getattr(_lib.lib(), name)
     args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), y.data_ptr(),
             kv_state.data_ptr() if return_state else None, k_state.data_ptr() if return_state else None, *at, float(eps), code)
     with _on_device(q.device):
         if n_seg > 1:
             # scratch for the per-segment states; torch's caching allocator makes this cheap
-            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
+            ws = _empty(q, torch.uint8, ws_bytes)
             _lib.check(run(*args, n_seg, ws.data_ptr(), ws_bytes, _stream_ptr(q)))
         else:
             _lib.check(run(*args, _stream_ptr(q)))
@@ -473,7 +475,7 @@ def gated_conv_prefill(u, weight, bias=None, state=None, gated: bool = True) -> 
         if tuple(state.shape) != (B, D, K) or not state.is_contiguous():
             raise ValueError(f"state must be a contiguous ({B}, {D}, {K}) tensor, got {tuple(state.shape)}")
         state_code = _dtype_code(state)
-    y = torch.empty(B, L, D, dtype=u.dtype, device=u.device)
+    y = _empty(u, u.dtype, B, L, D)
     fn = _lib.lib().based_gated_conv_prefill if gated else _lib.lib().based_short_conv_prefill
     with _on_device(u.device):
         _lib.check(fn(
@@ -524,10 +526,10 @@ def add_rms_norm(x, residual, weight, eps: float = 1e-5, residual_in_fp32: bool 
     """Prenorm block glue in one launch: r = x + residual (r = x when residual is None),
     y = rms_norm(r cast to x.dtype) * weight, and r itself (fp32 when residual_in_fp32, else
     x.dtype).  x: (..., D) with contiguous rows; returns (y, r) with r None if not wanted."""
-    D = x.shape[-1]
-    key = ("add_rms_norm", x.shape, x.stride(), x.dtype, x.device, weight.shape, weight.dtype, weight.device,
-           None if residual is None else (residual.shape, residual.stride(), residual.dtype, residual.device))
-    if key not in _CHECKED:
+    key = ("add_rms_norm", _form(x, weight, residual))
+    plan = _CHECKED.get(key)
+    if plan is None:
+        D = x.shape[-1]
         _require_cuda(x, weight)
         if weight.shape != (D,) or weight.dtype != x.dtype or not weight.is_contiguous():
             raise ValueError(f"weight must be a contiguous ({D},) of {x.dtype}, got {tuple(weight.shape)} {weight.dtype}")
@@ -539,32 +541,30 @@ def add_rms_norm(x, residual, weight, eps: float = 1e-5, residual_in_fp32: bool 
                 raise ValueError("fp32 activations need an fp32 residual stream")
             if residual.dtype not in (torch.float32, torch.bfloat16):
                 raise ValueError(f"unsupported residual dtype {residual.dtype}")
-        _dtype_code(x)
-        _CHECKED[key] = True
-    x2 = x if x.dim() == 2 else x.reshape(-1, D)
-    if x2.stride(-1) != 1:
-        x2 = x2.contiguous()
-    rows = x2.shape[0]
-    res_dtype = torch.float32 if residual_in_fp32 else x.dtype
-    r2 = None
-    if residual is not None:
-        # a residual stream of another dtype (first block with residual_in_fp32=False, ...) keeps its own
-        res_dtype = residual.dtype
-        r2 = residual if residual.dim() == 2 else residual.reshape(-1, D)
-        if r2.stride(-1) != 1:
-            r2 = r2.contiguous()
+        rows = x.numel() // D if D else 0
+        # (rows one behind the other, as a model's are, need no view: 2 us each of four)
+        plan = _CHECKED[key] = (rows, D, D > 0 and x.is_contiguous() and (residual is None or residual.is_contiguous()), _dtype_code(x), tuple(x.shape))
+    rows, D, plain, code, shape = plan
+    # a residual stream of another dtype (first block with residual_in_fp32=False, ...) keeps its own
+    res_dtype = residual.dtype if residual is not None else torch.float32 if residual_in_fp32 else x.dtype
     if x.dtype == torch.float32 and res_dtype != torch.float32:
         raise ValueError("fp32 activations need an fp32 residual stream")
-    y = torch.empty(rows, D, dtype=x.dtype, device=x.device)
-    out = torch.empty(rows, D, dtype=res_dtype, device=x.device) if want_residual else None
+    x2, r2 = x, residual
+    if not plain:
+        x2 = x.reshape(-1, D)
+        x2 = x2 if x2.stride(-1) == 1 else x2.contiguous()
+        rows = x2.shape[0]
+        if residual is not None:
+            r2 = residual.reshape(-1, D)
+            r2 = r2 if r2.stride(-1) == 1 else r2.contiguous()
+    y = _empty(x, x.dtype, *shape)
+    out = _empty(x, res_dtype, *shape) if want_residual else None
     res_code = _lib.BASED_F32 if res_dtype == torch.float32 else _lib.BASED_BF16
     with _on_device(x.device):
         _lib.check(_lib.lib().based_add_rms_norm(
-            x2.data_ptr(), r2.data_ptr() if r2 is not None else None, weight.data_ptr(), y.data_ptr(),
-            out.data_ptr() if out is not None else None, rows, D, x2.stride(0),
-            r2.stride(0) if r2 is not None else 0, D, D if out is not None else 0,
-            float(eps), _dtype_code(x), res_code, _stream_ptr(x)))
-    return y.view(x.shape), (out.view(x.shape) if out is not None else None)
+            x2.data_ptr(), _ptr(r2), weight.data_ptr(), y.data_ptr(), _ptr(out), rows, D, D if plain else x2.stride(0),
+            0 if r2 is None else D if plain else r2.stride(0), D, D if out is not None else 0, float(eps), code, res_code, _stream_ptr(x)))
+    return y, out
 
 
 def swiglu(u, weight=None, bias=None) -> torch.Tensor:
@@ -609,8 +609,7 @@ def linear_form(x, weight, bias=None) -> int:
     512 rows: from there on tiles of the wider matrices take a second round (513 rows: 4096 x 1024 13.3, 20.7, with the gate 17.3, 21.4; 2048 x 1024
     9.9, 11.2; 1024 x 2048 10.7, 12.1; 1024 x 1024 9.0, 8.3), which a recorded step of so many sequences would pay for.  A prompt that waits for the
     host would still gain: 4 x 129 to 4 x 512 tokens of the 360M model 4.8 ms here, 4.3 without this line, 4 x 128 3.1."""
-    key = ("linear", x.shape, x.stride(), x.dtype, x.device, weight.shape, weight.stride(), weight.dtype, weight.device,
-           None if bias is None else (bias.shape, bias.stride(), bias.dtype, bias.device))
+    key = ("linear", _form(x, weight, bias))
     form = _CHECKED.get(key)
     if form is None:
         form = LINEAR_LIBRARY
@@ -644,7 +643,7 @@ def _linear_as(form: int, x, weight, bias) -> torch.Tensor:
     N, K = weight.shape
     if form == LINEAR_PROMPT:
         return _prompt_linear(x, weight, bias, N, False)
-    y = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=x.device)
+    y = _empty(x, torch.bfloat16, *x.shape[:-1], N)
     with _on_device(x.device):
         _lib.check(_lib.lib().based_decode_linear(
             x.data_ptr(), K if x.is_contiguous() else x.stride(0), None, 0, weight.data_ptr(), weight.stride(0), None if bias is None else bias.data_ptr(),
@@ -654,7 +653,7 @@ def _linear_as(form: int, x, weight, bias) -> torch.Tensor:
 
 def _prompt_linear(x, weight, bias, N: int, gated: bool) -> torch.Tensor:
     K = weight.shape[1]
-    y = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=x.device)
+    y = _empty(x, torch.bfloat16, *x.shape[:-1], N)
     with _on_device(x.device):
         _lib.check(_lib.lib().based_prompt_linear(x.data_ptr(), K, weight.data_ptr(), weight.stride(0), None if bias is None else bias.data_ptr(),
                                                   y.data_ptr(), N, x.numel() // K, N, K, int(gated), _stream_ptr(x)))
@@ -1077,16 +1076,15 @@ def gated_delta_scan(q, k, v, a_gate, b_gate, a_log, dt_bias, state, heads: int,
         _check_delta(state, B, heads, d, dv)
         plan = _CHECKED[key] = (B, L, d, dv, state.shape[3], q.stride(0), q.stride(1), a_gate.stride(0), a_gate.stride(1), _dtype_code(q))
     B, L, d, dv, state_row, x_sb, x_sl, g_sb, g_sl, code = plan
-    o = torch.empty(B, L, heads, dv, dtype=torch.float32, device=q.device)
+    o = _empty(q, torch.float32, B, L, heads, dv)
     lib, floats = _lib.lib(), 0
     if L >= DELTA_CHUNKS_MIN:
         floats = lib.based_gated_delta_scan_work_as(q.data_ptr(), k.data_ptr(), B, L, heads, d, dv, x_sb, x_sl, code)
     if floats:
-        scan, work = lib.based_gated_delta_scan_chunks, torch.empty(floats, dtype=torch.float32, device=q.device)
+        scan, work = lib.based_gated_delta_scan_chunks, _empty(q, torch.float32, floats)
     else:
         scan = lib.based_gated_delta_scan
-        work = torch.empty(B, heads, 2 * ((L + 2 * DELTA_BLOCK - 1) // (2 * DELTA_BLOCK)), DELTA_PREP_FLOATS, dtype=torch.float32,
-                           device=q.device)
+        work = _empty(q, torch.float32, B, heads, 2 * ((L + 2 * DELTA_BLOCK - 1) // (2 * DELTA_BLOCK)), DELTA_PREP_FLOATS)
     with _on_device(q.device):
         _lib.check(scan(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), a_gate.data_ptr(), b_gate.data_ptr(), a_log.data_ptr(), dt_bias.data_ptr(),
@@ -1165,11 +1163,11 @@ def rglru_prefill(u, y, ra, rb, ri, ib, lam, state, decay_scale: float, fresh: b
     sizes, u_at, y_at, o_at, code = plan
     B, L, W, _ = sizes
     segs = (L + RGLRU_SEGMENT - 1) // RGLRU_SEGMENT
-    agg = torch.empty(B, segs + 1, 2, W, dtype=torch.float32, device=u.device)
+    agg = _empty(u, torch.float32, B, segs + 1, 2, W)
     lib, u_ptr, out_ptr = _lib.lib(), u.data_ptr(), out.data_ptr()
     # an output that shares memory with u is formed apart from it
     n = lib.based_rglru_prefill_work(u_ptr, out_ptr, B, L, W, *u_at, *o_at, code)
-    work = torch.empty(n, dtype=torch.float32, device=u.device) if n else None
+    work = _empty(u, torch.float32, n) if n else None
     with _on_device(u.device):
         _lib.check(lib.based_rglru_prefill(
             u_ptr, y.data_ptr(), ra.data_ptr(), rb.data_ptr(), ri.data_ptr(), ib.data_ptr(), lam.data_ptr(), None, _ptr(work), agg.data_ptr(),
@@ -1340,13 +1338,13 @@ def decay_scan(q, k, v, state, heads: int, *, channel_log2=None, bonus=None, hea
     sizes, strides, stride_bits, code = plan
     B, L, _, d, dv, _ = sizes
     lib = _lib.lib()
-    o = torch.empty(B, L, heads * dv, dtype=q.dtype, device=q.device)
+    o = _empty(q, q.dtype, B, L, heads * dv)
     at = [q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(channel_log2), _ptr(bonus), o.data_ptr()]
     work, by_channel = None, channel_log2 is not None and head_decay is None
     if L >= DECAY_SEGMENTS_MIN:
         bits = at[0] | at[1] | at[2] | (at[4] or 0) | at[5] | (at[3] or 0) >> 1 | stride_bits
         n = (lib.based_decay_scan_channels_work if by_channel else lib.based_decay_scan_work_of)(bits, *sizes, code)
-        work = torch.empty(n, dtype=torch.float32, device=q.device) if n else None
+        work = _empty(q, torch.float32, n) if n else None
     with _on_device(q.device):
         tail = (state.data_ptr(), _ptr(work), at[5], *sizes, *strides, int(activation), int(fresh), code, _stream_ptr(q))
         if by_channel:
@@ -1474,7 +1472,7 @@ def latent_step(q, x, norm_weight, weight, cache, heads: int, dim: int, window: 
             4 * n_q, 4 * (n_q + n_part), n_q + n_part + B * splits * heads * 2, n_pos, half, _dtype_code(x),
             (B, heads, dim, dv, S, R, rot, splits, q.stride(0), x.stride(0), weight.stride(0), cache.stride(0), cache.stride(1), out.stride(0)))
     at_part, at_ml, floats, n_pos, half, code, sizes = plan
-    work = torch.empty(floats, dtype=torch.float32, device=x.device)
+    work = _empty(x, torch.float32, floats)
     work_q = work.data_ptr()
     pos_ptr, pos_host = _pos_args(pos, sizes[0])
     with _on_device(x.device):
@@ -1523,8 +1521,8 @@ def experts(h, router, w1, w2, top: int, norm=None) -> torch.Tensor:
                 raise ValueError(f"the norm's weight must be a contiguous ({D},) on the device")
             normed = torch.empty_like(h2)
             norm_args = (_ptr(residual), _ptr(residual_out), weight.data_ptr(), normed.data_ptr(), float(mult), int(kind), float(eps))
-    y = torch.empty(n, D, dtype=h2.dtype, device=dev)
-    work = torch.empty(ints, dtype=torch.int32, device=dev)  # all that a call keeps between its launches
+    y = _empty(h2, h2.dtype, n, D)
+    work = _empty(h2, torch.int32, ints)  # all that a call keeps between its launches
     at = work.data_ptr()
     h_ptr, w1_ptr, w2_ptr = h2.data_ptr(), w1.data_ptr(), w2.data_ptr()
     # (scores in front of the choices)
