@@ -89,13 +89,15 @@ __global__ __launch_bounds__(256) void rglru_begin_kernel(unsigned long long* ag
 // by two kernels, 43 us: the vector unit is the bound, three exponentials, two reciprocals and a square root an element.  This way 28 us
 // with the kernel in front; B = 8, L = 4096: 92 (218).  The products lie with 16 consecutive tokens of a channel in one lane, where the
 // recurrence is two instructions an element, and 64 in a wavefront.
-template <typename T>
+// NI: tiles of 16 tokens in a segment, 4 NI tokens to a lane: 4, or as few as hold a short prompt, whose other rows would be products for nothing.
+template <typename T, int NI>
 __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_kernel(const RglruArgs a) {
   typedef GateMma<T> M;
   typedef typename Pack<T>::type vec_t;
   constexpr int V = Pack<T>::kN;
   constexpr int KT = 64, KS = KT + 16 / (int)sizeof(T);  // contraction staged at a time
-  __shared__ __attribute__((aligned(16))) T s_u[64 * KS], s_r[64 * KS], s_i[64 * KS];
+  constexpr int SEG = 16 * NI, TL = 4 * NI;
+  __shared__ __attribute__((aligned(16))) T s_u[SEG * KS], s_r[64 * KS], s_i[64 * KS];
   T* s_y = s_r;  // (the output gate, then the output, once the products are done)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4;
   const int tiles = (a.n + 63) / 64;
@@ -106,7 +108,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
     if (tid == 0) s_seg = atomicAdd(a.tickets + ((long)b * gridDim.y + blockIdx.y) * a.ticket_step, 1);
     __syncthreads();
   }
-  const int seg = a.segs > 1 ? __builtin_amdgcn_readfirstlane(s_seg) : 0, l0 = seg * kSeg;
+  const int seg = a.segs > 1 ? __builtin_amdgcn_readfirstlane(s_seg) : 0, l0 = seg * SEG;
   const T* u = static_cast<const T*>(a.u) + b * a.u_sb + (long)blk * a.n;
   const T* ra = static_cast<const T*>(a.ra) + (long)blk * a.n * a.n;
   const T* ri = static_cast<const T*>(a.ri) + (long)blk * a.n * a.n;
@@ -116,58 +118,69 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
   const float nrb = -kL * to_f32(static_cast<const T*>(a.rb)[w]), nib = -kL * to_f32(static_cast<const T*>(a.ib)[w]);
   const float k2 = -2.0f * a.c * softplus_f(to_f32(static_cast<const T*>(a.lam)[w]));
   const float kl = (0.5f * kL) * k2;
-  // Token q * 16 + i * 4 + j of the segment stands in row i * 16 + q * 4 + j: element j of product i in the lanes of quad q.
-  const auto token_of = [](int row) { return (row >> 2 & 3) * 16 + (row >> 4) * 4 + (row & 3); };
+  // Token q * TL + i * 4 + j of the segment stands in row i * 16 + q * 4 + j: element j of product i in the lanes of quad q.
+  const auto token_of = [](int row) { return (row >> 2 & 3) * TL + (row >> 4) * 4 + (row & 3); };
   // Rows of no whole pieces go element by element: as many columns as are live, rounded up to a power of two (and to `least`).  All 64
   // columns cost fp32 at B = 4, L = 2048, 7 blocks of 143 channels 180 us (124 now) and 1,024 blocks of one channel at L = 777 233 (167).
   const auto columns = [](int live, int least) { return 32 - __builtin_clz((live > least ? live : least) * 2 - 1) - 1; };
-  constexpr int YP = 64 * 64 / V / 256;
+  constexpr int YP = (SEG * 64 / V + 255) / 256, YN = SEG * 64 / V;
   vec_t yv[YP];
   const T* y = static_cast<const T*>(a.y) + b * a.y_sb + (long)blk * a.n + c0;
   if (a.vec_y) {
 #pragma unroll
     for (int i = 0; i < YP; ++i) {
-      const int p = i * 256 + tid, e = p % (64 / V) * V, t = l0 + token_of(p / (64 / V));
+      const int p = i * 256 + tid, e = p % (64 / V) * V, t = l0 + token_of(p / (64 / V) % SEG);
       yv[i] = *reinterpret_cast<const vec_t*>(y + (t < a.L ? t : a.L - 1) * a.y_sl + (c0 + e < a.n ? e : 0));
     }
   }
-  f32x4 zr[4], zi[4];  // wavefront: 64 tokens (rows) x 16 channels (columns)
+  f32x4 zr[NI], zi[NI];  // wavefront: 16 NI tokens (rows) x 16 channels (columns)
 #pragma unroll
-  for (int i = 0; i < 4; ++i) zr[i] = zi[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < NI; ++i) zr[i] = zi[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // 64 channels of u and of the gates' rows, asked for one round ahead where the tile is small: a round's products are then shorter than the
+  // wait.  A whole segment has other blocks on the unit meanwhile and no registers left (27 spilled, B = 4, L = 2,048 in 40 us for 31).
+  constexpr bool AHEAD = NI < 4;
+  constexpr int PIECES = 64 * (KT / V) / 256, UN = SEG * (KT / V), UP = (UN + 255) / 256;
+  vec_t xu[UP], xr[PIECES], xi[PIECES];
+  const auto fetch = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int p = i * 256 + tid, row = p / (KT / V), e = (p % (KT / V)) * V;
+      const int c = c0 + row < a.n ? c0 + row : a.n - 1, k = k0 + e < a.n ? k0 + e : 0;
+      if (i < UP) {
+        const int t = l0 + token_of(row % SEG);
+        xu[i] = *reinterpret_cast<const vec_t*>(u + (t < a.L ? t : a.L - 1) * a.u_sl + k);
+      }
+      xr[i] = *reinterpret_cast<const vec_t*>(ra + (long)c * a.n + k);
+      xi[i] = *reinterpret_cast<const vec_t*>(ri + (long)c * a.n + k);
+    }
+  };
+  const auto next = [&](int k0) { return k0 + KT < tiles * KT ? k0 + KT : 0; };
+  if (AHEAD && a.vec_u) fetch(next(c0));
   for (int it = 1, k0 = c0; it <= tiles; ++it) {  // the tile's own channels last: their u stays staged
-    k0 = k0 + KT < tiles * KT ? k0 + KT : 0;
+    k0 = next(k0);
     if (it > 1) __syncthreads();
     const int live = a.n - k0 < KT ? a.n - k0 : KT;
-    constexpr int PIECES = 64 * (KT / V) / 256;
     if (a.vec_u) {
-      vec_t xu[PIECES], xr[PIECES], xi[PIECES];
+      if (!AHEAD) fetch(k0);
 #pragma unroll
       for (int i = 0; i < PIECES; ++i) {
         const int p = i * 256 + tid, row = p / (KT / V), e = (p % (KT / V)) * V;
-        const int t = l0 + token_of(row), c = c0 + row < a.n ? c0 + row : a.n - 1;
-        const int k = k0 + e < a.n ? k0 + e : 0;
-        xu[i] = *reinterpret_cast<const vec_t*>(u + (t < a.L ? t : a.L - 1) * a.u_sl + k);
-        xr[i] = *reinterpret_cast<const vec_t*>(ra + (long)c * a.n + k);
-        xi[i] = *reinterpret_cast<const vec_t*>(ri + (long)c * a.n + k);
+        const bool in = k0 + e < a.n;
+        if (i < UP && (UN % 256 == 0 || p < UN)) *reinterpret_cast<vec_t*>(&s_u[row * KS + e]) = in ? xu[i < UP ? i : 0] : vec_t{};
+        *reinterpret_cast<vec_t*>(&s_r[row * KS + e]) = in ? xr[i] : vec_t{};
+        *reinterpret_cast<vec_t*>(&s_i[row * KS + e]) = in ? xi[i] : vec_t{};
       }
-#pragma unroll
-      for (int i = 0; i < PIECES; ++i) {
-        const int p = i * 256 + tid, row = p / (KT / V), e = (p % (KT / V)) * V;
-        if (k0 + e >= a.n) xu[i] = xr[i] = xi[i] = vec_t{};
-        *reinterpret_cast<vec_t*>(&s_u[row * KS + e]) = xu[i];
-        *reinterpret_cast<vec_t*>(&s_r[row * KS + e]) = xr[i];
-        *reinterpret_cast<vec_t*>(&s_i[row * KS + e]) = xi[i];
-      }
+      if (AHEAD && it < tiles) fetch(next(k0));
     } else {
       const int sh = columns(live, M::kK);
 #pragma unroll 4
       for (int p = tid; p < 64 << sh; p += 256) {
         const int row = p >> sh, e = p - (row << sh);
-        const int t = l0 + token_of(row), c = c0 + row < a.n ? c0 + row : a.n - 1;
+        const int t = l0 + token_of(row % SEG), c = c0 + row < a.n ? c0 + row : a.n - 1;
         const bool in = e < live;
         const int k = in ? k0 + e : 0;
         const T xu = u[(t < a.L ? t : a.L - 1) * a.u_sl + k], xr = ra[(long)c * a.n + k], xi = ri[(long)c * a.n + k];
-        s_u[row * KS + e] = in ? xu : (T)0.0f;
+        if (row < SEG) s_u[row * KS + e] = in ? xu : (T)0.0f;
         s_r[row * KS + e] = in ? xr : (T)0.0f;
         s_i[row * KS + e] = in ? xi : (T)0.0f;
       }
@@ -178,7 +191,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
       const typename M::frag_t fr = *reinterpret_cast<const typename M::frag_t*>(&s_r[(wave * 16 + l16) * KS + e]);
       const typename M::frag_t fi = *reinterpret_cast<const typename M::frag_t*>(&s_i[(wave * 16 + l16) * KS + e]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < NI; ++i) {
         const typename M::frag_t fu = *reinterpret_cast<const typename M::frag_t*>(&s_u[(i * 16 + l16) * KS + e]);
         zr[i] = M::run(fu, fr, zr[i]);
         zi[i] = M::run(fu, fi, zi[i]);
@@ -197,34 +210,35 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
 #pragma unroll
     for (int i = 0; i < YP; ++i) {
       const int p = i * 256 + tid;
+      if (YN % 256 != 0 && p >= YN) break;
       *reinterpret_cast<vec_t*>(&s_y[p / (64 / V) * KS + p % (64 / V) * V]) = yv[i];
     }
   } else {
     const int sh = columns(a.n - c0 < 64 ? a.n - c0 : 64, 1);
 #pragma unroll 4
-    for (int p = tid; p < 64 << sh; p += 256) {
+    for (int p = tid; p < SEG << sh; p += 256) {
       const int row = p >> sh, e = p - (row << sh), t = l0 + token_of(row);
       s_y[row * KS + e] = y[(t < a.L ? t : a.L - 1) * a.y_sl + (c0 + e < a.n ? e : 0)];
     }
   }
   __syncthreads();
-  float A[4][4], I[4][4];
+  float A[NI][4], I[NI][4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       lru_gates_of(zr[i][j], zi[i][j], nrb, nib, k2, kl, to_f32(s_u[(i * 16 + quad * 4 + j) * KS + wave * 16 + l16]), A[i][j], I[i][j]);
-  if (l0 + kSeg > a.L) {  // tokens behind the last one change nothing
-    const int live = a.L - l0 - quad * 16;
+  if (l0 + SEG > a.L) {  // tokens behind the last one change nothing
+    const int live = a.L - l0 - quad * TL;
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
+    for (int t = 0; t < TL; ++t) {
       A[t / 4][t % 4] = t < live ? A[t / 4][t % 4] : 1.f;
       I[t / 4][t % 4] = t < live ? I[t / 4][t % 4] : 0.f;
     }
   }
   float P = A[0][0], X = I[0][0];
 #pragma unroll
-  for (int t = 1; t < 16; ++t) {
+  for (int t = 1; t < TL; ++t) {
     X = __builtin_fmaf(A[t / 4][t % 4], X, I[t / 4][t % 4]);
     P *= A[t / 4][t % 4];
   }
@@ -292,7 +306,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
   S = __builtin_fmaf(before_p, S, before_x);
   if (seg < a.segs - 1 && mine && closes) leave(0.f, __builtin_fmaf(P, S, X));
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       S = __builtin_fmaf(A[i][j], S, I[i][j]);
@@ -306,11 +320,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void rglru_segment_ker
 #pragma unroll
     for (int i = 0; i < YP; ++i) {
       const int p = i * 256 + tid, row = p / (64 / V), e = p % (64 / V) * V, t = l0 + token_of(row);
+      if (YN % 256 != 0 && p >= YN) break;
       if (t < a.L && c0 + e < a.n) *reinterpret_cast<vec_t*>(out + t * a.o_sl + e) = *reinterpret_cast<const vec_t*>(&s_y[row * KS + e]);
     }
   } else {
     const int sh = columns(a.n - c0 < 64 ? a.n - c0 : 64, 1);
-    for (int p = tid; p < 64 << sh; p += 256) {
+    for (int p = tid; p < SEG << sh; p += 256) {
       const int row = p >> sh, e = p - (row << sh), t = l0 + token_of(row);
       if (t < a.L && c0 + e < a.n) out[t * a.o_sl + e] = s_y[row * KS + e];
     }
@@ -522,7 +537,14 @@ template <typename T> void launch_rglru_prefill(const RglruArgs& a, int tiles, T
     hipLaunchKernelGGL(rglru_begin_kernel, dim3((unsigned)(groups < 2048 ? groups : 2048)), block, 0, s, a.agg, words, a.tickets, a.B * tiles,
                        a.ticket_step);
   }
-  hipLaunchKernelGGL(rglru_segment_kernel<T>, grid, block, 0, s, t);
+  // One segment of as few 16-token tiles as hold a short prompt.  bf16, 15 rows of 9 tokens, W = 1536 in 6 blocks: 10.5 us on the whole tile,
+  // 6.5 on one of 16; 3 of 20, W = 1024 in 8: 6.9 and 5.3 on one of 32; fp32, 11 of 8 and 2 of 24 of these widths: 25 and 11, 11.3 and 7.7.
+  if (a.L <= 16)
+    hipLaunchKernelGGL((rglru_segment_kernel<T, 1>), grid, block, 0, s, t);
+  else if (a.L <= 32)
+    hipLaunchKernelGGL((rglru_segment_kernel<T, 2>), grid, block, 0, s, t);
+  else
+    hipLaunchKernelGGL((rglru_segment_kernel<T, kSeg / 16>), grid, block, 0, s, t);
   if (apart) {
     constexpr int V = Pack<T>::kN;
     const bool vec = a.W % V == 0 && a.o_sl % V == 0 && a.o_sb % V == 0 && aligned_to(a.out, 16) && aligned_to(apart, 16);

@@ -83,6 +83,14 @@ def test_narrow_blocks(dev, dtype, L, W, blocks):
     test_rglru_segments(dev, dtype, L, W, blocks, "own", True)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("L", [1, 3, 15, 16, 17, 20, 31, 32, 33])
+@pytest.mark.parametrize("W,blocks,rows,carry", [(64, 1, "own", True), (512, 2, "sliced", False), (144, 2, "shifted", True), (33, 1, "own", True)])
+def test_short_prompts(dev, dtype, L, W, blocks, rows, carry):
+    """Segments of one and of two 16-token tiles: rows in whole pieces and not, one round of the contraction and several."""
+    test_rglru_segments(dev, dtype, L, W, blocks, rows, carry)
+
+
 @pytest.mark.parametrize("L", [4095, 4096, 4097, 4160, 4161, 8192, 8193, 12500])
 def test_groups_of_segments(dev, L):
     """Lengths around one, two and three groups of 64 segments."""
