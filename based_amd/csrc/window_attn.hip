@@ -180,12 +180,15 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
 
 // DIRECT: keys and values of 64 channels each, straight into LDS, the next tile while one is worked on.  Piece p (16 bytes) of row r lies at
 // p ^ (r / 2 % 8), of values at p ^ (r / 2 % 4 * 2), so that reads of 16 rows (transposing reads of 8) meet every bank once; one barrier a tile.
-template <int KC, int VC, bool HALF, bool DIRECT>
-__global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 3 : KC <= 3 && VC <= 4 ? 2 : 1)
+// FILL, of such rows: the portion's keys and values are taken as they come, turned and normed on their way to LDS, and left in the cache by the
+// workgroups whose tokens they are; nobody reads there what is written.
+template <int KC, int VC, bool HALF, bool DIRECT, bool FILL = false>
+__global__ __launch_bounds__(256, FILL ? 2 : KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 3 : KC <= 3 && VC <= 4 ? 2 : 1)
 void window_prefill_mfma_kernel(const WindowArgs a) {
   constexpr int D = KC * 32, DV = VC * 32;
   constexpr int KS = D + 8, VS = kTileKeys + 8;  // LDS row strides: 16-lane reads of 16 bytes meet every bank once
   static_assert(!DIRECT || (KC == 2 && VC == 2), "rows of 64 channels");
+  static_assert(!FILL || DIRECT, "tiles as DIRECT has them");
   __shared__ __attribute__((aligned(16))) __bf16 lds_k[DIRECT ? 8 : kTileKeys * KS];
   __shared__ __attribute__((aligned(16))) __bf16 lds_v[DIRECT ? 8 : DV * VS];
   // (an array whose extent the launch gives: in front of every read of a static one the compiler waits for all loads that go to LDS)
@@ -278,7 +281,62 @@ void window_prefill_mfma_kernel(const WindowArgs a) {
     }
   };
 
-  if constexpr (DIRECT) ask(lo, 0);
+  // FILL: the same tile by way of registers, eight lanes to a row
+  u32x4 fresh_k[FILL ? 2 : 1], fresh_v[FILL ? 2 : 1];
+  Turn8<HALF> turn_k[FILL ? 2 : 1];
+  auto ask_fresh = [&](int k0) {
+    const __bf16* pk = static_cast<const __bf16*>(a.k) + b * a.k_sb + (long)g * a.d;
+    const __bf16* pv = static_cast<const __bf16*>(a.v) + b * a.v_sb + (long)g * a.dv;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int row = (i * 256 + tid) >> 3, c = (tid & 7) * 8, key = k0 + row <= last_pos ? k0 + row : last_pos;
+      const bool old = key < a.pos_host;
+      const __bf16* kr = old ? kv + (long)key * a.kv_st : pk + (long)(key - a.pos_host) * a.k_sl;
+      const __bf16* vr = old ? kv + (long)key * a.kv_st + a.d : pv + (long)(key - a.pos_host) * a.v_sl;
+      fresh_k[i] = *reinterpret_cast<const u32x4*>(kr + c);
+      fresh_v[i] = *reinterpret_cast<const u32x4*>(vr + c);
+      turn_k[i].load(kr, c, key, a);
+    }
+  };
+  auto settle = [&](int k0, int to) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int row = (i * 256 + tid) >> 3, piece = tid & 7, key = k0 + row;
+      if (key >= a.pos_host) {  // (the same in the eight lanes of a row)
+        float x[8], ss = 0.f;
+        bf16x8 out;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = to_f32(__builtin_bit_cast(bf16x8, fresh_k[i])[j]);
+        turn_k[i].apply(x, piece * 8, a);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) out[j] = from_f32<__bf16>(x[j]);
+        fresh_k[i] = __builtin_bit_cast(u32x4, out);
+        if (a.norm_v) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) x[j] = to_f32(__builtin_bit_cast(bf16x8, fresh_v[i])[j]);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(x[j], x[j], ss);
+          const float by = 1.0f / sqrtf(sum8(ss) / (float)a.dv + a.eps);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) out[j] = from_f32<__bf16>(x[j] * by);
+          fresh_v[i] = __builtin_bit_cast(u32x4, out);
+        }
+        if (key >= first_pos && key <= last_pos) {
+          __bf16* fill = const_cast<__bf16*>(kv) + (long)key * a.kv_st + piece * 8;
+          *reinterpret_cast<u32x4*>(fill) = fresh_k[i];
+          *reinterpret_cast<u32x4*>(fill + a.d) = fresh_v[i];
+        }
+      }
+      __bf16* tile = lds_tiles + to * kDirectTile + row * 64;
+      *reinterpret_cast<u32x4*>(tile + (piece ^ (row >> 1 & 7)) * 8) = fresh_k[i];
+      *reinterpret_cast<u32x4*>(tile + kTileKeys * 64 + (piece ^ (row >> 1 & 3) * 2) * 8) = fresh_v[i];
+    }
+  };
+
+  if constexpr (FILL)
+    ask_fresh(lo);
+  else if constexpr (DIRECT)
+    ask(lo, 0);
   // queries: lane holds channels quad*8 + 32 c .. of row l16 (+16): the MFMA's second operand.  Turned and
   // rounded after the first tile of keys has been asked for.
   bf16x8 qf[2][KC];
@@ -349,7 +407,12 @@ void window_prefill_mfma_kernel(const WindowArgs a) {
   const float scale2 = fabsf(a.scale) * 1.4426950408889634f;  // scores in powers of two; the sign is the queries'
   int place = 0;
   for (int k0 = lo; k0 <= last_pos; k0 += kTileKeys) {
-    if constexpr (DIRECT) {
+    if constexpr (FILL) {
+      settle(k0, place);
+      lds_barrier();  // (the reads of this place two tiles ago lie in front of the barrier of the last one)
+      if (k0 + kTileKeys <= last_pos) ask_fresh(k0 + kTileKeys);
+      __builtin_amdgcn_sched_barrier(0);
+    } else if constexpr (DIRECT) {
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_waitcnt(0x0070);  // own loads are there, own reads of the tile before are done
       __builtin_amdgcn_s_barrier();
@@ -1406,12 +1469,12 @@ template <int LPI> void launch_kv_write(const WindowArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((window_kv_write_vec_kernel<LPI, false>), grid, dim3(256), 0, s, a);
 }
 
-template <int KC, int VC, bool DIRECT> void launch_window_mfma_pairs(const WindowArgs& a, dim3 grid, hipStream_t s) {
+template <int KC, int VC, bool DIRECT, bool FILL = false> void launch_window_mfma_pairs(const WindowArgs& a, dim3 grid, hipStream_t s) {
   constexpr unsigned lds = DIRECT ? 2 * kDirectTile * sizeof(__bf16) : 0;
   if (a.half_split)
-    hipLaunchKernelGGL((window_prefill_mfma_kernel<KC, VC, true, DIRECT>), grid, dim3(256), lds, s, a);
+    hipLaunchKernelGGL((window_prefill_mfma_kernel<KC, VC, true, DIRECT, FILL>), grid, dim3(256), lds, s, a);
   else
-    hipLaunchKernelGGL((window_prefill_mfma_kernel<KC, VC, false, DIRECT>), grid, dim3(256), lds, s, a);
+    hipLaunchKernelGGL((window_prefill_mfma_kernel<KC, VC, false, DIRECT, FILL>), grid, dim3(256), lds, s, a);
 }
 
 template <int KC> void launch_window_mfma(const WindowArgs& a, dim3 grid, hipStream_t s) {
@@ -1509,34 +1572,50 @@ template <int KB, int VB> void launch_window_f32(const WindowArgs& a, dim3 grid,
 }
 
 // Whether memory that rows of `width` elements at these strides span overlaps.
-static bool rows_meet(const WindowArgs& a, const void* x, long x_sb, long x_sl, long x_width, const void* y, long y_sb, long y_sl, long y_width) {
-  const auto bytes = [&](long sb, long sl, long width) { return ((a.B - 1) * sb + (a.L - 1) * sl + width) * 4; };
+static bool rows_meet(const WindowArgs& a, const void* x, long x_sb, long x_sl, long x_width, const void* y, long y_sb, long y_sl, long y_width, int size) {
+  const auto bytes = [&](long sb, long sl, long width) { return ((a.B - 1) * sb + (a.L - 1) * sl + width) * size; };
   const uintptr_t p = reinterpret_cast<uintptr_t>(x), q = reinterpret_cast<uintptr_t>(y);
   return p < q + bytes(y_sb, y_sl, y_width) && q < p + bytes(x_sb, x_sl, x_width);
 }
 
-// Whether the fp32 form fills the cache itself: keys and values are read by every workgroup that sees them, so that nothing else may be written
-// there, and in 16-byte pieces.
-static bool window_f32_fills(const WindowArgs& a) {
-  if (!window_f32_small(a) || window_f32_keys(a) > 256 || a.d > 64) return false;
-  if (a.k_sb % 4 || a.k_sl % 4 || a.v_sb % 4 || a.v_sl % 4 || !aligned_to(a.k, 16) || !aligned_to(a.v, 16)) return false;
+// Whether the attention may fill the cache itself (elements of `size` bytes): keys and values are read by every workgroup that sees them, so that
+// nothing else may be written there, and in 16-byte pieces.
+static bool window_fresh(const WindowArgs& a, int size) {
+  const int n = 16 / size;
+  if (a.k_sb % n || a.k_sl % n || a.v_sb % n || a.v_sl % n || !aligned_to(a.k, 16) || !aligned_to(a.v, 16)) return false;
   if (a.k_sb < 0 || a.k_sl < 0 || a.v_sb < 0 || a.v_sl < 0 || a.o_sb < 0 || a.o_sl < 0 || a.kv_sb < 0 || a.kv_st < 0) return false;
   const long kw = (long)a.G * a.d, vw = (long)a.G * a.dv, row = kw + vw;
-  const float* cache = static_cast<const float*>(a.kv) + (long)a.pos_host * a.kv_st;
+  const char* cache = static_cast<const char*>(a.kv) + (long)a.pos_host * a.kv_st * size;
   const auto apart = [&](const void* x, long sb, long sl, long width) {
-    return !rows_meet(a, x, sb, sl, width, cache, a.kv_sb, a.kv_st, row) && !rows_meet(a, x, sb, sl, width, a.o, a.o_sb, a.o_sl, (long)a.H * a.dv);
+    return !rows_meet(a, x, sb, sl, width, cache, a.kv_sb, a.kv_st, row, size) && !rows_meet(a, x, sb, sl, width, a.o, a.o_sb, a.o_sl, (long)a.H * a.dv, size);
   };
   return apart(a.k, a.k_sb, a.k_sl, kw) && apart(a.v, a.v_sb, a.v_sl, vw);
 }
+static bool window_f32_fills(const WindowArgs& a) {
+  return window_f32_small(a) && window_f32_keys(a) <= 256 && a.d <= 64 && window_fresh(a, 4);
+}
+// The bf16 form with rows of 64 channels: a launch less for some workgroups turning every key that they see, `before` of them in front of their own
+// tokens, by way of registers and with two wavefronts to a SIMD.  Kernel us with a launch for the cache / filled, 16 heads, half-split pairs, by
+// workgroups and `before`: 16 (3 tokens), 0: 6.7 / 5.4; 8, 32: 8.6 / 6.9; 512, 0: 13.9 / 10.4; 512, 68: 15.5 / 13.4; 512, 112: 15.3 / 14.1;
+// 128 heads' tokens to a workgroup, 128, 128: 15.3 / 14.2; 256, 128: 14.6 / 13.2; 384, 128: 17.3 / 16.9; 512, 128: 17.4 / 18.2; 1,024, 128: 25.1 /
+// 28.6; 28, 168: 11.2 / 12.1; 256, 512: 23.0 / 27.8.
+static bool window_bf16_fills(const WindowArgs& a) {
+  if (a.d != 64 || a.dv != 64) return false;
+  const long qpk = a.H / a.G, groups = ((long)a.L * qpk + kTileRows - 1) / kTileRows * a.G * a.B, own = kTileRows / qpk;
+  const long front = (long)a.pos_host + a.L - own, before = front < 0 ? 0 : front < a.window - 1 ? front : a.window - 1;
+  return before <= 128 && groups <= 768 && groups * before <= 512 * 112 && window_fresh(a, 2);
+}
 
-// The attention of a portion whose keys and values are in place (fill: it puts them there itself; `window_f32_fills`).
+// The attention of a portion whose keys and values are in place (fill: it puts them there itself; `window_f32_fills`, `window_bf16_fills`).
 static void launch_window_attend(WindowArgs a, bool vec, int io_dtype, bool fill, hipStream_t s) {
   if (vec) {
     const uint32_t qpk = (uint32_t)(a.H / a.G);
     a.heads_inv = qpk == 1 ? ~0u : (uint32_t)((1ull << 32) / qpk);
     const dim3 grid((unsigned)(((long)a.L * qpk + kTileRows - 1) / kTileRows), (unsigned)a.G, (unsigned)a.B);
     const int kc = (int)((a.d + 31) / 32);
-    if (a.d == 64 && a.dv == 64)
+    if (fill)
+      launch_window_mfma_pairs<2, 2, true, true>(a, grid, s);
+    else if (a.d == 64 && a.dv == 64)
       launch_window_mfma_pairs<2, 2, true>(a, grid, s);
     else if (kc <= 1)
       launch_window_mfma<1>(a, grid, s);
@@ -1590,14 +1669,14 @@ extern "C" BASED_API int based_window_attn_prefill(
   const bool vec = io_dtype == BASED_BF16 && D <= 256 && DV <= 256 && rotary_dim % (half_split ? 16 : 8) == 0 && window_vec(a, 8);
   const int64_t items = B * L * G;
   BASED_REQUIRE(items < (1ll << 32), BASED_ERR_SHAPE, "window_attn_prefill: grid too large");
-  const bool fill = window_f32(a, io_dtype) && !window_f32_few(a) && window_f32_fills(a);
-  if (vec) {
+  const bool fill = vec ? window_bf16_fills(a) : window_f32(a, io_dtype) && !window_f32_few(a) && window_f32_fills(a);
+  if (fill)
+    ;
+  else if (vec) {
     const int64_t widest = D > DV ? D : DV;
     widest <= 64 ? launch_kv_write<8>(a, s) : widest <= 128 ? launch_kv_write<16>(a, s) : launch_kv_write<32>(a, s);
   } else if (io_dtype == BASED_BF16)
     hipLaunchKernelGGL(window_kv_write_kernel<__bf16>, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s, a);
-  else if (fill)
-    ;
   else if (window_f32(a, io_dtype) && k_sb % 4 == 0 && k_sl % 4 == 0 && v_sb % 4 == 0 && v_sl % 4 == 0 && aligned_to(k, 16) && aligned_to(v, 16))
     hipLaunchKernelGGL(window_kv_write_f32_kernel, dim3((unsigned)((items + 15) / 16)), dim3(256), 0, s, a);
   else

@@ -66,3 +66,44 @@ def test_weights_are_summed_in_32_bits(dev, d):
     ref = O.window_softmax(q[0].double(), k[0].double(), v[0].double(), -math.log(weight), window)[20:, 0]
     # (with weights of 0.5 the outputs 1 / (1 + n w) are 0.9 to 1.0 of 3.7e-3 too large)
     assert abs(float((out / ref - 1).mean())) < 5e-4
+
+
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("H,G,B,L,start,window,rot,half", [
+    (16, 4, 1, 3, 0, 129, 32, True), (16, 4, 2, 64, 1, 65, 64, False), (16, 4, 1, 777, 0, 129, 32, True), (16, 4, 1, 300, 77, 130, 32, True),
+    (12, 4, 3, 130, 0, 20, 8, False), (136, 1, 1, 33, 20, 64, 16, True), (16, 16, 2, 257, 0, 129, 0, False), (5, 1, 1, 140, 13, 500, 48, True),
+    (16, 2, 32, 128, 0, 513, 32, True), (16, 2, 33, 128, 0, 513, 32, True), (16, 4, 3, 1024, 0, 129, 32, True), (16, 4, 7, 512, 0, 129, 32, False)])
+def test_cache_that_the_attention_fills(dev, H, G, B, L, start, window, rot, half, norm):
+    """Rows of the cache behind a portion, and what a second portion makes of them: written by the attention itself, or in front of it where the
+    portion's own keys lie in the output's rows; both sides of the rule that tells them."""
+    from based_amd import ops
+    from based_amd.mixers.window_attention import _ExactRotary
+
+    g = torch.Generator().manual_seed(L + B)
+    n, d = L + start, 64
+    kw = dict(rope=_ExactRotary(rot, base=100.0, interleaved=not half).tables(n, dev) if rot else None, value_norm_eps=1e-5 if norm else None)
+    x = torch.randn(B, n, H * d + 2 * G * d, generator=g).bfloat16().to(dev)
+    q, k, v = x[..., :H * d], x[..., H * d:(H + G) * d], x[..., (H + G) * d:]
+
+    def run(inside):
+        cache = torch.full((B, n + 2, G, 2 * d), float("nan"), dtype=torch.bfloat16, device=dev)
+        room = x.clone()
+        kk, vv = (room[..., H * d:(H + G) * d], room[..., (H + G) * d:]) if inside else (k, v)
+        out = room[..., :H * d]
+        for lo, hi in ((0, start), (start, n)):
+            if hi > lo:
+                s = slice(lo, hi)
+                ops.window_attn_prefill(q[:, s], kk[:, s], vv[:, s], cache, H, G, window, d ** -0.5, lo, out=out[:, s], **kw)
+        return out.double(), cache
+
+    out, cache = run(False)
+    ref, rows = run(True)
+    # a rotation's two products and a norm's sum are added in one order or the other: now and then the other of two neighbours in bf16
+    assert float((cache[:, :n].double() - rows[:, :n].double()).norm() / rows[:, :n].double().norm()) < 2 ** -12
+    assert cache[:, n:].isnan().all() and rows[:, n:].isnan().all()
+    assert float((out - ref).norm() / ref.norm()) < 2 ** -10
+    want = v.view(B, n, G, d).double()
+    if norm:
+        want = want / (want.square().mean(-1, keepdim=True) + 1e-5).sqrt()
+    # eight significant bits: an element is rounded by at most 2^-8 of itself
+    assert float(((cache[:, :n, :, d:].double() - want).norm(dim=-1) / want.norm(dim=-1)).max()) < 2 ** -8
