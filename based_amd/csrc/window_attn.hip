@@ -1595,15 +1595,16 @@ static bool window_f32_fills(const WindowArgs& a) {
   return window_f32_small(a) && window_f32_keys(a) <= 256 && a.d <= 64 && window_fresh(a, 4);
 }
 // The bf16 form with rows of 64 channels: a launch less for some workgroups turning every key that they see, `before` of them in front of their own
-// tokens, by way of registers and with two wavefronts to a SIMD.  Kernel us with a launch for the cache / filled, 16 heads, half-split pairs, by
+// tokens, by way of registers and with two wavefronts to a SIMD.  Kernel us with a launch for the cache / filled, 16 heads, interleaved pairs, by
 // workgroups and `before`: 16 (3 tokens), 0: 6.7 / 5.4; 8, 32: 8.6 / 6.9; 512, 0: 13.9 / 10.4; 512, 68: 15.5 / 13.4; 512, 112: 15.3 / 14.1;
 // 128 heads' tokens to a workgroup, 128, 128: 15.3 / 14.2; 256, 128: 14.6 / 13.2; 384, 128: 17.3 / 16.9; 512, 128: 17.4 / 18.2; 1,024, 128: 25.1 /
-// 28.6; 28, 168: 11.2 / 12.1; 256, 512: 23.0 / 27.8.
+// 28.6; 28, 168: 11.2 / 12.1; 256, 512: 23.0 / 27.8.  Half-split pairs, which fetch partners and twice the angles: 16 (3 tokens), 0: 6.9 / 5.8; 512,
+// 68: 16.4 / 14.8; 98, 128: 12.3 / 12.4; 256, 128: 14.7 / 14.6; 384, 128: 18.1 / 18.8.
 static bool window_bf16_fills(const WindowArgs& a) {
   if (a.d != 64 || a.dv != 64) return false;
   const long qpk = a.H / a.G, groups = ((long)a.L * qpk + kTileRows - 1) / kTileRows * a.G * a.B, own = kTileRows / qpk;
   const long front = (long)a.pos_host + a.L - own, before = front < 0 ? 0 : front < a.window - 1 ? front : a.window - 1;
-  return before <= 128 && groups <= 768 && groups * before <= 512 * 112 && window_fresh(a, 2);
+  return before <= 128 && groups <= 768 && groups * before <= 512 * (a.half_split ? 72 : 112) && window_fresh(a, 2);
 }
 
 // The attention of a portion whose keys and values are in place (fill: it puts them there itself; `window_f32_fills`, `window_bf16_fills`).
