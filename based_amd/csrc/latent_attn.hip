@@ -452,6 +452,170 @@ __global__ __launch_bounds__(256, 1) void latent_step_mfma_kernel(const LatentAr
   }
 }
 
+// fp32, fp32 MFMA: 16 heads per workgroup, 16 keys at a time to a wavefront, which has a maximum and sums of its own; the four are put together
+// in the end.  KC: 16-channel pieces of a row, RT: 64-channel groups of the latent (both rounded up); rows of whole 16-byte pieces.
+// As elsewhere in fp32, keys and queries give up their channels in the same order, so that a lane reads 16 bytes for four products; scores come
+// with keys in rows, so that product i of the weighted latents takes the lane's own weight i, against key 4 quad + i, of which lane l16 holds
+// channels 4 l16 .. + 3: rows 4 r + j of the four tiles.  Keys go from memory to the products both times, without LDS or a barrier on the way.
+// Bound by the fp32 matrix rate, 136 products of 32 cycles for 16 keys of 288 channels, and for few sequences by its three launches.  Kernel us of a
+// step, 16 heads, R = 256, rot = 32, a workgroup per head on the vector unit / this way, by sequences and keys: 1, 129: 18.3 / 18.4; 4, 512: 23.7 /
+// 20.0; 13, 1,024: 66.8 / 24.9; 40, 129: 42.6 / 21.4; 116, 512: 261 / 44; 128, 1,024: 551 / 62.  One head, 40 of 1,024: 37.3 / 31.0.
+template <int KC, int RT>
+__global__ __launch_bounds__(256, RT <= 4 ? 2 : 1) void latent_step_f32_kernel(const LatentArgs a) {
+  constexpr int QS = KC * 16 + 4, RS = RT * 64 + 4;  // LDS row strides: 16-lane reads of 16 bytes meet every bank once
+  __shared__ __attribute__((aligned(16))) float lds[16 * (QS > 2 * RS ? QS : 2 * RS)];  // queries; in the end latents of two wavefronts
+  __shared__ float s_max[4][16], s_sum[4][16];
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4, W = a.R + a.rot;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int b = blockIdx.x, split = blockIdx.y, h0 = blockIdx.z * 16;
+  const int pos = row_pos(a.pos, a.pos_host, b);
+  if (pos < 0 || pos >= a.S) return;
+  int first, n;
+  split_range(a, pos, split, first, n);
+  const char* cache = reinterpret_cast<const char*>(static_cast<const float*>(a.cache) + b * a.c_sb + (long)first * a.c_st);
+  const uint32_t step = (uint32_t)a.c_st * 4;  // (bytes from one base in 32 bits: a pointer per piece of a row would be two registers each)
+  const long at = ((long)b * a.splits + split) * a.H + h0 + l16;  // of this lane's head
+  const bool head_in = h0 + l16 < a.H;
+  if (n == 0) {
+    if (head_in && tid < 16) a.part_ml[2 * at] = -INFINITY, a.part_ml[2 * at + 1] = 0.f;
+    return;
+  }
+  // (rows past the last key are fetched as the last one, channels past the sizes as the first, which meet queries of zero or are not stored)
+  f32x4 kf[KC];
+  int q4 = quad * 4;
+  const auto fetch = [&](int k0) {
+    const int key = k0 + l16;
+    asm volatile("" : "+v"(q4));  // (places in a row are worked out again: held, they would be KC registers)
+    const uint32_t row = (uint32_t)(key < n ? key : n - 1) * step;
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      const int e = c * 16 + q4;
+      kf[c] = *reinterpret_cast<const f32x4*>(cache + (row + (uint32_t)(e < W ? e * 4 : 0)));
+    }
+  };
+  int k0 = wave * 16;
+  fetch(k0);
+  for (int i = tid; i < 16 * KC * 4; i += 256) {
+    const int h = i / (KC * 4), e = i % (KC * 4) * 4;
+    const bool in = h0 + h < a.H && e < W;
+    const f32x4 x = *reinterpret_cast<const f32x4*>(a.qa + ((long)b * a.H + (in ? h0 + h : 0)) * W + (in ? e : 0));
+    *reinterpret_cast<f32x4*>(&lds[h * QS + e]) = in ? x : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  __syncthreads();
+  f32x4 acc[RT][4];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+  constexpr float kLog2e = 1.4426950408889634f;
+  int q_at = l16 * QS + quad * 4;
+  for (; k0 < n; k0 += 64) {
+    asm volatile("" : "+v"(q_at));  // (read again for every 16 keys: held, the queries would be 4 KC registers)
+    constexpr int VB = RT <= 4 ? 4 : 1;  // rows of latents in flight
+    f32x4 vf[VB][RT];
+    const auto latents = [&](int i, f32x4 (&to)[RT]) {
+      const int key = k0 + quad * 4 + i;
+      const uint32_t row = (uint32_t)(key < n ? key : n - 1) * step;
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        const int e = t * 64 + l16 * 4;
+        to[t] = *reinterpret_cast<const f32x4*>(cache + (row + (uint32_t)(e < a.R ? e * 4 : 0)));
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < VB; ++i) latents(i, vf[i]);
+    f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};  // (two sums of half the channels each round less than one)
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      const f32x4 q = *reinterpret_cast<const f32x4*>(&lds[q_at + c * 16]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s[c & 1] = mfma_f32(kf[c][j], q[j], s[c & 1]);
+    }
+    if (VB == 4 && k0 + 64 < n) fetch(k0 + 64);
+    float p[4], mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      p[i] = k0 + quad * 4 + i < n ? (s[0][i] + s[1][i]) * a.scale : -INFINITY;
+      mx = fmaxf(mx, p[i]);
+    }
+    if (__any(mx > m_run)) {
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float m_new = fmaxf(m_run, mx), alpha = __builtin_amdgcn_exp2f((m_run - m_new) * kLog2e);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[t][j] *= alpha;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      p[i] = __builtin_amdgcn_exp2f((p[i] - m_run) * kLog2e);
+      l_run += p[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (i >= VB) latents(i, vf[0]);
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[t][j] = mfma_f32(vf[i % VB][t][j], p[i], acc[t][j]);
+    }
+    if (VB < 4 && k0 + 64 < n) fetch(k0 + 64);
+  }
+  // the four wavefronts together
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
+  if (quad == 0) s_max[wave][l16] = m_run, s_sum[wave][l16] = l_run;
+  __syncthreads();
+  const float m_all = fmaxf(fmaxf(s_max[0][l16], s_max[1][l16]), fmaxf(s_max[2][l16], s_max[3][l16]));
+  const float mine = m_run == -INFINITY && l_run == 0.f ? 0.f : __builtin_amdgcn_exp2f((m_run - m_all) * kLog2e);  // (no key of its own: nothing)
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[t][j] *= mine;
+  const auto place = [&](int from, int t, int i) { return &lds[(from * 16 + l16) * RS + t * 64 + (quad * 4 + i) * 4]; };
+#pragma unroll
+  for (int half = 2; half >= 1; half /= 2) {
+    if (wave >= half && wave < 2 * half) {
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<f32x4*>(place(wave - half, t, i)) = f32x4{acc[t][0][i], acc[t][1][i], acc[t][2][i], acc[t][3][i]};
+    }
+    __syncthreads();
+    if (wave < half) {
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(place(wave, t, i));
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[t][j][i] += x[j];
+        }
+    }
+    __syncthreads();
+  }
+  if (wave > 0 || !head_in) return;
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int c = t * 64 + (quad * 4 + i) * 4;
+      if (c < a.R) *reinterpret_cast<f32x4*>(a.part + at * a.R + c) = f32x4{acc[t][0][i], acc[t][1][i], acc[t][2][i], acc[t][3][i]};
+    }
+  if (quad == 0) {
+    float sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      sum += s_max[w][l16] == -INFINITY && s_sum[w][l16] == 0.f ? 0.f : s_sum[w][l16] * __builtin_amdgcn_exp2f((s_max[w][l16] - m_all) * kLog2e);
+    a.part_ml[2 * at] = m_all;
+    a.part_ml[2 * at + 1] = sum;
+  }
+}
+
 constexpr int kValueRows = 4;   // sequences at a time
 constexpr int kValueCols = 16;  // value channels per workgroup
 constexpr int kMaxSplits = 64;
@@ -705,6 +869,28 @@ static bool launch_latent_step_mfma(const LatentArgs& a, hipStream_t s) {
   return true;
 }
 
+template <int KC, int RT> void launch_latent_f32(const LatentArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL((latent_step_f32_kernel<KC, RT>), dim3((unsigned)a.B, (unsigned)a.splits, (unsigned)((a.H + 15) / 16)), dim3(256), 0, s, a);
+}
+
+static bool launch_latent_step_f32(const LatentArgs& a, hipStream_t s) {
+  const int kc = (a.R + a.rot + 15) / 16, rt = (a.R + 63) / 64;
+  if (kc <= 6 && rt <= 1)
+    launch_latent_f32<6, 1>(a, s);
+  else if (kc <= 10 && rt <= 2)
+    launch_latent_f32<10, 2>(a, s);
+  else if (kc <= 20 && rt <= 4)
+    launch_latent_f32<20, 4>(a, s);
+  // (latents of 512 channels, a row at a time for their registers: with few workgroups on the vector unit their way is the shorter one.  Us, one
+  // way / the other, by those workgroups: 48 25.5 / 28.5; 96 26.1 / 28.8; 128 29.3 / 29.5; 192 29.3 / 29.6; 256 34.1 / 29.6; 120 of 40 sequences
+  // 31.4 / 30.3)
+  else if (kc <= 36 && rt <= 8 && (long)a.B * a.H * a.splits >= 120)
+    launch_latent_f32<36, 8>(a, s);
+  else
+    return false;
+  return true;
+}
+
 }  // namespace based
 
 extern "C" BASED_API int based_latent_write(const void* x, const void* norm_w, void* cache, int64_t start, int64_t B, int64_t L, int64_t S,
@@ -771,9 +957,10 @@ extern "C" BASED_API int based_latent_step(const void* q, const void* x, const v
     launch_latent_query<__bf16>(a, vec, s);
   else
     launch_latent_query<float>(a, vec, s);
-  const bool mfma = io_dtype == BASED_BF16 && R % 8 == 0 && rot % 8 == 0 && c_sb % 8 == 0 && c_st % 8 == 0 && aligned_to(cache, 16) &&
-                    aligned_to(work_q, 16) && aligned_to(work_part, 16);
-  if (!mfma || !launch_latent_step_mfma(a, s)) {
+  const bool near = io_dtype == BASED_BF16 || (c_st > 0 && S * c_st < (1ll << 30));  // (the fp32 form counts bytes of a sequence's cache in 32 bits)
+  const bool mfma = near && R % n == 0 && rot % n == 0 && c_sb % n == 0 && c_st % n == 0 && aligned_to(cache, 16) && aligned_to(work_q, 16) &&
+                    aligned_to(work_part, 16);
+  if (!mfma || !(io_dtype == BASED_BF16 ? launch_latent_step_mfma(a, s) : launch_latent_step_f32(a, s))) {
     const dim3 grid((unsigned)(B * H * splits));
     if (io_dtype == BASED_BF16)
       hipLaunchKernelGGL(latent_step_any_kernel<__bf16>, grid, dim3(256), 0, s, a);

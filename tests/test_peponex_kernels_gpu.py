@@ -392,6 +392,40 @@ def test_latent_steps_of_many_rows(dev, H, d, r, dv, R, window, dtype):
                 close(o[b, 0], latent_want(core, uk, uv, nw, q[b, :n].double(), x[b, :n].double())[-1], 2 * TOL[dtype])
 
 
+@pytest.mark.parametrize("H,d,r,dv,R,window,keys", [
+    (16, 16, 32, 16, 256, 129, 400), (1, 8, 4, 8, 4, 15, 40), (17, 16, 8, 20, 60, 16, 16), (3, 8, 12, 8, 64, 17, 300), (16, 8, 16, 8, 68, 64, 70),
+    (5, 16, 4, 16, 128, 65, 66), (2, 8, 60, 8, 260, 200, 260), (20, 16, 64, 16, 512, 130, 200), (16, 8, 64, 8, 516, 20, 30), (40, 8, 32, 8, 288, 1, 3)])
+def test_fp32_steps_on_the_matrix_unit(dev, H, d, r, dv, R, window, keys):
+    """Heads, keys and channels around whole tiles, rows of a wider cache, sequences with all, some and one of the keys: against 64 bits, and
+    against the other form, which takes rows that are not in whole pieces."""
+    from based_amd import ops
+
+    B, at = 5, [keys - 1, 0, keys // 2, min(15, keys - 1), keys // 3]
+    q, x = rnd(B, H * (r + d), seed=1).to(dev), rnd(B, R + r, seed=2).to(dev)
+    nw, w = rnd(R, seed=3, scale=0.2, mean=1.0).to(dev), rnd(H * (r + d + dv), R, seed=4, scale=R ** -0.5).to(dev)
+    rows = rnd(B, keys, R + r, seed=5)
+    pos = torch.tensor(at, dtype=torch.int32, device=dev)
+    ang = torch.outer(torch.arange(keys, dtype=torch.float64), 500.0 ** (-torch.arange(0, r, 2, dtype=torch.float64) / r))
+    rope = (ang.cos().float().to(dev), ang.sin().float().to(dev), False)
+    out = []
+    for wide in (4, 5):
+        cache = torch.full((B, keys, R + r + wide), float("nan"), device=dev)[..., :R + r]
+        for b, p in enumerate(at):
+            cache[b, :p] = rows[b, :p].to(dev)
+        out.append(ops.latent_step(q, x, nw, w, cache, H, d, window, 0.3, pos, 1e-5, rope, out=torch.empty(B, H * dv, device=dev)).double().cpu())
+    uk, uv = w.double().cpu().view(H, r + d + dv, R)[:, r:r + d], w.double().cpu().view(H, r + d + dv, R)[:, r + d:]
+    for b, p in enumerate(at):
+        own = cache[b, p].double().cpu()  # (the token's row as it is kept)
+        turned = lambda y: torch.cat([y[..., :r // 2] * ang[p].cos() - y[..., r // 2:] * ang[p].sin(),  # noqa: E731
+                                      y[..., r // 2:] * ang[p].cos() + y[..., :r // 2] * ang[p].sin()], -1)
+        c = torch.cat([rows[b, max(0, p - window + 1):p].double(), own[None]])
+        qb = q[b].double().cpu().view(H, r + d)
+        s = 0.3 * (torch.matmul(torch.matmul(qb[:, None, r:], uk)[:, 0], c[:, :R].T) + turned(qb[:, :r]) @ c[:, R:].T)
+        want = torch.matmul(uv, (s.softmax(-1) @ c[:, :R]).unsqueeze(-1))[..., 0].reshape(-1)
+        for o in out:  # sums of up to 576 products, scores of some tens of units: 2^-24 of each
+            close(o[b], want, 1e-5)
+
+
 # ---- experts ----
 def expert_case(n, D, F, E, top, dtype, seed=0):
     h, router = rnd(n, D, seed=seed, dtype=dtype), rnd(E, D, seed=seed + 1, dtype=dtype, scale=2 * D ** -0.5)
