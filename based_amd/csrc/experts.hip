@@ -40,29 +40,47 @@ struct RouteArgs {
 
 __device__ __forceinline__ f32x4 expert_mfma(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
-// Tiles of every expert from its count (of each its expert, 8 bits, and its rows), by threads 0 .. 255; scan: 256 ints of LDS.  Called by a whole workgroup.
-__device__ __forceinline__ void plan_tiles(const int* counts, int* scan, int* first_of, int32_t* tile_first, int32_t* tile_expert, int E, int tile_rows) {
+// scan[e] becomes the sum of own of threads 0 .. e (own 0 from thread E on; up to 256).  By one wavefront where it has a lane for each.
+__device__ __forceinline__ void sum_up(uint32_t own, uint32_t* scan, int E) {
   const int e = threadIdx.x;
-  const int tiles = e < E ? (counts[e] + tile_rows - 1) / tile_rows : 0;
-  if (e < 256) scan[e] = tiles;
+  if (E <= 64) {
+    if (e < 64) {
+#pragma unroll
+      for (int m = 1; m < 64; m <<= 1) {
+        const uint32_t add = __shfl_up(own, m, 64);
+        own += e >= m ? add : 0;
+      }
+      if (e < E) scan[e] = own;
+    }
+    __syncthreads();
+    return;
+  }
+  if (e < 256) scan[e] = own;
   __syncthreads();
   for (int m = 1; m < 256; m <<= 1) {
-    const int add = e < 256 && e >= m ? scan[e - m] : 0;
+    const uint32_t add = e < 256 && e >= m ? scan[e - m] : 0;
     __syncthreads();
     if (e < 256) scan[e] += add;
     __syncthreads();
   }
+}
+
+// Tiles of every expert from its count (of each its expert, 8 bits, and its rows), by threads 0 .. 255; scan: 256 ints of LDS.  Called by a whole workgroup.
+__device__ __forceinline__ void plan_tiles(const int* counts, uint32_t* scan, int* first_of, int32_t* tile_first, int32_t* tile_expert, int E, int tile_rows) {
+  const int e = threadIdx.x;
+  const int tiles = e < E ? (counts[e] + tile_rows - 1) / tile_rows : 0;
+  sum_up((uint32_t)tiles, scan, E);
   if (e < E) {
-    const int first = scan[e] - tiles;
+    const int first = (int)scan[e] - tiles;
     first_of[e] = first;
-    tile_first[e] = first;
+    if (tile_first != nullptr) tile_first[e] = first;
     if (tile_expert != nullptr)
       for (int t = 0; t < tiles; ++t) {
         const int left = counts[e] - t * tile_rows;
         tile_expert[first + t] = e | (left < tile_rows ? left : tile_rows) << 8;
       }
   }
-  if (e == 255) tile_first[E] = scan[255];
+  if (e == 0 && tile_first != nullptr) tile_first[E] = (int)scan[E - 1];
   __syncthreads();
 }
 
@@ -75,7 +93,8 @@ template <typename T, int ET, int NW, bool SPLIT, int TT>
 __global__ __launch_bounds__(64 * NW) void expert_route_kernel(const RouteArgs a) {
   constexpr int NT = 64 * NW, TOK = ET == 0 ? 16 : SPLIT ? 16 * TT : 16 * NW;
   extern __shared__ float logits[];  // [NW (SPLIT) or 1][TOK][E]
-  __shared__ int hist[kMaxExperts], base[kMaxExperts], scan[256];
+  __shared__ int hist[kMaxExperts], base[kMaxExperts];
+  __shared__ uint32_t scan[256];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4;
   const long n0 = (long)blockIdx.x * TOK;
   const int n = a.n - n0 < TOK ? (int)(a.n - n0) : TOK;
@@ -322,6 +341,30 @@ template <typename T> __global__ __launch_bounds__(512) void expert_route_row_ke
   }
 }
 
+// Tiles of BASED_EXPERT_TILE_ROWS rows: whole ones first, by expert, then what is left of every expert, the most rows first, so that the last to be
+// worked on are the smallest.  first_of: an expert's first whole tile; rest_of: the tile of what is left.  tile_first[0] is the number of whole ones.
+__device__ __forceinline__ void plan_large_tiles(const int* counts, uint32_t* scan, int* first_of, int* rest_of, int32_t* tile_first, int32_t* tile_expert, int E) {
+  constexpr int ROWS = BASED_EXPERT_TILE_ROWS;
+  const int e = threadIdx.x;
+  const int count = e < E ? counts[e] : 0, whole = count / ROWS, rest = count % ROWS;
+  sum_up((uint32_t)whole << 9 | (rest > 0), scan, E);  // whole tiles (less than 2^23) and rests (up to 256) at once
+  const int wholes = (int)(scan[E - 1] >> 9), rests = (int)(scan[E - 1] & 511);
+  if (e < E) {
+    const int first = (int)(scan[e] >> 9) - whole;
+    int rank = 0;
+#pragma unroll 8
+    for (int o = 0; o < E; ++o) rank += (counts[o] % ROWS << 8 | (255 - o)) > (rest << 8 | (255 - e));
+    first_of[e] = first;
+    rest_of[e] = wholes + rank;
+    if (tile_expert != nullptr) {
+      for (int t = 0; t < whole; ++t) tile_expert[first + t] = e | ROWS << 8;
+      if (rest > 0) tile_expert[wholes + rank] = e | rest << 8;
+    }
+  }
+  if (e == 0 && tile_expert != nullptr) tile_first[0] = wholes, tile_first[E] = wholes + rests;
+  __syncthreads();
+}
+
 constexpr int kPlaceThreads = 512, kPlaceGroups = 8;  // of the routing's workgroups, that one places
 constexpr long kPlaceHist = 1 << 15;                  // entries of hist up to which every workgroup may read all of it
 
@@ -337,15 +380,24 @@ struct PlaceArgs {
   int E, tile_rows, groups, group_slots;
 };
 
-// Workgroup i places the choices of groups kPlaceGroups i ..; each of them plans the tiles for itself, which is less than another launch.
+// Workgroup i places the choices of groups kPlaceGroups i ..; each of them plans the tiles for itself, which is less than another launch.  Bound by the
+// loads that wait for each other, so choices and own counts are asked for in front.  8192 tokens, 2 of 8 experts: 4.7 us; group after
+// group, and the tiles summed up by a whole workgroup, 7.2.
 __global__ __launch_bounds__(kPlaceThreads) void expert_place_kernel(const PlaceArgs a) {
-  __shared__ int scan[256], first_of[kMaxExperts], total[kMaxExperts], base[kPlaceGroups][kMaxExperts];
-  __shared__ int32_t unused[kMaxExperts + 1];
+  __shared__ uint32_t scan[256];
+  __shared__ int first_of[kMaxExperts], rest_of[kMaxExperts], total[kMaxExperts], base[kPlaceGroups][kMaxExperts];
   const int tid = threadIdx.x, g0 = blockIdx.x * kPlaceGroups;
   const int mine = a.groups - g0 < kPlaceGroups ? a.groups - g0 : kPlaceGroups;
-  for (int e = tid; e < a.E; e += kPlaceThreads) {
-    total[e] = a.hist != nullptr ? 0 : a.counts[e];
-    for (int g = 0; g < kPlaceGroups; ++g) base[g][e] = 0;
+  const long s0 = (long)g0 * a.group_slots;
+  const int n = a.slots - s0 < (long)mine * a.group_slots ? (int)(a.slots - s0) : mine * a.group_slots;
+  int id0 = 0, rank0 = 0, own[kPlaceGroups];
+  if (tid < n) id0 = a.ids[s0 + tid], rank0 = a.rank[s0 + tid];
+  static_assert(kMaxExperts <= kPlaceThreads, "");
+#pragma unroll
+  for (int g = 0; g < kPlaceGroups; ++g) own[g] = a.hist != nullptr && tid < a.E && g < mine ? a.hist[(long)(g0 + g) * a.E + tid] : 0;
+  if (tid < a.E) {
+    total[tid] = a.hist != nullptr ? 0 : a.counts[tid];
+    base[0][tid] = 0;
   }
   __syncthreads();
   if (a.hist != nullptr) {
@@ -364,31 +416,25 @@ __global__ __launch_bounds__(kPlaceThreads) void expert_place_kernel(const Place
       if (before != 0) atomicAdd(&base[0][e], before);
     }
     __syncthreads();
-    for (int x = tid; x < a.E; x += kPlaceThreads) {
-      int c[kPlaceGroups], at = base[0][x];
+  }
+  if (tid < a.E) {
+    int at = base[0][tid];
 #pragma unroll
-      for (int g = 0; g < kPlaceGroups; ++g) c[g] = g < mine ? a.hist[(long)(g0 + g) * a.E + x] : 0;
-#pragma unroll
-      for (int g = 0; g < kPlaceGroups; ++g) {
-        base[g][x] = at;
-        at += c[g];
-      }
+    for (int g = 0; g < kPlaceGroups; ++g) {
+      base[g][tid] = at;
+      at += own[g];
     }
   }
-  if (blockIdx.x == 0) {
-    plan_tiles(total, scan, first_of, a.tile_first, a.tile_expert, a.E, a.tile_rows);
-    if (a.hist != nullptr)
-      for (int e = tid; e < a.E; e += kPlaceThreads) a.counts[e] = total[e];
-  } else {
-    plan_tiles(total, scan, first_of, unused, nullptr, a.E, a.tile_rows);
-  }
-  for (int g = 0; g < mine; ++g) {
-    const long s0 = (long)(g0 + g) * a.group_slots;
-    const int n = a.slots - s0 < a.group_slots ? (int)(a.slots - s0) : a.group_slots;
-    for (int i = tid; i < n; i += kPlaceThreads) {
-      const int e = a.ids[s0 + i];
-      a.order[(long)first_of[e] * a.tile_rows + base[g][e] + a.rank[s0 + i]] = (int32_t)(s0 + i);
-    }
+  const bool large = a.tile_rows == BASED_EXPERT_TILE_ROWS, writes = blockIdx.x == 0;
+  if (large)
+    plan_large_tiles(total, scan, first_of, rest_of, a.tile_first, writes ? a.tile_expert : nullptr, a.E);
+  else
+    plan_tiles(total, scan, first_of, writes ? a.tile_first : nullptr, writes ? a.tile_expert : nullptr, a.E, a.tile_rows);
+  if (writes && a.hist != nullptr && tid < a.E) a.counts[tid] = total[tid];
+  for (int i = tid; i < n; i += kPlaceThreads) {
+    const int e = i < kPlaceThreads ? id0 : a.ids[s0 + i], r = base[i / a.group_slots][e] + (i < kPlaceThreads ? rank0 : a.rank[s0 + i]);
+    const bool rest = large && r >= total[e] / BASED_EXPERT_TILE_ROWS * BASED_EXPERT_TILE_ROWS;
+    a.order[rest ? (long)rest_of[e] * BASED_EXPERT_TILE_ROWS + r % BASED_EXPERT_TILE_ROWS : (long)first_of[e] * a.tile_rows + r] = (int32_t)(s0 + i);
   }
 }
 
@@ -543,16 +589,19 @@ template <bool PAIRED> __global__ __launch_bounds__(256, 2) void expert_gemm_ker
 }
 
 // ---- the same with tiles of 256 rows and 256 rows of the weights (PAIRED: 128 up, 128 gate), rows and weights straight into LDS ----
-// One workgroup of eight wavefronts to a compute unit.  Tiles are dealt to the dies in runs; what is left of a die's run after whole rounds
-// of its compute units goes in parts of 128 or 64 rows where that gives every part a compute unit of its own.
-// 8192 tokens of 1024 channels, 2 of 8 experts of 1024: 77 + 48 us (tiles of 128 x 256 through registers, two workgroups to a compute
-// unit: 106 + 70); without parts 93 + 64.  A whole tile alone takes 29 us: its matrix instructions 22, at the rate that they reach by
+// One workgroup of eight wavefronts to a compute unit.  Whole tiles are dealt to the dies in runs, the rests of the experts behind them, the smallest
+// last; what is left of a die's tiles after whole rounds of its compute units goes in parts, of 64 rows that are there and, where that gives every
+// part a compute unit of its own, of 128 or 64 rows of the weights.  8192 tokens of 1024 channels, 2 of 8 experts of 1024: 70 + 43 us (rests in
+// their experts' places, and parts of rows alone: 77 + 48; tiles of 128 x 256 through registers, two workgroups to a compute unit: 106 + 70);
+// 2048 rows to every expert, whole rounds alone, 65 + 39.  Calls, us, before and now: 8192 tokens 143 -> 130, 1000 49 -> 45, 500 41 -> 35;
+// 1 of 8 of 2048, 1000 53 -> 44; 4 of 16 of 512, 2000 69 -> 67.  A whole tile alone takes 29 us: its matrix instructions 22, at the rate that they reach by
 // themselves here (1.6 PFLOP/s), the rest in front of the first and behind the last.
 constexpr int kLargeRows = BASED_EXPERT_TILE_ROWS;
 constexpr int kDies = 8, kDieUnits = 32;
 constexpr int kHalf = 128 * kGemmK;  // elements of 128 rows of a round
-constexpr int kPartSlot = 3 * kHalf, kPartDepth = 3;
-constexpr int kLargeLds = kPartDepth * kPartSlot * 2 + kLargeRows * 4;  // bytes; whole tiles use 8 kHalf of the elements
+constexpr int kMaxParts = 16;
+constexpr int kPartElements = 9 * kHalf;
+constexpr int kLargeLds = kPartElements * 2 + 2 * kLargeRows * 4;  // bytes; whole tiles use 8 kHalf of the elements; choices and their scores behind them
 
 struct ExpertTile {
   const __bf16* w;  // matrices of the tile's expert
@@ -570,15 +619,18 @@ template <bool TAIL> __device__ __forceinline__ void load_to_lds(const __bf16* s
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
 }
 
-// the weights' row (of the expert's matrices) behind row r of a tile's 256
-template <bool PAIRED> __device__ __forceinline__ uint32_t large_w_row(const ExpertGemmArgs& a, int f0, int r) {
-  const int f = f0 + (PAIRED ? r & 127 : r);
-  return (uint32_t)((PAIRED && r >= 128 ? a.F : 0) + (f < a.F ? f : a.F - 1));
+// the weights' row (of the expert's matrices) behind row r of CW
+template <bool PAIRED, int CW = 256> __device__ __forceinline__ uint32_t large_w_row(const ExpertGemmArgs& a, int f0, int r) {
+  const int f = f0 + (PAIRED ? r % (CW / 2) : r);
+  return (uint32_t)((PAIRED && r >= CW / 2 ? a.F : 0) + (f < a.F ? f : a.F - 1));
 }
 
 template <bool PAIRED> __device__ __forceinline__ const __bf16* large_x_row(const ExpertGemmArgs& a, const ExpertTile& t, const int* slot_of, int r) {
   return a.x + (PAIRED ? (long)(slot_of[r] / a.top) * a.x_sr : (t.first + (r < t.rows ? r : 0)) * a.x_sr);
 }
+
+// scores of a tile's rows (PAIRED), in LDS behind their choices
+__device__ __forceinline__ const float* large_scores(const int* slot_of) { return reinterpret_cast<const float*>(slot_of + kLargeRows); }
 
 // four features of one row from their sums u (PAIRED: of up, and g of gate)
 template <bool PAIRED> __device__ __forceinline__ void large_store(const ExpertGemmArgs& a, __bf16* y, int f, float score, f32x4 u, f32x4 g) {
@@ -741,8 +793,9 @@ __device__ __forceinline__ void large_whole_tile(const ExpertGemmArgs& a, const 
   for (int h = 0; h < 2; ++h)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      slot[h][j] = slot_of[h * 128 + wm * 64 + j * 16 + l16];
-      score[h][j] = PAIRED ? a.scores[slot[h][j]] : 1.f;
+      const int r = h * 128 + wm * 64 + j * 16 + l16;
+      slot[h][j] = slot_of[r];
+      score[h][j] = PAIRED ? large_scores(slot_of)[r] : 1.f;
     }
 #pragma unroll
   for (int h = 0; h < 2; ++h)
@@ -760,13 +813,16 @@ __device__ __forceinline__ void large_whole_tile(const ExpertGemmArgs& a, const 
     }
 }
 
-// R rows from row r0 of a tile on, three rounds of 64 channels in LDS of which two are on their way; a wavefront has all of the rows and 32 rows
-// of the weights.
-template <int R, bool PAIRED, bool TAIL>
-__device__ __forceinline__ void large_part(const ExpertGemmArgs& a, const ExpertTile& t, __bf16* lds, const int* slot_of, int r0) {
-  constexpr int KS = kGemmK, XL = R / 64, WL = 4, MT = R / 16;
+// R rows from row r0 of a tile on and part `col` of CW of its 256 rows of the weights, as many rounds of 64 channels on their way as LDS holds; a
+// wavefront has 32 rows of the weights and as many of the rows as there are wavefronts to the same weights.
+template <int R, int CW, bool PAIRED, bool TAIL>
+__device__ __forceinline__ void large_part(const ExpertGemmArgs& a, const ExpertTile& t, __bf16* lds, const int* slot_of, int r0, int col) {
+  constexpr int KS = kGemmK, XL = R / 64, WL = CW / 64, WN = CW / 32, RW = R * WN / 8, MT = RW / 16, COLS = PAIRED ? CW / 2 : CW;
+  constexpr int SLOT = (CW + R) * KS, DEPTH = kPartElements / SLOT, FLYING = (DEPTH - 2) * (XL + WL);
+  static_assert(DEPTH >= 3 && FLYING < 16 && MT >= 1, "");
   if (r0 >= t.rows) return;  // (no barrier left)
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, quad = lane >> 4;
+  const int wn = wave % WN, wm = wave / WN, f0 = t.f0 + col * COLS;
   const int piece = (lane ^ (lane >> 4)) & 7;  // (rows of an odd group of eight: bit 2 the other way round)
   const __bf16* xrow[XL];
   uint32_t wrow[WL];  // bytes
@@ -778,11 +834,11 @@ __device__ __forceinline__ void large_part(const ExpertGemmArgs& a, const Expert
 #pragma unroll
   for (int i = 0; i < WL; ++i) {
     const int r = (wave * WL + i) * 8 + (lane >> 3);
-    wrow[i] = (large_w_row<PAIRED>(a, t.f0, r) * (uint32_t)a.K + (uint32_t)((piece ^ (r >> 1 & 4)) * 8)) * 2u;
+    wrow[i] = (large_w_row<PAIRED, CW>(a, f0, r) * (uint32_t)a.K + (uint32_t)((piece ^ (r >> 1 & 4)) * 8)) * 2u;
   }
   const int rounds = (a.K + KS - 1) / KS;
   auto ask = [&](int at_round, int place) {
-    __bf16* at = lds + place * kPartSlot;  // 256 rows of the weights, then the rows
+    __bf16* at = lds + place * SLOT;  // rows of the weights, then the rows
     const int round = at_round < rounds ? at_round : 0;  // (asked for and never read)
 #pragma unroll
     for (int i = 0; i < WL; ++i)
@@ -790,7 +846,7 @@ __device__ __forceinline__ void large_part(const ExpertGemmArgs& a, const Expert
                         round * KS + (piece ^ ((wave * WL + i) * 4 & 4)) * 8, a.K);
 #pragma unroll
     for (int i = 0; i < XL; ++i)
-      load_to_lds<TAIL>(xrow[i] + round * KS, at + 2 * kHalf + (wave * XL + i) * 8 * KS, round * KS + (piece ^ ((wave * XL + i) * 4 & 4)) * 8, a.K);
+      load_to_lds<TAIL>(xrow[i] + round * KS, at + CW * KS + (wave * XL + i) * 8 * KS, round * KS + (piece ^ ((wave * XL + i) * 4 & 4)) * 8, a.K);
   };
   f32x4 acc[2][MT];
 #pragma unroll
@@ -798,68 +854,79 @@ __device__ __forceinline__ void large_part(const ExpertGemmArgs& a, const Expert
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int turned = (l16 >> 1) & 7;
-  ask(0, 0);
-  ask(1, 1);
+  for (int i = 0; i < DEPTH - 1; ++i) ask(i, i);
   for (int round = 0, place = 0; round < rounds; ++round) {
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(0x0070 | (XL + WL));  // own reads are done, and all loads but those of the next round
+    __builtin_amdgcn_s_waitcnt(0x0070 | FLYING);  // own reads are done, and all loads but those of the rounds behind
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    ask(round + 2, place == 0 ? 2 : place - 1);
+    ask(round + DEPTH - 1, place == 0 ? DEPTH - 1 : place - 1);
     __builtin_amdgcn_sched_barrier(0);
-    const __bf16* at = lds + place * kPartSlot + l16 * KS;
+    const __bf16* at = lds + place * SLOT + l16 * KS;
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
       const int p = ((kk * 4 + quad) ^ turned) * 8;
       bf16x8 w[2];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) w[i] = *reinterpret_cast<const bf16x8*>(at + (PAIRED ? i * 128 + wave * 16 : wave * 32 + i * 16) * KS + p);
+      for (int i = 0; i < 2; ++i) w[i] = *reinterpret_cast<const bf16x8*>(at + (PAIRED ? i * COLS + wn * 16 : wn * 32 + i * 16) * KS + p);
 #pragma unroll
       for (int j = 0; j < MT; ++j) {
-        const bf16x8 x = *reinterpret_cast<const bf16x8*>(at + 2 * kHalf + j * 16 * KS + p);
+        const bf16x8 x = *reinterpret_cast<const bf16x8*>(at + (CW + wm * RW + j * 16) * KS + p);
 #pragma unroll
         for (int i = 0; i < 2; ++i) acc[i][j] = expert_mfma(w[i], x, acc[i][j]);
       }
     }
-    place = place == 2 ? 0 : place + 1;
+    place = place == DEPTH - 1 ? 0 : place + 1;
   }
   __builtin_amdgcn_s_waitcnt(0x0070);
   int slot[MT];
   float score[MT];
 #pragma unroll
   for (int j = 0; j < MT; ++j) {
-    slot[j] = slot_of[r0 + j * 16 + l16];
-    score[j] = PAIRED ? a.scores[slot[j]] : 1.f;
+    const int r = r0 + wm * RW + j * 16 + l16;
+    slot[j] = slot_of[r];
+    score[j] = PAIRED ? large_scores(slot_of)[r] : 1.f;
   }
 #pragma unroll
   for (int j = 0; j < MT; ++j) {
-    const int r = r0 + j * 16 + l16;
+    const int r = r0 + wm * RW + j * 16 + l16;
     if (r >= t.rows) continue;
     __bf16* y = a.y + (PAIRED ? t.first + r : (long)slot[j]) * a.F;
-    const int f = t.f0 + wave * (PAIRED ? 16 : 32) + quad * 4;
+    const int f = f0 + wn * (PAIRED ? 16 : 32) + quad * 4;
     large_store<PAIRED>(a, y, f, score[j], acc[0][j], acc[1][j]);
     if constexpr (!PAIRED) large_store<PAIRED>(a, y, f + 16, score[j], acc[1][j], acc[0][j]);
   }
 }
 
-// TAIL: the last round of channels is no whole one.  Block i is number i / 8 of die i % 8.
+// TAIL: the last round of channels is no whole one.  Block i is number i / 8 of die i % 8.  A die has a run of the whole tiles and, behind it, every
+// eighth of the rests, which differ least between the dies that way.
 template <bool PAIRED, bool TAIL> __global__ __launch_bounds__(512, 2) void expert_gemm_large_kernel(const ExpertGemmArgs a) {
   extern __shared__ __attribute__((aligned(16))) __bf16 lds[];
-  int* slot_of = reinterpret_cast<int*>(lds + kPartDepth * kPartSlot);
-  const int row_tiles = a.tile_first[a.E], all = row_tiles * a.col_tiles;
-  const int die = blockIdx.x % kDies, k = blockIdx.x / kDies, more = all % kDies;
-  const int first = die * (all / kDies) + (die < more ? die : more), mine = all / kDies + (die < more ? 1 : 0);
-  const int whole = mine / kDieUnits * kDieUnits, left = mine - whole;
-  const int parts = left * 4 <= kDieUnits ? 4 : left * 2 <= kDieUnits ? 2 : 1;
-  if (k >= whole + left * parts) return;
-  const int id = first + (k < whole ? k : whole + (k - whole) / parts), part = k < whole ? 0 : (k - whole) % parts;
-  // bands of kBand row tiles, walked down the rows first: what is in flight on a die shares its rows and its matrices
-  const int band = id / (kBand * a.col_tiles), in_band = id % (kBand * a.col_tiles);
-  const int deep = row_tiles - band * kBand < kBand ? row_tiles - band * kBand : kBand;
-  const int tile = band * kBand + in_band % deep, tid = threadIdx.x;
+  int* slot_of = reinterpret_cast<int*>(lds + kPartElements);
+  const int wholes = a.tile_first[0], full = wholes * a.col_tiles, rests = (a.tile_first[a.E] - wholes) * a.col_tiles;
+  const int die = blockIdx.x % kDies, k = blockIdx.x / kDies, more = full % kDies, turn = (die - more) & (kDies - 1);
+  const int first = die * (full / kDies) + (die < more ? die : more), mine_full = full / kDies + (die < more ? 1 : 0);
+  const int mine = mine_full + rests / kDies + (turn < rests % kDies ? 1 : 0);
+  const int in_rounds = mine / kDieUnits * kDieUnits, left = mine - in_rounds;
+  int parts = 1;
+  while (parts < kMaxParts && left * parts * 2 <= kDieUnits) parts *= 2;
+  if (k >= in_rounds + left * parts) return;
+  const int item = k < in_rounds ? k : in_rounds + (k - in_rounds) / parts, part = k < in_rounds ? 0 : (k - in_rounds) % parts;
+  if (k < in_rounds) parts = 1;
+  const int tid = threadIdx.x;
+  int tile, column;
+  if (item < mine_full) {
+    // bands of kBand row tiles, walked down the rows first: what is in flight on a die shares its rows and its matrices
+    const int id = first + item, band = id / (kBand * a.col_tiles), in_band = id % (kBand * a.col_tiles);
+    const int deep = wholes - band * kBand < kBand ? wholes - band * kBand : kBand;
+    tile = band * kBand + in_band % deep, column = in_band / deep;
+  } else {
+    const int id = (item - mine_full) * kDies + turn;
+    tile = wholes + id / a.col_tiles, column = id % a.col_tiles;
+  }
   ExpertTile t;
   t.first = (long)tile * kLargeRows;
-  t.f0 = in_band / deep * (PAIRED ? 128 : 256);
+  t.f0 = column * (PAIRED ? 128 : 256);
   // what the tile is and which choices it has, asked for together (one after the other, by way of the expert's count and first tile,
   // 700 tokens, 2 of 8 experts of 1024, 42.5 us a call: 42.0)
   const int what = a.tile_expert[tile];
@@ -870,9 +937,19 @@ template <bool PAIRED, bool TAIL> __global__ __launch_bounds__(512, 2) void expe
   __syncthreads();
   if (tid >= t.rows && tid < kLargeRows) slot_of[tid] = slot_of[0];  // (rows that nobody has put in order)
   __syncthreads();
-  if (k >= whole && parts == 4) return large_part<64, PAIRED, TAIL>(a, t, lds, slot_of, part * 64);
-  if (k >= whole && parts == 2) return large_part<128, PAIRED, TAIL>(a, t, lds, slot_of, part * 128);
-  large_whole_tile<PAIRED, TAIL>(a, t, lds, slot_of);
+  if (PAIRED && tid < kLargeRows)  // (in front of all other loads, so that they are there behind the first wait of the wavefront)
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(a.scores + slot_of[tid]),
+                                     (__attribute__((address_space(3))) void*)(slot_of + kLargeRows + (tid & ~63)), 4, 0, 0);
+  // blocks of 64 rows first (of 128 where there are no parts for that), then parts of the weights
+  const int rows = t.rows <= 64 ? 1 : t.rows <= 128 ? 2 : 4;
+  if (parts < rows) {
+    if (parts == 2 || rows == 2) return large_part<128, 256, PAIRED, TAIL>(a, t, lds, slot_of, part * 128, 0);
+    return large_whole_tile<PAIRED, TAIL>(a, t, lds, slot_of);
+  }
+  const int r0 = part % rows * 64, col = part / rows;
+  if (parts / rows == 1) return large_part<64, 256, PAIRED, TAIL>(a, t, lds, slot_of, r0, 0);
+  if (parts / rows == 2) return large_part<64, 128, PAIRED, TAIL>(a, t, lds, slot_of, r0, col);
+  if (col < 4) large_part<64, 64, PAIRED, TAIL>(a, t, lds, slot_of, r0, col);
 }
 
 // The same tiles of 32 rows with 64 rows of the weights (PAIRED: 32 up, 32 gate), rows and weights straight into LDS, rounds of 128 channels three

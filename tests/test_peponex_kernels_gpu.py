@@ -589,6 +589,26 @@ def test_experts_in_large_tiles(dev, n, D, F, E, top):
     close(got[clear], want[clear], 2 * TOL[BF16])
 
 
+@pytest.mark.parametrize("counts,D,F", [([382, 65, 1, 320], 1024, 1152), ([255, 129], 264, 3912), ([2504, 2916, 0, 64, 3], 128, 128),
+                                        ([2049, 2112, 2113, 2176, 2177, 2303, 2048, 2078], 256, 1024), ([200, 100, 60, 40] * 8, 512, 1024),
+                                        ([200, 100, 60, 40] * 8, 520, 1000)])
+def test_rests_of_large_tiles(dev, counts, D, F):
+    """What whole tiles of 256 rows leave of every expert: 1, 64, 65, 128, 129 and 255 rows, none, in the last places of a die cut into sixteen parts
+    of rows and weights, eight, four, two, and in places of whole tiles; an expert that nobody chooses; features and channels that end in a part."""
+    from based_amd import _lib, ops
+
+    n, E = sum(counts), len(counts)
+    assert _lib.lib().based_expert_tile_rows(n, E, 1) == 256
+    h, router, w1, w2, w = expert_case(n, D, F, E, 1, BF16, seed=n)
+    router = (0.3 * torch.eye(E, D)).to(BF16)  # channel e is what expert e is chosen for
+    own = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(n, generator=torch.Generator().manual_seed(n))]
+    h[:, :E] = (0.1 * h[:, :E].float() + 8.0 * torch.nn.functional.one_hot(own, E)).to(BF16)
+    w["m.router"] = router.double()
+    want = O.expert_mlp(h.double(), w, "m", {"router": {"top": 1}})
+    got = ops.experts(h.to(dev), router.to(dev), w1.to(dev), w2.to(dev), 1).double().cpu()
+    close(got, want, 2 * TOL[BF16])
+
+
 @pytest.mark.parametrize("n,E,top", [(33, 8, 1), (4095, 8, 2), (4096, 32, 2), (4097, 8, 2), (4100, 33, 2), (4223, 70, 4), (5000, 130, 3), (20000, 64, 2), (40000, 128, 1), (32767, 8, 2), (32768, 8, 2), (33000, 30, 1)])
 def test_places_of_the_choices(dev, n, E, top):
     """Every choice of a batch goes to the same expert as in batches of few tokens, whose places one workgroup plans: by the workgroups' counts (n E up
