@@ -5,7 +5,7 @@
 // sum of the latents is formed once per head, and uv_h is applied to that sum.
 //
 //   latent_write   norm and rotation of a portion's rows, into the cache
-//   latent_query   one token per sequence: q~ and the rotated q of every head, and the token's cache row
+//   latent_query   one token per sequence: q~ and the rotated q of every head, and the token's cache row (of few sequences in bf16 latent_step does it)
 //   latent_step    scores, softmax and weighted latents, the keys of a sequence dealt to several workgroups
 //   latent_values  their partial results put together, times uv
 // The first and the last have a form on MFMA for 16 sequences at a time.
@@ -324,7 +324,10 @@ __global__ __launch_bounds__(256) void latent_step_any_kernel(const LatentArgs a
 // bf16, MFMA: 16 heads per workgroup, 64 keys at a time; a wavefront forms the scores of 16 of them and a
 // quarter of the weighted latents.  KC: 32-channel pieces of a row (rounded up); RT: 16-channel tiles of the latent per
 // wavefront (rounded up).  R and rot multiples of 8.
-template <int KC, int RT>
+// OWN > 0: OWN heads per workgroup and at most 64 keys, and no launch in front: the workgroup forms its queries while its keys are on their way, and,
+// where the token's own row is among the keys, that row, which the workgroup of the first heads leaves in the cache.  uk is read by every
+// workgroup of its heads, so that this is the way of few sequences, whose time is waiting: what needs no position is asked for in front of it.
+template <int KC, int RT, int OWN>
 __global__ __launch_bounds__(256, 1) void latent_step_mfma_kernel(const LatentArgs a) {
   constexpr int KS = 64 + 8;  // keys per LDS row
   constexpr int RMAX = RT * 64;
@@ -332,14 +335,41 @@ __global__ __launch_bounds__(256, 1) void latent_step_mfma_kernel(const LatentAr
   __shared__ __attribute__((aligned(16))) __bf16 ps[16 * KS];    // [head][key]
   __shared__ float wmax[4][16], wsum[4][16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4, W = a.R + a.rot;
-  const int b = blockIdx.x, split = blockIdx.y, h0 = blockIdx.z * 16;
+  const int b = blockIdx.x, split = blockIdx.y, h0 = blockIdx.z * (OWN > 0 ? OWN : 16);
+  // OWN: 8 latent channels to a thread, rows of uk dealt to the groups, DU of each head in flight; asked for before the position is known
+  constexpr int HEADS = OWN > 0 ? OWN : 1, PIECES = RT * 8, GROUPS = 256 / PIECES, DU = 16 / HEADS;
+  const int col = tid % PIECES * 8, grp = tid / PIECES, per_head = a.rot + a.d, heads = a.H - h0 < HEADS ? a.H - h0 : HEADS;
+  bf16x8 uk[HEADS][DU], own_x, own_norm;
+  float own_q[HEADS * GROUPS * DU / 256 > 0 ? HEADS * GROUPS * DU / 256 : 1];
+  const __bf16* q_in = static_cast<const __bf16*>(a.q) + b * a.q_sb + (long)h0 * per_head;
+  auto ask_heads = [&](int d0) {
+#pragma unroll
+    for (int h = 0; h < HEADS; ++h)
+#pragma unroll
+      for (int u = 0; u < DU; ++u) {
+        const int d = d0 + u * GROUPS + grp;
+        uk[h][u] = *reinterpret_cast<const bf16x8*>(static_cast<const __bf16*>(a.w) + (col < a.R ? col : 0) +
+                                                    ((long)(h < heads ? h0 + h : h0) * (per_head + a.dv) + a.rot + (d < a.d ? d : 0)) * a.w_sr);
+      }
+#pragma unroll
+    for (int i = 0; i * 256 < HEADS * GROUPS * DU; ++i) {
+      const int at = i * 256 + tid, h = at / (GROUPS * DU), d = d0 + at % (GROUPS * DU);
+      own_q[i] = h < heads && d < a.d ? to_f32(q_in[h * per_head + a.rot + d]) : 0.f;
+    }
+  };
+  if constexpr (OWN > 0) {
+    ask_heads(0);
+    own_x = *reinterpret_cast<const bf16x8*>(static_cast<const __bf16*>(a.x) + b * a.x_sb + (lane * 8 < a.R ? lane * 8 : 0));
+    own_norm = *reinterpret_cast<const bf16x8*>(static_cast<const __bf16*>(a.norm_w) + (lane * 8 < a.R ? lane * 8 : 0));
+  }
   const int pos = row_pos(a.pos, a.pos_host, b);
   if (pos < 0 || pos >= a.S) return;
   int first, n;
   split_range(a, pos, split, first, n);
+  if (OWN > 0 && a.rot > 0 && pos >= a.n_pos) n = 0;  // (no angles: no row and no queries)
   const __bf16* cache = static_cast<const __bf16*>(a.cache) + b * a.c_sb + (long)first * a.c_st;
   const long at = ((long)b * a.splits + split) * a.H + h0 + l16;  // of this lane's head
-  const bool head_in = h0 + l16 < a.H;
+  const bool head_in = h0 + l16 < a.H && (OWN == 0 || l16 < OWN);
   if (n == 0) {
     if (head_in && tid < 16) a.part_ml[2 * at] = -INFINITY, a.part_ml[2 * at + 1] = 0.f;
     return;
@@ -367,16 +397,98 @@ __global__ __launch_bounds__(256, 1) void latent_step_mfma_kernel(const LatentAr
     }
   };
   fetch(0);
-  // queries of this lane's head, the score scale in them
+  // queries of this lane's head
   bf16x8 qf[KC];
-  const float* q = a.qa + ((long)b * a.H + (head_in ? h0 + l16 : 0)) * W;
+  if constexpr (OWN > 0) {
+    __shared__ float qs[OWN][GROUPS * DU];
+    __shared__ __attribute__((aligned(16))) float sums[GROUPS][OWN][RMAX];
+    __shared__ __attribute__((aligned(16))) __bf16 qt[OWN][KC * 32];
+    __shared__ __attribute__((aligned(16))) __bf16 row[KC * 32];
+    const bool own_row = first + n - 1 == pos;
+    float part[OWN][8];
 #pragma unroll
-  for (int c = 0; c < KC; ++c) {
-    const int e = c * 32 + quad * 8;
-    float x[8];
-    load_vec<float, 8>(q + (e < W ? e : 0), x);
+    for (int h = 0; h < OWN; ++h)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) qf[c][j] = (__bf16)(e < W ? x[j] : 0.f);
+      for (int j = 0; j < 8; ++j) part[h][j] = 0.f;
+    for (int d0 = 0; d0 < a.d; d0 += GROUPS * DU) {
+      if (d0 > 0) {
+        ask_heads(d0);
+        lds_barrier();
+      }
+#pragma unroll
+      for (int i = 0; i * 256 < OWN * GROUPS * DU; ++i)
+        if (i * 256 + tid < OWN * GROUPS * DU) qs[0][i * 256 + tid] = own_q[i];
+      lds_barrier();
+#pragma unroll
+      for (int h = 0; h < OWN; ++h)
+#pragma unroll
+        for (int u = 0; u < DU; ++u)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) part[h][j] = __builtin_fmaf(to_f32(uk[h][u][j]), qs[h][u * GROUPS + grp], part[h][j]);
+    }
+    if (own_row && wave == 0) {  // the token's row, 8 channels to a lane
+      float x[8], ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        x[j] = to_f32(own_x[j]);
+        ss = lane * 8 < a.R ? __builtin_fmaf(x[j], x[j], ss) : ss;
+      }
+      const float r = 1.0f / sqrtf(wave_sum(ss) / (float)a.R + a.eps);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] *= r * to_f32(own_norm[j]);
+      if (lane * 8 < a.R) store_vec<__bf16, 8>(&row[lane * 8], x);
+      for (int c = lane; c < a.rot; c += 64) row[a.R + c] = (__bf16)turned(static_cast<const __bf16*>(a.x) + b * a.x_sb + a.R, c, pos, a);
+    } else if (wave == 1 || wave == 2) {
+      for (int i = tid - 64; i < OWN * (KC * 32 - a.R); i += 128) {
+        const int h = i / (KC * 32 - a.R), c = i % (KC * 32 - a.R);
+        qt[h][a.R + c] = h < heads && c < a.rot ? (__bf16)turned(q_in + h * per_head, c, pos, a) : (__bf16)0.f;
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < OWN; ++h)
+#pragma unroll
+      for (int j = 0; j < 8; j += 4) *reinterpret_cast<f32x4*>(&sums[grp][h][col + j]) = f32x4{part[h][j], part[h][j + 1], part[h][j + 2], part[h][j + 3]};
+    lds_barrier();
+    for (int i = tid; i < OWN * RMAX; i += 256) {
+      const int h = i / RMAX, c = i % RMAX;
+      float x = 0.f;
+#pragma unroll
+      for (int g = 0; g < GROUPS; ++g) x += sums[g][h][c];
+      if (c < a.R) qt[h][c] = (__bf16)x;
+    }
+    if (own_row) {  // in place of the last key, and of what is asked for behind it
+      if (h0 == 0)
+        for (int c = tid; c < W; c += 256) static_cast<__bf16*>(a.cache)[b * a.c_sb + pos * a.c_st + c] = row[c];
+      if (wave * 16 + l16 >= n - 1)
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+          const int e = c * 32 + quad * 8;
+          kf[c] = *reinterpret_cast<const bf16x8*>(&row[e < W ? e : 0]);
+        }
+#pragma unroll
+      for (int i = 0; i < VU; ++i) {
+        const int p = i * 256 + tid, k4 = p & 15, e = (p >> 4) * 8;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (k4 * 4 + r >= n - 1) vf[i][r] = *reinterpret_cast<const u32x4*>(&row[e < a.R ? e : 0]);
+      }
+    }
+    lds_barrier();
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      const int e = c * 32 + quad * 8;
+      qf[c] = *reinterpret_cast<const bf16x8*>(&qt[head_in ? l16 : 0][e]);
+    }
+  } else {
+    const float* q = a.qa + ((long)b * a.H + (head_in ? h0 + l16 : 0)) * W;
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      const int e = c * 32 + quad * 8;
+      float x[8];
+      load_vec<float, 8>(q + (e < W ? e : 0), x);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) qf[c][j] = (__bf16)(e < W ? x[j] : 0.f);
+    }
   }
   const float scale2 = a.scale * 1.4426950408889634f;
   f32x4 acc[RT];
@@ -833,9 +945,18 @@ static int latent_check(const char* who, const LatentArgs& a, int64_t last, int 
   return BASED_OK;
 }
 
-template <int KC, int RT> void launch_latent_mfma(const LatentArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL((latent_step_mfma_kernel<KC, RT>), dim3((unsigned)a.B, (unsigned)a.splits, (unsigned)((a.H + 15) / 16)), dim3(256), 0,
-                     s, a);
+// Up to two workgroups to a compute unit.  Whole calls, us, with a launch for the queries and without, 16 heads, R = 256, by sequences and
+// keys (workgroups): 1, 129 (24): 16.2 / 12.2; 4, 512 (256): 16.9 / 13.2; 6, 512 (384): 17.1 / 15.1; 16, 129 (384): 16.0 / 14.2; 4, 1,024 (512): 18.0 /
+// 16.1; 24, 129 (576): 16.2 / 18.2; 12, 512 (768): 18.3 / 22.7.  Four heads to a workgroup take as long at 512 and 13.6 -> 14.8 at 256.
+constexpr int kOwnHeads = 2;
+constexpr int64_t kOwnMax = 512;
+
+template <int KC, int RT> void launch_latent_mfma(const LatentArgs& a, bool own, hipStream_t s) {
+  const auto grid = [&](int heads) { return dim3((unsigned)a.B, (unsigned)a.splits, (unsigned)((a.H + heads - 1) / heads)); };
+  if (own)
+    hipLaunchKernelGGL((latent_step_mfma_kernel<KC, RT, kOwnHeads>), grid(kOwnHeads), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((latent_step_mfma_kernel<KC, RT, 0>), grid(16), dim3(256), 0, s, a);
 }
 
 template <typename T> void launch_latent_query(const LatentArgs& a, bool vec, hipStream_t s) {
@@ -854,19 +975,18 @@ template <typename T> void launch_latent_values(const LatentArgs& a, bool vec, h
     hipLaunchKernelGGL((latent_values_kernel<T, 1>), grid, dim3(256), 0, s, a);
 }
 
-static bool launch_latent_step_mfma(const LatentArgs& a, hipStream_t s) {
+static bool latent_mfma_fits(const LatentArgs& a) { return (a.R + a.rot + 31) / 32 <= 18 && (a.R + 63) / 64 <= 8; }
+
+static void launch_latent_step_mfma(const LatentArgs& a, bool own, hipStream_t s) {
   const int kc = (a.R + a.rot + 31) / 32, rt = (a.R + 63) / 64;
   if (kc <= 3 && rt <= 1)
-    launch_latent_mfma<3, 1>(a, s);
+    launch_latent_mfma<3, 1>(a, own, s);
   else if (kc <= 5 && rt <= 2)
-    launch_latent_mfma<5, 2>(a, s);
+    launch_latent_mfma<5, 2>(a, own, s);
   else if (kc <= 10 && rt <= 4)
-    launch_latent_mfma<10, 4>(a, s);
-  else if (kc <= 18 && rt <= 8)
-    launch_latent_mfma<18, 8>(a, s);
+    launch_latent_mfma<10, 4>(a, own, s);
   else
-    return false;
-  return true;
+    launch_latent_mfma<18, 8>(a, own, s);
 }
 
 template <int KC, int RT> void launch_latent_f32(const LatentArgs& a, hipStream_t s) {
@@ -950,17 +1070,22 @@ extern "C" BASED_API int based_latent_step(const void* q, const void* x, const v
   const int n = io_dtype == BASED_BF16 ? 8 : 4;
   const bool vec = R % n == 0 && w_sr % n == 0 && aligned_to(weight, 16);
   const bool tiles = io_dtype == BASED_BF16 && vec && B >= kTileMinRows;
-  if (tiles && D % 8 == 0 && rot % 8 == 0 && q_sb % 8 == 0 && aligned_to(q, 16))
+  const bool near = io_dtype == BASED_BF16 || (c_st > 0 && S * c_st < (1ll << 30));  // (the fp32 form counts bytes of a sequence's cache in 32 bits)
+  const bool mfma = near && R % n == 0 && rot % n == 0 && c_sb % n == 0 && c_st % n == 0 && aligned_to(cache, 16) && aligned_to(work_q, 16) &&
+                    aligned_to(work_part, 16);
+  const bool mfma_bf16 = io_dtype == BASED_BF16 && mfma && latent_mfma_fits(a);
+  const bool own = mfma_bf16 && vec && x_sb % 8 == 0 && aligned_to(x, 16) && aligned_to(norm_w, 16) && (window < S ? window : S) <= 64 * splits && B * splits * ((H + kOwnHeads - 1) / kOwnHeads) <= kOwnMax;
+  if (own) {
+  } else if (tiles && D % 8 == 0 && rot % 8 == 0 && q_sb % 8 == 0 && aligned_to(q, 16))
     hipLaunchKernelGGL(latent_query_mfma_kernel, dim3((unsigned)(H * ((R + kQueryCols - 1) / kQueryCols) + kTileRows),
                        (unsigned)((B + kTileRows - 1) / kTileRows)), dim3(256), 0, s, a);
   else if (io_dtype == BASED_BF16)
     launch_latent_query<__bf16>(a, vec, s);
   else
     launch_latent_query<float>(a, vec, s);
-  const bool near = io_dtype == BASED_BF16 || (c_st > 0 && S * c_st < (1ll << 30));  // (the fp32 form counts bytes of a sequence's cache in 32 bits)
-  const bool mfma = near && R % n == 0 && rot % n == 0 && c_sb % n == 0 && c_st % n == 0 && aligned_to(cache, 16) && aligned_to(work_q, 16) &&
-                    aligned_to(work_part, 16);
-  if (!mfma || !(io_dtype == BASED_BF16 ? launch_latent_step_mfma(a, s) : launch_latent_step_f32(a, s))) {
+  if (mfma_bf16) {
+    launch_latent_step_mfma(a, own, s);
+  } else if (io_dtype == BASED_BF16 || !mfma || !launch_latent_step_f32(a, s)) {
     const dim3 grid((unsigned)(B * H * splits));
     if (io_dtype == BASED_BF16)
       hipLaunchKernelGGL(latent_step_any_kernel<__bf16>, grid, dim3(256), 0, s, a);

@@ -426,6 +426,36 @@ def test_fp32_steps_on_the_matrix_unit(dev, H, d, r, dv, R, window, keys):
             close(o[b], want, 1e-5)
 
 
+@pytest.mark.parametrize("H,d,r,dv,R,window,keys", [
+    (16, 64, 32, 64, 256, 512, 700), (1, 8, 8, 8, 8, 1, 3), (3, 24, 8, 16, 64, 63, 200), (2, 20, 16, 8, 72, 64, 66), (5, 136, 0, 40, 136, 65, 90),
+    (4, 72, 64, 16, 248, 128, 300), (6, 264, 24, 24, 264, 200, 260), (3, 130, 64, 8, 512, 700, 800), (16, 16, 32, 16, 256, 1000, 500)])
+def test_steps_of_few_sequences_form_their_own_queries(dev, H, d, r, dv, R, window, keys):
+    """Against the launches one after the other, which take an input that is not in whole 16-byte pieces: an odd number of heads, head channels that
+    end inside a round of uk, no turned channels, the first and the last key of 64; the token's row, over what was no number, and rows without a place."""
+    from based_amd import ops
+
+    B, at = 4, [keys - 1, 0, keys // 2, -1]
+    q, x = rnd(B, H * (r + d), seed=1, dtype=BF16).to(dev), rnd(B, R + r, seed=2, dtype=BF16).to(dev)
+    nw, w = rnd(R, seed=3, dtype=BF16, scale=0.2, mean=1.0).to(dev), rnd(H * (r + d + dv), R, seed=4, dtype=BF16, scale=R ** -0.5).to(dev)
+    rows = rnd(B, keys, R + r, seed=5, dtype=BF16)
+    pos = torch.tensor(at, dtype=torch.int32, device=dev)
+    ang = torch.outer(torch.arange(keys, dtype=torch.float64), 500.0 ** (-torch.arange(0, r, 2, dtype=torch.float64) / max(r, 1)))
+    rope = (ang.cos().float().to(dev), ang.sin().float().to(dev), False) if r else None
+    out = []
+    for offset in (0, 1):
+        cache = torch.full((B, keys, R + r), float("nan"), dtype=BF16, device=dev)
+        for b, p in enumerate(at):
+            cache[b, :max(p, 0)] = rows[b, :max(p, 0)].to(dev)
+        moved = torch.empty(x.numel() + offset, dtype=BF16, device=dev)[offset:].view_as(x).copy_(x)
+        got = ops.latent_step(q, moved, nw, w, cache, H, d, window, 0.3, pos, 1e-5, rope, out=torch.empty(B, H * dv, dtype=BF16, device=dev))
+        out.append((got[:3], cache))
+    close(out[0][0], out[1][0].cpu(), TOL[BF16])
+    for b, p in enumerate(at[:3]):  # the same row, but for sums of squares in another order
+        close(out[0][1][b, p], out[1][1][b, p].cpu(), TOL[BF16])
+        assert torch.equal(out[0][1][b, :p], out[1][1][b, :p]) and bool(out[0][1][b, p + 1:].isnan().all())
+    assert bool(out[0][1][3].isnan().all())
+
+
 # ---- experts ----
 def expert_case(n, D, F, E, top, dtype, seed=0):
     h, router = rnd(n, D, seed=seed, dtype=dtype), rnd(E, D, seed=seed + 1, dtype=dtype, scale=2 * D ** -0.5)
