@@ -21,7 +21,7 @@
 // with the state for 128 channels.  The quotients of decays are exponentials of differences of log
 // decays: none of them overflows, and a decay of zero is zero.
 //   gated_delta_prepare  T, P, the decays and the norm factors of every block, all blocks at once, one
-//                        wavefront each; T by forward substitution (a power series in A would lose
+//                        wavefront each (of prompts of up to 64 tokens the scan does it); T by forward substitution (a power series in A would lose
 //                        digits to cancellation)
 //   gated_delta_scan     walks the blocks with the state in MFMA accumulators.  The accumulator layout
 //                        (column = lane % 16, rows 4 (lane / 16) + i) is the second operand of
@@ -54,16 +54,10 @@ struct DeltaArgs {
   int fresh, vec;
 };
 
+// What block blk of head h leaves in out, by one wavefront (s_a: LDS of its own; `live`: it is written).  Called by a whole workgroup.
 template <typename T, bool VEC>
-__global__ __launch_bounds__(256) void gated_delta_prepare_kernel(const DeltaArgs a) {
-  __shared__ __attribute__((aligned(16))) float s_a[4][kBlk][kBlk + 4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, quad = lane >> 4;
-  const long n_items = (long)a.B * a.H * a.blocks;
-  const long item0 = (long)blockIdx.x * 4 + wave;
-  const bool live = item0 < n_items;
-  const long item = live ? item0 : n_items - 1;
-  const int blk = (int)(item % a.blocks);
-  const int h = (int)(item / a.blocks % a.H), b = (int)(item / a.blocks / a.H), hk = h / (a.H / a.G);
+__device__ __forceinline__ void prepare_block(const DeltaArgs& a, int b, int h, int blk, bool live, float (&s_a)[kBlk][kBlk + 4], float* out) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4, hk = h / (a.H / a.G);
   const int t0 = blk * kBlk, tok = t0 + l16;
   const bool in = tok < a.L;
   const long row = in ? tok : a.L - 1;
@@ -109,14 +103,13 @@ __global__ __launch_bounds__(256) void gated_delta_prepare_kernel(const DeltaArg
     if (l16 >= m) lc += up;
   }
   const double lc_end = __shfl(lc, 15, 64);
-  float* out = a.prep + item * kPrepFloats;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int t = quad * 4 + i;  // row; l16 is the column s
     const double lc_t = __shfl(lc, t, 64);
     const float beta_t = __shfl(beta, t, 64), fq_t = __shfl(fq, t, 64), fk_t = __shfl(fk, t, 64);
     const float ratio = l16 <= t ? expf(fminf((float)(lc_t - lc), 0.f)) : 0.f;
-    s_a[wave][t][l16] = l16 < t ? beta_t * kk[i] * fk_t * fk * ratio : 0.f;
+    s_a[t][l16] = l16 < t ? beta_t * kk[i] * fk_t * fk * ratio : 0.f;
     if (live) out[kPrepP + t * kBlk + l16] = qk[i] * fq_t * fk * ratio;
   }
   if (live && quad == 0) {
@@ -135,7 +128,7 @@ __global__ __launch_bounds__(256) void gated_delta_prepare_kernel(const DeltaArg
     float acc = t == l16 ? 1.f : 0.f;
 #pragma unroll
     for (int s4 = 0; s4 < t; s4 += 4) {
-      const f32x4 r = *reinterpret_cast<const f32x4*>(&s_a[wave][t][s4]);
+      const f32x4 r = *reinterpret_cast<const f32x4*>(&s_a[t][s4]);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (s4 + j < t) acc = __builtin_fmaf(-r[j], x[s4 + j], acc);
@@ -148,15 +141,38 @@ __global__ __launch_bounds__(256) void gated_delta_prepare_kernel(const DeltaArg
   }
 }
 
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void gated_delta_prepare_kernel(const DeltaArgs a) {
+  __shared__ __attribute__((aligned(16))) float s_a[4][kBlk][kBlk + 4];
+  const int wave = threadIdx.x >> 6;
+  const long n_items = (long)a.B * a.H * a.blocks;
+  const long item0 = (long)blockIdx.x * 4 + wave;
+  const bool live = item0 < n_items;
+  const long item = live ? item0 : n_items - 1;
+  prepare_block<T, VEC>(a, (int)(item / a.blocks / a.H), (int)(item / a.blocks % a.H), (int)(item % a.blocks), live, s_a[wave],
+                        a.prep + item * kPrepFloats);
+}
+
 // RB: 16-row blocks of the state; RS: wavefronts that share a 16-column tile, RB / RS row blocks each
 // (their partial products with the state are added up through LDS).  Four wavefronts per workgroup.
 // Queries and keys go from memory into the operands as they are: the factors that make unit vectors of
 // them are factors of rows of the products, and have been multiplied into the decays.
-template <typename T, int RB, int RS, int LAY>
-__global__ __launch_bounds__(256) void gated_delta_scan_kernel(const DeltaArgs a) {
+// SHORT: at most kShortBlocks blocks, which the workgroup prepares itself, a wavefront each, into LDS: no launch in front, none but the blocks that are
+// there are gone through, and each is asked for once.  Calls of few heads wait for their launches, those of many for registers, so that bf16 tiles of one
+// wavefront are held to three on a SIMD (two above 64 channels; fp32 and the last columns of a tile would spill).  Kernel us, two launches / one: one
+// sequence of 6 tokens, 16 heads of 64 x 64, 10.8 / 7.2; 8 of 9, 4 of 128 x 128, fp32, 13.3 / 8.9; 4 of 30, 16 of 64 x 128, 12.9 / 10.3; 18 of 9, 24.6
+// / 15.3 (one of 2 waves 19.5); 32 of 40, 16 of 128 x 64, 54.7 / 33.8 (one wave 45.7); 14 of 64, 8 of 64 x 128, 19.5 / 17.8.  Behind 64 tokens a
+// wavefront has two blocks to prepare: 4 of 100 17.9 / 18.6, 1 of 120, 16 of 128 x 128, 22.6 / 26.5.
+constexpr int kShortBlocks = 4;
+constexpr int short_waves(bool held, int rb, int lay) { return !held || (rb > 6 && lay == 1) ? 1 : rb <= 4 ? 3 : 2; }
+
+template <typename T, int RB, int RS, int LAY, bool SHORT>
+__global__ __launch_bounds__(256, short_waves(SHORT && sizeof(T) == 2 && RS == 1, RB, LAY)) void gated_delta_scan_kernel(const DeltaArgs a) {
   static_assert(RB % RS == 0 && 4 % RS == 0, "row blocks divide among the wavefronts of a tile");
   constexpr int CT = 4 / RS, RBW = RB / RS;
   __shared__ __attribute__((aligned(16))) f32x4 s_part[2][RS > 1 ? CT * RS * 2 * 64 : 1];
+  __shared__ __attribute__((aligned(16))) float s_prep[SHORT ? kShortBlocks : 1][SHORT ? kPrepFloats : 4];
+  __shared__ __attribute__((aligned(16))) float s_a[SHORT ? 4 : 1][kBlk][kBlk + 4];
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ct = wave / RS, rs = wave % RS, row0 = rs * RBW * 16;
@@ -215,6 +231,7 @@ __global__ __launch_bounds__(256) void gated_delta_scan_kernel(const DeltaArgs a
       }
       s.v[i] = vb[off + (unsigned)vcol];
     }
+    if constexpr (SHORT) return;
     s.t = *reinterpret_cast<const f32x4*>(pr + kPrepT + l16 * kBlk + quad * 4);
     s.p = *reinterpret_cast<const f32x4*>(pr + kPrepP + l16 * kBlk + quad * 4);
     s.gk = *reinterpret_cast<const f32x4*>(pr + kPrepGk + quad * 4);
@@ -236,13 +253,26 @@ __global__ __launch_bounds__(256) void gated_delta_scan_kernel(const DeltaArgs a
     }
     // copies of their own: values that are used later in the block would otherwise stay in the registers the
     // next load wants, and the load's result be moved (and waited for) at the end of the loop
+    if constexpr (SHORT) {
+      const float* pr = s_prep[blk];
+      s.t = *reinterpret_cast<const f32x4*>(pr + kPrepT + l16 * kBlk + quad * 4);
+      s.p = *reinterpret_cast<const f32x4*>(pr + kPrepP + l16 * kBlk + quad * 4);
+      s.gk = *reinterpret_cast<const f32x4*>(pr + kPrepGk + quad * 4);
+      s.gq = *reinterpret_cast<const f32x4*>(pr + kPrepGq + quad * 4);
+      s.tail = *reinterpret_cast<const f32x4*>(pr + kPrepTail + quad * 4);
+      s.beta = *reinterpret_cast<const f32x4*>(pr + kPrepBeta + quad * 4);
+      s.last = pr[kPrepG + kBlk - 1];
+    }
     f32x4 tm = s.t, pm = s.p, gk = s.gk, gq = s.gq, tail = s.tail, beta = s.beta;
     float last = s.last;
     asm volatile("" : "+v"(tm), "+v"(pm), "+v"(gk), "+v"(gq), "+v"(tail), "+v"(beta), "+v"(last));
     float vv[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) vv[i] = to_f32(s.v[i]);
-    fetch(s, blk + 2 < a.blocks ? blk + 2 : a.blocks - 1);
+    if constexpr (!SHORT)
+      fetch(s, blk + 2 < a.blocks ? blk + 2 : a.blocks - 1);
+    else if (blk < last_blk)  // (uniform)
+      fetch(s, blk + 1);
     // two sums each for keys and queries: a product that waits for the one before it leaves the pipe idle
     f32x4 kq[2][2] = {{none, none}, {none, none}};
 #pragma unroll
@@ -298,18 +328,29 @@ __global__ __launch_bounds__(256) void gated_delta_scan_kernel(const DeltaArgs a
     }
   };
 
-  Stage s0, s1;
-  // (kept apart: the wait for a set counts the loads behind it, and takes the least favourable order of
-  // those in front of the loop and in it)
-  fetch(s0, 0);
-  __builtin_amdgcn_sched_barrier(0);
-  fetch(s1, 1);
-  __builtin_amdgcn_sched_barrier(0);
-  // The number of blocks is even (an empty one changes nothing): a way out between the two would make
-  // copies of the registers that are being loaded, and wait for them.
-  for (int blk = 0; blk < a.blocks; blk += 2) {
-    block(s0, blk, 0);
-    block(s1, blk + 1, 1);
+  Stage s0;
+  if constexpr (SHORT) {
+    fetch(s0, 0);
+    for (int p = 0; p <= last_blk; p += 4) {
+      const bool live = p + wave <= last_blk;
+      prepare_block<T, LAY != 0>(a, b, h, live ? p + wave : last_blk, live, s_a[wave], s_prep[live ? p + wave : last_blk]);
+    }
+    __syncthreads();
+    for (int blk = 0; blk <= last_blk; ++blk) block(s0, blk, blk & 1);
+  } else {
+    Stage s1;
+    // (kept apart: the wait for a set counts the loads behind it, and takes the least favourable order of
+    // those in front of the loop and in it)
+    fetch(s0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(s1, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    // The number of blocks is even (an empty one changes nothing): a way out between the two would make
+    // copies of the registers that are being loaded, and wait for them.
+    for (int blk = 0; blk < a.blocks; blk += 2) {
+      block(s0, blk, 0);
+      block(s1, blk + 1, 1);
+    }
   }
 #pragma unroll
   for (int r = 0; r < RBW; ++r)
@@ -533,10 +574,18 @@ __global__ __launch_bounds__(NT) void gated_delta_step_kernel(const DeltaStepArg
     y[c] = from_f32<T>(so[c] * r * to_f32(static_cast<const T*>(a.norm_w)[c]) * silu_exact(to_f32(gate[c])) * a.scale);
 }
 
+static bool delta_short(const DeltaArgs& a) { return a.vec && a.d <= 128 && a.L <= kShortBlocks * kBlk; }
+
 template <typename T, int RB, int RS, int LAY> void launch_delta_scan_split(const DeltaArgs& a, hipStream_t s) {
   const int cols = 16 * (4 / RS);
   const dim3 grid((unsigned)(a.B * a.H), (unsigned)((a.dv + cols - 1) / cols));
-  hipLaunchKernelGGL((gated_delta_scan_kernel<T, RB, RS, LAY>), grid, dim3(256), 0, s, a);
+  if constexpr (LAY > 0 && RB <= 8) {
+    if (delta_short(a)) {
+      hipLaunchKernelGGL((gated_delta_scan_kernel<T, RB, RS, LAY, true>), grid, dim3(256), 0, s, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((gated_delta_scan_kernel<T, RB, RS, LAY, false>), grid, dim3(256), 0, s, a);
 }
 
 // Tiles are shared by as many wavefronts as it takes to give every SIMD one; tall ones always, for their
@@ -573,7 +622,8 @@ template <typename T, int RB> void launch_delta_scan(const DeltaArgs& a, hipStre
 template <typename T> void launch_delta(const DeltaArgs& a, hipStream_t s) {
   const long items = (long)a.B * a.H * a.blocks;
   const dim3 grid((unsigned)((items + 3) / 4));
-  if (a.vec)
+  if (delta_short(a)) {
+  } else if (a.vec)
     hipLaunchKernelGGL((gated_delta_prepare_kernel<T, true>), grid, dim3(256), 0, s, a);
   else
     hipLaunchKernelGGL((gated_delta_prepare_kernel<T, false>), grid, dim3(256), 0, s, a);

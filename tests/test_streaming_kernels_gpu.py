@@ -214,6 +214,33 @@ def test_gated_delta_scan_column_splits(dev, B, H, dv):
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("B,H,G,d,dv", [(2, 2, 1, 16, 8), (1, 4, 4, 28, 40), (1, 6, 2, 44, 20), (3, 4, 4, 64, 64), (30, 4, 2, 64, 96), (40, 6, 6, 60, 72), (2, 3, 3, 96, 16),
+                                        (30, 6, 3, 80, 128), (3, 4, 2, 128, 64), (34, 4, 4, 128, 64), (70, 4, 4, 128, 64), (70, 4, 1, 116, 64)])
+def test_gated_delta_scan_of_short_portions(dev, dtype, B, H, G, d, dv):
+    """Portions of 1 to 64 tokens, which their scan prepares itself, one behind the other on one state, and of 65, which it does not: one block to four,
+    the last of them whole or not, tiles of one wavefront, two and four, heads that fill their rows and others."""
+    from based_amd import ops
+
+    cuts = [1, 16, 17, 64, 65, 33, 15]
+    L = sum(cuts)
+    q, k, v = (rnd(s, B, L, n, dtype=dtype) for s, n in ((51, G * d), (52, G * d), (53, H * dv)))
+    a, b, al, db = rnd(54, B, L, H, dtype=dtype), rnd(55, B, L, H, dtype=dtype), (rnd(56, H) - 1).to(dtype), rnd(57, H, dtype=dtype)
+    c, ad, bd, n = torch.cat([q, k, v], -1).to(dev), a.to(dev), b.to(dev), G * d
+    state = torch.full((B, H, d, (dv + 3) // 4 * 4), float("nan"), device=dev)
+    out, at = [], 0
+    for m in cuts:
+        x = c[:, at:at + m]
+        out.append(ops.gated_delta_scan(x[..., :n], x[..., n:2 * n], x[..., 2 * n:], ad[:, at:at + m], bd[:, at:at + m], al.to(dev), db.to(dev), state, H, G, at == 0))
+        at += m
+    o = torch.cat(out, 1)
+    for i in (0, B - 1):
+        g = torch.exp(-torch.exp(al.double()) * O.softplus(a[i].double() + db.double()))
+        unit = lambda x: O.unit(x[i].double().view(L, G, d)).repeat_interleave(H // G, 1)  # noqa: E731
+        ref = O.delta_rule(unit(q) * d ** -0.5, unit(k), v[i].double().view(L, H, dv), g, torch.sigmoid(b[i].double()))
+        assert rel_l2(o[i], ref) < 3e-6  # sums of up to 128 products, and of the portions before: some tens of 2^-24
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("W,blocks", [(64, 1), (160, 2), (96, 3), (256, 1), (54, 2), (8, 8), (520, 2)])
 @pytest.mark.parametrize("B", [1, 11])
 def test_rglru(dev, dtype, W, blocks, B):
