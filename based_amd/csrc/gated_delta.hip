@@ -157,17 +157,20 @@ __global__ __launch_bounds__(256) void gated_delta_prepare_kernel(const DeltaArg
 // (their partial products with the state are added up through LDS).  Four wavefronts per workgroup.
 // Queries and keys go from memory into the operands as they are: the factors that make unit vectors of
 // them are factors of rows of the products, and have been multiplied into the decays.
-// SHORT: at most kShortBlocks blocks, which the workgroup prepares itself, a wavefront each, into LDS: no launch in front, none but the blocks that are
+// MODE: what a block needs is asked for two blocks ahead (kDeltaTwoSets) or one (kDeltaOneSet), or
+// kDeltaShort: at most kShortBlocks blocks, which the workgroup prepares itself, a wavefront each, into LDS: no launch in front, none but the blocks that are
 // there are gone through, and each is asked for once.  Calls of few heads wait for their launches, those of many for registers, so that bf16 tiles of one
 // wavefront are held to three on a SIMD (two above 64 channels; fp32 and the last columns of a tile would spill).  Kernel us, two launches / one: one
 // sequence of 6 tokens, 16 heads of 64 x 64, 10.8 / 7.2; 8 of 9, 4 of 128 x 128, fp32, 13.3 / 8.9; 4 of 30, 16 of 64 x 128, 12.9 / 10.3; 18 of 9, 24.6
 // / 15.3 (one of 2 waves 19.5); 32 of 40, 16 of 128 x 64, 54.7 / 33.8 (one wave 45.7); 14 of 64, 8 of 64 x 128, 19.5 / 17.8.  Behind 64 tokens a
 // wavefront has two blocks to prepare: 4 of 100 17.9 / 18.6, 1 of 120, 16 of 128 x 128, 22.6 / 26.5.
 constexpr int kShortBlocks = 4;
-constexpr int short_waves(bool held, int rb, int lay) { return !held || (rb > 6 && lay == 1) ? 1 : rb <= 4 ? 3 : 2; }
+constexpr int kDeltaTwoSets = 0, kDeltaShort = 1, kDeltaOneSet = 2;
+constexpr int scan_waves(bool held, int rb, int lay) { return !held || (rb > 6 && lay == 1) ? 1 : rb <= 4 ? 3 : 2; }
 
-template <typename T, int RB, int RS, int LAY, bool SHORT>
-__global__ __launch_bounds__(256, short_waves(SHORT && sizeof(T) == 2 && RS == 1, RB, LAY)) void gated_delta_scan_kernel(const DeltaArgs a) {
+template <typename T, int RB, int RS, int LAY, int MODE>
+__global__ __launch_bounds__(256, scan_waves(MODE != kDeltaTwoSets && sizeof(T) == 2 && RS == 1, RB, LAY)) void gated_delta_scan_kernel(const DeltaArgs a) {
+  constexpr bool SHORT = MODE == kDeltaShort;
   static_assert(RB % RS == 0 && 4 % RS == 0, "row blocks divide among the wavefronts of a tile");
   constexpr int CT = 4 / RS, RBW = RB / RS;
   __shared__ __attribute__((aligned(16))) f32x4 s_part[2][RS > 1 ? CT * RS * 2 * 64 : 1];
@@ -200,7 +203,7 @@ __global__ __launch_bounds__(256, short_waves(SHORT && sizeof(T) == 2 && RS == 1
       S[r][i] = in ? st[(long)row * a.dvp] : 0.f;
     }
 
-  // What a block needs from memory, asked for two blocks ahead into two sets of registers that take turns.
+  // What a block needs from memory, asked for two blocks ahead into two sets of registers that take turns, or one ahead into one.
   struct Stage {
     Four<T, LAY> k[RBW], q[RBW];
     T kt[RBW][4], v[4];
@@ -269,8 +272,10 @@ __global__ __launch_bounds__(256, short_waves(SHORT && sizeof(T) == 2 && RS == 1
     float vv[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) vv[i] = to_f32(s.v[i]);
-    if constexpr (!SHORT)
+    if constexpr (MODE == kDeltaTwoSets)
       fetch(s, blk + 2 < a.blocks ? blk + 2 : a.blocks - 1);
+    else if constexpr (MODE == kDeltaOneSet)
+      fetch(s, blk < last_blk ? blk + 1 : last_blk);
     else if (blk < last_blk)  // (uniform)
       fetch(s, blk + 1);
     // two sums each for keys and queries: a product that waits for the one before it leaves the pipe idle
@@ -336,6 +341,9 @@ __global__ __launch_bounds__(256, short_waves(SHORT && sizeof(T) == 2 && RS == 1
       prepare_block<T, LAY != 0>(a, b, h, live ? p + wave : last_blk, live, s_a[wave], s_prep[live ? p + wave : last_blk]);
     }
     __syncthreads();
+    for (int blk = 0; blk <= last_blk; ++blk) block(s0, blk, blk & 1);
+  } else if constexpr (MODE == kDeltaOneSet) {
+    fetch(s0, 0);
     for (int blk = 0; blk <= last_blk; ++blk) block(s0, blk, blk & 1);
   } else {
     Stage s1;
@@ -581,11 +589,20 @@ template <typename T, int RB, int RS, int LAY> void launch_delta_scan_split(cons
   const dim3 grid((unsigned)(a.B * a.H), (unsigned)((a.dv + cols - 1) / cols));
   if constexpr (LAY > 0 && RB <= 8) {
     if (delta_short(a)) {
-      hipLaunchKernelGGL((gated_delta_scan_kernel<T, RB, RS, LAY, true>), grid, dim3(256), 0, s, a);
+      hipLaunchKernelGGL((gated_delta_scan_kernel<T, RB, RS, LAY, kDeltaShort>), grid, dim3(256), 0, s, a);
       return;
     }
   }
-  hipLaunchKernelGGL((gated_delta_scan_kernel<T, RB, RS, LAY, false>), grid, dim3(256), 0, s, a);
+  // More wavefronts than find registers for two sets: one set takes less of them.  Kernels of a call, us, two sets / one, by tiles: 128 x 128: 1,280,
+  // 800 tokens 433 / 364; 4,096, 70 tokens 128 / 96; 64 x 128: 2,048, 200 tokens 67.3 / 63.2; 4,096, 120 tokens 77.5 / 74.8; fewer: 128 x 64, 1,024,
+  // 896 tokens 275 / 285; 64 x 128, 1,280, 1,232 tokens 273 / 283.
+  if constexpr (sizeof(T) == 2 && RS == 1 && ((RB == 4 && LAY > 0) || (RB == 8 && LAY == 2))) {
+    if ((long)a.B * a.H * ((a.dv + 15) / 16) >= (RB > 4 ? 1025 : 2048)) {
+      hipLaunchKernelGGL((gated_delta_scan_kernel<T, RB, RS, LAY, kDeltaOneSet>), grid, dim3(256), 0, s, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((gated_delta_scan_kernel<T, RB, RS, LAY, kDeltaTwoSets>), grid, dim3(256), 0, s, a);
 }
 
 // Tiles are shared by as many wavefronts as it takes to give every SIMD one; tall ones always, for their
