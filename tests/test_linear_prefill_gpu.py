@@ -221,6 +221,23 @@ def test_segmented_scan_matches_single_pass(dev, B, H, L, dv, split):
     assert torch.equal(y3, y2)  # deterministic, with or without the state outputs
 
 
+@pytest.mark.parametrize("B,L,dv,segments", [(3, 1000, 64, 4), (3, 1300, 64, 5), (5, 1984, 64, 4), (5, 1985, 64, 6), (2, 2100, 128, 7), (2, 2048, 112, 8), (5, 704, 80, 1),
+                                             (5, 705, 128, 3), (6, 1984, 112, 1), (8, 1985, 128, 2), (9, 4000, 128, 1)])
+def test_planned_segments(dev, B, L, dv, segments):
+    """16 heads: both sides of the lines of the plan, with workgroups of one channel block and of two, against the single pass."""
+    import ctypes
+    from based_amd import _lib, ops
+
+    n, w = ctypes.c_int64(), ctypes.c_int64()
+    assert _lib.lib().based_linear_attn_prefill_plan(B, 16, L, dv, 0, ctypes.byref(n), ctypes.byref(w)) == 0
+    assert n.value == segments
+    q, k, v = (t.to(dev) for t in _qkv(B, 16, L, dv, torch.bfloat16, seed=23))
+    y1, kv1, ks1 = ops.linear_attn_prefill(q, k, v, return_state=True, split=False)
+    y2, kv2, ks2 = ops.linear_attn_prefill(q, k, v, return_state=True)
+    assert rel_l2(y2.float(), y1.float()) < 5e-3
+    assert rel_l2(kv2, kv1) < 2e-3 and rel_l2(ks2, ks1) < 2e-3
+
+
 def test_split_plan(dev):
     import ctypes
     from based_amd import _lib
