@@ -49,6 +49,7 @@ struct DecayScanArgs {
   int segs, seg_chunks;  // segments, and 64-token pieces in each
   int silu, fresh;
   int wide;              // rows of q, k, v and o in whole 16-byte pieces (channel decays, bf16)
+  int narrow;            // workgroups of 64 value channels, not of 128 (channel decays, more than 64 key channels)
 };
 
 template <int CTRL> __device__ __forceinline__ float row_moved(float x) {  // lanes without a source receive 0
@@ -1383,8 +1384,19 @@ template <int DT, int HALVES, int COLS, bool CHANNEL, bool FOLD> int launch_deca
 static bool channel_split(int64_t B, int64_t H, int64_t DV, int64_t segs, int64_t seg_chunks) {
   return B * H * ((DV + 63) / 64) * segs <= 384 || seg_chunks == 1;
 }
-// More channels: workgroups of 64 value channels where the 98 KB of each find a compute unit of their own, of 128 beyond that.
-static bool channel_narrow(int64_t B, int64_t H, int64_t DV) { return B * H * ((DV + 63) / 64) <= 256; }
+// More channels: workgroups of 64 value channels where the 98 KB of each find a compute unit of their own, of 128 beyond that, and where the call has
+// work space (by_channel) for twice the segments that way, each so much shorter that decays and keys worked out once for 128 channels count for
+// more than the launch that puts segments together and the longer piece.  Calls, us, of 64 / of 128, 8 heads of 128 (pieces of a segment of
+// 64): 1 x 4000 (4) 59 / 68; 4 x 1000 (4) 53 / 56; 6 x 500 (4) 50 / 52; 2 x 4000 (8) 94 / 90; 6 x 1000 (8) 88 / 80; 4 x 4000 (16) 166 / 145; 6 x
+// 2426 (19) 194 / 140; in one, 10 x 700 (11) 78.5 / 80.3, 10 x 1472 (23) 156 / 137; 14 x 1100, two of 128 for one, 124 / 151.
+static bool channel_narrow(int64_t B, int64_t L, int64_t H, int64_t DV, bool by_channel) {
+  const int64_t wgs = B * H * ((DV + 63) / 64), chunks = (L + kScanTokens - 1) / kScanTokens;
+  if (wgs > 256) return false;
+  if (!by_channel || DV <= 64 || L < BASED_DECAY_SEGMENTS_MIN) return true;
+  const int64_t segs = 256 / wgs;
+  if (segs > 1) return (chunks + segs - 1) / segs < 7;
+  return chunks < 16 || 256 / (B * H * ((DV + 127) / 128)) < 3;
+}
 
 int launch_decay_head(const DecayScanArgs& a, bool fold, hipStream_t s) {
   if (a.d <= 32) return fold ? launch_decay_mfma<1, 1, 64, false, true>(a, s) : launch_decay_mfma<1, 1, 64, false, false>(a, s);
@@ -1399,7 +1411,7 @@ int launch_decay_channel(const DecayScanArgs& a, bool fold, hipStream_t s) {
       return fold ? launch_decay_mfma<1, 2, 64, true, true>(a, s) : launch_decay_mfma<1, 2, 64, true, false>(a, s);
     return fold ? launch_decay_mfma<2, 1, 64, true, true>(a, s) : launch_decay_mfma<2, 1, 64, true, false>(a, s);
   }
-  if (channel_narrow(a.B, a.H, a.dv)) return fold ? launch_decay_mfma<2, 2, 64, true, true>(a, s) : launch_decay_mfma<2, 2, 64, true, false>(a, s);
+  if (a.narrow) return fold ? launch_decay_mfma<2, 2, 64, true, true>(a, s) : launch_decay_mfma<2, 2, 64, true, false>(a, s);
   return launch_decay_mfma<2, 2, 128, true, false>(a, s);
 }
 
@@ -1491,7 +1503,7 @@ static int decay_channel_segments(int64_t B, int64_t L, int64_t H, int64_t D, in
     segs = wgs <= 256 ? 768 / wgs : 1;
     most = chunks / 4 > kFoldSegmentsChannel ? chunks / 4 : kFoldSegmentsChannel;
   } else {  // (one workgroup to a compute unit.  1 x 2000, 8 heads of 128: 41.9 in 16 of two pieces, 55 in eight of four)
-    segs = 256 / (B * H * (channel_narrow(B, H, DV) ? (DV + 63) / 64 : (DV + 127) / 128));
+    segs = 256 / (B * H * (channel_narrow(B, L, H, DV, true) ? (DV + 63) / 64 : (DV + 127) / 128));
   }
   if (segs > most) segs = most;
   if (segs > chunks) segs = chunks;
@@ -1559,7 +1571,7 @@ static int decay_scan_call(bool by_channel, const void* q, const void* k, const 
   if (B == 0 || L == 0) return BASED_OK;
   DecayScanArgs a{q,    k,    v,    channel_log2, head_decay, bonus, state, nullptr, nullptr, o,    (int)B, (int)L, (int)H, (int)D, (int)DV,
                   (int)state_row, q_sb, q_sl, k_sb, k_sl, v_sb, v_sl, o_sb, o_sl, 1, (int)((L + kScanTokens - 1) / kScanTokens),
-                  activation == BASED_ACT_SILU, fresh, 0};
+                  activation == BASED_ACT_SILU, fresh, 0, channel_narrow(B, L, H, DV, by_channel)};
   hipStream_t s = static_cast<hipStream_t>(stream);
   const auto at = [](const void* p) { return (int64_t)reinterpret_cast<uintptr_t>(p); };
   const int64_t strides = q_sb | q_sl | k_sb | k_sl | v_sb | v_sl | o_sb | o_sl;
@@ -1573,7 +1585,7 @@ static int decay_scan_call(bool by_channel, const void* q, const void* k, const 
     a.seg = work;
     a.seg_lw = work + B * H * a.segs * DV * state_row;
   }
-  const bool fold = vec && (D <= 64 || (channel_log2 != nullptr && channel_narrow(B, H, DV))) && a.segs > 1 && a.segs <= (channel_log2 != nullptr ? kFoldSegmentsChannel : kFoldSegmentsHead);
+  const bool fold = vec && (D <= 64 || (channel_log2 != nullptr && a.narrow)) && a.segs > 1 && a.segs <= (channel_log2 != nullptr ? kFoldSegmentsChannel : kFoldSegmentsHead);
   a.wide = bits % 16 == 0 && D % 8 == 0 && DV % 8 == 0;
   if (vec) {
     const int rc = channel_log2 != nullptr ? launch_decay_channel(a, fold, s) : launch_decay_head(a, fold, s);

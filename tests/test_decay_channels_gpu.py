@@ -14,7 +14,9 @@ CASES = [(2, 70, 3, 20, 12),        # up to 32 channels
          (30, 129, 14, 64, 64), (30, 66, 14, 60, 44),  # many heads: one wavefront
          (1, 193, 2, 64, 64), (3, 704, 2, 64, 64), (1, 705, 1, 52, 20), (65, 260, 6, 64, 64),  # segments: four of a piece, ten and more, none
          (2, 133, 2, 128, 128), (1, 64, 3, 96, 68), (2, 700, 2, 128, 64), (1, 1100, 1, 72, 128),  # workgroups of 64 value channels
-         (33, 66, 4, 128, 128), (34, 130, 4, 100, 132)]  # of 128
+         (33, 66, 4, 128, 128), (34, 130, 4, 100, 132),  # of 128
+         # segments of seven pieces and of six; one of 15 in all and three of 16; workgroups of 128 and 64
+         (2, 1700, 16, 128, 128), (4, 768, 8, 72, 128), (6, 833, 8, 128, 72), (5, 960, 16, 96, 128), (5, 961, 16, 96, 128), (2, 1700, 16, 128, 64)]
 
 
 @pytest.mark.parametrize("silu", [False, True])
@@ -55,7 +57,8 @@ def test_work_space_of_channel_decays():
     lib = _lib.lib()
     floats = lambda segs, B, H, D, DV: B * H * segs * (DV + 1) * D  # noqa: E731
     for B, L, H, D, segs in [(1, 192, 16, 64, 0), (1, 193, 16, 64, 4), (5, 320, 16, 64, 5), (4, 2048, 16, 64, 10), (1, 4096, 16, 64, 16), (30, 513, 16, 64, 0),
-                             (2, 500, 8, 128, 8), (4, 2048, 8, 128, 4), (16, 1024, 8, 128, 0), (30, 500, 8, 128, 0)]:
+                             (2, 500, 8, 128, 8), (4, 2048, 8, 128, 8), (4, 1536, 8, 128, 4), (10, 961, 8, 128, 3), (10, 960, 8, 128, 0), (16, 1024, 8, 128, 0),
+                             (30, 500, 8, 128, 0)]:
         sizes = (B, L, H, D, D, D)
         assert lib.based_decay_scan_channels_work(0, *sizes, 0) == floats(segs, B, H, D, D), (B, L, H, D)
         assert lib.based_decay_scan_channels_work(4, *sizes, 0) == lib.based_decay_scan_work_of(4, *sizes, 0)  # (off 8 bytes)
