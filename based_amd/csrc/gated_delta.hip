@@ -160,13 +160,13 @@ __global__ __launch_bounds__(256) void gated_delta_prepare_kernel(const DeltaArg
 // MODE: what a block needs is asked for two blocks ahead (kDeltaTwoSets) or one (kDeltaOneSet), or
 // kDeltaShort: at most kShortBlocks blocks, which the workgroup prepares itself, a wavefront each, into LDS: no launch in front, none but the blocks that are
 // there are gone through, and each is asked for once.  Calls of few heads wait for their launches, those of many for registers, so that bf16 tiles of one
-// wavefront are held to three on a SIMD (two above 64 channels; fp32 and the last columns of a tile would spill).  Kernel us, two launches / one: one
-// sequence of 6 tokens, 16 heads of 64 x 64, 10.8 / 7.2; 8 of 9, 4 of 128 x 128, fp32, 13.3 / 8.9; 4 of 30, 16 of 64 x 128, 12.9 / 10.3; 18 of 9, 24.6
-// / 15.3 (one of 2 waves 19.5); 32 of 40, 16 of 128 x 64, 54.7 / 33.8 (one wave 45.7); 14 of 64, 8 of 64 x 128, 19.5 / 17.8.  Behind 64 tokens a
-// wavefront has two blocks to prepare: 4 of 100 17.9 / 18.6, 1 of 120, 16 of 128 x 128, 22.6 / 26.5.
+// wavefront are held to three on a SIMD, two above 64 channels (fp32, and tiles that heads of 49 to 63 and 97 to 127 channels leave partly
+// empty, would spill).  Kernel us, two launches / one: one sequence of 6 tokens, 16 heads of 64 x 64, 10.8 / 7.2; 8 of 9, 4 of 128 x 128, fp32, 13.3 /
+// 8.9; 4 of 30, 16 of 64 x 128, 12.9 / 10.3; 18 of 9, 24.6 / 15.3 (two wavefronts 19.5); 32 of 40, 16 of 128 x 64, 54.7 / 33.8 (one 45.7); 14 of 64,
+// 8 of 64 x 128, 19.5 / 17.8.  Behind 64 tokens a wavefront has two blocks to prepare: 4 of 100 17.9 / 18.6, 1 of 120, 16 of 128 x 128, 22.6 / 26.5.
 constexpr int kShortBlocks = 4;
 constexpr int kDeltaTwoSets = 0, kDeltaShort = 1, kDeltaOneSet = 2;
-constexpr int scan_waves(bool held, int rb, int lay) { return !held || (rb > 6 && lay == 1) ? 1 : rb <= 4 ? 3 : 2; }
+constexpr int scan_waves(bool held, int rb, int lay) { return !held || (lay == 1 && (rb == 4 || rb > 6)) ? 1 : rb <= 4 ? 3 : 2; }
 
 template <typename T, int RB, int RS, int LAY, int MODE>
 __global__ __launch_bounds__(256, scan_waves(MODE != kDeltaTwoSets && sizeof(T) == 2 && RS == 1, RB, LAY)) void gated_delta_scan_kernel(const DeltaArgs a) {
@@ -596,7 +596,7 @@ template <typename T, int RB, int RS, int LAY> void launch_delta_scan_split(cons
   // More wavefronts than find registers for two sets: one set takes less of them.  Kernels of a call, us, two sets / one, by tiles: 128 x 128: 1,280,
   // 800 tokens 433 / 364; 4,096, 70 tokens 128 / 96; 64 x 128: 2,048, 200 tokens 67.3 / 63.2; 4,096, 120 tokens 77.5 / 74.8; fewer: 128 x 64, 1,024,
   // 896 tokens 275 / 285; 64 x 128, 1,280, 1,232 tokens 273 / 283.
-  if constexpr (sizeof(T) == 2 && RS == 1 && ((RB == 4 && LAY > 0) || (RB == 8 && LAY == 2))) {
+  if constexpr (sizeof(T) == 2 && RS == 1 && LAY == 2 && (RB == 4 || RB == 8)) {
     if ((long)a.B * a.H * ((a.dv + 15) / 16) >= (RB > 4 ? 1025 : 2048)) {
       hipLaunchKernelGGL((gated_delta_scan_kernel<T, RB, RS, LAY, kDeltaOneSet>), grid, dim3(256), 0, s, a);
       return;
