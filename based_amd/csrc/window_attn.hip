@@ -182,9 +182,7 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
 // p ^ (r / 2 % 8), of values at p ^ (r / 2 % 4 * 2), so that reads of 16 rows (transposing reads of 8) meet every bank once; one barrier a tile.
 // FILL, of such rows: the portion's keys and values are taken as they come, turned and normed on their way to LDS, and left in the cache by the
 // workgroups whose tokens they are; nobody reads there what is written.
-template <int KC, int VC, bool HALF, bool DIRECT, bool FILL = false>
-__global__ __launch_bounds__(256, FILL ? 2 : KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 3 : KC <= 3 && VC <= 4 ? 2 : 1)
-void window_prefill_mfma_kernel(const WindowArgs a) {
+template <int KC, int VC, bool HALF, bool DIRECT, bool FILL> __device__ __forceinline__ void window_prefill_mfma(const WindowArgs& a) {
   constexpr int D = KC * 32, DV = VC * 32;
   constexpr int KS = D + 8, VS = kTileKeys + 8;  // LDS row strides: 16-lane reads of 16 bytes meet every bank once
   static_assert(!DIRECT || (KC == 2 && VC == 2), "rows of 64 channels");
@@ -533,6 +531,15 @@ void window_prefill_mfma_kernel(const WindowArgs a) {
       }
     }
   }
+}
+
+template <int KC, int VC, bool HALF, bool DIRECT>
+__global__ __launch_bounds__(256, KC <= 2 && VC <= 2 ? 4 : KC <= 3 && VC <= 2 ? 3 : KC <= 3 && VC <= 4 ? 2 : 1)
+void window_prefill_mfma_kernel(const WindowArgs a) {
+  window_prefill_mfma<KC, VC, HALF, DIRECT, false>(a);
+}
+template <bool HALF> __global__ __launch_bounds__(256, 2) void window_prefill_fill_kernel(const WindowArgs a) {
+  window_prefill_mfma<2, 2, HALF, true, true>(a);
 }
 
 // ---- prefill, fp32, fp32 MFMA ----
@@ -1471,10 +1478,17 @@ template <int LPI> void launch_kv_write(const WindowArgs& a, hipStream_t s) {
 
 template <int KC, int VC, bool DIRECT, bool FILL = false> void launch_window_mfma_pairs(const WindowArgs& a, dim3 grid, hipStream_t s) {
   constexpr unsigned lds = DIRECT ? 2 * kDirectTile * sizeof(__bf16) : 0;
-  if (a.half_split)
-    hipLaunchKernelGGL((window_prefill_mfma_kernel<KC, VC, true, DIRECT, FILL>), grid, dim3(256), lds, s, a);
-  else
-    hipLaunchKernelGGL((window_prefill_mfma_kernel<KC, VC, false, DIRECT, FILL>), grid, dim3(256), lds, s, a);
+  if constexpr (FILL) {
+    static_assert(KC == 2 && VC == 2 && DIRECT, "rows of 64 channels");
+    if (a.half_split)
+      hipLaunchKernelGGL(window_prefill_fill_kernel<true>, grid, dim3(256), lds, s, a);
+    else
+      hipLaunchKernelGGL(window_prefill_fill_kernel<false>, grid, dim3(256), lds, s, a);
+  } else if (a.half_split) {
+    hipLaunchKernelGGL((window_prefill_mfma_kernel<KC, VC, true, DIRECT>), grid, dim3(256), lds, s, a);
+  } else {
+    hipLaunchKernelGGL((window_prefill_mfma_kernel<KC, VC, false, DIRECT>), grid, dim3(256), lds, s, a);
+  }
 }
 
 template <int KC> void launch_window_mfma(const WindowArgs& a, dim3 grid, hipStream_t s) {
