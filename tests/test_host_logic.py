@@ -324,3 +324,18 @@ def test_fp32_experts_share_matrices_only_where_that_is_faster():
         assert not shared(slots, D, F, E), (slots, D, F, E)
     for slots, D, F, E in ((25, 1024, 1024, 8), (140, 2048, 2048, 8), (49, 512, 512, 16), (16384, 512, 512, 8), (1024, 512, 512, 4), (256, 2048, 512, 64)):
         assert shared(slots, D, F, E), (slots, D, F, E)
+
+
+def test_long_prompts_of_few_heads_are_cut_for_every_compute_unit():
+    """Segments of linear attention: of 32 chunks while the workgroups stay within the chip, 256 of two channel blocks (heads of 65 to 128 channels) or 512
+    of one; beyond that no more of them."""
+    import ctypes
+
+    from based_amd import _lib
+
+    n, w = ctypes.c_int64(), ctypes.c_int64()
+    for heads, tokens, dv, segments in ((1, 32768, 128, 16), (1, 65536, 128, 32), (1, 262144, 128, 128), (2, 262144, 112, 128), (4, 65536, 128, 32),
+                                        (4, 262144, 128, 64), (8, 40000, 128, 32), (8, 262144, 128, 32), (16, 65536, 128, 16), (24, 65536, 128, 10),
+                                        (4, 262144, 64, 128), (8, 262144, 64, 64), (16, 65536, 64, 32), (8, 65536, 192, 20)):
+        assert _lib.lib().based_linear_attn_prefill_plan(1, heads, tokens, dv, 0, ctypes.byref(n), ctypes.byref(w)) == 0
+        assert n.value == segments and w.value == heads * ((dv + 63) // 64) * segments * 43008, (heads, tokens, dv, n.value)
