@@ -19,8 +19,8 @@
 //
 // Inside 64 tokens, with P_ts the weight of v_s in o_t, o = P v + (q scaled by the decay since the start) S0.
 // All scaling is by decays over tokens that lie in between, never by an inverse, so nothing overflows:
-//   * s and t in the same 16 tokens: k_s, multiplied by one more decay at each step, is passed from token to
-//     token (a lane is a token) and meets every q on its way;
+//   * s and t in the same 16 tokens: halves of 2, 4, 8 and 16 tokens meet, k_s decayed to the middle, q_t from there
+//     (head decays: a power of the decay, times the product of k_s and q_t);
 //   * s in an earlier 16 tokens: k_s decayed to the end of its 16, q_t to the start of its own, and to q
 //     also what lies between.
 // fp32 numbers enter a bf16 product as pairs (a number rounded to bf16, and the rest rounded to bf16), so
@@ -129,8 +129,11 @@ struct HeadPowers {
 // Inside 16 tokens the weights are found by halves: with b = 1, 2, 4, 8, tokens of the second half of each 2 b meet those of its first half, queries
 // decayed from the middle to their token, keys from theirs to the middle, so that one operand x (a query or a key, by the lane's half) times itself
 // holds all of them; the products of decays double with b on the way.  (Keys passed from token to token on the vector unit were 610 of a
-// wavefront's 1,500 instructions to 64 tokens.  x in fp32 on the fp32 matrix unit, which takes the vector unit's issue with it: 4 x 2048 tokens, 16 heads of
-// 64, 58.7 us for 55.5; the error against 64 bits is that of the rounding of o to bf16 either way, 1.659e-3.)
+// wavefront's 1,500 instructions to 64 tokens.)  Neighbours are the bf16 that came in; the others are products of fp32 numbers, of four keys with four
+// queries at a time, which leaves none of a product unused but the half that lies in front of the key.  Where keys nearly cancel, in two channels
+// of opposite sign whose decays differ by 2^-12, the error against 64 bits is 1.667e-3, of which the rounding of o to bf16 is all; with x as pairs of bf16
+// it was 5.5e-3.  Calls, us, as pairs / as 16 x 16 products in fp32 / this way: 4 x 2048 tokens, 16 heads of 64 57.9 / 61.5 / 58.7; 20 x 2048 220 / 244 /
+// 228; 16 x 1024, 8 heads of 128 114 / 128 / 119; 8 x 2000 144 / 149 / 141; 2 x 768, 16 heads of 64 22.2 / 23.1 / 22.1.
 // Across 16 tokens the keys wait in LDS, decayed to the end of theirs, for the queries decayed from the start of their own and what lies between;
 // the state takes the same keys, decayed itself by what each 16 tokens leave of it.  Outputs belong to the wavefronts of their tokens, so that neither
 // weights nor queries go through LDS, the state's tiles of 16 value channels to a wavefront each: two barriers to 64 tokens, one behind what is written
@@ -182,6 +185,10 @@ template <int B> __device__ __forceinline__ void join_halves2(float* q, float* k
 #undef BASED_HALF_STEP
 #undef BASED_HALF_REGS
 
+// 16 products of 4 x 4 numbers, each of four lanes: the rows are a's, of the lanes of number ABID of every 2^CBSZ such groups, the columns b's own.
+template <int CBSZ, int ABID> __device__ __forceinline__ f32x4 mfma_4(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, CBSZ, ABID, 0);
+}
 __device__ __forceinline__ f32x4 mfma_16_half(bf16x4 a, bf16x4 b, f32x4 c) {
   typedef __attribute__((ext_vector_type(4))) short s16x4;
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
@@ -337,12 +344,6 @@ __global__ __launch_bounds__(256 * HALVES, channel_waves(DT, HALVES)) void decay
     }
   }
   if constexpr (!STATE_ONLY) lds_barrier();  // (the bonus)
-  int apart = 0;  // byte i: the half length at which row s = 4 quad + i meets this lane's token, 0 where it does not
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int s = quad * 4 + i, z = l16 ^ s;
-    apart |= (s >= l16 ? 0 : 0x80000000u >> __builtin_clz(z | 1)) << i * 8;
-  }
   float seg_total = 1.f;  // (state pass) decay of the segment so far, of the channel that is this thread's number
 
   for (int chunk = first; chunk < last; ++chunk) {
@@ -417,10 +418,6 @@ __global__ __launch_bounds__(256 * HALVES, channel_waves(DT, HALVES)) void decay
       bonus = sum_quads4(bonus, bonus, bonus, bonus);  // (in every lane of the token)
 #pragma unroll
       for (int i = 0; i < 4; ++i) diag[i] = quad * 4 + i == l16 ? bonus : 0.f;
-      auto meet = [&](int half_len, f32x4 acc) {  // rows of the first half of this lane's second half
-#pragma unroll
-        for (int i = 0; i < 4; ++i) diag[i] = (apart >> i * 8 & 0xff) == half_len ? acc[i] : diag[i];
-      };
       {
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -433,25 +430,22 @@ __global__ __launch_bounds__(256 * HALVES, channel_waves(DT, HALVES)) void decay
         }
 #pragma unroll
         for (int i = 0; i < E; i += 2) join_halves2<1>(q + i, k + i, w + i, l16 & 1);
-        meet(1, acc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) diag[i] = (l16 & 1) && quad * 4 + i == l16 - 1 ? acc[i] : diag[i];
       }
+      // [of four tokens] itself, the four in front, of the first and second four of the eight in front: rows, this lane's token the column
+      f32x4 own = {0.f, 0.f, 0.f, 0.f}, front = own, first4 = own, second4 = own;
       auto level = [&](auto half_len) {
         constexpr int HB = decltype(half_len)::value;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int c = 0; c < DT; ++c) {
-          float x[8];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) x[i] = l16 & HB ? q[c * 8 + i] : k[c * 8 + i];
-          bf16x8 hi, lo;
-          split8(x, hi, lo);
-          acc = mfma_16(hi, hi, acc);
-          acc = mfma_16(lo, hi, acc);
-          acc = mfma_16(hi, lo, acc);
+        for (int i = 0; i < E; ++i) {
+          const float x = l16 & HB ? q[i] : k[i];
+          if constexpr (HB == 2) own = mfma_4<0, 0>(x, x, own);
+          if constexpr (HB == 4) front = mfma_4<1, 0>(x, x, front);
+          if constexpr (HB == 8) first4 = mfma_4<2, 0>(x, x, first4), second4 = mfma_4<2, 1>(x, x, second4);
         }
 #pragma unroll
         for (int i = 0; i < E; i += 2) join_halves2<HB>(q + i, k + i, w + i, l16 & HB);
-        meet(HB, acc);
       };
       ask(std::integral_constant<int, 1>{});
       level(std::integral_constant<int, 2>{});
@@ -460,6 +454,13 @@ __global__ __launch_bounds__(256 * HALVES, channel_waves(DT, HALVES)) void decay
       ask(std::integral_constant<int, 4>{});
       level(std::integral_constant<int, 8>{});
       ask(std::integral_constant<int, 8>{});
+      const int four = l16 >> 2;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {  // added up over the channels' lanes, each where its row is wanted
+        const float near = i < 2 && l16 & 2 ? own[i] : 0.f;
+        diag[i] += sum_quads4(four == 0 ? near : four == 1 ? front[i] : first4[i], four == 1 ? near : four >= 2 ? second4[i] : 0.f,
+                              four == 2 ? near : four == 3 ? front[i] : 0.f, four == 3 ? near : 0.f);
+      }
       // q is decayed from the start of the 16 tokens now, k to their end, w the decay over all of them
     } else {
 #pragma unroll

@@ -50,6 +50,29 @@ def test_channel_decays(dev, B, L, H, d, dv, fresh, silu):
     assert rel(state[..., :d], S.transpose(2, 3)) < (1e-4 if silu else 7.7e-6)
 
 
+@pytest.mark.parametrize("B,H,d,dv", [(2, 3, 32, 32), (4, 16, 64, 64), (40, 16, 64, 64), (2, 8, 128, 128), (40, 8, 128, 128)])
+def test_weights_inside_16_tokens_are_of_32_bits(dev, B, H, d, dv):
+    """Keys that nearly cancel, in two channels of opposite sign whose decays differ by 2^-12: what is left of a weight is 2^-12 of its two parts."""
+    from based_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(d + B)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    L = 80
+    q, k, lw = rnd(B, L, H, d // 2).bfloat16(), rnd(B, L, H, d // 2).bfloat16(), -0.1 * torch.rand(B, L, H, d // 2, generator=g, device=dev)
+    q, k, lw = (torch.stack(x, -1).reshape(B, L, H * d) for x in ((q, q), (k, -k), (lw, lw - 2.0 ** -12)))
+    v, u = rnd(B, L, H * dv).bfloat16(), torch.zeros(H, d, device=dev).bfloat16()
+    out = ops.decay_scan(q, k, v, torch.zeros(B, H, dv, d, device=dev), H, channel_log2=lw, bonus=u, fresh=True)[:, 2:16].double()
+    qd, kd, vd = (x[:, :16].double().view(B, 16, H, -1) for x in (q, k, v))
+    lc = torch.cumsum(lw[:, :16].double().view(B, 16, H, d), 1)
+    want = torch.zeros(B, 16, H, dv, dtype=torch.float64, device=dev)
+    for t in range(2, 16):  # (neighbours have no decay between them: their two parts are nothing together)
+        for s in range(t - 1):
+            want[:, t] += (qd[:, t] * kd[:, s] * 2.0 ** (lc[:, t - 1] - lc[:, s])).sum(-1, keepdim=True) * vd[:, s]
+    want = want[:, 2:].flatten(2)
+    # 2^-9 of an output for its rounding to bf16, and 2^-23 of its parts for their decays: n of them, of parts that differ by n 2^-12.5
+    assert ((out - want).norm() / want.norm()).item() < 2 ** -9 + 2 ** -10.5
+
+
 def test_work_space_of_channel_decays():
     """Segments by the rule of channel decays for aligned bf16, those of the general form for everything else; none for short prompts."""
     from based_amd import _lib
