@@ -327,6 +327,8 @@ __global__ __launch_bounds__(256) void latent_step_any_kernel(const LatentArgs a
 // OWN > 0: OWN heads per workgroup and at most 64 keys, and no launch in front: the workgroup forms its queries while its keys are on their way, and,
 // where the token's own row is among the keys, that row, which the workgroup of the first heads leaves in the cache.  uk is read by every
 // workgroup of its heads, so that this is the way of few sequences, whose time is waiting: what needs no position is asked for in front of it.
+// Queries and row are summed as latent_query sums them, in 16 groups of a head's channels and by lanes, so that the results are the same numbers
+// (0.2 us of the 13.0 of four sequences of 512 keys); from kTileMinRows sequences on those are summed on the matrix unit.
 template <int KC, int RT, int OWN>
 __global__ __launch_bounds__(256, 1) void latent_step_mfma_kernel(const LatentArgs a) {
   constexpr int KS = 64 + 8;  // keys per LDS row
@@ -336,20 +338,24 @@ __global__ __launch_bounds__(256, 1) void latent_step_mfma_kernel(const LatentAr
   __shared__ float wmax[4][16], wsum[4][16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, quad = lane >> 4, W = a.R + a.rot;
   const int b = blockIdx.x, split = blockIdx.y, h0 = blockIdx.z * (OWN > 0 ? OWN : 16);
-  // OWN: 8 latent channels to a thread, rows of uk dealt to the groups, DU of each head in flight; asked for before the position is known
-  constexpr int HEADS = OWN > 0 ? OWN : 1, PIECES = RT * 8, GROUPS = 256 / PIECES, DU = 16 / HEADS;
-  const int col = tid % PIECES * 8, grp = tid / PIECES, per_head = a.rot + a.d, heads = a.H - h0 < HEADS ? a.H - h0 : HEADS;
-  bf16x8 uk[HEADS][DU], own_x, own_norm;
+  // OWN: 8 latent channels to a thread, rows of uk dealt to 16 / SUMS groups, of each head (or, where there are threads for that, of one) DU in flight;
+  // asked for before the position is known
+  constexpr int HEADS = OWN > 0 ? OWN : 1, PIECES = RT * 8, APART = RT == 1 ? HEADS : 1, MINE = HEADS / APART;
+  constexpr int GROUPS = 256 / PIECES / APART, SUMS = 16 / GROUPS, DU = 16 / MINE;
+  static_assert(OWN == 0 || (SUMS * GROUPS == 16 && DU % SUMS == 0), "rows of uk, 16 apart, in one sum");
+  const int col = tid % PIECES * 8, grp = tid / PIECES % GROUPS, hm = tid / PIECES / GROUPS * MINE;
+  const int per_head = a.rot + a.d, heads = a.H - h0 < HEADS ? a.H - h0 : HEADS;
+  bf16x8 uk[MINE][DU], own_x, own_norm;
   float own_q[HEADS * GROUPS * DU / 256 > 0 ? HEADS * GROUPS * DU / 256 : 1];
   const __bf16* q_in = static_cast<const __bf16*>(a.q) + b * a.q_sb + (long)h0 * per_head;
   auto ask_heads = [&](int d0) {
 #pragma unroll
-    for (int h = 0; h < HEADS; ++h)
+    for (int h = 0; h < MINE; ++h)
 #pragma unroll
       for (int u = 0; u < DU; ++u) {
         const int d = d0 + u * GROUPS + grp;
         uk[h][u] = *reinterpret_cast<const bf16x8*>(static_cast<const __bf16*>(a.w) + (col < a.R ? col : 0) +
-                                                    ((long)(h < heads ? h0 + h : h0) * (per_head + a.dv) + a.rot + (d < a.d ? d : 0)) * a.w_sr);
+                                                    ((long)(hm + h < heads ? h0 + hm + h : h0) * (per_head + a.dv) + a.rot + (d < a.d ? d : 0)) * a.w_sr);
       }
 #pragma unroll
     for (int i = 0; i * 256 < HEADS * GROUPS * DU; ++i) {
@@ -401,15 +407,18 @@ __global__ __launch_bounds__(256, 1) void latent_step_mfma_kernel(const LatentAr
   bf16x8 qf[KC];
   if constexpr (OWN > 0) {
     __shared__ float qs[OWN][GROUPS * DU];
-    __shared__ __attribute__((aligned(16))) float sums[GROUPS][OWN][RMAX];
+    static_assert(16 * OWN * RMAX * sizeof(float) <= sizeof(vt), "sums in the place of the latents, which come later");
+    float(*sums)[OWN][RMAX] = reinterpret_cast<float(*)[OWN][RMAX]>(vt);
     __shared__ __attribute__((aligned(16))) __bf16 qt[OWN][KC * 32];
     __shared__ __attribute__((aligned(16))) __bf16 row[KC * 32];
     const bool own_row = first + n - 1 == pos;
-    float part[OWN][8];
+    float part[MINE][SUMS][8];
 #pragma unroll
-    for (int h = 0; h < OWN; ++h)
+    for (int h = 0; h < MINE; ++h)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) part[h][j] = 0.f;
+      for (int i = 0; i < SUMS; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) part[h][i][j] = 0.f;
     for (int d0 = 0; d0 < a.d; d0 += GROUPS * DU) {
       if (d0 > 0) {
         ask_heads(d0);
@@ -420,22 +429,25 @@ __global__ __launch_bounds__(256, 1) void latent_step_mfma_kernel(const LatentAr
         if (i * 256 + tid < OWN * GROUPS * DU) qs[0][i * 256 + tid] = own_q[i];
       lds_barrier();
 #pragma unroll
-      for (int h = 0; h < OWN; ++h)
+      for (int h = 0; h < MINE; ++h)
 #pragma unroll
         for (int u = 0; u < DU; ++u)
 #pragma unroll
-          for (int j = 0; j < 8; ++j) part[h][j] = __builtin_fmaf(to_f32(uk[h][u][j]), qs[h][u * GROUPS + grp], part[h][j]);
+          for (int j = 0; j < 8; ++j) part[h][u % SUMS][j] = __builtin_fmaf(to_f32(uk[h][u][j]), qs[hm + h][u * GROUPS + grp], part[h][u % SUMS][j]);
     }
     if (own_row && wave == 0) {  // the token's row, 8 channels to a lane
+      if (lane * 8 < a.R) *reinterpret_cast<bf16x8*>(&row[lane * 8]) = own_x;
+      __builtin_amdgcn_wave_barrier();  // (a wavefront's writes to LDS come before its reads)
       float x[8], ss = 0.f;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        x[j] = to_f32(own_x[j]);
-        ss = lane * 8 < a.R ? __builtin_fmaf(x[j], x[j], ss) : ss;
+      for (int i = 0; i < RT; ++i) {
+        const float y = to_f32(row[i * 64 + lane < a.R ? i * 64 + lane : 0]);
+        ss = i * 64 + lane < a.R ? __builtin_fmaf(y, y, ss) : ss;
       }
       const float r = 1.0f / sqrtf(wave_sum(ss) / (float)a.R + a.eps);
+      __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] *= r * to_f32(own_norm[j]);
+      for (int j = 0; j < 8; ++j) x[j] = to_f32(own_x[j]) * r * to_f32(own_norm[j]);
       if (lane * 8 < a.R) store_vec<__bf16, 8>(&row[lane * 8], x);
       for (int c = lane; c < a.rot; c += 64) row[a.R + c] = (__bf16)turned(static_cast<const __bf16*>(a.x) + b * a.x_sb + a.R, c, pos, a);
     } else if (wave == 1 || wave == 2) {
@@ -445,15 +457,18 @@ __global__ __launch_bounds__(256, 1) void latent_step_mfma_kernel(const LatentAr
       }
     }
 #pragma unroll
-    for (int h = 0; h < OWN; ++h)
+    for (int h = 0; h < MINE; ++h)
 #pragma unroll
-      for (int j = 0; j < 8; j += 4) *reinterpret_cast<f32x4*>(&sums[grp][h][col + j]) = f32x4{part[h][j], part[h][j + 1], part[h][j + 2], part[h][j + 3]};
+      for (int i = 0; i < SUMS; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; j += 4)
+          *reinterpret_cast<f32x4*>(&sums[i * GROUPS + grp][hm + h][col + j]) = f32x4{part[h][i][j], part[h][i][j + 1], part[h][i][j + 2], part[h][i][j + 3]};
     lds_barrier();
     for (int i = tid; i < OWN * RMAX; i += 256) {
       const int h = i / RMAX, c = i % RMAX;
       float x = 0.f;
 #pragma unroll
-      for (int g = 0; g < GROUPS; ++g) x += sums[g][h][c];
+      for (int g = 0; g < 16; ++g) x += sums[g][h][c];
       if (c < a.R) qt[h][c] = (__bf16)x;
     }
     if (own_row) {  // in place of the last key, and of what is asked for behind it

@@ -456,6 +456,31 @@ def test_steps_of_few_sequences_form_their_own_queries(dev, H, d, r, dv, R, wind
     assert bool(out[0][1][3].isnan().all())
 
 
+@pytest.mark.parametrize("H,d,r,dv,R,window,keys", [
+    (16, 64, 32, 64, 256, 512, 700), (1, 8, 8, 8, 8, 1, 3), (15, 24, 8, 16, 64, 63, 200), (12, 72, 16, 8, 48, 64, 66), (15, 136, 8, 40, 128, 65, 90),
+    (14, 72, 64, 16, 248, 128, 300), (6, 264, 24, 24, 264, 200, 260), (3, 130, 64, 8, 512, 700, 800), (13, 300, 32, 8, 64, 60, 64)])
+def test_steps_of_few_sequences_are_those_of_the_launches(dev, H, d, r, dv, R, window, keys):
+    """The same numbers, outputs and cache, whether queries and row are formed by the attention or by a launch in front of it (for an input that is not in
+    whole 16-byte pieces): one latent tile to eight, heads whose channels end inside a round of uk.  Sums in another order would fall the other way in
+    bf16 in one of some ten thousand numbers: so many tokens that there are hundreds of these."""
+    from based_amd import ops
+
+    B, g = 7 if window <= 200 else 3, torch.Generator(device=dev).manual_seed(R + d)
+    normal = lambda *s, scale=1.0: (torch.randn(*s, generator=g, device=dev) * scale).to(BF16)  # noqa: E731
+    nw, w = 1 + normal(R, scale=0.2), normal(H * (r + d + dv), R, scale=R ** -0.5)
+    pos = torch.tensor([keys - 1 - b * (keys // 8) for b in range(B)], dtype=torch.int32, device=dev)
+    ang = torch.outer(torch.arange(keys, dtype=torch.float64), 500.0 ** (-torch.arange(0, r, 2, dtype=torch.float64) / r))
+    rope, rows = (ang.cos().float().to(dev), ang.sin().float().to(dev), True), normal(B, keys, R + r)
+    for _ in range(60):
+        q, x, out = normal(B, H * (r + d)), normal(B, R + r), []
+        for offset in (0, 1):
+            cache = rows.clone()
+            moved = torch.empty(x.numel() + offset, dtype=BF16, device=dev)[offset:].view_as(x).copy_(x)
+            out.append((ops.latent_step(q, moved, nw, w, cache, H, d, window, 0.3, pos, 1e-5, rope, out=torch.empty(B, H * dv, dtype=BF16, device=dev)), cache))
+        assert torch.equal(out[0][1], out[1][1]) and not torch.equal(out[0][1], rows)
+        assert torch.equal(out[0][0], out[1][0])
+
+
 # ---- experts ----
 def expert_case(n, D, F, E, top, dtype, seed=0):
     h, router = rnd(n, D, seed=seed, dtype=dtype), rnd(E, D, seed=seed + 1, dtype=dtype, scale=2 * D ** -0.5)
