@@ -124,9 +124,10 @@ def linear_attn_step(q, k, v, kv_state, k_state, eps: float = 1e-12, out: Option
     if out is None:
         y, y_at = _empty(q, q.dtype, B, H, 1, dv), (H * dv, dv)
     else:
-        y, y_at = out, (out.stride(0), out.stride(1))
+        y = out
         if tuple(y.shape) != (B, H, 1, dv) or y.dtype != q.dtype or y.device != q.device or y.stride(-1) != 1:
             raise ValueError(f"out must be a ({B}, {H}, 1, {dv}) {q.dtype} tensor on {q.device}")
+        y_at = (y.stride(0), y.stride(1))
     with _on_device(q.device):
         _lib.check(_lib.lib().based_linear_attn_step(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), kv_state.data_ptr(), k_state.data_ptr(), y.data_ptr(),

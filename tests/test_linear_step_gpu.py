@@ -67,3 +67,14 @@ def test_step_rejects_bad_shapes(dev):
     ks = torch.zeros(1, 1, 1, 1, 273, device=dev)
     with pytest.raises(ValueError):
         ops.linear_attn_step(q, q, v, kv, ks)  # dv not a multiple of 16
+
+
+@pytest.mark.parametrize("shape", [(), (64,), (2, 64), (2, 3, 64), (2, 3, 1, 64, 1), (2, 3, 1, 48)])
+def test_step_rejects_an_output_of_another_shape(dev, shape):
+    from based_amd import ops
+
+    q, v = torch.zeros(2, 3, 1, 16, device=dev, dtype=torch.bfloat16), torch.zeros(2, 3, 1, 64, device=dev, dtype=torch.bfloat16)
+    kv, ks = torch.zeros(2, 3, 1, 64, 273, device=dev), torch.zeros(2, 3, 1, 1, 273, device=dev)
+    with pytest.raises(ValueError, match="out must be"):
+        ops.linear_attn_step(q, q, v, kv, ks, out=torch.zeros(shape, device=dev, dtype=torch.bfloat16))
+    assert not kv.any() and not ks.any()
