@@ -669,7 +669,7 @@ __global__ __launch_bounds__(256, RT <= 4 ? 2 : 1) void latent_step_f32_kernel(c
     if (__any(mx > m_run)) {
       mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float m_new = fmaxf(m_run, mx), alpha = __builtin_amdgcn_exp2f((m_run - m_new) * kLog2e);
+      const float m_new = fmaxf(m_run, mx), alpha = __builtin_amdgcn_exp2f((m_run - (m_new == -INFINITY ? 0.f : m_new)) * kLog2e);
       m_run = m_new;
       l_run *= alpha;
 #pragma unroll
@@ -677,9 +677,10 @@ __global__ __launch_bounds__(256, RT <= 4 ? 2 : 1) void latent_step_f32_kernel(c
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[t][j] *= alpha;
     }
+    const float base = m_run == -INFINITY ? 0.f : m_run;  // (no score of 16 keys needs to be a finite one: such keys count for nothing)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      p[i] = __builtin_amdgcn_exp2f((p[i] - m_run) * kLog2e);
+      p[i] = __builtin_amdgcn_exp2f((p[i] - base) * kLog2e);
       l_run += p[i];
     }
 #pragma unroll

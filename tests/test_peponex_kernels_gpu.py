@@ -426,6 +426,28 @@ def test_fp32_steps_on_the_matrix_unit(dev, H, d, r, dv, R, window, keys):
             close(o[b], want, 1e-5)
 
 
+@pytest.mark.parametrize("first,last", [(0, 16), (16, 32), (0, 64), (48, 80), (3, 90)])
+def test_fp32_steps_over_keys_that_count_for_nothing(dev, first, last):
+    """Scores of minus infinity, of all of the 16 keys that a wavefront takes at a time and of others: the softmax of those that are left."""
+    from based_amd import ops
+
+    B, H, d, r, dv, R, keys = 2, 16, 8, 4, 16, 64, 100
+    q, x, rows = rnd(B, H, r + d, seed=1), rnd(B, R + r, seed=2), rnd(B, keys, R + r, seed=5)
+    q[..., :r] = torch.tensor([1.0, 0.0, 0.0, 0.0])
+    q[:, ::2, 0] = 0.5
+    rows[:, first:last, R] = -float("inf")
+    nw, w = rnd(R, seed=3, scale=0.2, mean=1.0), rnd(H * (r + d + dv), R, seed=4, scale=R ** -0.5)
+    rope = (torch.ones(keys, r // 2, device=dev), torch.zeros(keys, r // 2, device=dev), True)
+    cache, pos = rows.to(dev), torch.full((B,), keys - 1, dtype=torch.int32, device=dev)
+    out = ops.latent_step(q.view(B, -1).to(dev), x.to(dev), nw.to(dev), w.to(dev), cache, H, d, keys, 0.3, pos, 1e-5, rope, out=torch.empty(B, H * dv, device=dev))
+    per = w.double().view(H, r + d + dv, R)
+    for b in range(B):
+        c = cache[b].double().cpu()
+        s = torch.matmul(torch.matmul(q[b, :, None, r:].double(), per[:, r:r + d])[:, 0], c[:, :R].T) + q[b, :, :1].double() * c[:, R]
+        want = torch.matmul(per[:, r + d:], ((0.3 * s).softmax(-1) @ c[:, :R]).unsqueeze(-1))[..., 0].reshape(-1)
+        close(out[b].double().cpu(), want, 1e-5)
+
+
 @pytest.mark.parametrize("H,d,r,dv,R,window,keys", [
     (16, 64, 32, 64, 256, 512, 700), (1, 8, 8, 8, 8, 1, 3), (3, 24, 8, 16, 64, 63, 200), (2, 20, 16, 8, 72, 64, 66), (5, 136, 0, 40, 136, 65, 90),
     (4, 72, 64, 16, 248, 128, 300), (6, 264, 24, 24, 264, 200, 260), (3, 130, 64, 8, 512, 700, 800), (16, 16, 32, 16, 256, 1000, 500)])
