@@ -27,6 +27,7 @@
 // an operand keeps 16 bits and the sums 24.
 #include <type_traits>
 
+#include "lds_limit.hpp"
 #include "stream_common.hpp"
 
 namespace based {
@@ -1344,13 +1345,6 @@ void launch_decay_join(const DecayScanArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(decay_join_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, a);
 }
 
-template <typename Kernel> int allow_lds(Kernel kernel, size_t bytes) {
-  if (bytes <= 64 * 1024) return BASED_OK;
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-  BASED_REQUIRE(e == hipSuccess, BASED_ERR_LAUNCH, "decay_scan: %zu bytes of LDS refused: %s", bytes, hipGetErrorString(e));
-  return BASED_OK;
-}
-
 template <int DT, int HALVES, int COLS, bool CHANNEL, bool FOLD> int launch_decay_mfma(const DecayScanArgs& a, hipStream_t s) {
   void (*scan)(DecayScanArgs);
   void (*states)(DecayScanArgs);
@@ -1364,11 +1358,10 @@ template <int DT, int HALVES, int COLS, bool CHANNEL, bool FOLD> int launch_deca
     scan = decay_head_kernel<DT, HALVES, false, FOLD>, states = decay_head_kernel<DT, HALVES, true, FOLD>;
     bytes = state_bytes = sizeof(HeadLds<DT, HALVES>);
   }
-  static const int allowed = [&] {
-    const int rc = allow_lds(scan, bytes);
-    return rc != BASED_OK ? rc : allow_lds(states, state_bytes);
-  }();
-  if (allowed != BASED_OK) return allowed;
+  static LdsAllowed scan_allowed, states_allowed;
+  hipError_t e = allow_lds(reinterpret_cast<const void*>(scan), bytes, scan_allowed);
+  if (e == hipSuccess && a.segs > 1) e = allow_lds(reinterpret_cast<const void*>(states), state_bytes, states_allowed);
+  BASED_REQUIRE(e == hipSuccess, BASED_ERR_LAUNCH, "decay_scan: %zu bytes of LDS refused: %s", bytes, hipGetErrorString(e));
   dim3 grid((unsigned)(a.B * a.H), (unsigned)((a.dv + COLS - 1) / COLS), (unsigned)a.segs);
   if (a.segs > 1) {
     dim3 all_but_last = grid;

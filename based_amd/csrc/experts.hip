@@ -13,8 +13,7 @@
 //   expert_route_row  the same for few tokens, with the norm in front of the layer
 //   expert_f32      fp32: 16 choices of one expert at a time on fp32 MFMA
 //   expert_rows     few tokens, or rows that are no whole 16-byte pieces: dot products, one choice at a time
-#include <atomic>
-
+#include "lds_limit.hpp"
 #include "stream_common.hpp"
 
 namespace based {
@@ -1052,24 +1051,10 @@ template <bool PAIRED> __global__ __launch_bounds__(256, 2) void expert_gemm_dir
   }
 }
 
-constexpr int kMaxDevices = 64;
-
-// Lets a kernel have `bytes` of LDS, once for each device.
-static int allow_lds(const void* kernel, int bytes, std::atomic<bool> (&allowed)[kMaxDevices]) {
-  int dev = 0;
-  BASED_REQUIRE(hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices, BASED_ERR_LAUNCH, "experts: cannot identify the current device");
-  if (!allowed[dev].load(std::memory_order_acquire)) {
-    const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    BASED_REQUIRE(e == hipSuccess, BASED_ERR_LAUNCH, "experts: %d bytes of LDS refused: %s", bytes, hipGetErrorString(e));
-    allowed[dev].store(true, std::memory_order_release);
-  }
-  return BASED_OK;
-}
-
 template <bool PAIRED, bool TAIL> int launch_expert_gemm_large(ExpertGemmArgs a, hipStream_t s) {
-  static std::atomic<bool> allowed[kMaxDevices];
-  const int rc = allow_lds(reinterpret_cast<const void*>(expert_gemm_large_kernel<PAIRED, TAIL>), kLargeLds, allowed);
-  if (rc != BASED_OK) return rc;
+  static LdsAllowed allowed;
+  const hipError_t e = allow_lds(reinterpret_cast<const void*>(expert_gemm_large_kernel<PAIRED, TAIL>), kLargeLds, allowed);
+  BASED_REQUIRE(e == hipSuccess, BASED_ERR_LAUNCH, "experts: %d bytes of LDS refused: %s", kLargeLds, hipGetErrorString(e));
   a.col_tiles = PAIRED ? (a.F + 127) / 128 : (a.F + 255) / 256;
   // (parts beyond the first of a tile: less than one for each of the 32 compute units of a die)
   const unsigned per_die = (unsigned)((a.col_tiles * a.tiles + kDies - 1) / kDies + kDieUnits);
@@ -1091,9 +1076,9 @@ template <bool PAIRED> int launch_expert_gemm(ExpertGemmArgs a, hipStream_t s) {
     hipLaunchKernelGGL(expert_gemm_kernel<PAIRED>, grid, dim3(256), 0, s, a);
     return BASED_OK;
   }
-  static std::atomic<bool> allowed[kMaxDevices];
-  const int rc = allow_lds(reinterpret_cast<const void*>(expert_gemm_direct_kernel<PAIRED>), kDirectLds, allowed);
-  if (rc != BASED_OK) return rc;
+  static LdsAllowed allowed;
+  const hipError_t e = allow_lds(reinterpret_cast<const void*>(expert_gemm_direct_kernel<PAIRED>), kDirectLds, allowed);
+  BASED_REQUIRE(e == hipSuccess, BASED_ERR_LAUNCH, "experts: %d bytes of LDS refused: %s", kDirectLds, hipGetErrorString(e));
   hipLaunchKernelGGL(expert_gemm_direct_kernel<PAIRED>, grid, dim3(256), kDirectLds, s, a);
   return BASED_OK;
 }
