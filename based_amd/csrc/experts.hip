@@ -819,7 +819,10 @@ __device__ __forceinline__ void large_part(const ExpertGemmArgs& a, const Expert
   constexpr int KS = kGemmK, XL = R / 64, WL = CW / 64, WN = CW / 32, RW = R * WN / 8, MT = RW / 16, COLS = PAIRED ? CW / 2 : CW;
   constexpr int SLOT = (CW + R) * KS, DEPTH = kPartElements / SLOT, FLYING = (DEPTH - 2) * (XL + WL);
   static_assert(DEPTH >= 3 && FLYING < 16 && MT >= 1, "");
-  if (r0 >= t.rows) return;  // (no barrier left)
+  if (r0 >= t.rows) {  // (no barrier left)
+    __builtin_amdgcn_s_waitcnt(0x0070);  // (scores: nothing may come into LDS that is no longer this workgroup's)
+    return;
+  }
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, quad = lane >> 4;
   const int wn = wave % WN, wm = wave / WN, f0 = t.f0 + col * COLS;
   const int piece = (lane ^ (lane >> 4)) & 7;  // (rows of an odd group of eight: bit 2 the other way round)
@@ -948,7 +951,7 @@ template <bool PAIRED, bool TAIL> __global__ __launch_bounds__(512, 2) void expe
   const int r0 = part % rows * 64, col = part / rows;
   if (parts / rows == 1) return large_part<64, 256, PAIRED, TAIL>(a, t, lds, slot_of, r0, 0);
   if (parts / rows == 2) return large_part<64, 128, PAIRED, TAIL>(a, t, lds, slot_of, r0, col);
-  if (col < 4) large_part<64, 64, PAIRED, TAIL>(a, t, lds, slot_of, r0, col);
+  large_part<64, 64, PAIRED, TAIL>(a, t, lds, slot_of, col < 4 ? r0 : kLargeRows, col);
 }
 
 // The same tiles of 32 rows with 64 rows of the weights (PAIRED: 32 up, 32 gate), rows and weights straight into LDS, rounds of 128 channels three
