@@ -584,6 +584,19 @@ __global__ __launch_bounds__(NT) void gated_delta_step_kernel(const DeltaStepArg
 
 static bool delta_short(const DeltaArgs& a) { return a.vec && a.d <= 128 && a.L <= kShortBlocks * kBlk; }
 
+// Whether tiles of one wavefront go with one set of registers.  A SIMD holds three of them with one set and two with two (64 channels), or two and
+// one (128), so that one set saves a round where there are more tiles than that; but a block waits for its loads then, which long prompts feel.  Kernels of a
+// call, us, two sets / one, by tiles (16 columns of a head) and tokens.  64 channels: 2,048, 200 68 / 63.5, 400 110.6 / 108.6, 500 130 / 132, 732 181 /
+// 186, 1,500 353 / 377; 3,072, 400 159 / 147, 1,000 364 / 361, 1,500 533 / 540; 4,096, 200 117 / 109, 400 202 / 198, 732 347 / 357; 6,144, 400 298 / 285,
+// 1,000 711 / 711; fewer: 1,280, 1,232 273 / 283.  128 channels: 1,088, 65 64 / 49, 732 397 / 334; 2,048, 400 248 / 202; 2,304, 200 199 / 181, 800 661 / 648;
+// 2,560, 100 123 / 103, 150 151 / 152, 400 360 / 370; 3,072, 100 124 / 115, 150 153 / 157, 400 364 / 375, 800 687 / 721 (the second of two rounds is half
+// empty, for three whole ones); 3,200, 400 472 / 378; 5,120, 400 603 / 562; 8,192, 400 999 / 777; fewer: 1,024, 896 275 / 285.
+static bool delta_one_set(int rb, long tiles, int L) {
+  if (rb > 4) return tiles > 1024 && !(tiles > 2400 && tiles <= 3072 && L > 110);
+  const bool fewer_rounds = (tiles + 3071) / 3072 < (tiles + 2047) / 2048;
+  return tiles >= 2048 && L <= (fewer_rounds ? 1000 : 400);
+}
+
 template <typename T, int RB, int RS, int LAY> void launch_delta_scan_split(const DeltaArgs& a, hipStream_t s) {
   const int cols = 16 * (4 / RS);
   const dim3 grid((unsigned)(a.B * a.H), (unsigned)((a.dv + cols - 1) / cols));
@@ -593,11 +606,8 @@ template <typename T, int RB, int RS, int LAY> void launch_delta_scan_split(cons
       return;
     }
   }
-  // More wavefronts than find registers for two sets: one set takes less of them.  Kernels of a call, us, two sets / one, by tiles: 128 x 128: 1,280,
-  // 800 tokens 433 / 364; 4,096, 70 tokens 128 / 96; 64 x 128: 2,048, 200 tokens 67.3 / 63.2; 4,096, 120 tokens 77.5 / 74.8; fewer: 128 x 64, 1,024,
-  // 896 tokens 275 / 285; 64 x 128, 1,280, 1,232 tokens 273 / 283.
   if constexpr (sizeof(T) == 2 && RS == 1 && LAY == 2 && (RB == 4 || RB == 8)) {
-    if ((long)a.B * a.H * ((a.dv + 15) / 16) >= (RB > 4 ? 1025 : 2048)) {
+    if (delta_one_set(RB, (long)a.B * a.H * ((a.dv + 15) / 16), a.L)) {
       hipLaunchKernelGGL((gated_delta_scan_kernel<T, RB, RS, LAY, kDeltaOneSet>), grid, dim3(256), 0, s, a);
       return;
     }
@@ -639,8 +649,9 @@ template <typename T, int RB> void launch_delta_scan(const DeltaArgs& a, hipStre
 template <typename T> void launch_delta(const DeltaArgs& a, hipStream_t s) {
   const long items = (long)a.B * a.H * a.blocks;
   const dim3 grid((unsigned)((items + 3) / 4));
-  if (delta_short(a)) {
-  } else if (a.vec)
+  if (delta_short(a))
+    ;  // (the scan does it)
+  else if (a.vec)
     hipLaunchKernelGGL((gated_delta_prepare_kernel<T, true>), grid, dim3(256), 0, s, a);
   else
     hipLaunchKernelGGL((gated_delta_prepare_kernel<T, false>), grid, dim3(256), 0, s, a);

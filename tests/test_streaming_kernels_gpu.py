@@ -242,6 +242,23 @@ def test_gated_delta_scan_of_short_portions(dev, dtype, B, H, G, d, dv):
         assert rel_l2(o[i], ref) < 3e-6  # sums of up to 128 products, and of the portions before: some tens of 2^-24
 
 
+@pytest.mark.parametrize("B,H,L,d,dv", [(32, 16, 400, 64, 64), (32, 16, 401, 64, 64), (33, 16, 401, 64, 64), (33, 16, 1001, 64, 64), (37, 16, 110, 128, 64),
+                                        (38, 16, 110, 128, 64), (38, 16, 111, 128, 64), (49, 16, 111, 128, 64)])
+def test_gated_delta_scan_of_many_tiles(dev, B, H, L, d, dv):
+    """Both sides of the rule for one set of registers and two: by tiles, rounds and tokens."""
+    from based_amd import ops
+
+    q, k, v = (rnd(s, B, L, H * n, dtype=BF16) for s, n in ((61, d), (62, d), (63, dv)))
+    a, b, al, db = rnd(64, B, L, H, dtype=BF16), rnd(65, B, L, H, dtype=BF16), (rnd(66, H) - 1).to(BF16), rnd(67, H, dtype=BF16)
+    c, n, state = torch.cat([q, k, v], -1).to(dev), H * d, torch.full((B, H, d, dv), float("nan"), device=dev)
+    o = ops.gated_delta_scan(c[..., :n], c[..., n:2 * n], c[..., 2 * n:], a.to(dev), b.to(dev), al.to(dev), db.to(dev), state, H, H, True)
+    for i in (0, B - 1):
+        g = torch.exp(-torch.exp(al.double()) * O.softplus(a[i].double() + db.double()))
+        unit = lambda x: O.unit(x[i].double().view(L, H, d))  # noqa: E731
+        ref = O.delta_rule(unit(q) * d ** -0.5, unit(k), v[i].double().view(L, H, dv), g, torch.sigmoid(b[i].double()))
+        assert rel_l2(o[i], ref) < 3e-6  # sums of up to 128 products, and of the tokens before: some tens of 2^-24
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("W,blocks", [(64, 1), (160, 2), (96, 3), (256, 1), (54, 2), (8, 8), (520, 2)])
 @pytest.mark.parametrize("B", [1, 11])
