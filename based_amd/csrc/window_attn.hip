@@ -84,18 +84,19 @@ template <bool HALF> struct Turn8 {
       load_vec<float, 4>((a.rot > 0 ? a.sin_t : reinterpret_cast<const float*>(a.kv)) + t, sn);
     }
   }
+  // (which of the two products is rounded is written out: left to the compiler, kernels differ in it)
   __device__ __forceinline__ void apply(float (&x)[8], int c, const WindowArgs& a) const {
     if (c >= a.rot) return;
     if constexpr (HALF) {
       const float sgn = c < a.rot / 2 ? -1.f : 1.f;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = x[j] * cs[j] + sgn * partner[j] * sn[j];
+      for (int j = 0; j < 8; ++j) x[j] = __builtin_fmaf(x[j], cs[j], (sgn * partner[j]) * sn[j]);
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float u = x[2 * j], v = x[2 * j + 1];
-        x[2 * j] = u * cs[j] - v * sn[j];
-        x[2 * j + 1] = v * cs[j] + u * sn[j];
+        x[2 * j] = __builtin_fmaf(u, cs[j], -(v * sn[j]));
+        x[2 * j + 1] = __builtin_fmaf(v, cs[j], u * sn[j]);
       }
     }
   }
@@ -1686,7 +1687,7 @@ extern "C" BASED_API int based_window_attn_prefill(
   BASED_REQUIRE(items < (1ll << 32), BASED_ERR_SHAPE, "window_attn_prefill: grid too large");
   const bool fill = vec ? window_bf16_fills(a) : window_f32(a, io_dtype) && !window_f32_few(a) && window_f32_fills(a);
   if (fill)
-    ;
+    ;  // (the attention does it)
   else if (vec) {
     const int64_t widest = D > DV ? D : DV;
     widest <= 64 ? launch_kv_write<8>(a, s) : widest <= 128 ? launch_kv_write<16>(a, s) : launch_kv_write<32>(a, s);

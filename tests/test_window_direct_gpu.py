@@ -107,3 +107,24 @@ def test_cache_that_the_attention_fills(dev, H, G, B, L, start, window, rot, hal
         want = want / (want.square().mean(-1, keepdim=True) + 1e-5).sqrt()
     # eight significant bits: an element is rounded by at most 2^-8 of itself
     assert float(((cache[:, :n, :, d:].double() - want).norm(dim=-1) / want.norm(dim=-1)).max()) < 2 ** -8
+
+
+@pytest.mark.parametrize("H,G,B,L,window,rot,half,norm", [
+    (16, 16, 28, 52, 129, 64, False, True), (16, 4, 32, 64, 129, 64, False, False), (16, 16, 28, 52, 129, 64, True, True), (16, 4, 3, 200, 65, 32, True, False)])
+def test_keys_are_turned_to_the_same_numbers(dev, H, G, B, L, window, rot, half, norm):
+    """Cache and outputs of a portion whose keys and values the attention leaves in the cache, and of the same one with a launch for that in front."""
+    from based_amd import ops
+    from based_amd.mixers.window_attention import _ExactRotary
+
+    d, g = 64, torch.Generator().manual_seed(L)
+    kw = dict(rope=_ExactRotary(rot, base=100.0, interleaved=not half).tables(L, dev), value_norm_eps=1e-5 if norm else None)
+    x = torch.randn(B, L, H * d + 2 * G * d, generator=g).bfloat16().to(dev)
+    got = []
+    for inside in (False, True):  # (a launch where keys and values lie in the output's rows)
+        cache, room = torch.zeros(B, L, G, 2 * d, dtype=torch.bfloat16, device=dev), x.clone()
+        own = room if inside else x
+        k, v = own[..., H * d:(H + G) * d], own[..., (H + G) * d:]
+        ops.window_attn_prefill(x[..., :H * d], k, v, cache, H, G, window, d ** -0.5, 0, out=room[..., :H * d], **kw)
+        got.append((room[..., :H * d].clone(), cache))
+    assert torch.equal(got[0][1], got[1][1]) and bool(got[0][1].any())
+    assert torch.equal(got[0][0], got[1][0])
