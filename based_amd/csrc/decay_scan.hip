@@ -8,7 +8,8 @@
 // with silu on q, k and v first where asked for.  Decays come as base-2 logarithms.  The state lies by
 // value channel, (B, H, dv, dp): rows of dp >= d key channels.
 //
-//   decay_scan_mfma   bf16: walks 64 tokens at a time with the state in MFMA accumulators, 16 value channels
+//   decay_channel, decay_head
+//                     bf16: walk 64 tokens at a time with the state in MFMA accumulators, 16 value channels
 //                     per wavefront.  Long sequences are cut into segments: a first pass leaves what every
 //                     segment adds to the state, `decay_join` turns that into the state at every segment's
 //                     start, and the second pass starts there; few segments it puts together itself.
@@ -24,7 +25,7 @@
 //   * s in an earlier 16 tokens: k_s decayed to the end of its 16, q_t to the start of its own, and to q
 //     also what lies between.
 // fp32 numbers enter a bf16 product as pairs (a number rounded to bf16, and the rest rounded to bf16), so
-// an operand keeps 16 bits and the sums 24.
+// an operand keeps 16 bits and the sums 24; the weights inside 16 tokens are formed in fp32.
 #include <type_traits>
 
 #include "lds_limit.hpp"
@@ -53,15 +54,11 @@ struct DecayScanArgs {
   int narrow;            // workgroups of 64 value channels, not of 128 (channel decays, more than 64 key channels)
 };
 
-template <int CTRL> __device__ __forceinline__ float row_moved(float x) {  // lanes without a source receive 0
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
-}
 // Products along the 16 lanes of a row, of several independent numbers at once.  A DPP multiplication leaves a lane
 // without a source as it is, which is the multiplication by one that is wanted; the compiler has no builtin that
 // says so.  A register must not be read through DPP in the two issue slots after it was written: four numbers in turn
 // keep that distance by themselves, the first ones are kept from what stands before by the s_nop.
-//   prefix[i]: product over lanes 0 .. l of w[i];  suffix[i]: over lanes l .. 15
-//   before[i] *= prefix of the lane before (nothing for lane 0);  after[i] *= suffix of the lane behind (nothing for lane 15)
+//   suffix[i]: product over lanes l .. 15 of w[i];  after[i] *= suffix of the lane behind (nothing for lane 15)
 #define BASED_ROW_STEP(ctrl) \
   "v_mul_f32_dpp %0, %0, %0 " ctrl " row_mask:0xf bank_mask:0xf\n\t" \
   "v_mul_f32_dpp %1, %1, %1 " ctrl " row_mask:0xf bank_mask:0xf\n\t" \
@@ -80,11 +77,6 @@ __device__ __forceinline__ void row_suffix4(float* suffix, float* after) {
 }
 #undef BASED_ROW_STEP
 #undef BASED_ROW_LAST
-// sum over the four lanes l16, l16 + 16, + 32, + 48, in all of them
-__device__ __forceinline__ float quad_rows_sum(float x) {
-  x += __shfl_xor(x, 16, 64);
-  return x + __shfl_xor(x, 32, 64);
-}
 
 __device__ __forceinline__ f32x4 mfma_16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 // two numbers as packed pairs of bf16: rounded, and what the rounding left
@@ -140,12 +132,16 @@ struct HeadPowers {
 // weights nor queries go through LDS, the state's tiles of 16 value channels to a wavefront each: two barriers to 64 tokens, one behind what is written
 // of each piece and one behind what is read.
 //
-// What bounds it: a wavefront issues an instruction in five cycles, whatever it waits for, so 64 tokens are a chain of 11,000 to 14,000 cycles; wavefronts
-// beside each other on a SIMD take next to nothing from one another up to three.  So channels are dealt to more wavefronts where heads are few, prompts
-// are cut into segments of a piece where that leaves compute units idle (decay_channel_segments), and nothing is kept in memory inside the loop:
-// a value fetched back from there waits for the tokens that were asked for before it (17 of them: 68.6 us for 62.9).
-// us before (tokens passed along, four barriers, segments of four pieces) and now: 4 x 2048 tokens, 16 heads of 64: 70.7, 54.6; 2 x 768: 46.7, 22.7;
-// 30 x 513: 123, 71; 2 x 27, 12 heads: 10.2, 8.3; 4 x 2048, 8 heads of 128: 100, 91; 16 x 1024: 184, 113; 2 x 133: 42.4, 24.8.
+// What bounds it: 64 tokens are a chain of instructions, two barriers and products that wait for each other, 10,000 cycles and more.  Heads of 64, us a
+// piece of 64 tokens in one chain: 4.5 with one workgroup of eight wavefronts, half of the channels each, to a compute unit; with workgroups of four
+// wavefronts 7.4 for two of them, 10.3 for three, so that another wavefront on a SIMD adds some 3 us (a fourth workgroup has to wait: 14.1).  Heads of 128:
+// 6.9, workgroups of 128 value channels 9.8.  4 x 2048 tokens, 16 heads of 64, two workgroups to a compute unit: scan 43 us for four pieces and the
+// states of up to seven segments, vector unit busy 41 %, matrix unit 15 %, wavefronts waiting for 40 % of their time; state pass 17, 29 %, 9 %, 42 %.
+// So channels are dealt to more wavefronts where heads are few, prompts are cut into segments of a piece where that leaves compute units idle
+// (decay_channel_segments), and nothing is kept in memory inside the loop: a value fetched back from there waits for the tokens that were asked for
+// before it (17 of them: 68.6 us for 62.9).
+// us before (tokens passed along, four barriers, segments of four pieces) and now: 4 x 2048 tokens, 16 heads of 64: 75, 58; 2 x 768: 48, 23;
+// 30 x 513: 123, 72; 2 x 27, 12 heads: 10.4, 8.2; 4 x 2048, 8 heads of 128: 102, 90; 16 x 1024: 173, 120; 2 x 133: 42.3, 25.7.
 template <int DT, int HALVES, int COLS> struct ChannelLds {
   static constexpr int CH = 32 * DT * HALVES, RS = CH + 8, VS = COLS + 8;
   static constexpr int OT = COLS / 16, OF = OT / HALVES;  // tiles of 16 value channels, and those a group of wavefronts finishes
@@ -1381,8 +1377,8 @@ static bool channel_split(int64_t B, int64_t H, int64_t DV, int64_t segs, int64_
 // More channels: workgroups of 64 value channels where the 98 KB of each find a compute unit of their own, of 128 beyond that, and where the call has
 // work space (by_channel) for twice the segments that way, each so much shorter that decays and keys worked out once for 128 channels count for
 // more than the launch that puts segments together and the longer piece.  Calls, us, of 64 / of 128, 8 heads of 128 (pieces of a segment of
-// 64): 1 x 4000 (4) 59 / 68; 4 x 1000 (4) 53 / 56; 6 x 500 (4) 50 / 52; 2 x 4000 (8) 94 / 90; 6 x 1000 (8) 88 / 80; 4 x 4000 (16) 166 / 145; 6 x
-// 2426 (19) 194 / 140; in one, 10 x 700 (11) 78.5 / 80.3, 10 x 1472 (23) 156 / 137; 14 x 1100, two of 128 for one, 124 / 151.
+// 64): 1 x 4000 (4) 65 / 67; 4 x 1000 (4) 58.6 / 58.7; 6 x 500 (4) 52.3 / 52.0; 2 x 4000 (8) 100 / 88; 6 x 1000 (8) 93 / 80; 4 x 4000 (16) 175 / 141; 6 x
+// 2426 (19) 204 / 138; in one, 10 x 700 (11) 83 / 81, 10 x 1472 (23) 166 / 136; 14 x 1100, one of 128 / two, 182 / 151.
 static bool channel_narrow(int64_t B, int64_t L, int64_t H, int64_t DV, bool by_channel) {
   const int64_t wgs = B * H * ((DV + 63) / 64), chunks = (L + kScanTokens - 1) / kScanTokens;
   if (wgs > 256) return false;
@@ -1467,11 +1463,13 @@ template <typename T, bool CHANNEL> void launch_decay_step(const DecayStepArgs& 
     launch_decay_step_rows<T, 64, CHANNEL>(a, s);
 }
 
-// Segments up to which those of the scan put the ones in front of them together themselves, heads of up to 64 channels: a launch less, and memory's
-// answer to four segments at a time in front of the scan, with channel decays also the segments' decays.  us with decay_join_kernel and without, 16 heads of 64,
-// channel decays: 4 x 2048 tokens (8 segments) 74.6, 72.9; 12 x 960 (3) 118.6, 110.7; 1 x 2304 (9) 53.0, 50.7; 1 x 2560 (10) 53.6, 52.3; 1 x 2816 (11)
-// 54.1, 55.0; 1 x 4096 (16) 57.3, 59.9.  Head decays: 1 x 2560 32.3, 28.7; 1 x 3584 (14) 34.5, 32.5; 1 x 4096 35.3, 34.0.  Heads of 128, channel
-// decays, 1 x 2000, 8 heads: 87.4, 96.0.
+// Segments up to which those of the scan put the ones in front of them together themselves, heads of up to 64 channels, of more with channel decays and
+// workgroups of 64 value channels: a launch less, and memory's answer to four (two) segments at a time in front of the scan, with channel decays
+// also the segments' decays.  Workgroups of 128 value channels go with the launch always.  us with decay_join_kernel and without.  Channel decays, 16 heads of
+// 64: 4 x 2048 tokens (8 segments) 61.1, 58.8; 12 x 960 (4) 78.8, 70.4; 1 x 2304 (9) 38.9, 36.7; 2 x 768 (10) 25.9, 22.6; 1 x 2560 (10) 39.7, 37.7; beyond
+// ten, 12 40.5, 39.1; 16 42.7, 42.5; 32 48.6, 53.3.  8 heads of 128: 4 x 500 (4) 39.1, 35.1; 2 x 1000 (8) 42.3, 40.0; 1 x 500 (8) 26.8, 27.5; 1 x 2000 (10)
+// 57.6, 57.4; 2 x 700, 2 heads (11) 27.3, 30.5; 1 x 2000 (16) 45.4, 48.3; 1 x 4000 (16) 61.8, 66.4.  Head decays: 1 x 2560 32.3, 28.7; 1 x 3584 (14) 34.5, 32.5;
+// 1 x 4096 35.3, 34.0.
 constexpr int kFoldSegmentsChannel = 10, kFoldSegmentsHead = 16;
 
 // Segments of a scan: enough workgroups to give every SIMD two wavefronts, none shorter than four pieces of 64 tokens.
@@ -1483,11 +1481,14 @@ static int decay_segments(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV
   return segs < 2 ? 1 : (int)segs;
 }
 
-// Those of a call that has work space by the rule of channel decays.  A piece of 64 tokens takes the scan about 4.5 us and the state pass 2, a launch
-// and the folding of some segments 3: pieces by themselves pay from four of them on (2 x 440 tokens, 12 heads of 64, us in segments of 1, 2 and
-// 4 pieces or in one: 16.2, 24.8, 34.9 (7 pieces); 5 x 320, 16 heads: 20.4, 25.1, 26.3), as long as the segments need no launch of their own to be put
-// together or are of four pieces anyway (1 x 4096, 16 heads: 42.6 in 16 of four, 47.9 in 32 of two).  Not where there are workgroups for
-// every compute unit without them: every token but those of the last segment is walked twice (30 x 513, 16 heads: 70.4, in two 83.0).
+// Those of a call that has work space by the rule of channel decays.  Where a compute unit has one workgroup, a piece of 64 tokens takes the scan about
+// 4.5 us and the state pass 2, a launch and the folding of some segments 3: pieces by themselves pay from four of them on (2 x 440 tokens, 12 heads of
+// 64, us in segments of 1, 2 and 4 pieces or in one: 16.8, 19.7, 30.1, 35.5; 5 x 320, 16 heads: 20.6, 20.3, 25.1, 27.0), as long as there are no more of
+// them than put themselves together or they are of four pieces anyway (1 x 4096, 16 heads: 42.5 in 16 of four, 48.6 in 32 of two; between the two, 1 x
+// 2560, 37.7 in ten of four, 32.3 in 14 of three).  Not where there are workgroups for every compute unit without them: every token but those of
+// the last segment is walked twice.  In one / in two, 16 heads, by workgroups, of 300, 960 and 2048 tokens: 480 43.2 / 52.6, 117 / 131, 243 / 282; 448
+// 43.6 / 52.0, 113 / 129, 232 / 276; 384 42.0 / 44.6, 112 / 105, 230 / 224; 320 41.7 / 43.5, 107 / 100, 227 / 203; 272 40.9 / 41.7, 107 / 98, 227 / 193:
+// from some 500 tokens on two would be the better ones up to 384.
 static int decay_channel_segments(int64_t B, int64_t L, int64_t H, int64_t D, int64_t DV) {
   if (L < BASED_DECAY_SEGMENTS_MIN) return 1;
   const int64_t chunks = (L + kScanTokens - 1) / kScanTokens;
@@ -1579,7 +1580,8 @@ static int decay_scan_call(bool by_channel, const void* q, const void* k, const 
     a.seg = work;
     a.seg_lw = work + B * H * a.segs * DV * state_row;
   }
-  const bool fold = vec && (D <= 64 || (channel_log2 != nullptr && a.narrow)) && a.segs > 1 && a.segs <= (channel_log2 != nullptr ? kFoldSegmentsChannel : kFoldSegmentsHead);
+  const bool fold = vec && (D <= 64 || (channel_log2 != nullptr && a.narrow)) && a.segs > 1 &&
+                    a.segs <= (channel_log2 != nullptr ? kFoldSegmentsChannel : kFoldSegmentsHead);
   a.wide = bits % 16 == 0 && D % 8 == 0 && DV % 8 == 0;
   if (vec) {
     const int rc = channel_log2 != nullptr ? launch_decay_channel(a, fold, s) : launch_decay_head(a, fold, s);

@@ -592,9 +592,9 @@ template <bool PAIRED> __global__ __launch_bounds__(256, 2) void expert_gemm_ker
 // last; what is left of a die's tiles after whole rounds of its compute units goes in parts, of 64 rows that are there and, where that gives every
 // part a compute unit of its own, of 128 or 64 rows of the weights.  8192 tokens of 1024 channels, 2 of 8 experts of 1024: 70 + 43 us (rests in
 // their experts' places, and parts of rows alone: 77 + 48; tiles of 128 x 256 through registers, two workgroups to a compute unit: 106 + 70);
-// 2048 rows to every expert, whole rounds alone, 65 + 39.  Calls, us, before and now: 8192 tokens 143 -> 130, 1000 49 -> 45, 500 41 -> 35;
-// 1 of 8 of 2048, 1000 53 -> 44; 4 of 16 of 512, 2000 69 -> 67.  A whole tile alone takes 29 us: its matrix instructions 22, at the rate that they reach by
-// themselves here (1.6 PFLOP/s), the rest in front of the first and behind the last.
+// 2048 rows to every expert, whole rounds alone, 65 + 39.  Calls in a recorded graph, us, before and now, in turn: 8192 tokens 150 -> 136,
+// 4096 94 -> 88.5, 1000 51 -> 47, 500 43 -> 36.7; 1 of 8 of 2048, 1000 54 -> 45; 4 of 16 of 512, 2000 71.5 -> 68.5.  A whole tile alone takes 29 us: its
+// matrix instructions 22, at the rate that they reach by themselves here (1.6 PFLOP/s), the rest in front of the first and behind the last.
 constexpr int kLargeRows = BASED_EXPERT_TILE_ROWS;
 constexpr int kDies = 8, kDieUnits = 32;
 constexpr int kHalf = 128 * kGemmK;  // elements of 128 rows of a round

@@ -962,8 +962,8 @@ static int latent_check(const char* who, const LatentArgs& a, int64_t last, int 
 }
 
 // Up to two workgroups to a compute unit.  Whole calls, us, with a launch for the queries and without, 16 heads, R = 256, by sequences and
-// keys (workgroups): 1, 129 (24): 16.2 / 12.2; 4, 512 (256): 16.9 / 13.2; 6, 512 (384): 17.1 / 15.1; 16, 129 (384): 16.0 / 14.2; 4, 1,024 (512): 18.0 /
-// 16.1; 24, 129 (576): 16.2 / 18.2; 12, 512 (768): 18.3 / 22.7.  Four heads to a workgroup take as long at 512 and 13.6 -> 14.8 at 256.
+// keys (workgroups): 1, 129 (24): 15.5 / 12.6; 4, 512 (256): 17.0 / 13.6; 6, 512 (384): 17.3 / 15.3; 16, 129 (384): 16.5 / 14.4; 4, 1,024 (512): 18.1 /
+// 16.0; 24, 129 (576): 16.6 / 18.6; 12, 512 (768): 18.7 / 22.6.  Four heads to a workgroup take as long at 512 and 13.6 -> 14.8 at 256.
 constexpr int kOwnHeads = 2;
 constexpr int64_t kOwnMax = 512;
 
@@ -1090,9 +1090,11 @@ extern "C" BASED_API int based_latent_step(const void* q, const void* x, const v
   const bool mfma = near && R % n == 0 && rot % n == 0 && c_sb % n == 0 && c_st % n == 0 && aligned_to(cache, 16) && aligned_to(work_q, 16) &&
                     aligned_to(work_part, 16);
   const bool mfma_bf16 = io_dtype == BASED_BF16 && mfma && latent_mfma_fits(a);
-  const bool own = mfma_bf16 && vec && x_sb % 8 == 0 && aligned_to(x, 16) && aligned_to(norm_w, 16) && (window < S ? window : S) <= 64 * splits && B * splits * ((H + kOwnHeads - 1) / kOwnHeads) <= kOwnMax;
-  if (own) {
-  } else if (tiles && D % 8 == 0 && rot % 8 == 0 && q_sb % 8 == 0 && aligned_to(q, 16))
+  const bool own = mfma_bf16 && vec && x_sb % 8 == 0 && aligned_to(x, 16) && aligned_to(norm_w, 16) && (window < S ? window : S) <= 64 * splits &&
+                   B * splits * ((H + kOwnHeads - 1) / kOwnHeads) <= kOwnMax;
+  if (own)
+    ;  // (the attention does it)
+  else if (tiles && D % 8 == 0 && rot % 8 == 0 && q_sb % 8 == 0 && aligned_to(q, 16))
     hipLaunchKernelGGL(latent_query_mfma_kernel, dim3((unsigned)(H * ((R + kQueryCols - 1) / kQueryCols) + kTileRows),
                        (unsigned)((B + kTileRows - 1) / kTileRows)), dim3(256), 0, s, a);
   else if (io_dtype == BASED_BF16)

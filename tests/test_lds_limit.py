@@ -1,4 +1,5 @@
-"""csrc/lds_limit.hpp against a runtime of its own: what a kernel may have of LDS is asked for on every device by itself, once, and again where it was refused."""
+"""csrc/lds_limit.hpp against a runtime of its own: what a kernel may have of LDS is asked for on every device by itself, once, and again where it
+was refused."""
 import os
 import shutil
 import subprocess
@@ -36,7 +37,8 @@ def test_every_device_is_asked(tmp_path):
     (tmp_path / "t.cpp").write_text(PROGRAM)
     rocm = os.path.dirname(os.path.dirname(os.path.realpath(build.HIPCC)))
     include = next(p for p in (os.path.join(rocm, "include"), "/opt/rocm/include") if os.path.exists(os.path.join(p, "hip", "hip_runtime_api.h")))
-    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-isystem", include, "-I", build.CSRC, str(tmp_path / "t.cpp"), "-o", str(tmp_path / "t")], check=True)
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-isystem", include, "-I", build.CSRC, str(tmp_path / "t.cpp"), "-o", str(tmp_path / "t")],
+                   check=True)
     assert subprocess.run([str(tmp_path / "t")]).returncode == 0
 
 
