@@ -991,6 +991,14 @@ template <typename T> void launch_latent_values(const LatentArgs& a, bool vec, h
     hipLaunchKernelGGL((latent_values_kernel<T, 1>), grid, dim3(256), 0, s, a);
 }
 
+// Whether a token's own rows may lie in the cache (bf16), as where a row is normed in its place.
+static bool latent_rows_meet(const LatentArgs& a) {
+  if (a.x_sb < 0 || a.c_sb < 0 || a.c_st < 0) return true;
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a.x), c = reinterpret_cast<uintptr_t>(a.cache);
+  const long W = a.R + a.rot;
+  return x < c + ((a.B - 1) * a.c_sb + (a.S - 1) * a.c_st + W) * 2 && c < x + ((a.B - 1) * a.x_sb + W) * 2;
+}
+
 static bool latent_mfma_fits(const LatentArgs& a) { return (a.R + a.rot + 31) / 32 <= 18 && (a.R + 63) / 64 <= 8; }
 
 static void launch_latent_step_mfma(const LatentArgs& a, bool own, hipStream_t s) {
@@ -1091,7 +1099,7 @@ extern "C" BASED_API int based_latent_step(const void* q, const void* x, const v
                     aligned_to(work_part, 16);
   const bool mfma_bf16 = io_dtype == BASED_BF16 && mfma && latent_mfma_fits(a);
   const bool own = mfma_bf16 && vec && x_sb % 8 == 0 && aligned_to(x, 16) && aligned_to(norm_w, 16) && (window < S ? window : S) <= 64 * splits &&
-                   B * splits * ((H + kOwnHeads - 1) / kOwnHeads) <= kOwnMax;
+                   B * splits * ((H + kOwnHeads - 1) / kOwnHeads) <= kOwnMax && !latent_rows_meet(a);  // (every workgroup reads x, one writes the row)
   if (own)
     ;  // (the attention does it)
   else if (tiles && D % 8 == 0 && rot % 8 == 0 && q_sb % 8 == 0 && aligned_to(q, 16))

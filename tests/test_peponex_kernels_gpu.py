@@ -426,6 +426,25 @@ def test_fp32_steps_on_the_matrix_unit(dev, H, d, r, dv, R, window, keys):
             close(o[b], want, 1e-5)
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("B,H,R,r", [(1, 16, 256, 32), (4, 6, 64, 16)])
+def test_steps_on_rows_in_their_place(dev, B, H, R, r, dtype):
+    """A token's row that lies in the cache where it is going to be: as from a copy of it."""
+    from based_amd import ops
+
+    d, dv, keys, at = 16, 16, 70, 60
+    q, rows = rnd(B, H * (r + d), seed=1, dtype=dtype).to(dev), rnd(B, keys, R + r, seed=2, dtype=dtype).to(dev)
+    nw, w = rnd(R, seed=3, dtype=dtype, scale=0.2, mean=1.0).to(dev), rnd(H * (r + d + dv), R, seed=4, dtype=dtype, scale=R ** -0.5).to(dev)
+    rope, pos = (torch.rand(keys, r // 2, device=dev), torch.rand(keys, r // 2, device=dev), True), torch.full((B,), at, dtype=torch.int32, device=dev)
+    got = []
+    for own in (False, True):
+        cache = rows.clone()
+        x = cache[:, at] if own else cache[:, at].clone()
+        got.append((ops.latent_step(q, x, nw, w, cache, H, d, keys, 0.3, pos, 1e-5, rope, out=torch.empty(B, H * dv, dtype=dtype, device=dev)), cache))
+    assert torch.equal(got[0][1], got[1][1]) and not torch.equal(got[0][1], rows)
+    assert torch.equal(got[0][0], got[1][0])
+
+
 @pytest.mark.parametrize("first,last", [(0, 16), (16, 32), (0, 64), (48, 80), (3, 90)])
 def test_fp32_steps_over_keys_that_count_for_nothing(dev, first, last):
     """Scores of minus infinity, of all of the 16 keys that a wavefront takes at a time and of others: the softmax of those that are left."""
