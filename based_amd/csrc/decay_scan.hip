@@ -1388,6 +1388,24 @@ static bool channel_narrow(int64_t B, int64_t L, int64_t H, int64_t DV, bool by_
   return chunks < 16 || 256 / (B * H * ((DV + 127) / 128)) < 3;
 }
 
+// Whether an output may lie in the rows of q, k or v: workgroups of 128 value channels are the only ones of their head, those of 64 would write what
+// others of it have yet to read.
+static bool decay_rows_meet(const DecayScanArgs& a) {
+  const auto span = [&](const void* p, long sb, long sl, long width, uintptr_t& lo, uintptr_t& hi) {
+    const long b = (a.B - 1) * sb, l = (a.L - 1) * sl;
+    lo = reinterpret_cast<uintptr_t>(p) + ((b < 0 ? b : 0) + (l < 0 ? l : 0)) * 2;
+    hi = reinterpret_cast<uintptr_t>(p) + ((b < 0 ? 0 : b) + (l < 0 ? 0 : l) + width) * 2;
+  };
+  uintptr_t o0, o1;
+  span(a.o, a.o_sb, a.o_sl, (long)a.H * a.dv, o0, o1);
+  const auto meets = [&](const void* p, long sb, long sl, long width) {
+    uintptr_t p0, p1;
+    span(p, sb, sl, width, p0, p1);
+    return p0 < o1 && o0 < p1;
+  };
+  return meets(a.q, a.q_sb, a.q_sl, (long)a.H * a.d) || meets(a.k, a.k_sb, a.k_sl, (long)a.H * a.d) || meets(a.v, a.v_sb, a.v_sl, (long)a.H * a.dv);
+}
+
 int launch_decay_head(const DecayScanArgs& a, bool fold, hipStream_t s) {
   if (a.d <= 32) return fold ? launch_decay_mfma<1, 1, 64, false, true>(a, s) : launch_decay_mfma<1, 1, 64, false, false>(a, s);
   if (a.d <= 64) return fold ? launch_decay_mfma<2, 1, 64, false, true>(a, s) : launch_decay_mfma<2, 1, 64, false, false>(a, s);
@@ -1580,6 +1598,7 @@ static int decay_scan_call(bool by_channel, const void* q, const void* k, const 
     a.seg = work;
     a.seg_lw = work + B * H * a.segs * DV * state_row;
   }
+  if (a.narrow && DV > 64 && decay_rows_meet(a)) a.narrow = 0;
   const bool fold = vec && (D <= 64 || (channel_log2 != nullptr && a.narrow)) && a.segs > 1 &&
                     a.segs <= (channel_log2 != nullptr ? kFoldSegmentsChannel : kFoldSegmentsHead);
   a.wide = bits % 16 == 0 && D % 8 == 0 && DV % 8 == 0;

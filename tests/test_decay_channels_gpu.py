@@ -73,6 +73,35 @@ def test_weights_inside_16_tokens_are_of_32_bits(dev, B, H, d, dv):
     assert ((out - want).norm() / want.norm()).item() < 2 ** -9 + 2 ** -10.5
 
 
+@pytest.mark.parametrize("B,L,H,channels", [(1, 40, 2, True), (3, 130, 4, True), (2, 700, 2, True), (2, 130, 3, False)])
+def test_outputs_in_the_place_of_queries(dev, B, L, H, channels):
+    """By the entry points themselves: heads of 128 whose outputs are written where their queries lie, as from a copy of these."""
+    from based_amd import _lib
+
+    d, lib = 128, _lib.lib()
+    g = torch.Generator(device=dev).manual_seed(L)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    q, k, v, u, row = rnd(B, L, H * d).bfloat16(), rnd(B, L, H * d).bfloat16(), rnd(B, L, H * d).bfloat16(), rnd(H, d).bfloat16(), H * d
+    lw = -torch.exp(rnd(B, L, H * d) - 3)
+    heads, got = torch.stack([torch.full((H,), -0.1, device=dev), torch.full((H,), 2 ** -0.1, device=dev)]), []
+    for own in (False, True):
+        state, room = torch.zeros(B, H, d, d, device=dev), q.clone()
+        src = room if own else q
+        sizes, tail = (B, L, H, d, d, d), (L * row, row) * 4 + (0, 1, 0, torch.cuda.current_stream().cuda_stream)
+        work = torch.empty(max(1, lib.based_decay_scan_channels_work(0, *sizes, 0), lib.based_decay_scan_work_of(0, *sizes, 0)), device=dev)
+        if channels:
+            code = lib.based_decay_scan_channels(src.data_ptr(), k.data_ptr(), v.data_ptr(), lw.data_ptr(), u.data_ptr(), state.data_ptr(), work.data_ptr(),
+                                                 room.data_ptr(), *sizes, *tail)
+        else:
+            code = lib.based_decay_scan(src.data_ptr(), k.data_ptr(), v.data_ptr(), None, heads.data_ptr(), None, state.data_ptr(), work.data_ptr(),
+                                        room.data_ptr(), *sizes, *tail)
+        assert code == 0
+        got.append((room.double(), state))
+    rel = lambda a, b: ((a.double() - b.double()).norm() / b.double().norm()).item()  # noqa: E731
+    # (sums in another order may round to the other of two neighbours in bf16; keys enter the state as pairs of bf16, within 2^-17 of themselves)
+    assert rel(got[1][0], got[0][0]) < 2 ** -10 and rel(got[1][1], got[0][1]) < 2 ** -16
+
+
 def test_work_space_of_channel_decays():
     """Segments by the rule of channel decays for aligned bf16, those of the general form for everything else; none for short prompts."""
     from based_amd import _lib
