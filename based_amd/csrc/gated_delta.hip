@@ -582,7 +582,22 @@ __global__ __launch_bounds__(NT) void gated_delta_step_kernel(const DeltaStepArg
     y[c] = from_f32<T>(so[c] * r * to_f32(static_cast<const T*>(a.norm_w)[c]) * silu_exact(to_f32(gate[c])) * a.scale);
 }
 
-static bool delta_short(const DeltaArgs& a) { return a.vec && a.d <= 128 && a.L <= kShortBlocks * kBlk; }
+// Whether a portion goes in one launch (`size`: bytes of an element).  Every workgroup of a head prepares all blocks for itself, on SIMDs that hold one
+// wavefront of its tiles where these take the registers of fp32 or leave rows empty, which is less than the launch while there are not many of them; an
+// odd number of blocks costs the two launches one more.  Kernels of a call, us, two launches / one, by tiles (16 columns of a head), of 2 and 3 blocks.
+// fp32, heads of 96: 768 20.3 / 15.2, 27.9 / 18.7; 1,536, of four 41.1 / 42.8, 38.1 / 35.1; 2,304 37.1 / 40.0, 54.4 / 52.1; 3,840 57 / 65, 84 / 86.  128: 2,048
+// 34.1 / 32.6, 50 / 43; 3,072 45.3 / 47.7, 71 / 64; 8,192 104 / 127, 170 / 166; bf16, of 112: 2,560 50.9 / 51.1, 76 / 67; 4,096 64 / 69, 100 / 89.  Whole rows,
+// bf16, 128: 5,120 61.6 / 60.7, 83.0 / 81.5; 8,192 87 / 92, 123 / 124; 64: 5,120 34.9 / 32.7, 45.9 / 43.7; 8,192 47.6 / 48.6, 63.5 / 63.3.  fp32 of up to 64: 8,192 65
+// / 56, 95 / 71.
+static bool delta_short(const DeltaArgs& a, int size) {
+  if (!a.vec || a.d > 128 || a.L > kShortBlocks * kBlk) return false;
+  const long tiles = (long)a.B * a.H * ((a.dv + 15) / 16);
+  const bool odd = (a.L + kBlk - 1) / kBlk % 2 == 1;
+  if (size == 2 && (a.d == 64 || a.d == 128)) return tiles <= 6000;
+  if (a.d > 96) return odd || tiles <= 2560;
+  if (size == 4 && a.d > 64) return tiles <= (odd ? 3000 : 1024);
+  return true;
+}
 
 // Whether tiles of one wavefront go with one set of registers.  A SIMD holds three of them with one set and two with two (64 channels), or two and
 // one (128), so that one set saves a round where there are more tiles than that; but a block waits for its loads then, which long prompts feel.  Kernels of a
@@ -601,7 +616,7 @@ template <typename T, int RB, int RS, int LAY> void launch_delta_scan_split(cons
   const int cols = 16 * (4 / RS);
   const dim3 grid((unsigned)(a.B * a.H), (unsigned)((a.dv + cols - 1) / cols));
   if constexpr (LAY > 0 && RB <= 8) {
-    if (delta_short(a)) {
+    if (delta_short(a, sizeof(T))) {
       hipLaunchKernelGGL((gated_delta_scan_kernel<T, RB, RS, LAY, kDeltaShort>), grid, dim3(256), 0, s, a);
       return;
     }
@@ -649,7 +664,7 @@ template <typename T, int RB> void launch_delta_scan(const DeltaArgs& a, hipStre
 template <typename T> void launch_delta(const DeltaArgs& a, hipStream_t s) {
   const long items = (long)a.B * a.H * a.blocks;
   const dim3 grid((unsigned)((items + 3) / 4));
-  if (delta_short(a))
+  if (delta_short(a, sizeof(T)))
     ;  // (the scan does it)
   else if (a.vec)
     hipLaunchKernelGGL((gated_delta_prepare_kernel<T, true>), grid, dim3(256), 0, s, a);

@@ -216,7 +216,7 @@ def test_gated_delta_scan_column_splits(dev, B, H, dv):
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("B,H,G,d,dv", [(2, 2, 1, 16, 8), (1, 4, 4, 28, 40), (1, 6, 2, 44, 20), (3, 4, 4, 64, 64), (30, 4, 2, 64, 96), (40, 6, 6, 60, 72), (2, 3, 3, 96, 16),
                                         (30, 6, 3, 80, 128), (3, 4, 2, 128, 64), (34, 4, 4, 128, 64), (70, 4, 4, 128, 64), (70, 4, 1, 116, 64), (70, 8, 8, 64, 64),
-                                        (70, 8, 4, 56, 64)])
+                                        (70, 8, 4, 56, 64), (70, 4, 4, 96, 96), (90, 4, 2, 128, 128), (150, 6, 6, 112, 48), (128, 6, 3, 128, 128)])
 def test_gated_delta_scan_of_short_portions(dev, dtype, B, H, G, d, dv):
     """Portions of 1 to 64 tokens, which their scan prepares itself, one behind the other on one state, and of 65, which it does not: one block to four,
     the last of them whole or not, tiles of one wavefront, two and four, and so many of one that the longer portion goes with one set of registers;
