@@ -342,12 +342,32 @@ template <typename T> __global__ __launch_bounds__(512) void expert_route_row_ke
 
 // Tiles of BASED_EXPERT_TILE_ROWS rows: whole ones first, by expert, then what is left of every expert, the most rows first, so that the last to be
 // worked on are the smallest.  first_of: an expert's first whole tile; rest_of: the tile of what is left.  tile_first[0] is the number of whole ones.
+// Many experts have few tiles each, and what is left of them, by itself and dealt out in columns, reads rows and matrices again that are not in its
+// die's cache any more: there all tiles go by expert and count as whole.  Calls, us, rests last / by expert: 1 of 64 of 512, 8192 tokens 101 / 86; 4 of 64 of
+// 512, 6000 186 / 169; 2 of 64 of 1024, 6000 182 / 168; 4 of 128 of 512, 8192 293 / 262; 2 of 24 of 1024, 6000 126 / 118, 3000 87 / 88; 4 of 16 of 512, 8192
+// 159.6 / 158.8, 3000 76 / 74; 2 of 8 of 1024, 8192 138.9 / 140.2, 3000 69 / 68.
+constexpr int kManyExperts = 24;
+
 __device__ __forceinline__ void plan_large_tiles(const int* counts, uint32_t* scan, int* first_of, int* rest_of, int32_t* tile_first, int32_t* tile_expert, int E) {
   constexpr int ROWS = BASED_EXPERT_TILE_ROWS;
   const int e = threadIdx.x;
   const int count = e < E ? counts[e] : 0, whole = count / ROWS, rest = count % ROWS;
   sum_up((uint32_t)whole << 9 | (rest > 0), scan, E);  // whole tiles (less than 2^23) and rests (up to 256) at once
   const int wholes = (int)(scan[E - 1] >> 9), rests = (int)(scan[E - 1] & 511);
+  if (E >= kManyExperts) {
+    if (e < E) {
+      const int first = (int)((scan[e] >> 9) + (scan[e] & 511)) - whole - (rest > 0);
+      first_of[e] = first;
+      rest_of[e] = first + whole;
+      if (tile_expert != nullptr) {
+        for (int t = 0; t < whole; ++t) tile_expert[first + t] = e | ROWS << 8;
+        if (rest > 0) tile_expert[first + whole] = e | rest << 8;
+      }
+    }
+    if (e == 0 && tile_expert != nullptr) tile_first[0] = tile_first[E] = wholes + rests;
+    __syncthreads();
+    return;
+  }
   if (e < E) {
     const int first = (int)(scan[e] >> 9) - whole;
     int rank = 0;
@@ -589,7 +609,7 @@ template <bool PAIRED> __global__ __launch_bounds__(256, 2) void expert_gemm_ker
 
 // ---- the same with tiles of 256 rows and 256 rows of the weights (PAIRED: 128 up, 128 gate), rows and weights straight into LDS ----
 // One workgroup of eight wavefronts to a compute unit.  Whole tiles are dealt to the dies in runs, the rests of the experts behind them, the smallest
-// last; what is left of a die's tiles after whole rounds of its compute units goes in parts, of 64 rows that are there and, where that gives every
+// last (of many experts each in its place, plan_large_tiles); what is left of a die's tiles after whole rounds of its compute units goes in parts, of 64 rows that are there and, where that gives every
 // part a compute unit of its own, of 128 or 64 rows of the weights.  8192 tokens of 1024 channels, 2 of 8 experts of 1024: 70 + 43 us (rests in
 // their experts' places, and parts of rows alone: 77 + 48; tiles of 128 x 256 through registers, two workgroups to a compute unit: 106 + 70);
 // 2048 rows to every expert, whole rounds alone, 65 + 39.  Calls in a recorded graph, us, before and now, in turn: 8192 tokens 150 -> 136,

@@ -688,11 +688,11 @@ def test_experts_in_large_tiles(dev, n, D, F, E, top):
 @pytest.mark.parametrize("counts,D,F", [([382, 65, 1, 320], 1024, 1152), ([255, 129], 264, 3912), ([2504, 2916, 0, 64, 3], 128, 128),
                                         ([2049, 2112, 2113, 2176, 2177, 2303, 2048, 2078], 256, 1024), ([200, 100, 60, 40] * 8, 512, 1024),
                                         ([200, 100, 60, 40] * 8, 520, 1000), ([140, 190, 385, 30], 512, 1024),
-                                                        ([300, 20, 500, 190, 70] * 3, 256, 512)])
+                                                        ([300, 20, 500, 190, 70] * 3, 256, 512), ([0, 300, 20, 500, 190, 256] * 4, 256, 512)])
 def test_rests_of_large_tiles(dev, counts, D, F):
     """What whole tiles of 256 rows leave of every expert: 1, 64, 65, 128, 129 and 255 rows, none, in the last places of a die cut into sixteen parts
     of rows and weights, eight, four, two, and in places of whole tiles; an expert that nobody chooses; features and channels that end in a part; parts
-    of 64 rows of which there are none, whose workgroups leave at once."""
+    of 64 rows of which there are none, whose workgroups leave at once; few experts and many, whose tiles stay together."""
     from based_amd import _lib, ops
 
     n, E = sum(counts), len(counts)
