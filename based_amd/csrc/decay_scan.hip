@@ -1481,13 +1481,13 @@ template <typename T, bool CHANNEL> void launch_decay_step(const DecayStepArgs& 
     launch_decay_step_rows<T, 64, CHANNEL>(a, s);
 }
 
-// Segments up to which those of the scan put the ones in front of them together themselves, heads of up to 64 channels, of more with channel decays and
-// workgroups of 64 value channels: a launch less, and memory's answer to four (two) segments at a time in front of the scan, with channel decays
-// also the segments' decays.  Workgroups of 128 value channels go with the launch always.  us with decay_join_kernel and without.  Channel decays, 16 heads of
-// 64: 4 x 2048 tokens (8 segments) 61.1, 58.8; 12 x 960 (4) 78.8, 70.4; 1 x 2304 (9) 38.9, 36.7; 2 x 768 (10) 25.9, 22.6; 1 x 2560 (10) 39.7, 37.7; beyond
-// ten, 12 40.5, 39.1; 16 42.7, 42.5; 32 48.6, 53.3.  8 heads of 128: 4 x 500 (4) 39.1, 35.1; 2 x 1000 (8) 42.3, 40.0; 1 x 500 (8) 26.8, 27.5; 1 x 2000 (10)
-// 57.6, 57.4; 2 x 700, 2 heads (11) 27.3, 30.5; 1 x 2000 (16) 45.4, 48.3; 1 x 4000 (16) 61.8, 66.4.  Head decays: 1 x 2560 32.3, 28.7; 1 x 3584 (14) 34.5, 32.5;
-// 1 x 4096 35.3, 34.0.
+// Segments up to which those of the scan put the ones in front of them together themselves, heads of up to 64 channels, of more with channel decays
+// and workgroups of 64 value channels: a launch less, and memory's answer to four (two) segments at a time in front of the scan, with channel decays
+// also the segments' decays.  Workgroups of 128 value channels go with the launch always.  us with decay_join_kernel and without.  Channel decays, 16
+// heads of 64: 4 x 2048 tokens (8 segments) 61.1, 58.8; 12 x 960 (4) 78.8, 70.4; 1 x 2304 (9) 38.9, 36.7; 2 x 768 (10) 25.9, 22.6; 1 x 2560 (10)
+// 39.7, 37.7; beyond ten, 12 40.5, 39.1; 16 42.7, 42.5; 32 48.6, 53.3.  8 heads of 128: 4 x 500 (4) 39.1, 35.1; 2 x 1000 (8) 42.3, 40.0; 1 x 500 (8)
+// 26.8, 27.5; 1 x 2000 (10) 57.6, 57.4; 2 x 700, 2 heads (11) 27.3, 30.5; 1 x 2000 (16) 45.4, 48.3; 1 x 4000 (16) 61.8, 66.4.  Head decays: 1 x 2560
+// 32.3, 28.7; 1 x 3584 (14) 34.5, 32.5; 1 x 4096 35.3, 34.0.
 constexpr int kFoldSegmentsChannel = 10, kFoldSegmentsHead = 16;
 
 // Segments of a scan: enough workgroups to give every SIMD two wavefronts, none shorter than four pieces of 64 tokens.

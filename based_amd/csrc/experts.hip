@@ -343,9 +343,9 @@ template <typename T> __global__ __launch_bounds__(512) void expert_route_row_ke
 // Tiles of BASED_EXPERT_TILE_ROWS rows: whole ones first, by expert, then what is left of every expert, the most rows first, so that the last to be
 // worked on are the smallest.  first_of: an expert's first whole tile; rest_of: the tile of what is left.  tile_first[0] is the number of whole ones.
 // Many experts have few tiles each, and what is left of them, by itself and dealt out in columns, reads rows and matrices again that are not in its
-// die's cache any more: there all tiles go by expert and count as whole.  Calls, us, rests last / by expert: 1 of 64 of 512, 8192 tokens 101 / 86; 4 of 64 of
-// 512, 6000 186 / 169; 2 of 64 of 1024, 6000 182 / 168; 4 of 128 of 512, 8192 293 / 262; 2 of 24 of 1024, 6000 126 / 118, 3000 87 / 88; 4 of 16 of 512, 8192
-// 159.6 / 158.8, 3000 76 / 74; 2 of 8 of 1024, 8192 138.9 / 140.2, 3000 69 / 68.
+// die's cache any more: there all tiles go by expert and count as whole.  Calls, us, rests last / by expert: 1 of 64 of 512, 8192 tokens 101 / 86; 4
+// of 64 of 512, 6000 186 / 169; 2 of 64 of 1024, 6000 182 / 168; 4 of 128 of 512, 8192 293 / 262; 2 of 24 of 1024, 6000 126 / 118, 3000 87 / 88; 4 of
+// 16 of 512, 8192 159.6 / 158.8, 3000 76 / 74; 2 of 8 of 1024, 8192 138.9 / 140.2, 3000 69 / 68.
 constexpr int kManyExperts = 24;
 
 __device__ __forceinline__ void plan_large_tiles(const int* counts, uint32_t* scan, int* first_of, int* rest_of, int32_t* tile_first, int32_t* tile_expert, int E) {
@@ -609,12 +609,13 @@ template <bool PAIRED> __global__ __launch_bounds__(256, 2) void expert_gemm_ker
 
 // ---- the same with tiles of 256 rows and 256 rows of the weights (PAIRED: 128 up, 128 gate), rows and weights straight into LDS ----
 // One workgroup of eight wavefronts to a compute unit.  Whole tiles are dealt to the dies in runs, the rests of the experts behind them, the smallest
-// last (of many experts each in its place, plan_large_tiles); what is left of a die's tiles after whole rounds of its compute units goes in parts, of 64 rows that are there and, where that gives every
-// part a compute unit of its own, of 128 or 64 rows of the weights.  8192 tokens of 1024 channels, 2 of 8 experts of 1024: 70 + 43 us (rests in
-// their experts' places, and parts of rows alone: 77 + 48; tiles of 128 x 256 through registers, two workgroups to a compute unit: 106 + 70);
-// 2048 rows to every expert, whole rounds alone, 65 + 39.  Calls in a recorded graph, us, before and now, in turn: 8192 tokens 150 -> 136,
-// 4096 94 -> 88.5, 1000 51 -> 47, 500 43 -> 36.7; 1 of 8 of 2048, 1000 54 -> 45; 4 of 16 of 512, 2000 71.5 -> 68.5.  A whole tile alone takes 29 us: its
-// matrix instructions 22, at the rate that they reach by themselves here (1.6 PFLOP/s), the rest in front of the first and behind the last.
+// last (of many experts each in its place, plan_large_tiles); what is left of a die's tiles after whole rounds of its compute units goes in parts, of
+// 64 rows that are there and, where that gives every part a compute unit of its own, of 128 or 64 rows of the weights.  8192 tokens of 1024 channels,
+// 2 of 8 experts of 1024: 70 + 43 us (rests in their experts' places, and parts of rows alone: 77 + 48; tiles of 128 x 256 through registers, two
+// workgroups to a compute unit: 106 + 70); 2048 rows to every expert, whole rounds alone, 65 + 39.  Calls in a recorded graph, us, before and now, in
+// turn: 8192 tokens 150 -> 136, 4096 94 -> 88.5, 1000 51 -> 47, 500 43 -> 36.7; 1 of 8 of 2048, 1000 54 -> 45; 4 of 16 of 512, 2000 71.5 -> 68.5.  A
+// whole tile alone takes 29 us: its matrix instructions 22, at the rate that they reach by themselves here (1.6 PFLOP/s), the rest in front of the
+// first and behind the last.
 constexpr int kLargeRows = BASED_EXPERT_TILE_ROWS;
 constexpr int kDies = 8, kDieUnits = 32;
 constexpr int kHalf = 128 * kGemmK;  // elements of 128 rows of a round

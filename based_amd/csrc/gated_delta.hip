@@ -582,13 +582,13 @@ __global__ __launch_bounds__(NT) void gated_delta_step_kernel(const DeltaStepArg
     y[c] = from_f32<T>(so[c] * r * to_f32(static_cast<const T*>(a.norm_w)[c]) * silu_exact(to_f32(gate[c])) * a.scale);
 }
 
-// Whether a portion goes in one launch (`size`: bytes of an element).  Every workgroup of a head prepares all blocks for itself, on SIMDs that hold one
-// wavefront of its tiles where these take the registers of fp32 or leave rows empty, which is less than the launch while there are not many of them; an
-// odd number of blocks costs the two launches one more.  Kernels of a call, us, two launches / one, by tiles (16 columns of a head), of 2 and 3 blocks.
-// fp32, heads of 96: 768 20.3 / 15.2, 27.9 / 18.7; 1,536, of four 41.1 / 42.8, 38.1 / 35.1; 2,304 37.1 / 40.0, 54.4 / 52.1; 3,840 57 / 65, 84 / 86.  128: 2,048
-// 34.1 / 32.6, 50 / 43; 3,072 45.3 / 47.7, 71 / 64; 8,192 104 / 127, 170 / 166; bf16, of 112: 2,560 50.9 / 51.1, 76 / 67; 4,096 64 / 69, 100 / 89.  Whole rows,
-// bf16, 128: 5,120 61.6 / 60.7, 83.0 / 81.5; 8,192 87 / 92, 123 / 124; 64: 5,120 34.9 / 32.7, 45.9 / 43.7; 8,192 47.6 / 48.6, 63.5 / 63.3.  fp32 of up to 64: 8,192 65
-// / 56, 95 / 71.
+// Whether a portion goes in one launch (`size`: bytes of an element).  Every workgroup of a head prepares all blocks for itself, on SIMDs that hold
+// one wavefront of its tiles where these take the registers of fp32 or leave rows empty, which is less than the launch while there are not many of
+// them; an odd number of blocks costs the two launches one more.  Kernels of a call, us, two launches / one, by tiles (16 columns of a head), of 2
+// and 3 blocks. fp32, heads of 96: 768 20.3 / 15.2, 27.9 / 18.7; 1,536, of four 41.1 / 42.8, 38.1 / 35.1; 2,304 37.1 / 40.0, 54.4 / 52.1; 3,840 57 /
+// 65, 84 / 86.  128: 2,048 34.1 / 32.6, 50 / 43; 3,072 45.3 / 47.7, 71 / 64; 8,192 104 / 127, 170 / 166; bf16, of 112: 2,560 50.9 / 51.1, 76 / 67;
+// 4,096 64 / 69, 100 / 89.  Whole rows, bf16, 128: 5,120 61.6 / 60.7, 83.0 / 81.5; 8,192 87 / 92, 123 / 124; 64: 5,120 34.9 / 32.7, 45.9 / 43.7;
+// 8,192 47.6 / 48.6, 63.5 / 63.3.  fp32 of up to 64: 8,192 65 / 56, 95 / 71.
 static bool delta_short(const DeltaArgs& a, int size) {
   if (!a.vec || a.d > 128 || a.L > kShortBlocks * kBlk) return false;
   const long tiles = (long)a.B * a.H * ((a.dv + 15) / 16);
@@ -600,12 +600,13 @@ static bool delta_short(const DeltaArgs& a, int size) {
 }
 
 // Whether tiles of one wavefront go with one set of registers.  A SIMD holds three of them with one set and two with two (64 channels), or two and
-// one (128), so that one set saves a round where there are more tiles than that; but a block waits for its loads then, which long prompts feel.  Kernels of a
-// call, us, two sets / one, by tiles (16 columns of a head) and tokens.  64 channels: 2,048, 200 68 / 63.5, 400 110.6 / 108.6, 500 130 / 132, 732 181 /
-// 186, 1,500 353 / 377; 3,072, 400 159 / 147, 1,000 364 / 361, 1,500 533 / 540; 4,096, 200 117 / 109, 400 202 / 198, 732 347 / 357; 6,144, 400 298 / 285,
-// 1,000 711 / 711; fewer: 1,280, 1,232 273 / 283.  128 channels: 1,088, 65 64 / 49, 732 397 / 334; 2,048, 400 248 / 202; 2,304, 200 199 / 181, 800 661 / 648;
-// 2,560, 100 123 / 103, 150 151 / 152, 400 360 / 370; 3,072, 100 124 / 115, 150 153 / 157, 400 364 / 375, 800 687 / 721 (the second of two rounds is half
-// empty, for three whole ones); 3,200, 400 472 / 378; 5,120, 400 603 / 562; 8,192, 400 999 / 777; fewer: 1,024, 896 275 / 285.
+// one (128), so that one set saves a round where there are more tiles than that; but a block waits for its loads then, which long prompts feel.
+// Kernels of a call, us, two sets / one, by tiles (16 columns of a head) and tokens.  64 channels: 2,048, 200 68 / 63.5, 400 110.6 / 108.6, 500 130 /
+// 132, 732 181 / 186, 1,500 353 / 377; 3,072, 400 159 / 147, 1,000 364 / 361, 1,500 533 / 540; 4,096, 200 117 / 109, 400 202 / 198, 732 347 / 357;
+// 6,144, 400 298 / 285, 1,000 711 / 711; fewer: 1,280, 1,232 273 / 283.  128 channels: 1,088, 65 64 / 49, 732 397 / 334; 2,048, 400 248 / 202; 2,304,
+// 200 199 / 181, 800 661 / 648; 2,560, 100 123 / 103, 150 151 / 152, 400 360 / 370; 3,072, 100 124 / 115, 150 153 / 157, 400 364 / 375, 800 687 / 721
+// (the second of two rounds is half empty, for three whole ones); 3,200, 400 472 / 378; 5,120, 400 603 / 562; 8,192, 400 999 / 777; fewer: 1,024, 896
+// 275 / 285.
 static bool delta_one_set(int rb, long tiles, int L) {
   if (rb > 4) return tiles > 1024 && !(tiles > 2400 && tiles <= 3072 && L > 110);
   const bool fewer_rounds = (tiles + 3071) / 3072 < (tiles + 2047) / 2048;

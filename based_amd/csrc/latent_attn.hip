@@ -961,11 +961,12 @@ static int latent_check(const char* who, const LatentArgs& a, int64_t last, int 
   return BASED_OK;
 }
 
-// Up to two workgroups to a compute unit, of latents of 65 to 256 channels; of more one, whose registers and LDS leave no second one room, and of fewer one, whose
-// queries are not worth more (kernels, with a launch / without, by workgroups: R = 512 256 25.9 / 21.0, 320 27.5 / 31.9, 512 25.6 / 29.7; R = 64 256 12.0 /
-// 11.1, 320 12.95 / 13.4, 504 12.4 / 13.0; R = 128 504 13.5 / 13.1).  Whole calls, us, with a launch for the queries and without, 16 heads, R = 256, by sequences and
-// keys (workgroups): 1, 129 (24): 15.5 / 12.6; 4, 512 (256): 17.0 / 13.6; 6, 512 (384): 17.3 / 15.3; 16, 129 (384): 16.5 / 14.4; 4, 1,024 (512): 18.1 /
-// 16.0; 24, 129 (576): 16.6 / 18.6; 12, 512 (768): 18.7 / 22.6.  Four heads to a workgroup take as long at 512 and 13.6 -> 14.8 at 256.
+// Up to two workgroups to a compute unit, of latents of 65 to 256 channels; of more one, whose registers and LDS leave no second one room, and of
+// fewer one, whose queries are not worth more (kernels, with a launch / without, by workgroups: R = 512 256 25.9 / 21.0, 320 27.5 / 31.9, 512 25.6 /
+// 29.7; R = 64 256 12.0 / 11.1, 320 12.95 / 13.4, 504 12.4 / 13.0; R = 128 504 13.5 / 13.1).  Whole calls, us, with a launch for the queries and
+// without, 16 heads, R = 256, by sequences and keys (workgroups): 1, 129 (24): 15.5 / 12.6; 4, 512 (256): 17.0 / 13.6; 6, 512 (384): 17.3 / 15.3; 16,
+// 129 (384): 16.5 / 14.4; 4, 1,024 (512): 18.1 / 16.0; 24, 129 (576): 16.6 / 18.6; 12, 512 (768): 18.7 / 22.6.  Four heads to a workgroup take as
+// long at 512 and 13.6 -> 14.8 at 256.
 constexpr int kOwnHeads = 2;
 static int64_t own_max(int64_t R) { return R > 64 && R <= 256 ? 512 : 256; }
 
@@ -1021,10 +1022,11 @@ template <int KC, int RT> void launch_latent_f32(const LatentArgs& a, hipStream_
 
 static bool launch_latent_step_f32(const LatentArgs& a, hipStream_t s) {
   const int kc = (a.R + a.rot + 15) / 16, rt = (a.R + 63) / 64;
-  // Few workgroups on the vector unit, of few keys each, are the shorter way for long rows.  Us, one way / the other, by those workgroups, 16 heads.  R =
-  // 256, 48 keys each: 48 17.7 / 18.2; 192 18.5 / 18.8; 336 19.1 / 19.1; 768 20.9 / 18.9; 8 heads, 24 17.7 / 17.7, 168 18.7 / 18.6; 64 keys: 128 19.7 / 18.9;
-  // 256 20.3 / 19.7.  R = 512, a row at a time for its registers, 48 keys: 48 26.2 / 27.9; 192 27.2 / 29.2; 336 28.7 / 29.3; 768 42.8 / 29.3; 8 heads, 168 27.5 /
-  // 28.8, 384 40.9 / 28.6; 64 keys: 128 29.6 / 29.0; 256 30.3 / 29.5; 512 42 / 30; in 32 splits, 128 28.8 / 29.8, 256 40.9 / 30.1.
+  // Few workgroups on the vector unit, of few keys each, are the shorter way for long rows.  Us, one way / the other, by those workgroups, 16 heads.
+  // R = 256, 48 keys each: 48 17.7 / 18.2; 192 18.5 / 18.8; 336 19.1 / 19.1; 768 20.9 / 18.9; 8 heads, 24 17.7 / 17.7, 168 18.7 / 18.6; 64 keys: 128
+  // 19.7 / 18.9; 256 20.3 / 19.7.  R = 512, a row at a time for its registers, 48 keys: 48 26.2 / 27.9; 192 27.2 / 29.2; 336 28.7 / 29.3; 768 42.8 /
+  // 29.3; 8 heads, 168 27.5 / 28.8, 384 40.9 / 28.6; 64 keys: 128 29.6 / 29.0; 256 30.3 / 29.5; 512 42 / 30; in 32 splits, 128 28.8 / 29.8, 256 40.9
+  // / 30.1.
   const long wgs = (long)a.B * a.H * a.splits, all = a.window < a.S ? a.window : a.S;
   const bool few_keys = ((all + a.splits - 1) / a.splits + 15) / 16 * 16 < 64;
   if (kc <= 6 && rt <= 1)

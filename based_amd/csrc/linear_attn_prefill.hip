@@ -1004,13 +1004,13 @@ extern "C" BASED_API int based_linear_attn_prefill_plan(int64_t B, int64_t H, in
   const int64_t chains = B * H * ((dv + 63) / 64);
   const int64_t chunks = (L + kChunk - 1) / kChunk;
   // About one workgroup per compute unit, or from 32 chunks on two of those of one channel block where one each would leave many compute units alone
-  // (alone it is only 12 % slower per chunk than two sharing it, and every segment reads k and v twice): up to 64 of them 256 / n
-  // segments, above 4 or 512 / n; wide ones, of two channel blocks, 256 / n, but three from 12 chunks on and two from 32; beyond 128 the single pass
-  // wins.  For long sequences segments of at most 32 chunks while that still fits the resident slots (wide: the compute units; 16 segments / now, dv = 128, 8
-  // of 65,536 tokens 212 / 154, of 262,144 737 / 501, 2 of 262,144 720 / 145).  Calls, us, four segments (wide: eight up to 16, none above 64) / now, by
-  // workgroups, at 4,000 tokens and 8,000: 48 39.5 / 35.1, 66 / 58; 80 54 / 49, 92 / 82; 96 59 / 54, 104 / 95; dv = 128: 16 40.9 / 38.2, 60 / 49; 32 59.5 /
-  // 44.7, 101 / 68; 48 61 / 54, 103 / 95; 80 119 / 79, 229 / 148; 96 120 / 102, 230 / 195; 128 122 / 118, 232 / 216; 160 125 / 167 with two.  Shorter: 80 of
-  // 300 tokens 16.6 / 20.7 in two, of 1,500 51 / 42; 96 of 700 29 / 31 in two; 128 of 1,500 51.6 / 53.2.
+  // (alone it is only 12 % slower per chunk than two sharing it, and every segment reads k and v twice): up to 64 of them 256 / n segments, above 4
+  // or 512 / n; wide ones, of two channel blocks, 256 / n, but three from 12 chunks on and two from 32; beyond 128 the single pass wins.  For long
+  // sequences segments of at most 32 chunks while that still fits the resident slots (wide: the compute units; 16 segments / now, dv = 128, 8 of
+  // 65,536 tokens 212 / 154, of 262,144 737 / 501, 2 of 262,144 720 / 145).  Calls, us, four segments (wide: eight up to 16, none above 64) / now, by
+  // workgroups, at 4,000 tokens and 8,000: 48 39.5 / 35.1, 66 / 58; 80 54 / 49, 92 / 82; 96 59 / 54, 104 / 95; dv = 128: 16 40.9 / 38.2, 60 / 49; 32
+  // 59.5 / 44.7, 101 / 68; 48 61 / 54, 103 / 95; 80 119 / 79, 229 / 148; 96 120 / 102, 230 / 195; 128 122 / 118, 232 / 216; 160 125 / 167 with two.
+  // Shorter: 80 of 300 tokens 16.6 / 20.7 in two, of 1,500 51 / 42; 96 of 700 29 / 31 in two; 128 of 1,500 51.6 / 53.2.
   const bool wide = prefill_wide(dv);
   const int64_t wgs = B * H * prefill_workgroups_per_head(dv);
   if (wgs > kPrefillSlots / 4 || chunks < 2) return BASED_OK;
